@@ -81,6 +81,23 @@ def load():
     return _lib
 
 
+_host = None
+
+
+def host_call():
+    """The native host calls (``csrc/host_call.cpp``), loaded once; no fallback either."""
+    global _host
+    if _host is None:
+        load()
+        import torch  # noqa: F401  (its libraries first: the module links against them)
+        try:
+            from . import _host_call
+        except ImportError as e:
+            raise RuntimeError(f"rode_amd/_host_call.so cannot be loaded ({e}): build it with `make -C rode_amd/csrc`") from e
+        _host = _host_call
+    return _host
+
+
 def check(code, what):
     if code != 0:
         msg = load().rode_hip_error_string(code).decode()

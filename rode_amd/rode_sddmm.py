@@ -2,11 +2,12 @@
 ``RoDe_SDDMM/rode_sddmm.py``: ``RoDeCSR`` (:12-191), ``rode_sddmm`` (:194-248),
 ``torch_sddmm_reference`` (:251-304) and ``compare_results`` (:307-378).
 """
+import ctypes
 import math
 
 import torch
 
-from . import rode_sddmm_hip
+from . import _lib, rode_sddmm_hip
 
 
 class RoDeCSR:
@@ -182,6 +183,16 @@ class RoDeCSR:
             self._shared[key] = plans
         return plans
 
+    def plans_address(self, spmm_width=None):
+        """Where ``call_plans`` keeps its struct (an int, for the native calls).  Only a hub
+        plan's struct depends on the width (it carries the workspace)."""
+        if spmm_width is None or not isinstance(self.plan, rode_sddmm_hip.HubPlan):
+            address = self._shared.get("plans_address")
+            if address is None:
+                address = self._shared["plans_address"] = ctypes.addressof(self.call_plans())
+            return address
+        return ctypes.addressof(self.call_plans(spmm_width, 4))
+
     def spmm_stores_every_row(self):
         """Whether an SpMM on this matrix leaves no row of C to be cleared beforehand: every row
         has slots (rows without any are never written) and a single work item, which then stores
@@ -199,8 +210,6 @@ class RoDeCSR:
                     if isinstance(plan, rode_sddmm_hip.GroupPlan) and plan.usable and plan.counts[2] == 0:
                         cached = True  # every row is in a kept group: one wave (or workgroup) owns it
                     else:
-                        import ctypes
-                        from . import _lib
                         limit = _lib.load().rode_hip_spmm_overwrite_limit(self.m1, ctypes.byref(self.call_plans()))
                         cached = longest < 32 or longest <= limit
             self._shared["spmm_stores_every_row"] = cached
@@ -303,6 +312,14 @@ def rode_sddmm(sparse_matrix, lhs, rhs, values=None):
     Differentiable with respect to lhs, rhs and values (the reference op is
     forward-only)."""
     m, n, k = sparse_matrix.m, sparse_matrix.n, sparse_matrix.k
+    if values is None:
+        # the ordinary call, natively; None for everything that needs (or refuses) more
+        out = _lib.host_call().sddmm(
+            sparse_matrix.block_indices, sparse_matrix.residue_indices, sparse_matrix.st_offsets, sparse_matrix.m1,
+            sparse_matrix.m2, sparse_matrix.row_offsets, sparse_matrix.column_indices, sparse_matrix.values, m, n, k, lhs, rhs,
+            sparse_matrix.plans_address(), rode_sddmm_hip._stream_handle(sparse_matrix.device))
+        if out is not None:
+            return out
     if tuple(lhs.shape) != (m, k):
         raise ValueError(f"lhs_matrix shape must be ({m}, {k}), got {tuple(lhs.shape)}")
     if tuple(rhs.shape) != (n, k):

@@ -2,7 +2,7 @@
 (``RoDe_SpMM/RoDeSpmm.h:4-8``); this wraps the same entry point for tensors."""
 import torch
 
-from . import rode_sddmm_hip
+from . import _lib, rode_sddmm_hip
 
 
 def rode_spmm(sparse_matrix, dense, out=None, values=None):
@@ -11,6 +11,16 @@ def rode_spmm(sparse_matrix, dense, out=None, values=None):
     (m, width) float32 tensor.  ``values`` (optional)
     replaces the values of S for this call.  Differentiable with respect to dense
     and values when ``out`` is not given."""
+    if values is None and out is None and sparse_matrix.config["k_block"] == 32 and sparse_matrix.config["vec_len"] == 4:
+        # the ordinary call, natively; None for everything that needs (or refuses) more
+        hub = isinstance(sparse_matrix.plan, rode_sddmm_hip.HubPlan)
+        c = _lib.host_call().spmm(
+            sparse_matrix.block_indices, sparse_matrix.residue_indices, sparse_matrix.st_offsets, sparse_matrix.m1,
+            sparse_matrix.m2, sparse_matrix.row_offsets, sparse_matrix.column_indices, sparse_matrix.values,
+            sparse_matrix.m, sparse_matrix.n, dense, sparse_matrix.plans_address(dense.shape[1] if hub and dense.dim() == 2 else None),
+            sparse_matrix.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(sparse_matrix.device))
+        if c is not None:
+            return c
     if dense.dim() != 2 or dense.shape[0] != sparse_matrix.n:
         raise ValueError(f"dense shape must be ({sparse_matrix.n}, width), got {tuple(dense.shape)}")
     vec = 8 if dense.dtype == torch.float16 else 4

@@ -1,0 +1,60 @@
+"""The native host calls behind rode_sddmm and rode_spmm: the same results as the module's functions, and everything
+that is not the ordinary call still reaches the Python layer."""
+import numpy as np
+import pytest
+import torch
+
+from rode_amd import RoDeCSR, _lib, rode_sddmm, rode_sddmm_hip, rode_spmm
+
+pytestmark = pytest.mark.gpu
+
+
+def _matrix(m, n, k, seed=0):
+    rng = np.random.default_rng(seed)
+    lens = np.minimum(rng.integers(0, 70, size=m), n)
+    rp = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, size=v, replace=False)) for v in lens] + [np.zeros(0)]).astype(np.int32)
+    return RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(rng.standard_normal(len(col)).astype(np.float32)),
+                   "cuda", m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k,half", [(1, 40, 32, False), (257, 300, 64, True), (1000, 77, 20, False)])
+def test_native_call_equals_the_module_functions(m, n, k, half):
+    a = _matrix(m, n, k)
+    kind = torch.float16 if half else torch.float32
+    lhs, rhs = torch.randn(m, k, device="cuda").to(kind), torch.randn(n, k, device="cuda").to(kind)
+    if k % (8 if half else 4) == 0:
+        args = (a.block_indices, a.residue_indices, a.st_offsets, a.m1, a.m2, a.row_offsets, a.column_indices, a.values, a.m, a.n)
+        got = _lib.host_call().sddmm(*args, k, lhs, rhs, a.plans_address(), rode_sddmm_hip._stream_handle(a.device))
+        want = rode_sddmm_hip.sddmm_forward(*args, lhs, rhs, k, plan=a.plan)
+        assert got is not None and torch.equal(got, want) and torch.equal(rode_sddmm(a, lhs, rhs), want)
+        got, want = rode_spmm(a, rhs), rode_sddmm_hip.spmm_forward(*args, rhs, plan=a.plan)
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-5)
+
+
+def test_other_calls_reach_the_python_layer():
+    a = _matrix(64, 50, 32)
+    lhs, rhs = torch.randn(64, 32, device="cuda"), torch.randn(50, 32, device="cuda")
+    want = rode_sddmm(a, lhs, rhs)
+    torch.testing.assert_close(rode_sddmm(a, lhs.t().contiguous().t(), rhs), want)  # not contiguous
+    assert rode_sddmm(a, lhs.clone().requires_grad_(), rhs).grad_fn is not None
+    assert rode_spmm(a, rhs.clone().requires_grad_()).grad_fn is not None
+    with torch.no_grad():
+        assert rode_spmm(a, rhs.clone().requires_grad_()).grad_fn is None
+    with pytest.raises(ValueError, match="lhs_matrix shape"):
+        rode_sddmm(a, rhs, lhs)
+    with pytest.raises(AssertionError, match="must be on"):
+        rode_sddmm(a, lhs.cpu(), rhs)
+    with pytest.raises(AssertionError, match="rhs must be"):
+        rode_sddmm(a, lhs, rhs.half())
+    with pytest.raises(ValueError, match="dense width"):
+        rode_spmm(a, torch.randn(50, 30, device="cuda"))
+    with pytest.raises(ValueError, match="dense shape"):
+        rode_spmm(a, torch.randn(50, device="cuda"))
+    torch.testing.assert_close(rode_sddmm(a.with_values(2 * a.values), lhs, rhs), 2 * want)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = rode_sddmm(a, lhs, rhs)
+    side.synchronize()
+    assert torch.equal(got, want)
