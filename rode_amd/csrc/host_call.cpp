@@ -1,5 +1,5 @@
 // Host side of the Python ops, natively: the calls that a program makes once per product
-// (rode_sddmm, rode_spmm), and the pass over the row offsets that a new matrix needs.
+// (rode_sddmm, rode_spmm), and what a new matrix needs (row statistics, decomposition).
 //
 // A small matrix takes a few microseconds on the GPU, so its calls are bound by what the host
 // does around the launch: argument checks, an allocation and the launch itself cost 10-11 us
@@ -19,6 +19,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <string>
 
 #include "../../include/rode_hip.h"
 
@@ -141,7 +142,164 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     return THPVariable_Wrap(std::move(out));
 }
 
+// ---- a new matrix ------------------------------------------------------------------------
+// What RoDeCSR asks of the row offsets, in one pass (a dozen vector instructions per eight
+// rows; as a chain of tensor operations it takes 0.3 - 1 ms for 65 K rows, mostly waking threads).
+struct RowStats {
+    long long max_len = 0;                             // longest row
+    long long shortest = INT64_MAX, longest = INT64_MIN; // ... counted in aligned slots (a row from its start & ~3)
+    long long blocked = 0;                             // rows with block segments (32 aligned slots or more)
+    long long segments_512 = 0;                        // segments of 512 slots that those rows have
+    long long up_to_512 = 0, up_to_1024 = 0;           // those of at most that many slots
+    long long hub_nonzeros = 0;                        // nonzeros of the rows of hub_min_len aligned slots or more
+};
+
+// (sums of a block in the offsets' own type: they cannot pass the last offset)
+template <typename T>
+__attribute__((target_clones("avx512f", "avx2", "default"))) void row_stats_block(const T* ro, long long rows, T hub_min_len, RowStats& r)
+{
+    T max_len = 0, shortest = r.shortest > INT32_MAX ? (T)INT32_MAX : (T)r.shortest, longest = INT32_MIN;
+    T blocked = 0, segments = 0, up_to_512 = 0, up_to_1024 = 0, hub = 0;
+    for (long long i = 0; i < rows; ++i) {
+        const T len = ro[i + 1] - ro[i], aligned = len + (ro[i] & 3);
+        const T is_blocked = aligned >= 32 ? 1 : 0, is_hub = aligned >= hub_min_len ? -1 : 0; // (a mask)
+        max_len = len > max_len ? len : max_len;
+        shortest = aligned < shortest ? aligned : shortest;
+        longest = aligned > longest ? aligned : longest;
+        blocked += is_blocked;
+        segments += is_blocked * ((aligned + 511) >> 9);
+        up_to_512 += is_blocked & (aligned <= 512 ? 1 : 0);
+        up_to_1024 += is_blocked & (aligned <= 1024 ? 1 : 0);
+        hub += len & is_hub;
+    }
+    r.max_len = std::max<long long>(r.max_len, max_len);
+    r.shortest = std::min<long long>(r.shortest, shortest);
+    r.longest = std::max<long long>(r.longest, longest);
+    r.blocked += blocked, r.segments_512 += segments, r.up_to_512 += up_to_512, r.up_to_1024 += up_to_1024;
+    r.hub_nonzeros += hub;
+}
+
+// row_stats(row offsets on the CPU, int32 or int64; hub_min_len) -> the fields of RowStats
+PyObject* row_stats(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    const at::Tensor* ro = count == 2 ? tensor_of(args[0]) : nullptr;
+    long long hub_min_len;
+    if (!ro || !int_of(args[1], hub_min_len) || !ro->is_cpu() || ro->dim() != 1 || !ro->is_contiguous() ||
+        (ro->scalar_type() != at::kInt && ro->scalar_type() != at::kLong))
+        return PyErr_Format(PyExc_ValueError, "row_stats takes a contiguous int32 or int64 vector on the CPU and an int");
+    const long long rows = ro->size(0) - 1;
+    RowStats r;
+    Py_BEGIN_ALLOW_THREADS
+    constexpr long long kBlock = 1 << 16; // (a block's sums are added up in 64 bits)
+    for (long long at = 0; at < rows; at += kBlock) {
+        const long long n = std::min(kBlock, rows - at);
+        if (ro->scalar_type() == at::kInt)
+            row_stats_block<int32_t>(static_cast<const int32_t*>(ro->data_ptr()) + at, n,
+                                     (int32_t)std::min<long long>(hub_min_len, INT32_MAX), r);
+        else
+            row_stats_block<int64_t>(static_cast<const int64_t*>(ro->data_ptr()) + at, n, hub_min_len, r);
+    }
+    Py_END_ALLOW_THREADS
+    if (rows <= 0) r.shortest = r.longest = 0;
+    return Py_BuildValue("(LLLLLLLL)", r.max_len, r.shortest, r.longest, r.blocked, r.segments_512, r.up_to_512, r.up_to_1024,
+                         r.hub_nonzeros);
+}
+
+// How many block segments and residue rows the decomposition has (k_block 32, vec_len 4): the
+// closed form per row that the GPU's decompose_kernel uses (rode_preprocess.hip, row_counts).
+__attribute__((target_clones("avx512f", "avx2", "default"))) void list_sizes_shift(const int32_t* ro, long long rows, int shift, long long& n_blk, long long& n_res)
+{
+    int32_t blk = 0, res = 0; // (both totals are below 2^31)
+    for (long long i = 0; i < rows; ++i) {
+        const int32_t n = ro[i + 1] - ro[i] + (ro[i] & 3);
+        const int32_t some = n > 0 ? 1 : 0;
+        const int32_t t = (n - some) >> shift, rest = n - (int32_t)((uint32_t)t << shift);
+        blk += some * (t + (rest >= 32 ? 1 : 0));
+        res += some & ((rest & 31) != 0 ? 1 : 0);
+    }
+    n_blk = blk, n_res = res;
+}
+
+void list_sizes(const int32_t* ro, long long rows, int seg, long long& n_blk, long long& n_res)
+{
+    if ((seg & (seg - 1)) == 0) return list_sizes_shift(ro, rows, __builtin_ctz(seg), n_blk, n_res);
+    n_blk = n_res = 0;
+    for (long long i = 0; i < rows; ++i) {
+        const int32_t n = ro[i + 1] - ro[i] + (ro[i] & 3);
+        if (n <= 0) continue;
+        const int32_t t = (n - 1) / seg, rest = n - t * seg;
+        n_blk += t + (rest >= 32 ? 1 : 0);
+        n_res += (rest & 31) != 0 ? 1 : 0;
+    }
+}
+
+// decompose(row offsets on the CPU, the same on the GPU, columns or None, dense rows, segment
+// length, stream) -> (block_indices, st_offsets, residue_indices, m1, m2, plan, counts): the row
+// decomposition and, with the columns given, the descriptors of a locality plan (tensor and its
+// four counts; else None, None).  The list lengths are counted here, so that the lists are
+// allocated at their size and everything is queued at once: one wait for the whole of it
+// instead of one for the counts, one for the plan and a copy of every list.
+PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    long long dense_rows, seg, stream;
+    if (count != 6 || !int_of(args[3], dense_rows) || !int_of(args[4], seg) || !int_of(args[5], stream))
+        return PyErr_Format(PyExc_ValueError, "decompose takes 6 arguments");
+    const at::Tensor *host = tensor_of(args[0]), *dev = tensor_of(args[1]), *col = args[2] == Py_None ? nullptr : tensor_of(args[2]);
+    if (!host || !dev || !host->is_cpu() || !dev->is_cuda() || host->scalar_type() != at::kInt || dev->scalar_type() != at::kInt ||
+        host->dim() != 1 || dev->dim() != 1 || host->size(0) < 1 || host->size(0) != dev->size(0) || !host->is_contiguous() ||
+        !dev->is_contiguous() || seg <= 0 || seg > INT32_MAX || (args[2] != Py_None && (!col || !col->is_cuda() || col->scalar_type() != at::kInt)))
+        return PyErr_Format(PyExc_ValueError, "decompose takes int32 row offsets on the CPU and on the GPU");
+    const long long m = dev->size(0) - 1;
+    at::Tensor blk, start, res, plan, scratch, counts;
+    long long m1 = 0, m2 = 0;
+    int code = 0;
+    const char* what = "rode_hip_preprocess";
+    std::string error;
+    Py_BEGIN_ALLOW_THREADS
+    try {
+        list_sizes(static_cast<const int32_t*>(host->data_ptr()), m, (int)seg, m1, m2);
+        blk = at::empty({std::max(m1, 1ll)}, dev->options());
+        start = at::empty({m1 + 1}, dev->options());
+        res = at::empty({std::max(m2, 1ll)}, dev->options());
+        const size_t ws_bytes = rode_hip_preprocess_workspace_bytes((int)m);
+        scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
+        // (pinned: the kernels write the counts where the host reads them)
+        counts = at::empty({8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        int* h = static_cast<int*>(counts.data_ptr());
+        h[0] = h[1] = -1;
+        const int* rp = static_cast<const int*>(dev->data_ptr());
+        hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+        code = rode_hip_preprocess((int)seg, 32, 4, (int)m, rp, static_cast<int*>(blk.data_ptr()), static_cast<int*>(start.data_ptr()),
+                                   static_cast<int*>(res.data_ptr()), h, h + 1, (int)m1, scratch.data_ptr(), ws_bytes, s);
+        if (code == 0 && col && m2 > 0) {
+            what = "rode_hip_window_plan";
+            const size_t bytes = rode_hip_window_plan_bytes((int)m2);
+            plan = at::empty({(int64_t)(bytes / 4)}, dev->options());
+            code = rode_hip_window_plan((int)m2, (int)dense_rows, static_cast<const int*>(res.data_ptr()), rp,
+                                        static_cast<const int*>(col->data_ptr()), plan.data_ptr(), bytes, nullptr, s);
+            if (code == 0) code = hipMemcpyAsync(h + 4, plan.data_ptr(), 4 * sizeof(int), hipMemcpyDeviceToHost, s);
+        }
+        const int waited = hipStreamSynchronize(s); // (also after an error: the scratch is in use until then)
+        if (code == 0) code = waited;
+        if (code == 0 && (h[0] != m1 || h[1] != m2)) error = "the row decomposition on the GPU does not have the expected size";
+    } catch (const std::exception& e) {
+        error = e.what();
+    }
+    Py_END_ALLOW_THREADS
+    if (!error.empty()) return PyErr_Format(PyExc_RuntimeError, "%s", error.c_str());
+    if (code != 0) return failed(what, code);
+    const int* h = static_cast<const int*>(counts.data_ptr());
+    PyObject* plan_counts = plan.defined() ? Py_BuildValue("[iiii]", h[4], h[5], h[6], h[7]) : Py_BuildValue("");
+    PyObject* plan_data = plan.defined() ? THPVariable_Wrap(std::move(plan)) : Py_BuildValue("");
+    return Py_BuildValue("(NNNLLNN)", THPVariable_Wrap(std::move(blk)), THPVariable_Wrap(std::move(start)), THPVariable_Wrap(std::move(res)),
+                         m1, m2, plan_data, plan_counts);
+}
+
 PyMethodDef methods[] = {
+    {"row_stats", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(row_stats)), METH_FASTCALL,
+     "row_stats(row_offsets, hub_min_len) -> (max_len, shortest, longest, blocked, segments_512, up_to_512, up_to_1024, hub_nonzeros)"},
+    {"decompose", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(decompose)), METH_FASTCALL,
+     "decompose(row_offsets_cpu, row_offsets, columns or None, dense_rows, seg_length, stream) -> (block, start, residue, m1, m2, plan, counts)"},
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(sddmm)), METH_FASTCALL,
      "sddmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, k, lhs, rhs, plans, stream) -> tensor or None"},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(spmm)), METH_FASTCALL,

@@ -53,10 +53,13 @@ class RoDeCSR:
             # what the operand checks of the ops compare with
             self.device = torch.device("cuda", torch.cuda.current_device())
         self.row_offsets_cpu = row_offsets.to(dtype=torch.int32, device="cpu").contiguous()
+        # one pass over the row offsets: the longest row, the choice of the segment length and of a plan
+        self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len())
+        self.max_row_length = self._stats[0]
         if isinstance(config, str):
             if config != "auto":
                 raise ValueError(f'config must be a dict, None or "auto", got {config!r}')
-            config = self.auto_config(self.row_offsets_cpu)
+            config = self._config_from(self._stats)
         self.config = dict(config) if config is not None else dict(self.CONFIGS.get(k, self.DEFAULT_CONFIG))
         cfg = self.config
         if cfg.get("k_block") != 32 or cfg.get("vec_len") != 4 or cfg.get("seg_length", 0) <= 0 \
@@ -67,8 +70,6 @@ class RoDeCSR:
         self.column_indices = column_indices.to(dtype=torch.int32, device=self.device).contiguous()
         self.values = values.to(dtype=torch.float32, device=self.device).contiguous()
         self.row_offsets = self.row_offsets_cpu.to(device=self.device)
-        ro = self.row_offsets_cpu
-        self.max_row_length = int((ro[1:] - ro[:-1]).max()) if ro.numel() > 1 else 0
         if locality not in (True, False, "auto"):
             raise ValueError(f'locality must be True, False or "auto", got {locality!r}')
         self.locality = locality
@@ -92,13 +93,13 @@ class RoDeCSR:
         ro = row_offsets.to(device="cpu")
         if ro.dtype not in (torch.int32, torch.int64):
             ro = ro.to(torch.int64)
-        start = ro[:-1]
-        aligned = (ro[1:] - start) + (start & 3)
-        blocked = aligned >= 32  # rows that have block segments
-        rows = int(blocked.sum())
+        return cls._config_from(_lib.host_call().row_stats(ro.contiguous(), 1))
+
+    @staticmethod
+    def _config_from(stats):
+        _, _, _, rows, segments, up_to_512, up_to_1024, _ = stats  # (rows: those that have block segments)
         seg = 512
         if rows > 0:
-            segments = int((((aligned + 511) >> 9) * blocked).sum())  # at 512 slots a segment (the sum is 64-bit)
             if segments < 16384:
                 seg = 128
             else:
@@ -106,28 +107,32 @@ class RoDeCSR:
                 # order statistic torch.quantile(..., "higher") returns lies at or below a length
                 # exactly when that many rows do (counting avoids quantile's 16 M element limit)
                 rank = min(rows, math.ceil(0.9 * (rows - 1)) + 1)
-                while seg < 2048 and int((blocked & (aligned <= seg)).sum()) < rank:
-                    seg *= 2
+                seg = 512 if up_to_512 >= rank else 1024 if up_to_1024 >= rank else 2048
         return {"seg_length": seg, "k_block": 32, "vec_len": 4}
 
     def _preprocess(self):
         """Row decomposition on the GPU; the index arrays never visit the host."""
-        cfg = self.config
-        blk, st, res, m1, m2 = rode_sddmm_hip.preprocess_device(
-            self.row_offsets, self.nnz, cfg["seg_length"], cfg["k_block"], cfg["vec_len"])
+        # Locality plan: chunks of the residue list whose dense rows cluster in a window that
+        # fits LDS (banded matrices) go to the window kernels.  Kept only when it pays:
+        # "auto" wants windows on at least half of the chunks and enough of them to fill the
+        # GPU twice (a few windowed chunks only add launches); True keeps any plan with a
+        # window; False makes none.  Unless another kind of plan may come first, its
+        # descriptors are queued along with the decomposition.
+        others = self.locality and (self._may_group() or self._may_hub())
+        rode_sddmm_hip._check_input(self.row_offsets, "row_offsets")
+        with rode_sddmm_hip._on_device(self.device):
+            blk, st, res, m1, m2, data, counts = _lib.host_call().decompose(
+                self.row_offsets_cpu, self.row_offsets, self.column_indices if self.locality and not others else None,
+                self.n, self.config["seg_length"], rode_sddmm_hip._stream_handle(self.device))
         self.block_indices = blk
         self.st_offsets = st
         self.residue_indices = res
         self.m1 = m1
         self.m2 = m2
-        # Locality plan: chunks of the residue list whose dense rows cluster in a window that
-        # fits LDS (banded matrices) go to the window kernels.  Kept only when it pays:
-        # "auto" wants windows on at least half of the chunks and enough of them to fill the
-        # GPU twice (a few windowed chunks only add launches); True keeps any plan with a
-        # window; False makes none.
-        self.plan = (self._group_plan() or self._hub_plan()) if self.locality else None
+        self.plan = (self._group_plan() or self._hub_plan()) if others else None
         if self.plan is None and self.locality and m2 > 0:
-            plan = rode_sddmm_hip.window_plan(res, m2, self.row_offsets, self.column_indices, self.n)
+            plan = rode_sddmm_hip.WindowPlan(data, counts) if data is not None else \
+                rode_sddmm_hip.window_plan(res, m2, self.row_offsets, self.column_indices, self.n)
             enough = plan.windowed >= max(self.PLAN_MIN_CHUNKS, (plan.counts[0] + 1) // 2)
             if plan.windowed > 0 and (self.locality is True or enough):
                 self.plan = rode_sddmm_hip.window_plan_rows(plan, res, m2, self.row_offsets, self.column_indices)
@@ -144,31 +149,32 @@ class RoDeCSR:
     # nonzeros per row (a shared run has at least 64 columns).
     GROUP_MIN_MEAN = 64
 
+    def _may_group(self):
+        return self.m >= 4 and self.nnz >= self.GROUP_MIN_MEAN * self.m
+
     def _group_plan(self):
         """Group plan (adjacent rows that share a long run of consecutive columns are processed
         together, each dense row of the run loaded once for all of them), or None."""
-        if self.m < 4 or self.nnz < self.GROUP_MIN_MEAN * self.m:
+        if not self._may_group():
             return None
         plan = rode_sddmm_hip.group_plan(self.row_offsets, self.column_indices, self.m)
         enough = 2 * plan.counts[1] >= plan.counts[0]
         return plan if plan.usable and (self.locality is True or enough) else None
 
+    def _hub_min_len(self):
+        return max(self.HUB_MIN_LEN, 8 * ((self.n + 4095) // 4096))
+
+    def _may_hub(self):
+        hub_nnz = self._stats[7]  # nonzeros of the rows of that (aligned) length or more
+        return (self.n + 4095) // 4096 >= self.HUB_MIN_SLABS and hub_nnz > 0 and \
+            (self.locality is True or hub_nnz >= self.HUB_MIN_SHARE * self.nnz)
+
     def _hub_plan(self):
         """Hub plan (rows with very many nonzeros are processed column slab by column slab so
         that they share the dense rows they fetch), or None when the pattern has no use for it."""
-        slabs = (self.n + 4095) // 4096
-        if slabs < self.HUB_MIN_SLABS or self.nnz == 0:
+        if not self._may_hub():
             return None
-        min_len = max(self.HUB_MIN_LEN, 8 * slabs)
-        start = self.row_offsets_cpu[:-1]
-        lens = self.row_offsets_cpu[1:] - start
-        hub = (lens + (start & 3)) >= min_len  # (aligned length, as the kernels count it)
-        hub_nnz = int((lens * hub).sum())  # (summed in 64 bits)
-        if self.locality is not True and hub_nnz < self.HUB_MIN_SHARE * self.nnz:
-            return None
-        if hub_nnz == 0:
-            return None
-        plan = rode_sddmm_hip.hub_plan(self.row_offsets, self.column_indices, self.m, self.n, int(min_len))
+        plan = rode_sddmm_hip.hub_plan(self.row_offsets, self.column_indices, self.m, self.n, self._hub_min_len())
         return plan if plan.usable else None
 
     def call_plans(self, spmm_width=None, spmm_elem_bytes=4):
@@ -202,9 +208,7 @@ class RoDeCSR:
         if cached is None:
             cached = False
             if self.m > 0 and self.nnz > 0:
-                start = self.row_offsets_cpu[:-1]
-                aligned = (self.row_offsets_cpu[1:] - start) + (start & 3)  # slots as the kernels count them
-                shortest, longest = int(aligned.min()), int(aligned.max())
+                shortest, longest = self._stats[1:3]  # (slots as the kernels count them)
                 if shortest > 0:
                     plan = self.plan
                     if isinstance(plan, rode_sddmm_hip.GroupPlan) and plan.usable and plan.counts[2] == 0:
