@@ -239,8 +239,11 @@ int rode_hip_hub_plan(int M, int dense_rows, int nnz, int min_len, const int* d_
  *   d_plan       rode_hip_group_plan_bytes(M) bytes, 16-byte aligned, out
  *   h_counts     HOST int[4], out (the call waits for its kernels): [0] groups (M / 4,
  *                whole groups only), [1] groups with a run, [2] rows outside those groups
- *                (0: the other kernels have nothing to do and are not launched); the
- *                *_planned entry points need it and ignore a plan with [1] == 0
+ *                (0: the other kernels have nothing to do and are not launched), [3] tiles:
+ *                blocks of 16 rows (from row 0 on) whose four groups all have runs that
+ *                overlap for the most part - the attention kernels work on those with the
+ *                matrix cores; the *_planned entry points need it and ignore a plan with
+ *                [1] == 0
  * A group plan belongs to the pattern it was made from and excludes the other two plans.
  * SDDMM uses it for k <= 128 elements (fp32 and fp16 alike: rows of one 128-element slab; wider
  * rows go through the list kernels, plan or not), SpMM for any width.

@@ -30,27 +30,10 @@ namespace rode {
 
 namespace {
 
-__device__ __forceinline__ float wave_max_f(float v)
-{
-    v = fmaxf(v, lane_xor1(v));
-    v = fmaxf(v, lane_xor2(v));
-    v = fmaxf(v, lane_xor4(v));
-    v = fmaxf(v, lane_xor8(v));
-    v = fmaxf(v, lane_xor16(v));
-    return fmaxf(v, lane_xor32(v));
-}
-
 // (four waves per SIMD: measured best on the attention-mask benchmark, 16384 rows of 570
 // nonzeros, against 3, 5, 6 and 8; the registers that frees go to gathers in flight)
 // Raw scores of a row that wait in LDS for the row's maximum and sum (per wave).
 constexpr int kScoresKept = 1024;
-
-// What a kernel leaves behind for the gradient.
-enum Keep : int {
-    kKeepNothing = 0,
-    kKeepProbs = 1,  // probs[idx] = the probability
-    kKeepScores = 2, // probs[idx] = the scaled score, stats[row] = (row maximum, 1 / row sum)
-};
 
 template <typename T, int D, int KEEP>
 __global__ void __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
@@ -69,7 +52,7 @@ attention_rows_kernel(int M, const int* __restrict__ row_ptr, const int* __restr
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     const int row = xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
     if (row >= M) return;
-    if (owned_elsewhere(owners, row, 0)) return; // a row of a group: attention_group_kernel has it
+    if (owned_elsewhere(owners, row, 0) || in_tile(owners, row)) return; // a row of a group or of a tile: their kernels have it
     const int s = row_ptr[row], e = row_ptr[row + 1];
     const int ls = lane % LPR, group = lane / LPR;
     float* out_lane = out + (size_t)row * D + ls * VEC;
@@ -106,7 +89,7 @@ attention_rows_kernel(int M, const int* __restrict__ row_ptr, const int* __restr
             const float d = sddmm_unit<T, D, 1, false>(k_lane, a, c, D, my_c, lane);
             if (live) sc = scale * (w * d);
         }
-        const float m_new = fmaxf(m_run, wave_max_f(sc));
+        const float m_new = fmaxf(m_run, butterfly_max<1, kWave>(sc));
         const float m_safe = m_new == -INFINITY ? 0.f : m_new;
         const float corr = __expf(m_run - m_safe);
         const float p = live ? __expf(sc - m_safe) : 0.f;
@@ -147,23 +130,6 @@ attention_rows_kernel(int M, const int* __restrict__ row_ptr, const int* __restr
     }
 }
 
-// One step of the running softmax of a row: the scores of up to 64 slots (sc, -inf for a
-// lane without a slot) move the maximum; the row's sum and accumulated output are rescaled.
-// Returns this lane's probability relative to the new maximum.
-template <int VEC>
-__device__ __forceinline__ float softmax_step(float sc, bool live, float& m_run, float& l_lane, float (&acc)[VEC])
-{
-    const float m_new = fmaxf(m_run, wave_max_f(sc));
-    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
-    const float corr = __expf(m_run - m_safe);
-    const float p = live ? __expf(sc - m_safe) : 0.f;
-    l_lane = fmaf(l_lane, corr, p);
-#pragma unroll
-    for (int x = 0; x < VEC; ++x) acc[x] *= corr;
-    m_run = m_new;
-    return p;
-}
-
 // The groups of a group plan (rode_group.hip): one wave per group of four adjacent rows
 // whose runs of consecutive columns overlap in a long shared run (shared_run).  Along it every
 // k row and every v row is loaded once for the four rows (the score part is the SDDMM group kernel's, the output
@@ -178,7 +144,7 @@ __global__ void __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu
 attention_group_kernel(int n_groups, const RowGroup* __restrict__ groups, const int* __restrict__ row_ptr,
                        const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ q,
                        const T* __restrict__ k, const T* __restrict__ v, float scale, float* __restrict__ out,
-                       float* probs, float2* __restrict__ stats, HeadStrides heads)
+                       float* probs, float2* __restrict__ stats, RowOwners owners, HeadStrides heads)
 {
     constexpr bool WRITE_P = KEEP == kKeepProbs;
     q = of_head(q, heads.rows), k = of_head(k, heads.cols), v = of_head(v, heads.cols);
@@ -192,7 +158,7 @@ attention_group_kernel(int n_groups, const RowGroup* __restrict__ groups, const 
     float* my_s = lds_s + (WRITE_P ? wave * R * kGroupScoresKept : 0);
     const int g = xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
     if (g >= n_groups) return;
-    if (groups[g].len <= 0) return; // not a group: attention_rows_kernel has its rows
+    if (groups[g].len <= 0 || in_tile(owners, g * R)) return; // not a group, or part of a tile: other kernels have its rows
     const RowGroup d = shared_run(groups[g]); // the columns [lo, lo + len) that all four runs hold
     const int ls = lane % LPR, group = lane / LPR;
     const int row0 = g * R;
@@ -363,14 +329,30 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
     HeadStrides heads;
     heads.rows = (size_t)M * D, heads.cols = (size_t)N * D, heads.nnz = (size_t)nnz;
     const Keep keep = probs == nullptr ? kKeepNothing : stats != nullptr ? kKeepScores : kKeepProbs;
-    // a group plan is used when a wave per group fills the GPU
+    // The tiles of a group plan first (the matrix cores); the other groups when a wave per group
+    // fills the GPU; what is left row by row.
     RowOwners owners;
-    const bool grouped = plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] >= attention_groups_min<T>();
+    int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
+    // (the tile kernel addresses a head's k and v with 32-bit offsets; N = 0: not said, one head.  With
+    // fewer tiles than CUs and short rows a wave per row is faster: 128 tiles, 144 nonzeros per row of 128
+    // halves 13 against 15 us; 576 per row 17 against 14 us.)
+    const bool enough = (long long)(groups_left > 0 ? plan.group_counts[3] : 0) * nheads >= 256 || nnz >= 256ll * M;
+    if (groups_left > 0 && plan.group_counts[3] > 0 && enough && attention_tiles_fit(N, D * sizeof(T))) {
+        owners.tiles = group_plan_tiles(plan.groups, M);
+        owners.n_tiles = row_tiles(M);
+        groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);
+        rows_left -= plan.group_counts[3] * kTileRows;
+        const hipError_t e = attention_tiles_launch<T>(nheads, M, N, nnz, D, row_ptr, col, val, q, k, v, scale, out, probs,
+                                                       reinterpret_cast<float*>(stats), plan.groups, stream);
+        if (e != hipSuccess) return e;
+    }
+    const bool grouped = groups_left >= attention_groups_min<T>();
     if (grouped) {
         owners.groups = reinterpret_cast<const RowGroup*>(plan.groups + kGroupHeaderInts);
         owners.n_groups = plan.group_counts[0];
+        rows_left -= groups_left * kGroupRows;
     }
-    if (!(grouped && plan.group_counts[2] == 0)) { // (else every row is in a group)
+    if (rows_left > 0) {
         const dim3 grid((unsigned)wgs, (unsigned)nheads);
         if (keep == kKeepScores)
             attention_rows_kernel<T, D, kKeepScores><<<grid, kWgThreads, 0, stream>>>(M, row_ptr, col, val, q, k, v, scale, out,
@@ -388,13 +370,13 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
         const dim3 grid((unsigned)gw, (unsigned)nheads);
         if (keep == kKeepScores)
             attention_group_kernel<T, D, kKeepScores><<<grid, kWgThreads, 0, stream>>>(
-                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, heads);
+                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, owners, heads);
         else if (keep == kKeepProbs)
             attention_group_kernel<T, D, kKeepProbs><<<grid, kWgThreads, 0, stream>>>(
-                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, heads);
+                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, owners, heads);
         else
             attention_group_kernel<T, D, kKeepNothing><<<grid, kWgThreads, 0, stream>>>(
-                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, heads);
+                owners.n_groups, owners.groups, row_ptr, col, val, q, k, v, scale, out, probs, stats, owners, heads);
     }
     return hipGetLastError();
 }

@@ -35,18 +35,6 @@ namespace rode {
 
 namespace {
 
-template <int LO, int HI>
-__device__ __forceinline__ float butterfly_max(float v)
-{
-    if (LO <= 1 && 1 < HI) v = fmaxf(v, lane_xor1(v));
-    if (LO <= 2 && 2 < HI) v = fmaxf(v, lane_xor2(v));
-    if (LO <= 4 && 4 < HI) v = fmaxf(v, lane_xor4(v));
-    if (LO <= 8 && 8 < HI) v = fmaxf(v, lane_xor8(v));
-    if (LO <= 16 && 16 < HI) v = fmaxf(v, lane_xor16(v));
-    if (LO <= 32 && 32 < HI) v = fmaxf(v, lane_xor32(v));
-    return v;
-}
-
 template <int N>
 __device__ __forceinline__ void load_floats(const float* p, float (&out)[N])
 {

@@ -1,0 +1,368 @@
+// Sparse attention, forward, for the tiles of 16 rows of a group plan (sliding windows and
+// other masks whose adjacent rows share long runs of consecutive columns), on the matrix cores:
+//     out[r, :] = sum_idx p[idx] * v[col(idx), :],   p = softmax of scale * values[idx] * <q[r, :], k[col(idx), :]>
+// (the contract of rode_attention.hip, whose kernels take the rows of no tile).
+//
+// One workgroup per tile and head.  Its four waves take the columns of the run 16 or 32 at a time, in
+// turn (score products of 16 x 16, a running softmax, D / 16 weighted-sum products; layouts in
+// rode_tile.hpp), and the nonzeros outside the run of four rows each, 64 at a time, as
+// attention_rows_kernel does; every wave, and every row outside its run, has a softmax of its own,
+// and the partial results meet in LDS.  Columns at the ends of the range that a row does not hold get
+// probability zero.  A non-finite row of v there would reach rows that do not reference it
+// (0 * Inf), and shows as a non-finite result: the tile's rows are then computed again, all of them
+// row by row.
+//
+// Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with
+// four rows at a time on the vector ALUs, 0.219 here; eight heads in fp32 0.693 -> 0.473.  Of the 0.219
+// about 0.06 are the columns of the run, 0.11 the nonzeros outside it (11 % of all; their dense rows
+// ask the vector memory pipe for 64 B/clk/CU half of the time, a quarter of them misses L2), 0.02 a
+// workgroup's start and end.  What was slow on the way: dense rows and values loaded straight into
+// operand layout (adjacent lanes on different rows: 64 clocks of the memory pipe per load, 0.38 ms).
+//
+// 32-bit operands use the 32-bit matrix instructions (exact products, 157 TFLOP/s against 79 on the
+// vector ALUs); 16-bit operands split the probabilities into two halves each (TileWeights).
+#include "rode_tile.hpp"
+#include "rode_units.hpp"
+#include "rode_internal.hpp"
+
+#include <type_traits>
+
+namespace rode {
+
+namespace {
+
+// Running softmax of the rows of a tile: 4 or 8 scores of this lane's row at a time (-inf: none), in
+// units in which a probability is exp2(unit * score).
+template <typename T, int D>
+struct TileSoftmax {
+    static constexpr int N = 4 * tile_blocks<T>();
+    float m = -INFINITY;             // maximum of the row (the same in its four lanes)
+    f32x4 l = {0.f, 0.f, 0.f, 0.f};  // sum of the row, four times
+    f32x4 acc[D / 16];
+    __device__ __forceinline__ TileSoftmax()
+    {
+#pragma unroll
+        for (int b = 0; b < D / 16; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    __device__ __forceinline__ void step(const float (&sc)[N], float unit, TileWeights<T>& weights)
+    {
+        float top = sc[0];
+#pragma unroll
+        for (int j = 1; j < N; ++j) top = fmaxf(top, sc[j]);
+        const float m_new = fmaxf(m, quad_max(top));
+        if (__any(m_new > m)) {
+            const float corr = __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * unit);
+            l *= corr;
+#pragma unroll
+            for (int b = 0; b < D / 16; ++b) acc[b] *= corr;
+            m = m_new;
+        }
+        const float off = TileWeights<T>::kShift - (m == -INFINITY ? 0.f : m) * unit;
+        float p[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(sc[j], unit, off));
+        weights.set(p);
+        weights.add_sums(l);
+    }
+};
+
+template <typename T, int D, int KEEP>
+__global__ void __launch_bounds__(kWgThreads)
+attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int* __restrict__ runs,
+                      const int* __restrict__ row_ptr, const int* __restrict__ col, const float* __restrict__ val,
+                      const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, float scale,
+                      float* __restrict__ out, float* probs, float2* __restrict__ stats, HeadStrides heads)
+{
+    constexpr int NB = D / 16, PAD = D + 4, NT = tile_blocks<T>(), kStep = 16 * NT;
+    using KStage = TileStage<T, D, true>;
+    using VStage = TileStage<T, D, false>;
+    // Per wave: staged rows of k and v and the values of a step.  Once the columns of the run are done:
+    // the wave's partial result, in the first wave's part the rows' results outside their runs behind
+    // it, and the wave's staging for those.
+    constexpr int kPart = kTileRows * PAD, kStageFloats = 2 * KStage::kBytes / 4 + TileSquare<T>::kFloats;
+    static_assert(2 * kPart + 2 * kWave <= kStageFloats, "what comes later fits");
+    __shared__ __attribute__((aligned(16))) float shared[kWavesPerWg][kStageFloats];
+    __shared__ float part_m[kWavesPerWg + 1][kTileRows], part_l[kWavesPerWg + 1][kTileRows]; // (the last: outside the runs)
+    const int tile = xcd_logical_block(blockIdx.x, gridDim.x);
+    if (tile >= n_tiles) return;
+    const RowTile rt = tiles[tile];
+    if (rt.hi <= rt.lo) return; // not a tile: other kernels have its rows
+    q = of_head(q, heads.rows), k = of_head(k, heads.cols), v = of_head(v, heads.cols);
+    out = of_head(out, heads.rows), probs = of_head(probs, heads.nnz), stats = of_head(stats, heads.rows / D);
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
+    const int n = lane % 16, gq = lane / 16;
+    const TileLane me = tile_lane(tile * kTileRows + n, row_ptr, runs);
+    const int base = me.base();
+    const int steps = (rt.hi - rt.lo + kStep - 1) / kStep;
+    u32x4* lds_k = reinterpret_cast<u32x4*>(shared[wave]);
+    u32x4* lds_v = lds_k + KStage::kBytes / 16;
+    f32x4* lds_w = reinterpret_cast<f32x4*>(lds_v + VStage::kBytes / 16);
+    TileRow<T, D> q_row;
+    q_row.load(q + (size_t)me.row * D, gq);
+    // a score is unit * (value * <q, k>) in powers of two; a negative scale goes into q
+    const float unit = fabsf(scale) * kLog2e;
+    if (scale < 0.f) {
+#pragma unroll
+        for (int i = 0; i < TileRow<T, D>::kChunks; ++i) q_row.c[i] ^= sizeof(T) == 2 ? 0x80008000u : 0x80000000u;
+    }
+    TileSoftmax<T, D> sm;
+
+    // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 at a time:
+    // LPR lanes read a dense row, 16 bytes each, every lane group the rows of its own LPR nonzeros.
+    auto rows_outside = [&](bool whole) __attribute__((always_inline)) {
+        using S = SddmmShape<T, D>;
+        constexpr int VEC = S::kVec, LPR = S::kLpr, R = kTileRows / kWavesPerWg;
+        const int ls = lane % LPR, group = lane / LPR;
+        const unsigned lane_at = ls * 16u; // (an operand of a tile is at most 4 GB: 32-bit offsets)
+        const char* k_bytes = reinterpret_cast<const char*>(k);
+        const char* v_bytes = reinterpret_cast<const char*>(v);
+        float* left_o = shared[0] + kPart;
+        unsigned* my_at = reinterpret_cast<unsigned*>(shared[wave] + 2 * kPart);
+        float* my_p = shared[wave] + 2 * kPart + kWave;
+        struct Row {
+            int first, cnt, split, jump, c;
+            float w;
+        };
+        // a row's extent, and the columns and values of its first step
+        auto row_of = [&](int r) __attribute__((always_inline)) {
+            Row x;
+            x.first = __builtin_amdgcn_readlane(me.s, r);
+            x.jump = whole ? 0 : __builtin_amdgcn_readlane(me.len, r);
+            x.split = __builtin_amdgcn_readlane(me.pos, r);
+            x.cnt = __builtin_amdgcn_readlane(me.e, r) - x.first - x.jump;
+            const int at = min(lane, x.cnt - 1), idx = x.first + at + (at >= x.split ? x.jump : 0);
+            x.c = x.cnt > 0 ? col[idx] : 0;
+            x.w = x.cnt > 0 ? val[idx] : 0.f;
+            return x;
+        };
+        Row next = row_of(R * wave);
+#pragma unroll 1
+        for (int r = R * wave; r < R * wave + R; ++r) {
+            const Row me_row = next;
+            if (r + 1 < R * wave + R) next = row_of(r + 1); // (asked for while this row is worked on)
+            const int cnt = me_row.cnt;
+            typename DotVec<T>::Reg a[1][DotVec<T>::kRegs];
+            load_lhs_slice<T, D, 1, false>(q, tile * kTileRows + r, D, lane, a);
+            float m_run = -INFINITY, l_lane = 0.f, acc[VEC];
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) acc[x] = 0.f;
+#pragma unroll 1
+            for (int off = 0; off < cnt; off += kWave) {
+                const bool live = off + lane < cnt;
+                const int at = min(off + lane, cnt - 1); // (lanes past the end repeat the last nonzero with probability 0)
+                const int idx = me_row.first + at + (at >= me_row.split ? me_row.jump : 0);
+                const int c = off == 0 ? me_row.c : col[idx];
+                const float w = off == 0 ? me_row.w : val[idx];
+                my_at[lane] = (unsigned)c * (unsigned)(D * sizeof(T));
+                wave_lds_sync();
+                float d = 0.f;
+                const bool busy = off + group * LPR < cnt; // does this lane group have a nonzero?
+                // (the first rows of v are asked for together with those of k)
+                constexpr int kEarly = S::kQuads < 2 ? S::kQuads : 2;
+                u32x4 v_early[kEarly][4];
+                if (busy) {
+#pragma unroll
+                    for (int qd = 0; qd < S::kQuads; ++qd) {
+                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
+                        uint4 k_part[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) k_part[j] = *reinterpret_cast<const uint4*>(k_bytes + (o[j] + lane_at));
+                        if (qd < kEarly) {
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) v_early[qd][j] = *reinterpret_cast<const u32x4*>(v_bytes + (o[j] + lane_at));
+                        }
+                        float p[4];
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) p[j] = DotVec<T>::dot_raw(a[0], k_part[j], 0.f);
+                        const float sum = sddmm_quad_reduce<LPR>(p, ls);
+                        if ((ls >> 2) == qd) d = sum;
+                    }
+                }
+                const float sc = live ? scale * (w * d) : -INFINITY;
+                my_p[lane] = softmax_step<VEC>(sc, live, m_run, l_lane, acc);
+                if (KEEP != kKeepNothing && live) probs[idx] = sc;
+                wave_lds_sync();
+                if (busy) {
+#pragma unroll
+                    for (int qd = 0; qd < S::kQuads; ++qd) {
+                        const f32x4 p = *reinterpret_cast<const f32x4*>(my_p + group * LPR + 4 * qd);
+                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const u32x4 raw = qd < kEarly ? v_early[qd][j] : *reinterpret_cast<const u32x4*>(v_bytes + (o[j] + lane_at));
+                            float b[VEC];
+                            DenseVec<T>::unpack(make_uint4(raw[0], raw[1], raw[2], raw[3]), b);
+#pragma unroll
+                            for (int x = 0; x < VEC; ++x) acc[x] = fmaf(p[j], b[x], acc[x]);
+                        }
+                    }
+                }
+                wave_lds_sync();
+            }
+            const float l = butterfly_sum<1, kWave>(l_lane);
+            using Reduce = GroupReduce<LPR, VEC>;
+            Reduce::run(acc);
+            if (Reduce::writes(lane)) {
+#pragma unroll
+                for (int x = 0; x < Reduce::kLeft; ++x) left_o[r * PAD + ls * VEC + Reduce::value(lane) + x] = acc[x];
+            }
+            if (lane == 0) part_m[kWavesPerWg][r] = m_run, part_l[kWavesPerWg][r] = l;
+        }
+    };
+
+    // a step's columns of the run, on their way
+    KStage k_rows;
+    VStage v_rows;
+    f32x4 w_rows[NT];
+    // (the row and the four columns that this lane fetches values of: TileSquare)
+    const int f_a = __shfl(me.a, lane / 4, kWave), f_end = f_a + __shfl(me.len, lane / 4, kWave), f_base = __shfl(base, lane / 4, kWave);
+    auto inside = [&](int c0) { return c0 >= rt.core_lo && c0 + kStep <= rt.core_hi; }; // does every row hold every one of them?
+    auto fetch = [&](int c0) __attribute__((always_inline)) {
+        const bool in = inside(c0);
+        k_rows.load(k + (size_t)c0 * D, rt.hi - 1 - c0, in, lane); // (columns past the range repeat its last)
+        v_rows.load(v + (size_t)c0 * D, rt.hi - 1 - c0, in, lane);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const int c = c0 + 16 * t + lane % 4 * 4;
+            if (in) {
+                w_rows[t] = *reinterpret_cast<const f32x4_u*>(val + f_base + c);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w_rows[t][i] = c + i >= f_a && c + i < f_end ? val[f_base + c + i] : 0.f;
+            }
+        }
+    };
+    auto run_columns = [&]() __attribute__((always_inline)) {
+        if (wave < steps) fetch(rt.lo + wave * kStep);
+        for (int it = wave; it < steps; it += kWavesPerWg) {
+            const int c0 = rt.lo + it * kStep;
+            const bool in = inside(c0);
+            k_rows.store(lds_k, lane);
+            v_rows.store(lds_v, lane);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) TileSquare<T>::in_order(lds_w, t, lane) = w_rows[t];
+            wave_lds_sync();
+            if (it + kWavesPerWg < steps) fetch(c0 + kWavesPerWg * kStep); // (in flight during this step)
+            float sc[4 * NT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                TileRow<T, D> k_row;
+                KStage::read(lds_k, t, lane, k_row);
+                const f32x4 dot = mma_rows<T, D>(k_row, q_row), w = TileSquare<T>::as_scores(lds_w, t, lane);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[4 * t + i] = w[i] * dot[i];
+            }
+            if (KEEP != kKeepNothing) { // the scores leave in the order of the values
+#pragma unroll
+                for (int t = 0; t < NT; ++t) TileSquare<T>::as_scores(lds_w, t, lane) = f32x4{sc[4 * t], sc[4 * t + 1], sc[4 * t + 2], sc[4 * t + 3]} * fabsf(scale);
+                wave_lds_sync();
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const f32x4 out4 = TileSquare<T>::in_order(lds_w, t, lane);
+                    const int c = c0 + 16 * t + lane % 4 * 4;
+                    if (in) {
+                        *reinterpret_cast<f32x4_u*>(probs + f_base + c) = out4;
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if (c + i >= f_a && c + i < f_end) probs[f_base + c + i] = out4[i];
+                    }
+                }
+            }
+            if (!in) {
+#pragma unroll
+                for (int j = 0; j < 4 * NT; ++j) {
+                    const int c = c0 + 16 * (j / 4) + 4 * gq + j % 4;
+                    sc[j] = c >= me.a && c < me.a + me.len ? sc[j] : -INFINITY;
+                }
+            }
+            TileWeights<T> weights;
+            sm.step(sc, unit, weights);
+            TileCols<T, D> v_cols;
+#pragma unroll
+            for (int j = 0; j < 4 * NT; ++j) v_cols.load(j, VStage::across(lds_v, 16 * (j / 4) + 4 * gq + j % 4, n));
+            v_cols.accumulate(weights, sm.acc);
+            wave_lds_sync();
+        }
+    };
+
+    run_columns();
+    const bool again = __syncthreads_or(!all_finite<NB>(sm.acc));
+    if (again) sm = TileSoftmax<T, D>();
+    rows_outside(again);
+
+    // the partial results, each relative to its own maximum
+    float* part = shared[wave];
+    if (gq == 0) part_m[wave][n] = sm.m * fabsf(scale), part_l[wave][n] = sm.l[0];
+#pragma unroll
+    for (int e = 0; e < D / 4; ++e) part[n * PAD + (D / 4) * gq + e] = sm.acc[e % NB][e / NB];
+    __syncthreads();
+    const int r = threadIdx.x / 16, e0 = threadIdx.x % 16 * NB, row = tile * kTileRows + r;
+    float top = part_m[0][r];
+#pragma unroll
+    for (int w = 1; w <= kWavesPerWg; ++w) top = fmaxf(top, part_m[w][r]);
+    const float top_safe = top == -INFINITY ? 0.f : top;
+    float f = __builtin_amdgcn_exp2f((part_m[kWavesPerWg][r] - top_safe) * kLog2e);
+    float total = part_l[kWavesPerWg][r] * f, o[NB];
+#pragma unroll
+    for (int x = 0; x < NB; ++x) o[x] = shared[0][kPart + r * PAD + e0 + x] * f;
+#pragma unroll
+    for (int w = 0; w < kWavesPerWg; ++w) {
+        f = __builtin_amdgcn_exp2f((part_m[w][r] - top_safe) * kLog2e - TileWeights<T>::kShift);
+        total = fmaf(part_l[w][r], f, total);
+#pragma unroll
+        for (int x = 0; x < NB; ++x) o[x] = fmaf(shared[w][r * PAD + e0 + x], f, o[x]);
+    }
+    const float inv = 1.0f / total;
+#pragma unroll
+    for (int x = 0; x < NB; x += 2)
+        *reinterpret_cast<float2*>(out + (size_t)row * D + e0 + x) = make_float2(o[x] * inv, o[x + 1] * inv);
+    if (KEEP == kKeepScores && threadIdx.x % 16 == 0) stats[row] = make_float2(top_safe, inv);
+    if (KEEP == kKeepProbs) {
+        // what the waves wrote are scores: normalised in place
+        __threadfence_block();
+        __syncthreads();
+        const int s = row_ptr[row], e = row_ptr[row + 1];
+        for (int slot = s + threadIdx.x % 16; slot < e; slot += 16) probs[slot] = __expf(probs[slot] - top_safe) * inv;
+    }
+}
+
+template <typename T, int D>
+hipError_t launch_tiles(int nheads, int M, int N, int nnz, const int* row_ptr, const int* col, const float* val, const T* q, const T* k,
+                        const T* v, float scale, float* out, float* probs, float2* stats, const int* plan, hipStream_t stream)
+{
+    const int n_tiles = row_tiles(M);
+    HeadStrides heads;
+    heads.rows = (size_t)M * D, heads.cols = (size_t)N * D, heads.nnz = (size_t)nnz;
+    const dim3 grid((n_tiles + kXcds - 1) / kXcds * kXcds, nheads);
+    auto kernel = probs == nullptr ? attention_tile_kernel<T, D, kKeepNothing>
+                  : stats != nullptr ? attention_tile_kernel<T, D, kKeepScores> : attention_tile_kernel<T, D, kKeepProbs>;
+    kernel<<<grid, kWgThreads, 0, stream>>>(n_tiles, group_plan_tiles(plan, M), group_plan_runs(plan, M), row_ptr, col, val, q, k, v,
+                                            scale, out, probs, stats, heads);
+    return hipGetLastError();
+}
+
+} // namespace
+
+// The tiles of a group plan (plan.groups, with plan.group_counts[3] > 0 of them); arguments as
+// attention_launch.  One head's k or v must not exceed 4 GB (attention_tiles_fit).
+template <typename T>
+hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
+                                  const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,
+                                  const int* plan, hipStream_t stream)
+{
+    float2* stats = reinterpret_cast<float2*>(row_stats);
+    switch (d) {
+    case 32: return launch_tiles<T, 32>(nheads, M, N, nnz, row_ptr, col, val, q, k, v, scale, out, probs, stats, plan, stream);
+    case 64: return launch_tiles<T, 64>(nheads, M, N, nnz, row_ptr, col, val, q, k, v, scale, out, probs, stats, plan, stream);
+    case 128: return launch_tiles<T, 128>(nheads, M, N, nnz, row_ptr, col, val, q, k, v, scale, out, probs, stats, plan, stream);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+template hipError_t attention_tiles_launch<float>(int, int, int, int, int, const int*, const int*, const float*, const float*, const float*,
+                                                  const float*, float, float*, float*, float*, const int*, hipStream_t);
+template hipError_t attention_tiles_launch<__half>(int, int, int, int, int, const int*, const int*, const float*, const __half*,
+                                                   const __half*, const __half*, float, float*, float*, float*, const int*, hipStream_t);
+
+} // namespace rode

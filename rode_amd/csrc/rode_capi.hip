@@ -197,6 +197,7 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
         // kernels do not know which rows the group kernels have taken)
         if (!p->group_counts || !aligned16(p->groups) || window || p->hub) return false;
         if (p->group_counts[0] < 0 || p->group_counts[1] < 0 || p->group_counts[1] > p->group_counts[0]) return false;
+        if (p->group_counts[3] < 0 || p->group_counts[3] * (rode::kTileRows / rode::kGroupRows) > p->group_counts[1]) return false;
         plan.groups = static_cast<const int*>(p->groups);
         plan.group_counts = p->group_counts;
     }

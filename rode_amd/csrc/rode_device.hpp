@@ -34,23 +34,32 @@ __device__ __forceinline__ float lane_xor2(float v)
 {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4E /*[2,3,0,1]*/, 0xF, 0xF, true));
 }
-// xor 4 / 8 / 16: ds_swizzle in bit-mask mode (and=0x1f, or=0, xor=mask); no LDS memory is touched.
+// xor 4: reversed inside quads, then the eight lanes of a half row mirrored (7 - (i ^ 3) == i ^ 4);
+// xor 8: a row of 16 lanes rotated by eight.  Both stay on the vector ALU; through the LDS unit
+// (ds_swizzle) every exchange costs a round trip of 60 clocks and more.
 __device__ __forceinline__ float lane_xor4(float v)
 {
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (4 << 10) | 0x1F));
+    const int r = __builtin_amdgcn_mov_dpp(__float_as_int(v), 0x1B /*[3,2,1,0]*/, 0xF, 0xF, true);
+    return __int_as_float(__builtin_amdgcn_mov_dpp(r, 0x141 /*row_half_mirror*/, 0xF, 0xF, true));
 }
 __device__ __forceinline__ float lane_xor8(float v)
 {
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (8 << 10) | 0x1F));
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128 /*row_ror:8*/, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float lane_xor16(float v)
+// The two values that lanes 16 (32) apart have, in either order: one exchange instruction of
+// gfx950 swaps the odd rows (the upper half) of one register with the even rows (the lower half) of the other.
+struct LanePair {
+    float a, b;
+};
+__device__ __forceinline__ LanePair lane_pair16(float v)
 {
-    return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), (16 << 10) | 0x1F));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return LanePair{__uint_as_float(r[0]), __uint_as_float(r[1])};
 }
-// xor 32: swap the two 32-lane halves of the wave.
-__device__ __forceinline__ float lane_xor32(float v)
+__device__ __forceinline__ LanePair lane_pair32(float v)
 {
-    return __shfl_xor(v, 32, kWave);
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return LanePair{__uint_as_float(r[0]), __uint_as_float(r[1])};
 }
 
 // Sum over the lanes l ^ m for every power of two m with LO <= m < HI.
@@ -62,8 +71,31 @@ __device__ __forceinline__ float butterfly_sum(float v)
     if (LO <= 2 && 2 < HI) v += lane_xor2(v);
     if (LO <= 4 && 4 < HI) v += lane_xor4(v);
     if (LO <= 8 && 8 < HI) v += lane_xor8(v);
-    if (LO <= 16 && 16 < HI) v += lane_xor16(v);
-    if (LO <= 32 && 32 < HI) v += lane_xor32(v);
+    if (LO <= 16 && 16 < HI) {
+        const LanePair p = lane_pair16(v);
+        v = p.a + p.b;
+    }
+    if (LO <= 32 && 32 < HI) {
+        const LanePair p = lane_pair32(v);
+        v = p.a + p.b;
+    }
+    return v;
+}
+template <int LO, int HI>
+__device__ __forceinline__ float butterfly_max(float v)
+{
+    if (LO <= 1 && 1 < HI) v = fmaxf(v, lane_xor1(v));
+    if (LO <= 2 && 2 < HI) v = fmaxf(v, lane_xor2(v));
+    if (LO <= 4 && 4 < HI) v = fmaxf(v, lane_xor4(v));
+    if (LO <= 8 && 8 < HI) v = fmaxf(v, lane_xor8(v));
+    if (LO <= 16 && 16 < HI) {
+        const LanePair p = lane_pair16(v);
+        v = fmaxf(p.a, p.b);
+    }
+    if (LO <= 32 && 32 < HI) {
+        const LanePair p = lane_pair32(v);
+        v = fmaxf(p.a, p.b);
+    }
     return v;
 }
 

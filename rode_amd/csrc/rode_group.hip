@@ -15,7 +15,9 @@
 //                       they cover between them; the group is kept if the common part has
 //                       at least kGroupMinRun columns and holds at least three quarters of
 //                       the group's nonzeros, and the runs start and end within 255 columns
-//                       of each other.
+//                       of each other;
+//   group_tiles_kernel  per four groups: whether their 16 rows make a tile for the attention
+//                       kernels on the matrix cores (rode_tile.hpp).
 #include "rode_items.hpp"
 #include "rode_internal.hpp"
 
@@ -113,13 +115,42 @@ group_desc_kernel(int groups, const int* __restrict__ row_ptr, const int* __rest
     }
 }
 
+// A tile per four groups: kept when all four are and the columns that the 16 runs cover between
+// them are at most half as many again as a run has on average (the tile kernels work on all of
+// the 16 x (hi - lo) rectangle).
+__global__ void __launch_bounds__(kWgThreads)
+group_tiles_kernel(int tiles, const RowGroup* __restrict__ groups, const int* __restrict__ runs, RowTile* __restrict__ out,
+                   int* __restrict__ plan)
+{
+    const int t = blockIdx.x * kWgThreads + threadIdx.x;
+    if (t >= tiles) return;
+    bool keep = true;
+#pragma unroll
+    for (int g = 0; g < kTileRows / kGroupRows; ++g) keep = keep && groups[t * (kTileRows / kGroupRows) + g].len > 0;
+    RowTile d{0, 0, 0, 0};
+    if (keep) {
+        d = RowTile{0x7fffffff, 0, 0, 0x7fffffff};
+        long long held = 0;
+        for (int r = 0; r < kTileRows; ++r) {
+            const int row = t * kTileRows + r, a = runs[3 * row], len = runs[3 * row + 1];
+            d.lo = min(d.lo, a), d.hi = max(d.hi, a + len);
+            d.core_lo = max(d.core_lo, a), d.core_hi = min(d.core_hi, a + len);
+            held += len;
+        }
+        keep = d.core_hi > d.core_lo && 2ll * kTileRows * (d.hi - d.lo) <= 3 * held;
+    }
+    if (!keep) d = RowTile{0, 0, 0, 0};
+    out[t] = d;
+    if (keep) atomicAdd(plan + 3, 1);
+}
+
 __global__ void group_header_kernel(int M, int groups, int* __restrict__ plan)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         plan[0] = groups;
         plan[1] = 0;
         plan[2] = M; // rows outside the groups with a run: counted down as groups are kept
-        plan[3] = 0;
+        plan[3] = 0; // tiles: counted up
     }
 }
 
@@ -130,9 +161,14 @@ hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* pla
     const int groups = row_groups(M);
     group_header_kernel<<<1, kWave, 0, stream>>>(M, groups, plan);
     if (groups > 0) {
-        int* runs = plan + kGroupHeaderInts + (size_t)groups * (sizeof(RowGroup) / sizeof(int)); // scratch behind the table
+        int* runs = plan + group_runs_at(M);
         group_runs_kernel<<<(M + kWavesPerWg - 1) / kWavesPerWg, kWgThreads, 0, stream>>>(M, row_ptr, col, runs);
         group_desc_kernel<<<(groups + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(groups, row_ptr, runs, plan);
+        const int tiles = row_tiles(M);
+        if (tiles > 0)
+            group_tiles_kernel<<<(tiles + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(
+                tiles, reinterpret_cast<const RowGroup*>(plan + kGroupHeaderInts), runs,
+                reinterpret_cast<RowTile*>(plan + group_tiles_at(M)), plan);
     }
     return hipGetLastError();
 }

@@ -56,6 +56,13 @@ hipError_t attention_launch(int nheads, int M, int N, int nnz, int d, const int*
                             const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,
                             PlanRef plan, hipStream_t stream);
 
+constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (size_t)N * row_bytes < (1ull << 32); }
+// (rode_attention_tile.hip) the rows of a group plan's tiles, the same arguments; plan: the group plan
+template <typename T>
+hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
+                                  const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,
+                                  const int* plan, hipStream_t stream);
+
 // Gradient of the attention kernel (rode_attention_backward.hip): the row pass over the
 // pattern, then the column pass over the transposed pattern (plan: only a group plan is used,
 // of the pattern the pass walks).  pz: nheads x 2 * nnz floats, written by the first in the

@@ -43,11 +43,14 @@ __host__ __device__ inline RowGroup shared_run(RowGroup d)
     d.heads = d.tails = 0u;
     return d;
 }
+struct RowTile; // (below: the group plan)
 struct RowOwners {
     int hub_min_len = 0;              // > 0: rows of that aligned length or more belong to the hub kernels
     const RowGroup* groups = nullptr; // the groups of a group plan, or null
     int n_groups = 0;
     bool overwrite = false;           // SpMM: a row with a single work item is stored, not added to C
+    const RowTile* tiles = nullptr;   // attention: the tiles of the group plan, or null
+    int n_tiles = 0;
 };
 __device__ __forceinline__ bool owned_elsewhere(const RowOwners& o, int row, int aligned_len)
 {
@@ -407,8 +410,8 @@ __device__ __forceinline__ WindowDesc plan_residue_desc(const int* __restrict__ 
 // ---- group plan -----------------------------------------------------------------
 // Groups of kGroupRows adjacent rows that share a long run of consecutive columns (see
 // rode_group.hip).  Layout, ints: header [0] groups (= rows / kGroupRows, whole groups
-// only)  [1] groups with a run  [2] rows outside those groups  [3] zero; then one RowGroup per group; then three
-// ints per row of scratch for the plan's own kernels.
+// only)  [1] groups with a run  [2] rows outside those groups  [3] tiles of 16 rows; then one RowGroup per
+// group; then the rows' runs and the tiles (below).
 constexpr int kGroupHeaderInts = 4;
 // SpMM / SDDMM: from this many groups with a run on, a group is one wave's work, below it a
 // workgroup's (measured on the attention-mask benchmark cut down to 128 .. 4096 groups: a wave
@@ -428,10 +431,23 @@ constexpr int attention_groups_min()
 constexpr int kAttentionColsGroupsMin = 1024;
 static_assert(sizeof(RowGroup) == 32 && kGroupRows == kWavesPerWg, "one wave per row of a group");
 __host__ __device__ inline int row_groups(int M) { return M / kGroupRows; }
-__host__ __device__ inline size_t group_plan_ints(int M)
-{
-    return kGroupHeaderInts + (size_t)row_groups(M) * (sizeof(RowGroup) / sizeof(int)) + 3 * (size_t)M;
-}
+
+// A tile of a group plan: four adjacent groups, all kept, whose rows' runs overlap for the most
+// part.  The runs of its 16 rows cover the columns [lo, hi) between them, all of them hold
+// [core_lo, core_hi); lo == hi: not a tile.  (Whole tiles of 16 rows from row 0 on only.)
+constexpr int kTileRows = 16;
+struct RowTile {
+    int lo, hi, core_lo, core_hi;
+};
+__host__ __device__ inline int row_tiles(int M) { return M / kTileRows; }
+
+// Behind the groups: per row its longest run (first column, length, position in the row), then,
+// 16-byte aligned, a RowTile per 16 rows.
+__host__ __device__ inline size_t group_runs_at(int M) { return kGroupHeaderInts + (size_t)row_groups(M) * (sizeof(RowGroup) / sizeof(int)); }
+__host__ __device__ inline size_t group_tiles_at(int M) { return (group_runs_at(M) + 3 * (size_t)M + 3) & ~(size_t)3; }
+__host__ __device__ inline size_t group_plan_ints(int M) { return group_tiles_at(M) + (size_t)row_tiles(M) * (sizeof(RowTile) / sizeof(int)); }
+inline const int* group_plan_runs(const int* plan, int M) { return plan + group_runs_at(M); }
+inline const RowTile* group_plan_tiles(const int* plan, int M) { return reinterpret_cast<const RowTile*>(plan + group_tiles_at(M)); }
 
 // ---- hub plan -------------------------------------------------------------------
 // Rows with very many nonzeros (hubs of a power-law graph) reference dense rows all over
@@ -475,6 +491,12 @@ __host__ __device__ inline int hub_merge(int width)
     return g < 1 ? 1 : (g > 64 ? 64 : g);
 }
 __host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs + merge - 1) / merge; }
+
+// Is this row in a tile that the tile kernels have (owners.tiles)?
+__device__ __forceinline__ bool in_tile(const RowOwners& o, int row)
+{
+    return o.tiles != nullptr && row / kTileRows < o.n_tiles && o.tiles[row / kTileRows].hi > o.tiles[row / kTileRows].lo;
+}
 
 struct HubPlan {
     int n_hub, slabs, min_len;

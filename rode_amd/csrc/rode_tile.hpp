@@ -1,0 +1,323 @@
+// Tiles of 16 rows on the matrix cores: what the attention kernels share (forward:
+// rode_attention_tile.hip).  A tile is four adjacent groups of a group plan whose runs of
+// consecutive columns overlap for the most part (RowTile, rode_items.hpp): along those columns
+// scores and weighted sums are dense 16 x 16 products, and every dense row loaded serves 16 rows.
+//
+// Lane layouts (n = lane % 16, gq = lane / 16; MFMA 16x16: operand A has m = lane % 16, operand B
+// has n = lane % 16, the result has column n = lane % 16 and rows 4 gq .. 4 gq + 3 in its four
+// registers; which k a lane's elements stand for may be chosen freely, the same for A and B):
+//   * a dense row as operand along its elements ("chunks"): 16 bytes at every 64 ch + 16 gq.
+//     Adjacent lanes then want different rows, which the vector memory pipe serves one lane per clock
+//     (64 clocks a load; 16 when every four adjacent lanes ask for 64 consecutive bytes): 32 rows are
+//     loaded in order and re-arranged in LDS (TileStage);
+//   * scores come out transposed, S^T = K Q^T: lane (n, gq) has row n of the tile and the four
+//     columns 4 gq + i of a 16-column block.  A row's statistics are then one number per lane, its
+//     values and scores are 16 consecutive bytes in memory, and the probabilities are operand B of
+//     the next product as they are (k slot (gq, t, i) stands for column 16 t + 4 gq + i);
+//   * the weighted sum too: O^T = V^T P^T.  Operand A has a lane per 16th of the elements: lane m
+//     loads the D / 16 consecutive elements from (D / 16) m of each of its eight columns' rows
+//     (16 lanes, a whole row), product nb takes element nb of each.  Lane (n, gq) ends up with the
+//     D / 4 consecutive elements from (D / 4) gq of row n: element e is acc[e % (D / 16)][e / (D / 16)].
+#pragma once
+#include "rode_items.hpp"
+#include "rode_device.hpp"
+
+namespace rode {
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4))); // four consecutive floats at any 4-byte address
+
+// 16-column blocks that a wave takes at a time: what one weighted-sum product of 16-bit operands
+// contracts over (32 columns); 32-bit operands take 16 (the same bytes in LDS and registers).
+template <typename T>
+constexpr int tile_blocks()
+{
+    return sizeof(T) == 2 ? 2 : 1;
+}
+
+// The sums over the lane groups (LPR lanes each) of N values per lane, shared out: a lane keeps kLeft of
+// the totals, from number value() on (halving what a lane still has to add at every exchange costs a
+// third of a butterfly per value).
+template <int LPR, int N>
+struct GroupReduce {
+    static constexpr int kGroups = kWave / LPR;
+    static constexpr int kLeft = N / (kGroups < N ? kGroups : N); // totals per lane
+    // (v: the values; in the end the totals in v[0 .. kLeft))
+    static __device__ __forceinline__ void run(float (&v)[N])
+    {
+        if (kGroups >= 2) { // lanes 32 apart
+#pragma unroll
+            for (int j = 0; j < N / 2; ++j) {
+                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[j]), __float_as_uint(v[N / 2 + j]), false, false);
+                v[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            }
+        }
+        if (kGroups >= 4) { // 16 apart
+            constexpr int H = N / 4 > 0 ? N / 4 : 1;
+#pragma unroll
+            for (int j = 0; j < H; ++j) {
+                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[H + j]), false, false);
+                v[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+            }
+        }
+        if (kGroups >= 8) { // 8 apart
+            if constexpr (N >= 8) {
+                const bool upper = __lane_id() & 8;
+                v[0] = (upper ? v[1] : v[0]) + lane_xor8(upper ? v[0] : v[1]);
+            } else {
+                v[0] += lane_xor8(v[0]);
+            }
+        }
+        if (kGroups >= 16) v[0] += lane_xor4(v[0]);
+    }
+    static __device__ __forceinline__ int value(int lane)
+    {
+        int at = 0;
+        if (kGroups >= 2) at += (lane >> 5 & 1) * (N / 2);
+        if (kGroups >= 4) at += (lane >> 4 & 1) * (N / 4);
+        if (kGroups >= 8 && N >= 8) at += (lane >> 3 & 1) * (N / 8);
+        return at;
+    }
+    // does this lane write its totals? (where there are more groups than values several have the same)
+    static __device__ __forceinline__ bool writes(int lane)
+    {
+        if (kGroups >= 16) return N >= 8 ? (lane & 4) == 0 : (lane & 12) == 0;
+        return !(kGroups >= 8 && N < 8) || (lane & 8) == 0;
+    }
+};
+
+constexpr float kLog2e = 1.44269504088896340736f;
+
+// Sum and maximum over the four lanes of a row (lanes 16 and 32 apart).
+__device__ __forceinline__ float quad_sum(float v) { return butterfly_sum<16, kWave>(v); }
+__device__ __forceinline__ float quad_max(float v) { return butterfly_max<16, kWave>(v); }
+
+// ---- chunks: a dense row along its elements ------------------------------------------------
+template <typename T, int D>
+struct TileRow {
+    static constexpr int kChunks = D * (int)sizeof(T) / 64;
+    u32x4 c[kChunks];
+    __device__ __forceinline__ void load(const T* row, int gq)
+    {
+#pragma unroll
+        for (int i = 0; i < kChunks; ++i) c[i] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(row) + 64 * i + 16 * gq);
+    }
+};
+
+__device__ __forceinline__ f32x4 mma_chunk(const __half*, const u32x4& a, const u32x4& b, f32x4 acc)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mma_chunk(const float*, const u32x4& a, const u32x4& b, f32x4 acc)
+{
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
+}
+// rows of a (16 of them, m = lane % 16) times rows of b (n = lane % 16)
+template <typename T, int D>
+__device__ __forceinline__ f32x4 mma_rows(const TileRow<T, D>& a, const TileRow<T, D>& b)
+{
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < TileRow<T, D>::kChunks; ++i) acc = mma_chunk(static_cast<const T*>(nullptr), a.c[i], b.c[i], acc);
+    return acc;
+}
+// The dense rows of a step on their way through LDS to operand A: loaded in order (every load 1024 consecutive
+// bytes), stored, and read back along or across their elements.  Where 16 bytes are put spreads the
+// 16 lanes that LDS serves together (lanes 0-3, 12-15, 20-27 and their like) over all of its banks:
+//   ALONG: chunk c of row r at position c ^ f(r) of the row (16 rows are read at one c);
+//   else (across, TileCols): the rows of lanes 16 apart, four apart in r, in different parts of 256 bytes.
+template <typename T, int D, bool ALONG>
+struct TileStage {
+    static constexpr int kPerRow = D * (int)sizeof(T) / 16; // 16-byte chunks of a row
+    static constexpr int kLoads = 16 * tile_blocks<T>() * kPerRow / kWave;
+    static constexpr int kBytes = 16 * tile_blocks<T>() * kPerRow * 16;
+    u32x4 x[kLoads];
+    static __device__ __forceinline__ int place(int row, int c)
+    {
+        if constexpr (ALONG) {
+            const int f = kPerRow == 4 ? (-(row >> 2)) & 3 : row & (kPerRow < 16 ? kPerRow - 1 : 15);
+            return row * kPerRow + (c ^ f);
+        } else {
+            constexpr int kParts = kPerRow < 16 ? 16 / kPerRow : 1; // rows in 256 bytes
+            return (row ^ ((row >> 2) & (kParts - 1))) * kPerRow + c;
+        }
+    }
+    // the rows from `first` on; rows past `last` (counted from there) repeat it
+    __device__ __forceinline__ void load(const T* first, int last, bool inside, int lane)
+    {
+        if (inside) {
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) x[i] = reinterpret_cast<const u32x4*>(first)[i * kWave + lane];
+        } else {
+#pragma unroll
+            for (int i = 0; i < kLoads; ++i) {
+                const int at = i * kWave + lane;
+                x[i] = reinterpret_cast<const u32x4*>(first)[min(at / kPerRow, last) * kPerRow + at % kPerRow];
+            }
+        }
+    }
+    __device__ __forceinline__ void store(u32x4* lds, int lane) const
+    {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) lds[place((i * kWave + lane) / kPerRow, (i * kWave + lane) % kPerRow)] = x[i];
+    }
+    // rows 16 t .. 16 t + 15 as operand A along their elements
+    static __device__ __forceinline__ void read(const u32x4* lds, int t, int lane, TileRow<T, D>& row)
+    {
+#pragma unroll
+        for (int i = 0; i < TileRow<T, D>::kChunks; ++i) row.c[i] = lds[place(16 * t + lane % 16, 4 * i + lane / 16)];
+    }
+    // this lane's D / 16 elements (from (D / 16) n) of row r
+    static __device__ __forceinline__ const T* across(const u32x4* lds, int r, int n)
+    {
+        constexpr int kElems = 16 / (int)sizeof(T), NB = D / 16;
+        return reinterpret_cast<const T*>(lds + place(r, NB * n / kElems)) + NB * n % kElems;
+    }
+};
+
+// One number per (row of the tile, column) of a step, between the layout that memory wants
+// (lane 4 r + part: row r, 4 consecutive columns from 4 part on, in each 16-column block) and
+// the scores' (lane (n, gq)), through LDS.
+template <typename T>
+struct TileSquare {
+    static constexpr int kFloats = tile_blocks<T>() * kTileRows * 16;
+    static __device__ __forceinline__ int place(int t, int row, int part) { return (t * kTileRows + row) * 4 + (part ^ ((-(row >> 2)) & 3)); }
+    static __device__ __forceinline__ f32x4& in_order(f32x4* lds, int t, int lane) { return lds[place(t, lane / 4, lane % 4)]; }
+    static __device__ __forceinline__ f32x4& as_scores(f32x4* lds, int t, int lane) { return lds[place(t, lane % 16, lane / 16)]; }
+};
+
+// ---- weights: operand B of the weighted sums -------------------------------------------------
+// fp16 dense operands: a weight is taken as the sum of two halves (22 bits and a sign), so that the
+// products carry what a 32-bit weight would; weights are kept below 2^15 by a power of two.
+template <typename T>
+struct TileWeights;
+template <>
+struct TileWeights<__half> {
+    static constexpr float kShift = 12.f; // probabilities are taken times 2^12
+    f16x8 hi, lo;
+    __device__ __forceinline__ void set(const float (&p)[8])
+    {
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            const f16x2 h = __builtin_convertvector(f32x2{p[j], p[j + 1]}, f16x2);
+            const f16x2 l = __builtin_convertvector(f32x2{fmaf((float)h[0], -1.f, p[j]), fmaf((float)h[1], -1.f, p[j + 1])}, f16x2);
+            hi[j] = h[0], hi[j + 1] = h[1], lo[j] = l[0], lo[j + 1] = l[1];
+        }
+    }
+    // acc += the sums of the weights per row, in each of its four elements
+    __device__ __forceinline__ void add_sums(f32x4& acc) const
+    {
+        const f16x8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, hi, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, lo, acc, 0, 0, 0);
+    }
+};
+template <>
+struct TileWeights<float> {
+    static constexpr float kShift = 0.f;
+    float p[4];
+    __device__ __forceinline__ void set(const float (&w)[4])
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j] = w[j];
+    }
+    __device__ __forceinline__ void add_sums(f32x4& acc) const
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, p[j], acc, 0, 0, 0);
+    }
+};
+
+// ---- columns: a lane's 4 or 8 dense rows across their elements, operand A of the weighted sums ----
+template <typename T, int D>
+struct TileCols;
+template <int D>
+struct TileCols<__half, D> {
+    static constexpr int kBlocks = D / 16, kWords = D / 32;
+    uint32_t w[8][kWords];
+    __device__ __forceinline__ void load(int j, const __half* at)
+    {
+        if constexpr (kWords == 1) {
+            w[j][0] = *reinterpret_cast<const uint32_t*>(at);
+        } else if constexpr (kWords == 2) {
+            const uint2 x = *reinterpret_cast<const uint2*>(at);
+            w[j][0] = x.x, w[j][1] = x.y;
+        } else {
+            const uint4 x = *reinterpret_cast<const uint4*>(at);
+            w[j][0] = x.x, w[j][1] = x.y, w[j][2] = x.z, w[j][3] = x.w;
+        }
+    }
+    __device__ __forceinline__ void accumulate(const TileWeights<__half>& p, f32x4 (&acc)[kBlocks]) const
+    {
+#pragma unroll
+        for (int nb = 0; nb < kBlocks; ++nb) {
+            const uint32_t select = nb % 2 ? 0x07060302u : 0x05040100u; // the upper / lower halves of two rows
+            const uint4 a = make_uint4(__builtin_amdgcn_perm(w[1][nb / 2], w[0][nb / 2], select),
+                                       __builtin_amdgcn_perm(w[3][nb / 2], w[2][nb / 2], select),
+                                       __builtin_amdgcn_perm(w[5][nb / 2], w[4][nb / 2], select),
+                                       __builtin_amdgcn_perm(w[7][nb / 2], w[6][nb / 2], select));
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.hi, acc[nb], 0, 0, 0);
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.lo, acc[nb], 0, 0, 0);
+        }
+    }
+};
+template <int D>
+struct TileCols<float, D> {
+    static constexpr int kBlocks = D / 16;
+    float x[4][kBlocks];
+    __device__ __forceinline__ void load(int j, const float* at)
+    {
+        if constexpr (kBlocks == 2) {
+            const float2 v = *reinterpret_cast<const float2*>(at);
+            x[j][0] = v.x, x[j][1] = v.y;
+        } else {
+#pragma unroll
+            for (int b = 0; b < kBlocks; b += 4) {
+                const float4 v = *reinterpret_cast<const float4*>(at + b);
+                x[j][b] = v.x, x[j][b + 1] = v.y, x[j][b + 2] = v.z, x[j][b + 3] = v.w;
+            }
+        }
+    }
+    __device__ __forceinline__ void accumulate(const TileWeights<float>& p, f32x4 (&acc)[kBlocks]) const
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int nb = 0; nb < kBlocks; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j][nb], p.p[j], acc[nb], 0, 0, 0);
+    }
+};
+
+template <int NB>
+__device__ __forceinline__ bool all_finite(const f32x4 (&acc)[NB])
+{
+    float s = 0.f; // (a sum of x * 0 is zero, or NaN as soon as one x is not finite)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s = fmaf(acc[b][i], 0.f, s);
+    return s == 0.f;
+}
+
+// One lane's row of a tile: its nonzeros, and the run of consecutive columns among them.
+struct TileLane {
+    int row, s, e;    // slots [s, e)
+    int a, len, pos;  // columns [a, a + len) from slot s + pos on
+    __device__ __forceinline__ int base() const { return s + pos - a; } // slot of column c of the run: base() + c
+};
+__device__ __forceinline__ TileLane tile_lane(int row, const int* __restrict__ row_ptr, const int* __restrict__ runs)
+{
+    TileLane t;
+    t.row = row;
+    t.s = row_ptr[row], t.e = row_ptr[row + 1];
+    t.a = runs[3 * row], t.len = runs[3 * row + 1], t.pos = runs[3 * row + 2];
+    return t;
+}
+
+} // namespace rode

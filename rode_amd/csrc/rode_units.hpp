@@ -1,5 +1,6 @@
 // Inner loops shared by the SDDMM, SpMM and fused attention kernels: the dot products of
-// one 32-slot unit (SDDMM) and the gather-accumulate over staged slot quads (SpMM).
+// one 32-slot unit (SDDMM), the gather-accumulate over staged slot quads (SpMM) and a step of the
+// running softmax (attention).
 #pragma once
 #include "rode_device.hpp"
 
@@ -33,6 +34,20 @@ __device__ __forceinline__ float lane_dot(const typename DotVec<T>::Reg (&a)[NS]
     return d;
 }
 
+// The sums over the LPR lanes of a dense row of four slots' partial products: a
+// transpose-reduce, after which lane (ls & 3) == j holds slot j of the quad.
+template <int LPR>
+__device__ __forceinline__ float sddmm_quad_reduce(const float (&p)[4], int ls)
+{
+    const bool hi2 = ls & 2, hi1 = ls & 1;
+    const float k0 = hi2 ? p[2] : p[0], s0 = hi2 ? p[0] : p[2];
+    const float k1 = hi2 ? p[3] : p[1], s1 = hi2 ? p[1] : p[3];
+    const float q0 = k0 + lane_xor2(s0);
+    const float q1 = k1 + lane_xor2(s1);
+    const float r = (hi1 ? q1 : q0) + lane_xor1(hi1 ? q0 : q1);
+    return butterfly_sum<4, LPR>(r);
+}
+
 // Dot products of the 32-slot units of one step, the slots' columns already in lds_cols
 // (lds_cols[e] = column of lane e's slot).  Returns the dot product for this lane's slot.
 template <typename T, int KT, int NS, bool EDGE>
@@ -55,14 +70,7 @@ __device__ __forceinline__ float sddmm_unit_staged(const T* __restrict__ rhs_lan
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             p[j] = lane_dot<T, KT, NS, EDGE>(a, rhs_lane + (size_t)c[j] * k, k, ls * S::kVec);
-        // transpose-reduce: afterwards lane (ls & 3) == j holds slot j of the quad
-        const bool hi2 = ls & 2, hi1 = ls & 1;
-        const float k0 = hi2 ? p[2] : p[0], s0 = hi2 ? p[0] : p[2];
-        const float k1 = hi2 ? p[3] : p[1], s1 = hi2 ? p[1] : p[3];
-        const float q0 = k0 + lane_xor2(s0);
-        const float q1 = k1 + lane_xor2(s1);
-        float r = (hi1 ? q1 : q0) + lane_xor1(hi1 ? q0 : q1);
-        r = butterfly_sum<4, LPR>(r);
+        const float r = sddmm_quad_reduce<LPR>(p, ls);
         if ((ls >> 2) == q) result = r;
     }
     return result;
@@ -193,6 +201,33 @@ __device__ __forceinline__ void spmm_gather_pairs(const T* __restrict__ b_lane, 
                     for (int x = 0; x < VEC; ++x) acc[x] = fma(v[h][j], b[h][j][x], acc[x]);
         }
     }
+}
+
+// ---- attention ----------------------------------------------------------------
+// What a kernel leaves behind for the gradient.
+enum Keep : int {
+    kKeepNothing = 0,
+    kKeepProbs = 1,  // probs[idx] = the probability
+    kKeepScores = 2, // probs[idx] = the scaled score, stats[row] = (row maximum, 1 / row sum)
+};
+
+// One step of the running softmax of a row: the scores of up to 64 slots (sc, -inf for a
+// lane without a slot) move the maximum; the row's sum and accumulated output are rescaled.
+// Returns this lane's probability relative to the new maximum.
+template <int VEC>
+__device__ __forceinline__ float softmax_step(float sc, bool live, float& m_run, float& l_lane, float (&acc)[VEC])
+{
+    const float m_new = fmaxf(m_run, butterfly_max<1, kWave>(sc));
+    const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+    const float corr = __expf(m_run - m_safe);
+    const float p = live ? __expf(sc - m_safe) : 0.f;
+    l_lane = fmaf(l_lane, corr, p);
+    if (m_run != -INFINITY) { // (nothing to rescale before the first step)
+#pragma unroll
+        for (int x = 0; x < VEC; ++x) acc[x] *= corr;
+    }
+    m_run = m_new;
+    return p;
 }
 
 } // namespace rode
