@@ -281,6 +281,10 @@ int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_ind
  *                         wavefront, and with the length known the grid is sized for that.
  *                         Without it the kernels read the length off the lists and the
  *                         grid is capped instead.  A wrong value costs time, never a result.
+ *   columns_local         0, or nonzero when the columns of neighbouring rows lie close together
+ *                         (most chunks of the residue list have a window: a band).  Knowledge as
+ *                         well: SpMM then does not deal column tiles out to the XCDs, which pays
+ *                         when dense rows are referenced at random.  Costs time at worst.
  * Same results as without a plan, up to the order of the fp32 additions inside a row.
  */
 typedef struct rode_hip_plans {
@@ -294,6 +298,7 @@ typedef struct rode_hip_plans {
     const void* groups;
     const int* group_counts;
     int seg_length;
+    int columns_local;
 } rode_hip_plans;
 
 /* rode_hip_spmm_ex with plans. */
@@ -316,6 +321,11 @@ int rode_hip_spmm_overwrite_limit(int m1, const rode_hip_plans* plans);
  * variants) or 8 (f64).  Must be ordered before both SpMM streams.
  */
 int rode_hip_spmm_clear_rows(int M, int n, int elem_bytes, const int* d_row_offsets, void* d_C, void* stream);
+
+/* The same before a call with RODE_SPMM_OVERWRITE: rows of at most stored_slots aligned slots
+ * (what rode_hip_spmm_overwrite_limit says of that call) are stored by it and left alone too. */
+int rode_hip_spmm_clear_rows_beyond(int M, int n, int elem_bytes, int stored_slots, const int* d_row_offsets, void* d_C,
+                                    void* stream);
 
 /* fp64 values, B and C.  Replaces the double overloads of RoDeSpmm_n32 / RoDeSpmm_n128,
  * RoDe_SpMM/RoDeSpmm.h:10-14, RoDeSpmm.cu:521-529.  Same contract as rode_hip_spmm_f32

@@ -123,19 +123,21 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
         return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
     }
     int code = 0;
-    const char* what = "rode_hip_spmm_clear_rows";
+    const char* what = "rode_hip_spmm_clear_rows_beyond";
+    const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
     void* s = reinterpret_cast<void*>(stream);
     Py_BEGIN_ALLOW_THREADS
     const int* row_ptr = static_cast<const int*>(a.row_ptr->data_ptr());
     // (only the rows that the kernels add to, or skip, need clearing)
-    if (!stored) code = rode_hip_spmm_clear_rows((int)a.m, (int)width, 4, row_ptr, out.data_ptr(), s);
+    if (!stored)
+        code = rode_hip_spmm_clear_rows_beyond((int)a.m, (int)width, 4, rode_hip_spmm_overwrite_limit((int)a.m1, p), row_ptr,
+                                               out.data_ptr(), s);
     if (code == 0) {
         what = "rode_hip_spmm_planned";
-        code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | (stored ? RODE_SPMM_OVERWRITE : 0), (int)a.m1, (int)a.m2, (int)a.n,
+        code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, (int)a.m1, (int)a.m2, (int)a.n,
                                      (int)width, a.val->data_ptr(), static_cast<const int*>(a.col->data_ptr()), row_ptr,
                                      static_cast<const int*>(a.block->data_ptr()), static_cast<const int*>(a.residue->data_ptr()),
-                                     static_cast<const int*>(a.start->data_ptr()), dense->data_ptr(), out.data_ptr(),
-                                     reinterpret_cast<const rode_hip_plans*>(plans), s, s);
+                                     static_cast<const int*>(a.start->data_ptr()), dense->data_ptr(), out.data_ptr(), p, s, s);
     }
     Py_END_ALLOW_THREADS
     if (code != 0) return failed(what, code);

@@ -191,6 +191,7 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
     if (!p) return true;
     if (p->seg_length < 0) return false;
     plan.seg_length = p->seg_length;
+    plan.columns_local = p->columns_local != 0;
     const bool window = p->window && p->window_rows; // (one without rows: the standard kernels do everything)
     if (p->groups) {
         // a group plan needs its header on the host, and excludes the other plans (their
@@ -239,7 +240,6 @@ int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, co
                           const int* d_row_indices2, const int* d_row_seg_st_offsets, const void* d_B, void* d_C,
                           const rode_hip_plans* plans, void* stream1, void* stream2)
 {
-    (void)k;
     constexpr int kKnown = RODE_SPMM_WHOLE_LISTS | RODE_SPMM_ONLY_BLOCK | RODE_SPMM_ONLY_RESIDUE | RODE_SPMM_ONLY_HUB |
                            RODE_SPMM_OVERWRITE;
     static_assert(RODE_SPMM_WHOLE_LISTS == rode::kSpmmWholeLists && RODE_SPMM_ONLY_BLOCK == rode::kSpmmOnlyBlock &&
@@ -255,6 +255,7 @@ int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, co
     hipStream_t s1 = as_stream(stream1), s2 = as_stream(stream2);
     rode::PlanRef plan;
     if (!plan_ref(plans, m2, plan)) return hipErrorInvalidValue;
+    plan.dense_rows = k > 0 ? k : 0;
     // the hub and group kernels replace work items of both lists: only with the complete decomposition
     if ((plan.hub || plan.groups) && !(flags & RODE_SPMM_WHOLE_LISTS)) return hipErrorInvalidValue;
     switch (dtype) {
@@ -290,11 +291,16 @@ int rode_hip_spmm_f32(int m1, int m2, int k, int n, const float* d_values, const
 
 int rode_hip_spmm_clear_rows(int M, int n, int elem_bytes, const int* d_row_offsets, void* d_C, void* stream)
 {
-    if (M < 0 || n <= 0 || (elem_bytes != 4 && elem_bytes != 8) || ((size_t)n * elem_bytes) % 16 != 0)
+    return rode_hip_spmm_clear_rows_beyond(M, n, elem_bytes, 0, d_row_offsets, d_C, stream);
+}
+
+int rode_hip_spmm_clear_rows_beyond(int M, int n, int elem_bytes, int stored_slots, const int* d_row_offsets, void* d_C, void* stream)
+{
+    if (M < 0 || n <= 0 || stored_slots < 0 || (elem_bytes != 4 && elem_bytes != 8) || ((size_t)n * elem_bytes) % 16 != 0)
         return hipErrorInvalidValue;
     if (M == 0) return hipSuccess;
     if (!d_row_offsets || !d_C || !aligned16(d_C)) return hipErrorInvalidValue;
-    return rode::spmm_clear_rows_launch(M, (size_t)n * elem_bytes, d_row_offsets, d_C, as_stream(stream));
+    return rode::spmm_clear_rows_launch(M, (size_t)n * elem_bytes, stored_slots, d_row_offsets, d_C, as_stream(stream));
 }
 
 int rode_hip_spmm_f64(int m1, int m2, int k, int n, const double* d_values, const int* d_column_indices,

@@ -43,6 +43,10 @@ struct PlanRef {
     const int* group_counts = nullptr;
     // SDDMM: the RODE_SPMM_ONLY_* bits of the call (SpMM carries them in its flags)
     int only = 0;
+    // SpMM: rows of the dense operand as the caller says (0: not said), and (set by spmm_launch) into how
+    // many column tiles it is dealt out to the XCDs
+    int dense_rows = 0, shards = 0;
+    bool columns_local = false; // the caller knows that the columns of neighbouring rows lie close together
     // Segment length of the decomposition the lists were made with, 0: not known
     int seg_length = 0;
 };
@@ -101,7 +105,8 @@ template <typename T>
 hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const float* val, const T* B, float* C,
                               const int* plan, const void* plan_rows, hipStream_t stream);
 
-hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, const int* row_ptr, void* C, hipStream_t stream);
+// (stored: rows of at most that many aligned slots are left alone as well)
+hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, int stored, const int* row_ptr, void* C, hipStream_t stream);
 
 template <typename T>
 hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int* residue_rows, const int* st_off,

@@ -54,7 +54,21 @@ constexpr int kMergeMinSegments = 16384;
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
 // are processed by one launch (spmm_pair_kernel).  Above it the residue kernel runs on its
 // own: it needs a quarter of the block kernel's registers and keeps twice the waves per CU.
+// (Sharded launches, below, keep to one launch for longer: their workgroups are smaller.  Power-law-like
+// rows, 65 K x 65 K, 1 M nonzeros, width 128: 75 us in two launches, 63 in one.)
 constexpr int kPairMaxWorkgroups = 16384;
+constexpr int kPairMaxSharded = 65536;
+
+// Sharding.  Every XCD has an L2 of its own (4 MB), and rows of B that are referenced at random are
+// fetched into all eight.  When a row of B is 2, 4 or 8 lines of 128 bytes, C is computed in column
+// tiles of one line and XCD x works on tile x mod lines only: of B it sees one line per row, so that a
+// matrix of up to lines x 4 MB stays in the L2s, and of twice that about half of it does.  The nonzeros'
+// columns and values are read once per tile (8 bytes against 128 gathered).  65 K x 65 K, 1 M nonzeros:
+// width 64 43 -> 35 us, 128 halves 64 -> 39 (with the rows of a single work item stored), width 128 77 -> 63;
+// 16 K x 16 K, width 128: 34 -> 21.  Below 4 MB every L2 holds all of B anyway.  Seven times an L2 per tile
+// is where the gain ends (200 K rows: 254 -> 240 us; 400 K rows of width 64: 472 -> 492), and rows whose
+// columns lie close together share their lines without it (band of 256 in 60 K rows: 32 -> 39).
+constexpr size_t kShardMinBytes = (size_t)4 << 20, kShardMaxTileBytes = (size_t)28 << 20;
 
 // A row of C that is written once and not read again by the kernel that writes it: stored
 // with the non-temporal hint, so that it does not push the gathered rows of B out of the
@@ -129,6 +143,20 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
     for (int x = 0; x < VEC; ++x) total[x] = butterfly_sum<LPR, kWave>(acc[x]);
 }
 
+// Which column tile of C, and which of the `blocks` workgroups of its grid row, a workgroup is.
+// shards == 1: tiles in blockIdx.y.  shards > 1 (a divisor of kXcds): XCD x only ever works on tile
+// x % shards, its grid rows dealt out one after the other in a one-dimensional grid.
+struct TilePlace {
+    int bid, tile;
+};
+__device__ __forceinline__ TilePlace tile_place(int b, int blocks, int shards)
+{
+    if (shards == 1) return TilePlace{b, (int)blockIdx.y};
+    const int x = b % kXcds, at = x / shards * (blocks / kXcds * shards) + b / kXcds; // position in the tile's row, contiguous per XCD
+    // (as the id that xcd_logical_block takes to that position)
+    return TilePlace{at % (blocks / kXcds) * kXcds + at / (blocks / kXcds), x % shards};
+}
+
 // One wave per block segment (see sddmm_block_kernel for the slot arithmetic,
 // identical at RoDeSpmm.cu:210-234).
 // (bid of nblocks: the workgroup's position in the part of the grid that works on block segments)
@@ -139,7 +167,7 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
 // that never takes it from 0.97 to 1.13 ms on the power-law benchmark).
 template <typename T, int TN, bool EDGE, int WALK, bool STORE>
 __device__ __forceinline__ void
-spmm_block_body(int bid, int nblocks, int m1, int n, int owned_slots, int chunk_hint, RowOwners owners,
+spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, int chunk_hint, RowOwners owners,
                 const int* __restrict__ block_rows,
                 const int* __restrict__ st_off, const int* __restrict__ row_ptr, const int* __restrict__ col,
                 const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
@@ -165,7 +193,6 @@ spmm_block_body(int bid, int nblocks, int m1, int n, int owned_slots, int chunk_
         if (first < 0) return;
         const int last = (int)min(first + chunk, (long long)m1);
         const int ls = lane % LPR, group = lane / LPR;
-        const int tile = blockIdx.y * TN;
         const bool col_ok = !EDGE || tile + ls * VEC < n;
         const T* b_lane = B + tile + (col_ok ? ls * VEC : 0);
         constexpr int EPG = VEC / G > 0 ? VEC / G : 1; // elements each lane group adds to C
@@ -229,7 +256,6 @@ spmm_block_body(int bid, int nblocks, int m1, int n, int owned_slots, int chunk_
     const int row = it.row, mask = it.mask, base = it.base, cnt = it.cnt;
 
     const int ls = lane % LPR, group = lane / LPR;
-    const int tile = blockIdx.y * TN;
     // EDGE: n is not a multiple of TN; lanes past the last column re-read the tile's
     // first columns (a valid address) and never write
     const bool col_ok = !EDGE || tile + ls * VEC < n;
@@ -279,7 +305,7 @@ spmm_block_body(int bid, int nblocks, int m1, int n, int owned_slots, int chunk_
 // group walks its row's slot quads one after the other, no cross-lane reduction.
 template <typename T, int TN, bool EDGE>
 __device__ __forceinline__ void
-spmm_residue_body(int bid, int nblocks, int m2, int n, int owned_slots, RowOwners owners,
+spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots, RowOwners owners,
                   const int* __restrict__ residue_rows,
                   const int* __restrict__ row_ptr, const int* __restrict__ col,
                   const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
@@ -306,7 +332,6 @@ spmm_residue_body(int bid, int nblocks, int m2, int n, int owned_slots, RowOwner
     if (owned_elsewhere(owners, row, it.aligned)) return; // another kernel has the whole row
     const int first = it.first, cnt = it.cnt;
 
-    const int tile = blockIdx.y * TN;
     const bool col_ok = !EDGE || tile + ls * VEC < n;
     int* my_c = lds_c + (wave * RPW + group) * kBlockItems;
     A* my_v = lds_v + (wave * RPW + group) * kBlockItems;
@@ -347,43 +372,48 @@ spmm_residue_body(int bid, int nblocks, int m2, int n, int owned_slots, RowOwner
 
 template <typename T, int TN, bool EDGE, int WALK, bool STORE>
 __global__ void __launch_bounds__(kWgThreads)
-spmm_block_kernel(int m1, int n, int owned_slots, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
+spmm_block_kernel(int shards, int m1, int n, int owned_slots, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                   const int* __restrict__ st_off,
                   const int* __restrict__ row_ptr, const int* __restrict__ col,
                   const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
                   typename DenseVec<T>::Acc* __restrict__ C)
 {
-    spmm_block_body<T, TN, EDGE, WALK, STORE>(blockIdx.x, gridDim.x, m1, n, owned_slots, chunk_hint, owners, block_rows, st_off,
+    const TilePlace at = tile_place(blockIdx.x, gridDim.x / shards, shards);
+    spmm_block_body<T, TN, EDGE, WALK, STORE>(at.bid, gridDim.x / shards, at.tile * TN, m1, n, owned_slots, chunk_hint, owners, block_rows, st_off,
                                        row_ptr, col, val, B, C);
 }
 
 template <typename T, int TN, bool EDGE>
 __global__ void __launch_bounds__(kWgThreads)
-spmm_residue_kernel(int m2, int n, int owned_slots, RowOwners owners, const int* __restrict__ residue_rows,
+spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners, const int* __restrict__ residue_rows,
                     const int* __restrict__ row_ptr, const int* __restrict__ col,
                     const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
                     typename DenseVec<T>::Acc* __restrict__ C, const int* __restrict__ plan)
 {
-    spmm_residue_body<T, TN, EDGE>(blockIdx.x, gridDim.x, m2, n, owned_slots, owners, residue_rows, row_ptr, col, val, B,
+    const TilePlace at = tile_place(blockIdx.x, gridDim.x / shards, shards);
+    spmm_residue_body<T, TN, EDGE>(at.bid, gridDim.x / shards, at.tile * TN, m2, n, owned_slots, owners, residue_rows, row_ptr, col, val, B,
                                    C, plan);
 }
 
-// Both lists in one launch: the first g1 workgroups of a grid row work on block segments,
-// the others on residue rows.  For matrices so small that a launch costs as much as its
+// Both lists in one launch: the first g1 workgroups of a grid row (of every tile of a sharded
+// grid) work on block segments, the others on residue rows.  For matrices so small that a launch costs as much as its
 // kernel (a kernel of a few microseconds); the two parts then also fill the GPU together.
-template <typename T, int TN, bool EDGE, bool STORE>
+template <typename T, int TN, bool EDGE, int WALK, bool STORE>
 __global__ void __launch_bounds__(kWgThreads)
-spmm_pair_kernel(int g1, int m1, int m2, int n, int owned_slots, int chunk_hint, RowOwners owners,
+spmm_pair_kernel(int shards, int g1, int m1, int m2, int n, int owned_slots, int chunk_hint, RowOwners owners,
                  const int* __restrict__ block_rows,
                  const int* __restrict__ residue_rows, const int* __restrict__ st_off, const int* __restrict__ row_ptr,
                  const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
                  const T* __restrict__ B, typename DenseVec<T>::Acc* __restrict__ C, const int* __restrict__ plan)
 {
-    if ((int)blockIdx.x < g1)
-        spmm_block_body<T, TN, EDGE, 2, STORE>(blockIdx.x, g1, m1, n, owned_slots, 0, owners, block_rows, st_off, row_ptr, col, val,
+    const bool segments = (int)blockIdx.x < g1 * shards;
+    const int g = segments ? g1 : gridDim.x / shards - g1;
+    const TilePlace at = tile_place(segments ? blockIdx.x : blockIdx.x - g1 * shards, g, shards);
+    if (segments)
+        spmm_block_body<T, TN, EDGE, WALK, STORE>(at.bid, g, at.tile * TN, m1, n, owned_slots, chunk_hint, owners, block_rows, st_off, row_ptr, col, val,
                                         B, C);
     else
-        spmm_residue_body<T, TN, EDGE>(blockIdx.x - g1, gridDim.x - g1, m2, n, max(owned_slots, 0), owners, residue_rows,
+        spmm_residue_body<T, TN, EDGE>(at.bid, g, at.tile * TN, m2, n, max(owned_slots, 0), owners, residue_rows,
                                        row_ptr, col, val,
                                        B, C, plan);
 }
@@ -664,11 +694,12 @@ spmm_hub_reduce_kernel(int n, int merge, const int* __restrict__ hub, const A* _
 constexpr int kClearRowsPerGroup = 8;
 
 // Zeroes exactly the rows of C that the two SpMM kernels do not overwrite: rows whose
-// aligned length N = len + (start & 3) is >= 32 are accumulated into, rows with N == 0
+// aligned length N = len + (start & 3) is >= 32 are accumulated into (but, under
+// kSpmmOverwrite, those of at most `stored` slots: spmm_overwrite_limit), rows with N == 0
 // belong to no work item; rows with 0 < N < 32 are stored by the residue kernel and
 // are left alone.  16 lanes x 16 bytes per step and row.
 __global__ void __launch_bounds__(kWgThreads)
-spmm_clear_rows_kernel(int M, size_t row_bytes, const int* __restrict__ row_ptr, char* __restrict__ C)
+spmm_clear_rows_kernel(int M, size_t row_bytes, int stored, const int* __restrict__ row_ptr, char* __restrict__ C)
 {
     constexpr int kLanes = 16, kGroups = kWgThreads / kLanes;
     const int group = threadIdx.x / kLanes, lane = threadIdx.x % kLanes;
@@ -684,7 +715,7 @@ spmm_clear_rows_kernel(int M, size_t row_bytes, const int* __restrict__ row_ptr,
 #pragma unroll
     for (int b = 0; b < kClearRowsPerGroup; ++b) {
         const int N = e[b] - s[b] + (s[b] & (kVecLen - 1));
-        if (N > 0 && N < kBlockItems) continue;
+        if (N > 0 && (N < kBlockItems || N <= stored)) continue;
         char* dst = C + (size_t)(first + b * kGroups + group) * row_bytes;
         for (size_t off = lane * 16; off < row_bytes; off += kLanes * 16)
             *reinterpret_cast<uint4*>(dst + off) = make_uint4(0, 0, 0, 0);
@@ -727,11 +758,16 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     const bool hubs = hub_plan && (only == 0 || only == kSpmmOnlyHub);
     const bool grouped = group_plan && (only == 0 || only == kSpmmOnlyHub); // (timed with the hub kernels)
     constexpr int RPW = kWave / SpmmShape<T, TN>::kLpr;
-    // (segments per wave: known only when the caller said how long its segments are and merging is on)
-    const int chunk_hint = block_owned != 0 ? chunk_for_segments(plan.seg_length, m1) : (plan.seg_length > 0 ? 1 : 0);
+    const int shards = plan.shards > 1 ? plan.shards : 1, tile_rows = plan.shards > 1 ? 1 : tiles;
+    // (segments per wave: known only when the caller said how long its segments are and merging is on.
+    // A sharded launch has a wave per segment and tile: with many of them a wave takes several rows - 16 K
+    // rows of 40 nonzeros, width 128: 41 -> 32 us - later than an unsharded one, as long rows need the waves)
+    const int walked = shards > 1 ? (int)min((long long)m1 * shards / 3, (long long)INT32_MAX) : m1;
+    const int chunk_hint = block_owned != 0 ? chunk_for_segments(plan.seg_length, walked) : (plan.seg_length > 0 ? 1 : 0);
     const int g1 = chunk_hint > 0 ? grid_for_waves((m1 + chunk_hint - 1) / chunk_hint) : grid_for_waves(min(m1, kBlockGridWaves));
     const int g2 = grid_for_waves(((long long)m2 + RPW - 1) / RPW);
     if (g1 < 0 || g2 < 0 || tiles > 65535) return hipErrorInvalidConfiguration;
+    if ((long long)max(g1, g2) * shards * kWgThreads >= (1ll << 32)) return hipErrorInvalidConfiguration;
     // With a host copy of the plan's header, a kernel that would find every chunk taken by
     // the other one is not launched at all.
     bool standard_residue = true, window_residue = plan.dev != nullptr;
@@ -744,15 +780,19 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     const bool block = lists && m1 > 0 && (only == 0 || only == kSpmmOnlyBlock);
     const bool residue = lists && m2 > 0 && (only == 0 || only == kSpmmOnlyResidue);
     hipError_t e = hipSuccess;
-    if (block && residue && standard_residue && s1 == s2 && (long long)(g1 + g2) * tiles <= kPairMaxWorkgroups) {
-        dim3 grid(g1 + g2, tiles);
-        auto kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, true> : spmm_pair_kernel<T, TN, EDGE, false>;
-        kernel<<<grid, kWgThreads, 0, s1>>>(g1, m1, m2, n, block_owned, chunk_hint, owners, block_rows, residue_rows, st_off,
+    if (block && residue && standard_residue && s1 == s2 && (long long)(g1 + g2) * tiles <= (shards > 1 ? kPairMaxSharded : kPairMaxWorkgroups)) {
+        dim3 grid((g1 + g2) * shards, tile_rows);
+        auto kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 2, true> : spmm_pair_kernel<T, TN, EDGE, 2, false>;
+        if (chunk_hint == 1)
+            kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 0, true> : spmm_pair_kernel<T, TN, EDGE, 0, false>;
+        else if (chunk_hint > 1)
+            kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 1, true> : spmm_pair_kernel<T, TN, EDGE, 1, false>;
+        kernel<<<grid, kWgThreads, 0, s1>>>(shards, g1, m1, m2, n, block_owned, chunk_hint, owners, block_rows, residue_rows, st_off,
                                             row_ptr, col, val, B, C, plan.dev);
         e = hipGetLastError();
     } else {
         if (block) {
-            dim3 grid(g1, tiles);
+            dim3 grid(g1 * shards, tile_rows);
             auto kernel = spmm_block_kernel<T, TN, EDGE, 2, false>;
             if (chunk_hint == 1)
                 kernel = owners.overwrite ? spmm_block_kernel<T, TN, EDGE, 0, true> : spmm_block_kernel<T, TN, EDGE, 0, false>;
@@ -760,12 +800,12 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
                 kernel = owners.overwrite ? spmm_block_kernel<T, TN, EDGE, 1, true> : spmm_block_kernel<T, TN, EDGE, 1, false>;
             else if (owners.overwrite)
                 kernel = spmm_block_kernel<T, TN, EDGE, 2, true>;
-            kernel<<<grid, kWgThreads, 0, s1>>>(m1, n, block_owned, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, B, C);
+            kernel<<<grid, kWgThreads, 0, s1>>>(shards, m1, n, block_owned, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, B, C);
             e = hipGetLastError();
         }
         if (residue && standard_residue) {
-            dim3 grid(g2, tiles);
-            spmm_residue_kernel<T, TN, EDGE><<<grid, kWgThreads, 0, s2>>>(m2, n, owned_slots, owners, residue_rows, row_ptr, col,
+            dim3 grid(g2 * shards, tile_rows);
+            spmm_residue_kernel<T, TN, EDGE><<<grid, kWgThreads, 0, s2>>>(shards, m2, n, owned_slots, owners, residue_rows, row_ptr, col,
                                                                           val, B, C, plan.dev);
             if (e == hipSuccess) e = hipGetLastError();
         }
@@ -845,6 +885,17 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
         plan.host_counts = nullptr;
     }
     constexpr int kMaxTile = 32 * DenseVec<T>::kElems >= 128 ? 128 : 32 * DenseVec<T>::kElems;
+    if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
+        constexpr int kLine = 128 / (int)sizeof(T);
+        const int lines = n / kLine;
+        const size_t bytes = (size_t)plan.dense_rows * n * sizeof(T);
+        // (a plan's kernels have their own ways to share dense rows)
+        if (n % kLine == 0 && (lines == 2 || lines == 4 || lines == 8) && bytes > kShardMinBytes && (size_t)plan.dense_rows * 128 <= kShardMaxTileBytes &&
+            !plan.columns_local && plan.hub == nullptr && plan.groups == nullptr && plan.dev == nullptr) {
+            plan.shards = lines;
+            return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
+        }
+    }
     auto padded = [n](int tn) { return (n + tn - 1) / tn * tn; };
     int best = 32;
     if (padded(64) <= padded(best)) best = 64;
@@ -860,14 +911,14 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
     return launch_edge<T, 32>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
 }
 
-hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, const int* row_ptr, void* C, hipStream_t stream)
+hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, int stored, const int* row_ptr, void* C, hipStream_t stream)
 {
     if (M <= 0) return hipSuccess;
     constexpr int kRowsPerWg = kWgThreads / 16 * kClearRowsPerGroup;
     long long wgs = ((long long)M + kRowsPerWg - 1) / kRowsPerWg;
     wgs = (wgs + kXcds - 1) / kXcds * kXcds;
     if (wgs * kWgThreads >= (1ll << 32)) return hipErrorInvalidConfiguration;
-    spmm_clear_rows_kernel<<<(int)wgs, kWgThreads, 0, stream>>>(M, row_bytes, row_ptr, static_cast<char*>(C));
+    spmm_clear_rows_kernel<<<(int)wgs, kWgThreads, 0, stream>>>(M, row_bytes, stored, row_ptr, static_cast<char*>(C));
     return hipGetLastError();
 }
 

@@ -130,9 +130,11 @@ class RoDeCSR:
         self.m1 = m1
         self.m2 = m2
         self.plan = (self._group_plan() or self._hub_plan()) if others else None
+        self.columns_local = False  # (known only when the residue list has been looked at)
         if self.plan is None and self.locality and m2 > 0:
             plan = rode_sddmm_hip.WindowPlan(data, counts) if data is not None else \
                 rode_sddmm_hip.window_plan(res, m2, self.row_offsets, self.column_indices, self.n)
+            self.columns_local = 2 * plan.windowed > plan.counts[0]
             enough = plan.windowed >= max(self.PLAN_MIN_CHUNKS, (plan.counts[0] + 1) // 2)
             if plan.windowed > 0 and (self.locality is True or enough):
                 self.plan = rode_sddmm_hip.window_plan_rows(plan, res, m2, self.row_offsets, self.column_indices)
@@ -185,7 +187,7 @@ class RoDeCSR:
         plans = self._shared.get(key)
         if plans is None:
             plans = rode_sddmm_hip.plans_struct(self.plan, spmm_width, spmm_elem_bytes, True,
-                                                seg_length=self.config["seg_length"])
+                                                seg_length=self.config["seg_length"], columns_local=self.columns_local)
             self._shared[key] = plans
         return plans
 

@@ -294,13 +294,15 @@ def group_plan(row_offsets, column_indices, m):
     return GroupPlan(data, list(counts))
 
 
-def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0):
+def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0, columns_local=False):
     """The ``rode_hip_plans`` struct of one call (keep it alive until the call returns; pass
     it with ``ctypes.byref``).  ``plan``: a ``WindowPlan``, a ``HubPlan``, a ``GroupPlan`` or None.
     ``spmm_width``: for an SpMM call the dense width, so that a hub plan's workspace is
     attached; a hub plan is left out of an SpMM call without the whole-lists promise.
-    ``seg_length``: the segment length the lists were made with, 0 when not known."""
+    ``seg_length``: the segment length the lists were made with, 0 when not known.
+    ``columns_local``: the columns of neighbouring rows are known to lie close together."""
     p = _lib.Plans()
+    p.columns_local = int(columns_local)
     p.seg_length = int(seg_length or 0)  # (the segment length of the decomposition, when the caller knows it)
     if isinstance(plan, GroupPlan):
         if plan.usable and (spmm_width is None or whole_lists):
@@ -428,18 +430,21 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     vec = _VEC[dense_matrix.dtype]
     _check(n > 0 and n % vec == 0, f"dense_matrix cols must be a positive multiple of {vec}")
     lib = _lib.load()
+    if plans is None:
+        plans = plans_struct(plan, n, values.element_size(), whole_lists, seg_length=seg_length)
+    overwrite = out is None and whole_lists  # (a caller's C is added to, as the kernels' contract says)
     if out is None:
         if m1 == 0 and m2 == 0:
             return torch.zeros((m, n), dtype=out_dtype, device=values.device)
         # only the rows the kernels add to (or skip) need clearing, the others are overwritten
         out = torch.empty((m, n), dtype=out_dtype, device=values.device)
-        every_row_stored = every_row_stored and whole_lists
-        with _on_device(values.device):
-            if not every_row_stored:
-                _lib.check(lib.rode_hip_spmm_clear_rows(m, n, out.element_size(), row_offsets.data_ptr(), out.data_ptr(),
-                                                        _stream_handle(values.device)), "rode_hip_spmm_clear_rows")
+        if not (every_row_stored and whole_lists):
+            stored = lib.rode_hip_spmm_overwrite_limit(m1, ctypes.byref(plans)) if whole_lists else 0
+            with _on_device(values.device):
+                _lib.check(lib.rode_hip_spmm_clear_rows_beyond(m, n, out.element_size(), stored, row_offsets.data_ptr(),
+                                                               out.data_ptr(), _stream_handle(values.device)),
+                           "rode_hip_spmm_clear_rows_beyond")
     else:
-        every_row_stored = False  # (the caller's C is added to, as the kernels' contract says)
         _check_input(out, "out")
         _check(out.dtype == out_dtype and tuple(out.shape) == (m, n), f"out must be {out_dtype} of shape (m, n)")
     if m1 == 0 and m2 == 0:
@@ -447,9 +452,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     dtype = {torch.float32: 0, torch.float16: 1, torch.float64: 2}[dense_matrix.dtype]  # RODE_DENSE_*
     with _on_device(values.device):
         s = _stream_handle(values.device)
-        if plans is None:
-            plans = plans_struct(plan, n, out.element_size(), whole_lists, seg_length=seg_length)
-        flags = (_lib.SPMM_WHOLE_LISTS if whole_lists else 0) | (_lib.SPMM_OVERWRITE if every_row_stored else 0)
+        flags = (_lib.SPMM_WHOLE_LISTS if whole_lists else 0) | (_lib.SPMM_OVERWRITE if overwrite else 0)
         code = lib.rode_hip_spmm_planned(dtype, flags, m1, m2, k, n,
                                          values.data_ptr(), column_indices.data_ptr(), row_offsets.data_ptr(),
                                          block_indices.data_ptr(), residue_indices.data_ptr(), st_offsets.data_ptr(),
