@@ -18,15 +18,29 @@ from . import _lib, rode_sddmm_hip
 
 
 def _sddmm(csr, values, lhs, rhs):
+    values, lhs, rhs = values.contiguous(), lhs.contiguous(), rhs.contiguous()
+    k = lhs.shape[1]
+    out = _lib.host_call().sddmm(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
+                                 csr.column_indices, values, csr.m, csr.n, k, lhs, rhs, csr.plans_address(),
+                                 rode_sddmm_hip._stream_handle(csr.device))
+    if out is not None:
+        return out
     return rode_sddmm_hip.sddmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2,
-                                        csr.row_offsets, csr.column_indices, values.contiguous(), csr.m, csr.n,
-                                        lhs.contiguous(), rhs.contiguous(), lhs.shape[1], plan=csr.plan, seg_length=csr.config["seg_length"])
+                                        csr.row_offsets, csr.column_indices, values, csr.m, csr.n, lhs, rhs, k,
+                                        plan=csr.plan, plans=csr.call_plans())
 
 
 def _spmm(csr, values, dense):
+    values, dense = values.contiguous(), dense.contiguous()
+    width = dense.shape[1]
+    out = _lib.host_call().spmm(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
+                                csr.column_indices, values, csr.m, csr.n, dense, csr.plans_address(width),
+                                csr.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(csr.device))
+    if out is not None:
+        return out
     return rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2,
-                                       csr.row_offsets, csr.column_indices, values.contiguous(), csr.m, csr.n,
-                                       dense.contiguous(), plan=csr.plan, seg_length=csr.config["seg_length"],
+                                       csr.row_offsets, csr.column_indices, values, csr.m, csr.n, dense, plan=csr.plan,
+                                       plans=csr.call_plans(width, values.element_size()),
                                        every_row_stored=csr.spmm_stores_every_row())
 
 

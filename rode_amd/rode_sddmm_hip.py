@@ -185,7 +185,7 @@ def permute(values, perm):
     _check(values.dtype == torch.float32 and perm.dtype == torch.int32, "values must be float32 and perm int32")
     _check(values.dim() == 1 and perm.dim() == 1 and values.device == perm.device, "values and perm must be vectors on one device")
     out = torch.empty(perm.numel(), dtype=torch.float32, device=values.device)
-    with torch.cuda.device(values.device):
+    with _on_device(values.device):
         _lib.check(_lib.load().rode_hip_permute_f32(perm.numel(), values.data_ptr(), perm.data_ptr(), out.data_ptr(),
                                                      _stream_handle(values.device)), "rode_hip_permute_f32")
     return out
