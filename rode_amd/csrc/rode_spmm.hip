@@ -316,8 +316,10 @@ spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots
     constexpr int VEC = S::kVec, LPR = S::kLpr;
     constexpr int RPW = kWave / LPR;        // rows per wave
     constexpr int OWN = kBlockItems / LPR;  // slots staged by one lane
-    __shared__ __attribute__((aligned(16))) int lds_c[kWavesPerWg * RPW * kBlockItems];
-    __shared__ __attribute__((aligned(16))) A lds_v[kWavesPerWg * RPW * kBlockItems];
+    // (16 bytes between the rows of a wave: its groups read their slots at the same time, from banks of their own)
+    constexpr int kStrideC = kBlockItems + 4, kStrideV = kBlockItems + 16 / (int)sizeof(A);
+    __shared__ __attribute__((aligned(16))) int lds_c[kWavesPerWg * RPW * kStrideC];
+    __shared__ __attribute__((aligned(16))) A lds_v[kWavesPerWg * RPW * kStrideV];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     const int group = lane / LPR, ls = lane % LPR;
     const int item = (xcd_logical_block(bid, nblocks) * kWavesPerWg + wave) * RPW + group;
@@ -333,8 +335,8 @@ spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots
     const int first = it.first, cnt = it.cnt;
 
     const bool col_ok = !EDGE || tile + ls * VEC < n;
-    int* my_c = lds_c + (wave * RPW + group) * kBlockItems;
-    A* my_v = lds_v + (wave * RPW + group) * kBlockItems;
+    int* my_c = lds_c + (wave * RPW + group) * kStrideC;
+    A* my_v = lds_v + (wave * RPW + group) * kStrideV;
 
     A acc[VEC];
 #pragma unroll
@@ -342,12 +344,22 @@ spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots
 
     if (cnt > 0) {
         const int padded = (cnt + 3) & ~3; // slots past the tail repeat its last column with value 0
+        int c[OWN];
+        A v[OWN]; // (all of them on their way before the first is waited for)
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) {
+            const int slot = ls + i * LPR, at = first + min(slot, cnt - 1);
+            if (slot < padded) {
+                c[i] = col[at];
+                v[i] = val[at];
+            }
+        }
 #pragma unroll
         for (int i = 0; i < OWN; ++i) {
             const int slot = ls + i * LPR;
             if (slot < padded) {
-                my_c[slot] = col[first + min(slot, cnt - 1)];
-                my_v[slot] = slot < cnt ? val[first + slot] : A(0);
+                my_c[slot] = c[i];
+                my_v[slot] = slot < cnt ? v[i] : A(0);
             }
         }
         wave_lds_sync();
