@@ -116,23 +116,27 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
 #pragma unroll
     for (int x = 0; x < VEC; ++x) acc[x] = A(0);
 
+    // slots of the previous row (head) and slots past the end (last quad) are neutralised:
+    // value 0, column of a real slot
+    auto fetch = [&](int off, int& c, A& v) __attribute__((always_inline)) {
+        const int slot = off + lane;
+        if (lane < ((min(cnt - off, kWave) + 3) & ~3)) {
+            const int at = min(max(slot, mask), cnt - 1);
+            const int idx = base + at + (at >= split ? jump : 0);
+            c = col[idx];
+            v = val[idx];
+        }
+    };
+    int c = 0;
+    A v = A(0);
+    fetch(0, c, v);
     for (int off = 0; off < cnt; off += kWave) {
         const int slot = off + lane;
         const int live = min(cnt - off, kWave); // 64, or less on the last step
-        int c = 0;
-        A v = A(0);
-        if (lane < ((live + 3) & ~3)) {
-            // slots of the previous row (head) and slots past the end (last quad) are
-            // neutralised: value 0, column of a real slot
-            const bool head = slot < mask, past = slot >= cnt;
-            const int at = head ? mask : (past ? cnt - 1 : slot);
-            const int idx = base + at + (at >= split ? jump : 0);
-            c = col[idx];
-            v = (head || past) ? A(0) : val[idx];
-        }
         my_c[lane] = c;
-        my_v[lane] = v;
+        my_v[lane] = slot < mask || slot >= cnt ? A(0) : v;
         wave_lds_sync();
+        if (off + kWave < cnt) fetch(off + kWave, c, v); // (on its way while the dense rows arrive)
         if (live == kWave)
             spmm_gather<T, TN, 16 / G, true>(b_lane, (size_t)n, acc, my_c, my_v, group, G, 16);
         else
