@@ -100,10 +100,10 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
                        typename SpmmAcc<T>::type* C, int flags, PlanRef plan, hipStream_t s1, hipStream_t s2);
 
-// the window kernel of SpMM over the planned chunks of the residue list (T = float or __half)
+// the window kernel of SpMM over the planned chunks of the residue list
 template <typename T>
-hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const float* val, const T* B, float* C,
-                              const int* plan, const void* plan_rows, hipStream_t stream);
+hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
+                              typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream);
 
 // (stored: rows of at most that many aligned slots are left alone as well)
 hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, int stored, const int* row_ptr, void* C, hipStream_t stream);

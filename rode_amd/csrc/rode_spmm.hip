@@ -70,32 +70,6 @@ constexpr int kPairMaxSharded = 65536;
 // columns lie close together share their lines without it (band of 256 in 60 K rows: 32 -> 39).
 constexpr size_t kShardMinBytes = (size_t)4 << 20, kShardMaxTileBytes = (size_t)28 << 20;
 
-// A row of C that is written once and not read again by the kernel that writes it: stored
-// with the non-temporal hint, so that it does not push the gathered rows of B out of the
-// caches on its way (config 4, K=128: residue kernel 1.19 -> 1.09 ms; the same hint on the
-// loads of B, on SDDMM's loads of rhs or on its stores of `out` made those kernels slower).
-template <int VEC>
-__device__ __forceinline__ void store_row(float* dst, const float (&acc)[VEC])
-{
-    typedef float Quad __attribute__((ext_vector_type(4)));
-#pragma unroll
-    for (int x = 0; x < VEC; x += 4) {
-        const Quad v = {acc[x], acc[x + 1], acc[x + 2], acc[x + 3]};
-        __builtin_nontemporal_store(v, reinterpret_cast<Quad*>(dst + x));
-    }
-}
-
-template <int VEC>
-__device__ __forceinline__ void store_row(double* dst, const double (&acc)[VEC])
-{
-    typedef double Pair __attribute__((ext_vector_type(2)));
-#pragma unroll
-    for (int x = 0; x < VEC; x += 2) {
-        const Pair v = {acc[x], acc[x + 1]};
-        __builtin_nontemporal_store(v, reinterpret_cast<Pair*>(dst + x));
-    }
-}
-
 // Sum over the aligned slots [base, base + cnt) of values * B rows, for this lane's columns
 // of the tile; the first `mask` slots (the previous row's) and the slots past cnt in the
 // last quad are neutralised.  Every lane of the wave returns the wave's total.
@@ -854,10 +828,8 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         }
         e = hipGetLastError();
     }
-    if constexpr (!std::is_same<T, double>::value) {
-        if (e == hipSuccess && residue && window_residue)
-            e = spmm_window_launch<T>(m2, n, owned_slots, col, val, B, C, plan.dev, plan.rows, s2);
-    }
+    if (e == hipSuccess && residue && window_residue)
+        e = spmm_window_launch<T>(m2, n, owned_slots, col, val, B, C, plan.dev, plan.rows, s2);
     return e;
 }
 
@@ -884,8 +856,8 @@ int spmm_overwrite_limit(int m1, bool hub_plan) { return m1 >= kOwnedMinSegments
 // dense row is cut into tiles of 32, 64 or 128 columns (at most 32 lanes per tile row);
 // the tile width with the least padding wins, the widest on a tie.  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
-// which `plan` holds a window go to the window kernel (fp32 and fp16 operands wider than
-// one 128-byte tile; fp64 and narrower operands ignore the plan: with a single tile the
+// which `plan` holds a window go to the window kernel (operands wider than one 128-byte tile;
+// narrower ones ignore the plan: with a single tile the
 // window is not reused often enough to repay its staging).
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
@@ -894,8 +866,9 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
 {
     static_assert(std::is_same<typename SpmmAcc<T>::type, typename DenseVec<T>::Acc>::value, "accumulation type");
     if (n <= 0 || n % DenseVec<T>::kElems != 0) return hipErrorInvalidValue;
-    // the window kernels are for fp32 / fp16 operands with more than one 128-byte tile per row
-    if (std::is_same<T, double>::value || (size_t)n * sizeof(T) <= 128) {
+    // the window kernels are for operands with more than one 128-byte tile per row (500 K rows of 32 doubles, band of
+    // 256: 0.204 -> 0.131 ms)
+    if ((size_t)n * sizeof(T) <= 128) {
         plan.dev = nullptr;
         plan.rows = nullptr;
         plan.host_counts = nullptr;

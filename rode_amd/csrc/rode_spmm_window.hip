@@ -3,149 +3,205 @@
 // the chunks are chosen).  Same rows, same slots and the same store/accumulate rule as
 // spmm_residue_kernel in rode_spmm.hip (reference: RoDe_SpMM/RoDeSpmm.cu:41-195); what
 // differs is where B comes from.
-#define RODE_PHASE_READER // (debug builds with RODE_PHASE_TIMING: this file holds the counters that are read back)
 #include "rode_window.hpp"
+#include "rode_units.hpp"
 #include "rode_internal.hpp"
 
 namespace rode {
 
 namespace {
 
+// 16 bytes of a row of B as numbers of the accumulator's type
+template <typename T>
+__device__ __forceinline__ void unpack_dense(const uint4& raw, typename DenseVec<T>::Acc (&out)[DenseVec<T>::kElems])
+{
+    if constexpr (sizeof(T) == 8) {
+        out[0] = __hiloint2double((int)raw.y, (int)raw.x);
+        out[1] = __hiloint2double((int)raw.w, (int)raw.z);
+    } else {
+        DenseVec<T>::unpack(raw, out);
+    }
+}
+
+// lane J of the quad's value
+template <int J>
+__device__ __forceinline__ float of_quad(float x)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x55 * J, 0xf, 0xf, true));
+}
+template <int J>
+__device__ __forceinline__ double of_quad(double x)
+{
+    return __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), 0x55 * J, 0xf, 0xf, true),
+                            __builtin_amdgcn_update_dpp(0, __double2loint(x), 0x55 * J, 0xf, 0xf, true));
+}
+
 template <typename T, bool EDGE>
 __global__ void __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-spmm_residue_window_kernel(int m2, int n, int owned_slots, const int* __restrict__ col, const float* __restrict__ val,
-                           const T* __restrict__ B, float* __restrict__ C, const PlannedChunk* __restrict__ rows)
+spmm_residue_window_kernel(int m2, int n, int owned_slots, const int* __restrict__ col,
+                           const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
+                           typename DenseVec<T>::Acc* __restrict__ C, const PlannedChunk* __restrict__ rows)
 {
+    using A = typename DenseVec<T>::Acc;
     constexpr int VEC = DenseVec<T>::kElems;
     constexpr int TW = kResLanes * VEC; // columns of one tile
     constexpr int QUADS = kBlockItems / 4;
-    __shared__ uint4 win[kResWinVecs];
-    __shared__ __attribute__((aligned(16))) float lds_val[kResRows * kResValStride];
+    __shared__ uint4 win[2 * kResWinVecs];
+    __shared__ uint4 records[2 * kRecordRoom];
 
-    const int part = xcd_logical_block(blockIdx.x, gridDim.x);
-    const int chunk = part / kResParts;
-    if (chunk >= plan_residue_chunks(m2)) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int group = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
-    const PlannedChunk& pc = rows[chunk];
-    struct { int w0, wn; } d = {pc.w0, pc.wn};
-    if (d.wn <= 0) return; // the standard kernel has this chunk
-    const int local = (part % kResParts) * kResRows + group; // this lane group's row of the chunk
-    const size_t row_bytes = (size_t)n * sizeof(T);
-    const int tiles = (n + TW - 1) / TW;
-    RODE_PHASE_BEGIN;
-
-    // first tile of the window on its way while the row is loaded
-    uint4 pf[kResPrefetch];
-    {
-        const bool ok = !EDGE || ls * VEC < n;
-        res_prefetch(pf, reinterpret_cast<const char*>(B + (size_t)d.w0 * n + (ok ? ls * VEC : 0)), row_bytes, d.wn, ok);
-    }
-    ResidueRow<false> rr;
-    float* my_v = lds_val + group * kResValStride;
-    load_planned_row(pc, local, owned_slots, val, my_v, rr);
-    const int wave_quads = wave_max_quads(rr.quads);
-    const bool wave_all_hit = __ballot(rr.missmask != 0) == 0ull;
-    RODE_PHASE(0);
-    res_commit(win, pf, d.wn);
-    __syncthreads();
-    RODE_PHASE(1);
-
+    const ChunkWalk walk(m2);
+    int chunk = walk.from(rows, walk.at);
+    if (chunk >= walk.end) return;
+    const int tiles = (n + TW - 1) / TW; // at least two
     const char* win_bytes = reinterpret_cast<const char*>(win);
-    for (int tile = 0; tile < tiles; ++tile) {
-        const int col_off = tile * TW + ls * VEC;
-        const bool col_ok = !EDGE || col_off < n;
-        const T* b_lane = B + (col_ok ? col_off : 0);
-        const bool more = tile + 1 < tiles;
-        if (more) {
-            const int next_off = col_off + TW;
-            const bool ok = !EDGE || next_off < n;
-            res_prefetch(pf, reinterpret_cast<const char*>(B + (size_t)d.w0 * n + (ok ? next_off : 0)), row_bytes, d.wn, ok);
-        }
-        __builtin_amdgcn_sched_barrier(0); // the loads above are issued before the work below, not after it
-        float acc[VEC];
-#pragma unroll
-        for (int x = 0; x < VEC; ++x) acc[x] = 0.f;
-        // (the miss path's inputs are made opaque per tile: otherwise the compiler computes
-        // every position's test and memory address once, outside the tile loop, and holds
-        // them in registers of their own - more than there are)
-        int first_t = rr.first;
-        unsigned miss_t = rr.missmask;
-        if (!wave_all_hit) asm volatile("" : "+v"(first_t), "+v"(miss_t));
+    const unsigned win_lds = lds_address(win), rec_lds = lds_address(records);
+
+    auto window = [&](int w0, int wn, int tile, int buf) __attribute__((always_inline)) {
+        const unsigned at = EDGE && tile * TW + ls * VEC >= n ? 0u : ls * 16u; // (lanes past the last column write nothing)
+        fetch_window(win_lds + buf * kResWinVecs * 16, B + (size_t)w0 * n + tile * TW, (unsigned)n * (unsigned)sizeof(T), wn, at, wave);
+    };
+    auto record = [&](int rec) __attribute__((always_inline)) -> const PlannedChunk& {
+        return *reinterpret_cast<const PlannedChunk*>(records + rec * kRecordRoom);
+    };
+    // a row's values lie in the quads of its group: position 4 q + j in lane j
+    const int lane_of_quad = ls % 4;
+    auto own_values = [&](const PlannedChunk& pc, A (&v)[QUADS]) __attribute__((always_inline)) {
+        const int4 meta = *reinterpret_cast<const int4*>(&pc.meta[group]);
 #pragma unroll
         for (int q = 0; q < QUADS; ++q) {
-            if (q < wave_quads) { // the same for every lane of the wave
-                const float4 v4 = *reinterpret_cast<const float4*>(my_v + 4 * q);
-                const float v[4] = {v4.x, v4.y, v4.z, v4.w};
-                uint4 raw[4];
+            const int pos = 4 * q + lane_of_quad;
+            v[q] = meta.x >= 0 && pos < (meta.z & 0xff) ? val[meta.y + planned_slot(pc, group, pos)] : A(0);
+        }
+    };
+
+    int w0 = rows[chunk].w0, wn = rows[chunk].wn;
+    fetch_record(rec_lds, rows + chunk, wave);
+    window(w0, wn, 0, 0);
+    copies_done();
+    __syncthreads();
+    A v_next[QUADS];
+    own_values(record(0), v_next);
+    int rec = 0, buf = 0;
+    // a tile's results, written during the next one: nobody waits for the stores then
+    A result[VEC];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) raw[j] = *reinterpret_cast<const uint4*>(win_bytes + rr.addr[4 * q + j]);
-                if (!wave_all_hit) {
+    for (int x = 0; x < VEC; ++x) result[x] = A(0);
+    A* result_at = nullptr;
+    bool result_adds = false;
+    auto write_result = [&]() __attribute__((always_inline)) {
+        if (result_at == nullptr) return;
+        if (result_adds) {
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) atomicAdd(result_at + x, result[x]);
+        } else {
+            store_row<VEC>(result_at, result);
+        }
+    };
+
+    while (true) {
+        const int after = walk.from(rows, chunk + walk.stride);
+        const bool last = after >= walk.end;
+        const int after_w0 = last ? 0 : rows[after].w0, after_wn = last ? 0 : rows[after].wn;
+        ResidueRow rr;
+        A v[QUADS];
+        int wave_quads = 0;
+        bool wave_all_hit = true;
+        for (int tile = 0; tile < tiles; ++tile) {
+            copies_done();
+            __syncthreads(); // this tile (and the chunk's record) is in LDS, and every wave is done with the one before
+            if (tile == 0) {
+                decode_planned_row(record(rec), group, owned_slots, rr);
+                wave_quads = wave_max_quads((rr.cnt + 3) / 4);
+                wave_all_hit = __ballot(rr.missmask != 0) == 0ull;
+#pragma unroll
+                for (int q = 0; q < QUADS; ++q) {
+                    v[q] = v_next[q];
+                    asm volatile("" : "+v"(v[q])); // waited for here, before the copies below
+                }
+                if (!last) fetch_record(rec_lds + (rec ^ 1) * kRecordRoom * 16, rows + after, wave);
+            }
+            if (tile + 1 < tiles) {
+                window(w0, wn, tile + 1, buf ^ 1);
+            } else if (!last) {
+                window(after_w0, after_wn, 0, buf ^ 1);
+                own_values(record(rec ^ 1), v_next);
+            }
+            write_result();
+            __builtin_amdgcn_sched_barrier(0); // the loads above are issued before the work below, not after it
+            const int col_off = tile * TW + ls * VEC;
+            const bool col_ok = !EDGE || col_off < n;
+            const T* b_lane = B + (col_ok ? col_off : 0);
+            A acc[VEC];
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) acc[x] = A(0);
+            const unsigned base = (unsigned)buf << 16;
+            int first_t = rr.first;
+            unsigned miss_t = rr.missmask;
+            // (opaque: not the tests and addresses of all positions, computed once and held in registers)
+            if (!wave_all_hit) asm volatile("" : "+v"(first_t), "+v"(miss_t));
+#pragma unroll
+            for (int q = 0; q < QUADS; ++q) {
+                if (q < wave_quads) { // the same for every lane of the wave
+                    uint4 raw[4];
+#pragma unroll
+                    for (int j = 0; j < 4; j += 2) {
+                        unsigned pair = rr.addr[2 * q + j / 2];
+                        asm volatile("" : "+v"(pair)); // unpacked here, per tile, not once for all tiles
+                        raw[j] = *reinterpret_cast<const uint4*>(win_bytes + window_offset<0>(pair, base));
+                        raw[j + 1] = *reinterpret_cast<const uint4*>(win_bytes + window_offset<1>(pair, base));
+                    }
+                    if (!wave_all_hit) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if ((miss_t >> (4 * q + j)) & 1u) { // outside the window: the row of B from memory
+                                const int c = col[first_t + planned_slot(record(rec), group, 4 * q + j)];
+                                raw[j] = *reinterpret_cast<const uint4*>(b_lane + (size_t)c * n);
+                            }
+                    }
+                    const A v4[4] = {of_quad<0>(v[q]), of_quad<1>(v[q]), of_quad<2>(v[q]), of_quad<3>(v[q])};
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        if ((miss_t >> (4 * q + j)) & 1u) {
-                            // outside the window: the slot's column, then the row of B from memory
-                            const int c = col[first_t + planned_slot(pc, local, 4 * q + j)];
-                            raw[j] = *reinterpret_cast<const uint4*>(b_lane + (size_t)c * n);
-                        }
+                        A b[VEC];
+                        unpack_dense<T>(raw[j], b);
+#pragma unroll
+                        for (int x = 0; x < VEC; ++x) acc[x] = fma(v4[j], b[x], acc[x]);
                     }
                 }
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    float b[VEC];
-                    DenseVec<T>::unpack(raw[j], b);
-#pragma unroll
-                    for (int x = 0; x < VEC; ++x) acc[x] = fmaf(v[j], b[x], acc[x]);
-                }
             }
-        }
-        if (rr.row >= 0 && col_ok) {
-            float* c_lane = C + (size_t)rr.row * n + col_off;
-            if (rr.accumulate) {
-                if (rr.quads > 0) {
+            // a listed row without slots of its own (empty, unaligned start) is stored as zeros
+            result_adds = rr.accumulate;
+            result_at = rr.row >= 0 && col_ok && (rr.cnt > 0 || !rr.accumulate) ? C + (size_t)rr.row * n + col_off : nullptr;
 #pragma unroll
-                    for (int x = 0; x < VEC; ++x) atomicAdd(c_lane + x, acc[x]);
-                }
-            } else {
-                // a listed row without slots of its own (empty, unaligned start) is stored as zeros
-                const bool any = rr.quads > 0;
-#pragma unroll
-                for (int x = 0; x < VEC; x += 4)
-                    *reinterpret_cast<float4*>(c_lane + x) = make_float4(any ? acc[x] : 0.f, any ? acc[x + 1] : 0.f,
-                                                                         any ? acc[x + 2] : 0.f, any ? acc[x + 3] : 0.f);
-            }
+            for (int x = 0; x < VEC; ++x) result[x] = rr.cnt > 0 ? acc[x] : A(0);
+            buf ^= 1;
         }
-        RODE_PHASE(2);
-        if (more) {
-            __syncthreads(); // every wave is done with this tile's window
-            RODE_PHASE(3);
-            res_commit(win, pf, d.wn);
-            __syncthreads();
-            RODE_PHASE(4);
-        }
+        if (last) break;
+        chunk = after;
+        w0 = after_w0;
+        wn = after_wn;
+        rec ^= 1;
     }
-    RODE_PHASE_END;
+    write_result();
 }
 
 } // namespace
 
-// The window kernel over the planned chunks of the residue list.  T = float or __half.
+// The window kernel over the planned chunks of the residue list, for dense rows of more than one tile.
 template <typename T>
-hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const float* val, const T* B, float* C,
-                              const int* plan, const void* plan_rows, hipStream_t stream)
+hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
+                              typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
-    const int g = grid_for_residue_parts(m2);
-    const PlannedChunk* rows = static_cast<const PlannedChunk*>(plan_rows);
-    if (((size_t)n * sizeof(T)) % (kResLanes * 16) != 0)
-        spmm_residue_window_kernel<T, true><<<g, kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, rows);
-    else
-        spmm_residue_window_kernel<T, false><<<g, kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, rows);
+    if ((size_t)n * sizeof(T) <= kResLanes * 16) return hipErrorInvalidValue;
+    auto kernel = ((size_t)n * sizeof(T)) % (kResLanes * 16) != 0 ? spmm_residue_window_kernel<T, true> : spmm_residue_window_kernel<T, false>;
+    kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
     return hipGetLastError();
 }
 
-template hipError_t spmm_window_launch<float>(int, int, int, const int*, const float*, const float*, float*, const int*,
-                                              const void*, hipStream_t);
-template hipError_t spmm_window_launch<__half>(int, int, int, const int*, const float*, const __half*, float*,
-                                               const int*, const void*, hipStream_t);
+template hipError_t spmm_window_launch<float>(int, int, int, const int*, const float*, const float*, float*, const int*, const void*, hipStream_t);
+template hipError_t spmm_window_launch<double>(int, int, int, const int*, const double*, const double*, double*, const int*, const void*, hipStream_t);
+template hipError_t spmm_window_launch<__half>(int, int, int, const int*, const float*, const __half*, float*, const int*, const void*, hipStream_t);
 
 } // namespace rode

@@ -203,6 +203,32 @@ __device__ __forceinline__ void spmm_gather_pairs(const T* __restrict__ b_lane, 
     }
 }
 
+// A row of C that is written once and not read again by the kernel that writes it: stored
+// with the non-temporal hint, so that it does not push the gathered rows of B out of the
+// caches on its way (config 4, K=128: residue kernel 1.19 -> 1.09 ms; the same hint on the
+// loads of B, on SDDMM's loads of rhs or on its stores of `out` made those kernels slower).
+template <int VEC>
+__device__ __forceinline__ void store_row(float* dst, const float (&acc)[VEC])
+{
+    typedef float Quad __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int x = 0; x < VEC; x += 4) {
+        const Quad v = {acc[x], acc[x + 1], acc[x + 2], acc[x + 3]};
+        __builtin_nontemporal_store(v, reinterpret_cast<Quad*>(dst + x));
+    }
+}
+
+template <int VEC>
+__device__ __forceinline__ void store_row(double* dst, const double (&acc)[VEC])
+{
+    typedef double Pair __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int x = 0; x < VEC; x += 2) {
+        const Pair v = {acc[x], acc[x + 1]};
+        __builtin_nontemporal_store(v, reinterpret_cast<Pair*>(dst + x));
+    }
+}
+
 // ---- attention ----------------------------------------------------------------
 // What a kernel leaves behind for the gradient.
 enum Keep : int {

@@ -2,204 +2,144 @@
 // rode_sddmm_window.hip): the kernels for chunks of the residue list whose dense rows
 // cluster in a window of consecutive rows (see the locality plan in rode_items.hpp).
 //
-// Shape of both kernels.  A workgroup of 512 threads takes 64 consecutive residue rows
-// (half a chunk of the plan), one group of 8 lanes per row, and walks the dense operand in
-// column tiles of 128 bytes (32 fp32 / 64 fp16 columns).  Per tile it copies the rows
-// [w0, w0 + wn) of the operand - the chunk's window - into LDS with coalesced 128-bit
-// loads, once (the loads of the next tile are issued before the current tile is worked
-// on), and every nonzero slot whose column falls into the window reads its dense row from
-// LDS (8 lanes x ds_read_b128, one contiguous 128-byte row per lane group) instead of
-// gathering it from L2; a slot outside the window is gathered from memory as before.
-// LDS (77 KB) and registers (128) are sized so that two workgroups share a CU: while one
-// waits for memory the other computes.  The lanes of a group keep the LDS address of every
-// slot's dense row in registers for all tiles, so a slot costs one ds_read_b128 plus its
-// multiply-adds.  Which window row a slot reads is not worked out here: the plan holds it
-// for every residue row of a chunk with a window (PlannedChunk), in an order that keeps
-// lane groups that meet in the LDS banks on rows of different parity.
+// Shape of both kernels.  A workgroup of 1024 threads per CU walks chunks of the plan (128
+// consecutive residue rows), one group of 8 lanes per row, and for each chunk the column tiles
+// of 128 bytes (32 fp32, 64 fp16, 16 fp64 columns) of the dense operand.  Per tile the rows
+// [w0, w0 + wn) of the operand - the chunk's window - are copied into LDS once, and every
+// nonzero slot whose column falls into the window reads its dense row there (8 lanes x
+// ds_read_b128, one contiguous 128-byte row per lane group) instead of gathering it from L2; a
+// slot outside the window is gathered from memory.  Which window row a slot reads is not worked
+// out here: the plan holds it for every residue row of a chunk with a window (PlannedChunk), in
+// an order that keeps lane groups that meet in the LDS banks on rows of different parity.
+//
+// What bounds them: for 128 columns of fp32, memory (the operands once, 80 % of a large copy's
+// rate) and the work on a tile (LDS reads and multiply-adds) take about as long as each other, so
+// everything is there to have both going all the time.  The copies go from memory to LDS without
+// registers in between, a tile ahead of the work (the next chunk's first tile during the last of
+// this one, and its record during the first); two windows and two records fill the LDS of a CU, hence
+// the one workgroup, which stays and takes chunk after chunk.  Measured on the banded benchmark
+// (1 M rows, band of 256) against two workgroups of 512 threads per CU that each took half a chunk and
+// loaded a tile between two barriers: SDDMM of width 128 0.531 -> 0.388 ms, width 64 0.361 -> 0.246, 500 K rows
+// of 128 halves 0.217 -> 0.141.  Of the 0.388 the work alone would take 0.301 and the copies alone 0.304.
+// Tried: LDS reads of the next four slots between the multiply-adds of these (0.465).
 #pragma once
 #include "rode_items.hpp"
 
-#ifdef RODE_PHASE_TIMING
-// Debug builds only: cycles spent per phase, summed over workgroups.
-static __device__ unsigned long long rode_phase_clk[8];
-#ifdef RODE_PHASE_READER
-extern "C" void rode_phase_read(unsigned long long* out, int reset)
-{
-    (void)hipMemcpyFromSymbol(out, HIP_SYMBOL(rode_phase_clk), sizeof(unsigned long long) * 8);
-    if (reset) {
-        unsigned long long z[8] = {0};
-        (void)hipMemcpyToSymbol(HIP_SYMBOL(rode_phase_clk), z, sizeof(z));
-    }
-}
-#endif
-#define RODE_PHASE(i)                                                                    \
-    do {                                                                                 \
-        const unsigned now_ = (unsigned)__builtin_readcyclecounter();                    \
-        phase_acc_[i] += now_ - phase_t_;                                                \
-        phase_t_ = now_;                                                                 \
-    } while (0)
-#define RODE_PHASE_BEGIN                                                                 \
-    unsigned phase_acc_[5] = {0, 0, 0, 0, 0};                                            \
-    unsigned phase_t_ = (unsigned)__builtin_readcyclecounter()
-#define RODE_PHASE_END                                                                   \
-    do {                                                                                 \
-        if (threadIdx.x == 0)                                                            \
-            for (int i_ = 0; i_ < 5; ++i_) atomicAdd(&rode_phase_clk[i_], (unsigned long long)phase_acc_[i_]); \
-    } while (0)
-#else
-#define RODE_PHASE(i)
-#define RODE_PHASE_BEGIN
-#define RODE_PHASE_END
-#endif
-
 namespace rode {
 
-constexpr int kResThreads = 512;
-constexpr int kResLanes = 8;                              // lanes per residue row: 8 x 16 bytes = one 128-byte tile row
-constexpr int kResRows = kResThreads / kResLanes;         // residue rows per workgroup
-constexpr int kResParts = kPlanResidueChunk / kResRows;   // workgroups per chunk of the plan
-constexpr int kResWinVecs = kResidueWindowRowsMax * kResLanes;                 // 16-byte pieces of a window
-constexpr int kResPrefetch = (kResWinVecs + kResThreads - 1) / kResThreads;    // pieces one thread moves per tile
-// A group's 32 values in LDS are 36 floats apart: the eight groups of a wave read their
-// float4 of the same quad from eight different sets of banks (32 apart, four groups would
-// share each set).
-constexpr int kResValStride = kBlockItems + 4;
-static_assert(kPlanResidueChunk % kResRows == 0, "a workgroup takes a whole fraction of a chunk");
-static_assert(kResWinVecs * 16 <= 65536, "an LDS address of the window fits 16 bits");
+constexpr int kResLanes = 8;                                   // lanes per residue row: 8 x 16 bytes = one 128-byte tile row
+constexpr int kResThreads = kPlanResidueChunk * kResLanes;     // a workgroup takes a chunk
+constexpr int kResWgs = 256;                                   // one per CU
+constexpr int kResWinVecs = kResidueWindowRowsMax * kResLanes; // 16-byte pieces of a window
+constexpr int kRecordVecs = (int)sizeof(PlannedChunk) / 16;    // ... of a chunk's record
+constexpr int kRecordRoom = (kRecordVecs + kWave - 1) / kWave * kWave; // (a wave copies 64 pieces, needed or not)
+static_assert(kResThreads <= 1024, "a workgroup");
+static_assert(kResWinVecs * 16 == 65536, "the buffer of a window is a bit above its 16-bit addresses");
+static_assert((2 * kResWinVecs + 2 * kRecordRoom) * 16 <= 160 * 1024, "LDS of a CU");
 static_assert(kResidueWindowRowsMax == 512 && kBlockItems == 32, "a plan entry holds 9 bits of window row and 5 of slot");
 
-inline int grid_for_residue_parts(int m2)
-{
-    const int parts = plan_residue_chunks(m2) * kResParts;
-    return (parts + kXcds - 1) / kXcds * kXcds; // xcd_logical_block needs a multiple of kXcds
-}
+inline int window_grid(int m2) { return min(kResWgs, (plan_residue_chunks(m2) + kXcds - 1) / kXcds * kXcds); }
 
-// Issues this thread's loads of one column tile of the window rows [0, wn): src_lane
-// points at this lane's 16 bytes of the first row, rows are row_bytes apart.  Lanes with
-// !ok (past the last column of an edge tile) get zeros.
-__device__ __forceinline__ void res_prefetch(uint4 (&pf)[kResPrefetch], const char* src_lane, size_t row_bytes, int wn,
-                                             bool ok)
-{
-    constexpr int RS = kResThreads / kResLanes;
-    const int r0 = threadIdx.x / kResLanes;
-#pragma unroll
-    for (int u = 0; u < kResPrefetch; ++u) {
-        pf[u] = make_uint4(0, 0, 0, 0);
-        if (ok && r0 + u * RS < wn) pf[u] = *reinterpret_cast<const uint4*>(src_lane + (size_t)(r0 + u * RS) * row_bytes);
+// The chunks of one workgroup: a contiguous share of the list per XCD, adjacent chunks to its
+// workgroups at the same time (their windows overlap), chunks without a window left out.
+struct ChunkWalk {
+    int at, end, stride;
+    __device__ __forceinline__ ChunkWalk(int m2)
+    {
+        const int chunks = plan_residue_chunks(m2), share = (chunks + kXcds - 1) / kXcds, xcd = blockIdx.x % kXcds;
+        at = xcd * share + blockIdx.x / kXcds;
+        end = min(chunks, (xcd + 1) * share);
+        stride = gridDim.x / kXcds;
     }
-}
-
-__device__ __forceinline__ void res_commit(uint4* win, const uint4 (&pf)[kResPrefetch], int wn)
-{
-    constexpr int RS = kResThreads / kResLanes;
-    const int r0 = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
-#pragma unroll
-    for (int u = 0; u < kResPrefetch; ++u)
-        if (r0 + u * RS < wn) win[(r0 + u * RS) * kResLanes + ls] = pf[u];
-}
-
-// Copies one column tile of the window rows [0, wn) from memory into LDS without keeping
-// it in registers meanwhile (for a kernel that has none to spare).
-__device__ __forceinline__ void res_fill(uint4* win, const char* src_lane, size_t row_bytes, int wn, bool ok)
-{
-    constexpr int RS = kResThreads / kResLanes, U = 4;
-    const int r0 = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
-    for (int r = r0; r < wn; r += U * RS) {
-        uint4 v[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            v[u] = make_uint4(0, 0, 0, 0);
-            if (ok && r + u * RS < wn) v[u] = *reinterpret_cast<const uint4*>(src_lane + (size_t)(r + u * RS) * row_bytes);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (r + u * RS < wn) win[(r + u * RS) * kResLanes + ls] = v[u];
+    // the first one with a window from c on (end or later: none)
+    __device__ __forceinline__ int from(const PlannedChunk* __restrict__ rows, int c) const
+    {
+        while (c < end && rows[c].wn <= 0) c += stride; // (the standard kernel has those)
+        return c;
     }
+};
+
+__device__ __forceinline__ unsigned lds_address(const void* p)
+{
+    return (unsigned)(size_t)(const __attribute__((address_space(3))) char*)p;
+}
+
+// Copies 16 bytes per lane from base + offset to LDS at lds + 16 * lane, without a register in
+// between.  The compiler does not know of the copy: copies_done waits for all of the wave's.
+__device__ __forceinline__ void copy_to_lds(unsigned lds, const void* base, unsigned offset)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(offset), "s"(base) : "memory", "m0");
+}
+__device__ __forceinline__ void copies_done()
+{
+    __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+}
+
+// A chunk's record to LDS.
+__device__ __forceinline__ void fetch_record(unsigned lds, const PlannedChunk* chunk, int wave)
+{
+    if (wave * kWave < kRecordVecs) copy_to_lds(lds + wave * kWave * 16, chunk, min((int)threadIdx.x, kRecordVecs - 1) * 16);
+}
+
+// One column tile of the window rows [0, wn) to LDS: `tile` points at it in the first row, rows are
+// row_bytes apart, `at` is this lane's 16 bytes of a row (any valid place of it for a lane past the last column).
+__device__ __forceinline__ void fetch_window(unsigned lds, const void* tile, unsigned row_bytes, int wn, unsigned at, int wave)
+{
+#pragma unroll
+    for (int u = 0; u < kResidueWindowRowsMax / kPlanResidueChunk; ++u)
+        if (u * kPlanResidueChunk + wave * (kWave / kResLanes) < wn) // (a wave's rows past the window: its last one again)
+            copy_to_lds(lds + (u * kResThreads + wave * kWave) * 16, tile,
+                        (unsigned)min(u * kPlanResidueChunk + (int)threadIdx.x / kResLanes, wn - 1) * row_bytes + at);
 }
 
 // One residue row as its lane group keeps it: cnt slots at positions 0 .. cnt - 1 (the order
 // of the plan), the rest of the 32 positions carry value 0.
-// addr[i]: LDS byte address of this lane's 16 bytes of the dense row of position i; for a
-// position whose dense row is outside the window (bit i of missmask) it is the address of
+// addr[i]: the offsets in a window of this lane's 16 bytes of the dense rows of positions 2 i (low half)
+// and 2 i + 1; for a position whose dense row is outside the window (its bit of missmask) it is that of
 // one of the row's positions that is inside, and the data has to come from memory instead.
-// PACKED: two addresses (each below 64 K) per register, position 2 i in the low half of
-// addr[i] and 2 i + 1 in the high half - for a kernel that needs the 16 registers elsewhere
-// and pays one extra instruction per read for it.
-template <bool PACKED>
 struct ResidueRow {
     int row;   // -1: nothing to do
     int first; // first residue slot of the row in column_indices / values
-    int cnt, quads;
+    int cnt;
     unsigned missmask;
     bool accumulate; // the row also has block segments (SpMM adds instead of storing)
-    unsigned addr[PACKED ? kBlockItems / 2 : kBlockItems];
+    unsigned addr[kBlockItems / 2];
 };
 
-// The slot (counted from rr.first) that the plan put at position i of row `local` of a chunk.
+// The slot (counted from its row's first) that the plan put at position i of row `local` of a chunk.
 __device__ __forceinline__ int planned_slot(const PlannedChunk& pc, int local, int i)
 {
     return (pc.entry[local][i] >> 9) & (kBlockItems - 1);
 }
 
-// Turns a row record of the plan and the row's 32 entries into the lane group's view of
-// the row (everything but the values).  skip_owned_slots: rows with block segments and at
-// most that many aligned slots are left to the block kernel (SpMM under the whole-lists
-// promise); 0 for SDDMM.  usable = false: the chunk has no window (its records are not
-// filled in), the row is skipped.
-template <bool PACKED>
-__device__ __forceinline__ void decode_planned_row(const int4& meta, const uint4 (&e4)[kBlockItems / 8], bool usable,
-                                                   int skip_owned_slots, ResidueRow<PACKED>& rr)
-{
-    const int ls = threadIdx.x % kResLanes;
-    rr.row = meta.x;
-    rr.first = meta.y;
-    rr.cnt = meta.z & 0xff;
-    rr.accumulate = (meta.z >> 8) & 1;
-    rr.missmask = (unsigned)meta.w;
-    if (!usable || rr.row < 0 || (rr.accumulate && ((meta.z >> 16) & 0xffff) <= skip_owned_slots)) {
-        rr.row = -1;
-        rr.first = 0;
-        rr.cnt = 0;
-        rr.missmask = 0;
-    }
-    rr.quads = (rr.cnt + 3) / 4;
-#pragma unroll
-    for (int i = 0; i < kBlockItems / 8; ++i) {
-        const unsigned w[4] = {e4[i].x, e4[i].y, e4[i].z, e4[i].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const unsigned even = (((w[j] & 0xffffu) & (kResidueWindowRowsMax - 1)) * kResLanes + ls) * 16;
-            const unsigned odd = (((w[j] >> 16) & (kResidueWindowRowsMax - 1)) * kResLanes + ls) * 16;
-            if (PACKED) {
-                rr.addr[4 * i + j] = even | (odd << 16);
-            } else {
-                rr.addr[8 * i + 2 * j] = even;
-                rr.addr[8 * i + 2 * j + 1] = odd;
-            }
-        }
-    }
-}
-
-// Loads row `local` of a planned chunk for this lane group: the LDS addresses of its 32
-// positions into registers, its values (in position order, 0 past the row) into `my_val`
-// (32 floats of this group; the 8 lanes write 4 each).
-template <bool PACKED>
-__device__ __forceinline__ void load_planned_row(const PlannedChunk& pc, int local, int skip_owned_slots,
-                                                 const float* __restrict__ val, float* my_val, ResidueRow<PACKED>& rr)
+// The lane group's view of its row (everything but the values).  skip_owned_slots: rows with block
+// segments and at most that many aligned slots are left to the block kernel (SpMM under the whole-lists
+// promise); 0 for SDDMM.
+__device__ __forceinline__ void decode_planned_row(const PlannedChunk& pc, int local, int skip_owned_slots, ResidueRow& rr)
 {
     const int ls = threadIdx.x % kResLanes;
     const int4 meta = *reinterpret_cast<const int4*>(&pc.meta[local]);
-    const uint4* entries = reinterpret_cast<const uint4*>(pc.entry[local]);
-    uint4 e4[kBlockItems / 8];
+    const bool mine = meta.x >= 0 && !(((meta.z >> 8) & 1) && ((meta.z >> 16) & 0xffff) <= skip_owned_slots);
+    rr.row = mine ? meta.x : -1;
+    rr.first = mine ? meta.y : 0;
+    rr.cnt = mine ? meta.z & 0xff : 0;
+    rr.accumulate = (meta.z >> 8) & 1;
+    rr.missmask = mine ? (unsigned)meta.w : 0u;
 #pragma unroll
-    for (int i = 0; i < kBlockItems / 8; ++i) e4[i] = entries[i];
-    decode_planned_row(meta, e4, true, skip_owned_slots, rr);
-    constexpr int OWN = kBlockItems / kResLanes;
+    for (int i = 0; i < kBlockItems / 8; ++i) {
+        const uint4 e = reinterpret_cast<const uint4*>(pc.entry[local])[i];
+        const unsigned w[4] = {e.x, e.y, e.z, e.w};
 #pragma unroll
-    for (int i = 0; i < OWN; ++i) {
-        const int pos = ls + i * kResLanes;
-        my_val[pos] = pos < rr.cnt ? val[rr.first + planned_slot(pc, local, pos)] : 0.f;
+        for (int j = 0; j < 4; ++j) // two entries at once
+            rr.addr[4 * i + j] = ((w[j] & (0x10001u * (kResidueWindowRowsMax - 1))) * (kResLanes * 16)) | (0x10001u * 16 * ls);
     }
+}
+
+// Where position 2 i (odd = 0) or 2 i + 1 of a row is in the two windows: addr[i] unpacked, the buffer put above it.
+template <int ODD>
+__device__ __forceinline__ unsigned window_offset(unsigned pair, unsigned buffer_bit)
+{
+    return __builtin_amdgcn_perm(buffer_bit, pair, ODD ? 0x07060302u : 0x07060100u);
 }
 
 // Longest row (in slot quads) among the 8 lane groups of the wave, as a scalar: quads at
