@@ -12,6 +12,7 @@
 
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
+#include <ATen/ops/zeros.h>
 #include <c10/core/GradMode.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -260,9 +261,9 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
     Py_BEGIN_ALLOW_THREADS
     try {
         list_sizes(static_cast<const int32_t*>(host->data_ptr()), m, (int)seg, m1, m2);
-        blk = at::empty({std::max(m1, 1ll)}, dev->options());
+        blk = m1 > 0 ? at::empty({m1}, dev->options()) : at::zeros({1}, dev->options()); // (an empty list has one place that is never read)
         start = at::empty({m1 + 1}, dev->options());
-        res = at::empty({std::max(m2, 1ll)}, dev->options());
+        res = m2 > 0 ? at::empty({m2}, dev->options()) : at::zeros({1}, dev->options());
         const size_t ws_bytes = rode_hip_preprocess_workspace_bytes((int)m);
         scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
         // (pinned: the kernels write the counts where the host reads them)
