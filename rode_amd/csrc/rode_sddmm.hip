@@ -30,8 +30,11 @@ namespace {
 // [base, base + cnt) of one row, 64 slots per step; the first `mask` slots (the previous
 // row's) are computed but not stored.
 // (split, jump: the slots are [base, base + split) followed by [base + split + jump, ...):
-// a row with a hole that somebody else works on; split >= cnt for one plain range.)
-template <typename T, int KT, int NS, bool EDGE>
+// a row with a hole that somebody else works on; split >= cnt for one plain range.
+// AHEAD: the next step's columns and values are on their way while this one's dense rows arrive.  Costs a
+// quarter of the waves in registers: for rows of many steps on a full GPU (power-law benchmark, 64 halves:
+// 0.956 -> 0.943 ms; 300 K rows of width 128: 0.647 -> 0.637), not for small matrices (14 K rows of 40: 24.7 -> 26.1 us).)
+template <typename T, int KT, int NS, bool EDGE, bool AHEAD>
 __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int cnt, int split, int jump, int k, int lane,
                                                 int* lds_cols,
                                                 const int* __restrict__ col, const float* __restrict__ val,
@@ -43,20 +46,32 @@ __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int
     load_lhs_slice<T, KT, NS, EDGE>(lhs, row, k, lane, a);
     const T* rhs_lane = rhs + (lane % S::kLpr) * S::kVec;
 
-    for (int off = 0; off < cnt; off += kWave) {
+    // cnt is a multiple of 32 for every decomposition the kernels are specified for
+    // (segment length a multiple of 32).  Lists made with another segment length must
+    // still never make a lane read or write beyond its row's block part: such lanes
+    // repeat the last slot and store nothing.
+    auto index_of = [&](int slot) __attribute__((always_inline)) {
+        const int at = min(slot, cnt - 1);
+        return base + at + (at >= split ? jump : 0);
+    };
+    int c = 0, idx = 0;
+    float v = 0.f;
+    auto fetch = [&](int off) __attribute__((always_inline)) {
         if (off + (lane & 32) < cnt) { // the upper half sits out a trailing 32-slot step
-            const int slot = off + lane;
-            // cnt is a multiple of 32 for every decomposition the kernels are specified for
-            // (segment length a multiple of 32).  Lists made with another segment length must
-            // still never make a lane read or write beyond its row's block part: such lanes
-            // repeat the last slot and store nothing.
-            const bool live = slot < cnt;
-            const int at = live ? slot : cnt - 1;
-            const int idx = base + at + (at >= split ? jump : 0);
-            const int c = col[idx];
-            const float v = val[idx];
-            const float d = sddmm_unit<T, KT, NS, EDGE>(rhs_lane, a, c, k, lds_cols, lane);
-            if (slot >= mask && live) out[idx] = v * d;
+            idx = index_of(off + lane);
+            c = col[idx];
+            v = val[idx];
+        }
+    };
+    if (AHEAD) fetch(0);
+    for (int off = 0; off < cnt; off += kWave) {
+        if (!AHEAD) fetch(off);
+        const int slot = off + lane, c_now = c, idx_now = idx;
+        const float v_now = v;
+        if (AHEAD) fetch(off + kWave);
+        if (off + (lane & 32) < cnt) {
+            const float d = sddmm_unit<T, KT, NS, EDGE>(rhs_lane, a, c_now, k, lds_cols, lane);
+            if (slot >= mask && slot < cnt) out[idx_now] = v_now * d;
         }
     }
 }
@@ -66,7 +81,9 @@ __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int
 // (RoDeSddmm.cu:35-54); the first `mask` slots belong to the previous row and are
 // computed but never stored (RoDeSddmm.cu:56-58, 197).
 // (bid of nblocks: the workgroup's position in the part of the grid that works on block segments)
-template <typename T, int KT, int NS, bool EDGE>
+// WALK: 0 one wave per segment only, 1 chunks only (chunk_hint > 1), 2 either, found out here.  (Kernels of their
+// own, so that the code of one way does not cost the other registers.)
+template <typename T, int KT, int NS, bool EDGE, int WALK, bool AHEAD>
 __device__ __forceinline__ void
 sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                  const int* __restrict__ st_off,
@@ -77,9 +94,11 @@ sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     // Lists with short segments, and many of them: a wave walks a chunk of consecutive
     // segments from leader to leader, with windows of kWalkSlots slots (rode_items.hpp).
-    const int chunk = chunk_hint > 0 ? chunk_hint
-                                     : block_chunk_for_grid(m1 >= kWalkMinSegments ? block_chunk(m1, block_rows, st_off) : 1, m1, nblocks);
-    if (chunk > 1) {
+    int chunk = 1;
+    if constexpr (WALK == 1) chunk = chunk_hint;
+    if constexpr (WALK == 2)
+        chunk = block_chunk_for_grid(m1 >= kWalkMinSegments ? block_chunk(m1, block_rows, st_off) : 1, m1, nblocks);
+    if (WALK != 0 && chunk > 1) {
         const long long first = chunk_first_segment(bid, wave, m1, chunk);
         if (first < 0) return;
         const int last = (int)min(first + chunk, (long long)m1);
@@ -88,7 +107,7 @@ sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners 
             const int count = min(last - from, kScanSegments);
             for (unsigned long long todo = scan.items & ((1ull << count) - 1ull); todo; todo &= todo - 1ull) {
                 const BlockItem it = chunk_item(scan, __builtin_ctzll(todo));
-                sddmm_row_slots<T, KT, NS, EDGE>(it.row, it.base, it.mask, it.cnt, it.cnt, 0, k, lane, lds + wave * kWave, col,
+                sddmm_row_slots<T, KT, NS, EDGE, AHEAD>(it.row, it.base, it.mask, it.cnt, it.cnt, 0, k, lane, lds + wave * kWave, col,
                                                  val, lhs, rhs, out);
             }
         }
@@ -107,7 +126,7 @@ sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners 
     if (!sddmm_block_item(seg, m1, owners, lane, block_rows, st_off, row_ptr, it)) return;
     const int row = it.row, mask = it.mask, base = it.base, cnt = it.cnt;
 
-    sddmm_row_slots<T, KT, NS, EDGE>(row, base, mask, cnt, cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
+    sddmm_row_slots<T, KT, NS, EDGE, AHEAD>(row, base, mask, cnt, cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
 }
 
 // One group of LPR lanes per residue row.  Tail selection follows RoDeSddmm.cu:237-243:
@@ -126,7 +145,8 @@ sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const 
     constexpr int RPW = kWave / LPR;          // rows per wave
     constexpr int OWN = kBlockItems / LPR;    // slots owned by one lane
     constexpr int LQ = LPR / 4;               // lane quads per group
-    __shared__ __attribute__((aligned(16))) int lds[kWavesPerWg * RPW * kBlockItems];
+    constexpr int kStride = kBlockItems + 4;  // (the groups of a wave read their slots from LDS banks of their own)
+    __shared__ __attribute__((aligned(16))) int lds[kWavesPerWg * RPW * kStride];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     const int group = lane / LPR, ls = lane % LPR;
     const int item = (xcd_logical_block(bid, nblocks) * kWavesPerWg + wave) * RPW + group;
@@ -139,7 +159,8 @@ sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const 
     if (cnt <= 0) return; // an empty, unaligned row is listed as a residue but owns no slot
     if (owned_elsewhere(owners, row, it.aligned)) return; // another kernel has the whole row
 
-    int* my_cols = lds + (wave * RPW + group) * kBlockItems;
+    int* my_cols = lds + (wave * RPW + group) * kStride;
+    int cols[OWN];
     float v[OWN];
     const int padded = (cnt + 3) & ~3; // slots past the tail repeat its last column
 #pragma unroll
@@ -148,10 +169,13 @@ sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const 
         v[i] = 0.f;
         if (slot < padded) {
             const int idx = first + min(slot, cnt - 1);
-            my_cols[slot] = col[idx];
+            cols[i] = col[idx];
             v[i] = val[idx];
         }
     }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+        if (ls + i * LPR < padded) my_cols[ls + i * LPR] = cols[i];
     typename S::Reg a[NS][S::kRegs];
     load_lhs_slice<T, KT, NS, EDGE, true>(lhs, row, k, lane, a);
     const T* rhs_lane = rhs + ls * VEC;
@@ -186,14 +210,14 @@ sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const 
     }
 }
 
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, bool EDGE, int WALK>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_block_kernel(int m1, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                    const int* __restrict__ st_off,
                    const int* __restrict__ row_ptr, const int* __restrict__ col, const float* __restrict__ val,
                    const T* __restrict__ lhs, const T* __restrict__ rhs, float* __restrict__ out)
 {
-    sddmm_block_body<T, KT, NS, EDGE>(blockIdx.x, gridDim.x, m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val,
+    sddmm_block_body<T, KT, NS, EDGE, WALK, true>(blockIdx.x, gridDim.x, m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val,
                                       lhs, rhs, out);
 }
 
@@ -209,7 +233,7 @@ sddmm_residue_kernel(int m2, int k, RowOwners owners, const int* __restrict__ re
 
 // Both lists in one launch: the first g1 workgroups work on block segments, the others on
 // residue rows.  For matrices so small that a launch costs as much as its kernel.
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, bool EDGE, int WALK>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_pair_kernel(int g1, int m1, int m2, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                   const int* __restrict__ residue_rows,
@@ -218,7 +242,7 @@ sddmm_pair_kernel(int g1, int m1, int m2, int k, int chunk_hint, RowOwners owner
                   float* __restrict__ out, const int* __restrict__ plan)
 {
     if ((int)blockIdx.x < g1)
-        sddmm_block_body<T, KT, NS, EDGE>(blockIdx.x, g1, m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, lhs,
+        sddmm_block_body<T, KT, NS, EDGE, WALK, false>(blockIdx.x, g1, m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, lhs,
                                           rhs, out);
     else
         sddmm_residue_body<T, KT, NS, EDGE>(blockIdx.x - g1, gridDim.x - g1, m2, k, owners, residue_rows, row_ptr, col, val, lhs,
@@ -391,7 +415,7 @@ sddmm_group_kernel(int k, int n_groups, const RowGroup* __restrict__ groups, con
             const int row = row0 + r, s = row_ptr[row], e = row_ptr[row + 1];
             const int run_first = s + d.pos[r], run_end = run_first + d.run(r);
             // (the slots before the run and, in the same pass, those after it)
-            sddmm_row_slots<T, KT, 1, EDGE>(row, s, 0, (run_first - s) + (e - run_end), run_first - s, d.run(r), k, lane,
+            sddmm_row_slots<T, KT, 1, EDGE, false>(row, s, 0, (run_first - s) + (e - run_end), run_first - s, d.run(r), k, lane,
                                             lds + wave * kWave, col, val, lhs, rhs, out);
         }
     }
@@ -414,7 +438,7 @@ sddmm_hub_kernel(int k, int merge, const int* __restrict__ hub, const int* __res
     const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
     const int base = piece[slab], cnt = piece[min(slab + merge, hp.slabs)] - base;
     if (cnt <= 0) return;
-    sddmm_row_slots<T, KT, NS, EDGE>(hp.rows[h], base, 0, cnt, cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
+    sddmm_row_slots<T, KT, NS, EDGE, true>(hp.rows[h], base, 0, cnt, cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
 }
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
@@ -464,12 +488,15 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     }
     if (group_plan && plan.group_counts[2] == 0) m1 = m2 = 0; // every row in a group with a run: nothing for the lists' kernels
     if (m1 > 0 && m2 > 0 && standard_residue && s1 == s2 && g1 + g2 <= kPairMaxWorkgroups) {
-        sddmm_pair_kernel<T, KT, NS, EDGE><<<g1 + g2, kWgThreads, 0, s1>>>(
-            g1, m1, m2, k, chunk_hint, owners, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs, out, plan.dev);
+        auto kernel = chunk_hint == 1 ? sddmm_pair_kernel<T, KT, NS, EDGE, 0> : chunk_hint > 1 ? sddmm_pair_kernel<T, KT, NS, EDGE, 1>
+                                                                                           : sddmm_pair_kernel<T, KT, NS, EDGE, 2>;
+        kernel<<<g1 + g2, kWgThreads, 0, s1>>>(g1, m1, m2, k, chunk_hint, owners, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs,
+                                               out, plan.dev);
     } else {
         if (m1 > 0) {
-            sddmm_block_kernel<T, KT, NS, EDGE><<<g1, kWgThreads, 0, s1>>>(
-                m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, lhs, rhs, out);
+            auto kernel = chunk_hint == 1 ? sddmm_block_kernel<T, KT, NS, EDGE, 0> : chunk_hint > 1 ? sddmm_block_kernel<T, KT, NS, EDGE, 1>
+                                                                                               : sddmm_block_kernel<T, KT, NS, EDGE, 2>;
+            kernel<<<g1, kWgThreads, 0, s1>>>(m1, k, chunk_hint, owners, block_rows, st_off, row_ptr, col, val, lhs, rhs, out);
         }
         if (m2 > 0 && standard_residue) {
             sddmm_residue_kernel<T, KT, NS, EDGE><<<g2, kWgThreads, 0, s2>>>(
