@@ -333,11 +333,7 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
     // fills the GPU; what is left row by row.
     RowOwners owners;
     int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
-    // (the tile kernel addresses a head's k and v with 32-bit offsets; N = 0: not said, one head.  With
-    // fewer tiles than CUs and short rows a wave per row is faster: 128 tiles, 144 nonzeros per row of 128
-    // halves 13 against 15 us; 576 per row 17 against 14 us.)
-    const bool enough = (long long)(groups_left > 0 ? plan.group_counts[3] : 0) * nheads >= 256 || nnz >= 256ll * M;
-    if (groups_left > 0 && plan.group_counts[3] > 0 && enough && attention_tiles_fit(N, D * sizeof(T))) {
+    if (attention_uses_tiles(plan, nheads, M, N, nnz, D * sizeof(T))) {
         owners.tiles = group_plan_tiles(plan.groups, M);
         owners.n_tiles = row_tiles(M);
         groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);

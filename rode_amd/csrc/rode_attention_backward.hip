@@ -118,7 +118,7 @@ attention_backward_rows_kernel(int M, const int* __restrict__ row_ptr, const int
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     const int row = xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
     if (row >= M) return;
-    if (owned_elsewhere(owners, row, 0)) return; // a row of a group: attention_backward_group_kernel has it
+    if (owned_elsewhere(owners, row, 0) || in_tile(owners, row)) return; // a row of a group, or of a tile: other kernels have it
     const int s = row_ptr[row], e = row_ptr[row + 1];
     const int ls = lane % LPR, group = lane / LPR;
     float acc[VEC];
@@ -185,7 +185,7 @@ attention_backward_group_kernel(int n_groups, const RowGroup* __restrict__ group
                                 const float* __restrict__ probs, const float2* __restrict__ stats,
                                 const float* __restrict__ g, const float* __restrict__ out, const T* __restrict__ k,
                                 const T* __restrict__ v, float scale, const int* __restrict__ t_slot,
-                                float* __restrict__ dq, float2* __restrict__ pz, HeadStrides heads)
+                                float* __restrict__ dq, float2* __restrict__ pz, RowOwners owners, HeadStrides heads)
 {
     probs = of_head(probs, heads.nnz), g = of_head(g, heads.rows), out = of_head(out, heads.rows);
     stats = of_head(stats, heads.rows / D);
@@ -199,6 +199,7 @@ attention_backward_group_kernel(int n_groups, const RowGroup* __restrict__ group
     const int grp = xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
     if (grp >= n_groups) return;
     if (groups[grp].len <= 0) return; // not a group: attention_backward_rows_kernel has its rows
+    if (in_tile(owners, grp * kGroupRows)) return; // part of a tile: attention_backward_tile_kernel has its rows
     const RowGroup d = shared_run(groups[grp]); // the columns [lo, lo + len) that all four runs hold
     const int ls = lane % LPR, group = lane / LPR;
     const int row0 = grp * R;
@@ -629,21 +630,38 @@ inline bool use_groups(const PlanRef& plan, int groups_min, RowOwners& owners)
 }
 
 template <typename T, int D>
-hipError_t launch_rows(HeadStrides heads, int nheads, int M, const int* row_ptr, const int* col, const float* val,
+hipError_t launch_rows(HeadStrides heads, int nheads, int M, int N, int nnz, const int* row_ptr, const int* col, const float* val,
                        const float* probs, const float2* stats, const float* g, const float* out, const T* k, const T* v,
                        float scale, const int* t_slot, float* dq, float* pz, PlanRef plan, hipStream_t stream)
 {
     const int wgs = wave_grid(M);
     if (wgs < 0 || nheads > 65535) return hipErrorInvalidConfiguration;
+    // The tiles of a group plan first (the matrix cores), by the forward pass's rule; the other groups when a
+    // wave per group fills the GPU; what is left row by row.
     RowOwners owners;
-    const bool grouped = use_groups(plan, attention_groups_min<T>(), owners);
+    int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
+    if (attention_uses_tiles(plan, nheads, M, N, nnz, D * sizeof(T))) {
+        owners.tiles = group_plan_tiles(plan.groups, M);
+        owners.n_tiles = row_tiles(M);
+        groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);
+        rows_left -= plan.group_counts[3] * kTileRows;
+        const hipError_t e = attention_backward_tiles_launch<T>(nheads, M, N, nnz, D, row_ptr, col, val, probs, reinterpret_cast<const float*>(stats),
+                                                                g, out, k, v, scale, t_slot, dq, pz, plan.groups, stream);
+        if (e != hipSuccess) return e;
+    }
+    const bool grouped = groups_left >= attention_groups_min<T>();
+    if (grouped) {
+        owners.groups = reinterpret_cast<const RowGroup*>(plan.groups + kGroupHeaderInts);
+        owners.n_groups = plan.group_counts[0];
+        rows_left -= groups_left * kGroupRows;
+    }
     float2* pairs = reinterpret_cast<float2*>(pz);
-    if (!(grouped && plan.group_counts[2] == 0)) // (else every row is in a group)
+    if (rows_left > 0)
         attention_backward_rows_kernel<T, D><<<dim3(wgs, nheads), kWgThreads, 0, stream>>>(
             M, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pairs, owners, heads);
     if (grouped)
         attention_backward_group_kernel<T, D><<<dim3(wave_grid(owners.n_groups), nheads), kWgThreads, 0, stream>>>(
-            owners.n_groups, owners.groups, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pairs, heads);
+            owners.n_groups, owners.groups, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pairs, owners, heads);
     return hipGetLastError();
 }
 
@@ -681,9 +699,9 @@ hipError_t attention_backward_rows_launch(int nheads, int M, int N, int nnz, int
     HeadStrides heads;
     heads.rows = (size_t)M * d, heads.cols = (size_t)N * d, heads.nnz = (size_t)nnz;
     switch (d) {
-    case 32: return launch_rows<T, 32>(heads, nheads, M, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
-    case 64: return launch_rows<T, 64>(heads, nheads, M, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
-    case 128: return launch_rows<T, 128>(heads, nheads, M, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
+    case 32: return launch_rows<T, 32>(heads, nheads, M, N, nnz, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
+    case 64: return launch_rows<T, 64>(heads, nheads, M, N, nnz, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
+    case 128: return launch_rows<T, 128>(heads, nheads, M, N, nnz, row_ptr, col, val, probs, stats, g, out, k, v, scale, t_slot, dq, pz, plan, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -61,6 +61,14 @@ hipError_t attention_launch(int nheads, int M, int N, int nnz, int d, const int*
                             PlanRef plan, hipStream_t stream);
 
 constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (size_t)N * row_bytes < (1ull << 32); }
+// Do the tiles of a group plan go to the tile kernels?  (They address a head's k and v with 32-bit offsets; N = 0:
+// not said, one head.  With fewer tiles than CUs and short rows a wave per row is faster: 128 tiles, 144 nonzeros per
+// row of 128 halves 13 against 15 us; 576 per row 17 against 14 us.)
+inline bool attention_uses_tiles(const PlanRef& plan, int nheads, int M, int N, long long nnz, size_t row_bytes)
+{
+    if (plan.groups == nullptr || plan.group_counts == nullptr || plan.group_counts[1] <= 0 || plan.group_counts[3] <= 0) return false;
+    return ((long long)plan.group_counts[3] * nheads >= 256 || nnz >= 256ll * M) && attention_tiles_fit(N, row_bytes);
+}
 // (rode_attention_tile.hip) the rows of a group plan's tiles, the same arguments; plan: the group plan
 template <typename T>
 hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
@@ -78,6 +86,13 @@ hipError_t attention_backward_rows_launch(int nheads, int M, int N, int nnz, int
                                           const float* val, const float* probs, const float* row_stats, const float* g,
                                           const float* out, const T* k, const T* v, float scale, const int* t_slot, float* dq,
                                           float* pz, PlanRef plan, hipStream_t stream);
+// (rode_attention_backward_tile.hip) the row pass for the rows of a group plan's tiles; plan: the group plan
+template <typename T>
+hipError_t attention_backward_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
+                                           const float* probs, const float* row_stats, const float* g, const float* out, const T* k,
+                                           const T* v, float scale, const int* t_slot, float* dq, float* pz, const int* plan,
+                                           hipStream_t stream);
+
 template <typename T>
 hipError_t attention_backward_cols_launch(int nheads, int M, int N, int nnz, int d, const int* t_row_ptr, const int* t_col,
                                           const float* pz, const float* g, const T* q, float* dk, float* dv, PlanRef plan,

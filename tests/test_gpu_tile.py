@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from rode_amd import RoDeCSR, sparse_attention
-from rode_amd.autograd import _attention_call
+from rode_amd.autograd import _attention_backward_call, _attention_call
 
 pytestmark = pytest.mark.gpu
 
@@ -83,3 +83,52 @@ def test_non_finite_rows_of_v_stay_in_their_rows(half):
     assert touched.any() and not touched.all()
     assert not torch.isfinite(out[touched]).all(dim=1).any()
     assert (out[~touched].double() - clean[~touched]).abs().max() <= 2e-5 * clean.abs().max()
+
+
+@pytest.mark.parametrize("m,window,shift,extra,d,half,scale", CASES)
+def test_gradients_on_tiles_against_fp64(m, window, shift, extra, d, half, scale):
+    csr, dense = _mask(m, window, shift, extra, seed=m + window, short_rows=(40,) if m == 160 else ())
+    dt = torch.float16 if half else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    heads = 256
+    q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    q, k, v = (t.to(dt) for t in (q, k, v))
+    g[1] *= 1e-6  # (rows of very different gradients)
+    ins = [t.double().requires_grad_() for t in (q, k, v)]
+    want = torch.autograd.grad(_reference(dense, *ins, scale), ins, g.double())
+    ins = [t.expand(heads, *t.shape).contiguous() for t in (q, k, v)]
+    out, scores, stats = _attention_call(csr, csr.values, *ins, scale, "scores")
+    got = _attention_backward_call(csr, csr.transpose(with_values=False)[0], csr.transposed_slots(), scores, stats,
+                                   g.expand(heads, m, d).contiguous(), out, *ins, scale)
+    of_g = g.double().abs().amax(1, keepdim=True)
+    for a, b in zip(got, want):
+        # (the kernels round g to halves for its products with halves: an error of g's size where one probability is nearly 1)
+        size = b.abs().amax(1, keepdim=True) + (of_g if half and b is want[0] else 0.0) if b is want[0] else b.abs().max()
+        assert ((a[heads - 1].double() - b).abs() / size).max() <= (5e-3 if half else 1e-4)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_gradients_on_tiles_twice_held_column_and_inf(half):
+    """A row that holds a column of its run twice (its slots in the transposed pattern are not the next row's), and a row of
+    k that is not finite and that most rows of its tile do not hold: as without a plan."""
+    m, d, dt = 256, 64, torch.float16 if half else torch.float32
+    csr, _ = _mask(m, 130, 1, 12, seed=5)
+    rp, col = csr.row_offsets.cpu().numpy(), csr.column_indices.cpu().numpy().copy()
+    for row, at in ((21, 100), (40, 80)):  # the columns outside the run name one inside it
+        c = col[rp[row]:rp[row + 1]]
+        out = np.flatnonzero((c < row) | (c >= row + 130))
+        c[out[0]] = row + at
+    args = [torch.from_numpy(rp), torch.from_numpy(col), csr.values.cpu(), "cuda", m, csr.n, 64]
+    tiled, plain = RoDeCSR(*args, locality=True), RoDeCSR(*args, locality=False)
+    assert tiled.plan.counts[3] == m // 16 and plain.plan is None
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v, g = (torch.randn(16, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    k[:, 200, 3] = float("inf")
+    res = []
+    for c in (tiled, plain):
+        ins = [t.to(dt).requires_grad_() for t in (q, k, v)]
+        res.append(torch.autograd.grad(sparse_attention(c, *ins, scale=0.1), ins, g))
+    for a, b in zip(*res):
+        assert torch.equal(a.isfinite(), b.isfinite()) and b.isfinite().any() and not b.isfinite().all()
+        ok = b.isfinite()
+        assert (a[ok].float() - b[ok].float()).abs().max() <= (4e-3 if half else 2e-5) * b[ok].float().abs().max()
