@@ -146,6 +146,11 @@ def _attention_call(csr, values, q, k, v, scale, keep):
     and None; with keep == "scores" the scaled scores in their place and the
     (maximum, 1 / sum) pair of every row, (m, 2) or (heads, m, 2) - cheaper to write, and
     p = exp(score - maximum) / sum; with keep == None two Nones."""
+    if keep != "probs" and q.shape[-2] == csr.m and k.shape[-2] == csr.n:
+        got = _lib.host_call().attention(csr.row_offsets, csr.column_indices, values, q, k, v, scale, keep is not None,
+                                         csr.plans_address(), rode_sddmm_hip._stream_handle(q.device))
+        if got is not None:
+            return got
     lib = _lib.load()
     heads = q.shape[0] if q.dim() == 3 else 1
     m, d = q.shape[-2:]
@@ -172,6 +177,12 @@ def _attention_backward_call(csr, csr_t, t_slot, probs, stats, g, out, q, k, v, 
     """(dq, dk, dv) in float32 through the two gradient kernels: the row pass over the
     pattern, the column pass over the transposed pattern; every head in the same two launches.
     probs, stats: what ``_attention_call`` kept (stats None: probs holds probabilities)."""
+    if k.shape[-2] == csr.n:
+        got = _lib.host_call().attention_backward(csr.row_offsets, csr.column_indices, csr.values, csr_t.row_offsets, csr_t.column_indices,
+                                                  t_slot, probs, stats, g, out, q, k, v, scale, csr.plans_address(), csr_t.plans_address(),
+                                                  rode_sddmm_hip._stream_handle(q.device))
+        if got is not None:
+            return got
     lib = _lib.load()
     heads = q.shape[0] if q.dim() == 3 else 1
     m, d = q.shape[-2:]

@@ -1,5 +1,5 @@
 // Host side of the Python ops, natively: the calls that a program makes once per product
-// (rode_sddmm, rode_spmm), and what a new matrix needs (row statistics, decomposition).
+// (rode_sddmm, rode_spmm, attention and its gradient), and what a new matrix needs (row statistics, decomposition).
 //
 // A small matrix takes a few microseconds on the GPU, so its calls are bound by what the host
 // does around the launch: argument checks, an allocation and the launch itself cost 10-11 us
@@ -143,6 +143,142 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     Py_END_ALLOW_THREADS
     if (code != 0) return failed(what, code);
     return THPVariable_Wrap(std::move(out));
+}
+
+// ---- attention -----------------------------------------------------------------------------
+struct Pattern {
+    const at::Tensor *row_ptr, *col, *val;
+    int device;
+};
+
+// args: row_offsets, column_indices, values
+bool pattern_of(PyObject* const* args, Pattern& a)
+{
+    a.row_ptr = tensor_of(args[0]), a.col = tensor_of(args[1]), a.val = tensor_of(args[2]);
+    if (!a.row_ptr || !a.col || !a.val || !a.val->is_cuda() || a.val->scalar_type() != at::kFloat || !a.val->is_contiguous()) return false;
+    if (a.val->numel() == 0) return false;
+    a.device = a.val->device().index();
+    int current = -1;
+    return hipGetDevice(&current) == hipSuccess && current == a.device;
+}
+
+bool dense_like(const Pattern& a, const at::Tensor* t, at::ScalarType type, long long heads, int dims, long long rows, long long d)
+{
+    return t && t->is_cuda() && t->device().index() == a.device && t->scalar_type() == type && t->is_contiguous() && t->dim() == dims &&
+           (dims == 2 || t->size(0) == heads) && t->size(dims - 2) == rows && t->size(dims - 1) == d;
+}
+
+// What q, k and v have in common, if they are ordinary.
+struct Heads {
+    int kind = -1, dims = 0;
+    long long heads = 1, m = 0, n = 0, d = 0;
+};
+bool heads_of(const Pattern& a, const at::Tensor* q, const at::Tensor* k, const at::Tensor* v, Heads& h)
+{
+    if (!q || !k || !v || (q->dim() != 2 && q->dim() != 3) || k->dim() != q->dim()) return false;
+    h.dims = (int)q->dim();
+    h.heads = h.dims == 3 ? q->size(0) : 1;
+    h.m = q->size(h.dims - 2), h.n = k->size(h.dims - 2), h.d = q->size(h.dims - 1);
+    h.kind = q->scalar_type() == at::kFloat ? RODE_DENSE_F32 : q->scalar_type() == at::kHalf ? RODE_DENSE_F16 : -1;
+    const at::ScalarType type = q->scalar_type();
+    return h.kind >= 0 && h.m == a.row_ptr->numel() - 1 && h.heads > 0 && dense_like(a, q, type, h.heads, h.dims, h.m, h.d) &&
+           dense_like(a, k, type, h.heads, h.dims, h.n, h.d) && dense_like(a, v, type, h.heads, h.dims, h.n, h.d);
+}
+
+bool float_of(PyObject* o, double& v)
+{
+    v = PyFloat_AsDouble(o);
+    if (v == -1.0 && PyErr_Occurred()) {
+        PyErr_Clear();
+        return false;
+    }
+    return true;
+}
+
+// attention(<pattern>, q, k, v, scale, keep scores, plans address, stream) -> (out, scores or None, stats or None), or None
+PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    Pattern a;
+    Heads h;
+    long long keep, plans, stream;
+    double scale;
+    if (count != 10 || !pattern_of(args, a) || !float_of(args[6], scale) || !int_of(args[7], keep) || !int_of(args[8], plans) ||
+        !int_of(args[9], stream))
+        Py_RETURN_NONE;
+    const at::Tensor *q = tensor_of(args[3]), *k = tensor_of(args[4]), *v = tensor_of(args[5]);
+    if (!heads_of(a, q, k, v, h)) Py_RETURN_NONE;
+    at::Tensor out, scores, stats;
+    const long long nnz = a.val->numel();
+    try {
+        const auto f32 = a.val->options().requires_grad(false);
+        out = at::empty(q->sizes(), f32);
+        if (keep) {
+            scores = h.dims == 3 ? at::empty({h.heads, nnz}, f32) : at::empty({nnz}, f32);
+            stats = h.dims == 3 ? at::empty({h.heads, h.m, 2}, f32) : at::empty({h.m, 2}, f32);
+        }
+    } catch (const std::exception& e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+    int code;
+    Py_BEGIN_ALLOW_THREADS
+    code = rode_hip_attention_forward_batched(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(a.row_ptr->data_ptr()),
+                                              static_cast<const int*>(a.col->data_ptr()), static_cast<const float*>(a.val->data_ptr()), q->data_ptr(),
+                                              k->data_ptr(), v->data_ptr(), (float)scale, static_cast<float*>(out.data_ptr()),
+                                              keep ? static_cast<float*>(scores.data_ptr()) : nullptr, keep ? static_cast<float*>(stats.data_ptr()) : nullptr,
+                                              reinterpret_cast<const rode_hip_plans*>(plans), reinterpret_cast<void*>(stream));
+    Py_END_ALLOW_THREADS
+    if (code != 0) return failed("rode_hip_attention_forward_batched", code);
+    if (!keep) return Py_BuildValue("(NOO)", THPVariable_Wrap(std::move(out)), Py_None, Py_None);
+    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(out)), THPVariable_Wrap(std::move(scores)), THPVariable_Wrap(std::move(stats)));
+}
+
+// attention_backward(<pattern>, row_offsets_t, column_indices_t, slots_t, scores, stats or None, grad, out, q, k, v, scale, plans address,
+// plans address of the transposed pattern, stream) -> (dq, dk, dv) in float32, or None
+PyObject* attention_backward(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    Pattern a;
+    Heads h;
+    long long plans, plans_t, stream;
+    double scale;
+    if (count != 17 || !pattern_of(args, a) || !float_of(args[13], scale) || !int_of(args[14], plans) || !int_of(args[15], plans_t) ||
+        !int_of(args[16], stream))
+        Py_RETURN_NONE;
+    const at::Tensor *t_row_ptr = tensor_of(args[3]), *t_col = tensor_of(args[4]), *t_slot = tensor_of(args[5]), *scores = tensor_of(args[6]);
+    const at::Tensor *stats = args[7] == Py_None ? nullptr : tensor_of(args[7]), *g = tensor_of(args[8]), *out = tensor_of(args[9]);
+    const at::Tensor *q = tensor_of(args[10]), *k = tensor_of(args[11]), *v = tensor_of(args[12]);
+    if (!t_row_ptr || !t_col || !t_slot || !scores || (args[7] != Py_None && !stats) || !heads_of(a, q, k, v, h)) Py_RETURN_NONE;
+    if (!dense_like(a, g, at::kFloat, h.heads, h.dims, h.m, h.d) || !dense_like(a, out, at::kFloat, h.heads, h.dims, h.m, h.d)) Py_RETURN_NONE;
+    const long long nnz = a.val->numel();
+    if (t_slot->numel() != nnz || t_row_ptr->numel() != h.n + 1 || scores->numel() != h.heads * nnz) Py_RETURN_NONE;
+    at::Tensor dq, dk, dv, pairs;
+    try {
+        const auto f32 = a.val->options().requires_grad(false);
+        dq = at::empty(q->sizes(), f32), dk = at::empty(k->sizes(), f32), dv = at::empty(v->sizes(), f32);
+        pairs = at::empty({2 * h.heads * nnz}, f32);
+    } catch (const std::exception& e) {
+        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    }
+    int code;
+    const char* what = "rode_hip_attention_backward_rows";
+    void* s = reinterpret_cast<void*>(stream);
+    Py_BEGIN_ALLOW_THREADS
+    const float* grad = static_cast<const float*>(g->data_ptr());
+    float* pz = static_cast<float*>(pairs.data_ptr());
+    code = rode_hip_attention_backward_rows(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(a.row_ptr->data_ptr()),
+                                            static_cast<const int*>(a.col->data_ptr()), static_cast<const float*>(a.val->data_ptr()),
+                                            static_cast<const float*>(scores->data_ptr()), stats ? static_cast<const float*>(stats->data_ptr()) : nullptr,
+                                            grad, static_cast<const float*>(out->data_ptr()), k->data_ptr(), v->data_ptr(), (float)scale,
+                                            static_cast<const int*>(t_slot->data_ptr()), static_cast<float*>(dq.data_ptr()), pz,
+                                            reinterpret_cast<const rode_hip_plans*>(plans), s);
+    if (code == 0) {
+        what = "rode_hip_attention_backward_cols";
+        code = rode_hip_attention_backward_cols(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(t_row_ptr->data_ptr()),
+                                                static_cast<const int*>(t_col->data_ptr()), pz, grad, q->data_ptr(), static_cast<float*>(dk.data_ptr()),
+                                                static_cast<float*>(dv.data_ptr()), reinterpret_cast<const rode_hip_plans*>(plans_t), s);
+    }
+    Py_END_ALLOW_THREADS
+    if (code != 0) return failed(what, code);
+    return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(dq)), THPVariable_Wrap(std::move(dk)), THPVariable_Wrap(std::move(dv)));
 }
 
 // ---- a new matrix ------------------------------------------------------------------------
@@ -307,6 +443,11 @@ PyMethodDef methods[] = {
      "sddmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, k, lhs, rhs, plans, stream) -> tensor or None"},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(spmm)), METH_FASTCALL,
      "spmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, dense, plans, stored, stream) -> tensor or None"},
+    {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention)), METH_FASTCALL,
+     "attention(row_offsets, columns, values, q, k, v, scale, keep, plans, stream) -> (out, scores, stats) or None"},
+    {"attention_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention_backward)), METH_FASTCALL,
+     "attention_backward(row_offsets, columns, values, row_offsets_t, columns_t, slots_t, scores, stats, grad, out, q, k, v, scale, plans, "
+     "plans_t, stream) -> (dq, dk, dv) or None"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_call", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
