@@ -62,12 +62,15 @@ hipError_t attention_launch(int nheads, int M, int N, int nnz, int d, const int*
 
 constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (size_t)N * row_bytes < (1ull << 32); }
 // Do the tiles of a group plan go to the tile kernels?  (They address a head's k and v with 32-bit offsets; N = 0:
-// not said, one head.  With fewer tiles than CUs and short rows a wave per row is faster: 128 tiles, 144 nonzeros per
-// row of 128 halves 13 against 15 us; 576 per row 17 against 14 us.)
-inline bool attention_uses_tiles(const PlanRef& plan, int nheads, int M, int N, long long nnz, size_t row_bytes)
+// not said, one head.)  Where the other kernel is the one for groups (groups_min, the pass's own figure), always: 4500 rows
+// of 200 columns in fp32, width 32 / 64 / 128: 17 -> 14, 24 -> 18, 70 -> 28 us.  Where it is a wave per row, from 1.5 M nonzeros
+// over all heads on: a tile takes 11 to 48 us however few there are (its rows' nonzeros outside the run come one row after the
+// other).  400 columns and 64 random ones, halves of width 32 / 64 / 128: 1.0 M nonzeros 12 / 17 / 28 us row by row, 16 / 20 / 28
+// on tiles; 1.4 M 13 / 18 / 29 and 17 / 21 / 29; 2.0 M 19 / 26 / 42 and 18 / 23 / 33; 3.9 M 30 / 42 / 71 and 22 / 27 / 52.
+inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads, int N, long long nnz, size_t row_bytes)
 {
     if (plan.groups == nullptr || plan.group_counts == nullptr || plan.group_counts[1] <= 0 || plan.group_counts[3] <= 0) return false;
-    return ((long long)plan.group_counts[3] * nheads >= 256 || nnz >= 256ll * M) && attention_tiles_fit(N, row_bytes);
+    return (plan.group_counts[1] >= groups_min || nnz * nheads >= 1500000) && attention_tiles_fit(N, row_bytes);
 }
 // (rode_attention_tile.hip) the rows of a group plan's tiles, the same arguments; plan: the group plan
 template <typename T>

@@ -32,6 +32,10 @@ def _reference(dense, q, k, v, scale):
     return torch.softmax(s.masked_fill(dense == 0, float("-inf")), dim=1) @ v.double()
 
 
+def _heads(csr):
+    return -(-1500000 // csr.nnz)  # (fewer nonzeros over all heads take other kernels)
+
+
 CASES = [  # m, window, columns the window moves per row, random columns, width, half, scale
     (16, 64, 0, 0, 64, False, 0.3),      # one tile, nothing outside the run, whole steps only
     (75, 69, 1, 5, 64, True, 0.3),       # rows after the last tile, a cut-short last step
@@ -50,7 +54,7 @@ def test_tiles_against_fp64(m, window, shift, extra, d, half, scale):
     assert csr.plan.counts[3] == m // 16 - (1 if m == 160 else 0)
     dt = torch.float16 if half else torch.float32
     g = torch.Generator(device="cuda").manual_seed(d)
-    heads = 256  # (fewer tiles than CUs may take other kernels)
+    heads = _heads(csr)
     q, k, v = (torch.randn(r, d, device="cuda", generator=g).to(dt).expand(heads, r, d).contiguous() for r in (m, csr.n, csr.n))
     outs, all_scores, all_stats = _attention_call(csr, csr.values, q, k, v, scale, "scores")
     assert torch.equal(outs, sparse_attention(csr, q, k, v, scale=scale)) and torch.equal(outs, outs[:1].expand_as(outs))
@@ -78,7 +82,7 @@ def test_non_finite_rows_of_v_stay_in_their_rows(half):
     v[bad] = float("inf")
     if half:
         q, k, v = q.half(), k.half(), v.half()
-    out = sparse_attention(csr, *(t.expand(64, *t.shape).contiguous() for t in (q, k, v)), scale=0.2)[63]
+    out = sparse_attention(csr, *(t.expand(_heads(csr), *t.shape).contiguous() for t in (q, k, v)), scale=0.2)[63]
     touched = (dense[:, bad] != 0).any(dim=1)
     assert touched.any() and not touched.all()
     assert not torch.isfinite(out[touched]).all(dim=1).any()
@@ -90,7 +94,7 @@ def test_gradients_on_tiles_against_fp64(m, window, shift, extra, d, half, scale
     csr, dense = _mask(m, window, shift, extra, seed=m + window, short_rows=(40,) if m == 160 else ())
     dt = torch.float16 if half else torch.float32
     gen = torch.Generator(device="cuda").manual_seed(d)
-    heads = 256
+    heads = _heads(csr)
     q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
     q, k, v = (t.to(dt) for t in (q, k, v))
     g[1] *= 1e-6  # (rows of very different gradients)
@@ -122,7 +126,7 @@ def test_gradients_on_tiles_twice_held_column_and_inf(half):
     tiled, plain = RoDeCSR(*args, locality=True), RoDeCSR(*args, locality=False)
     assert tiled.plan.counts[3] == m // 16 and plain.plan is None
     gen = torch.Generator(device="cuda").manual_seed(1)
-    q, k, v, g = (torch.randn(16, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    q, k, v, g = (torch.randn(48, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
     k[:, 200, 3] = float("inf")
     res = []
     for c in (tiled, plain):
