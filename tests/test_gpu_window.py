@@ -1,56 +1,177 @@
-"""The window kernels (banded matrices) against fp64 on the CPU."""
+"""GPU parity tests of the locality plan and the window kernels (chunks of the residue
+list whose dense rows fit an LDS window): the planned entry points against the fp64 oracle
+and against the same call without a plan, through the Python op (ctypes over the C ABI)."""
 import numpy as np
 import pytest
-import scipy.sparse
 import torch
 
-from rode_amd import RoDeCSR, rode_sddmm, rode_sddmm_hip, rode_spmm
+import oracle
+from gpu_common import DEV, TOL_F16, TOL_F32, round_half, t
+from rode_amd import RoDeCSR, rode_sddmm, rode_spmm, workloads
 
 pytestmark = pytest.mark.gpu
 
 
-def _banded(m, degree, band, far, k, seed):
-    """Rows of 0 .. degree nonzeros in a band, rows % 7 == 3 with `far` columns anywhere; some rows of 128 have their
-    columns anywhere (a chunk without a window)."""
+def banded(rows, cols, per_row, band, seed, far=0, long_every=0, long_len=0, empty_every=0):
+    """Rows with `per_row` distinct columns inside a band around the diagonal, `far` more
+    anywhere (outside the window), every `long_every`-th row `long_len` columns long (it gets
+    block segments and a tail), every `empty_every`-th row empty."""
     rng = np.random.default_rng(seed)
-    rows = []
-    for r in range(m):
-        lo = min(max(0, r - band // 2), m - band)
-        c = lo + rng.choice(band, rng.integers(0, degree + 1), replace=False)
-        if m > 1000 and r // 128 % 5 == 2:
-            c = rng.choice(m, 8, replace=False)
-        if far and r % 7 == 3:
-            c = np.concatenate([c, rng.choice(m, far, replace=False)])
-        rows.append(np.unique(c))
-    rp = np.concatenate([[0], np.cumsum([len(c) for c in rows])]).astype(np.int32)
-    col = np.concatenate(rows).astype(np.int32)
-    val = rng.uniform(0.5, 1.5, len(col)).astype(np.float32)
-    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), "cuda", m, m, k, locality=True)
-    assert csr.plan is not None and csr.plan.counts[1] > 0
-    return csr, scipy.sparse.csr_matrix((val.astype(np.float64), col, rp), shape=(m, m))
+    cols_of = []
+    for r in range(rows):
+        if empty_every and r % empty_every == empty_every - 1:
+            cols_of.append(np.empty(0, dtype=np.int64))
+            continue
+        want = long_len if long_every and r % long_every == 0 else per_row
+        centre = int(r * (cols - 1) / max(rows - 1, 1))
+        lo, hi = max(0, centre - band // 2), min(cols, centre + band // 2)
+        pick = rng.choice(np.arange(lo, hi), size=min(want, hi - lo), replace=False)
+        if far:
+            pick = np.concatenate([pick, rng.integers(0, cols, far)])
+        cols_of.append(np.unique(pick))
+    lens = np.array([len(c) for c in cols_of])
+    row_ptr = np.zeros(rows + 1, dtype=np.int32)
+    row_ptr[1:] = np.cumsum(lens)
+    col = np.concatenate(cols_of).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(np.float32)
+    return row_ptr, col, val
 
 
-CASES = [  # rows, nonzeros of a row at most, band, columns outside it: one chunk cut short; several per workgroup, with misses; none missing
-    (101, 25, 60, 0), (128 * 261 + 5, 21, 200, 3), (128 * 520, 31, 90, 0)]
+def both(row_ptr, col, val, m, n, k):
+    planned = RoDeCSR(t(row_ptr), t(col), t(val), DEV, m, n, k, locality=True)
+    plain = RoDeCSR(t(row_ptr), t(col), t(val), DEV, m, n, k, locality=False)
+    return planned, plain
 
 
-@pytest.mark.parametrize("m,degree,band,far", CASES)
-@pytest.mark.parametrize("dtype,k", [(torch.float32, 36), (torch.float32, 128), (torch.float16, 72), (torch.float16, 128),
-                                     (torch.float64, 18), (torch.float64, 48)])
-def test_window_kernels_against_fp64(m, degree, band, far, dtype, k):
-    csr, ref = _banded(m, degree, band, far, 64 if dtype == torch.float64 else k, seed=m + far)
-    g = torch.Generator().manual_seed(k)
-    dense = torch.randn(m, k, generator=g, dtype=torch.float64).to(dtype)
-    want = ref @ dense.double().numpy()
-    if dtype == torch.float64:
-        got = rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
-                                          csr.column_indices, csr.values.double(), m, m, dense.cuda(), plan=csr.plan)
-        assert np.abs(got.cpu().numpy() - want).max() <= 1e-12 * np.abs(want).max()
-        return
-    got = rode_spmm(csr, dense.cuda())
-    assert np.abs(got.cpu().double().numpy() - want).max() <= 1e-5 * np.abs(want).max()
-    lhs = torch.randn(m, k, generator=g).to(dtype)
-    got = rode_sddmm(csr, lhs.cuda(), dense.cuda()).cpu().double().numpy()
-    rows = np.repeat(np.arange(m), np.diff(ref.indptr))
-    want = ref.data * np.einsum("ij,ij->i", lhs.double().numpy()[rows], dense.double().numpy()[ref.indices])
-    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max()
+def check_products(row_ptr, col, val, m, n, k, half=False, expect_plan=True):
+    planned, plain = both(row_ptr, col, val, m, n, k)
+    assert (planned.plan is not None) == expect_plan
+    assert plain.plan is None
+    rng = np.random.default_rng(17)
+    B = rng.standard_normal((n, k)).astype(np.float32)
+    L = rng.standard_normal((m, k)).astype(np.float32)
+    dt = torch.float16 if half else torch.float32
+    Bd, Ld = t(B).to(DEV, dt), t(L).to(DEV, dt)
+    if half:
+        B, L = round_half(B), round_half(L)
+    tol = TOL_F16 if half else TOL_F32
+    c64 = oracle.spmm_f64(row_ptr, col, val, B)
+    l1 = np.maximum(np.abs(c64).sum(axis=1), 1e-30)
+    o64, scale = oracle.sddmm_f64(row_ptr, col, val, L, B, with_abs=True)
+    for csr in (planned, plain):
+        C = rode_spmm(csr, Bd).cpu().numpy()
+        assert np.max(np.abs(C - c64).max(axis=1) / l1) <= tol
+        out = rode_sddmm(csr, Ld, Bd).cpu().numpy()
+        # per element against the magnitude of the summed terms (strict for any row)
+        assert np.max(np.abs(out - o64) / np.maximum(scale, 1e-30)) <= (2e-3 if half else 2e-6)
+    return planned
+
+
+def test_plan_of_a_banded_matrix_has_a_window_on_every_chunk():
+    m, n, rp, col, val = workloads.config("c3_banded", 0.01)
+    csr = RoDeCSR(t(rp), t(col), t(val), DEV, m, n, 128, locality=True)
+    assert csr.m1 == 0 and csr.plan is not None
+    d = csr.plan.descriptors()
+    assert len(d) == (csr.m2 + 127) // 128 == csr.plan.counts[0] == csr.plan.counts[1]
+    assert (d[:, 1] > 0).all() and (d[:, 1] <= 512).all()
+    assert (d[:, 3] == 0).all()                            # every nonzero inside its chunk's window
+    assert int(d[:, 2].sum()) == int(rp[-1])               # the residue list holds every nonzero here
+    rows = np.arange(len(d)) * 128
+    assert (d[:, 0] <= rows + 128).all() and (d[:, 0] + d[:, 1] >= rows - 128).all()  # windows follow the diagonal
+    assert (d[:, 0] >= 0).all() and (d[:, 0] + d[:, 1] <= n).all()
+
+
+def test_plan_of_scattered_columns_has_no_window():
+    m, n, rp, col, val = workloads.config("c2_lognormal", 0.1)
+    assert RoDeCSR(t(rp), t(col), t(val), DEV, m, n, 128, locality=True).plan is None
+    # "auto" also drops a plan that covers too few chunks to be worth two more launches
+    m, n, rp, col, val = workloads.config("c3_banded", 0.01)
+    assert RoDeCSR(t(rp), t(col), t(val), DEV, m, n, 128).plan is None
+
+
+@pytest.mark.parametrize("k,half", [(128, False), (64, False), (256, False), (200, False), (36, False), (128, True),
+                                    (72, True), (32, False)])
+def test_banded_matrix_planned_against_oracle(k, half):
+    # 36 and 200: partial last tile; 32 fp32 / 64 fp16 and narrower: one tile, the plan is ignored by the kernels
+    m, n, rp, col, val = workloads.config("c3_banded", 0.004)
+    check_products(rp, col, val, m, n, k, half)
+
+
+def test_rows_with_segments_tails_far_columns_and_empty_rows():
+    # long rows (block segments + tails in the residue list, summed whole by the block kernel
+    # under the whole-lists promise when there are many segments), columns outside the window,
+    # empty rows with an unaligned start, a last chunk that is not full
+    m = n = 3000
+    rp, col, val = banded(m, n, 21, 200, seed=5, far=2, long_every=97, long_len=150, empty_every=13)
+    csr = check_products(rp, col, val, m, n, 128)
+    d = csr.plan.descriptors()
+    win = d[d[:, 1] > 0]
+    assert len(win) > 0 and (win[:, 3] > 0).any()           # some slots are outside their window
+    check_products(rp, col, val, m, n, 64, half=False)
+    check_products(rp, col, val, m, n, 128, half=True)
+
+
+def test_window_clipped_at_the_matrix_edges_and_rectangular_operand():
+    m, n = 2000, 700  # the band runs from column 0 to column n - 1
+    rp, col, val = banded(m, n, 17, 300, seed=9)
+    check_products(rp, col, val, m, n, 128)
+
+
+def test_non_finite_dense_rows_stay_in_the_rows_that_reference_them():
+    m = n = 1500
+    rp, col, val = banded(m, n, 15, 120, seed=3, far=1)
+    planned, plain = both(rp, col, val, m, n, 128)
+    assert planned.plan is not None
+    B = torch.randn(n, 128, device=DEV)
+    bad = [0, 7, 640, n - 1]
+    B[bad] = float("inf")
+    touched = np.zeros(m, dtype=bool)
+    rows = np.repeat(np.arange(m), np.diff(rp))
+    touched[rows[np.isin(col, bad)]] = True
+    for csr in (planned, plain):
+        C = rode_spmm(csr, B).cpu().numpy()
+        assert np.isfinite(C[~touched]).all()
+        assert (~np.isfinite(C[touched])).any(axis=1).all()
+
+
+def test_values_replaced_per_call_and_gradients_use_the_plan():
+    m = n = 2048
+    rp, col, val = banded(m, n, 19, 160, seed=11)
+    planned, plain = both(rp, col, val, m, n, 64)
+    assert planned.plan is not None and planned.with_values(planned.values * 2).plan is planned.plan
+    L = torch.randn(m, 64, device=DEV, requires_grad=True)
+    R = torch.randn(n, 64, device=DEV, requires_grad=True)
+    outs = []
+    for csr in (planned, plain):
+        L.grad = R.grad = None
+        s = rode_sddmm(csr, L, R)
+        C = rode_spmm(csr, R, values=s)
+        C.square().sum().backward()
+        outs.append((s.detach().clone(), C.detach().clone(), L.grad.clone(), R.grad.clone()))
+    for a, b in zip(*outs):
+        assert torch.allclose(a, b, rtol=2e-4, atol=2e-4 * float(b.abs().max()))
+
+
+def test_full_size_banded_configuration_planned():
+    # configuration 3 at full size, K = 128: linearity and a row sample against the oracle
+    m, n, rp, col, val = workloads.config("c3_banded", 1.0)
+    csr = RoDeCSR(t(rp), t(col), t(val), DEV, m, n, 128)
+    assert csr.plan is not None and csr.plan.counts[0] == csr.plan.counts[1]
+    rng = np.random.default_rng(23)
+    B = rng.standard_normal((n, 128)).astype(np.float32)
+    L = rng.standard_normal((m, 128)).astype(np.float32)
+    Bd, Ld = t(B).to(DEV), t(L).to(DEV)
+    C = rode_spmm(csr, Bd)
+    out = rode_sddmm(csr, Ld, Bd)
+    sample = np.unique(np.concatenate([np.arange(0, 300), rng.integers(0, m, 400), np.arange(m - 300, m)]))
+    idx = np.concatenate([np.arange(rp[r], rp[r + 1]) for r in sample])
+    srp = np.zeros(len(sample) + 1, dtype=np.int32)
+    srp[1:] = np.cumsum(rp[sample + 1] - rp[sample])
+    c64 = oracle.spmm_f64(srp, col[idx], val[idx], B)
+    l1 = np.maximum(np.abs(c64).sum(axis=1), 1e-30)
+    assert np.max(np.abs(C[sample].cpu().numpy() - c64).max(axis=1) / l1) <= TOL_F32
+    o64, scale = oracle.sddmm_f64(srp, col[idx], val[idx], L[sample], B, with_abs=True)
+    assert np.max(np.abs(out.cpu().numpy()[idx] - o64) / np.maximum(scale, 1e-30)) <= 2e-6
+    # linearity in the dense operand (exact property at any size)
+    C2 = rode_spmm(csr, 2 * Bd)
+    assert torch.equal(C2, 2 * C)
