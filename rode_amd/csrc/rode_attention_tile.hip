@@ -345,7 +345,7 @@ hipError_t launch_tiles(int nheads, int M, int N, int nnz, const int* row_ptr, c
 } // namespace
 
 // The tiles of a group plan (plan.groups, with plan.group_counts[3] > 0 of them); arguments as
-// attention_launch.  One head's k or v must not exceed 4 GB (attention_tiles_fit).
+// attention_launch, scale not zero.  One head's k or v must not exceed 4 GB (attention_tiles_fit).
 template <typename T>
 hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
                                   const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,

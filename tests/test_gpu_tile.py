@@ -89,6 +89,27 @@ def test_non_finite_rows_of_v_stay_in_their_rows(half):
     assert (out[~touched].double() - clean[~touched]).abs().max() <= 2e-5 * clean.abs().max()
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-42])
+def test_a_scale_of_zero_weighs_all_columns_alike(scale, half):
+    m, d, dt = 48, 64, torch.float16 if half else torch.float32
+    csr, dense = _mask(m, 97, 2, 20, seed=3)
+    assert csr.plan.counts[3] == m // 16
+    heads = _heads(csr)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    ins = [t.to(dt).expand(heads, *t.shape).contiguous().requires_grad_() for t in (q, k, v)]
+    out = sparse_attention(csr, *ins, scale=scale)
+    grads = torch.autograd.grad(out, ins, g.expand(heads, m, d).contiguous())
+    want = (dense != 0).double() @ v.to(dt).double() / (dense != 0).sum(1, keepdim=True)
+    assert (out[heads - 1].double() - want).abs().max() <= 2e-5 * want.abs().max()
+    mean = (dense != 0).double() / (dense != 0).sum(1, keepdim=True)
+    want = mean.t().contiguous() @ g.double()
+    assert (grads[2][heads - 1].double() - want).abs().max() <= (5e-3 if half else 1e-4) * want.abs().max()
+    for t in grads[:2]:  # (their size is the scale's)
+        assert t.abs().max() <= 1e-30
+
+
 @pytest.mark.parametrize("m,window,shift,extra,d,half,scale", CASES)
 def test_gradients_on_tiles_against_fp64(m, window, shift, extra, d, half, scale):
     csr, dense = _mask(m, window, shift, extra, seed=m + window, short_rows=(40,) if m == 160 else ())
