@@ -186,20 +186,21 @@ class RoDeCSR:
         key = ("plans", spmm_width, spmm_elem_bytes)
         plans = self._shared.get(key)
         if plans is None:
-            plans = rode_sddmm_hip.plans_struct(self.plan, spmm_width, spmm_elem_bytes, True,
-                                                seg_length=self.config["seg_length"], columns_local=self.columns_local)
-            self._shared[key] = plans
+            # (set once: of two threads' first calls one struct stays, for both)
+            plans = self._shared.setdefault(key, rode_sddmm_hip.plans_struct(
+                self.plan, spmm_width, spmm_elem_bytes, True, seg_length=self.config["seg_length"], columns_local=self.columns_local))
         return plans
 
     def plans_address(self, spmm_width=None):
-        """Where ``call_plans`` keeps its struct (an int, for the native calls).  Only a hub
-        plan's struct depends on the width (it carries the workspace)."""
-        if spmm_width is None or not isinstance(self.plan, rode_sddmm_hip.HubPlan):
-            address = self._shared.get("plans_address")
-            if address is None:
-                address = self._shared["plans_address"] = ctypes.addressof(self.call_plans())
-            return address
-        return ctypes.addressof(self.call_plans(spmm_width, 4))
+        """The struct of ``call_plans`` as the native calls take it: a ``PlansAddress``, which holds
+        the struct.  Only a hub plan's struct depends on the width (it carries the workspace)."""
+        if not isinstance(self.plan, rode_sddmm_hip.HubPlan):
+            spmm_width = None
+        key = "plans_address" if spmm_width is None else ("plans_address", spmm_width)
+        address = self._shared.get(key)
+        if address is None:
+            address = self._shared.setdefault(key, rode_sddmm_hip.PlansAddress(self.call_plans(spmm_width)))
+        return address
 
     def spmm_stores_every_row(self):
         """Whether an SpMM on this matrix leaves no row of C to be cleared beforehand: every row

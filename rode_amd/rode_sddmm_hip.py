@@ -207,10 +207,12 @@ class HubPlan:
         hub row and slab); kept for the next call.  Calls that overlap in time on different
         streams must not share it."""
         key = (n, elem_bytes)
-        if key not in self._workspaces:
+        ws = self._workspaces.get(key)
+        if ws is None:
             nbytes = _lib.load().rode_hip_hub_workspace_bytes(ctypes.addressof(self._header), n, elem_bytes)
-            self._workspaces[key] = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.data.device)
-        return self._workspaces[key]
+            # (set once: the structs of plans_struct keep its address)
+            ws = self._workspaces.setdefault(key, torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.data.device))
+        return ws
 
     @property
     def usable(self):
@@ -317,6 +319,15 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
         p.window, p.window_rows = plan.data.data_ptr(), plan.rows.data_ptr()
         p.window_counts = ctypes.addressof(plan._header)
     return p
+
+
+class PlansAddress(int):
+    """Where a ``rode_hip_plans`` struct is.  Whoever holds the address holds the struct."""
+
+    def __new__(cls, plans):
+        self = super().__new__(cls, ctypes.addressof(plans))
+        self.plans = plans
+        return self
 
 
 def preprocess(row_offsets, nnz, seg_length, k_block, vec_len):

@@ -1,9 +1,12 @@
-"""The native pass over the row offsets, against numpy."""
+"""Host side of the native calls, without a GPU: the pass over the row offsets against numpy, and what a matrix keeps for them."""
+import ctypes
+import types
+
 import numpy as np
 import pytest
 import torch
 
-from rode_amd import _lib
+from rode_amd import RoDeCSR, _lib, rode_sddmm_hip
 
 
 @pytest.mark.parametrize("rows", [0, 1, 7, 65535, 65536, 65537, 200_001])  # (sums are taken per 65536 rows)
@@ -20,3 +23,42 @@ def test_row_stats(rows):
         assert _lib.host_call().row_stats(torch.from_numpy(ro.astype(kind)), 500) == tuple(int(v) for v in want)
     with pytest.raises(ValueError):
         _lib.host_call().row_stats(torch.zeros(3), 500)
+
+
+def _stand_in(plan=None):
+    csr = object.__new__(RoDeCSR)
+    csr.plan, csr.config, csr.columns_local, csr._shared = plan, {"seg_length": 512}, False, {}
+    return csr
+
+
+def test_two_first_calls_get_one_plans_struct(monkeypatch):
+    """Another thread's first call runs from start to end while this one builds its struct."""
+    csr, build, other = _stand_in(), rode_sddmm_hip.plans_struct, []
+
+    def interrupted(*args, **kwargs):
+        if not other:
+            other.append(None)
+            other[0] = csr.plans_address()
+        return build(*args, **kwargs)
+
+    monkeypatch.setattr(rode_sddmm_hip, "plans_struct", interrupted)
+    address = csr.plans_address()
+    assert address == other[0] == ctypes.addressof(csr.call_plans()) == csr.plans_address()
+    held = address.plans  # the struct lives as long as its address is held, whatever the matrix keeps
+    csr._shared.clear()
+    assert ctypes.addressof(held) == address and held.seg_length == 512
+
+
+def test_two_first_calls_get_one_hub_workspace(monkeypatch):
+    plan, other = rode_sddmm_hip.HubPlan(torch.zeros(16, dtype=torch.int32), [1, 1, 32, 1, 1, 0, 0, 0]), []
+
+    def size(header, n, elem_bytes):
+        if not other:
+            other.append(None)
+            other[0] = plan.workspace(n, elem_bytes)
+        return 64
+
+    monkeypatch.setattr(_lib, "load", lambda: types.SimpleNamespace(rode_hip_hub_workspace_bytes=size))
+    assert plan.workspace(32, 4) is other[0] is plan.workspace(32, 4)
+    csr = _stand_in(plan)
+    assert csr.plans_address(32).plans.hub_workspace == other[0].data_ptr() and csr.plans_address() != csr.plans_address(32)
