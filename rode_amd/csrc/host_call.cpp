@@ -14,6 +14,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/zeros.h>
 #include <c10/core/GradMode.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <hip/hip_runtime_api.h>
@@ -26,11 +27,33 @@
 
 namespace {
 
-// The tensor behind a Python object, or null for anything but a plain tensor or parameter.
-const at::Tensor* tensor_of(PyObject* o)
+// (Every function's body is between HANDLE_TH_ERRORS and END_HANDLE_TH_ERRORS: what torch throws - no memory, no
+// data behind a tensor, a Python error of a dispatch mode - becomes the Python exception it stands for.)
+
+// Without the interpreter's lock, until the end of the scope however it is left.
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    NoGil() = default;
+    NoGil(const NoGil&) = delete;
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
+// The tensor behind a Python object if its elements are in memory as its sizes and strides say, else null: not one of
+// another layout (sparse), not a wrapper (vmap, jvp, functionalization), not one with a dispatch of its own (fake
+// tensors) and no lazy negation or zero.
+const at::Tensor* strided_of(PyObject* o)
 {
-    return THPVariable_Check(o) ? &THPVariable_Unpack(o) : nullptr;
+    using K = c10::DispatchKey;
+    static const c10::DispatchKeySet wrapped({K::Python, K::Functionalize, K::FuncTorchBatched, K::FuncTorchGradWrapper, K::Batched, K::Negative,
+                                              K::Conjugate, K::ZeroTensor});
+    if (!THPVariable_Check(o)) return nullptr;
+    const at::Tensor& t = THPVariable_Unpack(o);
+    if (!t.defined() || t.layout() != at::kStrided || !t.has_storage() || t.unsafeGetTensorImpl()->key_set().has_any(wrapped)) return nullptr;
+    return &t;
 }
+
+// The same, or null for anything but a tensor or parameter itself: a subclass may mean something else by the call.
+const at::Tensor* tensor_of(PyObject* o) { return THPVariable_CheckExact(o) ? strided_of(o) : nullptr; }
 
 bool int_of(PyObject* o, long long& v)
 {
@@ -68,6 +91,17 @@ int dense_kind(const Matrix& a, const at::Tensor* t, long long rows)
     return t->scalar_type() == at::kFloat ? RODE_DENSE_F32 : t->scalar_type() == at::kHalf ? RODE_DENSE_F16 : -1;
 }
 
+// The memory of a tensor.  (What a dispatch mode made of an allocation of ours may have none.)
+void* data(const at::Tensor& t)
+{
+    void* p = t.data_ptr();
+    TORCH_CHECK(p != nullptr || t.numel() == 0, "a tensor without data");
+    return p;
+}
+const int* ints(const at::Tensor* t) { return static_cast<const int*>(data(*t)); }
+const float* floats(const at::Tensor* t) { return static_cast<const float*>(data(*t)); }
+float* floats(const at::Tensor& t) { return static_cast<float*>(data(t)); }
+
 bool wants_grad(const at::Tensor& t) { return t.requires_grad(); }
 
 PyObject* failed(const char* what, int code)
@@ -78,6 +112,7 @@ PyObject* failed(const char* what, int code)
 // sddmm(<matrix>, k, lhs, rhs, plans address, stream) -> out or None
 PyObject* sddmm(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
+    HANDLE_TH_ERRORS
     Matrix a;
     long long k, plans, stream;
     if (count != 15 || !matrix_of(args, a) || !int_of(args[10], k) || !int_of(args[13], plans) || !int_of(args[14], stream)) Py_RETURN_NONE;
@@ -86,28 +121,27 @@ PyObject* sddmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (kind < 0 || dense_kind(a, rhs, a.n) != kind || lhs->size(1) != k || rhs->size(1) != k) Py_RETURN_NONE;
     if (k <= 0 || k > 512 || k % (kind == RODE_DENSE_F16 ? 8 : 4) != 0) Py_RETURN_NONE;
     if (c10::GradMode::is_enabled() && (wants_grad(*lhs) || wants_grad(*rhs) || wants_grad(*a.val))) Py_RETURN_NONE;
-    at::Tensor out;
-    try {
-        out = at::empty({a.val->size(0)}, a.val->options().requires_grad(false));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    const at::Tensor out = at::empty({a.val->size(0)}, a.val->options().requires_grad(false));
+    const int *block = ints(a.block), *residue = ints(a.residue), *start = ints(a.start), *row_ptr = ints(a.row_ptr), *col = ints(a.col);
+    const float* val = floats(a.val);
+    float* o = floats(out);
+    const void *l = data(*lhs), *r = data(*rhs);
     int code;
-    void* s = reinterpret_cast<void*>(stream);
-    Py_BEGIN_ALLOW_THREADS
-    code = rode_hip_sddmm_planned(kind, 0, (int)a.m1, (int)a.m2, (int)a.n, (int)k, static_cast<const int*>(a.block->data_ptr()),
-                                  static_cast<const int*>(a.residue->data_ptr()), static_cast<const int*>(a.start->data_ptr()),
-                                  static_cast<const int*>(a.row_ptr->data_ptr()), static_cast<const int*>(a.col->data_ptr()),
-                                  static_cast<const float*>(a.val->data_ptr()), lhs->data_ptr(), rhs->data_ptr(),
-                                  static_cast<float*>(out.data_ptr()), reinterpret_cast<const rode_hip_plans*>(plans), s, s);
-    Py_END_ALLOW_THREADS
+    {
+        NoGil no_gil;
+        void* s = reinterpret_cast<void*>(stream);
+        code = rode_hip_sddmm_planned(kind, 0, (int)a.m1, (int)a.m2, (int)a.n, (int)k, block, residue, start, row_ptr, col, val, l, r, o,
+                                      reinterpret_cast<const rode_hip_plans*>(plans), s, s);
+    }
     if (code != 0) return failed("rode_hip_sddmm_planned", code);
-    return THPVariable_Wrap(std::move(out));
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
 }
 
 // spmm(<matrix>, dense, plans address, every row stored, stream) -> C or None
 PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
+    HANDLE_TH_ERRORS
     Matrix a;
     long long plans, stored, stream;
     if (count != 14 || !matrix_of(args, a) || !int_of(args[11], plans) || !int_of(args[12], stored) || !int_of(args[13], stream)) Py_RETURN_NONE;
@@ -117,32 +151,29 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     const long long width = dense->size(1);
     if (width <= 0 || width > 0x7fffffff || width % (kind == RODE_DENSE_F16 ? 8 : 4) != 0) Py_RETURN_NONE;
     if (c10::GradMode::is_enabled() && (wants_grad(*dense) || wants_grad(*a.val))) Py_RETURN_NONE;
-    at::Tensor out;
-    try {
-        out = at::empty({(int64_t)a.m, (int64_t)width}, a.val->options().requires_grad(false));
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    const at::Tensor out = at::empty({(int64_t)a.m, (int64_t)width}, a.val->options().requires_grad(false));
+    const int *block = ints(a.block), *residue = ints(a.residue), *start = ints(a.start), *row_ptr = ints(a.row_ptr), *col = ints(a.col);
+    const float* val = floats(a.val);
+    const void* b = data(*dense);
+    float* c = floats(out);
     int code = 0;
     const char* what = "rode_hip_spmm_clear_rows_beyond";
-    const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
-    void* s = reinterpret_cast<void*>(stream);
-    Py_BEGIN_ALLOW_THREADS
-    const int* row_ptr = static_cast<const int*>(a.row_ptr->data_ptr());
-    // (only the rows that the kernels add to, or skip, need clearing)
-    if (!stored)
-        code = rode_hip_spmm_clear_rows_beyond((int)a.m, (int)width, 4, rode_hip_spmm_overwrite_limit((int)a.m1, p), row_ptr,
-                                               out.data_ptr(), s);
-    if (code == 0) {
-        what = "rode_hip_spmm_planned";
-        code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, (int)a.m1, (int)a.m2, (int)a.n,
-                                     (int)width, a.val->data_ptr(), static_cast<const int*>(a.col->data_ptr()), row_ptr,
-                                     static_cast<const int*>(a.block->data_ptr()), static_cast<const int*>(a.residue->data_ptr()),
-                                     static_cast<const int*>(a.start->data_ptr()), dense->data_ptr(), out.data_ptr(), p, s, s);
+    {
+        NoGil no_gil;
+        const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
+        void* s = reinterpret_cast<void*>(stream);
+        // (only the rows that the kernels add to, or skip, need clearing)
+        if (!stored)
+            code = rode_hip_spmm_clear_rows_beyond((int)a.m, (int)width, 4, rode_hip_spmm_overwrite_limit((int)a.m1, p), row_ptr, c, s);
+        if (code == 0) {
+            what = "rode_hip_spmm_planned";
+            code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, (int)a.m1, (int)a.m2, (int)a.n, (int)width, val, col,
+                                         row_ptr, block, residue, start, b, c, p, s, s);
+        }
     }
-    Py_END_ALLOW_THREADS
     if (code != 0) return failed(what, code);
-    return THPVariable_Wrap(std::move(out));
+    return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- attention -----------------------------------------------------------------------------
@@ -198,6 +229,7 @@ bool float_of(PyObject* o, double& v)
 // attention(<pattern>, q, k, v, scale, keep scores, plans address, stream) -> (out, scores or None, stats or None), or None
 PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
+    HANDLE_TH_ERRORS
     Pattern a;
     Heads h;
     long long keep, plans, stream;
@@ -209,33 +241,34 @@ PyObject* attention(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (!heads_of(a, q, k, v, h)) Py_RETURN_NONE;
     at::Tensor out, scores, stats;
     const long long nnz = a.val->numel();
-    try {
-        const auto f32 = a.val->options().requires_grad(false);
-        out = at::empty(q->sizes(), f32);
-        if (keep) {
-            scores = h.dims == 3 ? at::empty({h.heads, nnz}, f32) : at::empty({nnz}, f32);
-            stats = h.dims == 3 ? at::empty({h.heads, h.m, 2}, f32) : at::empty({h.m, 2}, f32);
-        }
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
+    const auto f32 = a.val->options().requires_grad(false);
+    out = at::empty(q->sizes(), f32);
+    if (keep) {
+        scores = h.dims == 3 ? at::empty({h.heads, nnz}, f32) : at::empty({nnz}, f32);
+        stats = h.dims == 3 ? at::empty({h.heads, h.m, 2}, f32) : at::empty({h.m, 2}, f32);
     }
+    const int *row_ptr = ints(a.row_ptr), *col = ints(a.col);
+    const float* val = floats(a.val);
+    const void *qp = data(*q), *kp = data(*k), *vp = data(*v);
+    float *o = floats(out), *kept = keep ? floats(scores) : nullptr, *row_stats = keep ? floats(stats) : nullptr;
     int code;
-    Py_BEGIN_ALLOW_THREADS
-    code = rode_hip_attention_forward_batched(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(a.row_ptr->data_ptr()),
-                                              static_cast<const int*>(a.col->data_ptr()), static_cast<const float*>(a.val->data_ptr()), q->data_ptr(),
-                                              k->data_ptr(), v->data_ptr(), (float)scale, static_cast<float*>(out.data_ptr()),
-                                              keep ? static_cast<float*>(scores.data_ptr()) : nullptr, keep ? static_cast<float*>(stats.data_ptr()) : nullptr,
-                                              reinterpret_cast<const rode_hip_plans*>(plans), reinterpret_cast<void*>(stream));
-    Py_END_ALLOW_THREADS
+    {
+        NoGil no_gil;
+        code = rode_hip_attention_forward_batched(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, row_ptr, col, val, qp, kp, vp,
+                                                  (float)scale, o, kept, row_stats, reinterpret_cast<const rode_hip_plans*>(plans),
+                                                  reinterpret_cast<void*>(stream));
+    }
     if (code != 0) return failed("rode_hip_attention_forward_batched", code);
     if (!keep) return Py_BuildValue("(NOO)", THPVariable_Wrap(std::move(out)), Py_None, Py_None);
     return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(out)), THPVariable_Wrap(std::move(scores)), THPVariable_Wrap(std::move(stats)));
+    END_HANDLE_TH_ERRORS
 }
 
 // attention_backward(<pattern>, row_offsets_t, column_indices_t, slots_t, scores, stats or None, grad, out, q, k, v, scale, plans address,
 // plans address of the transposed pattern, stream) -> (dq, dk, dv) in float32, or None
 PyObject* attention_backward(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
+    HANDLE_TH_ERRORS
     Pattern a;
     Heads h;
     long long plans, plans_t, stream;
@@ -250,35 +283,29 @@ PyObject* attention_backward(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (!dense_like(a, g, at::kFloat, h.heads, h.dims, h.m, h.d) || !dense_like(a, out, at::kFloat, h.heads, h.dims, h.m, h.d)) Py_RETURN_NONE;
     const long long nnz = a.val->numel();
     if (t_slot->numel() != nnz || t_row_ptr->numel() != h.n + 1 || scores->numel() != h.heads * nnz) Py_RETURN_NONE;
-    at::Tensor dq, dk, dv, pairs;
-    try {
-        const auto f32 = a.val->options().requires_grad(false);
-        dq = at::empty(q->sizes(), f32), dk = at::empty(k->sizes(), f32), dv = at::empty(v->sizes(), f32);
-        pairs = at::empty({2 * h.heads * nnz}, f32);
-    } catch (const std::exception& e) {
-        return PyErr_Format(PyExc_RuntimeError, "%s", e.what());
-    }
+    const auto f32 = a.val->options().requires_grad(false);
+    at::Tensor dq = at::empty(q->sizes(), f32), dk = at::empty(k->sizes(), f32), dv = at::empty(v->sizes(), f32);
+    const at::Tensor pairs = at::empty({2 * h.heads * nnz}, f32);
+    const int *row_ptr = ints(a.row_ptr), *col = ints(a.col), *rows_t = ints(t_row_ptr), *col_t = ints(t_col), *slot = ints(t_slot);
+    const float *val = floats(a.val), *kept = floats(scores), *row_stats = stats ? floats(stats) : nullptr, *grad = floats(g), *o = floats(out);
+    const void *qp = data(*q), *kp = data(*k), *vp = data(*v);
+    float *pz = floats(pairs), *dqp = floats(dq), *dkp = floats(dk), *dvp = floats(dv);
     int code;
     const char* what = "rode_hip_attention_backward_rows";
-    void* s = reinterpret_cast<void*>(stream);
-    Py_BEGIN_ALLOW_THREADS
-    const float* grad = static_cast<const float*>(g->data_ptr());
-    float* pz = static_cast<float*>(pairs.data_ptr());
-    code = rode_hip_attention_backward_rows(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(a.row_ptr->data_ptr()),
-                                            static_cast<const int*>(a.col->data_ptr()), static_cast<const float*>(a.val->data_ptr()),
-                                            static_cast<const float*>(scores->data_ptr()), stats ? static_cast<const float*>(stats->data_ptr()) : nullptr,
-                                            grad, static_cast<const float*>(out->data_ptr()), k->data_ptr(), v->data_ptr(), (float)scale,
-                                            static_cast<const int*>(t_slot->data_ptr()), static_cast<float*>(dq.data_ptr()), pz,
-                                            reinterpret_cast<const rode_hip_plans*>(plans), s);
-    if (code == 0) {
-        what = "rode_hip_attention_backward_cols";
-        code = rode_hip_attention_backward_cols(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, static_cast<const int*>(t_row_ptr->data_ptr()),
-                                                static_cast<const int*>(t_col->data_ptr()), pz, grad, q->data_ptr(), static_cast<float*>(dk.data_ptr()),
-                                                static_cast<float*>(dv.data_ptr()), reinterpret_cast<const rode_hip_plans*>(plans_t), s);
+    {
+        NoGil no_gil;
+        void* s = reinterpret_cast<void*>(stream);
+        code = rode_hip_attention_backward_rows(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, row_ptr, col, val, kept, row_stats, grad,
+                                                o, kp, vp, (float)scale, slot, dqp, pz, reinterpret_cast<const rode_hip_plans*>(plans), s);
+        if (code == 0) {
+            what = "rode_hip_attention_backward_cols";
+            code = rode_hip_attention_backward_cols(h.kind, (int)h.heads, (int)h.m, (int)h.n, (int)nnz, (int)h.d, rows_t, col_t, pz, grad, qp, dkp, dvp,
+                                                    reinterpret_cast<const rode_hip_plans*>(plans_t), s);
+        }
     }
-    Py_END_ALLOW_THREADS
     if (code != 0) return failed(what, code);
     return Py_BuildValue("(NNN)", THPVariable_Wrap(std::move(dq)), THPVariable_Wrap(std::move(dk)), THPVariable_Wrap(std::move(dv)));
+    END_HANDLE_TH_ERRORS
 }
 
 // ---- a new matrix ------------------------------------------------------------------------
@@ -321,27 +348,31 @@ __attribute__((target_clones("avx512f", "avx2", "default"))) void row_stats_bloc
 // row_stats(row offsets on the CPU, int32 or int64; hub_min_len) -> the fields of RowStats
 PyObject* row_stats(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
-    const at::Tensor* ro = count == 2 ? tensor_of(args[0]) : nullptr;
+    HANDLE_TH_ERRORS
+    const at::Tensor* ro = count == 2 ? strided_of(args[0]) : nullptr;
     long long hub_min_len;
     if (!ro || !int_of(args[1], hub_min_len) || !ro->is_cpu() || ro->dim() != 1 || !ro->is_contiguous() ||
         (ro->scalar_type() != at::kInt && ro->scalar_type() != at::kLong))
         return PyErr_Format(PyExc_ValueError, "row_stats takes a contiguous int32 or int64 vector on the CPU and an int");
     const long long rows = ro->size(0) - 1;
+    const void* offsets = data(*ro);
+    const bool is_int = ro->scalar_type() == at::kInt;
     RowStats r;
-    Py_BEGIN_ALLOW_THREADS
-    constexpr long long kBlock = 1 << 16; // (a block's sums are added up in 64 bits)
-    for (long long at = 0; at < rows; at += kBlock) {
-        const long long n = std::min(kBlock, rows - at);
-        if (ro->scalar_type() == at::kInt)
-            row_stats_block<int32_t>(static_cast<const int32_t*>(ro->data_ptr()) + at, n,
-                                     (int32_t)std::min<long long>(hub_min_len, INT32_MAX), r);
-        else
-            row_stats_block<int64_t>(static_cast<const int64_t*>(ro->data_ptr()) + at, n, hub_min_len, r);
+    {
+        NoGil no_gil;
+        constexpr long long kBlock = 1 << 16; // (a block's sums are added up in 64 bits)
+        for (long long at = 0; at < rows; at += kBlock) {
+            const long long n = std::min(kBlock, rows - at);
+            if (is_int)
+                row_stats_block<int32_t>(static_cast<const int32_t*>(offsets) + at, n, (int32_t)std::min<long long>(hub_min_len, INT32_MAX), r);
+            else
+                row_stats_block<int64_t>(static_cast<const int64_t*>(offsets) + at, n, hub_min_len, r);
+        }
     }
-    Py_END_ALLOW_THREADS
     if (rows <= 0) r.shortest = r.longest = 0;
     return Py_BuildValue("(LLLLLLLL)", r.max_len, r.shortest, r.longest, r.blocked, r.segments_512, r.up_to_512, r.up_to_1024,
                          r.hub_nonzeros);
+    END_HANDLE_TH_ERRORS
 }
 
 // How many block segments and residue rows the decomposition has (k_block 32, vec_len 4): the
@@ -380,10 +411,11 @@ void list_sizes(const int32_t* ro, long long rows, int seg, long long& n_blk, lo
 // instead of one for the counts, one for the plan and a copy of every list.
 PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
+    HANDLE_TH_ERRORS
     long long dense_rows, seg, stream;
     if (count != 6 || !int_of(args[3], dense_rows) || !int_of(args[4], seg) || !int_of(args[5], stream))
         return PyErr_Format(PyExc_ValueError, "decompose takes 6 arguments");
-    const at::Tensor *host = tensor_of(args[0]), *dev = tensor_of(args[1]), *col = args[2] == Py_None ? nullptr : tensor_of(args[2]);
+    const at::Tensor *host = strided_of(args[0]), *dev = strided_of(args[1]), *col = args[2] == Py_None ? nullptr : strided_of(args[2]);
     if (!host || !dev || !host->is_cpu() || !dev->is_cuda() || host->scalar_type() != at::kInt || dev->scalar_type() != at::kInt ||
         host->dim() != 1 || dev->dim() != 1 || host->size(0) < 1 || host->size(0) != dev->size(0) || !host->is_contiguous() ||
         !dev->is_contiguous() || seg <= 0 || seg > INT32_MAX || (args[2] != Py_None && (!col || !col->is_cuda() || col->scalar_type() != at::kInt)))
@@ -394,9 +426,9 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
     int code = 0;
     const char* what = "rode_hip_preprocess";
     std::string error;
-    Py_BEGIN_ALLOW_THREADS
-    try {
-        list_sizes(static_cast<const int32_t*>(host->data_ptr()), m, (int)seg, m1, m2);
+    {
+        NoGil no_gil;
+        list_sizes(static_cast<const int32_t*>(data(*host)), m, (int)seg, m1, m2);
         blk = m1 > 0 ? at::empty({m1}, dev->options()) : at::zeros({1}, dev->options()); // (an empty list has one place that is never read)
         start = at::empty({m1 + 1}, dev->options());
         res = m2 > 0 ? at::empty({m2}, dev->options()) : at::zeros({1}, dev->options());
@@ -404,34 +436,32 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
         // (pinned: the kernels write the counts where the host reads them)
         counts = at::empty({8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-        int* h = static_cast<int*>(counts.data_ptr());
+        int* h = static_cast<int*>(data(counts));
         h[0] = h[1] = -1;
-        const int* rp = static_cast<const int*>(dev->data_ptr());
+        const int* rp = static_cast<const int*>(data(*dev));
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-        code = rode_hip_preprocess((int)seg, 32, 4, (int)m, rp, static_cast<int*>(blk.data_ptr()), static_cast<int*>(start.data_ptr()),
-                                   static_cast<int*>(res.data_ptr()), h, h + 1, (int)m1, scratch.data_ptr(), ws_bytes, s);
+        code = rode_hip_preprocess((int)seg, 32, 4, (int)m, rp, static_cast<int*>(data(blk)), static_cast<int*>(data(start)),
+                                   static_cast<int*>(data(res)), h, h + 1, (int)m1, data(scratch), ws_bytes, s);
         if (code == 0 && col && m2 > 0) {
             what = "rode_hip_window_plan";
             const size_t bytes = rode_hip_window_plan_bytes((int)m2);
             plan = at::empty({(int64_t)(bytes / 4)}, dev->options());
-            code = rode_hip_window_plan((int)m2, (int)dense_rows, static_cast<const int*>(res.data_ptr()), rp,
-                                        static_cast<const int*>(col->data_ptr()), plan.data_ptr(), bytes, nullptr, s);
-            if (code == 0) code = hipMemcpyAsync(h + 4, plan.data_ptr(), 4 * sizeof(int), hipMemcpyDeviceToHost, s);
+            code = rode_hip_window_plan((int)m2, (int)dense_rows, static_cast<const int*>(data(res)), rp,
+                                        static_cast<const int*>(data(*col)), data(plan), bytes, nullptr, s);
+            if (code == 0) code = hipMemcpyAsync(h + 4, data(plan), 4 * sizeof(int), hipMemcpyDeviceToHost, s);
         }
         const int waited = hipStreamSynchronize(s); // (also after an error: the scratch is in use until then)
         if (code == 0) code = waited;
         if (code == 0 && (h[0] != m1 || h[1] != m2)) error = "the row decomposition on the GPU does not have the expected size";
-    } catch (const std::exception& e) {
-        error = e.what();
     }
-    Py_END_ALLOW_THREADS
     if (!error.empty()) return PyErr_Format(PyExc_RuntimeError, "%s", error.c_str());
     if (code != 0) return failed(what, code);
-    const int* h = static_cast<const int*>(counts.data_ptr());
+    const int* h = static_cast<const int*>(data(counts));
     PyObject* plan_counts = plan.defined() ? Py_BuildValue("[iiii]", h[4], h[5], h[6], h[7]) : Py_BuildValue("");
     PyObject* plan_data = plan.defined() ? THPVariable_Wrap(std::move(plan)) : Py_BuildValue("");
     return Py_BuildValue("(NNNLLNN)", THPVariable_Wrap(std::move(blk)), THPVariable_Wrap(std::move(start)), THPVariable_Wrap(std::move(res)),
                          m1, m2, plan_data, plan_counts);
+    END_HANDLE_TH_ERRORS
 }
 
 PyMethodDef methods[] = {

@@ -27,6 +27,12 @@ def _check(cond, msg):
 def _check_input(x, name):
     _check(x.device.type == "cuda", f"{name} must be a CUDA tensor")
     _check(x.is_contiguous(), f"{name} must be contiguous")
+    _check_data(x, name)
+
+
+def _check_data(x, name):
+    """(A fake tensor has a device and a shape like any other, and nothing behind them.)"""
+    _check(x.data_ptr() != 0 or x.numel() == 0, f"{name} has no data")
 
 
 def _stream_handle(device):
@@ -391,6 +397,8 @@ def sddmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offset
         return torch.zeros(nnz, dtype=torch.float32, device=values.device)
     # (every nonzero is in exactly one work item and every work item stores its outputs: nothing to clear)
     out = torch.empty(nnz, dtype=torch.float32, device=values.device)
+    _check_data(values, "values")
+    _check_data(out, "out")
     lib = _lib.load()
     with _on_device(values.device):
         s = _stream_handle(values.device)
@@ -449,6 +457,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
             return torch.zeros((m, n), dtype=out_dtype, device=values.device)
         # only the rows the kernels add to (or skip) need clearing, the others are overwritten
         out = torch.empty((m, n), dtype=out_dtype, device=values.device)
+        _check_data(out, "out")
         if not (every_row_stored and whole_lists):
             stored = lib.rode_hip_spmm_overwrite_limit(m1, ctypes.byref(plans)) if whole_lists else 0
             with _on_device(values.device):
@@ -460,6 +469,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
         _check(out.dtype == out_dtype and tuple(out.shape) == (m, n), f"out must be {out_dtype} of shape (m, n)")
     if m1 == 0 and m2 == 0:
         return out
+    _check_data(values, "values")
     dtype = {torch.float32: 0, torch.float16: 1, torch.float64: 2}[dense_matrix.dtype]  # RODE_DENSE_*
     with _on_device(values.device):
         s = _stream_handle(values.device)

@@ -1,10 +1,13 @@
 """The native host calls behind rode_sddmm and rode_spmm: the same results as the module's functions, and everything
 that is not the ordinary call still reaches the Python layer."""
+import threading
+
 import numpy as np
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
-from rode_amd import RoDeCSR, _lib, rode_sddmm, rode_sddmm_hip, rode_spmm
+from rode_amd import RoDeCSR, _lib, rode_sddmm, rode_sddmm_hip, rode_spmm, sparse_attention
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +61,56 @@ def test_other_calls_reach_the_python_layer():
         got = rode_sddmm(a, lhs, rhs)
     side.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("op", ["sddmm", "spmm", "attention"])
+@pytest.mark.parametrize("kind", ["fake", "vmap", "jvp", "sparse", "subclass", "fake mode", "other dtype"])
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor", "ignore:Sparse CSR tensor support")
+def test_operands_that_are_no_plain_tensors(op, kind):
+    """Refused with an exception (or, a mere subclass, taken): none ends in an abort or reaches a kernel without memory."""
+    a = _matrix(64, 64, 32)
+    x, y = torch.randn(64, 32, device="cuda"), torch.randn(64, 32, device="cuda")
+
+    def call(t):
+        if op == "sddmm":
+            return rode_sddmm(a, x, t)
+        return rode_spmm(a, t) if op == "spmm" else sparse_attention(a, x, x, t)
+
+    want = call(y)
+    if kind == "subclass":
+        assert torch.equal(torch.Tensor(call(y.as_subclass(type("Subclass", (torch.Tensor,), {})))), want)
+        return
+    with pytest.raises((RuntimeError, AssertionError, ValueError)):
+        if kind == "fake":
+            call(FakeTensorMode().from_tensor(y))
+        elif kind == "vmap":
+            torch.vmap(call)(y.expand(2, 64, 32))
+        elif kind == "jvp":
+            torch.func.jvp(call, (y,), (y,))
+        elif kind == "sparse":
+            call(y.to_sparse_csr())
+        elif kind == "fake mode":
+            with FakeTensorMode(allow_non_fake_inputs=True):
+                call(y)
+        else:
+            call(y.to(torch.complex64))
+    assert torch.equal(call(y), want)
+
+
+def test_two_threads_make_the_first_calls():
+    x, y = torch.randn(300, 32, device="cuda"), torch.randn(300, 32, device="cuda")
+    want = rode_sddmm(_matrix(300, 300, 32), x, y)
+    for _ in range(20):
+        a, start, got = _matrix(300, 300, 32), threading.Barrier(2), [None, None]
+
+        def work(i):
+            start.wait()
+            got[i] = [rode_sddmm(a, x, y) for _ in range(3)]
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        assert all(torch.equal(g, want) for thread in got for g in thread)

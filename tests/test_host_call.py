@@ -5,6 +5,7 @@ import types
 import numpy as np
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from rode_amd import RoDeCSR, _lib, rode_sddmm_hip
 
@@ -23,6 +24,30 @@ def test_row_stats(rows):
         assert _lib.host_call().row_stats(torch.from_numpy(ro.astype(kind)), 500) == tuple(int(v) for v in want)
     with pytest.raises(ValueError):
         _lib.host_call().row_stats(torch.zeros(3), 500)
+
+
+@pytest.mark.parametrize("kind", ["fake", "vmap", "sparse", "subclass"])
+def test_row_stats_of_other_tensors(kind):
+    """No tensor of its kind ends in an abort or a read of memory that is not there."""
+    ro = torch.tensor([0, 3, 5], dtype=torch.int32)
+    got = []
+
+    def call(t):
+        if kind == "subclass":  # its elements are where a tensor's are
+            got.append(_lib.host_call().row_stats(t, 5)[:3] == (3, 3, 5))
+        else:
+            with pytest.raises(ValueError):
+                _lib.host_call().row_stats(t, 5)
+            got.append(True)
+        return t
+
+    if kind == "fake":
+        call(FakeTensorMode().from_tensor(ro))
+    elif kind == "vmap":
+        torch.vmap(call)(ro.expand(2, 3))
+    else:
+        call(ro.to_sparse() if kind == "sparse" else ro.as_subclass(type("Subclass", (torch.Tensor,), {})))
+    assert got == [True]
 
 
 def _stand_in(plan=None):
