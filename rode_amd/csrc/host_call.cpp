@@ -434,21 +434,25 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         res = m2 > 0 ? at::empty({m2}, dev->options()) : at::zeros({1}, dev->options());
         const size_t ws_bytes = rode_hip_preprocess_workspace_bytes((int)m);
         scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
+        size_t plan_bytes = 0;
+        if (col && m2 > 0) {
+            plan_bytes = rode_hip_window_plan_bytes((int)m2);
+            plan = at::empty({(int64_t)(plan_bytes / 4)}, dev->options());
+        }
         // (pinned: the kernels write the counts where the host reads them)
         counts = at::empty({8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-        int* h = static_cast<int*>(data(counts));
+        int *h = static_cast<int*>(data(counts)), *segments = static_cast<int*>(data(blk)), *starts = static_cast<int*>(data(start));
+        int* rows = static_cast<int*>(data(res));
         h[0] = h[1] = -1;
-        const int* rp = static_cast<const int*>(data(*dev));
+        const int *rp = static_cast<const int*>(data(*dev)), *columns = plan_bytes ? static_cast<const int*>(data(*col)) : nullptr;
+        void *work = data(scratch), *windows = plan_bytes ? data(plan) : nullptr;
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-        code = rode_hip_preprocess((int)seg, 32, 4, (int)m, rp, static_cast<int*>(data(blk)), static_cast<int*>(data(start)),
-                                   static_cast<int*>(data(res)), h, h + 1, (int)m1, data(scratch), ws_bytes, s);
-        if (code == 0 && col && m2 > 0) {
+        // From here to the end of the wait nothing throws: what is queued uses the memory above.
+        code = rode_hip_preprocess((int)seg, 32, 4, (int)m, rp, segments, starts, rows, h, h + 1, (int)m1, work, ws_bytes, s);
+        if (code == 0 && plan_bytes) {
             what = "rode_hip_window_plan";
-            const size_t bytes = rode_hip_window_plan_bytes((int)m2);
-            plan = at::empty({(int64_t)(bytes / 4)}, dev->options());
-            code = rode_hip_window_plan((int)m2, (int)dense_rows, static_cast<const int*>(data(res)), rp,
-                                        static_cast<const int*>(data(*col)), data(plan), bytes, nullptr, s);
-            if (code == 0) code = hipMemcpyAsync(h + 4, data(plan), 4 * sizeof(int), hipMemcpyDeviceToHost, s);
+            code = rode_hip_window_plan((int)m2, (int)dense_rows, rows, rp, columns, windows, plan_bytes, nullptr, s);
+            if (code == 0) code = hipMemcpyAsync(h + 4, windows, 4 * sizeof(int), hipMemcpyDeviceToHost, s);
         }
         const int waited = hipStreamSynchronize(s); // (also after an error: the scratch is in use until then)
         if (code == 0) code = waited;

@@ -6,6 +6,7 @@ import numpy as np
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
 
 from rode_amd import RoDeCSR, _lib, rode_sddmm, rode_sddmm_hip, rode_spmm, sparse_attention
 
@@ -114,3 +115,41 @@ def test_two_threads_make_the_first_calls():
             t.join()
         torch.cuda.synchronize()
         assert all(torch.equal(g, want) for thread in got for g in thread)
+
+
+class _Refuse(TorchDispatchMode):
+    """The `at`-th tensor operation fails, as an allocation without memory does."""
+
+    def __init__(self, at):
+        super().__init__()
+        self.left = at
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.left -= 1
+        if self.left == 0:
+            raise MemoryError("refused")
+        return func(*args, **(kwargs or {}))
+
+
+def test_decomposition_without_memory_leaves_nothing_running():
+    m = 1_000_000  # (rows of 40: both lists have entries)
+    ro = torch.arange(m + 1, dtype=torch.int32) * 40
+    on_gpu, col = ro.cuda(), torch.arange(40 * m, dtype=torch.int32, device="cuda") // 40
+    args = (ro, on_gpu, col, m, 512, rode_sddmm_hip._stream_handle(on_gpu.device))
+    want = _lib.host_call().decompose(*args)
+    assert want[5] is not None  # (with a plan)
+    refused = 0
+    while True:
+        torch.cuda.synchronize()
+        mode = _Refuse(refused + 1)
+        with mode:
+            try:
+                got = _lib.host_call().decompose(*args)
+            except MemoryError:
+                refused += 1
+                assert torch.cuda.current_stream().query()
+                continue
+        break
+    assert refused >= 6 and mode.left == 1  # the lists, the scratch, the plan and the counts
+    for a, b in zip(got, want):
+        assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
