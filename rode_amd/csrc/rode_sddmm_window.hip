@@ -174,14 +174,14 @@ sddmm_residue_window_kernel(int m2, int k, const int* __restrict__ col, const fl
 
 } // namespace
 
-// The window kernel over the planned chunks of the residue list, for dense rows of more than one tile.
+// The window kernel over the planned chunks of the residue list, for dense rows that window_takes.
 // T = float or __half.
 template <typename T>
 hipError_t sddmm_window_launch(int m2, int k, const int* col, const float* val, const T* lhs, const T* rhs, float* out,
                                const int* plan, const void* plan_rows, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
-    if ((size_t)k * sizeof(T) <= kResLanes * 16) return hipErrorInvalidValue;
+    if (!window_takes((size_t)k * sizeof(T))) return hipErrorInvalidValue;
     auto kernel = ((size_t)k * sizeof(T)) % (kResLanes * 16) != 0 ? sddmm_residue_window_kernel<T, true> : sddmm_residue_window_kernel<T, false>;
     kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, static_cast<const PlannedChunk*>(plan_rows));
     return hipGetLastError();

@@ -856,9 +856,7 @@ int spmm_overwrite_limit(int m1, bool hub_plan) { return m1 >= kOwnedMinSegments
 // dense row is cut into tiles of 32, 64 or 128 columns (at most 32 lanes per tile row);
 // the tile width with the least padding wins, the widest on a tie.  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
-// which `plan` holds a window go to the window kernel (operands wider than one 128-byte tile;
-// narrower ones ignore the plan: with a single tile the
-// window is not reused often enough to repay its staging).
+// which `plan` holds a window go to the window kernel (window_takes; other widths ignore the plan).
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
@@ -866,9 +864,8 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
 {
     static_assert(std::is_same<typename SpmmAcc<T>::type, typename DenseVec<T>::Acc>::value, "accumulation type");
     if (n <= 0 || n % DenseVec<T>::kElems != 0) return hipErrorInvalidValue;
-    // the window kernels are for operands with more than one 128-byte tile per row (500 K rows of 32 doubles, band of
-    // 256: 0.204 -> 0.131 ms)
-    if ((size_t)n * sizeof(T) <= 128) {
+    // (500 K rows of 32 doubles, two tiles, band of 256: 0.204 -> 0.131 ms)
+    if (!window_takes((size_t)n * sizeof(T))) {
         plan.dev = nullptr;
         plan.rows = nullptr;
         plan.host_counts = nullptr;

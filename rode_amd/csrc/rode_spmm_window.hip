@@ -188,13 +188,13 @@ spmm_residue_window_kernel(int m2, int n, int owned_slots, const int* __restrict
 
 } // namespace
 
-// The window kernel over the planned chunks of the residue list, for dense rows of more than one tile.
+// The window kernel over the planned chunks of the residue list, for dense rows that window_takes.
 template <typename T>
 hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
                               typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
-    if ((size_t)n * sizeof(T) <= kResLanes * 16) return hipErrorInvalidValue;
+    if (!window_takes((size_t)n * sizeof(T))) return hipErrorInvalidValue;
     auto kernel = ((size_t)n * sizeof(T)) % (kResLanes * 16) != 0 ? spmm_residue_window_kernel<T, true> : spmm_residue_window_kernel<T, false>;
     kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
     return hipGetLastError();

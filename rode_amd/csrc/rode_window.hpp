@@ -82,7 +82,8 @@ __device__ __forceinline__ void fetch_record(unsigned lds, const PlannedChunk* c
 }
 
 // One column tile of the window rows [0, wn) to LDS: `tile` points at it in the first row, rows are
-// row_bytes apart, `at` is this lane's 16 bytes of a row (any valid place of it for a lane past the last column).
+// row_bytes apart (window_takes: 32-bit offsets), `at` is this lane's 16 bytes of a row (any valid place of it for a lane
+// past the last column).
 __device__ __forceinline__ void fetch_window(unsigned lds, const void* tile, unsigned row_bytes, int wn, unsigned at, int wave)
 {
 #pragma unroll

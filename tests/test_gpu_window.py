@@ -175,3 +175,23 @@ def test_full_size_banded_configuration_planned():
     # linearity in the dense operand (exact property at any size)
     C2 = rode_spmm(csr, 2 * Bd)
     assert torch.equal(C2, 2 * C)
+
+
+@pytest.mark.parametrize("width", [4_194_304, 6_300_008])  # (rows of 8 MiB, the widest the window kernel takes, and of 12.6 MB)
+def test_very_wide_operand(width):
+    """Windows of more than 4 GiB of dense rows: halves, 450 rows."""
+    m, n = 128, 450
+    rng = np.random.default_rng(11)
+    col = np.concatenate([np.sort(rng.choice(n, 27, replace=False)) for _ in range(m)]).astype(np.int32)
+    row_ptr = np.arange(0, 27 * m + 1, 27, dtype=np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(np.float32)
+    csr = RoDeCSR(t(row_ptr), t(col), t(val), DEV, m, n, 128, locality=True)
+    assert csr.plan is not None and csr.plan.windowed == 1
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    B = torch.randn(n, width, device=DEV, generator=gen, dtype=torch.float16)
+    C = rode_spmm(csr, B)
+    dense = torch.zeros(m, n, dtype=torch.float64, device=DEV)
+    dense[torch.arange(m, device=DEV).repeat_interleave(27), csr.column_indices.long()] = csr.values.double()
+    for at in (0, 8 * rng.integers(width // 8), width - 64):
+        want = dense @ B[:, at:at + 64].double()
+        assert (C[:, at:at + 64].double() - want).abs().max() <= 1e-5 * want.abs().max()
