@@ -330,11 +330,10 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
     heads.rows = (size_t)M * D, heads.cols = (size_t)N * D, heads.nnz = (size_t)nnz;
     const Keep keep = probs == nullptr ? kKeepNothing : stats != nullptr ? kKeepScores : kKeepProbs;
     // The tiles of a group plan first (the matrix cores); the other groups when a wave per group
-    // fills the GPU; what is left row by row.  (Not with a scale of zero: the tiles' running maximum is of
-    // scores before the scale, and "no score yet" times zero is NaN.)
+    // fills the GPU; what is left row by row.
     RowOwners owners;
     int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
-    if (scale != 0.f && attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T))) {
+    if (attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T))) {
         owners.tiles = group_plan_tiles(plan.groups, M);
         owners.n_tiles = row_tiles(M);
         groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);

@@ -20,7 +20,12 @@
 // operand layout (adjacent lanes on different rows: 64 clocks of the memory pipe per load, 0.38 ms).
 //
 // 32-bit operands use the 32-bit matrix instructions (exact products, 157 TFLOP/s against 79 on the
-// vector ALUs); 16-bit operands split the probabilities into two halves each (TileWeights).
+// vector ALUs); 16-bit operands split the probabilities into two halves each (TileWeights).  Errors against 64 bits of
+// the output and of the gradients that follow from it, against those of the kernels on the vector ALUs (2-norms, masks of
+// 200 to 700 columns, widths 32 to 128, scores with a deviation of 1 and of 8): fp32 0.72 to 1.03 times, halves 0.82 to
+// 1.01 times.  That took sums in trees (mma_rows, TileCols), exponents that are rounded once (TileSoftmax) and row
+// sums of the 32-bit weights on the vector ALUs; as chains of matrix products with a rounded offset in the exponent it
+// was 1.4 to 3.1 and 1.0 to 1.7 times.
 #include "rode_tile.hpp"
 #include "rode_units.hpp"
 #include "rode_internal.hpp"
@@ -31,43 +36,51 @@ namespace rode {
 
 namespace {
 
-// Running softmax of the rows of a tile: 4 or 8 scores of this lane's row at a time (-inf: none), in
-// units in which a probability is exp2(unit * score).
+// Running softmax of the rows of a tile: 4 or 8 scores of this lane's row at a time (-inf: none).  A weight is exp(score)
+// over a power of two, 2^ref, the first one that no score so far passes: the exponent of a weight is then a single rounding away
+// from score * log2(e), and the steps and the waves rescale each other's sums exactly.
 template <typename T, int D>
 struct TileSoftmax {
     static constexpr int N = 4 * tile_blocks<T>();
-    float m = -INFINITY;             // maximum of the row (the same in its four lanes)
-    f32x4 l = {0.f, 0.f, 0.f, 0.f};  // sum of the row, four times
-    f32x4 acc[D / 16];
+    float m = -INFINITY;      // largest score of the row (the same in its four lanes)
+    float ref = -0x1p126f;    // (no score yet)
+    float l = 0.f;            // sum of this lane's weights
+    f32x4 acc[D / 16];        // weighted sums, times TileWeights<T>::kScale
     __device__ __forceinline__ TileSoftmax()
     {
 #pragma unroll
-        for (int b = 0; b < D / 16; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < D / 16; ++b) acc[b] = kNothing;
     }
-    __device__ __forceinline__ void step(const float (&sc)[N], float unit, TileWeights<T>& weights)
+    __device__ __forceinline__ void step(const float (&sc)[N], TileWeights<T>& weights)
     {
         float top = sc[0];
 #pragma unroll
         for (int j = 1; j < N; ++j) top = fmaxf(top, sc[j]);
-        const float m_new = fmaxf(m, quad_max(top));
-        if (__any(m_new > m)) {
-            const float corr = __builtin_amdgcn_exp2f((m - (m_new == -INFINITY ? 0.f : m_new)) * unit);
+        m = fmaxf(m, quad_max(top));
+        const float now = m == -INFINITY ? ref : ceilf(m * kLog2e);
+        if (__any(now != ref)) {
+            const float corr = __builtin_amdgcn_exp2f(ref - now);
             l *= corr;
 #pragma unroll
             for (int b = 0; b < D / 16; ++b) acc[b] *= corr;
-            m = m_new;
+            ref = now;
         }
-        const float off = TileWeights<T>::kShift - (m == -INFINITY ? 0.f : m) * unit;
-        float p[N];
+        float p[N], sum[N];
 #pragma unroll
-        for (int j = 0; j < N; ++j) p[j] = __builtin_amdgcn_exp2f(fmaf(sc[j], unit, off));
-        weights.set(p);
-        weights.add_sums(l);
+        for (int j = 0; j < N; ++j) sum[j] = p[j] = __builtin_amdgcn_exp2f(fmaf(sc[j], kLog2e, -ref));
+#pragma unroll
+        for (int h = N / 2; h >= 1; h /= 2)
+#pragma unroll
+            for (int j = 0; j < h; ++j) sum[j] += sum[j + h];
+        l += sum[0];
+        weights.set(p, TileWeights<T>::kScale); // (the scale not in the exponent, which would lose digits to it)
     }
+    // (a score beyond the range of the powers of two gives none of its row a weight)
+    __device__ __forceinline__ bool finite() const { return all_finite<D / 16>(acc) && fabsf(ref) <= 0x1p126f; }
 };
 
 template <typename T, int D, int KEEP>
-__global__ void __launch_bounds__(kWgThreads)
+__global__ void __launch_bounds__(kWgThreads, (tile_waves<T, D>()))
 attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int* __restrict__ runs,
                       const int* __restrict__ row_ptr, const int* __restrict__ col, const float* __restrict__ val,
                       const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, float scale,
@@ -83,6 +96,7 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     static_assert(2 * kPart + 2 * kWave <= kStageFloats, "what comes later fits");
     __shared__ __attribute__((aligned(16))) float shared[kWavesPerWg][kStageFloats];
     __shared__ float part_m[kWavesPerWg + 1][kTileRows], part_l[kWavesPerWg + 1][kTileRows]; // (the last: outside the runs)
+    __shared__ float part_ref[kWavesPerWg][kTileRows];
     const int tile = xcd_logical_block(blockIdx.x, gridDim.x);
     if (tile >= n_tiles) return;
     const RowTile rt = tiles[tile];
@@ -99,12 +113,6 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     f32x4* lds_w = reinterpret_cast<f32x4*>(lds_v + VStage::kBytes / 16);
     TileRow<T, D> q_row;
     q_row.load(q + (size_t)me.row * D, gq);
-    // a score is unit * (value * <q, k>) in powers of two; a negative scale goes into q
-    const float unit = fabsf(scale) * kLog2e;
-    if (scale < 0.f) {
-#pragma unroll
-        for (int i = 0; i < TileRow<T, D>::kChunks; ++i) q_row.c[i] ^= sizeof(T) == 2 ? 0x80008000u : 0x80000000u;
-    }
     TileSoftmax<T, D> sm;
 
     // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 at a time:
@@ -250,11 +258,11 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
                 KStage::read(lds_k, t, lane, k_row);
                 const f32x4 dot = mma_rows<T, D>(k_row, q_row), w = TileSquare<T>::as_scores(lds_w, t, lane);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) sc[4 * t + i] = w[i] * dot[i];
+                for (int i = 0; i < 4; ++i) sc[4 * t + i] = scale * (w[i] * dot[i]);
             }
             if (KEEP != kKeepNothing) { // the scores leave in the order of the values
 #pragma unroll
-                for (int t = 0; t < NT; ++t) TileSquare<T>::as_scores(lds_w, t, lane) = f32x4{sc[4 * t], sc[4 * t + 1], sc[4 * t + 2], sc[4 * t + 3]} * fabsf(scale);
+                for (int t = 0; t < NT; ++t) TileSquare<T>::as_scores(lds_w, t, lane) = f32x4{sc[4 * t], sc[4 * t + 1], sc[4 * t + 2], sc[4 * t + 3]};
                 wave_lds_sync();
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
@@ -277,7 +285,7 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
                 }
             }
             TileWeights<T> weights;
-            sm.step(sc, unit, weights);
+            sm.step(sc, weights);
             TileCols<T, D> v_cols;
 #pragma unroll
             for (int j = 0; j < 4 * NT; ++j) v_cols.load(j, VStage::across(lds_v, 16 * (j / 4) + 4 * gq + j % 4, n));
@@ -287,13 +295,14 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     };
 
     run_columns();
-    const bool again = __syncthreads_or(!all_finite<NB>(sm.acc));
+    const bool again = __syncthreads_or(!sm.finite());
     if (again) sm = TileSoftmax<T, D>();
     rows_outside(again);
 
-    // the partial results, each relative to its own maximum
+    // the partial results, a wave's relative to its power of two, those outside the runs to the exponential of their maximum
     float* part = shared[wave];
-    if (gq == 0) part_m[wave][n] = sm.m * fabsf(scale), part_l[wave][n] = sm.l[0];
+    const float l_row = quad_sum(sm.l);
+    if (gq == 0) part_m[wave][n] = sm.m, part_ref[wave][n] = sm.ref, part_l[wave][n] = l_row;
 #pragma unroll
     for (int e = 0; e < D / 4; ++e) part[n * PAD + (D / 4) * gq + e] = sm.acc[e % NB][e / NB];
     __syncthreads();
@@ -308,8 +317,9 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     for (int x = 0; x < NB; ++x) o[x] = shared[0][kPart + r * PAD + e0 + x] * f;
 #pragma unroll
     for (int w = 0; w < kWavesPerWg; ++w) {
-        f = __builtin_amdgcn_exp2f((part_m[w][r] - top_safe) * kLog2e - TileWeights<T>::kShift);
+        f = __builtin_amdgcn_exp2f(-fmaf(top_safe, kLog2e, -part_ref[w][r]));
         total = fmaf(part_l[w][r], f, total);
+        f *= 1.f / TileWeights<T>::kScale;
 #pragma unroll
         for (int x = 0; x < NB; ++x) o[x] = fmaf(shared[w][r * PAD + e0 + x], f, o[x]);
     }
@@ -345,7 +355,7 @@ hipError_t launch_tiles(int nheads, int M, int N, int nnz, const int* row_ptr, c
 } // namespace
 
 // The tiles of a group plan (plan.groups, with plan.group_counts[3] > 0 of them); arguments as
-// attention_launch, scale not zero.  One head's k or v must not exceed 4 GB (attention_tiles_fit).
+// attention_launch.  One head's k or v must not exceed 4 GB (attention_tiles_fit).
 template <typename T>
 hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
                                   const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,

@@ -38,6 +38,16 @@ constexpr int tile_blocks()
     return sizeof(T) == 2 ? 2 : 1;
 }
 
+// Waves per SIMD that the compiler has to leave registers for.  It is told only where it would otherwise miss by a few the
+// number that LDS allows (fp32: width 32 131 registers instead of 128, width 128 262 and 293 instead of 256): a
+// kernel that is told keeps the accumulators out of the second half of the registers, and with halves that
+// costs more than it gives (two heads of width 32 / 64 / 128: 39.6, 59.8, 125 us left alone, 40.8, 63.1, 129 told).
+template <typename T, int D>
+constexpr int tile_waves()
+{
+    return sizeof(T) == 2 || D == 64 ? 1 : D == 32 ? 4 : 2;
+}
+
 // The sums over the lane groups (LPR lanes each) of N values per lane, shared out: a lane keeps kLeft of
 // the totals, from number value() on (halving what a lane still has to add at every exchange costs a
 // third of a butterfly per value).
@@ -107,26 +117,41 @@ struct TileRow {
     }
 };
 
-__device__ __forceinline__ f32x4 mma_chunk(const __half*, const u32x4& a, const u32x4& b, f32x4 acc)
-{
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), acc, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4 mma_chunk(const float*, const u32x4& a, const u32x4& b, f32x4 acc)
-{
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.x), __uint_as_float(b.x), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.y), __uint_as_float(b.y), acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
-}
-// rows of a (16 of them, m = lane % 16) times rows of b (n = lane % 16)
+constexpr f32x4 kNothing = {0.f, 0.f, 0.f, 0.f};
+
+// Rows of a (16 of them, m = lane % 16) times rows of b (n = lane % 16).  Every instruction has a sum of its own, and
+// the sums meet in a tree, as the lanes' do in the row kernels: along one chain of D products the rounding errors are up
+// to 2.8 times theirs (rms over the square root of D, fp32, D = 32 / 64 / 128: 1.03e-7, 1.44e-7, 2.04e-7 along a chain, 0.62e-7,
+// 0.68e-7, 0.73e-7 here and there; halves 0.44e-7, 0.57e-7, 0.76e-7 against 0.44e-7, 0.52e-7, 0.59e-7, row kernels 0.55e-7, 0.62e-7, 0.67e-7).
+// (Two heads of fp32, width 128: 297 us along a chain, 306 with two instructions a sum, 310 with one.)
 template <typename T, int D>
 __device__ __forceinline__ f32x4 mma_rows(const TileRow<T, D>& a, const TileRow<T, D>& b)
 {
-    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    constexpr int N = TileRow<T, D>::kChunks;
+    f32x4 sum[N];
+    if constexpr (sizeof(T) == 2) {
 #pragma unroll
-    for (int i = 0; i < TileRow<T, D>::kChunks; ++i) acc = mma_chunk(static_cast<const T*>(nullptr), a.c[i], b.c[i], acc);
-    return acc;
+        for (int i = 0; i < N; ++i)
+            sum[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a.c[i]), __builtin_bit_cast(f16x8, b.c[i]), kNothing, 0, 0, 0);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            u32x4 c = a.c[i];
+            asm volatile("" : "+v"(c)); // (the products of a chunk at a time: all of them at once cost up to 128 registers)
+            f32x4 x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(c[j]), __uint_as_float(b.c[i][j]), kNothing, 0, 0, 0);
+            sum[i] = (x[0] + x[1]) + (x[2] + x[3]);
+            asm volatile("" : "+v"(sum[i]));
+        }
+    }
+#pragma unroll
+    for (int h = 1; h < N; h *= 2)
+#pragma unroll
+        for (int i = 0; i < N; i += 2 * h) sum[i] += sum[i + h];
+    return sum[0];
 }
+
 // The dense rows of a step on their way through LDS to operand A: loaded in order (every load 1024 consecutive
 // bytes), stored, and read back along or across their elements.  Where 16 bytes are put spreads the
 // 16 lanes that LDS serves together (lanes 0-3, 12-15, 20-27 and their like) over all of its banks:
@@ -193,49 +218,39 @@ struct TileSquare {
 };
 
 // ---- weights: operand B of the weighted sums -------------------------------------------------
-// fp16 dense operands: a weight is taken as the sum of two halves (22 bits and a sign), so that the
-// products carry what a 32-bit weight would; weights are kept below 2^15 by a power of two.
+// fp16 dense operands: a weight is the sum of two halves, each rounded to nearest.  Weights are kept below 2^15 by a power of
+// two; from 2^-2 on the sum is within 2^-23 of the weight (a 32-bit number: 2^-24), below that within 2^-25 of it in all.
 template <typename T>
 struct TileWeights;
 template <>
 struct TileWeights<__half> {
-    static constexpr float kShift = 12.f; // probabilities are taken times 2^12
+    static constexpr float kScale = 0x1p15f; // probabilities are taken times that
     f16x8 hi, lo;
-    __device__ __forceinline__ void set(const float (&p)[8])
+    // the weights p times a power of two (both parts by v_fma_mix: a product, a difference and a rounding in one)
+    __device__ __forceinline__ void set(const float (&p)[8], float scale)
     {
-        typedef float f32x2 __attribute__((ext_vector_type(2)));
 #pragma unroll
-        for (int j = 0; j < 8; j += 2) {
-            const f16x2 h = __builtin_convertvector(f32x2{p[j], p[j + 1]}, f16x2);
-            const f16x2 l = __builtin_convertvector(f32x2{fmaf((float)h[0], -1.f, p[j]), fmaf((float)h[1], -1.f, p[j + 1])}, f16x2);
-            hi[j] = h[0], hi[j + 1] = h[1], lo[j] = l[0], lo[j + 1] = l[1];
+        for (int j = 0; j < 8; ++j) {
+            hi[j] = (_Float16)(p[j] * scale);
+            lo[j] = (_Float16)fmaf(p[j], scale, -(float)hi[j]);
         }
-    }
-    // acc += the sums of the weights per row, in each of its four elements
-    __device__ __forceinline__ void add_sums(f32x4& acc) const
-    {
-        const f16x8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, hi, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ones, lo, acc, 0, 0, 0);
     }
 };
 template <>
 struct TileWeights<float> {
-    static constexpr float kShift = 0.f;
+    static constexpr float kScale = 1.f;
     float p[4];
-    __device__ __forceinline__ void set(const float (&w)[4])
+    __device__ __forceinline__ void set(const float (&w)[4], float)
     {
 #pragma unroll
         for (int j = 0; j < 4; ++j) p[j] = w[j];
     }
-    __device__ __forceinline__ void add_sums(f32x4& acc) const
-    {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(1.f, p[j], acc, 0, 0, 0);
-    }
 };
 
 // ---- columns: a lane's 4 or 8 dense rows across their elements, operand A of the weighted sums ----
+// (accumulate: halves along one chain of products per wave, the small parts of a step's weights before the large ones; fp32 a
+// chain per step and the steps' sums added, as one chain over a wave's columns - 128 roundings of a growing sum where the row kernels
+// have 72 and a tree - had 1.3 to 1.6 times their error)
 template <typename T, int D>
 struct TileCols;
 template <int D>
@@ -263,8 +278,8 @@ struct TileCols<__half, D> {
                                        __builtin_amdgcn_perm(w[3][nb / 2], w[2][nb / 2], select),
                                        __builtin_amdgcn_perm(w[5][nb / 2], w[4][nb / 2], select),
                                        __builtin_amdgcn_perm(w[7][nb / 2], w[6][nb / 2], select));
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.hi, acc[nb], 0, 0, 0);
             acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.lo, acc[nb], 0, 0, 0);
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.hi, acc[nb], 0, 0, 0);
         }
     }
 };
@@ -287,10 +302,17 @@ struct TileCols<float, D> {
     }
     __device__ __forceinline__ void accumulate(const TileWeights<float>& p, f32x4 (&acc)[kBlocks]) const
     {
+        constexpr int kAtOnce = kBlocks < 4 ? kBlocks : 4;
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int b = 0; b < kBlocks; b += kAtOnce) {
+            f32x4 sum[kAtOnce];
 #pragma unroll
-            for (int nb = 0; nb < kBlocks; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j][nb], p.p[j], acc[nb], 0, 0, 0);
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < kAtOnce; ++i) sum[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[j][b + i], p.p[j], j == 0 ? kNothing : sum[i], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < kAtOnce; ++i) acc[b + i] += sum[i];
+        }
     }
 };
 

@@ -69,6 +69,73 @@ def test_tiles_against_fp64(m, window, shift, extra, d, half, scale):
     assert (probs - torch.exp(scores - stats[rows, 0]) * stats[rows, 1]).abs().max() <= 2e-6
 
 
+def _without_tiles(csr):
+    """The same matrix whose plan says that it has no tiles: its groups go to the kernels for groups and rows."""
+    args = [csr.row_offsets_cpu, csr.column_indices, csr.values, "cuda", csr.m, csr.n, 64]
+    other = RoDeCSR(*args, locality=True)
+    other.plan.counts[3] = other.plan._header[3] = 0
+    return other
+
+
+@pytest.mark.parametrize("sharp", [1.0, 8.0])
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_tiles_are_as_exact_as_the_other_kernels(d, half, sharp):
+    """Errors against fp64 (2-norms), of the output and the gradients, not above those of the kernels on the vector ALUs.
+    Both round every product and every sum once, in trees of the same depth; the 0.1 is for chance, in 65 K values and more."""
+    m, scale, dt = 1024, sharp * d ** -0.5, torch.float16 if half else torch.float32
+    csr, dense = _mask(m, 250, 1, 30, seed=d)
+    assert csr.plan.counts[3] == m // 16
+    heads = max(2, _heads(csr))
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    q, k, v = (t.to(dt) for t in (q, k, v))
+    ins = [t.double().requires_grad_() for t in (q, k, v)]
+    want = _reference(dense, *ins, scale)
+    want = (want,) + torch.autograd.grad(want, ins, g.double())
+    errors = []
+    for c in (csr, _without_tiles(csr)):
+        ins = [t.expand(heads, *t.shape).contiguous() for t in (q, k, v)]
+        out, scores, stats = _attention_call(c, c.values, *ins, scale, "scores")
+        got = (out,) + _attention_backward_call(c, c.transpose(with_values=False)[0], c.transposed_slots(), scores, stats,
+                                                g.expand(heads, m, d).contiguous(), out, *ins, scale)
+        errors.append([((a[0].double() - b).norm() / b.norm()).item() for a, b in zip(got, want)])
+    print(*errors)
+    for tiles, others in zip(*errors):
+        assert 0 < tiles <= 1.1 * others
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_scores_without_range(half):
+    """Infinite and largest scores, in a run and outside it, rows without a finite one: as on the other kernels."""
+    m, d = 96, 64
+    csr, dense = _mask(m, 100, 2, 30, seed=5)
+    values = csr.values.clone()
+    rows = torch.repeat_interleave(torch.arange(m, device="cuda"), (csr.row_offsets[1:] - csr.row_offsets[:-1]).long())
+    inf, most = float("inf"), 0.9 * torch.finfo(torch.float32).max / 16  # (products of 16 below: log2(e) times the score has no range)
+    for row, at, value in ((3, slice(None), -inf), (5, slice(0, 40), -inf), (20, slice(60, 61), most), (21, slice(60, 61), -most), (37, slice(7, 9), -16 * most),
+                           (50, slice(129, 130), most), (52, slice(0, 1), most), (53, slice(0, 1), -inf), (70, slice(50, 51), inf)):
+        picked = (rows == row).nonzero().flatten()
+        values[picked[at]] = value
+    csr = csr.with_values(values)
+    csr._shared = {}
+    other = RoDeCSR(csr.row_offsets_cpu, csr.column_indices, values, "cuda", m, csr.n, 64, locality=False)
+    heads = _heads(csr)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.rand(heads, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n))
+    q[:, [20, 21, 50, 52]] = 0.5
+    k.fill_(0.5)
+    if half:
+        q, k, v = q.half(), k.half(), v.half()
+    for scale in (0.125, 1.0):
+        a, b = (_attention_call(c, c.values, q, k, v, scale, "scores") for c in (csr, other))
+        assert not b[0][:, [3, 70]].isfinite().any() and b[0][:, [5, 20, 21, 37, 50, 52, 53]].isfinite().all()
+        for x, y in zip(a, b):
+            assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isinf(), y.isinf())
+            ok = y.isfinite()
+            torch.testing.assert_close(x[ok], y[ok], rtol=2e-5, atol=2e-5)
+
+
 @pytest.mark.parametrize("half", [False, True])
 def test_non_finite_rows_of_v_stay_in_their_rows(half):
     """A column at either end of a tile's range is held by some of its rows only."""
