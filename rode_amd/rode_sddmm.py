@@ -194,9 +194,12 @@ class RoDeCSR:
     def plans_address(self, spmm_width=None):
         """The struct of ``call_plans`` as the native calls take it: a ``PlansAddress``, which holds
         the struct.  Only a hub plan's struct depends on the width (it carries the workspace)."""
-        if not isinstance(self.plan, rode_sddmm_hip.HubPlan):
-            spmm_width = None
-        key = "plans_address" if spmm_width is None else ("plans_address", spmm_width)
+        key = "plans_address"
+        if spmm_width is not None:
+            if isinstance(self.plan, rode_sddmm_hip.HubPlan):
+                key = ("plans_address", spmm_width)
+            else:
+                spmm_width = None
         address = self._shared.get(key)
         if address is None:
             address = self._shared.setdefault(key, rode_sddmm_hip.PlansAddress(self.call_plans(spmm_width)))
