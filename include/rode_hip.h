@@ -285,6 +285,8 @@ int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_ind
  *                         (most chunks of the residue list have a window: a band).  Knowledge as
  *                         well: SpMM then does not deal column tiles out to the XCDs, which pays
  *                         when dense rows are referenced at random.  Costs time at worst.
+ *   nonzeros              0, or the nonzeros of the matrix: whether that dealing out pays depends
+ *                         on how often a dense row is used.  Costs time at worst.
  * Same results as without a plan, up to the order of the fp32 additions inside a row.
  */
 typedef struct rode_hip_plans {
@@ -299,6 +301,7 @@ typedef struct rode_hip_plans {
     const int* group_counts;
     int seg_length;
     int columns_local;
+    int nonzeros;
 } rode_hip_plans;
 
 /* rode_hip_spmm_ex with plans. */

@@ -192,6 +192,7 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
     if (p->seg_length < 0) return false;
     plan.seg_length = p->seg_length;
     plan.columns_local = p->columns_local != 0;
+    plan.nonzeros = p->nonzeros;
     const bool window = p->window && p->window_rows; // (one without rows: the standard kernels do everything)
     if (p->groups) {
         // a group plan needs its header on the host, and excludes the other plans (their

@@ -46,6 +46,7 @@ struct PlanRef {
     // SpMM: rows of the dense operand as the caller says (0: not said), and (set by spmm_launch) into how
     // many column tiles it is dealt out to the XCDs
     int dense_rows = 0, shards = 0;
+    int nonzeros = 0;           // of the matrix, as the caller says (0: not said)
     bool columns_local = false; // the caller knows that the columns of neighbouring rows lie close together
     // Segment length of the decomposition the lists were made with, 0: not known
     int seg_length = 0;

@@ -63,12 +63,33 @@ constexpr int kPairMaxSharded = 65536;
 // fetched into all eight.  When a row of B is 2, 4 or 8 lines of 128 bytes, C is computed in column
 // tiles of one line and XCD x works on tile x mod lines only: of B it sees one line per row, so that a
 // matrix of up to lines x 4 MB stays in the L2s, and of twice that about half of it does.  The nonzeros'
-// columns and values are read once per tile (8 bytes against 128 gathered).  65 K x 65 K, 1 M nonzeros:
-// width 64 43 -> 35 us, 128 halves 64 -> 39 (with the rows of a single work item stored), width 128 77 -> 63;
-// 16 K x 16 K, width 128: 34 -> 21.  Below 4 MB every L2 holds all of B anyway.  Seven times an L2 per tile
-// is where the gain ends (200 K rows: 254 -> 240 us; 400 K rows of width 64: 472 -> 492), and rows whose
-// columns lie close together share their lines without it (band of 256 in 60 K rows: 32 -> 39).
-constexpr size_t kShardMinBytes = (size_t)4 << 20, kShardMaxTileBytes = (size_t)28 << 20;
+// columns and values are read once per tile (8 bytes against 128 gathered), and every work item is there once per tile.
+// Rows whose columns lie close together share their lines without it (band of 256 in 60 K rows: 32 -> 39).
+//
+// Where it pays (us unsharded -> sharded; dense rows x width, nonzeros per row drawn from a Poisson (p) or a lognormal (l) distribution):
+//   * B above 4 MB, which one L2 does not hold: l 16 K x 128 of 16: 26.7 -> 17.3, 65 K x 128 72 -> 59, 65 K x 64 36.8 -> 32.6; 8.5 K x 128
+//     (4.4 MB) p of 8 5.5 -> 5.9, of 16 10.7 -> 10.0;
+//   * up to 26 MB per tile, where half of a tile and more misses the L2 (l of 16: 200 K x 64 126 -> 120, x 128 243 -> 235; p 212 K x 64
+//     124 -> 128, 400 K x 64 472 -> 492), up to 14 MB with eight tiles (l of 16: 100 K x 256 228 -> 211, 150 K 339 -> 347, 200 K 463 -> 490);
+//   * where a row of B is used less than six times: from 12 MB up to 9 MB per tile (p of 4: 33 K x 64 8.4 -> 8.9, 33 K x 128 15.2 -> 13.1,
+//     65 K x 128 26.6 -> 23.9, 150 K 54.1 -> 56.2; p of 2: 65 K 19.1 either way, 150 K 37.4 -> 40.2);
+//   * where many rows have a block segment beside their tail (p of 28 and more): twice the work items, and more of B has to miss.
+//     Work items of 24 nonzeros and more: from 8 MB on, 16 with eight tiles, 48 with halves (p of 64: 12 K x 128 26.5 -> 29.0,
+//     16 K x 128 43.4 -> 38.5, 24 K x 64 28.1 -> 28.9, 33 K x 64 45.1 -> 39.0, 8.5 K x 256 34.0 -> 38.7, 16 K x 256 84 -> 75, 16 K x 512 halves
+//     69 -> 82, of 50 33 K 155 -> 167, 65 K 382 -> 354).  Smaller ones: from 16 MB on, 32 with eight tiles (p of 40: 12 K x 128 23.6 -> 30.0,
+//     24 K 54.8 -> 56.4, 33 K 79.3 -> 76.3, 33 K x 64 37.0 -> 40.3, 65 K x 64 83 -> 76, 24 K x 256 104 -> 108, 65 K x 256 336 -> 297), not with
+//     halves (p of 36, x 128: 65 K 79.8 -> 82.7, 150 K 188 -> 199; of 40, x 512: 65 K 316 -> 336).
+// items: of both lists; segments: do many rows have one; nonzeros: 0 when the caller did not say.
+inline bool sharding_pays(int lines, bool halves, size_t dense_rows, long long items, bool segments, long long nonzeros)
+{
+    constexpr size_t MB = (size_t)1 << 20;
+    const size_t tile = dense_rows * 128, bytes = tile * lines;
+    if (tile > (lines == 8 ? 14 : 26) * MB || bytes <= 4 * MB) return false;
+    if (nonzeros > 0 && (size_t)nonzeros < 6 * dense_rows && (tile > 9 * MB || bytes < 12 * MB)) return false;
+    if (!segments) return true;
+    if (nonzeros > 0 && nonzeros < 24 * items) return !halves && bytes >= (lines == 8 ? 32 : 16) * MB;
+    return bytes >= (lines < 8 ? 8 : halves ? 48 : 16) * MB;
+}
 
 // Sum over the aligned slots [base, base + cnt) of values * B rows, for this lane's columns
 // of the tile; the first `mask` slots (the previous row's) and the slots past cnt in the
@@ -874,9 +895,9 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
     if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
         constexpr int kLine = 128 / (int)sizeof(T);
         const int lines = n / kLine;
-        const size_t bytes = (size_t)plan.dense_rows * n * sizeof(T);
         // (a plan's kernels have their own ways to share dense rows)
-        if (n % kLine == 0 && (lines == 2 || lines == 4 || lines == 8) && bytes > kShardMinBytes && (size_t)plan.dense_rows * 128 <= kShardMaxTileBytes &&
+        if (n % kLine == 0 && (lines == 2 || lines == 4 || lines == 8) && plan.dense_rows > 0 &&
+            sharding_pays(lines, sizeof(T) == 2, plan.dense_rows, (long long)m1 + m2, 3ll * m1 > m2, plan.nonzeros) &&
             !plan.columns_local && plan.hub == nullptr && plan.groups == nullptr && plan.dev == nullptr) {
             plan.shards = lines;
             return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);

@@ -188,7 +188,8 @@ class RoDeCSR:
         if plans is None:
             # (set once: of two threads' first calls one struct stays, for both)
             plans = self._shared.setdefault(key, rode_sddmm_hip.plans_struct(
-                self.plan, spmm_width, spmm_elem_bytes, True, seg_length=self.config["seg_length"], columns_local=self.columns_local))
+                self.plan, spmm_width, spmm_elem_bytes, True, seg_length=self.config["seg_length"], columns_local=self.columns_local,
+                nonzeros=self.nnz))
         return plans
 
     def plans_address(self, spmm_width=None):

@@ -302,15 +302,18 @@ def group_plan(row_offsets, column_indices, m):
     return GroupPlan(data, list(counts))
 
 
-def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0, columns_local=False):
+def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0, columns_local=False,
+                 nonzeros=0):
     """The ``rode_hip_plans`` struct of one call (keep it alive until the call returns; pass
     it with ``ctypes.byref``).  ``plan``: a ``WindowPlan``, a ``HubPlan``, a ``GroupPlan`` or None.
     ``spmm_width``: for an SpMM call the dense width, so that a hub plan's workspace is
     attached; a hub plan is left out of an SpMM call without the whole-lists promise.
     ``seg_length``: the segment length the lists were made with, 0 when not known.
-    ``columns_local``: the columns of neighbouring rows are known to lie close together."""
+    ``columns_local``: the columns of neighbouring rows are known to lie close together.
+    ``nonzeros``: of the matrix, 0 when not known."""
     p = _lib.Plans()
     p.columns_local = int(columns_local)
+    p.nonzeros = int(nonzeros)
     p.seg_length = int(seg_length or 0)  # (the segment length of the decomposition, when the caller knows it)
     if isinstance(plan, GroupPlan):
         if plan.usable and (spmm_width is None or whole_lists):

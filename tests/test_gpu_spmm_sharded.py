@@ -28,8 +28,9 @@ def _lengths(kind, rng):
 
 @pytest.mark.parametrize("half,width", [(False, 64), (False, 128), (False, 256), (True, 128), (True, 512)])
 @pytest.mark.parametrize("kind", ["one", "short", "long", "mixed"])
-def test_sharded_against_fp64(kind, half, width):
-    n = 4 * 2**20 // (width * (2 if half else 4)) + 3  # just over one L2
+@pytest.mark.parametrize("megabytes", [4, 8, 16, 48])  # (of B: just over an L2, and over the lines that rows with block segments have)
+def test_sharded_against_fp64(kind, half, width, megabytes):
+    n = megabytes * 2**20 // (width * (2 if half else 4)) + 3
     lengths = np.minimum(_lengths(kind, np.random.default_rng(width)), n // 2)
     csr = _matrix(lengths, n, width, seed=width)
     g = torch.Generator(device="cuda").manual_seed(width)

@@ -52,7 +52,7 @@ def test_row_stats_of_other_tensors(kind):
 
 def _stand_in(plan=None):
     csr = object.__new__(RoDeCSR)
-    csr.plan, csr.config, csr.columns_local, csr._shared = plan, {"seg_length": 512}, False, {}
+    csr.plan, csr.config, csr.columns_local, csr.nnz, csr._shared = plan, {"seg_length": 512}, False, 1, {}
     return csr
 
 
