@@ -285,8 +285,10 @@ int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_ind
  *                         (most chunks of the residue list have a window: a band).  Knowledge as
  *                         well: SpMM then does not deal column tiles out to the XCDs, which pays
  *                         when dense rows are referenced at random.  Costs time at worst.
- *   nonzeros              0, or the nonzeros of the matrix: whether that dealing out pays depends
- *                         on how often a dense row is used.  Costs time at worst.
+ *   nonzeros              0, or the nonzeros of the matrix.  With it a call may leave a locality plan
+ *                         unused where the window kernels do not pay (short rows, a last round of few
+ *                         chunks), and dealing tiles out depends on how often a dense row is used.
+ *                         Costs time at worst.
  * Same results as without a plan, up to the order of the fp32 additions inside a row.
  */
 typedef struct rode_hip_plans {

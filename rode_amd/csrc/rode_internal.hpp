@@ -29,6 +29,7 @@ constexpr int kOnlyMask = kSpmmOnlyBlock | kSpmmOnlyResidue | kSpmmOnlyHub;
 // A locality plan (rode_plan.hip): device array, and optionally a host copy of its four
 // header ints (chunk counts), with which launches that have nothing to do are left out.
 struct PlanRef {
+    void no_window() { dev = nullptr, rows = nullptr, host_counts = nullptr; }
     const int* dev = nullptr;         // descriptors
     const void* rows = nullptr;       // planned rows of the chunks with a window
     const int* host_counts = nullptr;
@@ -51,6 +52,33 @@ struct PlanRef {
     // Segment length of the decomposition the lists were made with, 0: not known
     int seg_length = 0;
 };
+
+// Do the window kernels pay for a call?  They take kWindowWgs chunks at a time, and a last round with few of them
+// takes as long as a full one; against the standard kernels a full round gains the more, the more slots a row has
+// (the window is copied either way).  full_round: that gain at s slots a row, base + per_slot * s, measured on bands of 128 to
+// 256 in 130 K rows (1030 chunks); large: what becomes of it when the dense operands outgrow the last-level cache (256 MB; above
+// large_from bytes of them).  us, standard -> window kernels, 9 / 14 / 18 / 27 slots:
+//   SDDMM  f32 x 128    45 -> 38, 55 -> 43, 64 -> 46, 83 -> 53        {1.24, 0.026}
+//          f32 x 64     23.7 -> 25.2, 29 -> 27.4, 33.4 -> 29.1, 44 -> 33.7   {0.95, 0.0245}; 512 K rows 84 -> 90, 106 -> 102, 126 -> 108, 204 -> 129
+//          f16 x 128    24.1 -> 26.7, 29.4 -> 29.5, 33.8 -> 32.0, 44 -> 37.5 {0.92, 0.0195}; 512 K rows 85 -> 96, 107 -> 109, 127 -> 117, 203 -> 139
+//   SpMM   f32 x 128    35 -> 40, 43 -> 45, 51 -> 48, 67 -> 55        {0.87, 0.0237}; 512 K rows 199 -> 159, 253 -> 184, 292 -> 187, 380 -> 213
+//          f32 x 64     19.1 -> 25.4, 23.2 -> 27.8, 27 -> 29, 35.5 -> 32.6   {0.715, 0.0235}; 704 K rows 98 -> 111, 150 -> 135; 1 M rows 192 -> 174, 251 -> 199, 288 -> 204, 383 -> 233
+//          f16 x 128    23.9 -> 31.1, 28.5 -> 35.3, 32.6 -> 38.3, 41 -> 44   {0.79, 0.0113}; 65 K rows of 14 13.4 -> 15.9; 1 M rows 273 -> 223, 341 -> 262, 384 -> 272, 475 -> 318
+//          f64 x 32     22.4 -> 29.1, 26.8 -> 30.9, 31.3 -> 32.0, 40 -> 36.8 {0.75, 0.0228}; 704 K rows 112 -> 133, 186 -> 152; 1 M rows 208 -> 190, 269 -> 214, 313 -> 219, 411 -> 249
+// The number of nonzeros not said: the caller wants the plan used.
+struct WindowGain {
+    float base, per_slot, large;
+    size_t large_from;
+};
+inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes, const WindowGain& full_round)
+{
+    if (plan.dev == nullptr || plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) return true;
+    const int chunks = plan.host_counts[0], rounds = (chunks + round - 1) / round;
+    const float slots = plan.nonzeros < 31ll * m2 ? (float)plan.nonzeros / (float)m2 : 31.f;
+    float gain = full_round.base + full_round.per_slot * slots;
+    if (2 * (size_t)m2 * row_bytes > full_round.large_from) gain *= full_round.large;
+    return gain * (float)chunks >= (float)rounds * (float)round;
+}
 
 hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* plan, hipStream_t stream);
 

@@ -370,6 +370,7 @@ constexpr int kResidueWindowRowsMax = 512; // dense rows of one window (9 bits o
 // Do the window kernels take dense rows of so many bytes?  More than one tile of 128 bytes (with a single tile a
 // window is not used often enough to repay its copy), and no more than their 32-bit offsets into a window reach.
 constexpr bool window_takes(size_t row_bytes) { return row_bytes > 128 && row_bytes <= (1ull << 32) / kResidueWindowRowsMax; }
+constexpr int kWindowWgs = 256; // workgroups of the window kernels, one per CU: they take the chunks in rounds of that many
 
 // Window of one chunk: dense rows [w0, w0 + wn); wn == 0: no window.  slots / misses: how
 // many nonzero slots the chunk has / how many of them fall outside the window.

@@ -547,20 +547,18 @@ hipError_t launch_edge(bool edge, int m1, int m2, int k, const int* block_rows, 
 // k: any positive multiple of the 128-bit vector width (4 for fp32, 8 for fp16) up to 512.
 // 32, 64 and 128 (the reference has 32 and 128) run without any bounds test.  Chunks of the
 // residue list for which `plan` holds a window go to the window kernel when a dense row
-// is wider than one 128-byte tile (with a single tile the window is not reused often
-// enough to repay its staging).
+// is wider than one 128-byte tile (window_takes) and that pays (window_pays).
 template <typename T>
 hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int* residue_rows, const int* st_off,
                         const int* row_ptr, const int* col, const float* val, const T* lhs, const T* rhs,
                         float* out, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
     if (k <= 0 || k % DenseVec<T>::kElems != 0 || k > 512) return hipErrorInvalidValue;
-    // the window kernels are for rows of more than one 128-byte tile
-    if ((size_t)k * sizeof(T) <= 128) {
-        plan.dev = nullptr;
-        plan.rows = nullptr;
-        plan.host_counts = nullptr;
-    }
+    constexpr WindowGain kWide = {1.24f, 0.026f, 1.f, ~(size_t)0}, kNarrow = {0.95f, 0.0245f, 0.82f, (size_t)240 << 20},
+                         kHalves = {0.92f, 0.0195f, 0.82f, (size_t)240 << 20};
+    const size_t row_bytes = (size_t)k * sizeof(T);
+    if (!window_takes(row_bytes) || !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
+        plan.no_window();
 #define RODE_SDDMM_CASE(KT, NS)                                                                                   \
     return launch_edge<T, KT, NS>(k != (KT) * (NS), m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, \
                                   lhs, rhs, out, plan, s1, s2)

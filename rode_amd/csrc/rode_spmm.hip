@@ -877,7 +877,8 @@ int spmm_overwrite_limit(int m1, bool hub_plan) { return m1 >= kOwnedMinSegments
 // dense row is cut into tiles of 32, 64 or 128 columns (at most 32 lanes per tile row);
 // the tile width with the least padding wins, the widest on a tie.  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
-// which `plan` holds a window go to the window kernel (window_takes; other widths ignore the plan).
+// which `plan` holds a window go to the window kernel where it takes the
+// width (window_takes) and pays (window_pays).
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
@@ -885,12 +886,13 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
 {
     static_assert(std::is_same<typename SpmmAcc<T>::type, typename DenseVec<T>::Acc>::value, "accumulation type");
     if (n <= 0 || n % DenseVec<T>::kElems != 0) return hipErrorInvalidValue;
-    // (500 K rows of 32 doubles, two tiles, band of 256: 0.204 -> 0.131 ms)
-    if (!window_takes((size_t)n * sizeof(T))) {
-        plan.dev = nullptr;
-        plan.rows = nullptr;
-        plan.host_counts = nullptr;
-    }
+    constexpr size_t kLarge = (size_t)300 << 20;
+    constexpr WindowGain kWide = {0.87f, 0.0237f, 1.17f, kLarge}, kNarrow = {0.715f, 0.0235f, 1.1f, kLarge},
+                         kHalves = {0.79f, 0.0113f, 1.17f, kLarge}, kDoubles = {0.75f, 0.0228f, 1.07f, kLarge};
+    const size_t row_bytes = (size_t)n * sizeof(T);
+    if (!window_takes(row_bytes) ||
+        !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
+        plan.no_window();
     constexpr int kMaxTile = 32 * DenseVec<T>::kElems >= 128 ? 128 : 32 * DenseVec<T>::kElems;
     if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
         constexpr int kLine = 128 / (int)sizeof(T);

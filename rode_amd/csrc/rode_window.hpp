@@ -29,7 +29,6 @@ namespace rode {
 
 constexpr int kResLanes = 8;                                   // lanes per residue row: 8 x 16 bytes = one 128-byte tile row
 constexpr int kResThreads = kPlanResidueChunk * kResLanes;     // a workgroup takes a chunk
-constexpr int kResWgs = 256;                                   // one per CU
 constexpr int kResWinVecs = kResidueWindowRowsMax * kResLanes; // 16-byte pieces of a window
 constexpr int kRecordVecs = (int)sizeof(PlannedChunk) / 16;    // ... of a chunk's record
 constexpr int kRecordRoom = (kRecordVecs + kWave - 1) / kWave * kWave; // (a wave copies 64 pieces, needed or not)
@@ -38,7 +37,7 @@ static_assert(kResWinVecs * 16 == 65536, "the buffer of a window is a bit above 
 static_assert((2 * kResWinVecs + 2 * kRecordRoom) * 16 <= 160 * 1024, "LDS of a CU");
 static_assert(kResidueWindowRowsMax == 512 && kBlockItems == 32, "a plan entry holds 9 bits of window row and 5 of slot");
 
-inline int window_grid(int m2) { return min(kResWgs, (plan_residue_chunks(m2) + kXcds - 1) / kXcds * kXcds); }
+inline int window_grid(int m2) { return min(kWindowWgs, (plan_residue_chunks(m2) + kXcds - 1) / kXcds * kXcds); }
 
 // The chunks of one workgroup: a contiguous share of the list per XCD, adjacent chunks to its
 // workgroups at the same time (their windows overlap), chunks without a window left out.

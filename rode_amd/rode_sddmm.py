@@ -38,7 +38,12 @@ class RoDeCSR:
 
     DEFAULT_CONFIG = {"seg_length": 512, "k_block": 32, "vec_len": 4}  # for a k that is not in CONFIGS
     MAX_K = 512
-    PLAN_MIN_CHUNKS = 512  # windowed chunks of 128 residue rows below which "auto" drops the plan
+    # Windowed chunks of 128 residue rows below which "auto" drops the plan: two full rounds of the window
+    # kernels.  With fewer, what is won by some calls (us without -> with a plan, 400 chunks of rows of 27: SDDMM
+    # of width 128 34.8 -> 22.9, of 64 18.8 -> 14.8, of 128 halves 18.8 -> 16.3, SpMM of 128 28.3 -> 23.7) others lose
+    # (SpMM of 128 halves 15.6 -> 17.9; rows of 9: 8.9 -> 11.0 and 9.6 -> 12.4), and the plan has to be made.  From
+    # here on every call decides for itself (what counts there: how full the last round is, and slots per row).
+    PLAN_MIN_CHUNKS = 512
 
     def __init__(self, row_offsets, column_indices, values, device, m, n, k=128, config=None, locality="auto"):
         if not (isinstance(k, int) and 0 < k <= self.MAX_K and k % 4 == 0):
@@ -113,10 +118,10 @@ class RoDeCSR:
     def _preprocess(self):
         """Row decomposition on the GPU; the index arrays never visit the host."""
         # Locality plan: chunks of the residue list whose dense rows cluster in a window that
-        # fits LDS (banded matrices) go to the window kernels.  Kept only when it pays:
+        # fits LDS (banded matrices) go to the window kernels.  Kept only when it can pay:
         # "auto" wants windows on at least half of the chunks and enough of them to fill the
-        # GPU twice (a few windowed chunks only add launches); True keeps any plan with a
-        # window; False makes none.  Unless another kind of plan may come first, its
+        # GPU twice, and a call then uses it where its rows are long and its chunks many enough; True
+        # keeps any plan with a window and uses it always; False makes none.  Unless another kind of plan may come first, its
         # descriptors are queued along with the decomposition.
         others = self.locality and (self._may_group() or self._may_hub())
         rode_sddmm_hip._check_input(self.row_offsets, "row_offsets")
@@ -138,6 +143,7 @@ class RoDeCSR:
             enough = plan.windowed >= max(self.PLAN_MIN_CHUNKS, (plan.counts[0] + 1) // 2)
             if plan.windowed > 0 and (self.locality is True or enough):
                 self.plan = rode_sddmm_hip.window_plan_rows(plan, res, m2, self.row_offsets, self.column_indices)
+                plan.nonzeros = 0 if self.locality is True else self.nnz
 
     # A hub plan is made when the rows of at least HUB_MIN_LEN nonzeros (and 8 per 4096
     # columns) hold a tenth of the matrix and the matrix has at least HUB_MIN_SLABS times 4096

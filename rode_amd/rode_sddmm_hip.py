@@ -111,6 +111,7 @@ class WindowPlan:
         self.rows = rows                                       # planned rows of the chunks with a window (device bytes)
         self.counts = counts                                   # list of 4 ints
         self._header = (ctypes.c_int * 4)(*counts)             # what the C ABI reads
+        self.nonzeros = 0                                      # of the matrix: calls use the plan where it pays; 0: always
 
     @property
     def windowed(self):
@@ -327,6 +328,8 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
     elif plan is not None and plan.rows is not None:
         p.window, p.window_rows = plan.data.data_ptr(), plan.rows.data_ptr()
         p.window_counts = ctypes.addressof(plan._header)
+        p.nonzeros = plan.nonzeros
+        p.columns_local = int(columns_local or 2 * plan.windowed > plan.counts[0])
     return p
 
 

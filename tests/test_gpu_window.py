@@ -7,7 +7,7 @@ import torch
 
 import oracle
 from gpu_common import DEV, TOL_F16, TOL_F32, round_half, t
-from rode_amd import RoDeCSR, rode_sddmm, rode_spmm, workloads
+from rode_amd import RoDeCSR, rode_sddmm, rode_sddmm_hip, rode_spmm, workloads
 
 pytestmark = pytest.mark.gpu
 
@@ -195,3 +195,26 @@ def test_very_wide_operand(width):
     for at in (0, 8 * rng.integers(width // 8), width - 64):
         want = dense @ B[:, at:at + 64].double()
         assert (C[:, at:at + 64].double() - want).abs().max() <= 1e-5 * want.abs().max()
+
+
+@pytest.mark.parametrize("per_row,chunks", [(9, 513), (14, 640), (27, 513)])
+@pytest.mark.parametrize("k,dtype", [(128, torch.float32), (64, torch.float32), (128, torch.float16), (32, torch.float64)])
+def test_calls_that_may_leave_the_plan_unused(per_row, chunks, k, dtype):
+    """"auto" uses a plan where it pays, locality=True always: the same products, within the rounding of their order."""
+    m = 128 * chunks - 5
+    gen = torch.Generator(device=DEV).manual_seed(per_row)
+    row = torch.arange(m, device=DEV)
+    pick = torch.rand(m, 128, device=DEV, generator=gen).argsort(1)[:, :per_row].sort(1)[0]
+    col = ((row - 64).clamp(0, m - 128)[:, None] + pick).flatten().int()
+    ro, val = torch.arange(0, m * per_row + 1, per_row, dtype=torch.int32), torch.rand(m * per_row, device=DEV, generator=gen) - 0.5
+    auto, always = (RoDeCSR(ro, col, val, DEV, m, m, k, locality=how) for how in ("auto", True))
+    assert auto.plan.windowed == always.plan.windowed == chunks and auto.plan.nonzeros == auto.nnz and always.plan.nonzeros == 0
+    B, L = (torch.randn(m, k, device=DEV, generator=gen).to(dtype) for _ in range(2))
+    if dtype == torch.float64:
+        a, b = (rode_sddmm_hip.spmm_forward(c.block_indices, c.residue_indices, c.st_offsets, c.m1, c.m2, c.row_offsets, c.column_indices,
+                                            c.values.double(), m, m, B, plan=c.plan) for c in (auto, always))
+        assert (a - b).abs().max() <= 1e-14 * b.abs().max()
+        return
+    for op in (lambda c: rode_spmm(c, B), lambda c: rode_sddmm(c, L, B)):
+        a, b = op(auto), op(always)
+        assert (a - b).abs().max() <= 2e-6 * b.abs().max()
