@@ -32,8 +32,9 @@ namespace {
 // (split, jump: the slots are [base, base + split) followed by [base + split + jump, ...):
 // a row with a hole that somebody else works on; split >= cnt for one plain range.
 // AHEAD: the next step's columns and values are on their way while this one's dense rows arrive.  Costs a
-// quarter of the waves in registers: for rows of many steps on a full GPU (power-law benchmark, 64 halves:
-// 0.956 -> 0.943 ms; 300 K rows of width 128: 0.647 -> 0.637), not for small matrices (14 K rows of 40: 24.7 -> 26.1 us).)
+// quarter of the waves in registers and gives 0 to 1.5 % where block segments have a launch of their own (this switch
+// alone, us: power law 2 M x 64 halves 949 -> 945, 2 M x 128 3727 -> 3715, 300 K x 128 645 -> 637, of halves 338 -> 333; 400 K rows of 100,
+// width 64 1456 -> 1444; lognormal 65 K either way); not for small matrices (14 K rows of 40: 24.7 -> 26.1).
 template <typename T, int KT, int NS, bool EDGE, bool AHEAD>
 __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int cnt, int split, int jump, int k, int lane,
                                                 int* lds_cols,

@@ -157,6 +157,27 @@ def test_non_finite_rows_of_v_stay_in_their_rows(half):
 
 
 @pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_every_head_has_operands_of_its_own(d, half):
+    m, dt = 336, torch.float16 if half else torch.float32
+    csr, dense = _mask(m, 300, 1, 40, seed=d, short_rows=(100,))
+    assert csr.plan.counts[3] == m // 16 - 1
+    heads, scale = _heads(csr), 0.2
+    assert heads > 8
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v, g = (torch.randn(heads, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    ins = [t.to(dt).requires_grad_() for t in (q, k, v)]
+    out = sparse_attention(csr, *ins, scale=scale)
+    grads = torch.autograd.grad(out, ins, g)
+    for h in (0, 1, heads // 2, heads - 1):
+        one = [t[h].detach().double().requires_grad_() for t in ins]
+        want = _reference(dense, *one, scale)
+        assert (out[h].double() - want).abs().max() <= 2e-5 * want.abs().max()
+        for a, b in zip(grads, torch.autograd.grad(want, one, g[h].double())):
+            assert (a[h].double() - b).norm() <= (2e-3 if half else 1e-5) * b.norm()
+
+
+@pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("scale", [0.0, -0.0, 1e-42])
 def test_a_scale_of_zero_weighs_all_columns_alike(scale, half):
     m, d, dt = 48, 64, torch.float16 if half else torch.float32
