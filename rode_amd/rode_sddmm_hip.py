@@ -35,12 +35,15 @@ def _check_data(x, name):
     _check(x.data_ptr() != 0 or x.numel() == 0, f"{name} has no data")
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(device):
     """Raw handle of PyTorch's current stream on ``device`` (the direct lookup costs a
     fraction of a microsecond; building a ``torch.cuda.Stream`` object costs several)."""
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None and device.index is not None:
-        return raw(device.index)
+    index = device.index
+    if index is not None and _raw_stream is not None:
+        return _raw_stream(index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
