@@ -3,7 +3,7 @@
 //
 // A small matrix takes a few microseconds on the GPU, so its calls are bound by what the host
 // does around the launch: argument checks, an allocation and the launch itself cost 10-11 us
-// through ctypes, 3-4 us here.  The functions take the ordinary case only - plain float32 or
+// through ctypes, 5 us here.  The functions take the ordinary case only - plain float32 or
 // float16 tensors on the current GPU, contiguous, nothing to differentiate - and return None
 // for every other one, which the Python layer then handles (or refuses with its own message).
 //

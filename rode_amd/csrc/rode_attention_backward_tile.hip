@@ -18,8 +18,8 @@
 // there: dq is 2e-4 to 7e-4 off with and without tiles.
 //
 // Measured (16 384 rows, window 512 and 64 random columns, width 64, one head; forward and both gradient kernels), against
-// four rows at a time on the vector ALUs: 0.330 -> 0.277 ms, halves 0.259 -> 0.222.  The row pass is now bound by the
-// staging of v and k, by the waves in flight (174 registers: two per SIMD) and by 190 MB of
+// four rows at a time on the vector ALUs: 0.330 -> 0.279 ms, halves 0.259 -> 0.21; the row pass itself 0.130 -> 0.088.  It is now bound by the
+// staging of v and k, by the waves in flight (184 registers: two per SIMD) and by 190 MB of
 // values, scores, slots and pairs.  Tried: three waves per SIMD (fp16 spills, 0.250; fp32 0.282).
 #include "rode_tile.hpp"
 #include "rode_units.hpp"

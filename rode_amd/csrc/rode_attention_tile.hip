@@ -13,7 +13,7 @@
 // row by row.
 //
 // Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with
-// four rows at a time on the vector ALUs, 0.219 here; eight heads in fp32 0.693 -> 0.473.  Of the 0.219
+// four rows at a time on the vector ALUs, 0.219 here; eight heads in fp32 0.693 -> 0.423.  Of the 0.219
 // about 0.06 are the columns of the run, 0.11 the nonzeros outside it (11 % of all; their dense rows
 // ask the vector memory pipe for 64 B/clk/CU half of the time, a quarter of them misses L2), 0.02 a
 // workgroup's start and end.  What was slow on the way: dense rows and values loaded straight into
