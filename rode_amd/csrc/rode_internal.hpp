@@ -56,19 +56,23 @@ struct PlanRef {
 // Do the window kernels pay for a call?  They take kWindowWgs chunks at a time, and a last round with few of them
 // takes as long as a full one; against the standard kernels a full round gains the more, the more slots a row has
 // (the window is copied either way).  full_round: that gain at s slots a row, base + per_slot * s, measured on bands of 128 to
-// 256 in 130 K rows (1030 chunks); large: what becomes of it when the dense operands outgrow the last-level cache (256 MB; above
-// large_from bytes of them).  us, standard -> window kernels, 9 / 14 / 18 / 27 slots:
-//   SDDMM  f32 x 128    45 -> 38, 55 -> 43, 64 -> 46, 83 -> 53        {1.24, 0.026}
-//          f32 x 64     23.7 -> 25.2, 29 -> 27.4, 33.4 -> 29.1, 44 -> 33.7   {0.95, 0.0245}; 512 K rows 84 -> 90, 106 -> 102, 126 -> 108, 204 -> 129
-//          f16 x 128    24.1 -> 26.7, 29.4 -> 29.5, 33.8 -> 32.0, 44 -> 37.5 {0.92, 0.0195}; 512 K rows 85 -> 96, 107 -> 109, 127 -> 117, 203 -> 139
-//   SpMM   f32 x 128    35 -> 40, 43 -> 45, 51 -> 48, 67 -> 55        {0.87, 0.0237}; 512 K rows 199 -> 159, 253 -> 184, 292 -> 187, 380 -> 213
-//          f32 x 64     19.1 -> 25.4, 23.2 -> 27.8, 27 -> 29, 35.5 -> 32.6   {0.715, 0.0235}; 704 K rows 98 -> 111, 150 -> 135; 1 M rows 192 -> 174, 251 -> 199, 288 -> 204, 383 -> 233
-//          f16 x 128    23.9 -> 31.1, 28.5 -> 35.3, 32.6 -> 38.3, 41 -> 44   {0.79, 0.0113}; 65 K rows of 14 13.4 -> 15.9; 1 M rows 273 -> 223, 341 -> 262, 384 -> 272, 475 -> 318
-//          f64 x 32     22.4 -> 29.1, 26.8 -> 30.9, 31.3 -> 32.0, 40 -> 36.8 {0.75, 0.0228}; 704 K rows 112 -> 133, 186 -> 152; 1 M rows 208 -> 190, 269 -> 214, 313 -> 219, 411 -> 249
+// 256 in 130 K rows (1024 chunks); larger, largest: what becomes of it where the dense operands come near the size of the
+// last-level cache (256 MB) and where they outgrow it (SDDMM: between the two the standard kernels still hit it, the copied windows
+// no longer do; SpMM: the standard kernels lose it first).  us, standard -> window kernels, 9 / 14 / 18 / 27 slots:
+//   SDDMM  f32 x 128    45 -> 32, 55 -> 36, 63 -> 38, 82 -> 44        1 M rows 358 -> 292, 458 -> 328, 544 -> 335, 740 -> 395
+//          f32 x 64     24.3 -> 22.2, 29.4 -> 23.7, 34.1 -> 25.4, 44.5 -> 29.8   524 K rows 86 -> 94, 107 -> 108, 128 -> 112, 202 -> 132; 1 M rows 184 -> 178, 240 -> 199, 287 -> 209, 396 -> 247
+//          f16 x 128    24.2 -> 24.2, 29.7 -> 27.1, 34.5 -> 29.5, 44.4 -> 34.3   524 K rows 89 -> 103, 112 -> 117, 133 -> 128, 203 -> 148; 1 M rows 184 -> 193, 241 -> 217, 289 -> 233, 396 -> 278
+//   SpMM   f32 x 128    35 -> 34, 43 -> 39, 50 -> 41, 67 -> 46        524 K rows 200 -> 161, 254 -> 186, 293 -> 191, 384 -> 217
+//          f32 x 64     19.7 -> 22.1, 23.4 -> 24.1, 27.2 -> 25.1, 35.5 -> 27.9   717 K rows 91 -> 104, 144 -> 139, 203 -> 143, 271 -> 166; 1 M rows 196 -> 175, 253 -> 198, 289 -> 203, 381 -> 231
+//          f16 x 128    23.9 -> 27.5, 28.7 -> 31.7, 32.8 -> 33.3, 41 -> 40       717 K rows 116 -> 156, 188 -> 184, 265 -> 195, 338 -> 228; 1 M rows 272 -> 223, 339 -> 261, 383 -> 272, 473 -> 318
+//          f64 x 32     22.4 -> 29.1, 26.8 -> 30.9, 31.3 -> 32.0, 40 -> 36.8 (1030 chunks); 704 K rows 112 -> 133, 186 -> 152; 1 M rows 208 -> 190, 269 -> 214, 313 -> 219, 411 -> 249
 // The number of nonzeros not said: the caller wants the plan used.
 struct WindowGain {
-    float base, per_slot, large;
-    size_t large_from;
+    float base, per_slot;
+    float larger;       // above larger_mb MiB of dense operands ...
+    size_t larger_mb;
+    float largest;      // ... and above largest_mb
+    size_t largest_mb;
 };
 inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes, const WindowGain& full_round)
 {
@@ -76,7 +80,8 @@ inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes
     const int chunks = plan.host_counts[0], rounds = (chunks + round - 1) / round;
     const float slots = plan.nonzeros < 31ll * m2 ? (float)plan.nonzeros / (float)m2 : 31.f;
     float gain = full_round.base + full_round.per_slot * slots;
-    if (2 * (size_t)m2 * row_bytes > full_round.large_from) gain *= full_round.large;
+    const size_t mb = 2 * (size_t)m2 * row_bytes >> 20;
+    gain *= mb >= full_round.largest_mb ? full_round.largest : mb >= full_round.larger_mb ? full_round.larger : 1.f;
     return gain * (float)chunks >= (float)rounds * (float)round;
 }
 

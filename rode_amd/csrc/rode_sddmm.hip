@@ -555,8 +555,8 @@ hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int*
                         float* out, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
     if (k <= 0 || k % DenseVec<T>::kElems != 0 || k > 512) return hipErrorInvalidValue;
-    constexpr WindowGain kWide = {1.24f, 0.026f, 1.f, ~(size_t)0}, kNarrow = {0.95f, 0.0245f, 0.82f, (size_t)240 << 20},
-                         kHalves = {0.92f, 0.0195f, 0.82f, (size_t)240 << 20};
+    constexpr WindowGain kWide = {1.24f, 0.026f, 1.f, 0, 1.f, 0}, kNarrow = {0.95f, 0.0245f, 0.82f, 210, 0.92f, 370},
+                         kHalves = {0.92f, 0.0155f, 0.86f, 210, 0.92f, 345};
     const size_t row_bytes = (size_t)k * sizeof(T);
     if (!window_takes(row_bytes) || !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
         plan.no_window();

@@ -888,9 +888,8 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
 {
     static_assert(std::is_same<typename SpmmAcc<T>::type, typename DenseVec<T>::Acc>::value, "accumulation type");
     if (n <= 0 || n % DenseVec<T>::kElems != 0) return hipErrorInvalidValue;
-    constexpr size_t kLarge = (size_t)300 << 20;
-    constexpr WindowGain kWide = {0.87f, 0.0237f, 1.17f, kLarge}, kNarrow = {0.715f, 0.0235f, 1.1f, kLarge},
-                         kHalves = {0.79f, 0.0113f, 1.17f, kLarge}, kDoubles = {0.75f, 0.0228f, 1.07f, kLarge};
+    constexpr WindowGain kWide = {0.87f, 0.0237f, 1.17f, 300, 1.17f, 300}, kNarrow = {0.715f, 0.0235f, 1.f, 380, 1.17f, 380},
+                         kHalves = {0.79f, 0.0113f, 1.07f, 270, 1.17f, 380}, kDoubles = {0.75f, 0.0228f, 1.f, 360, 1.17f, 360};
     const size_t row_bytes = (size_t)n * sizeof(T);
     if (!window_takes(row_bytes) ||
         !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
