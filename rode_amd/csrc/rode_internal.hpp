@@ -130,6 +130,12 @@ hipError_t attention_backward_tiles_launch(int nheads, int M, int N, int nnz, in
                                            const T* v, float scale, const int* t_slot, float* dq, float* pz, const int* plan,
                                            hipStream_t stream);
 
+// (rode_attention_backward_cols_tile.hip) the column pass for the tiles of a group plan of the transposed pattern; plan: that plan
+template <typename T>
+hipError_t attention_backward_cols_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* t_row_ptr, const int* t_col,
+                                                const float* pz, const float* g, const T* q, float* dk, float* dv, const int* plan,
+                                                hipStream_t stream);
+
 template <typename T>
 hipError_t attention_backward_cols_launch(int nheads, int M, int N, int nnz, int d, const int* t_row_ptr, const int* t_col,
                                           const float* pz, const float* g, const T* q, float* dk, float* dv, PlanRef plan,

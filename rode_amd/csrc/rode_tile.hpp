@@ -157,11 +157,12 @@ __device__ __forceinline__ f32x4 mma_rows(const TileRow<T, D>& a, const TileRow<
 // 16 lanes that LDS serves together (lanes 0-3, 12-15, 20-27 and their like) over all of its banks:
 //   ALONG: chunk c of row r at position c ^ f(r) of the row (16 rows are read at one c);
 //   else (across, TileCols): the rows of lanes 16 apart, four apart in r, in different parts of 256 bytes.
-template <typename T, int D, bool ALONG>
+template <typename T, int D, bool ALONG, int ROWS = 16 * tile_blocks<T>()>
 struct TileStage {
     static constexpr int kPerRow = D * (int)sizeof(T) / 16; // 16-byte chunks of a row
-    static constexpr int kLoads = 16 * tile_blocks<T>() * kPerRow / kWave;
-    static constexpr int kBytes = 16 * tile_blocks<T>() * kPerRow * 16;
+    static constexpr int kLoads = ROWS * kPerRow / kWave;
+    static_assert(ROWS * kPerRow % kWave == 0, "whole loads");
+    static constexpr int kBytes = ROWS * kPerRow * 16;
     u32x4 x[kLoads];
     static __device__ __forceinline__ int place(int row, int c)
     {
@@ -298,6 +299,14 @@ struct TileCols<float, D> {
                 const float4 v = *reinterpret_cast<const float4*>(at + b);
                 x[j][b] = v.x, x[j][b + 1] = v.y, x[j][b + 2] = v.z, x[j][b + 3] = v.w;
             }
+        }
+    }
+    __device__ __forceinline__ void load(int j, const __half* at) // (widened)
+    {
+#pragma unroll
+        for (int b = 0; b < kBlocks; b += 2) {
+            const float2 v = __half22float2(*reinterpret_cast<const __half2*>(at + b));
+            x[j][b] = v.x, x[j][b + 1] = v.y;
         }
     }
     __device__ __forceinline__ void accumulate(const TileWeights<float>& p, f32x4 (&acc)[kBlocks]) const

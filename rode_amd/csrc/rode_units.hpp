@@ -256,4 +256,52 @@ __device__ __forceinline__ float softmax_step(float sc, bool live, float& m_run,
     return p;
 }
 
+// ---- attention, column pass of the gradient ----------------------------------------
+// Lane layout of the column pass for every operand type: D / 4 lanes per dense row, four
+// elements each (g is fp32 whatever q is, and both feed accumulators of the same shape).
+__device__ __forceinline__ void load4(const float* p, float (&out)[4])
+{
+    const float4 t = *reinterpret_cast<const float4*>(p);
+    out[0] = t.x; out[1] = t.y; out[2] = t.z; out[3] = t.w;
+}
+__device__ __forceinline__ void load4(const __half* p, float (&out)[4])
+{
+    const uint2 raw = *reinterpret_cast<const uint2*>(p);
+    const float2 lo = __half22float2(*reinterpret_cast<const __half2*>(&raw.x));
+    const float2 hi = __half22float2(*reinterpret_cast<const __half2*>(&raw.y));
+    out[0] = lo.x; out[1] = lo.y; out[2] = hi.x; out[3] = hi.y;
+}
+
+// dv += p * g[row], dk += dz * q[row] over the slot quads {first_quad, first_quad + stride, ...}
+// < nquads of a staged step (rows, p and dz of the slots in LDS).
+template <typename T, int D, int QUADS_MAX, bool FULL>
+__device__ __forceinline__ void cols_gather(const float* __restrict__ g_lane, const T* __restrict__ q_lane,
+                                            float (&acc_v)[4], float (&acc_k)[4], const int* lds_row,
+                                            const float* lds_p, const float* lds_z, int first_quad, int stride, int nquads)
+{
+#pragma unroll
+    for (int i = 0; i < QUADS_MAX; ++i) {
+        const int qd = first_quad + i * stride;
+        if (FULL || qd < nquads) {
+            const int4 r4 = *reinterpret_cast<const int4*>(lds_row + 4 * qd);
+            const int r[4] = {r4.x, r4.y, r4.z, r4.w};
+            float pv[4], zv[4], bg[4][4], bq[4][4];
+            load_quad(lds_p + 4 * qd, pv);
+            load_quad(lds_z + 4 * qd, zv);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                load4(g_lane + (size_t)r[t] * D, bg[t]);
+                load4(q_lane + (size_t)r[t] * D, bq[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int x = 0; x < 4; ++x) {
+                    acc_v[x] = fmaf(pv[t], bg[t][x], acc_v[x]);
+                    acc_k[x] = fmaf(zv[t], bq[t][x], acc_k[x]);
+                }
+        }
+    }
+}
+
 } // namespace rode

@@ -1,9 +1,11 @@
 """Attention on the tiles of 16 rows (matrix cores) against fp64 on dense matrices."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
-from rode_amd import RoDeCSR, sparse_attention
+from rode_amd import RoDeCSR, _lib, sparse_attention
 from rode_amd.autograd import _attention_backward_call, _attention_call
 
 pytestmark = pytest.mark.gpu
@@ -245,3 +247,63 @@ def test_gradients_on_tiles_twice_held_column_and_inf(half):
         assert torch.equal(a.isfinite(), b.isfinite()) and b.isfinite().any() and not b.isfinite().all()
         ok = b.isfinite()
         assert (a[ok].float() - b[ok].float()).abs().max() <= (4e-3 if half else 2e-5) * b[ok].float().abs().max()
+
+
+COLS = [  # columns of the mask, window, rows that the window moves per column, other rows, width, half
+    (16, 64, 0, 0, 64, False),     # one tile, whole steps only, nothing outside the runs
+    (75, 69, 1, 5, 64, True),      # columns after the last tile, a cut-short last step
+    (320, 260, 3, 70, 64, False),  # a tile that is none, more nonzeros outside than are staged at a time, some columns with none
+    (320, 260, 3, 70, 64, True),
+    (48, 97, 2, 20, 128, True),
+    (48, 400, 2, 130, 128, False),
+    (48, 130, 1, 16, 32, True),
+    (48, 130, 1, 65, 32, False),
+]
+
+
+@pytest.mark.parametrize("m,window,shift,extra,d,half", COLS)
+def test_column_pass_on_tiles_against_fp64(m, window, shift, extra, d, half):
+    """dv = P^T g and dk = dZ^T q on a pattern whose rows are the mask's columns, with weights of its own per head; then with
+    rows of g and q that are not finite and that not all columns of a tile hold."""
+    csr, _ = _mask(m, window, shift, extra, seed=m + window, short_rows=(40,) if m == 320 else ())
+    if m == 320:  # (columns 33 and 34 lose what they hold outside their runs)
+        rp, col = csr.row_offsets.cpu().numpy(), csr.column_indices.cpu().numpy()
+        row = np.repeat(np.arange(m), np.diff(rp))
+        keep = ~np.isin(row, (33, 34)) | ((col >= shift * row) & (col < shift * row + window))
+        rp = np.concatenate([[0], np.cumsum(np.bincount(row[keep], minlength=m))]).astype(np.int32)
+        csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col[keep]), csr.values.cpu()[torch.from_numpy(keep)], "cuda", m, csr.n, 64, locality=True)
+    assert csr.plan.counts[3] == m // 16 - (1 if m == 320 else 0)
+    assert 5 * 4 * csr.plan.counts[3] >= 4 * csr.plan.counts[1]  # (with fewer in tiles other kernels take them)
+    heads, dt = _heads(csr), torch.float16 if half else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    g = torch.randn(heads, csr.n, d, device="cuda", generator=gen)
+    q = torch.randn(heads, csr.n, d, device="cuda", generator=gen).to(dt)
+    pairs = torch.randn(heads, csr.nnz, 2, device="cuda", generator=gen)
+    rows = torch.repeat_interleave(torch.arange(m, device="cuda"), (csr.row_offsets[1:] - csr.row_offsets[:-1]).long())
+    weights = torch.zeros(2, m, csr.n, device="cuda", dtype=torch.float64)
+    held = weights[0] != 0
+    held[rows, csr.column_indices.long()] = True
+
+    def run():
+        dk, dv = (torch.full((heads, m, d), float("nan"), device="cuda") for _ in range(2))
+        _lib.check(_lib.load().rode_hip_attention_backward_cols(
+            _lib.DENSE_CODE["f16" if half else "f32"], heads, csr.n, m, csr.nnz, d, csr.row_offsets.data_ptr(), csr.column_indices.data_ptr(),
+            pairs.data_ptr(), g.data_ptr(), q.data_ptr(), dk.data_ptr(), dv.data_ptr(), ctypes.byref(csr.call_plans()), None), "cols")
+        torch.cuda.synchronize()
+        return dv, dk
+
+    clean = run()
+    for h in (0, heads // 2, heads - 1):
+        for i, dense in ((0, g[h]), (1, q[h])):
+            weights[i][rows, csr.column_indices.long()] = pairs[h, :, i].double()
+            # every product and sum rounds once; a sum of n terms in trees of chains of 64 at most
+            bound = 2.0 ** -24 * (64 + 12) * (weights[i].abs() @ dense.double().abs())
+            assert ((clean[i][h].double() - weights[i] @ dense.double()).abs() <= bound + 1e-30).all()
+    first = int(csr.column_indices[0])
+    last = shift * (m - 1) + window - 1
+    g[:, first], q[:, last] = float("inf"), float("nan")
+    for i, (now, row) in enumerate(zip(run(), (first, last))):
+        touched = held[:, row]
+        assert touched.any()
+        assert not now[:, touched].isfinite().all(dim=2).any()
+        torch.testing.assert_close(now[:, ~touched], clean[i][:, ~touched], rtol=1e-4, atol=1e-4)
