@@ -5,19 +5,21 @@
 //
 // One workgroup per tile and head.  Its four waves take the columns of the run 16 or 32 at a time, in
 // turn (score products of 16 x 16, a running softmax, D / 16 weighted-sum products; layouts in
-// rode_tile.hpp), and the nonzeros outside the run of four rows each, 64 at a time, as
-// attention_rows_kernel does; every wave, and every row outside its run, has a softmax of its own,
+// rode_tile.hpp), and then the nonzeros outside the run of four rows each, side by side, 64 of every row at a time
+// (TileOutside); every wave, and every row outside its run, has a softmax of its own,
 // and the partial results meet in LDS.  Columns at the ends of the range that a row does not hold get
 // probability zero.  A non-finite row of v there would reach rows that do not reference it
 // (0 * Inf), and shows as a non-finite result: the tile's rows are then computed again, all of them
 // row by row.
 //
 // Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with
-// four rows at a time on the vector ALUs, 0.219 here; eight heads in fp32 0.693 -> 0.423.  Of the 0.219
-// about 0.06 are the columns of the run, 0.11 the nonzeros outside it (11 % of all; their dense rows
-// ask the vector memory pipe for 64 B/clk/CU half of the time, a quarter of them misses L2), 0.02 a
-// workgroup's start and end.  What was slow on the way: dense rows and values loaded straight into
-// operand layout (adjacent lanes on different rows: 64 clocks of the memory pipe per load, 0.38 ms).
+// four rows at a time on the vector ALUs, 0.209 here; eight heads in fp32 0.693 -> 0.39.  Bound by what passes the L2s: 1.2 GB
+// in the 0.209 (values 0.4, operands of eight heads in eight L2s 0.3, the rest dense rows outside the runs, a third of which
+// miss), 3.9 GB out of them.  What was slow on the way: dense rows and values loaded straight into
+// operand layout (adjacent lanes on different rows: 64 clocks of the memory pipe per load, 0.38 ms); the nonzeros outside
+// the run of one row after the other (us, fp32 / halves of width 64, one head: 75 / 36 -> 69 / 34, width 128 164 / 68 -> 131 / 58; 20 000 rows of 300 and 96
+// random columns 121 / 62 -> 97 / 55, width 128 274 / 129 -> 196 / 100; eight heads of halves 222 -> 209).  (The extent of a row outside its run waits in LDS:
+// in registers it cost halves of width 64 a wave per SIMD, 248 us.)
 //
 // 32-bit operands use the 32-bit matrix instructions (exact products, 157 TFLOP/s against 79 on the
 // vector ALUs); 16-bit operands split the probabilities into two halves each (TileWeights).  Errors against 64 bits of
@@ -89,14 +91,14 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     constexpr int NB = D / 16, PAD = D + 4, NT = tile_blocks<T>(), kStep = 16 * NT;
     using KStage = TileStage<T, D, true>;
     using VStage = TileStage<T, D, false>;
-    // Per wave: staged rows of k and v and the values of a step.  Once the columns of the run are done:
-    // the wave's partial result, in the first wave's part the rows' results outside their runs behind
-    // it, and the wave's staging for those.
+    // Per wave: staged rows of k and v and the values of a step.  Once the columns of the run are done: staging for the nonzeros
+    // outside, then the wave's partial result and behind it the results of its four rows outside their runs.
     constexpr int kPart = kTileRows * PAD, kStageFloats = 2 * KStage::kBytes / 4 + TileSquare<T>::kFloats;
-    static_assert(2 * kPart + 2 * kWave <= kStageFloats, "what comes later fits");
+    static_assert(kPart + kOutsideRows * PAD <= kStageFloats && 2 * kOutsideSteps * kWave <= kStageFloats, "what comes later fits");
     __shared__ __attribute__((aligned(16))) float shared[kWavesPerWg][kStageFloats];
     __shared__ float part_m[kWavesPerWg + 1][kTileRows], part_l[kWavesPerWg + 1][kTileRows]; // (the last: outside the runs)
     __shared__ float part_ref[kWavesPerWg][kTileRows];
+    __shared__ int4 extents[kTileRows]; // (for the nonzeros outside the runs: not in registers until then)
     const int tile = xcd_logical_block(blockIdx.x, gridDim.x);
     if (tile >= n_tiles) return;
     const RowTile rt = tiles[tile];
@@ -107,6 +109,7 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     const int n = lane % 16, gq = lane / 16;
     const TileLane me = tile_lane(tile * kTileRows + n, row_ptr, runs);
     const int base = me.base();
+    if (threadIdx.x < kTileRows) extents[threadIdx.x] = me.packed();
     const int steps = (rt.hi - rt.lo + kStep - 1) / kStep;
     u32x4* lds_k = reinterpret_cast<u32x4*>(shared[wave]);
     u32x4* lds_v = lds_k + KStage::kBytes / 16;
@@ -115,107 +118,102 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     q_row.load(q + (size_t)me.row * D, gq);
     TileSoftmax<T, D> sm;
 
-    // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 at a time:
-    // LPR lanes read a dense row, 16 bytes each, every lane group the rows of its own LPR nonzeros.
+    // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 of each row at a time: 16 lanes
+    // have a row's nonzeros, LPR lanes read a dense row, 16 bytes each, every lane group the rows of its own LPR
+    // nonzeros.  The scores of all 64 first, then their rows of v.
     auto rows_outside = [&](bool whole) __attribute__((always_inline)) {
-        using S = SddmmShape<T, D>;
-        constexpr int VEC = S::kVec, LPR = S::kLpr, R = kTileRows / kWavesPerWg;
+        using Out = TileOutside<T, D>;
+        constexpr int VEC = Out::kVec, LPR = Out::kLpr, RPG = Out::kRows, QUADS = Out::kQuads, S = kOutsideSteps;
         const int ls = lane % LPR, group = lane / LPR;
         const unsigned lane_at = ls * 16u; // (an operand of a tile is at most 4 GB: 32-bit offsets)
         const char* k_bytes = reinterpret_cast<const char*>(k);
         const char* v_bytes = reinterpret_cast<const char*>(v);
-        float* left_o = shared[0] + kPart;
-        unsigned* my_at = reinterpret_cast<unsigned*>(shared[wave] + 2 * kPart);
-        float* my_p = shared[wave] + 2 * kPart + kWave;
-        struct Row {
-            int first, cnt, split, jump, c;
-            float w;
-        };
-        // a row's extent, and the columns and values of its first step
-        auto row_of = [&](int r) __attribute__((always_inline)) {
-            Row x;
-            x.first = __builtin_amdgcn_readlane(me.s, r);
-            x.jump = whole ? 0 : __builtin_amdgcn_readlane(me.len, r);
-            x.split = __builtin_amdgcn_readlane(me.pos, r);
-            x.cnt = __builtin_amdgcn_readlane(me.e, r) - x.first - x.jump;
-            const int at = min(lane, x.cnt - 1), idx = x.first + at + (at >= x.split ? x.jump : 0);
-            x.c = x.cnt > 0 ? col[idx] : 0;
-            x.w = x.cnt > 0 ? val[idx] : 0.f;
-            return x;
-        };
-        Row next = row_of(R * wave);
-#pragma unroll 1
-        for (int r = R * wave; r < R * wave + R; ++r) {
-            const Row me_row = next;
-            if (r + 1 < R * wave + R) next = row_of(r + 1); // (asked for while this row is worked on)
-            const int cnt = me_row.cnt;
-            typename DotVec<T>::Reg a[1][DotVec<T>::kRegs];
-            load_lhs_slice<T, D, 1, false>(q, tile * kTileRows + r, D, lane, a);
-            float m_run = -INFINITY, l_lane = 0.f, acc[VEC];
+        unsigned* my_at = reinterpret_cast<unsigned*>(shared[wave]); // (the step's staging is free)
+        float* my_p = shared[wave] + S * kWave;
+        const Out of(extents, wave, lane, whole);
+        typename DotVec<T>::Reg a[RPG][1][DotVec<T>::kRegs];
 #pragma unroll
-            for (int x = 0; x < VEC; ++x) acc[x] = 0.f;
+        for (int i = 0; i < RPG; ++i) load_lhs_slice<T, D, 1, false>(q, tile * kTileRows + of.row(i), D, lane, a[i]);
+        float m_run = -INFINITY, l_lane = 0.f, acc[RPG][VEC];
+#pragma unroll
+        for (int i = 0; i < RPG; ++i)
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) acc[i][x] = 0.f;
 #pragma unroll 1
-            for (int off = 0; off < cnt; off += kWave) {
-                const bool live = off + lane < cnt;
-                const int at = min(off + lane, cnt - 1); // (lanes past the end repeat the last nonzero with probability 0)
-                const int idx = me_row.first + at + (at >= me_row.split ? me_row.jump : 0);
-                const int c = off == 0 ? me_row.c : col[idx];
-                const float w = off == 0 ? me_row.w : val[idx];
-                my_at[lane] = (unsigned)c * (unsigned)(D * sizeof(T));
-                wave_lds_sync();
+        for (int off = 0; off < of.most; off += 16 * S) {
+            float w[S], sc[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                int c = 0;
+                w[s] = 0.f;
+                if (off + 16 * s < of.cnt) { // (lanes past the end repeat the last nonzero with probability 0)
+                    const int idx = of.slot(off + 16 * s + lane % 16);
+                    c = col[idx];
+                    w[s] = val[idx];
+                }
+                my_at[s * kWave + lane] = (unsigned)c * (unsigned)(D * sizeof(T));
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
                 float d = 0.f;
-                const bool busy = off + group * LPR < cnt; // does this lane group have a nonzero?
-                // (the first rows of v are asked for together with those of k)
-                constexpr int kEarly = S::kQuads < 2 ? S::kQuads : 2;
-                u32x4 v_early[kEarly][4];
-                if (busy) {
 #pragma unroll
-                    for (int qd = 0; qd < S::kQuads; ++qd) {
-                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
-                        uint4 k_part[4];
+                for (int i = 0; i < RPG; ++i)
+                    if (off + 16 * s < of.cnt_of[i]) {
+                        uint4 k_part[QUADS][4];
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) k_part[j] = *reinterpret_cast<const uint4*>(k_bytes + (o[j] + lane_at));
-                        if (qd < kEarly) {
+                        for (int u = 0; u < QUADS; ++u) {
+                            const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + s * kWave + group * LPR + 4 * (i * QUADS + u));
 #pragma unroll
-                            for (int j = 0; j < 4; ++j) v_early[qd][j] = *reinterpret_cast<const u32x4*>(v_bytes + (o[j] + lane_at));
+                            for (int j = 0; j < 4; ++j) k_part[u][j] = *reinterpret_cast<const uint4*>(k_bytes + (o[j] + lane_at));
                         }
-                        float p[4];
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) p[j] = DotVec<T>::dot_raw(a[0], k_part[j], 0.f);
-                        const float sum = sddmm_quad_reduce<LPR>(p, ls);
-                        if ((ls >> 2) == qd) d = sum;
-                    }
-                }
-                const float sc = live ? scale * (w * d) : -INFINITY;
-                my_p[lane] = softmax_step<VEC>(sc, live, m_run, l_lane, acc);
-                if (KEEP != kKeepNothing && live) probs[idx] = sc;
-                wave_lds_sync();
-                if (busy) {
+                        for (int u = 0; u < QUADS; ++u) {
+                            float p[4];
 #pragma unroll
-                    for (int qd = 0; qd < S::kQuads; ++qd) {
-                        const f32x4 p = *reinterpret_cast<const f32x4*>(my_p + group * LPR + 4 * qd);
-                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const u32x4 raw = qd < kEarly ? v_early[qd][j] : *reinterpret_cast<const u32x4*>(v_bytes + (o[j] + lane_at));
-                            float b[VEC];
-                            DenseVec<T>::unpack(make_uint4(raw[0], raw[1], raw[2], raw[3]), b);
-#pragma unroll
-                            for (int x = 0; x < VEC; ++x) acc[x] = fmaf(p[j], b[x], acc[x]);
+                            for (int j = 0; j < 4; ++j) p[j] = DotVec<T>::dot_raw(a[i][0], k_part[u][j], 0.f);
+                            const float sum = sddmm_quad_reduce<LPR>(p, ls);
+                            if ((ls >> 2) == i * QUADS + u) d = sum;
                         }
                     }
-                }
-                wave_lds_sync();
+                const int slot = off + 16 * s + lane % 16;
+                sc[s] = slot < of.cnt ? scale * (w[s] * d) : -INFINITY;
+                if (KEEP != kKeepNothing && slot < of.cnt) probs[of.slot(slot)] = sc[s];
             }
-            const float l = butterfly_sum<1, kWave>(l_lane);
-            using Reduce = GroupReduce<LPR, VEC>;
-            Reduce::run(acc);
-            if (Reduce::writes(lane)) {
+            // the running softmax of the row (the same in its 16 lanes but for l_lane)
+            float top = sc[0];
 #pragma unroll
-                for (int x = 0; x < Reduce::kLeft; ++x) left_o[r * PAD + ls * VEC + Reduce::value(lane) + x] = acc[x];
+            for (int s = 1; s < S; ++s) top = fmaxf(top, sc[s]);
+            const float m_new = fmaxf(m_run, butterfly_max<1, 16>(top));
+            const float m_safe = m_new == -INFINITY ? 0.f : m_new;
+            const float corr = __expf(m_run - m_safe);
+            m_run = m_new;
+            float p_sum = 0.f;
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                const float p = off + 16 * s + lane % 16 < of.cnt ? __expf(sc[s] - m_safe) : 0.f;
+                p_sum += p;
+                my_p[s * kWave + lane] = p;
             }
-            if (lane == 0) part_m[kWavesPerWg][r] = m_run, part_l[kWavesPerWg][r] = l;
+            l_lane = fmaf(l_lane, corr, p_sum);
+            if (off > 0) { // (nothing to rescale before)
+                const float corr_of[2] = {RPG > 1 ? lane_pair16(corr).a : corr, RPG > 1 ? lane_pair16(corr).b : corr};
+#pragma unroll
+                for (int i = 0; i < RPG; ++i)
+#pragma unroll
+                    for (int x = 0; x < VEC; ++x) acc[i][x] *= corr_of[i];
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < RPG; ++i)
+                    if (off + 16 * s < of.cnt_of[i]) Out::add(v_bytes, lane_at, my_at + s * kWave, my_p + s * kWave, group * LPR + 4 * i * QUADS, acc[i]);
+            wave_lds_sync();
         }
+        const float l = butterfly_sum<1, 16>(l_lane);
+        of.store(acc, shared[wave] + kPart, PAD, lane);
+        if (lane % 16 == 0) part_m[kWavesPerWg][of.mine] = m_run, part_l[kWavesPerWg][of.mine] = l;
     };
 
     // a step's columns of the run, on their way
@@ -314,7 +312,7 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     float f = __builtin_amdgcn_exp2f((part_m[kWavesPerWg][r] - top_safe) * kLog2e);
     float total = part_l[kWavesPerWg][r] * f, o[NB];
 #pragma unroll
-    for (int x = 0; x < NB; ++x) o[x] = shared[0][kPart + r * PAD + e0 + x] * f;
+    for (int x = 0; x < NB; ++x) o[x] = shared[r / kOutsideRows][kPart + r % kOutsideRows * PAD + e0 + x] * f;
 #pragma unroll
     for (int w = 0; w < kWavesPerWg; ++w) {
         f = __builtin_amdgcn_exp2f(-fmaf(top_safe, kLog2e, -part_ref[w][r]));

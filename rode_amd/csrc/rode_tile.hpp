@@ -341,6 +341,7 @@ struct TileLane {
     int row, s, e;    // slots [s, e)
     int a, len, pos;  // columns [a, a + len) from slot s + pos on
     __device__ __forceinline__ int base() const { return s + pos - a; } // slot of column c of the run: base() + c
+    __device__ __forceinline__ int4 packed() const { return make_int4(s, e - s, pos, len); }
 };
 __device__ __forceinline__ TileLane tile_lane(int row, const int* __restrict__ row_ptr, const int* __restrict__ runs)
 {
@@ -350,5 +351,82 @@ __device__ __forceinline__ TileLane tile_lane(int row, const int* __restrict__ r
     t.a = runs[3 * row], t.len = runs[3 * row + 1], t.pos = runs[3 * row + 2];
     return t;
 }
+
+// ---- the nonzeros outside the runs -------------------------------------------------------------
+// A wave has four rows of the tile and 16 lanes for the nonzeros of each (kOutsideSteps of them per lane at a time): the rows'
+// dependent steps - columns, dense rows, reductions, the softmax - then go on side by side instead of one row after
+// the other, and each lane group's sums belong to one row (width 128 in fp32: to two, kRows).
+constexpr int kOutsideRows = kTileRows / kWavesPerWg, kOutsideSteps = 4;
+static_assert(kOutsideRows * 16 == kWave, "16 lanes per row");
+template <typename T, int D>
+struct TileOutside {
+    static constexpr int kVec = 16 / (int)sizeof(T), kLpr = D / kVec, kRows = kLpr > 16 ? kLpr / 16 : 1; // (rows of a lane group)
+    static constexpr int kQuads = kLpr / 4 / kRows;                                                       // quads of a row per lane group and step
+    int mine, first, split, jump, cnt, most; // this lane's row (of the tile) and its nonzeros; the most that one of the four rows has
+    int cnt_of[kRows];                       // a row of this lane group has work in the step from nonzero n on while n < cnt_of
+    int group;
+    // (rows: what tile_lane says of every row of the tile, TileLane::packed)
+    __device__ __forceinline__ TileOutside(const int4* rows, int wave, int lane, bool whole) : group(lane / kLpr)
+    {
+        mine = kOutsideRows * wave + lane / 16;
+        const int4 r = rows[mine];
+        first = r.x, split = r.z, jump = whole ? 0 : r.w;
+        cnt = r.y - jump;
+        most = 0;
+#pragma unroll
+        for (int i = 0; i < kOutsideRows; ++i) most = max(most, __builtin_amdgcn_readlane(cnt, 16 * i));
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) cnt_of[i] = kRows == 1 ? cnt - group * kLpr % 16 : __shfl(cnt, group * kLpr + 16 * i, kWave);
+    }
+    // row i of this lane group (of the tile)
+    __device__ __forceinline__ int row(int i) const { return kRows == 1 ? mine : (mine & ~(kRows - 1)) + i; }
+    // where nonzero `at` of this lane's row is (past the end: its last one)
+    __device__ __forceinline__ int slot(int at) const
+    {
+        at = min(at, cnt - 1);
+        return first + at + (at >= split ? jump : 0);
+    }
+    // acc += the kQuads quads of weights from `from` on times their dense rows (a sum of their own first)
+    static __device__ __forceinline__ void add(const char* dense, unsigned lane_at, const unsigned* row_at, const float* weight, int from, float (&acc)[kVec])
+    {
+        u32x4 raw[kQuads][4];
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const u32x4 o = *reinterpret_cast<const u32x4*>(row_at + from + 4 * u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) raw[u][j] = *reinterpret_cast<const u32x4*>(dense + (o[j] + lane_at));
+        }
+        float sum[kVec];
+#pragma unroll
+        for (int u = 0; u < kQuads; ++u) {
+            const f32x4 w = *reinterpret_cast<const f32x4*>(weight + from + 4 * u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                float b[kVec];
+                DenseVec<T>::unpack(make_uint4(raw[u][j][0], raw[u][j][1], raw[u][j][2], raw[u][j][3]), b);
+#pragma unroll
+                for (int x = 0; x < kVec; ++x) sum[x] = u == 0 && j == 0 ? w[j] * b[x] : fmaf(w[j], b[x], sum[x]);
+            }
+        }
+#pragma unroll
+        for (int x = 0; x < kVec; ++x) acc[x] += sum[x];
+    }
+    // the four rows' sums to LDS, `stride` floats apart
+    __device__ __forceinline__ void store(float (&acc)[kRows][kVec], float* to, int stride, int lane) const
+    {
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            if constexpr (kLpr < 16) { // (several lane groups have a row)
+#pragma unroll
+                for (int x = 0; x < kVec; ++x) acc[i][x] = butterfly_sum<kLpr, 16>(acc[i][x]);
+            }
+            if (kLpr >= 16 || group % (16 / (kLpr < 16 ? kLpr : 16)) == 0) {
+#pragma unroll
+                for (int x = 0; x < kVec; x += 4)
+                    *reinterpret_cast<f32x4*>(to + row(i) % kOutsideRows * stride + lane % kLpr * kVec + x) = f32x4{acc[i][x], acc[i][x + 1], acc[i][x + 2], acc[i][x + 3]};
+            }
+        }
+    }
+};
 
 } // namespace rode

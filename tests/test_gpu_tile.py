@@ -47,6 +47,8 @@ CASES = [  # m, window, columns the window moves per row, random columns, width,
     (48, 97, 2, 20, 128, False, 0.2),
     (48, 130, 1, 16, 32, True, 0.4),
     (48, 130, 1, 16, 32, False, 0.4),
+    (48, 400, 2, 130, 128, False, 0.1),  # three times 64 outside a run
+    (48, 400, 2, 130, 32, True, 0.2),
 ]
 
 
@@ -307,3 +309,43 @@ def test_column_pass_on_tiles_against_fp64(m, window, shift, extra, d, half):
         assert touched.any()
         assert not now[:, touched].isfinite().all(dim=2).any()
         torch.testing.assert_close(now[:, ~touched], clean[i][:, ~touched], rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_rows_with_very_different_numbers_outside_their_runs(d, half):
+    """Four rows share a wave outside their runs, 16 lanes each, 64 nonzeros at a time: none beside many, and either side of
+    16, 64 and 128.  Column 0, which only some rows hold, is not finite: a row that holds nothing there must not meet it."""
+    m, window, dt = 64, 900, torch.float16 if half else torch.float32
+    counts = [0, 130, 1, 16, 0, 0, 0, 0, 17, 15, 64, 65, 128, 129, 63, 3] + [0, 200, 0, 70, 2, 0, 0, 0, 0, 0, 0, 33, 80, 0, 31, 32] + list(range(50, 82))
+    rng = np.random.default_rng(d)
+    n = 1300
+    cols = [np.sort(np.concatenate([np.arange(300 + r, 300 + r + window), rng.choice(298, k, replace=False)])) for r, k in enumerate(counts)]
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32)
+    col = np.concatenate(cols).astype(np.int32)
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.ones(len(col)), "cuda", m, n, 64, locality=True)
+    assert csr.plan.counts[3] == m // 16
+    held = torch.zeros(m, n, dtype=torch.bool, device="cuda")
+    held[torch.from_numpy(np.repeat(np.arange(m), np.diff(rp))).cuda(), csr.column_indices.long()] = True
+    heads, scale = _heads(csr), d ** -0.5
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, n, n, m))
+    q, k, v = (t.to(dt) for t in (q, k, v))
+    ins = [t.double().requires_grad_() for t in (q, k, v)]
+    want = _reference(held.double(), *ins, scale)
+    want = (want,) + torch.autograd.grad(want, ins, g.double())
+    ins = [t.expand(heads, *t.shape).contiguous().requires_grad_() for t in (q, k, v)]
+    out = sparse_attention(csr, *ins, scale=scale)
+    got = (out,) + torch.autograd.grad(out, ins, g.expand(heads, m, d).contiguous())
+    for a, b in zip(got, want):
+        assert (a[heads - 1].double() - b).norm() <= (2e-3 if half and b is not want[0] else 2e-6) * b.norm()
+    k[0], v[0] = float("nan"), float("inf")
+    ins = [t.expand(heads, *t.shape).contiguous().requires_grad_() for t in (q, k, v)]
+    bad = sparse_attention(csr, *ins, scale=scale)
+    dq, = torch.autograd.grad(bad, ins[:1], g.expand(heads, m, d).contiguous())
+    touched = held[:, 0]
+    assert touched.any() and not touched.all()
+    for now, was in ((bad, out), (dq, got[1])):
+        assert not now[:, touched].isfinite().all(dim=2).any()
+        # (their tiles may be computed row by row now: either is within the bound above)
+        assert (now[:, ~touched] - was[:, ~touched]).norm() <= (4e-3 if half and was is not out else 4e-6) * was[:, ~touched].norm()
