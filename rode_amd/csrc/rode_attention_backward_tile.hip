@@ -17,10 +17,12 @@
 // follows the largest |dz| so far (the sums are rescaled when it moves, exactly).  The rounding of g is what decides
 // there: dq is 2e-4 to 7e-4 off with and without tiles.
 //
-// Measured (16 384 rows, window 512 and 64 random columns, width 64, one head; forward and both gradient kernels), against
-// four rows at a time on the vector ALUs: 0.330 -> 0.279 ms, halves 0.259 -> 0.21; the row pass itself 0.130 -> 0.088.  It is now bound by the
-// staging of v and k, by the waves in flight (184 registers: two per SIMD) and by 190 MB of
-// values, scores, slots and pairs.  Tried: three waves per SIMD (fp16 spills, 0.250; fp32 0.282).
+// Measured (16 384 rows, window 512 and 64 random columns, width 64, one head in fp32; the kernel's own time): 107 us with the
+// nonzeros outside the run of one row after the other, 95 with those of four rows side by side (TileOutside); training step, us, the other two
+// passes unchanged: fp32 250 -> 244, halves 172 -> 167, width 128 457 -> 422 and 316 -> 302; 20 000 rows of 300 + 96, width 64 430 -> 410.
+// Bound by what passes the L2s (600 MB: 190 MB of values, scores, slots and pairs, the dense rows of eight L2s, a third of those outside the
+// runs) with two waves per SIMD in flight.  Tried: three waves per SIMD (halves spill, step 0.250 ms instead of 0.21; fp32 0.282
+// instead of 0.279).
 #include "rode_tile.hpp"
 #include "rode_units.hpp"
 #include "rode_internal.hpp"
@@ -78,11 +80,12 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
     constexpr bool kHalf = std::is_same<T, __half>::value;
     using VStage = TileStage<T, D, true>;  // (v meets g along its elements, k is summed across)
     using KStage = TileStage<T, D, false>;
-    // Per wave: staged rows of v and k, the values and what the forward pass kept of a step.  Then the wave's
-    // partial sums, in the first wave's part the rows' sums outside their runs behind them, and the wave's staging for those.
+    // Per wave: staged rows of v and k, the values and what the forward pass kept of a step.  Then staging for the nonzeros outside
+    // the runs, then the wave's partial sums and behind them the sums of its four rows outside their runs.
     constexpr int kPart = kTileRows * PAD, kStageFloats = 2 * VStage::kBytes / 4 + 2 * TileSquare<T>::kFloats;
-    static_assert(2 * kPart + 2 * kWave <= kStageFloats, "what comes later fits");
+    static_assert(kPart + kOutsideRows * PAD <= kStageFloats && 2 * kOutsideSteps * kWave <= kStageFloats, "what comes later fits");
     __shared__ __attribute__((aligned(16))) float shared[kWavesPerWg][kStageFloats];
+    __shared__ int4 extents[kTileRows]; // (for the nonzeros outside the runs: not in registers until then)
     const int tile = xcd_logical_block(blockIdx.x, gridDim.x);
     if (tile >= n_tiles) return;
     const RowTile rt = tiles[tile];
@@ -94,6 +97,7 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
     const int n = lane % 16, gq = lane / 16;
     const TileLane me = tile_lane(tile * kTileRows + n, row_ptr, runs);
     const int base = me.base();
+    if (threadIdx.x < kTileRows) extents[threadIdx.x] = me.packed();
     const int steps = (rt.hi - rt.lo + kStep - 1) / kStep;
     u32x4* lds_v = reinterpret_cast<u32x4*>(shared[wave]);
     u32x4* lds_k = lds_v + VStage::kBytes / 16;
@@ -154,126 +158,97 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
     clear();
     TileRange<T> range;
 
-    // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 at a time:
-    // LPR lanes read a dense row, 16 bytes each, every lane group the rows of its own LPR nonzeros.
+    // This wave's four rows without the nonzeros of their runs (or, `whole`, with them), 64 of each row at a time: 16 lanes
+    // have a row's nonzeros, LPR lanes read a dense row, 16 bytes each, every lane group the rows of its own LPR
+    // nonzeros.  The rows of v of all 64 first, then those of k.
     auto rows_outside = [&](bool whole) __attribute__((always_inline)) {
-        using S = SddmmShape<T, D>;
-        constexpr int VEC = S::kVec, LPR = S::kLpr, R = kTileRows / kWavesPerWg;
+        using Out = TileOutside<T, D>;
+        constexpr int VEC = Out::kVec, LPR = Out::kLpr, RPG = Out::kRows, QUADS = Out::kQuads, S = kOutsideSteps;
         const int ls = lane % LPR, group = lane / LPR;
         const unsigned lane_at = ls * 16u; // (an operand of a tile is at most 4 GB: 32-bit offsets)
         const char* k_bytes = reinterpret_cast<const char*>(k);
         const char* v_bytes = reinterpret_cast<const char*>(v);
-        float* left = shared[0] + kPart;
-        unsigned* my_at = reinterpret_cast<unsigned*>(shared[wave] + 2 * kPart);
-        float* my_z = shared[wave] + 2 * kPart + kWave;
-        struct Row {
-            int first, cnt, split, jump, c, to;
-            float w, kept;
-        };
-        auto slot_of = [](const Row& x, int at) __attribute__((always_inline)) { return x.first + at + (at >= x.split ? x.jump : 0); };
-        // a row's extent, and what its first step needs
-        auto row_of = [&](int r) __attribute__((always_inline)) {
-            Row x;
-            x.first = __builtin_amdgcn_readlane(me.s, r);
-            x.jump = whole ? 0 : __builtin_amdgcn_readlane(me.len, r);
-            x.split = __builtin_amdgcn_readlane(me.pos, r);
-            x.cnt = __builtin_amdgcn_readlane(me.e, r) - x.first - x.jump;
-            x.c = x.to = 0;
-            x.w = x.kept = 0.f;
-            if (x.cnt > 0) {
-                const int idx = slot_of(x, min(lane, x.cnt - 1));
-                x.c = col[idx], x.to = t_slot[idx], x.w = val[idx], x.kept = probs[idx];
-            }
-            return x;
-        };
-        auto of_row = [&](float x, int r) __attribute__((always_inline)) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), r)); };
-        Row next = row_of(R * wave);
-#pragma unroll 1
-        for (int r = R * wave; r < R * wave + R; ++r) {
-            const Row now = next;
-            if (r + 1 < R * wave + R) next = row_of(r + 1); // (asked for while this row is worked on)
-            const int cnt = now.cnt;
-            const float row_max = of_row(stat_max, r), row_inv = of_row(stat_inv, r), row_delta = of_row(delta, r);
-            const float row_scale = of_row(g_scale, r), row_back = of_row(g_inv, r);
-            typename DotVec<T>::Reg a[DotVec<T>::kRegs];
-            {
-                const float* g_at = g + (size_t)(tile * kTileRows + r) * D + ls * VEC;
-                f32x4 x[VEC / 4];
+        unsigned* my_at = reinterpret_cast<unsigned*>(shared[wave]); // (the step's staging is free)
+        float* my_z = shared[wave] + S * kWave;
+        const Out of(extents, wave, lane, whole);
+        const float row_max = __shfl(stat_max, of.mine, kWave), row_inv = __shfl(stat_inv, of.mine, kWave);
+        const float row_delta = __shfl(delta, of.mine, kWave), row_scale = __shfl(g_scale, of.mine, kWave);
+        typename DotVec<T>::Reg a[RPG][DotVec<T>::kRegs];
 #pragma unroll
-                for (int h = 0; h < VEC / 4; ++h) x[h] = *reinterpret_cast<const f32x4*>(g_at + 4 * h);
-                if constexpr (kHalf) {
+        for (int i = 0; i < RPG; ++i) {
+            const float* g_at = g + (size_t)(tile * kTileRows + of.row(i)) * D + ls * VEC;
+            f32x4 x[VEC / 4];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const __half2 h2 = __floats2half2_rn(x[i / 2][2 * (i % 2)] * row_back, x[i / 2][2 * (i % 2) + 1] * row_back);
-                        a[i] = *reinterpret_cast<const uint32_t*>(&h2);
-                    }
-                } else {
+            for (int h = 0; h < VEC / 4; ++h) x[h] = *reinterpret_cast<const f32x4*>(g_at + 4 * h);
+            if constexpr (kHalf) {
+                const float row_back = __shfl(g_inv, of.row(i), kWave);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) a[i] = x[0][i];
+                for (int y = 0; y < 4; ++y) {
+                    const __half2 h2 = __floats2half2_rn(x[y / 2][2 * (y % 2)] * row_back, x[y / 2][2 * (y % 2) + 1] * row_back);
+                    a[i][y] = *reinterpret_cast<const uint32_t*>(&h2);
                 }
-            }
-            float sum[VEC];
+            } else {
 #pragma unroll
-            for (int x = 0; x < VEC; ++x) sum[x] = 0.f;
-#pragma unroll 1
-            for (int off = 0; off < cnt; off += kWave) {
-                const bool live = off + lane < cnt; // (lanes past the end repeat the last nonzero with weight 0)
-                const int idx = slot_of(now, min(off + lane, cnt - 1));
-                const int c = off == 0 ? now.c : col[idx], to = off == 0 ? now.to : t_slot[idx];
-                const float w = off == 0 ? now.w : val[idx], p = prob_of(off == 0 ? now.kept : probs[idx], row_max, row_inv);
-                my_at[lane] = (unsigned)c * (unsigned)(D * sizeof(T));
-                wave_lds_sync();
-                float d = 0.f;
-                const bool busy = off + group * LPR < cnt; // does this lane group have a nonzero?
-                // (the first rows of k are asked for together with those of v)
-                constexpr int kEarly = S::kQuads < 2 ? S::kQuads : 2;
-                u32x4 k_early[kEarly][4];
-                if (busy) {
-#pragma unroll
-                    for (int qd = 0; qd < S::kQuads; ++qd) {
-                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
-                        uint4 v_part[4];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) v_part[j] = *reinterpret_cast<const uint4*>(v_bytes + (o[j] + lane_at));
-                        if (qd < kEarly) {
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) k_early[qd][j] = *reinterpret_cast<const u32x4*>(k_bytes + (o[j] + lane_at));
-                        }
-                        float part[4];
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) part[j] = DotVec<T>::dot_raw(a, v_part[j], 0.f);
-                        const float dot = sddmm_quad_reduce<LPR>(part, ls);
-                        if ((ls >> 2) == qd) d = dot;
-                    }
-                }
-                const float dz = live ? scale * w * p * (d * row_scale - row_delta) : 0.f;
-                if (live) pz[to] = make_float2(p, dz);
-                my_z[lane] = dz;
-                wave_lds_sync();
-                if (busy) {
-#pragma unroll
-                    for (int qd = 0; qd < S::kQuads; ++qd) {
-                        const f32x4 z = *reinterpret_cast<const f32x4*>(my_z + group * LPR + 4 * qd);
-                        const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + group * LPR + 4 * qd);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const u32x4 raw = qd < kEarly ? k_early[qd][j] : *reinterpret_cast<const u32x4*>(k_bytes + (o[j] + lane_at));
-                            float b[VEC];
-                            DenseVec<T>::unpack(make_uint4(raw[0], raw[1], raw[2], raw[3]), b);
-#pragma unroll
-                            for (int x = 0; x < VEC; ++x) sum[x] = fmaf(z[j], b[x], sum[x]);
-                        }
-                    }
-                }
-                wave_lds_sync();
-            }
-            using Reduce = GroupReduce<LPR, VEC>;
-            Reduce::run(sum);
-            if (Reduce::writes(lane)) {
-#pragma unroll
-                for (int x = 0; x < Reduce::kLeft; ++x) left[r * PAD + ls * VEC + Reduce::value(lane) + x] = sum[x];
+                for (int y = 0; y < 4; ++y) a[i][y] = x[0][y];
             }
         }
+        float sum[RPG][VEC];
+#pragma unroll
+        for (int i = 0; i < RPG; ++i)
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) sum[i][x] = 0.f;
+#pragma unroll 1
+        for (int off = 0; off < of.most; off += 16 * S) {
+            float w[S], kept[S];
+            int to[S];
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                int c = 0;
+                w[s] = kept[s] = 0.f;
+                to[s] = 0;
+                if (off + 16 * s < of.cnt) { // (lanes past the end repeat the last nonzero with weight 0)
+                    const int idx = of.slot(off + 16 * s + lane % 16);
+                    c = col[idx], to[s] = t_slot[idx], w[s] = val[idx], kept[s] = probs[idx];
+                }
+                my_at[s * kWave + lane] = (unsigned)c * (unsigned)(D * sizeof(T));
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int s = 0; s < S; ++s) {
+                float d = 0.f;
+#pragma unroll
+                for (int i = 0; i < RPG; ++i)
+                    if (off + 16 * s < of.cnt_of[i]) {
+                        uint4 v_part[QUADS][4];
+#pragma unroll
+                        for (int u = 0; u < QUADS; ++u) {
+                            const u32x4 o = *reinterpret_cast<const u32x4*>(my_at + s * kWave + group * LPR + 4 * (i * QUADS + u));
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) v_part[u][j] = *reinterpret_cast<const uint4*>(v_bytes + (o[j] + lane_at));
+                        }
+#pragma unroll
+                        for (int u = 0; u < QUADS; ++u) {
+                            float part[4];
+#pragma unroll
+                            for (int j = 0; j < 4; ++j) part[j] = DotVec<T>::dot_raw(a[i], v_part[u][j], 0.f);
+                            const float dot = sddmm_quad_reduce<LPR>(part, ls);
+                            if ((ls >> 2) == i * QUADS + u) d = dot;
+                        }
+                    }
+                const bool live = off + 16 * s + lane % 16 < of.cnt;
+                const float p = prob_of(kept[s], row_max, row_inv), dz = live ? scale * w[s] * p * (d * row_scale - row_delta) : 0.f;
+                if (live) pz[to[s]] = make_float2(p, dz);
+                my_z[s * kWave + lane] = dz;
+            }
+            wave_lds_sync();
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int i = 0; i < RPG; ++i)
+                    if (off + 16 * s < of.cnt_of[i]) Out::add(k_bytes, lane_at, my_at + s * kWave, my_z + s * kWave, group * LPR + 4 * i * QUADS, sum[i]);
+            wave_lds_sync();
+        }
+        of.store(sum, shared[wave] + kPart, PAD, lane);
     };
 
     // a step's columns of the run, on their way
@@ -376,7 +351,7 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
     float o[NB];
 #pragma unroll
     for (int x = 0; x < NB; ++x) {
-        o[x] = shared[0][kPart + r * PAD + e0 + x];
+        o[x] = shared[r / kOutsideRows][kPart + r % kOutsideRows * PAD + e0 + x];
 #pragma unroll
         for (int w = 0; w < kWavesPerWg; ++w) o[x] += shared[w][r * PAD + e0 + x];
     }
