@@ -202,7 +202,7 @@ int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_
  * rows (hubs of a power-law graph) whose dense operand is far larger than the caches: the
  * rows of at least min_len aligned nonzero slots are cut into pieces by column slab
  * (RODE_HIP_HUB_SLAB_ROWS dense rows) and worked on slab after slab - a few neighbouring
- * slabs, about 4 MB of the dense operand, at a time - by kernels of their own, so that the
+ * slabs, 2 to 4 MB of the dense operand, at a time - by kernels of their own, so that the
  * hub rows' nonzeros of those slabs meet in one L2 and a dense row is fetched from memory
  * once for all of them.  The other kernels leave those rows out.  Results are
  * the same up to the order of the fp32 additions inside a hub row.

@@ -166,7 +166,8 @@ size_t rode_hip_hub_workspace_bytes(const int* h_hub_counts, int n, int elem_byt
 {
     if (!h_hub_counts || n <= 0 || (elem_bytes != 4 && elem_bytes != 8) || h_hub_counts[0] <= 0 || h_hub_counts[1] <= 0)
         return 0;
-    const int merge = rode::hub_merge(n * elem_bytes / 4);
+    // (an operand of halves has pieces twice as long)
+    const int merge = rode::hub_merge((size_t)n * elem_bytes, h_hub_counts[1]);
     return (size_t)h_hub_counts[0] * rode::hub_groups(h_hub_counts[1], merge) * n * elem_bytes;
 }
 

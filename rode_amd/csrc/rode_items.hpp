@@ -459,9 +459,7 @@ inline const RowTile* group_plan_tiles(const int* plan, int M) { return reinterp
 // the operand, and so does every other hub: the same dense rows, at other times, long
 // evicted from L2.  A hub plan cuts every hub row into pieces by column slab (a slab is
 // kHubSlabRows consecutive dense rows) and the hub kernels take the pieces slab by slab,
-// a few neighbouring slabs at a time (hub_merge: about 4 MB of the dense operand, the size
-// of an XCD's L2 - measured best on the power-law benchmark against half, twice and four
-// times that; smaller pieces cost more than they save): all hub rows' nonzeros of those
+// a few neighbouring slabs at a time (hub_merge: 2 or 4 MB of the dense operand): all hub rows' nonzeros of those
 // slabs at the same time on one XCD, so that a dense row is fetched from memory once and
 // then found in L2 by the other hubs.
 // Needs rows whose column indices ascend (the plan checks).  The standard kernels skip
@@ -488,12 +486,15 @@ __host__ __device__ inline size_t hub_plan_ints(int M, int dense_rows, int nnz, 
     return hub_table_ints(dense_rows, nnz, min_len) + (M + kHubSelectBlockRows - 1) / kHubSelectBlockRows + 1;
 }
 
-// Slabs taken together by one work item of the hub kernels, for dense rows of `width`
-// 4-byte elements (16-bit operands count as 4 bytes too: the pieces matter more than the bytes).
-__host__ __device__ inline int hub_merge(int width)
+// Slabs taken together by the work items of the hub kernels, for dense rows of so many bytes: 4 MB of the operand, the size of an XCD's L2;
+// 2 MB of one of up to 320 MB, whose pieces are long enough (us, SDDMM / SpMM with its reduction at 2 -> 4 MB: 2 M x 128 727 / 653 -> 551 / 551,
+// halves 296 / 388 -> 300 / 317; 2 M x 32 162 / 155 -> 174 / 159, 2 M x 64 halves 164 / 169 -> 174 / 165, 1 M x 64 136 / 153 -> 152 / 156,
+// 500 K x 64 114 / 122 -> 129 / 132, 200 K x 32 38 / 41 -> 52 / 61).
+__host__ __device__ inline int hub_merge(size_t row_bytes, int slabs)
 {
-    const int g = (4 << 20) / kHubSlabRows / (width > 0 ? width * 4 : 4);
-    return g < 1 ? 1 : (g > 64 ? 64 : g);
+    const size_t whole = row_bytes * slabs * kHubSlabRows, at_once = (size_t)(whole <= ((size_t)320 << 20) ? 2 : 4) << 20;
+    const size_t g = at_once / kHubSlabRows / (row_bytes > 0 ? row_bytes : 4);
+    return g < 1 ? 1 : (g > 64 ? 64 : (int)g);
 }
 __host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs + merge - 1) / merge; }
 
@@ -517,6 +518,80 @@ __device__ __forceinline__ HubPlan hub_plan_view(const int* __restrict__ plan)
     v.rows = plan + kHubHeaderInts;
     v.pieces = plan + kHubHeaderInts + plan[4];
     return v;
+}
+
+// What a workgroup of the hub kernels works on: `pieces` pieces next to each other in the order slab group by slab group,
+// in steps of 64 nonzeros that its waves share evenly, each a stretch of the steps.  (A wave per piece left the longest pieces to the end:
+// a row of 200 000 nonzeros has pieces of 800 in a matrix of 2 M columns and width 128, of 28 000 in one of 200 K and width 32.)
+// As many pieces as leave enough workgroups, eight waves instead of four where there are few.  us, SDDMM / SpMM hub kernel, a wave per piece ->
+// now, and what half and twice the pieces give (rows of 4096 nonzeros and more of power-law matrices; dense rows x width, pieces):
+//   2 M x 128, 213 K     567 / 517 -> 547 / 515 (8 pieces; 4: 536 / 569, 16: 678 / 603)    2 M x 64 halves, 107 K  169 / 151 -> 165 / 157 (8; 4: 161 / 170, 16: 189 / 163)
+//   2 M x 32, 54 K       203 / 170 -> 173 / 150 (4; 2: 168 / 158, 8: 203 / 169)            1 M x 64, 27 K          198 / 162 -> 153 / 144 (2; 1: 151 / 163, 4: 170 / 144)
+//   500 K x 128, 12.6 K  234 / 208 -> 152 / 157 (2; 1: 166 / 194, 4: 177 / 162)            500 K x 64, 6.3 K       171 / 143 -> 93 / 87 (2; 1: 94 / 102, 4: 105 / 96)
+//   500 K x 32, 3.2 K    147 / 112 -> 57 / 57 (1; 2: 64 / 53)                              200 K x 32, 567         204 / 141 -> 39 / 35 (1; 2: 64 / 49)
+// (four waves: 500 K x 64 102 / 89, 200 K x 32 55 / 43; eight: 2 M x 128 548 / 535 and halves of 64 166 / 168 with 16 pieces)
+constexpr int kHubWavesMax = 8, kHubPiecesMax = 8;
+struct HubGrid {
+    int wgs;           // workgroups, a multiple of kXcds for xcd_logical_block; -1: more than a launch holds
+    int waves, pieces; // of a workgroup
+};
+inline HubGrid hub_grid(const int* counts, int merge)
+{
+    const long long items = (long long)counts[0] * hub_groups(counts[1], merge);
+    HubGrid g;
+    g.waves = items >= 20000 ? 4 : kHubWavesMax;
+    g.pieces = items >= 80000 ? kHubPiecesMax : items >= 40000 ? 4 : items >= 5000 ? 2 : 1;
+    const long long wgs = (items + g.pieces * kXcds - 1) / (g.pieces * kXcds) * kXcds;
+    g.wgs = wgs * g.waves * kWave < (1ll << 32) ? (int)wgs : -1;
+    return g;
+}
+struct HubShare {
+    int row, base, cnt, steps, before; // lane i: piece i, its steps and those before it
+    int first, last;                   // this wave's steps [first, last)
+    unsigned long long pieces;         // bit i: some of them are piece i's
+};
+__device__ __forceinline__ int hub_first_step(const HubGrid& grid, int total, int wave) { return (int)((long long)total * wave / grid.waves); }
+__device__ __forceinline__ HubShare hub_share(const HubPlan& hp, int merge, const HubGrid& grid, int wg, int wave, int lane, int& total)
+{
+    HubShare s;
+    const long long items = (long long)hp.n_hub * hub_groups(hp.slabs, merge), item = (long long)wg * grid.pieces + lane;
+    s.row = s.base = s.cnt = 0;
+    if (lane < grid.pieces && item < items) {
+        const int h = items <= INT32_MAX ? (int)item % hp.n_hub : (int)(item % hp.n_hub);
+        const int slab = (items <= INT32_MAX ? (int)item / hp.n_hub : (int)(item / hp.n_hub)) * merge;
+        const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
+        s.row = hp.rows[h];
+        s.base = piece[slab];
+        s.cnt = piece[min(slab + merge, hp.slabs)] - s.base;
+    }
+    s.steps = (s.cnt + kWave - 1) / kWave;
+    int through = s.steps;
+#pragma unroll
+    for (int d = 1; d < kHubPiecesMax; d <<= 1) {
+        const int up = __shfl_up(through, d, kWave);
+        if (lane >= d) through += up;
+    }
+    s.before = through - s.steps;
+    total = __builtin_amdgcn_readlane(through, kHubPiecesMax - 1);
+    s.first = hub_first_step(grid, total, wave), s.last = hub_first_step(grid, total, wave + 1);
+    s.pieces = __ballot(s.steps > 0 && through > s.first && s.before < s.last);
+    return s;
+}
+// This wave's part of piece i (the same i in all lanes): slots [base, base + cnt), starting with the piece's or later, ending with it or before.
+struct HubPart {
+    int row, base, cnt;
+    bool starts, ends;
+};
+__device__ __forceinline__ HubPart hub_part(const HubShare& s, int i)
+{
+    const int before = __builtin_amdgcn_readlane(s.before, i), steps = __builtin_amdgcn_readlane(s.steps, i);
+    const int from = max(0, s.first - before), to = min(steps, s.last - before);
+    HubPart p;
+    p.row = __builtin_amdgcn_readlane(s.row, i);
+    p.base = __builtin_amdgcn_readlane(s.base, i) + from * kWave;
+    p.cnt = min(__builtin_amdgcn_readlane(s.cnt, i), to * kWave) - from * kWave;
+    p.starts = from == 0, p.ends = to == steps;
+    return p;
 }
 
 } // namespace rode

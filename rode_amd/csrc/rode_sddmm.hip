@@ -422,24 +422,21 @@ sddmm_group_kernel(int k, int n_groups, const RowGroup* __restrict__ groups, con
     }
 }
 
-// The rows of a hub plan, cut into pieces by column slab (rode_items.hpp): one wave per
-// piece, slab after slab, so that the hub rows' nonzeros of one slab of rhs are worked on
-// at the same time on one XCD and find its rows in that XCD's L2.
+// The rows of a hub plan, cut into pieces by column slab (rode_items.hpp), slab after slab, so that the hub rows' nonzeros of
+// one slab of rhs are worked on at the same time on one XCD and find rhs's rows in its L2.
 template <typename T, int KT, int NS, bool EDGE>
-__global__ void __launch_bounds__(kWgThreads)
-sddmm_hub_kernel(int k, int merge, const int* __restrict__ hub, const int* __restrict__ col, const float* __restrict__ val,
+__global__ void __launch_bounds__(kHubWavesMax * kWave)
+sddmm_hub_kernel(int k, int merge, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col, const float* __restrict__ val,
                  const T* __restrict__ lhs, const T* __restrict__ rhs, float* __restrict__ out)
 {
-    __shared__ __attribute__((aligned(16))) int lds[kWavesPerWg * kWave];
+    __shared__ __attribute__((aligned(16))) int lds[kHubWavesMax * kWave];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
-    const HubPlan hp = hub_plan_view(hub);
-    const long long item = (long long)xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
-    if (item >= (long long)hp.n_hub * hub_groups(hp.slabs, merge)) return;
-    const int slab = (int)(item / hp.n_hub) * merge, h = (int)(item % hp.n_hub);
-    const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
-    const int base = piece[slab], cnt = piece[min(slab + merge, hp.slabs)] - base;
-    if (cnt <= 0) return;
-    sddmm_row_slots<T, KT, NS, EDGE, true>(hp.rows[h], base, 0, cnt, cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
+    int total;
+    const HubShare share = hub_share(hub_plan_view(hub), merge, grid, xcd_logical_block(blockIdx.x, gridDim.x), wave, lane, total);
+    for (unsigned long long todo = share.pieces; todo; todo &= todo - 1ull) {
+        const HubPart p = hub_part(share, __builtin_ctzll(todo));
+        sddmm_row_slots<T, KT, NS, EDGE, true>(p.row, p.base, 0, p.cnt, p.cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
+    }
 }
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
@@ -506,10 +503,10 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && hubs) {
-        const int merge = hub_merge(k);
-        const int gh = grid_for_waves((long long)plan.hub_counts[0] * hub_groups(plan.hub_counts[1], merge));
-        if (gh < 0) return hipErrorInvalidConfiguration;
-        sddmm_hub_kernel<T, KT, NS, EDGE><<<gh, kWgThreads, 0, s1>>>(k, merge, plan.hub, col, val, lhs, rhs, out);
+        const int merge = hub_merge((size_t)k * sizeof(T), plan.hub_counts[1]);
+        const HubGrid hub_wgs = hub_grid(plan.hub_counts, merge);
+        if (hub_wgs.wgs < 0) return hipErrorInvalidConfiguration;
+        sddmm_hub_kernel<T, KT, NS, EDGE><<<hub_wgs.wgs, hub_wgs.waves * kWave, 0, s1>>>(k, merge, hub_wgs, plan.hub, col, val, lhs, rhs, out);
         e = hipGetLastError();
     }
     if constexpr (NS == 1) {

@@ -614,47 +614,67 @@ spmm_group_kernel(int n, int n_groups, const RowGroup* __restrict__ groups, cons
     }
 }
 
-// The rows of a hub plan, cut into pieces by column slab (rode_items.hpp): one wave per
-// piece, slab after slab, so that the hub rows' nonzeros of one slab of B are worked on at
-// the same time on one XCD and find B's rows in its L2.  A piece's sum goes to its own row
+// The rows of a hub plan, cut into pieces by column slab (rode_items.hpp), slab after slab, so that the hub rows' nonzeros of
+// one slab of B are worked on at the same time on one XCD and find B's rows in its L2.  A piece's sum goes to its own row
 // of `partial` (piece = slab group * hub rows + hub row; spmm_hub_reduce_kernel adds a row's
 // pieces up), or, without that workspace, is added to its row of C atomically (a hub row
 // then gets one atomic row update per slab: slower than the plain kernels at 512-byte rows).
+// A piece that waves share is finished by the wave that has its first step.
 template <typename T, int TN, bool EDGE>
-__global__ void __launch_bounds__(kWgThreads)
-spmm_hub_kernel(int n, int merge, const int* __restrict__ hub, const int* __restrict__ col,
+__global__ void __launch_bounds__(kHubWavesMax * kWave)
+spmm_hub_kernel(int n, int merge, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col,
                 const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
                 typename DenseVec<T>::Acc* __restrict__ C, typename DenseVec<T>::Acc* __restrict__ partial)
 {
     using S = SpmmShape<T, TN>;
     using A = typename S::Acc;
     constexpr int VEC = S::kVec, LPR = S::kLpr, G = S::kGroupsWave;
-    __shared__ __attribute__((aligned(16))) int lds_c[kWavesPerWg * kWave];
-    __shared__ __attribute__((aligned(16))) A lds_v[kWavesPerWg * kWave];
+    __shared__ __attribute__((aligned(16))) int lds_c[kHubWavesMax * kWave];
+    __shared__ __attribute__((aligned(16))) A lds_v[kHubWavesMax * kWave];
+    __shared__ __attribute__((aligned(16))) A heads[kHubWavesMax][TN]; // a wave's sum of a piece that an earlier wave began
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     const HubPlan hp = hub_plan_view(hub);
-    const long long item = (long long)xcd_logical_block(blockIdx.x, gridDim.x) * kWavesPerWg + wave;
-    if (item >= (long long)hp.n_hub * hub_groups(hp.slabs, merge)) return;
-    const int slab = (int)(item / hp.n_hub) * merge, h = (int)(item % hp.n_hub);
-    const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
-    const int base = piece[slab], cnt = piece[min(slab + merge, hp.slabs)] - base;
-    if (cnt <= 0) return; // (the reduction skips empty pieces too)
-    const int row = hp.rows[h];
+    const int wg = xcd_logical_block(blockIdx.x, gridDim.x);
+    int steps;
+    const HubShare share = hub_share(hp, merge, grid, wg, wave, lane, steps);
     const int ls = lane % LPR, group = lane / LPR;
     const int tile = blockIdx.y * TN;
     const bool col_ok = !EDGE || tile + ls * VEC < n;
     const T* b_lane = B + tile + (col_ok ? ls * VEC : 0);
     constexpr int EPG = VEC / G > 0 ? VEC / G : 1; // elements each group adds
     A total[VEC];
-    spmm_sum_slots<T, TN>(base, 0, cnt, cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
-    if (partial) {
-        if (group == 0 && col_ok) store_row<VEC>(partial + (size_t)item * n + tile + ls * VEC, total);
-        return;
-    }
-    A* c_lane = C + (size_t)row * n + tile + ls * VEC;
+    int open = -1; // the piece that `total` is the first part of
+    for (unsigned long long todo = share.pieces; todo; todo &= todo - 1ull) {
+        const int i = __builtin_ctzll(todo);
+        const HubPart p = hub_part(share, i);
+        spmm_sum_slots<T, TN>(p.base, 0, p.cnt, p.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
+        if (!partial) {
+            A* c_lane = C + (size_t)p.row * n + tile + ls * VEC;
 #pragma unroll
-    for (int x = 0; x < VEC; ++x)
-        if (group == x / EPG && col_ok) atomicAdd(c_lane + x, total[x]);
+            for (int x = 0; x < VEC; ++x)
+                if (group == x / EPG && col_ok) atomicAdd(c_lane + x, total[x]);
+        } else if (!p.starts) {
+            if (group == 0) {
+#pragma unroll
+                for (int x = 0; x < VEC; ++x) heads[wave][ls * VEC + x] = total[x];
+            }
+        } else if (p.ends) {
+            if (group == 0 && col_ok) store_row<VEC>(partial + ((size_t)wg * grid.pieces + i) * n + tile + ls * VEC, total);
+        } else {
+            open = i; // (the last of this wave's pieces)
+        }
+    }
+    if (!partial) return;
+    __syncthreads();
+    if (open >= 0) {
+        const int end = __builtin_amdgcn_readlane(share.before, open) + __builtin_amdgcn_readlane(share.steps, open);
+        for (int w = wave + 1; w < grid.waves && hub_first_step(grid, steps, w) < end; ++w) {
+            if (hub_first_step(grid, steps, w) == hub_first_step(grid, steps, w + 1)) continue; // (fewer steps than waves: it has none)
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) total[x] += heads[w][ls * VEC + x];
+        }
+        if (group == 0 && col_ok) store_row<VEC>(partial + ((size_t)wg * grid.pieces + open) * n + tile + ls * VEC, total);
+    }
 }
 
 // C[hub row, :] += sum of the row's pieces (a hub row is in no other work item, so no
@@ -825,14 +845,14 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     }
     if (e == hipSuccess && hubs) {
         using A = typename DenseVec<T>::Acc;
-        const int merge = hub_merge(n * (int)sizeof(A) / 4);
+        const int merge = hub_merge((size_t)n * sizeof(T), plan.hub_counts[1]);
         const long long pieces = (long long)plan.hub_counts[0] * hub_groups(plan.hub_counts[1], merge);
-        const int gh = grid_for_waves(pieces);
-        if (gh < 0) return hipErrorInvalidConfiguration;
-        dim3 grid(gh, tiles);
+        const HubGrid hub_wgs = hub_grid(plan.hub_counts, merge);
+        if (hub_wgs.wgs < 0) return hipErrorInvalidConfiguration;
+        dim3 grid(hub_wgs.wgs, tiles);
         const size_t need = (size_t)pieces * n * sizeof(A);
         A* partial = plan.hub_workspace && plan.hub_workspace_bytes >= need ? static_cast<A*>(plan.hub_workspace) : nullptr;
-        spmm_hub_kernel<T, TN, EDGE><<<grid, kWgThreads, 0, s1>>>(n, merge, plan.hub, col, val, B, C, partial);
+        spmm_hub_kernel<T, TN, EDGE><<<grid, hub_wgs.waves * kWave, 0, s1>>>(n, merge, hub_wgs, plan.hub, col, val, B, C, partial);
         if (partial) spmm_hub_reduce_kernel<A><<<plan.hub_counts[0], kWgThreads, 0, s1>>>(n, merge, plan.hub, partial, C);
         e = hipGetLastError();
     }

@@ -167,3 +167,35 @@ def test_hub_plan_through_the_c_abi(k):
     assert (written[0].int() + written[1].int() + written[2].int() == 1).all()
     fake = torch.zeros(64, dtype=torch.int32, device=DEV)
     assert sddmm(0, True, fake)[0] != 0
+
+
+@pytest.mark.parametrize("hubs,k,half", [(2, 64, False), (40, 128, False), (300, 128, False), (1200, 128, True), (2300, 64, False), (4600, 128, False)])
+def test_pieces_shared_by_waves(hubs, k, half):
+    """The ways the waves of a workgroup share pieces (by their number: one piece for eight waves, two, four and eight for four), with pieces
+    of one nonzero, empty ones and some that several waves have a part of."""
+    import oracle
+    from gpu_common import TOL_F16, TOL_F32, make_csr, round_half, run_sddmm, run_spmm
+    from helpers import spmm_row_l1_error, sddmm_row_l1_errors
+    from rode_amd import RoDeCSR
+    rng = np.random.default_rng(hubs)
+    m, n = 5000, 70000
+    lens = rng.integers(150, 400, hubs)
+    lens[:2] = 30000, 7000
+    rp, col, val, where = _matrix(rng, m, n, lens)
+    old = RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
+    RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = 64, 1, 0.0
+    try:
+        csr = make_csr(rp, col, val, m, n, k)
+    finally:
+        RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = old
+    assert csr.plan.counts[0] >= hubs
+    B = rng.standard_normal((n, k)).astype(np.float32)
+    L = rng.standard_normal((m, k)).astype(np.float32)
+    Bq, Lq = (round_half(B), round_half(L)) if half else (B, L)
+    tol = TOL_F16 if half else TOL_F32
+    got = run_spmm(csr, B, half)
+    assert spmm_row_l1_error(got, oracle.spmm_f64(rp, col, val, Bq)) <= tol
+    assert np.array_equal(got[where], run_spmm(csr, B, half)[where])  # (a piece's parts are added in one order)
+    ref, scale = oracle.sddmm_f64(rp, col, val, Lq, Bq, with_abs=True)
+    err, cond = sddmm_row_l1_errors(run_sddmm(csr, L, B, half), ref, scale, rp)
+    assert float(err[cond <= 100].max(initial=0.0)) <= tol
