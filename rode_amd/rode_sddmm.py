@@ -59,7 +59,7 @@ class RoDeCSR:
             self.device = torch.device("cuda", torch.cuda.current_device())
         self.row_offsets_cpu = row_offsets.to(dtype=torch.int32, device="cpu").contiguous()
         # one pass over the row offsets: the longest row, the choice of the segment length and of a plan
-        self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len())
+        self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len(8))
         self.max_row_length = self._stats[0]
         if isinstance(config, str):
             if config != "auto":
@@ -145,10 +145,13 @@ class RoDeCSR:
                 self.plan = rode_sddmm_hip.window_plan_rows(plan, res, m2, self.row_offsets, self.column_indices)
                 plan.nonzeros = 0 if self.locality is True else self.nnz
 
-    # A hub plan is made when the rows of at least HUB_MIN_LEN nonzeros (and 8 per 4096
-    # columns) hold a tenth of the matrix and the matrix has at least HUB_MIN_SLABS times 4096
+    # A hub plan takes the rows of at least HUB_MIN_LEN nonzeros, and 8 per 4096 columns: with fewer, the pieces into which the
+    # plan cuts a row are too short (us of SpMM / SDDMM on power-law matrices with rows of 4096 and more -> with this:
+    # 200 K x 128 369 / 345 -> 321 / 309, 330 K x 64 302 / 293 -> 293 / 281, 500 K x 128 837 / 814 -> 809 / 803, 1 M x 128 1684 / 1695 -> 1623 / 1635; rows of
+    # 1024 and more of 2 M x 128: 3585 / 3685 -> 3735 / 3975).  It is made when the rows of eight times HUB_MIN_LEN and more hold a tenth
+    # of the matrix (few long rows reference the same dense rows too seldom) and the matrix has at least HUB_MIN_SLABS times 4096
     # columns (a smaller dense operand stays in the caches by itself).
-    HUB_MIN_LEN = 4096
+    HUB_MIN_LEN = 512
     HUB_MIN_SLABS = 16
     HUB_MIN_SHARE = 0.1
 
@@ -169,8 +172,8 @@ class RoDeCSR:
         enough = 2 * plan.counts[1] >= plan.counts[0]
         return plan if plan.usable and (self.locality is True or enough) else None
 
-    def _hub_min_len(self):
-        return max(self.HUB_MIN_LEN, 8 * ((self.n + 4095) // 4096))
+    def _hub_min_len(self, factor=1):
+        return max(factor * self.HUB_MIN_LEN, 8 * ((self.n + 4095) // 4096))
 
     def _may_hub(self):
         hub_nnz = self._stats[7]  # nonzeros of the rows of that (aligned) length or more
