@@ -333,7 +333,7 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
     // fills the GPU; what is left row by row.
     RowOwners owners;
     int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
-    if (attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T))) {
+    if (attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T), sizeof(T) == 2)) {
         owners.tiles = group_plan_tiles(plan.groups, M);
         owners.n_tiles = row_tiles(M);
         groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);

@@ -587,7 +587,7 @@ hipError_t launch_rows(HeadStrides heads, int nheads, int M, int N, int nnz, con
     // wave per group fills the GPU; what is left row by row.
     RowOwners owners;
     int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = M;
-    if (attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T))) {
+    if (attention_uses_tiles(plan, attention_groups_min<T>(), nheads, N, nnz, D * sizeof(T), sizeof(T) == 2)) {
         owners.tiles = group_plan_tiles(plan.groups, M);
         owners.n_tiles = row_tiles(M);
         groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);
@@ -624,7 +624,7 @@ hipError_t launch_cols(HeadStrides heads, int nheads, int M, int N, int nnz, con
     // by share of the groups in tiles: 0.13 472 -> 500 us, 0.52 470 -> 483, 0.72 473 -> 479, 0.85 465 -> 447, 0.99 457 -> 433.)
     RowOwners owners;
     int groups_left = plan.groups != nullptr && plan.group_counts != nullptr ? plan.group_counts[1] : 0, rows_left = N;
-    if (attention_uses_tiles(plan, kAttentionColsGroupsMin, nheads, M, nnz, D * sizeof(float)) &&
+    if (attention_uses_tiles(plan, kAttentionColsGroupsMin, nheads, M, nnz, D * sizeof(float), sizeof(T) == 2) &&
         5ll * (kTileRows / kGroupRows) * plan.group_counts[3] >= 4ll * plan.group_counts[1]) {
         owners.tiles = group_plan_tiles(plan.groups, N);
         owners.n_tiles = row_tiles(N);

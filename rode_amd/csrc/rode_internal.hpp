@@ -98,13 +98,18 @@ constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (s
 // Do the tiles of a group plan go to the tile kernels?  (They address a head's k and v with 32-bit offsets; N = 0:
 // not said, one head.)  Where the other kernel is the one for groups (groups_min, the pass's own figure), always: 4500 rows
 // of 200 columns in fp32, width 32 / 64 / 128: 17 -> 14, 24 -> 18, 70 -> 28 us.  Where it is a wave per row, from 1.5 M nonzeros
-// over all heads on: a tile takes 11 to 48 us however few there are (its rows' nonzeros outside the run come one row after the
-// other).  400 columns and 64 random ones, halves of width 32 / 64 / 128: 1.0 M nonzeros 12 / 17 / 28 us row by row, 16 / 20 / 28
-// on tiles; 1.4 M 13 / 18 / 29 and 17 / 21 / 29; 2.0 M 19 / 26 / 42 and 18 / 23 / 33; 3.9 M 30 / 42 / 71 and 22 / 27 / 52.
-inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads, int N, long long nnz, size_t row_bytes)
+// over all heads on: a tile takes 10 to 45 us however few there are, and rows in no tile are a launch more.  Us row by row -> on tiles, fp32 / halves:
+// 4096 rows of 256 and 64 random columns, a few rows left over, 1.3 M nonzeros, width 64: 25.4 -> 26.5 / 15.7 -> 19.1, 128: 48.9 -> 47.7 / 25.7 -> 24.9; 3000 of
+// 200 and 16, 1.3 M: 28.7 -> 22.0 / 17.6 -> 14.7, 54.4 -> 37.5 / 29.1 -> 19.5, 0.65 M: 16.3 -> 17.6 / 10.7 -> 13.2, 27.1 -> 26.2 / 16.7 -> 15.7.
+// Where the tiles have all rows, from 0.4 M on (but for fp32 of width 32: 2048 rows of 600 and 96, 1.4 M, 16.3 -> 17.1): 2000 rows of 200 and 16,
+// 0.43 M, width 64: 12.2 -> 11.9 / 9.6 -> 9.8, 128: 19.3 -> 17.5 / 12.6 -> 10.0; 4000 rows, 0.86 M: 20.1 -> 12.1 / 12.9 -> 9.8, 36.3 -> 20.0 / 20.6 -> 10.3;
+// 2000 of 400 and 64, 0.93 M: 21.4 -> 19.0 / 14.0 -> 11.7, 36.7 -> 30.2 / 21.3 -> 16.5.
+inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads, int N, long long nnz, size_t row_bytes, bool halves)
 {
     if (plan.groups == nullptr || plan.group_counts == nullptr || plan.group_counts[1] <= 0 || plan.group_counts[3] <= 0) return false;
-    return (plan.group_counts[1] >= groups_min || nnz * nheads >= 1500000) && attention_tiles_fit(N, row_bytes);
+    const bool all_rows = plan.group_counts[2] == 0 && 4 * plan.group_counts[3] == plan.group_counts[1];
+    const long long enough = all_rows && (halves || row_bytes > 128) ? 400000 : 1500000;
+    return (plan.group_counts[1] >= groups_min || nnz * nheads >= enough) && attention_tiles_fit(N, row_bytes);
 }
 // (rode_attention_tile.hip) the rows of a group plan's tiles, the same arguments; plan: the group plan
 template <typename T>

@@ -349,3 +349,19 @@ def test_rows_with_very_different_numbers_outside_their_runs(d, half):
         assert not now[:, touched].isfinite().all(dim=2).any()
         # (their tiles may be computed row by row now: either is within the bound above)
         assert (now[:, ~touched] - was[:, ~touched]).norm() <= (4e-3 if half and was is not out else 4e-6) * was[:, ~touched].norm()
+
+
+@pytest.mark.parametrize("m,rows_left", [(1600, 0), (1608, 8)])
+def test_fewer_nonzeros_where_the_tiles_have_all_rows(m, rows_left):
+    """0.4 M nonzeros and more, on either side of the rule that gives them to the tiles."""
+    csr, dense = _mask(m, 250, 1, 20, seed=m)
+    assert csr.plan.counts[3] == m // 16 and 400_000 < csr.nnz < 1_500_000 and csr.plan.counts[2] == 0 and m % 16 == rows_left
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    q, k, v, g = (torch.randn(r, 64, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    ins = [t.double().requires_grad_() for t in (q, k, v)]
+    want = _reference(dense, *ins, 0.125)
+    want = (want,) + torch.autograd.grad(want, ins, g.double())
+    ins = [t.clone().requires_grad_() for t in (q, k, v)]
+    out = sparse_attention(csr, *ins, scale=0.125)
+    for a, b in zip((out,) + torch.autograd.grad(out, ins, g), want):
+        assert (a.double() - b).norm() <= 2e-6 * b.norm()
