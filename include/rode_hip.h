@@ -193,6 +193,14 @@ int rode_hip_spmm_ex(int dtype, int flags, int m1, int m2, int k, int n, const v
 size_t rode_hip_window_plan_bytes(int m2);
 int rode_hip_window_plan(int m2, int dense_rows, const int* d_row_indices_residue, const int* d_row_offsets,
                          const int* d_column_indices, void* d_plan, size_t plan_bytes, int* h_counts, void* stream);
+/*
+ * rode_hip_preprocess (k_block 32, vec_len 4) and rode_hip_window_plan in three launches, for a caller that has counted the
+ * residue rows already (m2, which must be what the decomposition finds).  h_counts: HOST int[8] that the GPU can write (pinned memory);
+ * once the stream has been waited for, [0] = n_blk, [1] = n_res, [4..7] = the plan's header.
+ */
+int rode_hip_preprocess_with_plan(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind,
+                                  int* h_counts, int capacity_blocks, void* d_workspace, size_t workspace_bytes, int m2, int dense_rows,
+                                  const int* d_column_indices, void* d_plan, size_t plan_bytes, void* stream);
 size_t rode_hip_window_rows_bytes(int m2);
 int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_row_offsets,
                          const int* d_column_indices, const void* d_plan, void* d_rows, size_t rows_bytes, void* stream);

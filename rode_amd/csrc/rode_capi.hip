@@ -104,6 +104,22 @@ int rode_hip_preprocess_host(int seg_length, int k_block, int vec_len, int M, co
     return e;
 }
 
+int rode_hip_preprocess_with_plan(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind,
+                                  int* h_counts, int capacity_blocks, void* d_workspace, size_t workspace_bytes, int m2, int dense_rows,
+                                  const int* d_column_indices, void* d_plan, size_t plan_bytes, void* stream)
+{
+    if (seg_length <= 0 || M <= 0 || m2 <= 0 || dense_rows < 0 || capacity_blocks < 0) return hipErrorInvalidValue;
+    if (!d_row_ptr || !d_block_r_ind || !d_st_off || !d_residue_r_ind || !h_counts || !d_workspace || !d_column_indices || !d_plan)
+        return hipErrorInvalidValue;
+    if (workspace_bytes < rode::preprocess_workspace_bytes(M) || (reinterpret_cast<uintptr_t>(d_workspace) & 7u)) return hipErrorInvalidValue;
+    if (plan_bytes < rode_hip_window_plan_bytes(m2) || !aligned16(d_plan)) return hipErrorInvalidValue;
+    int* plan = static_cast<int*>(d_plan);
+    const hipError_t e = rode::preprocess_launch(seg_length, 32, 4, M, d_row_ptr, d_block_r_ind, d_st_off, d_residue_r_ind, h_counts,
+                                                 h_counts + 1, d_workspace, capacity_blocks, as_stream(stream), rode::window_plan_chunks(m2), plan);
+    if (e != hipSuccess) return e;
+    return rode::window_plan_launch(m2, dense_rows, d_residue_r_ind, d_row_ptr, d_column_indices, plan, as_stream(stream), h_counts + 4);
+}
+
 size_t rode_hip_window_plan_bytes(int m2) { return m2 < 0 ? 0 : rode::window_plan_ints(m2) * sizeof(int); }
 
 int rode_hip_window_plan(int m2, int dense_rows, const int* d_row_indices_residue, const int* d_row_offsets,

@@ -15,7 +15,7 @@ hipError_t preprocess_static_workspace(void** ptr);
 
 hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind,
                              int* st_off, int* residue_r_ind, int* n_blk, int* n_res, void* workspace,
-                             int capacity_blocks, hipStream_t stream);
+                             int capacity_blocks, hipStream_t stream, int plan_chunks = 0, int* plan_header = nullptr);
 
 // T = dense operand type; values, accumulators and C are float for T = float / __half
 // and double for T = double.
@@ -151,8 +151,11 @@ hipError_t hub_pieces_launch(int hub_rows, int dense_rows, const int* row_ptr, c
 
 size_t window_plan_ints(int m2);
 size_t window_plan_rows_bytes(int m2);
+// (header_counts: null, or where the last workgroup writes the header's four ints; the header itself is then cleared already,
+// by preprocess_launch, which has `chunks` from window_plan_chunks)
+int window_plan_chunks(int m2);
 hipError_t window_plan_launch(int m2, int dense_rows, const int* residue_rows, const int* row_ptr, const int* col,
-                              int* plan, hipStream_t stream);
+                              int* plan, hipStream_t stream, int* header_counts = nullptr);
 hipError_t window_plan_rows_launch(int m2, const int* residue_rows, const int* row_ptr, const int* col, const int* plan,
                                    void* rows, hipStream_t stream);
 

@@ -128,10 +128,13 @@ __device__ __forceinline__ unsigned long long unpack_counts(unsigned long long s
     return (((status >> 31) & 0x7fffffffull) << 32) | (status & 0x7fffffffull);
 }
 
-__global__ void __launch_bounds__(kWgThreads) clear_status_kernel(int words, unsigned long long* __restrict__ status)
+// (header: four ints of a plan that is made after the decomposition, or null; the first is `first`)
+__global__ void __launch_bounds__(kWgThreads)
+clear_status_kernel(int words, unsigned long long* __restrict__ status, int first, int* __restrict__ header)
 {
     const int i = blockIdx.x * kWgThreads + threadIdx.x;
     if (i < words) status[i] = 0ull;
+    if (header != nullptr && i < 4) header[i] = i == 0 ? first : 0;
 }
 
 // A wait that cannot be met (it never happened in testing: a tile only waits for tiles that
@@ -303,7 +306,7 @@ hipError_t preprocess_static_workspace(void** ptr)
 
 hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind,
                              int* st_off, int* residue_r_ind, int* n_blk, int* n_res, void* workspace,
-                             int capacity_blocks, hipStream_t stream)
+                             int capacity_blocks, hipStream_t stream, int plan_chunks, int* plan_header)
 {
     const TileShape shape = tile_shape_for((size_t)(M > 0 ? M : 0));
     const int ntiles = (int)(((size_t)M + shape.rows() - 1) / shape.rows());
@@ -313,7 +316,7 @@ hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* 
     }
     unsigned long long* ws = static_cast<unsigned long long*>(workspace);
     // (a fill kernel, not a memset: the call may be recorded into a HIP graph)
-    clear_status_kernel<<<(ntiles + 2 + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(ntiles + 2, ws);
+    clear_status_kernel<<<(ntiles + 2 + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(ntiles + 2, ws, plan_chunks, plan_header);
 #define RODE_DECOMPOSE(THREADS, RPT)                                                                                      \
     decompose_kernel<THREADS, RPT><<<ntiles, THREADS, 0, stream>>>(make_params(seg, kblock, veclen), M, ntiles, capacity_blocks, row_ptr, \
                                                                    ws, block_r_ind, st_off, residue_r_ind, n_blk, n_res)

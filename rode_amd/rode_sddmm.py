@@ -74,7 +74,7 @@ class RoDeCSR:
 
         self.column_indices = column_indices.to(dtype=torch.int32, device=self.device).contiguous()
         self.values = values.to(dtype=torch.float32, device=self.device).contiguous()
-        self.row_offsets = self.row_offsets_cpu.to(device=self.device)
+        self.row_offsets = torch.empty(self.row_offsets_cpu.shape, dtype=torch.int32, device=self.device) # (filled along with the decomposition)
         if locality not in (True, False, "auto"):
             raise ValueError(f'locality must be True, False or "auto", got {locality!r}')
         self.locality = locality
@@ -128,7 +128,7 @@ class RoDeCSR:
         with rode_sddmm_hip._on_device(self.device):
             blk, st, res, m1, m2, data, counts = _lib.host_call().decompose(
                 self.row_offsets_cpu, self.row_offsets, self.column_indices if self.locality and not others else None,
-                self.n, self.config["seg_length"], rode_sddmm_hip._stream_handle(self.device))
+                self.n, self.config["seg_length"], rode_sddmm_hip._stream_handle(self.device), True)
         self.block_indices = blk
         self.st_offsets = st
         self.residue_indices = res

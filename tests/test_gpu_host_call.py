@@ -153,3 +153,33 @@ def test_decomposition_without_memory_leaves_nothing_running():
     assert refused >= 6 and mode.left == 1  # the lists, the scratch, the plan and the counts
     for a, b in zip(got, want):
         assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
+
+
+@pytest.mark.parametrize("upload", [False, True])
+@pytest.mark.parametrize("m,n", [(1, 600), (127, 600), (128, 600), (129, 600), (33000, 33000)])
+def test_decomposition_with_a_plan_equals_its_parts(m, n, upload):
+    """The lists and the plan that one call makes (counts written by the last workgroup) against the separate entries,
+    and the plan's numbers against a count of the columns inside each window.  Rows of at most 28 (31 from their aligned start), so that all
+    of their nonzeros are in the residue list; every third run of 128 rows has its columns anywhere."""
+    rng = np.random.default_rng(m + 7 * upload)
+    lens = rng.integers(1, 29, m)
+    ro = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    row = np.repeat(np.arange(m), lens)
+    near = np.clip(row * n // m + rng.integers(-90, 90, len(row)), 0, n - 1)
+    col = np.where(row // 128 % 3 == 1, rng.integers(0, n, len(row)), near).astype(np.int32)
+    host, cols = torch.from_numpy(ro), torch.from_numpy(col).cuda()
+    on_gpu = torch.full((m + 1,), -1, dtype=torch.int32, device="cuda") if upload else host.cuda()
+    args = (host, on_gpu, cols, n, 512, rode_sddmm_hip._stream_handle(cols.device))
+    blk, st, res, m1, m2, data, counts = _lib.host_call().decompose(*args, *([True] if upload else []))
+    assert torch.equal(on_gpu.cpu(), host)
+    parts = rode_sddmm_hip.preprocess_device(on_gpu, int(ro[-1]), 512, 32, 4)
+    assert (m1, m2) == tuple(parts[3:]) and all(torch.equal(a, b) for a, b in zip((st, res), parts[1:3]))
+    plan = rode_sddmm_hip.window_plan(res, m2, on_gpu, cols, n)
+    assert counts == plan.counts and data[:4].tolist() == counts and torch.equal(data[4:4 + 4 * counts[0]], plan.data[4:4 + 4 * counts[0]])
+    listed = data[4:4 + 4 * counts[0]].view(-1, 4).tolist()
+    assert counts[0] == (m2 + 127) // 128 and counts[1] == sum(d[1] > 0 for d in listed)
+    rows = res[:m2].cpu().numpy()
+    for chunk, (first, count, slots, misses) in enumerate(listed):
+        c = np.concatenate([col[ro[r]:ro[r + 1]] for r in rows[128 * chunk:128 * chunk + 128]])
+        assert slots == len(c) and (count == 0 or misses == np.sum((c < first) | (c >= first + count)))
+    assert m < 128 or counts[1] > 0
