@@ -320,6 +320,12 @@ int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, co
                           const int* d_row_indices2, const int* d_row_seg_st_offsets, const void* d_B, void* d_C,
                           const rode_hip_plans* plans, void* stream1, void* stream2);
 
+/* C[M x n] = A B into a C that holds anything: the whole lists, every row of C stored or cleared as it needs, in one launch
+ * where that is possible (no row is longer than `longest` aligned slots, which the caller knows; 0: not known) and with rode_hip_spmm_clear_rows_beyond before it otherwise. */
+int rode_hip_spmm_new(int dtype, int M, int longest, int m1, int m2, int k, int n, const void* d_values, const int* d_column_indices,
+                      const int* d_row_offsets, const int* d_row_indices1, const int* d_row_indices2, const int* d_row_seg_st_offsets,
+                      const void* d_B, void* d_C, const rode_hip_plans* plans, void* stream);
+
 /* The longest row, in aligned slots, that rode_hip_spmm_planned(..., RODE_SPMM_WHOLE_LISTS |
  * RODE_SPMM_OVERWRITE, m1, ..., plans, ...) stores with one work item; 0: none of the rows
  * with 32 aligned slots or more (few block segments: every work item adds; a hub plan).

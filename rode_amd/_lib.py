@@ -35,6 +35,7 @@ SIGNATURES = {
     "rode_hip_hub_plan": (c_int, [c_int] * 4 + [c_void_p] * 3 + [c_size_t, c_void_p, c_void_p]),
     "rode_hip_hub_workspace_bytes": (c_size_t, [c_void_p, c_int, c_int]),
     "rode_hip_spmm_planned": (c_int, [c_int] * 6 + [c_void_p] * 11),
+    "rode_hip_spmm_new": (c_int, [c_int] * 7 + [c_void_p] * 10),
     "rode_hip_spmm_clear_rows_beyond": (c_int, [c_int] * 4 + [c_void_p] * 3),
     "rode_hip_spmm_clear_rows": (c_int, [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "rode_hip_sddmm_f32": (c_int, [c_int] * 4 + [c_void_p] * 11),

@@ -35,13 +35,13 @@ def _spmm(csr, values, dense):
     width = dense.shape[1]
     out = _lib.host_call().spmm(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
                                 csr.column_indices, values, csr.m, csr.n, dense, csr.plans_address(width),
-                                csr.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(csr.device))
+                                csr.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(csr.device), csr.longest_row)
     if out is not None:
         return out
     return rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2,
                                        csr.row_offsets, csr.column_indices, values, csr.m, csr.n, dense, plan=csr.plan,
                                        plans=csr.call_plans(width, values.element_size()),
-                                       every_row_stored=csr.spmm_stores_every_row())
+                                       every_row_stored=csr.spmm_stores_every_row(), longest_row=csr.longest_row)
 
 
 class SddmmFunction(torch.autograd.Function):

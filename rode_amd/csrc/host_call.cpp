@@ -145,13 +145,15 @@ PyObject* sddmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     }
 }
 
-// spmm(<matrix>, dense, plans address, every row stored, stream) -> C or None
+// spmm(<matrix>, dense, plans address, every row stored, stream[, longest row in aligned slots]) -> C or None
 PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     try {
     Matrix a;
-    long long plans, stored, stream;
-    if (count != 14 || !matrix_of(args, a) || !int_of(args[11], plans) || !int_of(args[12], stored) || !int_of(args[13], stream)) Py_RETURN_NONE;
+    long long plans, stored, stream, longest = 0;
+    if ((count != 14 && count != 15) || !matrix_of(args, a) || !int_of(args[11], plans) || !int_of(args[12], stored) || !int_of(args[13], stream) ||
+        (count == 15 && (!int_of(args[14], longest) || longest < 0 || longest > INT32_MAX)))
+        Py_RETURN_NONE;
     const at::Tensor* dense = tensor_of(args[10]);
     const int kind = dense_kind(a, dense, a.n);
     if (kind < 0) Py_RETURN_NONE;
@@ -164,19 +166,17 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     const void* b = data(*dense);
     float* c = floats(out);
     int code = 0;
-    const char* what = "rode_hip_spmm_clear_rows_beyond";
+    const char* what = stored ? "rode_hip_spmm_planned" : "rode_hip_spmm_new";
     {
         NoGil no_gil;
         const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
         void* s = reinterpret_cast<void*>(stream);
-        // (only the rows that the kernels add to, or skip, need clearing)
-        if (!stored)
-            code = rode_hip_spmm_clear_rows_beyond((int)a.m, (int)width, 4, rode_hip_spmm_overwrite_limit((int)a.m1, p), row_ptr, c, s);
-        if (code == 0) {
-            what = "rode_hip_spmm_planned";
+        if (stored)
             code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, (int)a.m1, (int)a.m2, (int)a.n, (int)width, val, col,
                                          row_ptr, block, residue, start, b, c, p, s, s);
-        }
+        else // (some rows are added to, or in no list)
+            code = rode_hip_spmm_new(kind, (int)a.m, (int)longest, (int)a.m1, (int)a.m2, (int)a.n, (int)width,
+                                     val, col, row_ptr, block, residue, start, b, c, p, s);
     }
     if (code != 0) return failed(what, code);
     return THPVariable_Wrap(out);
@@ -519,7 +519,7 @@ PyMethodDef methods[] = {
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(sddmm)), METH_FASTCALL,
      "sddmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, k, lhs, rhs, plans, stream) -> tensor or None"},
     {"spmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(spmm)), METH_FASTCALL,
-     "spmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, dense, plans, stored, stream) -> tensor or None"},
+     "spmm(block, residue, start, m1, m2, row_offsets, columns, values, m, n, dense, plans, stored, stream[, longest]) -> tensor or None"},
     {"attention", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention)), METH_FASTCALL,
      "attention(row_offsets, columns, values, q, k, v, scale, keep, plans, stream) -> (out, scores, stats) or None"},
     {"attention_backward", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(attention_backward)), METH_FASTCALL,

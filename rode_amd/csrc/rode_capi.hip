@@ -253,10 +253,10 @@ int rode_hip_spmm_ex(int dtype, int flags, int m1, int m2, int k, int n, const v
                                  d_row_indices2, d_row_seg_st_offsets, d_B, d_C, nullptr, stream1, stream2);
 }
 
-int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, const void* d_values,
-                          const int* d_column_indices, const int* d_row_offsets, const int* d_row_indices1,
-                          const int* d_row_indices2, const int* d_row_seg_st_offsets, const void* d_B, void* d_C,
-                          const rode_hip_plans* plans, void* stream1, void* stream2)
+static int spmm_any(int dtype, int flags, int rows, int longest, int m1, int m2, int k, int n, const void* d_values,
+                    const int* d_column_indices, const int* d_row_offsets, const int* d_row_indices1,
+                    const int* d_row_indices2, const int* d_row_seg_st_offsets, const void* d_B, void* d_C,
+                    const rode_hip_plans* plans, void* stream1, void* stream2)
 {
     constexpr int kKnown = RODE_SPMM_WHOLE_LISTS | RODE_SPMM_ONLY_BLOCK | RODE_SPMM_ONLY_RESIDUE | RODE_SPMM_ONLY_HUB |
                            RODE_SPMM_OVERWRITE;
@@ -274,6 +274,7 @@ int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, co
     rode::PlanRef plan;
     if (!plan_ref(plans, m2, plan)) return hipErrorInvalidValue;
     plan.dense_rows = k > 0 ? k : 0;
+    plan.c_rows = rows, plan.longest = longest;
     // the hub and group kernels replace work items of both lists: only with the complete decomposition
     if ((plan.hub || plan.groups) && !(flags & RODE_SPMM_WHOLE_LISTS)) return hipErrorInvalidValue;
     switch (dtype) {
@@ -291,6 +292,26 @@ int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, co
                                          static_cast<const double*>(d_B), static_cast<double*>(d_C), flags, plan, s1, s2);
     default: return hipErrorInvalidValue;
     }
+}
+
+int rode_hip_spmm_planned(int dtype, int flags, int m1, int m2, int k, int n, const void* d_values,
+                          const int* d_column_indices, const int* d_row_offsets, const int* d_row_indices1,
+                          const int* d_row_indices2, const int* d_row_seg_st_offsets, const void* d_B, void* d_C,
+                          const rode_hip_plans* plans, void* stream1, void* stream2)
+{
+    return spmm_any(dtype, flags, 0, 0, m1, m2, k, n, d_values, d_column_indices, d_row_offsets, d_row_indices1, d_row_indices2, d_row_seg_st_offsets,
+                    d_B, d_C, plans, stream1, stream2);
+}
+
+int rode_hip_spmm_new(int dtype, int M, int longest, int m1, int m2, int k, int n, const void* d_values, const int* d_column_indices,
+                      const int* d_row_offsets, const int* d_row_indices1, const int* d_row_indices2, const int* d_row_seg_st_offsets,
+                      const void* d_B, void* d_C, const rode_hip_plans* plans, void* stream)
+{
+    if (M < 0 || longest < 0 || (dtype != RODE_DENSE_F32 && dtype != RODE_DENSE_F16 && dtype != RODE_DENSE_F64)) return hipErrorInvalidValue;
+    if (m1 == 0 && m2 == 0) return rode_hip_spmm_clear_rows(M, n, dtype == RODE_DENSE_F64 ? 8 : 4, d_row_offsets, d_C, stream);
+    if (M == 0 || !d_row_offsets || !d_C) return hipErrorInvalidValue;
+    return spmm_any(dtype, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, M, longest, m1, m2, k, n, d_values, d_column_indices, d_row_offsets,
+                    d_row_indices1, d_row_indices2, d_row_seg_st_offsets, d_B, d_C, plans, stream, stream);
 }
 
 int rode_hip_spmm_overwrite_limit(int m1, const rode_hip_plans* plans)

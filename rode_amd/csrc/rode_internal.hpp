@@ -48,6 +48,8 @@ struct PlanRef {
     // many column tiles it is dealt out to the XCDs
     int dense_rows = 0, shards = 0;
     int nonzeros = 0;           // of the matrix, as the caller says (0: not said)
+    // SpMM: rows of C where it is not cleared (0: it is, or every row is stored), the longest row in aligned slots (0: not said)
+    int c_rows = 0, longest = 0;
     bool columns_local = false; // the caller knows that the columns of neighbouring rows lie close together
     // Segment length of the decomposition the lists were made with, 0: not known
     int seg_length = 0;

@@ -47,6 +47,10 @@ namespace {
 // segments on the difference is below 1 %.
 constexpr int kOwnedRowSlots = 1024;
 constexpr int kOwnedMinSegments = 1024;
+// Where the caller knows that no row is longer than this, a matrix of fewer segments has its rows summed whole as well: a wave has no
+// more than two steps to do, every row is stored, and C is not cleared beforehand (us, cleared and added to -> stored: 512 x 512
+// of 16 to 64 nonzeros, widths 32 to 128 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3 -> 15.0, 250 K 150 -> 143).
+constexpr int kShortRowSlots = 128;
 // Without the promise the block kernel may still merge the short segments of a row that
 // the list it was given holds, when there are this many of them.
 constexpr int kMergeMinSegments = 16384;
@@ -58,6 +62,10 @@ constexpr int kMergeMinSegments = 16384;
 // rows, 65 K x 65 K, 1 M nonzeros, width 128: 75 us in two launches, 63 in one.)
 constexpr int kPairMaxWorkgroups = 16384;
 constexpr int kPairMaxSharded = 65536;
+// Residue rows alone, with the rows without slots of an uncleared C: up to this many (a clearing launch costs 2 to 3 us: 512 rows of 4 x 64
+// 8.4 -> 6.3, 16 K of 8 x 128 9.9 -> 7.8, 100 K of 8 x 32 18.6 -> 16.4, 40 K of 8 halves x 128 14.7 -> 12.5), then the residue kernel, which
+// has more waves per CU, with a launch before it.
+constexpr int kPairMaxAlone = 4096;
 
 // Sharding.  Every XCD has an L2 of its own (4 MB), and rows of B that are referenced at random are
 // fetched into all eight.  When a row of B is 2, 4 or 8 lines of 128 bytes, C is computed in column
@@ -408,19 +416,47 @@ spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners
                                    C, plan);
 }
 
+// The rows of C without slots, which are in neither list, where nobody cleared C: 64 at a time to the waves.
+// (Rows of more than 1024 slots, which several waves add to, still need the launch before: with a workgroup for each of them in here
+// spmm of 65 K x 128, ten such rows, took 57.8 us instead of 60.0, but the registers of that cost the kernel a wave per SIMD: 40 K rows of 32 x 64
+// 38.6 -> 43.2, lognormal 100 K of 16 x 32 30.4 -> 35.3.)
+template <typename A, int TN, bool EDGE>
+__device__ __forceinline__ void spmm_empty_rows(int bid, int nblocks, int tile, int rows, int n, const int* __restrict__ row_ptr, A* __restrict__ C)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    for (long long from = ((long long)bid * kWavesPerWg + wave) * kWave; from < rows; from += (long long)nblocks * kWgThreads) {
+        const int mine = (int)min(from + lane, (long long)rows - 1);
+        const int start = row_ptr[mine];
+        const bool empty = from + lane < rows && row_ptr[mine + 1] - start + (start & (kVecLen - 1)) <= 0;
+        for (unsigned long long todo = __ballot(empty); todo; todo &= todo - 1ull) {
+            A* to = C + (size_t)(from + __builtin_ctzll(todo)) * n + tile;
+            for (int x = lane; x < TN; x += kWave)
+                if (!EDGE || tile + x < n) to[x] = A(0);
+        }
+    }
+}
+inline int empty_row_workgroups(int rows) { return (min((rows + 1023) / 1024, 4096) + kXcds - 1) / kXcds * kXcds; }
+
 // Both lists in one launch: the first g1 workgroups of a grid row (of every tile of a sharded
 // grid) work on block segments, the others on residue rows.  For matrices so small that a launch costs as much as its
 // kernel (a kernel of a few microseconds); the two parts then also fill the GPU together.
+// g0 > 0 (with STORE: every other row is stored): as many workgroups after them zero the rows without slots.
 template <typename T, int TN, bool EDGE, int WALK, bool STORE>
 __global__ void __launch_bounds__(kWgThreads)
-spmm_pair_kernel(int shards, int g1, int m1, int m2, int n, int owned_slots, int chunk_hint, RowOwners owners,
+spmm_pair_kernel(int shards, int g0, int rows, int g1, int m1, int m2, int n, int owned_slots, int chunk_hint, RowOwners owners,
                  const int* __restrict__ block_rows,
                  const int* __restrict__ residue_rows, const int* __restrict__ st_off, const int* __restrict__ row_ptr,
                  const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
                  const T* __restrict__ B, typename DenseVec<T>::Acc* __restrict__ C, const int* __restrict__ plan)
 {
+    const int lists = gridDim.x - (STORE ? g0 * shards : 0);
+    if (STORE && (int)blockIdx.x >= lists) {
+        const TilePlace at = tile_place(blockIdx.x - lists, g0, shards);
+        spmm_empty_rows<typename DenseVec<T>::Acc, TN, EDGE>(at.bid, g0, at.tile * TN, rows, n, row_ptr, C);
+        return;
+    }
     const bool segments = (int)blockIdx.x < g1 * shards;
-    const int g = segments ? g1 : gridDim.x / shards - g1;
+    const int g = segments ? g1 : lists / shards - g1;
     const TilePlace at = tile_place(segments ? blockIdx.x : blockIdx.x - g1 * shards, g, shards);
     if (segments)
         spmm_block_body<T, TN, EDGE, WALK, STORE>(at.bid, g, at.tile * TN, m1, n, owned_slots, chunk_hint, owners, block_rows, st_off, row_ptr, col, val,
@@ -770,7 +806,9 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
                   typename DenseVec<T>::Acc* C, int flags, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
     const int tiles = (n + TN - 1) / TN;
-    const int owned_slots = (flags & kSpmmWholeLists) && m1 >= kOwnedMinSegments ? kOwnedRowSlots : 0;
+    // (rows known to be short: one wave has no more to do for all of a row)
+    const bool short_rows = plan.longest > 0 && plan.longest <= kShortRowSlots;
+    const int owned_slots = (flags & kSpmmWholeLists) && (m1 >= kOwnedMinSegments || short_rows) ? kOwnedRowSlots : 0;
     // what the block kernel is told: rows it owns, or (negative) only that it may merge short
     // segments - which needs no promise, and with this many segments costs no parallelism
     const int block_owned = owned_slots > 0 ? owned_slots : (m1 >= kMergeMinSegments ? -1 : 0);
@@ -786,7 +824,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     }
     // rows with a single work item are stored instead of added (spmm_overwrite_limit says which)
     const bool overwrite = (flags & kSpmmOverwrite) != 0;
-    owners.overwrite = overwrite && spmm_overwrite_limit(m1, hub_plan) > 0;
+    owners.overwrite = overwrite && owned_slots > 0 && !hub_plan;
     const int only = flags & kOnlyMask; // one kernel family of the call (timing each on its own)
     const bool hubs = hub_plan && (only == 0 || only == kSpmmOnlyHub);
     const bool grouped = group_plan && (only == 0 || only == kSpmmOnlyHub); // (timed with the hub kernels)
@@ -813,14 +851,27 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     const bool block = lists && m1 > 0 && (only == 0 || only == kSpmmOnlyBlock);
     const bool residue = lists && m2 > 0 && (only == 0 || only == kSpmmOnlyResidue);
     hipError_t e = hipSuccess;
-    if (block && residue && standard_residue && s1 == s2 && (long long)(g1 + g2) * tiles <= (shards > 1 ? kPairMaxSharded : kPairMaxWorkgroups)) {
-        dim3 grid((g1 + g2) * shards, tile_rows);
+    // (without block segments only where C is not cleared and the launch is small: the residue kernel has more waves per CU)
+    const bool alone = m1 == 0 && plan.c_rows > 0 && short_rows && (long long)g2 * tiles <= kPairMaxAlone;
+    const bool pair = (block || alone) && residue && standard_residue && s1 == s2 &&
+                      (long long)(g1 + g2) * tiles <= (shards > 1 ? kPairMaxSharded : kPairMaxWorkgroups);
+    int g0 = 0;
+    if (plan.c_rows > 0) { // C is not cleared
+        if (pair && owners.overwrite && !group_plan && plan.dev == nullptr && plan.longest > 0 && plan.longest <= kOwnedRowSlots) {
+            g0 = empty_row_workgroups(plan.c_rows);
+        } else {
+            e = spmm_clear_rows_launch(plan.c_rows, (size_t)n * sizeof(typename DenseVec<T>::Acc), owners.overwrite ? kOwnedRowSlots : 0, row_ptr, C, s1);
+            if (e != hipSuccess) return e;
+        }
+    }
+    if (pair) {
+        dim3 grid((g0 + g1 + g2) * shards, tile_rows);
         auto kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 2, true> : spmm_pair_kernel<T, TN, EDGE, 2, false>;
         if (chunk_hint == 1)
             kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 0, true> : spmm_pair_kernel<T, TN, EDGE, 0, false>;
         else if (chunk_hint > 1)
             kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 1, true> : spmm_pair_kernel<T, TN, EDGE, 1, false>;
-        kernel<<<grid, kWgThreads, 0, s1>>>(shards, g1, m1, m2, n, block_owned, chunk_hint, owners, block_rows, residue_rows, st_off,
+        kernel<<<grid, kWgThreads, 0, s1>>>(shards, g0, plan.c_rows, g1, m1, m2, n, block_owned, chunk_hint, owners, block_rows, residue_rows, st_off,
                                             row_ptr, col, val, B, C, plan.dev);
         e = hipGetLastError();
     } else {

@@ -423,7 +423,7 @@ def sddmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offset
 
 def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets, column_indices, values, m, k,
                  dense_matrix, out=None, whole_lists=True, plan=None, seg_length=0, checked_lists=False, plans=None,
-                 every_row_stored=False):
+                 every_row_stored=False, longest_row=0):
     """C = A_csr @ dense_matrix through ``rode_hip_spmm_f32`` / ``_f16``
     (host API ``RoDe_SpMM/RoDeSpmm.h:4-8``).  ``dense_matrix`` is (k, n) with n a
     multiple of 4 (8 for fp16, 2 for fp64), fp32 / fp16 (fp32 ``values``) or fp64 (fp64 ``values``); the
@@ -436,7 +436,8 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     ``sddmm_forward`` (``plans``: of (plan, this width and element size, whole_lists, seg_length)).
     ``every_row_stored``: with ``out`` None and ``whole_lists``, the caller has checked
     (``rode_hip_spmm_overwrite_limit``) that every row of the matrix has slots and a single
-    work item: the kernels then store their rows (``RODE_SPMM_OVERWRITE``) and nothing is cleared."""
+    work item: the kernels then store their rows (``RODE_SPMM_OVERWRITE``) and nothing is cleared.
+    ``longest_row``: the longest row in aligned slots (0: not known; ``rode_hip_spmm_new``)."""
     if not checked_lists:
         for t, name in ((block_indices, "block_indices"), (residue_indices, "residue_indices"),
                         (st_offsets, "st_offsets"), (row_offsets, "row_offsets"), (column_indices, "column_indices"),
@@ -467,10 +468,11 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
         # only the rows the kernels add to (or skip) need clearing, the others are overwritten
         out = torch.empty((m, n), dtype=out_dtype, device=values.device)
         _check_data(out, "out")
-        if not (every_row_stored and whole_lists):
-            stored = lib.rode_hip_spmm_overwrite_limit(m1, ctypes.byref(plans)) if whole_lists else 0
+        # (no block segment, and every row in the residue list: every row is stored)
+        every_row_stored = every_row_stored or (m1 == 0 and m2 == m)
+        if not whole_lists:
             with _on_device(values.device):
-                _lib.check(lib.rode_hip_spmm_clear_rows_beyond(m, n, out.element_size(), stored, row_offsets.data_ptr(),
+                _lib.check(lib.rode_hip_spmm_clear_rows_beyond(m, n, out.element_size(), 0, row_offsets.data_ptr(),
                                                                out.data_ptr(), _stream_handle(values.device)),
                            "rode_hip_spmm_clear_rows_beyond")
     else:
@@ -482,6 +484,12 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     dtype = {torch.float32: 0, torch.float16: 1, torch.float64: 2}[dense_matrix.dtype]  # RODE_DENSE_*
     with _on_device(values.device):
         s = _stream_handle(values.device)
+        if overwrite and not every_row_stored: # (some rows are added to, or in no list)
+            code = lib.rode_hip_spmm_new(dtype, m, longest_row, m1, m2, k, n, values.data_ptr(), column_indices.data_ptr(), row_offsets.data_ptr(),
+                                         block_indices.data_ptr(), residue_indices.data_ptr(), st_offsets.data_ptr(),
+                                         dense_matrix.data_ptr(), out.data_ptr(), ctypes.byref(plans), s)
+            _lib.check(code, "rode_hip_spmm_new")
+            return out
         flags = (_lib.SPMM_WHOLE_LISTS if whole_lists else 0) | (_lib.SPMM_OVERWRITE if overwrite else 0)
         code = lib.rode_hip_spmm_planned(dtype, flags, m1, m2, k, n,
                                          values.data_ptr(), column_indices.data_ptr(), row_offsets.data_ptr(),

@@ -590,3 +590,52 @@ def test_overwrite_leaves_other_rows_to_the_callers_clearing():
     want = oracle.spmm_f64(rp, col, val, B) + np.where(added[:, None], 7.0, 0.0)
     assert np.abs(C.cpu().numpy() - want).max() <= 1e-4 * max(1.0, np.abs(want).max())
     assert _spmm_overwrite(csr, dB, C, _lib.SPMM_OVERWRITE) != 0   # not without the whole-lists promise
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
+@pytest.mark.parametrize("rows,lengths,longest,k", [
+    (300, (0, 5), 0, 32),           # residue rows only, and empty ones
+    (5000, (0, 9), 0, 64),
+    (40000, (0, 4), 0, 128),        # ... too many workgroups for one launch (fp32)
+    (700, (0, 60), 0, 128),         # fewer than 1024 segments, every row short: owned by a wave each
+    (700, (0, 60), 128, 40),        # (the longest such row; a width that ends inside a tile)
+    (700, (0, 60), 129, 64),        # one row past it: cleared beforehand
+    (3000, (0, 80), 1024, 64),      # the longest row with one owner
+    (3000, (0, 80), 1025, 64),      # more than that: cleared beforehand
+    (6000, (0, 70), 500, 256),      # column tiles dealt out to the XCDs
+    (64, (32, 33), 0, 32),          # (aligned lists: most rows have no tail)
+])
+def test_product_into_memory_that_holds_anything(rows, lengths, longest, k, dtype):
+    """rode_hip_spmm_new: every row of C stored or cleared, whatever C holds before (NaN here), against 64 bits.  A
+    sum of n products is off by at most (n + 2) roundings of the sum of their magnitudes (twice that where the reference is
+    no wider).  ``longest``: the longest row, in aligned slots (0: as drawn)."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, _lib, rode_spmm
+    rng = np.random.default_rng(rows + k)
+    lens = rng.integers(*lengths, rows)
+    lens[rng.integers(0, rows, rows // 8)] = 0
+    if longest:
+        lens[rows // 2] = longest - sum(lens[:rows // 2]) % 4
+    cols = 6000
+    row_ptr = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(cols, n, replace=False)) for n in lens]).astype(np.int32)
+    val, B = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((cols, k)).astype(np.float32)
+    B = round_half(B) if dtype == "f16" else B
+    want, scale = oracle.spmm_f64(row_ptr, col, val, B, with_abs=True)
+    bound = torch.from_numpy(scale * (lens[:, None] + 2) * (2.0 ** -52 if dtype == "f64" else 2.0 ** -24)).to(DEV)
+    want, val = torch.from_numpy(want).to(DEV), torch.from_numpy(val).to(DEV, torch.float64 if dtype == "f64" else torch.float32)
+    B = torch.from_numpy(B).to(DEV, torch.float16 if dtype == "f16" else val.dtype)
+    csr = RoDeCSR(torch.from_numpy(row_ptr), torch.from_numpy(col), val.float(), DEV, rows, cols, k, config="auto").with_values(val)
+    assert not longest or csr.longest_row == longest
+    lib = _lib.load()
+    for longest_row in (csr.longest_row, 0):
+        out = torch.full((rows, k), float("nan"), dtype=val.dtype, device=DEV)
+        code = lib.rode_hip_spmm_new({"f32": 0, "f16": 1, "f64": 2}[dtype], rows, longest_row, csr.m1, csr.m2, cols, k, val.data_ptr(),
+                                     csr.column_indices.data_ptr(), csr.row_offsets.data_ptr(), csr.block_indices.data_ptr(),
+                                     csr.residue_indices.data_ptr(), csr.st_offsets.data_ptr(), B.data_ptr(), out.data_ptr(),
+                                     ctypes.addressof(csr.call_plans(k, val.element_size())), torch.cuda.current_stream().cuda_stream)
+        assert code == 0
+        assert bool(((out.double() - want).abs() <= bound).all())
+    if dtype != "f64":
+        assert bool(((rode_spmm(csr, B).double() - want).abs() <= bound).all())
