@@ -50,7 +50,7 @@ def kernel_sources_fingerprint():
     h = hashlib.sha256()
     for name in ("rode_device.hpp", "rode_items.hpp", "rode_tile.hpp", "rode_units.hpp", "rode_window.hpp", "rode_spmm.hip", "rode_sddmm.hip",
                  "rode_spmm_window.hip", "rode_sddmm_window.hip", "rode_attention.hip", "rode_attention_tile.hip",
-                 "rode_attention_backward.hip", "rode_attention_backward_tile.hip",
+                 "rode_attention_backward.hip", "rode_attention_backward_tile.hip", "rode_attention_backward_cols_tile.hip",
                  "rode_group.hip", "rode_hub.hip"):
         with open(os.path.join(ROOT, "rode_amd", "csrc", name), "r", encoding="utf-8") as f:
             for line in f:

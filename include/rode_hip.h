@@ -215,9 +215,9 @@ int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_
  * once for all of them.  The other kernels leave those rows out.  Results are
  * the same up to the order of the fp32 additions inside a hub row.
  *   dense_rows   rows of the dense operand (columns of the sparse matrix)
- *   min_len      >= RODE_HIP_HUB_MIN_LEN; a piece should hold dozens of nonzeros: 4096 and
- *                dense_rows / 512 are sensible lower bounds (measured on a 2 M x 2 M
- *                power-law matrix: 4096 is best, 2048 and 8192 gain less, 1024 loses)
+ *   min_len      >= RODE_HIP_HUB_MIN_LEN; 512 and dense_rows / 512 (8 nonzeros per 4096 columns) are sensible lower
+ *                bounds (power-law matrices of 200 K to 2 M columns: half of that loses, the rows of
+ *                eight times that should hold a tenth of the nonzeros for the plan to pay)
  *   d_plan       rode_hip_hub_plan_bytes(M, dense_rows, nnz, min_len) bytes, 16-byte aligned, out
  *   h_counts     HOST int[8], out (the call waits for its two kernels): [0] hub rows,
  *                [1] slabs, [2] min_len, [3] 1 if the plan is usable - every hub row's column

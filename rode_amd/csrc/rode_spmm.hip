@@ -48,9 +48,11 @@ namespace {
 constexpr int kOwnedRowSlots = 1024;
 constexpr int kOwnedMinSegments = 1024;
 // Where the caller knows that no row is longer than this, a matrix of fewer segments has its rows summed whole as well: a wave has no
-// more than two steps to do, every row is stored, and C is not cleared beforehand (us, cleared and added to -> stored: 512 x 512
-// of 16 to 64 nonzeros, widths 32 to 128 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3 -> 15.0, 250 K 150 -> 143).
-constexpr int kShortRowSlots = 128;
+// more than six steps to do, every row is stored, and C is not cleared beforehand (us, cleared and added to -> stored, widths 32 / 128 / 128 of
+// halves: 512 x 512 of 16 to 64 nonzeros 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3 -> 15.0, 250 K 150 -> 143; longest
+// row 168 7.7 / 10.6 / 12.0 -> 5.7 / 6.0 / 5.7, 227 7.8 / 9.8 / 10.7 -> 5.7 / 6.4 / 5.7, 338 7.5 / 8.7 / 9.0 -> 5.8 / 7.3 / 6.7, 471 7.9 / 9.9 / 10.4 -> 5.8 / 9.1 / 7.8,
+// 502 8.4 / 8.4 / 8.2 -> 5.9 / 9.4 / 8.2, 1001 7.4 / 8.5 / 7.9 -> 8.0 / 15.0 / 12.6).
+constexpr int kShortRowSlots = 384;
 // Without the promise the block kernel may still merge the short segments of a row that
 // the list it was given holds, when there are this many of them.
 constexpr int kMergeMinSegments = 16384;

@@ -598,8 +598,8 @@ def test_overwrite_leaves_other_rows_to_the_callers_clearing():
     (5000, (0, 9), 0, 64),
     (40000, (0, 4), 0, 128),        # ... too many workgroups for one launch (fp32)
     (700, (0, 60), 0, 128),         # fewer than 1024 segments, every row short: owned by a wave each
-    (700, (0, 60), 128, 40),        # (the longest such row; a width that ends inside a tile)
-    (700, (0, 60), 129, 64),        # one row past it: cleared beforehand
+    (700, (0, 60), 384, 40),        # (the longest such row; a width that ends inside a tile)
+    (700, (0, 60), 385, 64),        # one row past it: cleared beforehand
     (3000, (0, 80), 1024, 64),      # the longest row with one owner
     (3000, (0, 80), 1025, 64),      # more than that: cleared beforehand
     (6000, (0, 70), 500, 256),      # column tiles dealt out to the XCDs
