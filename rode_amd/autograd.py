@@ -32,15 +32,14 @@ def _sddmm(csr, values, lhs, rhs):
 
 def _spmm(csr, values, dense):
     values, dense = values.contiguous(), dense.contiguous()
-    width = dense.shape[1]
     out = _lib.host_call().spmm(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
-                                csr.column_indices, values, csr.m, csr.n, dense, csr.plans_address(width),
+                                csr.column_indices, values, csr.m, csr.n, dense, csr.plans_address(),
                                 csr.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(csr.device), csr.longest_row)
     if out is not None:
         return out
     return rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2,
                                        csr.row_offsets, csr.column_indices, values, csr.m, csr.n, dense, plan=csr.plan,
-                                       plans=csr.call_plans(width, values.element_size()),
+                                       plans=csr.call_plans(),
                                        every_row_stored=csr.spmm_stores_every_row(), longest_row=csr.longest_row)
 
 

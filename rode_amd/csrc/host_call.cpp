@@ -165,11 +165,21 @@ PyObject* spmm(PyObject*, PyObject* const* args, Py_ssize_t count)
     const float* val = floats(a.val);
     const void* b = data(*dense);
     float* c = floats(out);
+    const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
+    // A hub plan's partial rows are this call's own (the allocator orders their next use on the stream): calls on one matrix
+    // may overlap on other streams, and those of other threads come between two kernels of this one.
+    rode_hip_plans own;
+    at::Tensor scratch;
+    if (p && p->hub && !p->hub_workspace) {
+        own = *p, p = &own;
+        own.hub_workspace_bytes = rode_hip_hub_workspace_bytes(own.hub_counts, (int)width, 4);
+        scratch = at::empty({(int64_t)own.hub_workspace_bytes}, a.val->options().dtype(at::kByte).requires_grad(false));
+        own.hub_workspace = data(scratch);
+    }
     int code = 0;
     const char* what = stored ? "rode_hip_spmm_planned" : "rode_hip_spmm_new";
     {
         NoGil no_gil;
-        const rode_hip_plans* p = reinterpret_cast<const rode_hip_plans*>(plans);
         void* s = reinterpret_cast<void*>(stream);
         if (stored)
             code = rode_hip_spmm_planned(kind, RODE_SPMM_WHOLE_LISTS | RODE_SPMM_OVERWRITE, (int)a.m1, (int)a.m2, (int)a.n, (int)width, val, col,

@@ -190,9 +190,9 @@ class RoDeCSR:
         return plan if plan.usable else None
 
     def call_plans(self, spmm_width=None, spmm_elem_bytes=4):
-        """The ``rode_hip_plans`` struct of this matrix for an SDDMM call (no arguments) or an
-        SpMM call of the given dense width and output element size; built once per pattern
-        and kind of call (the plan and the segment length never change after construction)."""
+        """The ``rode_hip_plans`` struct of this matrix, built once per pattern (the plan and the segment length never
+        change after construction).  With a dense width and output element size, a hub plan's struct has the workspace that the
+        plan keeps for them (``HubPlan.workspace``: one SpMM call at a time)."""
         key = ("plans", spmm_width, spmm_elem_bytes)
         plans = self._shared.get(key)
         if plans is None:
@@ -204,7 +204,7 @@ class RoDeCSR:
 
     def plans_address(self, spmm_width=None):
         """The struct of ``call_plans`` as the native calls take it: a ``PlansAddress``, which holds
-        the struct.  Only a hub plan's struct depends on the width (it carries the workspace)."""
+        the struct.  Only a hub plan's struct depends on the width."""
         key = "plans_address"
         if spmm_width is not None:
             if isinstance(self.plan, rode_sddmm_hip.HubPlan):

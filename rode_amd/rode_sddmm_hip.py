@@ -214,8 +214,9 @@ class HubPlan:
 
     def workspace(self, n, elem_bytes):
         """Scratch for the SpMM hub kernels at dense width ``n`` (one partial row of C per
-        hub row and slab); kept for the next call.  Calls that overlap in time on different
-        streams must not share it."""
+        hub row and slab group), kept: for a caller of the C ABI with one call at a time.  The
+        calls here (``spmm_forward``, ``rode_spmm``) allocate theirs anew, since calls on one matrix may overlap on
+        other streams or come from other threads."""
         key = (n, elem_bytes)
         ws = self._workspaces.get(key)
         if ws is None:
@@ -310,8 +311,8 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
                  nonzeros=0):
     """The ``rode_hip_plans`` struct of one call (keep it alive until the call returns; pass
     it with ``ctypes.byref``).  ``plan``: a ``WindowPlan``, a ``HubPlan``, a ``GroupPlan`` or None.
-    ``spmm_width``: for an SpMM call the dense width, so that a hub plan's workspace is
-    attached; a hub plan is left out of an SpMM call without the whole-lists promise.
+    ``spmm_width``: the dense width of SpMM calls that share the hub plan's kept workspace (None: none is
+    attached).  ``whole_lists``: without that promise a hub or group plan is left out.
     ``seg_length``: the segment length the lists were made with, 0 when not known.
     ``columns_local``: the columns of neighbouring rows are known to lie close together.
     ``nonzeros``: of the matrix, 0 when not known."""
@@ -320,10 +321,10 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
     p.nonzeros = int(nonzeros)
     p.seg_length = int(seg_length or 0)  # (the segment length of the decomposition, when the caller knows it)
     if isinstance(plan, GroupPlan):
-        if plan.usable and (spmm_width is None or whole_lists):
+        if plan.usable and whole_lists:
             p.groups, p.group_counts = plan.data.data_ptr(), ctypes.addressof(plan._header)
     elif isinstance(plan, HubPlan):
-        if plan.usable and (spmm_width is None or whole_lists):
+        if plan.usable and whole_lists:
             p.hub, p.hub_counts = plan.data.data_ptr(), ctypes.addressof(plan._header)
             if spmm_width is not None:
                 ws = plan.workspace(spmm_width, spmm_elem_bytes)
@@ -334,6 +335,18 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
         p.nonzeros = plan.nonzeros
         p.columns_local = int(columns_local or 2 * plan.windowed > plan.counts[0])
     return p
+
+
+def _with_scratch(plans, n, elem_bytes, device):
+    """``(plans, scratch)`` of one SpMM call of dense width ``n``: the struct of a hub plan without a workspace as a copy
+    with partial rows of the call's own, which the caller holds until everything is queued."""
+    if not plans.hub or plans.hub_workspace:
+        return plans, None
+    nbytes = _lib.load().rode_hip_hub_workspace_bytes(plans.hub_counts, n, elem_bytes)
+    scratch = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    plans = _lib.Plans.from_buffer_copy(plans)
+    plans.hub_workspace, plans.hub_workspace_bytes = scratch.data_ptr(), nbytes
+    return plans, scratch
 
 
 class PlansAddress(int):
@@ -433,7 +446,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     complete decomposition (always true for a ``RoDeCSR``); pass False for a slice.
     ``plan``: a ``WindowPlan`` made from these very lists, a ``HubPlan`` of this pattern
     (used only with ``whole_lists``), or None.  ``checked_lists`` / ``plans``: as for
-    ``sddmm_forward`` (``plans``: of (plan, this width and element size, whole_lists, seg_length)).
+    ``sddmm_forward`` (``plans``: of (plan, whole_lists, seg_length), with or without a hub plan's workspace).
     ``every_row_stored``: with ``out`` None and ``whole_lists``, the caller has checked
     (``rode_hip_spmm_overwrite_limit``) that every row of the matrix has slots and a single
     work item: the kernels then store their rows (``RODE_SPMM_OVERWRITE``) and nothing is cleared.
@@ -460,7 +473,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     _check(n > 0 and n % vec == 0, f"dense_matrix cols must be a positive multiple of {vec}")
     lib = _lib.load()
     if plans is None:
-        plans = plans_struct(plan, n, values.element_size(), whole_lists, seg_length=seg_length)
+        plans = plans_struct(plan, whole_lists=whole_lists, seg_length=seg_length)
     overwrite = out is None and whole_lists  # (a caller's C is added to, as the kernels' contract says)
     if out is None:
         if m1 == 0 and m2 == 0:
@@ -481,6 +494,7 @@ def spmm_forward(block_indices, residue_indices, st_offsets, m1, m2, row_offsets
     if m1 == 0 and m2 == 0:
         return out
     _check_data(values, "values")
+    plans, scratch = _with_scratch(plans, n, values.element_size(), values.device)  # (scratch: held to the end)
     dtype = {torch.float32: 0, torch.float16: 1, torch.float64: 2}[dense_matrix.dtype]  # RODE_DENSE_*
     with _on_device(values.device):
         s = _stream_handle(values.device)

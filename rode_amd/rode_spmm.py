@@ -13,11 +13,10 @@ def rode_spmm(sparse_matrix, dense, out=None, values=None):
     and values when ``out`` is not given."""
     if values is None and out is None and sparse_matrix.config["k_block"] == 32 and sparse_matrix.config["vec_len"] == 4:
         # the ordinary call, natively; None for everything that needs (or refuses) more
-        hub = isinstance(sparse_matrix.plan, rode_sddmm_hip.HubPlan)
         c = _lib.host_call().spmm(
             sparse_matrix.block_indices, sparse_matrix.residue_indices, sparse_matrix.st_offsets, sparse_matrix.m1,
             sparse_matrix.m2, sparse_matrix.row_offsets, sparse_matrix.column_indices, sparse_matrix.values,
-            sparse_matrix.m, sparse_matrix.n, dense, sparse_matrix.plans_address(dense.shape[1] if hub and dense.dim() == 2 else None),
+            sparse_matrix.m, sparse_matrix.n, dense, sparse_matrix.plans_address(),
             sparse_matrix.spmm_stores_every_row(), rode_sddmm_hip._stream_handle(sparse_matrix.device), sparse_matrix.longest_row)
         if c is not None:
             return c
@@ -42,5 +41,5 @@ def rode_spmm(sparse_matrix, dense, out=None, values=None):
         sparse_matrix.m1, sparse_matrix.m2, sparse_matrix.row_offsets, sparse_matrix.column_indices,
         sparse_matrix.values, sparse_matrix.m, sparse_matrix.n, dense.contiguous(), out, plan=sparse_matrix.plan,
         seg_length=sparse_matrix.config["seg_length"], checked_lists=True,
-        plans=sparse_matrix.call_plans(dense.shape[1], 4),
+        plans=sparse_matrix.call_plans(),
         every_row_stored=out is None and sparse_matrix.spmm_stores_every_row(), longest_row=sparse_matrix.longest_row)

@@ -199,3 +199,44 @@ def test_pieces_shared_by_waves(hubs, k, half):
     ref, scale = oracle.sddmm_f64(rp, col, val, Lq, Bq, with_abs=True)
     err, cond = sddmm_row_l1_errors(run_sddmm(csr, L, B, half), ref, scale, rp)
     assert float(err[cond <= 100].max(initial=0.0)) <= tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64])
+def test_calls_on_one_matrix_from_two_streams(dtype):
+    """Overlapping products of one matrix have partial rows of their own: every result is the one that the call gives alone.
+    (Rows of the plan are summed in one order whatever else runs, so the bits are equal.)"""
+    from gpu_common import DEV, make_csr
+    from rode_amd import RoDeCSR, rode_sddmm_hip, rode_spmm
+    rng = np.random.default_rng(17)
+    m, n, k = 3000, 70000, 128
+    lens = rng.integers(600, 900, 400)
+    lens[:2] = 30000, 7000
+    rp, col, val, where = _matrix(rng, m, n, lens)
+    old = RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
+    RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = 1, 0.0
+    try:
+        csr = make_csr(rp, col, val, m, n, k)
+    finally:
+        RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = old
+    assert csr.plan.usable and csr.plan.counts[0] == len(where)
+    where = torch.from_numpy(where).to(DEV)
+    operands = [torch.from_numpy(rng.standard_normal((n, k))).to(DEV, dtype) for _ in range(2)]
+
+    def product(B):
+        if dtype == torch.float64:
+            return rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets,
+                                               csr.column_indices, csr.values.double(), m, n, B, plan=csr.plan)
+        return rode_spmm(csr, B)
+
+    alone = [product(B)[where] for B in operands]
+    streams = [torch.cuda.Stream() for _ in operands]
+    torch.cuda.synchronize()
+    got = [[], []]
+    for _ in range(8):
+        for i, (s, B) in enumerate(zip(streams, operands)):
+            with torch.cuda.stream(s):
+                got[i].append(product(B)[where])
+    torch.cuda.synchronize()
+    assert not torch.equal(*alone)
+    assert all(torch.equal(a, alone[i]) for i in range(2) for a in got[i])
+    assert csr.plan._workspaces == {}  # nothing that two calls could share is kept
