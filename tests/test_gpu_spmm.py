@@ -639,3 +639,42 @@ def test_product_into_memory_that_holds_anything(rows, lengths, longest, k, dtyp
         assert bool(((out.double() - want).abs() <= bound).all())
     if dtype != "f64":
         assert bool(((rode_spmm(csr, B).double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", ["f32", "f16", "f64"])
+@pytest.mark.parametrize("rows,filled,length,k", [
+    (1, [], 5, 32), (1, [0], 5, 32), (63, [62], 5, 64), (64, [0], 40, 128), (65, [64], 5, 128), (257, [3, 256], 40, 40),
+    (1000, [0, 63, 64, 127, 128, 999], 200, 96), (70000, [5, 69999], 8, 32), (70000, [5, 69999], 40, 200),
+])
+def test_product_of_mostly_empty_rows(rows, filled, length, k, dtype):
+    """A C of which nearly every row is one that no work item has: exactly zero there, the products in the others."""
+    from gpu_common import DEV
+    from rode_amd import RoDeCSR, _lib
+    rng = np.random.default_rng(rows + k)
+    lens = np.zeros(rows, dtype=np.int64)
+    lens[filled] = length
+    lens[filled[-1:]] += -lens.sum() % 4  # (a row without nonzeros after a ragged end has slots: here none does)
+    lens[filled] += -lens[filled] % 4
+    cols = 300
+    row_ptr = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(cols, n, replace=False)) for n in lens[filled]] or [np.zeros(0)]).astype(np.int32)
+    val = torch.from_numpy(rng.uniform(-1, 1, len(col))).to(torch.float64 if dtype == "f64" else torch.float32)
+    dense = torch.from_numpy(rng.standard_normal((cols, k))).to(torch.float16 if dtype == "f16" else val.dtype)
+    csr = RoDeCSR(torch.from_numpy(row_ptr), torch.from_numpy(col), val.float(), DEV, rows, cols, 32, config="auto")
+    val, B = val.to(DEV), dense.to(DEV)
+    code, lib = {"f32": 0, "f16": 1, "f64": 2}[dtype], _lib.load()
+    for longest in (csr.longest_row, 0):
+        out = torch.full((rows, k), float("nan"), dtype=val.dtype, device=DEV)
+        assert lib.rode_hip_spmm_new(code, rows, longest, csr.m1, csr.m2, cols, k, val.data_ptr(), csr.column_indices.data_ptr(),
+                                     csr.row_offsets.data_ptr(), csr.block_indices.data_ptr(), csr.residue_indices.data_ptr(),
+                                     csr.st_offsets.data_ptr(), B.data_ptr(), out.data_ptr(), ctypes.addressof(csr.call_plans()),
+                                     torch.cuda.current_stream().cuda_stream) == 0
+        want = torch.zeros(rows, k, dtype=torch.float64)
+        for r in filled:
+            want[r] = val.cpu().double()[row_ptr[r]:row_ptr[r + 1]] @ dense.double()[col[row_ptr[r]:row_ptr[r + 1]].astype(np.int64)]
+        got = out.cpu().double()
+        # (a sum of up to 204 products of at most 5: (n + 2) roundings of the sum of their magnitudes)
+        assert (got - want).abs().max() <= 206 * 204 * 5 * (2.0 ** -52 if dtype == "f64" else 2.0 ** -24)
+        empty = torch.ones(rows, dtype=torch.bool)
+        empty[filled] = False
+        assert bool((got[empty] == 0).all())
