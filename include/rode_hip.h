@@ -217,11 +217,13 @@ int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_
  *   dense_rows   rows of the dense operand (columns of the sparse matrix)
  *   min_len      >= RODE_HIP_HUB_MIN_LEN; 512 and dense_rows / 512 (8 nonzeros per 4096 columns) are sensible lower
  *                bounds (power-law matrices of 200 K to 2 M columns: half of that loses, the rows of
- *                eight times that should hold a tenth of the nonzeros for the plan to pay)
+ *                eight times that should hold a tenth of the nonzeros for the plan to pay).  A call takes all of these rows or,
+ *                where its dense rows are so wide that the pieces would be too short, those of 4096 slots and more
  *   d_plan       rode_hip_hub_plan_bytes(M, dense_rows, nnz, min_len) bytes, 16-byte aligned, out
  *   h_counts     HOST int[8], out (the call waits for its two kernels): [0] hub rows,
  *                [1] slabs, [2] min_len, [3] 1 if the plan is usable - every hub row's column
- *                indices ascend and lie inside the operand - else 0, [4] room for hub rows;
+ *                indices ascend and lie inside the operand - else 0, [4] room for hub rows, [5] hub rows of
+ *                4096 slots and more, [6] and [7] nonzeros of all hub rows and of those;
  *                the *_planned entry points need it and ignore a plan with [3] == 0 or [0] == 0
  * A hub plan belongs to the pattern it was made from, and excludes a locality plan: the
  * *_planned entry points refuse to take both.

@@ -182,9 +182,7 @@ size_t rode_hip_hub_workspace_bytes(const int* h_hub_counts, int n, int elem_byt
 {
     if (!h_hub_counts || n <= 0 || (elem_bytes != 4 && elem_bytes != 8) || h_hub_counts[0] <= 0 || h_hub_counts[1] <= 0)
         return 0;
-    // (an operand of halves has pieces twice as long)
-    const int merge = rode::hub_merge((size_t)n * elem_bytes, h_hub_counts[1]);
-    return (size_t)h_hub_counts[0] * rode::hub_groups(h_hub_counts[1], merge) * n * elem_bytes;
+    return rode::spmm_hub_partial_rows(h_hub_counts, n, elem_bytes) * n * elem_bytes;
 }
 
 size_t rode_hip_group_plan_bytes(int M) { return M < 0 ? 0 : rode::group_plan_ints(M) * sizeof(int); }
@@ -225,7 +223,7 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
         // kernels do not know which rows the hub kernels have taken)
         if (!p->hub_counts || !aligned16(p->hub) || window) return false;
         if (p->hub_counts[0] < 0 || p->hub_counts[0] > p->hub_counts[4] || p->hub_counts[1] < 0 ||
-            p->hub_counts[2] < RODE_HIP_HUB_MIN_LEN)
+            p->hub_counts[2] < RODE_HIP_HUB_MIN_LEN || p->hub_counts[5] < 0 || p->hub_counts[5] > p->hub_counts[0])
             return false;
         plan.hub = static_cast<const int*>(p->hub);
         plan.hub_counts = p->hub_counts;

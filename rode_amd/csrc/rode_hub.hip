@@ -5,9 +5,9 @@
 // RoDe_SDDMM/RoDeSddmm.cu:96-140).  The plan changes no result.
 //
 //   hub_count_kernel, hub_scan_kernel, hub_write_kernel
-//                      the hub rows, in ascending order: counted per block of 2048 rows, a
-//                      prefix sum over the blocks (one workgroup; it also fills in the
-//                      header), then every block writes its hub rows to its place.
+//                      the hub rows, and which of them are long (kHubLongSlots), in ascending order: counted
+//                      per block of 2048 rows, a prefix sum over the blocks (one workgroup; it also fills in the
+//                      header), then every block writes its hub rows to their places.
 //   hub_pieces_kernel  one workgroup per hub row: a binary search per slab boundary in the
 //                      row's column indices, and a pass over the row that checks that its
 //                      columns ascend (if one does not, the plan is marked unusable).
@@ -20,10 +20,12 @@ namespace {
 
 constexpr int kSelectThreads = 1024;
 
-__device__ __forceinline__ bool is_hub(const int* __restrict__ row_ptr, int row, int min_len)
+// Hub rows and, in the upper half, long ones among them.
+typedef unsigned long long HubCount;
+__device__ __forceinline__ HubCount hub_count_of(const int* __restrict__ row_ptr, int row, int min_len)
 {
-    const int s = row_ptr[row];
-    return row_ptr[row + 1] - s + (s & (kVecLen - 1)) >= min_len;
+    const int s = row_ptr[row], slots = row_ptr[row + 1] - s + (s & (kVecLen - 1));
+    return slots < min_len ? 0ull : slots < kHubLongSlots ? 1ull : (1ull << 32) + 1ull;
 }
 
 // Hub rows among the rows [first, first + 256 * kSelectRows) of one workgroup, thread t
@@ -31,18 +33,18 @@ __device__ __forceinline__ bool is_hub(const int* __restrict__ row_ptr, int row,
 constexpr int kSelectRows = kHubSelectBlockRows / kWgThreads;
 
 __global__ void __launch_bounds__(kWgThreads)
-hub_count_kernel(int M, int min_len, const int* __restrict__ row_ptr, int* __restrict__ block_counts)
+hub_count_kernel(int M, int min_len, const int* __restrict__ row_ptr, HubCount* __restrict__ block_counts)
 {
-    __shared__ int wave_sum[kWavesPerWg];
+    __shared__ HubCount wave_sum[kWavesPerWg];
     const int first = (blockIdx.x * kWgThreads + threadIdx.x) * kSelectRows;
-    int count = 0;
-    for (int r = first; r < min(M, first + kSelectRows); ++r) count += is_hub(row_ptr, r, min_len) ? 1 : 0;
+    HubCount count = 0;
+    for (int r = first; r < min(M, first + kSelectRows); ++r) count += hub_count_of(row_ptr, r, min_len);
 #pragma unroll
     for (int d = kWave / 2; d > 0; d >>= 1) count += __shfl_xor(count, d, kWave);
     if (threadIdx.x % kWave == 0) wave_sum[threadIdx.x / kWave] = count;
     __syncthreads();
     if (threadIdx.x == 0) {
-        int total = 0;
+        HubCount total = 0;
         for (int w = 0; w < kWavesPerWg; ++w) total += wave_sum[w];
         block_counts[blockIdx.x] = total;
     }
@@ -50,57 +52,76 @@ hub_count_kernel(int M, int min_len, const int* __restrict__ row_ptr, int* __res
 
 // One workgroup: exclusive prefix over the block counts (in place) and the header.
 __global__ void __launch_bounds__(kSelectThreads)
-hub_scan_kernel(int nblocks, int dense_rows, int room, int min_len, int* __restrict__ block_counts, int* __restrict__ plan)
+hub_scan_kernel(int nblocks, int dense_rows, int room, int min_len, HubCount* __restrict__ block_counts, int* __restrict__ plan)
 {
-    __shared__ int partial[kSelectThreads];
+    __shared__ HubCount partial[kSelectThreads];
     const int per = (nblocks + kSelectThreads - 1) / kSelectThreads;
     const int lo = min(nblocks, (int)threadIdx.x * per), hi = min(nblocks, lo + per);
-    int count = 0;
+    HubCount count = 0;
     for (int i = lo; i < hi; ++i) count += block_counts[i];
     partial[threadIdx.x] = count;
     __syncthreads();
     for (int d = 1; d < kSelectThreads; d <<= 1) {
-        const int add = (int)threadIdx.x >= d ? partial[threadIdx.x - d] : 0;
+        const HubCount add = (int)threadIdx.x >= d ? partial[threadIdx.x - d] : 0;
         __syncthreads();
         partial[threadIdx.x] += add;
         __syncthreads();
     }
-    int run = partial[threadIdx.x] - count;
+    HubCount run = partial[threadIdx.x] - count;
     for (int i = lo; i < hi; ++i) {
-        const int c = block_counts[i];
+        const HubCount c = block_counts[i];
         block_counts[i] = run;
         run += c;
     }
     if (threadIdx.x == kSelectThreads - 1) {
-        const int total = partial[kSelectThreads - 1];
+        const int total = (int)(unsigned)partial[kSelectThreads - 1];
         plan[0] = min(total, room);
         plan[1] = hub_slabs(dense_rows);
         plan[2] = min_len;
         plan[3] = total <= room ? 1 : 0; // (room = hub_room(nnz, min_len) always suffices)
         plan[4] = room;
-        plan[5] = plan[6] = plan[7] = 0;
+        plan[5] = (int)(partial[kSelectThreads - 1] >> 32);
+        plan[6] = plan[7] = 0; // (hub_write_kernel adds them up)
     }
 }
 
 __global__ void __launch_bounds__(kWgThreads)
-hub_write_kernel(int M, int room, int min_len, const int* __restrict__ row_ptr, const int* __restrict__ block_starts,
+hub_write_kernel(int M, int room, int min_len, const int* __restrict__ row_ptr, const HubCount* __restrict__ block_starts,
                  int* __restrict__ plan)
 {
-    __shared__ int thread_count[kWgThreads];
+    __shared__ HubCount thread_count[kWgThreads];
     const int first = (blockIdx.x * kWgThreads + threadIdx.x) * kSelectRows;
-    int count = 0;
-    for (int r = first; r < min(M, first + kSelectRows); ++r) count += is_hub(row_ptr, r, min_len) ? 1 : 0;
+    HubCount count = 0;
+    int nonzeros = 0, in_long = 0;
+    for (int r = first; r < min(M, first + kSelectRows); ++r) {
+        const HubCount c = hub_count_of(row_ptr, r, min_len);
+        count += c;
+        if (c != 0) nonzeros += row_ptr[r + 1] - row_ptr[r];
+        if (c > 1) in_long += row_ptr[r + 1] - row_ptr[r];
+    }
+    if (__any(count != 0)) {
+#pragma unroll
+        for (int d = kWave / 2; d > 0; d >>= 1) nonzeros += __shfl_xor(nonzeros, d, kWave), in_long += __shfl_xor(in_long, d, kWave);
+        if (threadIdx.x % kWave == 0) {
+            atomicAdd(plan + 6, nonzeros);
+            if (in_long > 0) atomicAdd(plan + 7, in_long);
+        }
+    }
     thread_count[threadIdx.x] = count;
     __syncthreads();
     if (count == 0) return;
-    int at = block_starts[blockIdx.x];
+    HubCount at = block_starts[blockIdx.x];
     for (int t = 0; t < (int)threadIdx.x; ++t) at += thread_count[t]; // (hub rows are few: hardly any thread gets here)
     int* rows = plan + kHubHeaderInts;
-    for (int r = first; r < min(M, first + kSelectRows); ++r)
-        if (is_hub(row_ptr, r, min_len)) {
-            if (at < room) rows[at] = r;
-            ++at;
+    int* longs = rows + room + (size_t)room * (plan[1] + 1);
+    for (int r = first; r < min(M, first + kSelectRows); ++r) {
+        const HubCount c = hub_count_of(row_ptr, r, min_len);
+        if (c != 0 && (int)(unsigned)at < room) {
+            rows[(unsigned)at] = r;
+            if (c > 1) longs[at >> 32] = (int)(unsigned)at;
         }
+        at += c;
+    }
 }
 
 __global__ void __launch_bounds__(kWgThreads)
@@ -136,7 +157,7 @@ hipError_t hub_plan_launch(int M, int dense_rows, int nnz, int min_len, const in
 {
     const int room = hub_room(nnz, min_len);
     const int nblocks = (M + kHubSelectBlockRows - 1) / kHubSelectBlockRows;
-    int* block_counts = plan + hub_table_ints(dense_rows, nnz, min_len); // scratch behind the tables
+    HubCount* block_counts = reinterpret_cast<HubCount*>(plan + hub_table_ints(dense_rows, nnz, min_len)); // scratch behind the tables
     hub_count_kernel<<<max(nblocks, 1), kWgThreads, 0, stream>>>(M, min_len, row_ptr, block_counts);
     hub_scan_kernel<<<1, kSelectThreads, 0, stream>>>(nblocks, dense_rows, room, min_len, block_counts, plan);
     hub_write_kernel<<<max(nblocks, 1), kWgThreads, 0, stream>>>(M, room, min_len, row_ptr, block_counts, plan);

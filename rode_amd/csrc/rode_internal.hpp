@@ -163,6 +163,7 @@ hipError_t window_plan_rows_launch(int m2, const int* residue_rows, const int* r
 
 // (rode_spmm.hip) which rows an SpMM call under kSpmmOverwrite stores instead of adding to
 int spmm_overwrite_limit(int m1, bool hub_plan);
+size_t spmm_hub_partial_rows(const int* hub_counts, int n, int acc_bytes);
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,

@@ -459,44 +459,81 @@ inline const RowTile* group_plan_tiles(const int* plan, int M) { return reinterp
 // the operand, and so does every other hub: the same dense rows, at other times, long
 // evicted from L2.  A hub plan cuts every hub row into pieces by column slab (a slab is
 // kHubSlabRows consecutive dense rows) and the hub kernels take the pieces slab by slab,
-// a few neighbouring slabs at a time (hub_merge: 2 or 4 MB of the dense operand): all hub rows' nonzeros of those
+// a few neighbouring slabs at a time (hub_rows_of_call: 2 or 4 MB of the dense operand): all hub rows' nonzeros of those
 // slabs at the same time on one XCD, so that a dense row is fetched from memory once and
 // then found in L2 by the other hubs.
 // Needs rows whose column indices ascend (the plan checks).  The standard kernels skip
 // the rows of a usable plan (by their length), so every nonzero is still processed once.
 // Layout, ints: header [0] hub rows  [1] slabs  [2] shortest hub row (aligned length)
-// [3] usable (every hub row's columns ascend)  [4] room for hub rows  [5..7] zero;
+// [3] usable (every hub row's columns ascend)  [4] room for hub rows  [5] how many of the hub rows have kHubLongSlots aligned
+// slots or more  [6], [7] nonzeros of all hub rows and of those;
 // then the hub rows, ascending (room for [4] of them); then per hub row slabs + 1 piece
-// starts (indices into column_indices / values; the last one is the row's end).
+// starts (indices into column_indices / values; the last one is the row's end); then which of the hub rows are those of [5]
+// (room for [4] again).
 constexpr int kHubSlabRows = 2048;
 constexpr int kHubHeaderInts = 8;
+constexpr int kHubLongSlots = 4096;
 
 __host__ __device__ inline int hub_slabs(int dense_rows) { return (dense_rows + kHubSlabRows - 1) / kHubSlabRows; }
 // (a hub row has at least min_len aligned slots, up to three of which belong to the row before it)
 __host__ __device__ inline int hub_room(int nnz, int min_len) { return min_len > kVecLen ? nnz / (min_len - (kVecLen - 1)) + 1 : 0; }
-// (after the piece table: one int per 2048 rows of the matrix, scratch of the selection)
+// (after the piece table: two ints per 2048 rows of the matrix, scratch of the selection)
 constexpr int kHubSelectBlockRows = 2048;
 __host__ __device__ inline size_t hub_table_ints(int dense_rows, int nnz, int min_len)
 {
-    const size_t room = hub_room(nnz, min_len);
-    return kHubHeaderInts + room + room * (hub_slabs(dense_rows) + 1);
+    const size_t room = hub_room(nnz, min_len), ints = kHubHeaderInts + room + room * (hub_slabs(dense_rows) + 1) + room;
+    return (ints + 1) / 2 * 2;
 }
 __host__ __device__ inline size_t hub_plan_ints(int M, int dense_rows, int nnz, int min_len)
 {
-    return hub_table_ints(dense_rows, nnz, min_len) + (M + kHubSelectBlockRows - 1) / kHubSelectBlockRows + 1;
+    return hub_table_ints(dense_rows, nnz, min_len) + 2 * ((M + kHubSelectBlockRows - 1) / kHubSelectBlockRows + 1);
 }
 
-// Slabs taken together by the work items of the hub kernels, for dense rows of so many bytes: 4 MB of the operand, the size of an XCD's L2;
-// 2 MB of one of up to 320 MB, whose pieces are long enough (us, SDDMM / SpMM with its reduction at 2 -> 4 MB: 2 M x 128 727 / 653 -> 551 / 551,
-// halves 296 / 388 -> 300 / 317; 2 M x 32 162 / 155 -> 174 / 159, 2 M x 64 halves 164 / 169 -> 174 / 165, 1 M x 64 136 / 153 -> 152 / 156,
-// 500 K x 64 114 / 122 -> 129 / 132, 200 K x 32 38 / 41 -> 52 / 61).
-__host__ __device__ inline int hub_merge(size_t row_bytes, int slabs)
+__host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs + merge - 1) / merge; }
+
+// What a call takes of a hub plan: `rows` of its rows (all, or the long ones), and how many slabs together.  A piece should hold
+// enough nonzeros that reading its columns, its last step of 64 and, in SpMM, its partial row are little beside its dense rows,
+// and enough rows should share a slab.  Counted in nonzeros of a row per piece (in brackets) at 4 MB of the operand, an XCD's L2:
+//   * all rows from 18 on, in SDDMM with a width that is no multiple of its slabs from 28 on, else the long ones.  us, long ones -> all,
+//     power law (p) or 8 nonzeros a row and thousands of rows of 512 to 2000 (s), dense rows x width of SDDMM: p 200 K x 256 659 -> 627 (49),
+//     p 330 K x 512 2173 -> 2264 (18), s 262 K x 256 3393 -> 2477 (23), x 512 6864 -> 8511 (12), s 500 K x 128 1957 -> 1526 (32), x 256 3953 -> 4149 (16);
+//     no multiple: s 262 K x 160 2459 -> 2313 (35), x 192 2775 -> 2994 (23), s 100 K x 320 3914 -> 2935 (29), s 500 K x 160 3007 -> 3870 (25);
+//   * in SpMM also only with 600 rows: 314 of p 70 K x 64 67 -> 79, 412 of p 100 K x 128 halves 105 -> 108, x 320 halves 227 -> 254,
+//     928 of p 200 K x 128 361 -> 325, 2100 of s 100 K x 64 136 -> 109;
+//   * 2 MB instead of 4 in operands of up to 320 MB with (40) at that.  SDDMM / SpMM, 2 -> 4 MB: p 200 K x 32 95 / 112 -> 105 / 117 (185),
+//     x 128 310 / 325 -> 323 / 345 (49), p 330 K x 128 496 / 512 -> 490 / 507 (36), s 262 K x 64 517 / 601 -> 482 / 499 (47), x 128 1310 / 1201 -> 919 / 981 (23);
+//   * SpMM counts the bytes of the column tile that a grid row works on, as long as that leaves 2048 pieces: s 180 K x 512 2827 -> 2024,
+//     halves 2436 -> 1182.
+// With every row, and 2 MB up to 320 MB, wide calls were slower than with the long rows alone: SDDMM s 262 K x 160 2435 -> 4797, x 512 6864 -> 8443, SpMM
+// s 262 K x 512 halves 3494 -> 6179, s 500 K x 1024 halves 8684 -> 17715.
+struct HubRows {
+    int rows = 0, min_len = 0; // 0: the call goes without the plan
+    int merge = 1;
+    bool longs = false;
+};
+inline int hub_merge(size_t row_bytes, int mb)
 {
-    const size_t whole = row_bytes * slabs * kHubSlabRows, at_once = (size_t)(whole <= ((size_t)320 << 20) ? 2 : 4) << 20;
-    const size_t g = at_once / kHubSlabRows / (row_bytes > 0 ? row_bytes : 4);
+    const size_t g = ((size_t)mb << 20) / kHubSlabRows / (row_bytes > 0 ? row_bytes : 4);
     return g < 1 ? 1 : (g > 64 ? 64 : (int)g);
 }
-__host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs + merge - 1) / merge; }
+inline HubRows hub_rows_of_call(const int* counts, size_t row_bytes, size_t tile_bytes, int tiles, int pieces_min, int rows_min)
+{
+    const int slabs = counts[1], min_len = counts[2];
+    // (a header of before those counts: every row as short as the plan allows)
+    auto mean = [&](int rows, int nonzeros) { return rows > 0 && nonzeros > 0 ? nonzeros / rows : min_len; };
+    const bool all = counts[0] >= rows_min && mean(counts[0], counts[6]) >= pieces_min * hub_groups(slabs, hub_merge(tile_bytes, 4));
+    HubRows use;
+    use.rows = all ? counts[0] : counts[5];
+    if (use.rows <= 0) return use;
+    use.min_len = all || min_len > kHubLongSlots ? min_len : kHubLongSlots;
+    use.longs = !all;
+    const int length = all ? mean(counts[0], counts[6]) : mean(counts[5], counts[7]);
+    const bool small = tile_bytes * slabs * kHubSlabRows <= ((size_t)320 << 20) && length >= 40 * hub_groups(slabs, hub_merge(tile_bytes, 2));
+    const int most = hub_merge(tile_bytes, small ? 2 : 4);
+    use.merge = hub_merge(row_bytes, small ? 2 : 4);
+    while (2 * use.merge <= most && (long long)use.rows * hub_groups(slabs, 2 * use.merge) * tiles >= 2048) use.merge *= 2;
+    return use;
+}
 
 // Is this row in a tile that the tile kernels have (owners.tiles)?
 __device__ __forceinline__ bool in_tile(const RowOwners& o, int row)
@@ -505,18 +542,18 @@ __device__ __forceinline__ bool in_tile(const RowOwners& o, int row)
 }
 
 struct HubPlan {
-    int n_hub, slabs, min_len;
-    const int* rows;   // [n_hub]
-    const int* pieces; // [n_hub][slabs + 1]
+    int slabs;
+    const int* rows;   // [hub rows]
+    const int* pieces; // [hub rows][slabs + 1]
+    const int* longs;  // [long ones]: which of the hub rows
 };
 __device__ __forceinline__ HubPlan hub_plan_view(const int* __restrict__ plan)
 {
     HubPlan v;
-    v.n_hub = plan[0];
     v.slabs = plan[1];
-    v.min_len = plan[2];
     v.rows = plan + kHubHeaderInts;
     v.pieces = plan + kHubHeaderInts + plan[4];
+    v.longs = v.pieces + (size_t)plan[4] * (v.slabs + 1);
     return v;
 }
 
@@ -534,11 +571,14 @@ constexpr int kHubWavesMax = 8, kHubPiecesMax = 8;
 struct HubGrid {
     int wgs;           // workgroups, a multiple of kXcds for xcd_logical_block; -1: more than a launch holds
     int waves, pieces; // of a workgroup
+    int rows, merge;   // rows of the plan, slabs taken together
+    bool longs;        // ... its long rows
 };
-inline HubGrid hub_grid(const int* counts, int merge)
+inline HubGrid hub_grid(const HubRows& use, int slabs)
 {
-    const long long items = (long long)counts[0] * hub_groups(counts[1], merge);
+    const long long items = (long long)use.rows * hub_groups(slabs, use.merge);
     HubGrid g;
+    g.rows = use.rows, g.merge = use.merge, g.longs = use.longs;
     g.waves = items >= 20000 ? 4 : kHubWavesMax;
     g.pieces = items >= 80000 ? kHubPiecesMax : items >= 40000 ? 4 : items >= 5000 ? 2 : 1;
     const long long wgs = (items + g.pieces * kXcds - 1) / (g.pieces * kXcds) * kXcds;
@@ -551,14 +591,16 @@ struct HubShare {
     unsigned long long pieces;         // bit i: some of them are piece i's
 };
 __device__ __forceinline__ int hub_first_step(const HubGrid& grid, int total, int wave) { return (int)((long long)total * wave / grid.waves); }
-__device__ __forceinline__ HubShare hub_share(const HubPlan& hp, int merge, const HubGrid& grid, int wg, int wave, int lane, int& total)
+__device__ __forceinline__ HubShare hub_share(const HubPlan& hp, const HubGrid& grid, int wg, int wave, int lane, int& total)
 {
     HubShare s;
-    const long long items = (long long)hp.n_hub * hub_groups(hp.slabs, merge), item = (long long)wg * grid.pieces + lane;
+    const int merge = grid.merge;
+    const long long items = (long long)grid.rows * hub_groups(hp.slabs, merge), item = (long long)wg * grid.pieces + lane;
     s.row = s.base = s.cnt = 0;
     if (lane < grid.pieces && item < items) {
-        const int h = items <= INT32_MAX ? (int)item % hp.n_hub : (int)(item % hp.n_hub);
-        const int slab = (items <= INT32_MAX ? (int)item / hp.n_hub : (int)(item / hp.n_hub)) * merge;
+        int h = items <= INT32_MAX ? (int)item % grid.rows : (int)(item % grid.rows);
+        if (grid.longs) h = hp.longs[h];
+        const int slab = (items <= INT32_MAX ? (int)item / grid.rows : (int)(item / grid.rows)) * merge;
         const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
         s.row = hp.rows[h];
         s.base = piece[slab];

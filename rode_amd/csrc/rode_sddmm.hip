@@ -426,13 +426,13 @@ sddmm_group_kernel(int k, int n_groups, const RowGroup* __restrict__ groups, con
 // one slab of rhs are worked on at the same time on one XCD and find rhs's rows in its L2.
 template <typename T, int KT, int NS, bool EDGE>
 __global__ void __launch_bounds__(kHubWavesMax * kWave)
-sddmm_hub_kernel(int k, int merge, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col, const float* __restrict__ val,
+sddmm_hub_kernel(int k, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col, const float* __restrict__ val,
                  const T* __restrict__ lhs, const T* __restrict__ rhs, float* __restrict__ out)
 {
     __shared__ __attribute__((aligned(16))) int lds[kHubWavesMax * kWave];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave; // (uniform: scalar registers)
     int total;
-    const HubShare share = hub_share(hub_plan_view(hub), merge, grid, xcd_logical_block(blockIdx.x, gridDim.x), wave, lane, total);
+    const HubShare share = hub_share(hub_plan_view(hub), grid, xcd_logical_block(blockIdx.x, gridDim.x), wave, lane, total);
     for (unsigned long long todo = share.pieces; todo; todo &= todo - 1ull) {
         const HubPart p = hub_part(share, __builtin_ctzll(todo));
         sddmm_row_slots<T, KT, NS, EDGE, true>(p.row, p.base, 0, p.cnt, p.cnt, 0, k, lane, lds + wave * kWave, col, val, lhs, rhs, out);
@@ -469,11 +469,14 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
         standard_residue = plan.host_counts[1] < plan.host_counts[0];
         window_residue = plan.host_counts[1] > 0;
     }
-    const bool hub_plan = plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 && plan.hub_counts[0] > 0;
+    HubRows hub_rows;
+    if (plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 && plan.hub_counts[0] > 0)
+        hub_rows = hub_rows_of_call(plan.hub_counts, (size_t)k * sizeof(T), (size_t)k * sizeof(T), 1, EDGE ? 28 : 18, 1);
+    const bool hub_plan = hub_rows.rows > 0;
     // (the group kernel keeps four lhs slices in registers: rows of one slab only)
     const bool group_plan = NS == 1 && plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] > 0;
     RowOwners owners;
-    owners.hub_min_len = hub_plan ? plan.hub_counts[2] : 0;
+    owners.hub_min_len = hub_rows.min_len;
     if (group_plan) {
         owners.groups = reinterpret_cast<const RowGroup*>(plan.groups + kGroupHeaderInts);
         owners.n_groups = plan.group_counts[0];
@@ -503,10 +506,9 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && hubs) {
-        const int merge = hub_merge((size_t)k * sizeof(T), plan.hub_counts[1]);
-        const HubGrid hub_wgs = hub_grid(plan.hub_counts, merge);
+        const HubGrid hub_wgs = hub_grid(hub_rows, plan.hub_counts[1]);
         if (hub_wgs.wgs < 0) return hipErrorInvalidConfiguration;
-        sddmm_hub_kernel<T, KT, NS, EDGE><<<hub_wgs.wgs, hub_wgs.waves * kWave, 0, s1>>>(k, merge, hub_wgs, plan.hub, col, val, lhs, rhs, out);
+        sddmm_hub_kernel<T, KT, NS, EDGE><<<hub_wgs.wgs, hub_wgs.waves * kWave, 0, s1>>>(k, hub_wgs, plan.hub, col, val, lhs, rhs, out);
         e = hipGetLastError();
     }
     if constexpr (NS == 1) {

@@ -664,7 +664,7 @@ spmm_group_kernel(int n, int n_groups, const RowGroup* __restrict__ groups, cons
 // A piece that waves share is finished by the wave that has its first step.
 template <typename T, int TN, bool EDGE>
 __global__ void __launch_bounds__(kHubWavesMax * kWave)
-spmm_hub_kernel(int n, int merge, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col,
+spmm_hub_kernel(int n, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col,
                 const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
                 typename DenseVec<T>::Acc* __restrict__ C, typename DenseVec<T>::Acc* __restrict__ partial)
 {
@@ -678,7 +678,7 @@ spmm_hub_kernel(int n, int merge, HubGrid grid, const int* __restrict__ hub, con
     const HubPlan hp = hub_plan_view(hub);
     const int wg = xcd_logical_block(blockIdx.x, gridDim.x);
     int steps;
-    const HubShare share = hub_share(hp, merge, grid, wg, wave, lane, steps);
+    const HubShare share = hub_share(hp, grid, wg, wave, lane, steps);
     const int ls = lane % LPR, group = lane / LPR;
     const int tile = blockIdx.y * TN;
     const bool col_ok = !EDGE || tile + ls * VEC < n;
@@ -725,13 +725,14 @@ spmm_hub_kernel(int n, int merge, HubGrid grid, const int* __restrict__ hub, con
 // sums are added up through LDS in a fixed order.
 template <typename A>
 __global__ void __launch_bounds__(kWgThreads)
-spmm_hub_reduce_kernel(int n, int merge, const int* __restrict__ hub, const A* __restrict__ partial, A* __restrict__ C)
+spmm_hub_reduce_kernel(int n, HubGrid grid, const int* __restrict__ hub, const A* __restrict__ partial, A* __restrict__ C)
 {
     constexpr int V = 16 / sizeof(A);
     __shared__ __attribute__((aligned(16))) A sums[kWgThreads * V];
     const HubPlan hp = hub_plan_view(hub);
-    const int h = blockIdx.x;
-    if (h >= hp.n_hub) return;
+    const int merge = grid.merge, i = blockIdx.x;
+    if (i >= grid.rows) return;
+    const int h = grid.longs ? hp.longs[i] : i;
     const int* piece = hp.pieces + (size_t)h * (hp.slabs + 1);
     A* c_row = C + (size_t)hp.rows[h] * n;
     const int vecs = n / V; // 16-byte pieces of a row (n * sizeof(A) is a multiple of 16)
@@ -745,7 +746,7 @@ spmm_hub_reduce_kernel(int n, int merge, const int* __restrict__ hub, const A* _
         if (group < groups) {
             for (int sg = group; sg * merge < hp.slabs; sg += groups) {
                 if (piece[min(sg * merge + merge, hp.slabs)] > piece[sg * merge]) {
-                    const A* src = partial + ((size_t)sg * hp.n_hub + h) * n + (size_t)v * V;
+                    const A* src = partial + ((size_t)sg * grid.rows + i) * n + (size_t)v * V;
 #pragma unroll
                     for (int x = 0; x < V; ++x) sum[x] += src[x];
                 }
@@ -806,6 +807,11 @@ inline int grid_for_waves(long long nwaves)
     return wgs * kWgThreads < (1ll << 32) ? (int)wgs : -1;
 }
 
+inline HubRows spmm_hub_rows(const int* counts, int n, int tile, size_t elem)
+{
+    return hub_rows_of_call(counts, n * elem, tile * elem, (n + tile - 1) / tile, 18, 600);
+}
+
 template <typename T, int TN, bool EDGE>
 hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                   const int* row_ptr, const int* col, const typename DenseVec<T>::Acc* val, const T* B,
@@ -819,11 +825,13 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     // segments - which needs no promise, and with this many segments costs no parallelism
     const int block_owned = owned_slots > 0 ? owned_slots : (m1 >= kMergeMinSegments ? -1 : 0);
     // a usable hub plan takes its rows out of both lists (the caller promised whole lists with it)
-    const bool hub_plan = plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 &&
-                          plan.hub_counts[0] > 0;
+    HubRows hub_rows;
+    if (plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 && plan.hub_counts[0] > 0)
+        hub_rows = spmm_hub_rows(plan.hub_counts, n, TN, sizeof(T));
+    const bool hub_plan = hub_rows.rows > 0;
     const bool group_plan = plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] > 0;
     RowOwners owners;
-    owners.hub_min_len = hub_plan ? plan.hub_counts[2] : 0;
+    owners.hub_min_len = hub_rows.min_len;
     if (group_plan) {
         owners.groups = reinterpret_cast<const RowGroup*>(plan.groups + kGroupHeaderInts);
         owners.n_groups = plan.group_counts[0];
@@ -902,15 +910,14 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     }
     if (e == hipSuccess && hubs) {
         using A = typename DenseVec<T>::Acc;
-        const int merge = hub_merge((size_t)n * sizeof(T), plan.hub_counts[1]);
-        const long long pieces = (long long)plan.hub_counts[0] * hub_groups(plan.hub_counts[1], merge);
-        const HubGrid hub_wgs = hub_grid(plan.hub_counts, merge);
+        const long long pieces = (long long)hub_rows.rows * hub_groups(plan.hub_counts[1], hub_rows.merge);
+        const HubGrid hub_wgs = hub_grid(hub_rows, plan.hub_counts[1]);
         if (hub_wgs.wgs < 0) return hipErrorInvalidConfiguration;
         dim3 grid(hub_wgs.wgs, tiles);
         const size_t need = (size_t)pieces * n * sizeof(A);
         A* partial = plan.hub_workspace && plan.hub_workspace_bytes >= need ? static_cast<A*>(plan.hub_workspace) : nullptr;
-        spmm_hub_kernel<T, TN, EDGE><<<grid, hub_wgs.waves * kWave, 0, s1>>>(n, merge, hub_wgs, plan.hub, col, val, B, C, partial);
-        if (partial) spmm_hub_reduce_kernel<A><<<plan.hub_counts[0], kWgThreads, 0, s1>>>(n, merge, plan.hub, partial, C);
+        spmm_hub_kernel<T, TN, EDGE><<<grid, hub_wgs.waves * kWave, 0, s1>>>(n, hub_wgs, plan.hub, col, val, B, C, partial);
+        if (partial) spmm_hub_reduce_kernel<A><<<hub_rows.rows, kWgThreads, 0, s1>>>(n, hub_wgs, plan.hub, partial, C);
         e = hipGetLastError();
     }
     if (e == hipSuccess && grouped) {
@@ -952,9 +959,30 @@ hipError_t launch_edge(int m1, int m2, int n, const int* block_rows, const int* 
 // stored, rows of kept groups of a group plan under kSpmmOverwrite as well).
 int spmm_overwrite_limit(int m1, bool hub_plan) { return m1 >= kOwnedMinSegments && !hub_plan ? kOwnedRowSlots : 0; }
 
-// n: any positive multiple of the 128-bit vector width (4 fp32, 8 fp16, 2 fp64).  The
-// dense row is cut into tiles of 32, 64 or 128 columns (at most 32 lanes per tile row);
-// the tile width with the least padding wins, the widest on a tie.  Multiples of 32 (all
+// The dense row is cut into tiles of 32, 64 or 128 columns (at most 32 lanes of 16 bytes per tile row);
+// the tile width with the least padding wins, the widest on a tie.
+static int spmm_tile_width(int n, size_t elem)
+{
+    auto padded = [n](int tn) { return (n + tn - 1) / tn * tn; };
+    int best = 32;
+    if (padded(64) <= padded(best)) best = 64;
+    if (elem <= 4 && padded(128) <= padded(best)) best = 128;
+    return best;
+}
+
+// The partial rows that the hub kernels of an SpMM of this width want, for operands of 4 (or, if more, 2) or of 8 bytes an element.
+size_t spmm_hub_partial_rows(const int* counts, int n, int acc_bytes)
+{
+    size_t most = 0;
+    for (size_t elem = acc_bytes; elem >= (acc_bytes == 8 ? 8 : 2); elem /= 2) {
+        const HubRows use = spmm_hub_rows(counts, n, spmm_tile_width(n, elem), elem);
+        const size_t rows = (size_t)use.rows * hub_groups(counts[1], use.merge);
+        most = rows > most ? rows : most;
+    }
+    return most;
+}
+
+// n: any positive multiple of the 128-bit vector width (4 fp32, 8 fp16, 2 fp64).  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
 // which `plan` holds a window go to the window kernel where it takes the
 // width (window_takes) and pays (window_pays).
@@ -971,7 +999,6 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
     if (!window_takes(row_bytes) ||
         !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
         plan.no_window();
-    constexpr int kMaxTile = 32 * DenseVec<T>::kElems >= 128 ? 128 : 32 * DenseVec<T>::kElems;
     if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
         constexpr int kLine = 128 / (int)sizeof(T);
         const int lines = n / kLine;
@@ -983,11 +1010,8 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
             return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
         }
     }
-    auto padded = [n](int tn) { return (n + tn - 1) / tn * tn; };
-    int best = 32;
-    if (padded(64) <= padded(best)) best = 64;
-    if (kMaxTile >= 128 && padded(128) <= padded(best)) best = 128;
-    if constexpr (kMaxTile >= 128) {
+    const int best = spmm_tile_width(n, sizeof(T));
+    if constexpr (sizeof(T) <= 4) {
         if (best == 128)
             return launch_edge<T, 128>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags,
                                        plan, s1, s2);

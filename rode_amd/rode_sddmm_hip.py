@@ -203,7 +203,7 @@ def permute(values, perm):
 
 class HubPlan:
     """Hub plan of one pattern (``rode_hip_hub_plan``): the device array and a host copy
-    of its header ``[hub rows, slabs, min_len, usable, room, 0, 0, 0]``."""
+    of its header ``[hub rows, slabs, min_len, usable, room, long rows, nonzeros of the hub rows, of the long ones]``."""
 
     def __init__(self, data, counts):
         self.data = data
@@ -260,12 +260,9 @@ def hub_plan(row_offsets, column_indices, m, n, min_len):
     if counts[3] != 0 and 0 < hub_rows < room:
         # the call needs room for the most hub rows a matrix of this many nonzeros can have; what it
         # found is kept in an array of its own size (header, the rows, their pieces)
-        small = torch.empty(8 + hub_rows + hub_rows * (slabs + 1), dtype=torch.int32, device=dev)
-        small[:8] = data[:8]
-        small[4] = hub_rows
-        small[8:8 + hub_rows] = data[8:8 + hub_rows]
-        small[8 + hub_rows:] = data[8 + room:8 + room + hub_rows * (slabs + 1)]
-        data, counts[4] = small, hub_rows
+        pieces, longs = 8 + room, 8 + room * (slabs + 2)
+        data = torch.cat((data[:8 + hub_rows], data[pieces:pieces + hub_rows * (slabs + 1)], data[longs:longs + counts[5]]))
+        data[4] = counts[4] = hub_rows
     return HubPlan(data, counts)
 
 

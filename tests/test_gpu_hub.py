@@ -209,7 +209,7 @@ def test_calls_on_one_matrix_from_two_streams(dtype):
     from rode_amd import RoDeCSR, rode_sddmm_hip, rode_spmm
     rng = np.random.default_rng(17)
     m, n, k = 3000, 70000, 128
-    lens = rng.integers(600, 900, 400)
+    lens = rng.integers(600, 900, 700)
     lens[:2] = 30000, 7000
     rp, col, val, where = _matrix(rng, m, n, lens)
     old = RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
@@ -240,3 +240,83 @@ def test_calls_on_one_matrix_from_two_streams(dtype):
     assert not torch.equal(*alone)
     assert all(torch.equal(a, alone[i]) for i in range(2) for a in got[i])
     assert csr.plan._workspaces == {}  # nothing that two calls could share is kept
+
+
+@pytest.mark.parametrize("rows,k,dtype,spmm_all,sddmm_all", [
+    (700, 64, "f32", True, True),      # 500 to 600 nonzeros in 5 pieces each
+    (700, 128, "f16", True, True),
+    (700, 512, "f32", True, False),    # SDDMM: 35 pieces; SpMM works on 128 columns at a time: 9
+    (700, 512, "f16", True, True),
+    (700, 200, "f32", True, True),     # no multiple of 128: 18 pieces, SDDMM wants 28 nonzeros in each, has 32
+    (700, 260, "f32", True, False),    # (35)
+    (700, 320, "f32", True, False),
+    (300, 128, "f32", False, True),    # SpMM: too few rows share a slab
+    (300, 36, "f32", False, True),
+    (700, 64, "f64", True, None),
+    (700, 130, "f64", True, None),
+    (300, 32, "f64", False, None),
+])
+def test_rows_of_the_plan_that_a_call_takes(rows, k, dtype, spmm_all, sddmm_all):
+    """All hub rows or the long ones (4096 slots and more), by the width of the call: which ones the hub kernels write, and the whole
+    result against 64 bits, where the other rows are the list kernels'."""
+    import ctypes
+    import oracle
+    from gpu_common import DEV, TOL_F16, TOL_F32, make_csr, round_half
+    from helpers import spmm_row_l1_error
+    from rode_amd import RoDeCSR, _lib, rode_sddmm_hip
+    rng = np.random.default_rng(rows + k)
+    m, n = 3000, 70000
+    lens = rng.integers(516, 600, rows)
+    lens[:5] = 4100, 4200, 5000, 6000, 4097
+    rp, col, val, where = _matrix(rng, m, n, lens, mean_len=8)
+    long_rows = where[np.diff(rp)[where] >= 4097]
+    old = RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
+    RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = 1, 0.0
+    try:
+        csr = make_csr(rp, col, val, m, n, 32)
+    finally:
+        RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = old
+    assert csr.plan.counts[0] == rows and csr.plan.counts[5] == 5
+    assert csr.plan.counts[6] == np.diff(rp)[where].sum() and csr.plan.counts[7] == np.diff(rp)[long_rows].sum()
+    assert np.array_equal(csr.plan.hub_rows(), where)
+    half, lib, plans = dtype == "f16", _lib.load(), csr.call_plans()
+    B, L = rng.standard_normal((n, k)).astype(np.float32), rng.standard_normal((m, k)).astype(np.float32)
+    B, L = (round_half(B), round_half(L)) if half else (B, L)
+    kind = {"f32": torch.float32, "f16": torch.float16, "f64": torch.float64}[dtype]
+    values = csr.values.double() if dtype == "f64" else csr.values
+    dB, dL = torch.from_numpy(B).to(DEV, kind), torch.from_numpy(L).to(DEV, kind)
+    own, scratch = rode_sddmm_hip._with_scratch(plans, k, values.element_size(), csr.device)
+    assert (own.hub_workspace_bytes > rows * 2 * k * values.element_size()) == spmm_all
+
+    def spmm(flags, plans, C):
+        assert lib.rode_hip_spmm_planned(_lib.DENSE_CODE[dtype], _lib.SPMM_WHOLE_LISTS | flags, csr.m1, csr.m2, n, k, values.data_ptr(),
+                                         csr.column_indices.data_ptr(), csr.row_offsets.data_ptr(), csr.block_indices.data_ptr(),
+                                         csr.residue_indices.data_ptr(), csr.st_offsets.data_ptr(), dB.data_ptr(), C.data_ptr(),
+                                         ctypes.byref(plans), None, None) == 0
+        return C.cpu().numpy()
+
+    want, tol = oracle.spmm_f64(rp, col, val, B), 1e-12 if dtype == "f64" else TOL_F16 if half else TOL_F32
+    for p in (own, plans):  # (partial rows; atomics)
+        written = np.nonzero(np.abs(spmm(_lib.SPMM_ONLY_HUB, p, torch.zeros(m, k, device=DEV, dtype=values.dtype))).max(axis=1))[0]
+        assert np.array_equal(written, where if spmm_all else long_rows)
+        assert spmm_row_l1_error(spmm(0, p, torch.zeros(m, k, device=DEV, dtype=values.dtype)), want) <= tol
+    if sddmm_all is None:
+        return
+    ref, scale = oracle.sddmm_f64(rp, col, val, L, B, with_abs=True)
+    row = np.repeat(np.arange(m), np.diff(rp))
+    stale = _lib.Plans.from_buffer_copy(plans)  # (a header made before its last three counts were: whatever rows it leads to, the result holds)
+    header = (ctypes.c_int * 8)(*csr.plan.counts[:5], 0, 0, 0)
+    stale.hub_counts = ctypes.addressof(header)
+    for p in (plans, stale):
+        for flags in (_lib.SPMM_ONLY_HUB, 0):
+            out = torch.full((len(val),), float("nan"), device=DEV)
+            assert lib.rode_hip_sddmm_planned(_lib.DENSE_CODE[dtype], flags, csr.m1, csr.m2, n, k, csr.block_indices.data_ptr(),
+                                              csr.residue_indices.data_ptr(), csr.st_offsets.data_ptr(), csr.row_offsets.data_ptr(),
+                                              csr.column_indices.data_ptr(), csr.values.data_ptr(), dL.data_ptr(), dB.data_ptr(),
+                                              out.data_ptr(), ctypes.byref(p), None, None) == 0
+            got = out.cpu().numpy()
+            if flags and p is plans:
+                assert np.array_equal(~np.isnan(got), np.isin(row, where if sddmm_all else long_rows))
+            elif not flags:
+                # (products and a sum of k terms: k + 2 roundings of the sum of their magnitudes at most)
+                assert (np.abs(got - ref) <= (k + 2) * 2.0 ** -24 * scale).all()
