@@ -503,12 +503,14 @@ __host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs 
 //   * 2 MB instead of 4 in operands of up to 320 MB with (40) at that.  SDDMM / SpMM, 2 -> 4 MB: p 200 K x 32 95 / 112 -> 105 / 117 (185),
 //     x 128 310 / 325 -> 323 / 345 (49), p 330 K x 128 496 / 512 -> 490 / 507 (36), s 262 K x 64 517 / 601 -> 482 / 499 (47), x 128 1310 / 1201 -> 919 / 981 (23);
 //   * SpMM counts the bytes of the column tile that a grid row works on, as long as that leaves 2048 pieces: s 180 K x 512 2827 -> 2024,
-//     halves 2436 -> 1182.
+//     halves 2436 -> 1182;
+//   * the partial rows of SpMM with all rows take no more than eight times the memory of a dense operand of 32 bits (100 000 rows of 1200
+//     nonzeros in 262 K columns: 6.4 M pieces, 3.3 GB at width 128 beside an operand of 134 MB; the long rows have few).
 // With every row, and 2 MB up to 320 MB, wide calls were slower than with the long rows alone: SDDMM s 262 K x 160 2435 -> 4797, x 512 6864 -> 8443, SpMM
 // s 262 K x 512 halves 3494 -> 6179, s 500 K x 1024 halves 8684 -> 17715.
 struct HubRows {
     int rows = 0, min_len = 0; // 0: the call goes without the plan
-    int merge = 1;
+    int merge = 1, mean = 0;   // ..., nonzeros of a row
     bool longs = false;
 };
 inline int hub_merge(size_t row_bytes, int mb)
@@ -516,23 +518,26 @@ inline int hub_merge(size_t row_bytes, int mb)
     const size_t g = ((size_t)mb << 20) / kHubSlabRows / (row_bytes > 0 ? row_bytes : 4);
     return g < 1 ? 1 : (g > 64 ? 64 : (int)g);
 }
-inline HubRows hub_rows_of_call(const int* counts, size_t row_bytes, size_t tile_bytes, int tiles, int pieces_min, int rows_min)
+inline HubRows hub_rows_of_call(const int* counts, size_t row_bytes, size_t tile_bytes, int tiles, int pieces_min, int rows_min, size_t pieces_max)
 {
     const int slabs = counts[1], min_len = counts[2];
-    // (a header of before those counts: every row as short as the plan allows)
-    auto mean = [&](int rows, int nonzeros) { return rows > 0 && nonzeros > 0 ? nonzeros / rows : min_len; };
-    const bool all = counts[0] >= rows_min && mean(counts[0], counts[6]) >= pieces_min * hub_groups(slabs, hub_merge(tile_bytes, 4));
-    HubRows use;
-    use.rows = all ? counts[0] : counts[5];
-    if (use.rows <= 0) return use;
-    use.min_len = all || min_len > kHubLongSlots ? min_len : kHubLongSlots;
-    use.longs = !all;
-    const int length = all ? mean(counts[0], counts[6]) : mean(counts[5], counts[7]);
-    const bool small = tile_bytes * slabs * kHubSlabRows <= ((size_t)320 << 20) && length >= 40 * hub_groups(slabs, hub_merge(tile_bytes, 2));
-    const int most = hub_merge(tile_bytes, small ? 2 : 4);
-    use.merge = hub_merge(row_bytes, small ? 2 : 4);
-    while (2 * use.merge <= most && (long long)use.rows * hub_groups(slabs, 2 * use.merge) * tiles >= 2048) use.merge *= 2;
-    return use;
+    auto take = [&](bool all) {
+        HubRows use;
+        const int nonzeros = counts[all ? 6 : 7];
+        use.rows = counts[all ? 0 : 5];
+        if (use.rows <= 0) return use;
+        use.min_len = all || min_len > kHubLongSlots ? min_len : kHubLongSlots;
+        use.longs = !all;
+        use.mean = nonzeros > 0 ? nonzeros / use.rows : use.min_len; // (a header of before that count: as short as the plan allows)
+        const bool small = tile_bytes * slabs * kHubSlabRows <= ((size_t)320 << 20) && use.mean >= 40 * hub_groups(slabs, hub_merge(tile_bytes, 2));
+        const int most = hub_merge(tile_bytes, small ? 2 : 4);
+        use.merge = hub_merge(row_bytes, small ? 2 : 4);
+        while (2 * use.merge <= most && (long long)use.rows * hub_groups(slabs, 2 * use.merge) * tiles >= 2048) use.merge *= 2;
+        return use;
+    };
+    const HubRows all = take(true);
+    const bool enough = all.rows >= rows_min && all.mean >= pieces_min * hub_groups(slabs, hub_merge(tile_bytes, 4));
+    return enough && (size_t)all.rows * hub_groups(slabs, all.merge) <= pieces_max ? all : take(false);
 }
 
 // Is this row in a tile that the tile kernels have (owners.tiles)?

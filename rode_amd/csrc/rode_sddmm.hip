@@ -471,7 +471,7 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     }
     HubRows hub_rows;
     if (plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 && plan.hub_counts[0] > 0)
-        hub_rows = hub_rows_of_call(plan.hub_counts, (size_t)k * sizeof(T), (size_t)k * sizeof(T), 1, EDGE ? 28 : 18, 1);
+        hub_rows = hub_rows_of_call(plan.hub_counts, (size_t)k * sizeof(T), (size_t)k * sizeof(T), 1, EDGE ? 28 : 18, 1, SIZE_MAX);
     const bool hub_plan = hub_rows.rows > 0;
     // (the group kernel keeps four lhs slices in registers: rows of one slab only)
     const bool group_plan = NS == 1 && plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] > 0;

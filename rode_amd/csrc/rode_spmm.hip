@@ -809,7 +809,7 @@ inline int grid_for_waves(long long nwaves)
 
 inline HubRows spmm_hub_rows(const int* counts, int n, int tile, size_t elem)
 {
-    return hub_rows_of_call(counts, n * elem, tile * elem, (n + tile - 1) / tile, 18, 600);
+    return hub_rows_of_call(counts, n * elem, tile * elem, (n + tile - 1) / tile, 18, 600, (size_t)8 * kHubSlabRows * counts[1]);
 }
 
 template <typename T, int TN, bool EDGE>

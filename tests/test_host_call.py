@@ -87,3 +87,21 @@ def test_two_first_calls_get_one_hub_workspace(monkeypatch):
     assert plan.workspace(32, 4) is other[0] is plan.workspace(32, 4)
     csr = _stand_in(plan)
     assert csr.plans_address(32).plans.hub_workspace == other[0].data_ptr() and csr.plans_address() != csr.plans_address(32)
+
+
+@pytest.mark.parametrize("n", [32, 128, 256, 1024])
+@pytest.mark.parametrize("elem", [4, 8])
+def test_hub_workspace_is_bounded(n, elem):
+    """The partial rows of an SpMM with all rows of a hub plan take up to eight dense operands (of 4 or 8 bytes an element); with more a
+    call takes the long rows, which are few."""
+    lib, slabs, longs = _lib.load(), 128, 300
+
+    def size(rows, mean):
+        header = (ctypes.c_int * 8)(rows, slabs, 512, 1, rows, longs, rows * mean, longs * 9000)
+        return lib.rode_hip_hub_workspace_bytes(ctypes.addressof(header), n, elem)
+
+    operand, few = slabs * 2048 * n * elem, size(599, 1200)  # (fewer than 600 rows: the long ones)
+    assert 0 < few <= longs * slabs * n * elem
+    for rows in (600, 8000, 16500, 40000, 100_000, 200_000):
+        assert few < size(rows, 4000) <= 8 * operand or size(rows, 4000) == few
+    assert size(600, 4000) > few and size(2_000_000, 1000) == few
