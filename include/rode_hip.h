@@ -222,7 +222,8 @@ int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_
  *   d_plan       rode_hip_hub_plan_bytes(M, dense_rows, nnz, min_len) bytes, 16-byte aligned, out
  *   h_counts     HOST int[8], out (the call waits for its two kernels): [0] hub rows,
  *                [1] slabs, [2] min_len, [3] 1 if the plan is usable - every hub row's column
- *                indices ascend and lie inside the operand - else 0, [4] room for hub rows, [5] hub rows of
+ *                indices ascend and lie inside the operand -, 2 if that holds for the rows of 4096 slots and more
+ *                (calls then take only those), else 0, [4] room for hub rows, [5] hub rows of
  *                4096 slots and more, [6] and [7] nonzeros of all hub rows and of those;
  *                the *_planned entry points need it and ignore a plan with [3] == 0 or [0] == 0
  * A hub plan belongs to the pattern it was made from, and excludes a locality plan: the

@@ -175,6 +175,8 @@ int rode_hip_hub_plan(int M, int dense_rows, int nnz, int min_len, const int* d_
             e = rode::hub_pieces_launch(h_counts[0], dense_rows, d_row_offsets, d_column_indices, plan, as_stream(stream));
         }
     }
+    // (2 and 4: a shorter and a long row without ascending columns)
+    if (e == hipSuccess && h_counts[3] > 1) h_counts[3] = h_counts[3] & 4 || h_counts[5] == 0 ? 0 : 2;
     return e;
 }
 

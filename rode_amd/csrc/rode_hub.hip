@@ -10,7 +10,7 @@
 //                      header), then every block writes its hub rows to their places.
 //   hub_pieces_kernel  one workgroup per hub row: a binary search per slab boundary in the
 //                      row's column indices, and a pass over the row that checks that its
-//                      columns ascend (if one does not, the plan is marked unusable).
+//                      columns ascend (else the plan is good for the long rows alone, or, with a long row, for nothing).
 #include "rode_items.hpp"
 #include "rode_internal.hpp"
 
@@ -147,7 +147,7 @@ hub_pieces_kernel(int dense_rows, const int* __restrict__ row_ptr, const int* __
     for (int i = s + threadIdx.x; i + 1 < e; i += kWgThreads) ascending = ascending && col[i] <= col[i + 1];
     // also: every column is inside the operand (else a piece past the last slab would be lost)
     for (int i = s + threadIdx.x; i < e; i += kWgThreads) ascending = ascending && (unsigned)col[i] < (unsigned)dense_rows;
-    if (!ascending) plan[3] = 0;
+    if (!ascending) atomicOr(plan + 3, e - s + (s & (kVecLen - 1)) < kHubLongSlots ? 2 : 4); // (rode_hip_hub_plan reads them)
 }
 
 } // namespace

@@ -462,10 +462,11 @@ inline const RowTile* group_plan_tiles(const int* plan, int M) { return reinterp
 // a few neighbouring slabs at a time (hub_rows_of_call: 2 or 4 MB of the dense operand): all hub rows' nonzeros of those
 // slabs at the same time on one XCD, so that a dense row is fetched from memory once and
 // then found in L2 by the other hubs.
-// Needs rows whose column indices ascend (the plan checks).  The standard kernels skip
+// Needs rows whose column indices ascend (the plan checks; rows of less than kHubLongSlots are left out
+// together if one of them does not).  The standard kernels skip
 // the rows of a usable plan (by their length), so every nonzero is still processed once.
 // Layout, ints: header [0] hub rows  [1] slabs  [2] shortest hub row (aligned length)
-// [3] usable (every hub row's columns ascend)  [4] room for hub rows  [5] how many of the hub rows have kHubLongSlots aligned
+// [3] usable: 1 all hub rows, 2 those of [5], 0 none  [4] room for hub rows  [5] how many of the hub rows have kHubLongSlots aligned
 // slots or more  [6], [7] nonzeros of all hub rows and of those;
 // then the hub rows, ascending (room for [4] of them); then per hub row slabs + 1 piece
 // starts (indices into column_indices / values; the last one is the row's end); then which of the hub rows are those of [5]
@@ -536,7 +537,7 @@ inline HubRows hub_rows_of_call(const int* counts, size_t row_bytes, size_t tile
         return use;
     };
     const HubRows all = take(true);
-    const bool enough = all.rows >= rows_min && all.mean >= pieces_min * hub_groups(slabs, hub_merge(tile_bytes, 4));
+    const bool enough = counts[3] != 2 && all.rows >= rows_min && all.mean >= pieces_min * hub_groups(slabs, hub_merge(tile_bytes, 4));
     return enough && (size_t)all.rows * hub_groups(slabs, all.merge) <= pieces_max ? all : take(false);
 }
 

@@ -320,3 +320,39 @@ def test_rows_of_the_plan_that_a_call_takes(rows, k, dtype, spmm_all, sddmm_all)
             elif not flags:
                 # (products and a sum of k terms: k + 2 roundings of the sum of their magnitudes at most)
                 assert (np.abs(got - ref) <= (k + 2) * 2.0 ** -24 * scale).all()
+
+
+@pytest.mark.parametrize("bad", ["none", "shorter", "long", "shorter, no long"])
+def test_hub_rows_without_ascending_columns(bad):
+    """One row of 512 to 4095 nonzeros in another order leaves a plan of the rows of 4096 and more; one of those leaves none."""
+    import oracle
+    from gpu_common import TOL_F32, make_csr, run_sddmm, run_spmm
+    from helpers import spmm_row_l1_error
+    from rode_amd import RoDeCSR
+    rng = np.random.default_rng(5)
+    m, n, k = 3000, 70000, 64
+    lens = rng.integers(520, 600, 700)
+    if bad != "shorter, no long":
+        lens[:3] = 4500, 6000, 9000
+    rp, col, val, where = _matrix(rng, m, n, lens, mean_len=8)
+    length = np.diff(rp)
+    if bad != "none":
+        row = where[(length[where] > 4096) == (bad == "long")][1]
+        col[rp[row]:rp[row + 1]] = rng.permutation(col[rp[row]:rp[row + 1]])
+    old = RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
+    RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = 1, 0.0
+    try:
+        csr = make_csr(rp, col, val, m, n, k)
+        if bad == "shorter, no long":  # (_may_hub asks for one; a caller of the C ABI may still want the plan)
+            from rode_amd import rode_sddmm_hip
+            assert not rode_sddmm_hip.hub_plan(csr.row_offsets, csr.column_indices, m, n, 512).usable
+    finally:
+        RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = old
+    if bad in ("none", "shorter"):
+        assert csr.plan.usable and csr.plan.counts[3] == (1 if bad == "none" else 2) and csr.plan.counts[5] == 3
+    else:
+        assert csr.plan is None or not hasattr(csr.plan, "hub_rows")
+    B, L = rng.standard_normal((n, k)).astype(np.float32), rng.standard_normal((m, k)).astype(np.float32)
+    assert spmm_row_l1_error(run_spmm(csr, B), oracle.spmm_f64(rp, col, val, B)) <= TOL_F32
+    ref, scale = oracle.sddmm_f64(rp, col, val, L, B, with_abs=True)
+    assert (np.abs(run_sddmm(csr, L, B) - ref) <= (k + 2) * 2.0 ** -24 * scale).all()
