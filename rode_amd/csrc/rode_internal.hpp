@@ -103,14 +103,24 @@ constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (s
 // over all heads on: a tile takes 10 to 45 us however few there are, and rows in no tile are a launch more.  Us row by row -> on tiles, fp32 / halves:
 // 4096 rows of 256 and 64 random columns, a few rows left over, 1.3 M nonzeros, width 64: 25.4 -> 26.5 / 15.7 -> 19.1, 128: 48.9 -> 47.7 / 25.7 -> 24.9; 3000 of
 // 200 and 16, 1.3 M: 28.7 -> 22.0 / 17.6 -> 14.7, 54.4 -> 37.5 / 29.1 -> 19.5, 0.65 M: 16.3 -> 17.6 / 10.7 -> 13.2, 27.1 -> 26.2 / 16.7 -> 15.7.
-// Where the tiles have all rows, from 0.4 M on (but for fp32 of width 32: 2048 rows of 600 and 96, 1.4 M, 16.3 -> 17.1): 2000 rows of 200 and 16,
-// 0.43 M, width 64: 12.2 -> 11.9 / 9.6 -> 9.8, 128: 19.3 -> 17.5 / 12.6 -> 10.0; 4000 rows, 0.86 M: 20.1 -> 12.1 / 12.9 -> 9.8, 36.3 -> 20.0 / 20.6 -> 10.3;
-// 2000 of 400 and 64, 0.93 M: 21.4 -> 19.0 / 14.0 -> 11.7, 36.7 -> 30.2 / 21.3 -> 16.5.
+// Where the tiles have all rows (but for fp32 of width 32: 2048 rows of 600 and 96, 1.4 M, 16.3 -> 17.1):
+//   * more than 64 tiles over all heads (with up to 1024 rows every wave of the other kernel has a SIMD of its own), from 0.4 M on:
+//     1280 rows of 400 and 64, width 64 19.5 -> 18.2 / 12.7 -> 10.9, 128 34.2 -> 29.5 / 19.8 -> 15.3; 2000 of 250 12.0 -> 10.7 / 8.5 -> 6.9, 20.4 -> 15.7 / 12.6 -> 8.6;
+//     2800 of 400 23.4 -> 13.9 / 14.7 -> 7.7, 41.7 -> 20.8 / 24.3 -> 10.0; halves of width 32 from 0.6 M: 2000 of 250 and 20 7.0 -> 7.6, 2800 of 250 7.0 -> 6.2;
+//   * fewer, with 700 nonzeros a row, from 0.4 M on but not in fp32 of width 64: 1024 rows of 800 and 64, width 64 22.5 -> 25.9 / 17.1 -> 13.4, 128 48.4 -> 41.6 /
+//     23.9 -> 19.5, halves of width 32 13.1 -> 11.1; of 400 and 64 14.5 -> 18.2 / 11.6 -> 10.8, 26.1 -> 28.7 / 14.5 -> 15.2, 8.5 -> 9.3, training step 68 -> 74 / 64 -> 67.
 inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads, int N, long long nnz, size_t row_bytes, bool halves)
 {
     if (plan.groups == nullptr || plan.group_counts == nullptr || plan.group_counts[1] <= 0 || plan.group_counts[3] <= 0) return false;
-    const bool all_rows = plan.group_counts[2] == 0 && 4 * plan.group_counts[3] == plan.group_counts[1];
-    const long long enough = all_rows && (halves || row_bytes > 128) ? 400000 : 1500000;
+    const long long tiles = plan.group_counts[3];
+    const bool all_rows = plan.group_counts[2] == 0 && 4 * tiles == plan.group_counts[1];
+    long long enough = 1500000;
+    if (all_rows && (halves || row_bytes > 128)) {
+        if (tiles * nheads > 64)
+            enough = row_bytes > 64 ? 400000 : 600000;
+        else if (nnz >= 700 * 16 * tiles && (halves || row_bytes > 256))
+            enough = 400000;
+    }
     return (plan.group_counts[1] >= groups_min || nnz * nheads >= enough) && attention_tiles_fit(N, row_bytes);
 }
 // (rode_attention_tile.hip) the rows of a group plan's tiles, the same arguments; plan: the group plan

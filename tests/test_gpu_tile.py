@@ -365,3 +365,26 @@ def test_fewer_nonzeros_where_the_tiles_have_all_rows(m, rows_left):
     out = sparse_attention(csr, *ins, scale=0.125)
     for a, b in zip((out,) + torch.autograd.grad(out, ins, g), want):
         assert (a.double() - b).norm() <= 2e-6 * b.norm()
+
+
+@pytest.mark.parametrize("m,window,extra,d,half", [
+    (1024, 360, 40, 64, False), (1024, 720, 40, 64, False), (1040, 360, 40, 64, False),  # up to 64 tiles, and more
+    (1024, 360, 40, 128, True), (1024, 720, 40, 128, True), (1040, 360, 40, 128, True),
+    (512, 660, 40, 128, False), (512, 740, 40, 128, False),  # below and above 700 nonzeros a row, and 0.4 M
+    (1600, 240, 20, 32, True), (2400, 240, 20, 32, True),    # below and above 0.6 M
+])
+def test_few_tiles_that_have_all_rows(m, window, extra, d, half):
+    """Either side of the lines between a wave per row and the tiles, where these have all rows."""
+    csr, dense = _mask(m, window, 1, extra, seed=m + window)
+    assert csr.plan.counts[3] == m // 16 and csr.plan.counts[2] == 0 and csr.nnz < 1_500_000
+    dt = torch.float16 if half else torch.float32
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    q, k, v, g = (torch.randn(r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n, m))
+    q, k, v = (t.to(dt) for t in (q, k, v))
+    ins = [t.double().requires_grad_() for t in (q, k, v)]
+    want = _reference(dense, *ins, d ** -0.5)
+    want = (want,) + torch.autograd.grad(want, ins, g.double())
+    ins = [t.clone().requires_grad_() for t in (q, k, v)]
+    out = sparse_attention(csr, *ins, scale=d ** -0.5)
+    for a, b in zip((out,) + torch.autograd.grad(out, ins, g), want):
+        assert (a.double() - b).norm() <= (2e-3 if half and b is not want[0] else 2e-6) * b.norm()
