@@ -825,10 +825,9 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     // segments - which needs no promise, and with this many segments costs no parallelism
     const int block_owned = owned_slots > 0 ? owned_slots : (m1 >= kMergeMinSegments ? -1 : 0);
     // a usable hub plan takes its rows out of both lists (the caller promised whole lists with it)
-    HubRows hub_rows;
-    if (plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 && plan.hub_counts[0] > 0)
-        hub_rows = spmm_hub_rows(plan.hub_counts, n, TN, sizeof(T));
-    const bool hub_plan = hub_rows.rows > 0;
+    const bool hub_plan = plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 &&
+                          plan.hub_counts[0] > 0;
+    const HubRows hub_rows = hub_plan ? spmm_hub_rows(plan.hub_counts, n, TN, sizeof(T)) : HubRows();
     const bool group_plan = plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] > 0;
     RowOwners owners;
     owners.hub_min_len = hub_rows.min_len;
@@ -840,7 +839,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     const bool overwrite = (flags & kSpmmOverwrite) != 0;
     owners.overwrite = overwrite && owned_slots > 0 && !hub_plan;
     const int only = flags & kOnlyMask; // one kernel family of the call (timing each on its own)
-    const bool hubs = hub_plan && (only == 0 || only == kSpmmOnlyHub);
+    const bool hubs = hub_rows.rows > 0 && (only == 0 || only == kSpmmOnlyHub);
     const bool grouped = group_plan && (only == 0 || only == kSpmmOnlyHub); // (timed with the hub kernels)
     constexpr int RPW = kWave / SpmmShape<T, TN>::kLpr;
     const int shards = plan.shards > 1 ? plan.shards : 1, tile_rows = plan.shards > 1 ? 1 : tiles;

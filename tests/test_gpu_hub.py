@@ -356,3 +356,31 @@ def test_hub_rows_without_ascending_columns(bad):
     assert spmm_row_l1_error(run_spmm(csr, B), oracle.spmm_f64(rp, col, val, B)) <= TOL_F32
     ref, scale = oracle.sddmm_f64(rp, col, val, L, B, with_abs=True)
     assert (np.abs(run_sddmm(csr, L, B) - ref) <= (k + 2) * 2.0 ** -24 * scale).all()
+
+
+def test_plan_that_a_product_takes_no_rows_of():
+    """A plan of 300 rows without a long one: SpMM leaves them to the list kernels, which add to them as
+    ``rode_hip_spmm_overwrite_limit`` says (0 with a hub plan)."""
+    import ctypes
+    import oracle
+    from gpu_common import DEV, TOL_F32, make_csr
+    from helpers import spmm_row_l1_error
+    from rode_amd import _lib, rode_sddmm_hip
+    lib, rng = _lib.load(), np.random.default_rng(8)
+    m, n, k = 3000, 70000, 64
+    rp, col, val, _ = _matrix(rng, m, n, rng.integers(516, 600, 1100), mean_len=8)
+    csr = make_csr(rp, col, val, m, n, k, locality=False)
+    lens = np.diff(rp) + rp[:-1] % 4
+    plan = rode_sddmm_hip.hub_plan(csr.row_offsets, csr.column_indices, m, n, int(np.sort(lens)[-300]))
+    assert plan.usable and 300 <= plan.counts[0] < 400 and plan.counts[5] == 0 and csr.m1 >= 1024
+    plans, B = rode_sddmm_hip.plans_struct(plan), rng.standard_normal((n, k)).astype(np.float32)
+    assert lib.rode_hip_spmm_overwrite_limit(csr.m1, ctypes.byref(plans)) == 0
+    dB, C = torch.from_numpy(B).to(DEV), torch.full((m, k), 7.0, device=DEV)
+    assert lib.rode_hip_spmm_planned(0, _lib.SPMM_WHOLE_LISTS | _lib.SPMM_OVERWRITE, csr.m1, csr.m2, n, k, csr.values.data_ptr(),
+                                     csr.column_indices.data_ptr(), csr.row_offsets.data_ptr(), csr.block_indices.data_ptr(),
+                                     csr.residue_indices.data_ptr(), csr.st_offsets.data_ptr(), dB.data_ptr(), C.data_ptr(),
+                                     ctypes.byref(plans), None, None) == 0
+    C = C.cpu().numpy()
+    touched = lens > 0
+    want = oracle.spmm_f64(rp, col, val, B) + np.where(lens >= 32, 7.0, 0.0)[:, None]
+    assert spmm_row_l1_error(C[touched], want[touched]) <= TOL_F32
