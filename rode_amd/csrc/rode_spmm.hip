@@ -52,6 +52,7 @@ constexpr int kOwnedMinSegments = 1024;
 // halves: 512 x 512 of 16 to 64 nonzeros 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3 -> 15.0, 250 K 150 -> 143; longest
 // row 168 7.7 / 10.6 / 12.0 -> 5.7 / 6.0 / 5.7, 227 7.8 / 9.8 / 10.7 -> 5.7 / 6.4 / 5.7, 338 7.5 / 8.7 / 9.0 -> 5.8 / 7.3 / 6.7, 471 7.9 / 9.9 / 10.4 -> 5.8 / 9.1 / 7.8,
 // 502 8.4 / 8.4 / 8.2 -> 5.9 / 9.4 / 8.2, 1001 7.4 / 8.5 / 7.9 -> 8.0 / 15.0 / 12.6).
+// Each 64 slots of such a row have a sum of their own, as the row's segments had: one chain over all of a row had up to 1.7 times their error.
 constexpr int kShortRowSlots = 384;
 // Without the promise the block kernel may still merge the short segments of a row that
 // the list it was given holds, when there are this many of them.
@@ -106,7 +107,8 @@ inline bool sharding_pays(int lines, bool halves, size_t dense_rows, long long i
 // last quad are neutralised.  Every lane of the wave returns the wave's total.
 // (split, jump: the slots are [base, base + split) followed by [base + split + jump, ...):
 // a row with a hole that somebody else works on; split >= cnt for one plain range.)
-template <typename T, int TN>
+// PARTS: every 64 slots have a sum of their own, and the total is the sum of those.
+template <typename T, int TN, bool PARTS = false>
 __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int split, int jump, int lane, int* my_c,
                                                typename DenseVec<T>::Acc* my_v, const T* b_lane, int n,
                                                const int* __restrict__ col,
@@ -117,9 +119,9 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
     using A = typename S::Acc;
     constexpr int VEC = S::kVec, LPR = S::kLpr, G = S::kGroupsWave;
     const int group = lane / LPR;
-    A acc[VEC];
+    A acc[VEC], parts[VEC];
 #pragma unroll
-    for (int x = 0; x < VEC; ++x) acc[x] = A(0);
+    for (int x = 0; x < VEC; ++x) acc[x] = parts[x] = A(0);
 
     // slots of the previous row (head) and slots past the end (last quad) are neutralised:
     // value 0, column of a real slot
@@ -148,10 +150,14 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
             spmm_gather<T, TN, 16 / G, true>(b_lane, (size_t)n, acc, my_c, my_v, group, G, 16);
         else
             spmm_gather<T, TN, 16 / G, false>(b_lane, (size_t)n, acc, my_c, my_v, group, G, (live + 3) / 4);
+        if constexpr (PARTS) {
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) parts[x] += acc[x], acc[x] = A(0);
+        }
         wave_lds_sync();
     }
 #pragma unroll
-    for (int x = 0; x < VEC; ++x) total[x] = butterfly_sum<LPR, kWave>(acc[x]);
+    for (int x = 0; x < VEC; ++x) total[x] = butterfly_sum<LPR, kWave>(PARTS ? parts[x] : acc[x]);
 }
 
 // Which column tile of C, and which of the `blocks` workgroups of its grid row, a workgroup is.
@@ -171,7 +177,8 @@ __device__ __forceinline__ TilePlace tile_place(int b, int blocks, int shards)
 // One wave per block segment (see sddmm_block_kernel for the slot arithmetic,
 // identical at RoDeSpmm.cu:210-234).
 // (bid of nblocks: the workgroup's position in the part of the grid that works on block segments)
-// WALK: 0 one wave per segment only, 1 chunks only (chunk_hint > 1), 2 either, found out here.
+// WALK: 0 one wave per segment only, 1 chunks only (chunk_hint > 1), 2 either, found out here; 3 one wave per segment, which
+// sums its row in parts (kShortRowSlots).
 // (Kernels of their own, so that the code of one way does not cost the other registers.)
 // STORE: a row's only work item stores its sum instead of adding it (owners.overwrite; a
 // kernel of its own as well: as a run-time branch it slowed the fp16 kernel of width 128
@@ -199,7 +206,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     if constexpr (WALK == 2)
         chunk = block_chunk_for_grid(owned_slots != 0 && m1 >= kWalkMinSegments ? block_chunk(m1, block_rows, st_off) : 1, m1,
                                      nblocks);
-    if (WALK != 0 && chunk > 1) {
+    if (WALK != 0 && WALK != 3 && chunk > 1) {
         const long long first = chunk_first_segment(bid, wave, m1, chunk);
         if (first < 0) return;
         const int last = (int)min(first + chunk, (long long)m1);
@@ -277,7 +284,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     // combine the lane groups, then spread the atomics over them
     constexpr int EPG = VEC / G > 0 ? VEC / G : 1; // elements each group adds
     A total[VEC];
-    spmm_sum_slots<T, TN>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total);
+    spmm_sum_slots<T, TN, WALK == 3>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total);
     if (shared_row) {
         __shared__ __attribute__((aligned(16))) A wg_sum[kWavesPerWg][TN];
         if (group == 0) {
@@ -818,16 +825,16 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
                   typename DenseVec<T>::Acc* C, int flags, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
     const int tiles = (n + TN - 1) / TN;
-    // (rows known to be short: one wave has no more to do for all of a row)
-    const bool short_rows = plan.longest > 0 && plan.longest <= kShortRowSlots;
-    const int owned_slots = (flags & kSpmmWholeLists) && (m1 >= kOwnedMinSegments || short_rows) ? kOwnedRowSlots : 0;
-    // what the block kernel is told: rows it owns, or (negative) only that it may merge short
-    // segments - which needs no promise, and with this many segments costs no parallelism
-    const int block_owned = owned_slots > 0 ? owned_slots : (m1 >= kMergeMinSegments ? -1 : 0);
     // a usable hub plan takes its rows out of both lists (the caller promised whole lists with it)
     const bool hub_plan = plan.hub != nullptr && plan.hub_counts != nullptr && plan.hub_counts[3] != 0 &&
                           plan.hub_counts[0] > 0;
     const HubRows hub_rows = hub_plan ? spmm_hub_rows(plan.hub_counts, n, TN, sizeof(T)) : HubRows();
+    // (rows known to be short: one wave has no more to do for all of a row)
+    const bool short_rows = plan.longest > 0 && plan.longest <= kShortRowSlots && !hub_plan;
+    const int owned_slots = (flags & kSpmmWholeLists) && (m1 >= kOwnedMinSegments || short_rows) ? kOwnedRowSlots : 0;
+    // what the block kernel is told: rows it owns, or (negative) only that it may merge short
+    // segments - which needs no promise, and with this many segments costs no parallelism
+    const int block_owned = owned_slots > 0 ? owned_slots : (m1 >= kMergeMinSegments ? -1 : 0);
     const bool group_plan = plan.groups != nullptr && plan.group_counts != nullptr && plan.group_counts[1] > 0;
     RowOwners owners;
     owners.hub_min_len = hub_rows.min_len;
@@ -838,6 +845,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     // rows with a single work item are stored instead of added (spmm_overwrite_limit says which)
     const bool overwrite = (flags & kSpmmOverwrite) != 0;
     owners.overwrite = overwrite && owned_slots > 0 && !hub_plan;
+    const bool in_parts = short_rows && m1 < kOwnedMinSegments && owners.overwrite;
     const int only = flags & kOnlyMask; // one kernel family of the call (timing each on its own)
     const bool hubs = hub_rows.rows > 0 && (only == 0 || only == kSpmmOnlyHub);
     const bool grouped = group_plan && (only == 0 || only == kSpmmOnlyHub); // (timed with the hub kernels)
@@ -880,7 +888,9 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     if (pair) {
         dim3 grid((g0 + g1 + g2) * shards, tile_rows);
         auto kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 2, true> : spmm_pair_kernel<T, TN, EDGE, 2, false>;
-        if (chunk_hint == 1)
+        if (in_parts)
+            kernel = spmm_pair_kernel<T, TN, EDGE, 3, true>;
+        else if (chunk_hint == 1)
             kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 0, true> : spmm_pair_kernel<T, TN, EDGE, 0, false>;
         else if (chunk_hint > 1)
             kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 1, true> : spmm_pair_kernel<T, TN, EDGE, 1, false>;
@@ -891,7 +901,9 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         if (block) {
             dim3 grid(g1 * shards, tile_rows);
             auto kernel = spmm_block_kernel<T, TN, EDGE, 2, false>;
-            if (chunk_hint == 1)
+            if (in_parts)
+                kernel = spmm_block_kernel<T, TN, EDGE, 3, true>;
+            else if (chunk_hint == 1)
                 kernel = owners.overwrite ? spmm_block_kernel<T, TN, EDGE, 0, true> : spmm_block_kernel<T, TN, EDGE, 0, false>;
             else if (chunk_hint > 1)
                 kernel = owners.overwrite ? spmm_block_kernel<T, TN, EDGE, 1, true> : spmm_block_kernel<T, TN, EDGE, 1, false>;
