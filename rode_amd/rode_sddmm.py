@@ -61,7 +61,6 @@ class RoDeCSR:
         # one pass over the row offsets: the longest row, the choice of the segment length and of a plan
         self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len(8))
         self.max_row_length = self._stats[0]
-        self.longest_row = self._stats[2]  # in aligned slots
         if isinstance(config, str):
             if config != "auto":
                 raise ValueError(f'config must be a dict, None or "auto", got {config!r}')
@@ -81,6 +80,11 @@ class RoDeCSR:
         self.locality = locality
         self._shared = {}  # per-pattern cache (the transposed pattern); with_values() copies share it
         self._preprocess()
+
+    @property
+    def longest_row(self):
+        """The longest row in aligned slots."""
+        return self._stats[2]
 
     @classmethod
     def auto_config(cls, row_offsets):

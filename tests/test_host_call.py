@@ -105,3 +105,12 @@ def test_hub_workspace_is_bounded(n, elem):
     for rows in (600, 8000, 16500, 40000, 100_000, 200_000):
         assert few < size(rows, 4000) <= 8 * operand or size(rows, 4000) == few
     assert size(600, 4000) > few and size(2_000_000, 1000) == few
+
+
+def test_matrix_kept_without_its_longest_row():
+    """A matrix that a program has pickled holds the statistics of its rows, not what later versions read off them."""
+    import pickle
+    csr = _stand_in()
+    csr._stats = (300, 1, 303, 7, 7, 7, 7, 0)
+    assert "longest_row" not in pickle.loads(pickle.dumps(csr)).__dict__
+    assert pickle.loads(pickle.dumps(csr)).longest_row == 303
