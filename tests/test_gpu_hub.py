@@ -171,8 +171,8 @@ def test_hub_plan_through_the_c_abi(k):
 
 @pytest.mark.parametrize("hubs,k,half", [(2, 64, False), (40, 128, False), (300, 128, False), (1200, 128, True), (2300, 64, False), (4600, 128, False)])
 def test_pieces_shared_by_waves(hubs, k, half):
-    """The ways the waves of a workgroup share pieces (by their number: one piece for eight waves, two, four and eight for four), with pieces
-    of one nonzero, empty ones and some that several waves have a part of."""
+    """Pieces shared by the waves of a workgroup, with pieces of one nonzero, empty ones and some that several waves have a part
+    of.  (How many waves and pieces: test_pieces_per_workgroup.)"""
     import oracle
     from gpu_common import TOL_F16, TOL_F32, make_csr, round_half, run_sddmm, run_spmm
     from helpers import spmm_row_l1_error, sddmm_row_l1_errors
@@ -384,3 +384,51 @@ def test_plan_that_a_product_takes_no_rows_of():
     touched = lens > 0
     want = oracle.spmm_f64(rp, col, val, B) + np.where(lens >= 32, 7.0, 0.0)[:, None]
     assert spmm_row_l1_error(C[touched], want[touched]) <= TOL_F32
+
+
+@pytest.mark.parametrize("rows,n,k,dtype,waves,pieces", [
+    (300, 70000, 128, "f32", 8, 1),      # the three long rows alone: 9 groups of slabs
+    (1200, 70000, 128, "f32", 8, 2),
+    (1200, 70000, 64, "f64", 8, 2),
+    (2300, 70000, 128, "f32", 4, 2),
+    (2300, 70000, 64, "f64", 4, 2),
+    (4600, 70000, 128, "f32", 4, 4),
+    (4600, 70000, 64, "f64", 4, 4),
+    (4600, 140000, 128, "f32", 4, 8),    # 18 groups
+    (4600, 140000, 64, "f64", 4, 8),
+])
+def test_pieces_per_workgroup(rows, n, k, dtype, waves, pieces):
+    """Every number of waves and pieces that a workgroup of the hub kernels can have (by the pieces there are in all, which the
+    workspace has a row each for)."""
+    import oracle
+    from gpu_common import DEV, make_csr
+    from rode_amd import RoDeCSR, rode_sddmm_hip
+    rng = np.random.default_rng(rows + n)
+    m = 5000
+    lens = rng.integers(0, 40, m)
+    where = rng.choice(m, rows, replace=False)
+    lens[where] = rng.integers(350, 420, rows) if n > 100000 else rng.integers(200, 400, rows)
+    lens[where[:3]] = 30000, 7000, 4200
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    row = np.repeat(np.arange(m), lens)
+    step = n // lens[row]  # (one column in every n / length: ascending, distinct)
+    col = ((np.arange(len(row)) - rp[row]) * step + rng.integers(0, step)).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(np.float32)
+    old = RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE
+    RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = 64, 1, 0.0
+    try:
+        csr = make_csr(rp, col, val, m, n, k)
+    finally:
+        RoDeCSR.HUB_MIN_LEN, RoDeCSR.HUB_MIN_SLABS, RoDeCSR.HUB_MIN_SHARE = old
+    assert csr.plan.usable
+    values = csr.values.double() if dtype == "f64" else csr.values
+    plans, scratch = rode_sddmm_hip._with_scratch(csr.call_plans(), k, values.element_size(), csr.device)
+    items = plans.hub_workspace_bytes // (k * values.element_size())
+    assert waves == (4 if items >= 20000 else 8)
+    assert pieces == (8 if items >= 80000 else 4 if items >= 40000 else 2 if items >= 5000 else 1)
+    B = rng.standard_normal((n, k)).astype(np.float32)
+    got = rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets, csr.column_indices,
+                                      values, m, n, torch.from_numpy(B).to(DEV, values.dtype), plans=plans)
+    want, scale = oracle.spmm_f64(rp, col, val, B, with_abs=True)
+    # (a sum of n products: n + 2 roundings of the sum of their magnitudes at most)
+    assert (np.abs(got.cpu().numpy() - want) <= scale * (lens[:, None] + 2) * (2.0 ** -52 if dtype == "f64" else 2.0 ** -24)).all()

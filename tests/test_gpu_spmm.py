@@ -602,7 +602,7 @@ def test_overwrite_leaves_other_rows_to_the_callers_clearing():
     (700, (0, 60), 385, 64),        # one row past it: cleared beforehand
     (3000, (0, 80), 1024, 64),      # the longest row with one owner
     (3000, (0, 80), 1025, 64),      # more than that: cleared beforehand
-    (6000, (0, 70), 500, 256),      # column tiles dealt out to the XCDs
+    (6000, (0, 70), 500, 256),      # several column tiles
     (64, (32, 33), 0, 32),          # (aligned lists: most rows have no tail)
 ])
 def test_product_into_memory_that_holds_anything(rows, lengths, longest, k, dtype):
@@ -724,3 +724,88 @@ def test_whole_rows_in_small_matrices_are_no_less_exact(length, k, half, groups)
         mine += ((got - want) ** 2).sum()
         segments += ((_sum_in_segments(val, dense[col], groups) - want) ** 2).sum()
     assert mine ** 0.5 <= 1.05 * segments ** 0.5
+
+
+def _into_nan(csr, B, longest, plans):
+    """rode_hip_spmm_new into a C full of NaN."""
+    from rode_amd import _lib
+    code = {torch.float32: 0, torch.float16: 1, torch.float64: 2}[B.dtype]
+    out = torch.full((csr.m, B.shape[1]), float("nan"), dtype=csr.values.dtype, device=B.device)
+    assert _lib.load().rode_hip_spmm_new(code, csr.m, longest, csr.m1, csr.m2, csr.n, B.shape[1], csr.values.data_ptr(), csr.column_indices.data_ptr(),
+                                         csr.row_offsets.data_ptr(), csr.block_indices.data_ptr(), csr.residue_indices.data_ptr(),
+                                         csr.st_offsets.data_ptr(), B.data_ptr(), out.data_ptr(), ctypes.addressof(plans),
+                                         torch.cuda.current_stream().cuda_stream) == 0
+    return out.double().cpu().numpy()
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("long_rows,longest", [(60, 380), (400, 1000)])  # fewer than 1024 segments, summed in parts; more
+def test_new_product_with_column_tiles_dealt_out(long_rows, longest, half):
+    """Tiles of C dealt out to the XCDs and rows without slots zeroed in the same launch: block segments, tails and empty rows."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR
+    rng = np.random.default_rng(long_rows)
+    m, n, k = 20000, 20000, 128
+    lens = rng.integers(4, 20, m)
+    lens[rng.choice(m, long_rows, replace=False)] = rng.integers(100, longest - 3, long_rows)
+    lens[rng.choice(m, m // 10, replace=False)] = 0
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    row = np.repeat(np.arange(m), lens)
+    col = ((np.arange(len(row)) - rp[row]) * n // np.maximum(lens[row], 1) + rng.integers(0, 20, len(row))).astype(np.int32)  # (ascending, distinct)
+    val, dense = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    dense = round_half(dense) if half else dense
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, config="auto")
+    assert csr.plan is None and not csr.columns_local and csr.longest_row <= longest and (csr.m1 >= 1024) == (long_rows == 400)
+    # where tiles are dealt out: 2, 4 or 8 lines of 128 bytes a row, more than 4 MB, up to 9 MB a tile, few segments, 6 nonzeros a dense row
+    size = n * k * (2 if half else 4)
+    assert size > 4 << 20 and n * 128 <= 9 << 20 and 3 * csr.m1 <= csr.m2 and csr.nnz >= 6 * n
+    want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
+    got = _into_nan(csr, torch.from_numpy(dense).to(DEV, torch.float16 if half else torch.float32), csr.longest_row, csr.call_plans())
+    assert (np.abs(got - want) <= scale * (lens[:, None] + 2) * 2.0 ** -24).all()  # (n + 2 roundings)
+
+
+@pytest.mark.parametrize("kind,k,dtype", [(kind, k, dtype) for kind in ("group", "hub", "hub without scratch", "window")
+                                          for k, dtype in ((64, "f32"), (128, "f16"), (200, "f32"), (32, "f64"), (64, "f64"))])
+def test_new_product_with_plans(kind, k, dtype):
+    """rode_hip_spmm_new into NaN with each kind of plan, in matrices with empty rows: C is what it should be in every row, known
+    longest row or not."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, rode_sddmm_hip
+    rng = np.random.default_rng(k)
+    if kind == "group":  # runs of 100 columns, with other columns beside them
+        m, n = 1000, 1300
+        rows = [np.union1d(np.arange(r, r + 100), rng.choice(n, 12, replace=False)) for r in range(m)]
+    elif kind == "window":
+        m, n = 3000, 3000
+        rows = [np.unique(np.clip(r + rng.integers(-100, 100, 20), 0, n - 1)) for r in range(m)]
+    else:
+        m, n = 2500, 70000
+        rows = [np.unique(rng.integers(0, n, L)) for L in np.where(rng.random(m) < 0.3, rng.integers(540, 600, m), rng.integers(0, 70, m))]
+        for r in (5, 77, 900):
+            rows[r] = np.unique(rng.integers(0, n, 6000))
+    for r in (0, 1, 2, 3, 50, 51, 64, 999, m - 1):  # (among them all rows of a group)
+        rows[r] = rows[r][:0]
+    lens = np.array([len(r) for r in rows])
+    rp, col = np.concatenate(([0], np.cumsum(lens))).astype(np.int32), np.concatenate(rows).astype(np.int32)
+    val, dense = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    dense = round_half(dense) if dtype == "f16" else dense
+    old = RoDeCSR.HUB_MIN_SLABS
+    RoDeCSR.HUB_MIN_SLABS = 1 if "hub" in kind else 10 ** 6
+    try:
+        csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, locality=True)
+    finally:
+        RoDeCSR.HUB_MIN_SLABS = old
+    assert isinstance(csr.plan, {"group": rode_sddmm_hip.GroupPlan, "window": rode_sddmm_hip.WindowPlan}.get(kind, rode_sddmm_hip.HubPlan))
+    if dtype == "f64":
+        csr = csr.with_values(csr.values.double())
+    B = torch.from_numpy(dense).to(DEV, {"f32": torch.float32, "f16": torch.float16, "f64": torch.float64}[dtype])
+    plans, scratch = csr.call_plans(), None
+    if kind == "hub":
+        plans, scratch = rode_sddmm_hip._with_scratch(plans, k, csr.values.element_size(), csr.device)
+        assert scratch.numel() > 0
+    want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
+    for longest in (csr.longest_row, 0):
+        got = _into_nan(csr, B, longest, plans)
+        assert (np.abs(got - want) <= scale * (lens[:, None] + 2) * (2.0 ** -52 if dtype == "f64" else 2.0 ** -24)).all()
