@@ -38,66 +38,17 @@ constexpr int tile_blocks()
     return sizeof(T) == 2 ? 2 : 1;
 }
 
-// Waves per SIMD that the compiler has to leave registers for.  It is told only where it would otherwise miss by a few the
-// number that LDS allows (fp32: width 32 131 registers instead of 128, width 128 262 and 293 instead of 256): a
-// kernel that is told keeps the accumulators out of the second half of the registers, and with halves that
-// costs more than it gives (two heads of width 32 / 64 / 128: 39.6, 59.8, 125 us left alone, 40.8, 63.1, 129 told).
+// Waves per SIMD that the compiler has to leave registers for, in the forward and the row pass.  It is told only where it would
+// otherwise miss by a few the number that LDS allows (row pass in fp32: width 32 136 registers instead of 128, width 128 289
+// instead of 256; forward of width 128 with scores 258): a kernel that is told keeps the accumulators out of the second half of the
+// registers, and with halves that cost more than it gave (forward, two heads of width 32 / 64 / 128: 39.6, 59.8, 125 us left
+// alone, 40.8, 63.1, 129 told; measured with the nonzeros outside the runs one row after the other).  The row pass with halves of width
+// 128 has one workgroup per CU whatever it is told: its 82 432 bytes of LDS are 512 more than half of what there is.
 template <typename T, int D>
 constexpr int tile_waves()
 {
     return sizeof(T) == 2 || D == 64 ? 1 : D == 32 ? 4 : 2;
 }
-
-// The sums over the lane groups (LPR lanes each) of N values per lane, shared out: a lane keeps kLeft of
-// the totals, from number value() on (halving what a lane still has to add at every exchange costs a
-// third of a butterfly per value).
-template <int LPR, int N>
-struct GroupReduce {
-    static constexpr int kGroups = kWave / LPR;
-    static constexpr int kLeft = N / (kGroups < N ? kGroups : N); // totals per lane
-    // (v: the values; in the end the totals in v[0 .. kLeft))
-    static __device__ __forceinline__ void run(float (&v)[N])
-    {
-        if (kGroups >= 2) { // lanes 32 apart
-#pragma unroll
-            for (int j = 0; j < N / 2; ++j) {
-                const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[j]), __float_as_uint(v[N / 2 + j]), false, false);
-                v[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-            }
-        }
-        if (kGroups >= 4) { // 16 apart
-            constexpr int H = N / 4 > 0 ? N / 4 : 1;
-#pragma unroll
-            for (int j = 0; j < H; ++j) {
-                const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[j]), __float_as_uint(v[H + j]), false, false);
-                v[j] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-            }
-        }
-        if (kGroups >= 8) { // 8 apart
-            if constexpr (N >= 8) {
-                const bool upper = __lane_id() & 8;
-                v[0] = (upper ? v[1] : v[0]) + lane_xor8(upper ? v[0] : v[1]);
-            } else {
-                v[0] += lane_xor8(v[0]);
-            }
-        }
-        if (kGroups >= 16) v[0] += lane_xor4(v[0]);
-    }
-    static __device__ __forceinline__ int value(int lane)
-    {
-        int at = 0;
-        if (kGroups >= 2) at += (lane >> 5 & 1) * (N / 2);
-        if (kGroups >= 4) at += (lane >> 4 & 1) * (N / 4);
-        if (kGroups >= 8 && N >= 8) at += (lane >> 3 & 1) * (N / 8);
-        return at;
-    }
-    // does this lane write its totals? (where there are more groups than values several have the same)
-    static __device__ __forceinline__ bool writes(int lane)
-    {
-        if (kGroups >= 16) return N >= 8 ? (lane & 4) == 0 : (lane & 12) == 0;
-        return !(kGroups >= 8 && N < 8) || (lane & 8) == 0;
-    }
-};
 
 constexpr float kLog2e = 1.44269504088896340736f;
 
