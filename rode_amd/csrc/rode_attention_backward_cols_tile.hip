@@ -14,7 +14,8 @@
 // shows as a non-finite sum: the tile is then computed again column by column.
 //
 // Measured (16 384 rows, window 512 and 64 random columns): the pass in fp32, width 64, 89 us with four columns at a time on the
-// vector ALUs, 69 here (along the run 38, 32-bit matrix products and the pairs; outside it 31, 340 MB past the L2s in all).  Training step, one
+// vector ALUs, 69 here (along the run 38, 32-bit matrix products and the pairs; outside it 31; 346 MB past the L2s, the vector
+// ALUs issue 24 % of the time; 2.9 waves per SIMD wait for memory 29 % of theirs and for their turn 57 %).  Training step, one
 // head, fp32 widths 32 / 64 / 128: 159 -> 145, 274 -> 253, 550 -> 491 us; halves 138 -> 127, 193 -> 175, 360 -> 328; four heads of
 // width 64 1079 -> 985, halves 827 -> 745; without random columns 627 -> 521, halves 539 -> 435.  On the way, the pass in fp32: nonzeros
 // outside the run of one column after the other 80; of four columns, g and q together 75; outside first 76 (spills);

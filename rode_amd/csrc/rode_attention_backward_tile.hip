@@ -20,8 +20,10 @@
 // Measured (16 384 rows, window 512 and 64 random columns, width 64, one head in fp32; the kernel's own time): 107 us with the
 // nonzeros outside the run of one row after the other, 95 with those of four rows side by side (TileOutside); training step, us, the other two
 // passes unchanged: fp32 250 -> 244, halves 172 -> 167, width 128 457 -> 422 and 316 -> 302; 20 000 rows of 300 + 96, width 64 430 -> 410.
-// Bound by what passes the L2s (600 MB: 190 MB of values, scores, slots and pairs, the dense rows of eight L2s, a third of those outside the
-// runs) with two waves per SIMD in flight.  Tried: three waves per SIMD (halves spill, step 0.250 ms instead of 0.21; fp32 0.282
+// Bound by latency: 1.7 waves per SIMD (registers: two in fp32, three with halves of width 32, one with halves of width 128, whose LDS leaves
+// one workgroup per CU) wait for memory 42 % of their time and for their turn 33 %; the vector ALUs issue 28 % of it, the address
+// units are busy for 57 %, and 382 MB pass the L2s (4.3 TB/s; 190 MB of them values, scores, slots and pairs).  Tried before the
+// nonzeros outside the run went side by side: three waves per SIMD (halves spill, step 0.250 ms instead of 0.21; fp32 0.282
 // instead of 0.279).
 #include "rode_tile.hpp"
 #include "rode_units.hpp"

@@ -12,14 +12,15 @@
 // (0 * Inf), and shows as a non-finite result: the tile's rows are then computed again, all of them
 // row by row.
 //
-// Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with
-// four rows at a time on the vector ALUs, 0.209 here; eight heads in fp32 0.693 -> 0.39.  Bound by what passes the L2s: 1.2 GB
-// in the 0.209 (values 0.4, operands of eight heads in eight L2s 0.3, the rest dense rows outside the runs, a third of which
-// miss), 3.9 GB out of them.  What was slow on the way: dense rows and values loaded straight into
-// operand layout (adjacent lanes on different rows: 64 clocks of the memory pipe per load, 0.38 ms); the nonzeros outside
-// the run of one row after the other (us, fp32 / halves of width 64, one head: 75 / 36 -> 69 / 34, width 128 164 / 68 -> 131 / 58; 20 000 rows of 300 and 96
-// random columns 121 / 62 -> 97 / 55, width 128 274 / 129 -> 196 / 100; eight heads of halves 222 -> 209).  (The extent of a row outside its run waits in LDS:
-// in registers it cost halves of width 64 a wave per SIMD, 248 us.)
+// Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with four rows at a time on
+// the vector ALUs, 0.206 here; eight heads in fp32 0.693 -> 0.39.  No rate is at its limit: the vector ALUs issue 66 % of the time
+// (a fifth of it the tiles' prologues, once per head), the address units are busy for 63 %, 3.2 GB leave the L2s and 0.62 GB pass
+// them (3.1 TB/s); 2.7 waves per SIMD, which the registers allow, wait for memory 48 % of their time.  What was slow on
+// the way: dense rows and values loaded straight into operand layout (adjacent lanes on different rows: 64 clocks of the
+// memory pipe per load, 0.38 ms); the nonzeros outside the run of one row after the other (us, fp32 / halves of width 64, one head:
+// 75 / 36 -> 69 / 34, width 128 164 / 68 -> 131 / 58; 20 000 rows of 300 and 96 random columns 121 / 62 -> 97 / 55, width 128 274 / 129 ->
+// 196 / 100; eight heads of halves 222 -> 209).  (The extent of a row outside its run waits in LDS: in registers it
+// cost halves of width 64 a wave per SIMD, 248 us.)
 //
 // 32-bit operands use the 32-bit matrix instructions (exact products, 157 TFLOP/s against 79 on the
 // vector ALUs); 16-bit operands split the probabilities into two halves each (TileWeights).  Errors against 64 bits of

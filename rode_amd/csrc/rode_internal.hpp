@@ -97,18 +97,20 @@ hipError_t attention_launch(int nheads, int M, int N, int nnz, int d, const int*
                             PlanRef plan, hipStream_t stream);
 
 constexpr bool attention_tiles_fit(int N, size_t row_bytes) { return N > 0 && (size_t)N * row_bytes < (1ull << 32); }
-// Do the tiles of a group plan go to the tile kernels?  (They address a head's k and v with 32-bit offsets; N = 0:
-// not said, one head.)  Where the other kernel is the one for groups (groups_min, the pass's own figure), always: 4500 rows
-// of 200 columns in fp32, width 32 / 64 / 128: 17 -> 14, 24 -> 18, 70 -> 28 us.  Where it is a wave per row, from 1.5 M nonzeros
-// over all heads on: a tile takes 10 to 45 us however few there are, and rows in no tile are a launch more.  Us row by row -> on tiles, fp32 / halves:
-// 4096 rows of 256 and 64 random columns, a few rows left over, 1.3 M nonzeros, width 64: 25.4 -> 26.5 / 15.7 -> 19.1, 128: 48.9 -> 47.7 / 25.7 -> 24.9; 3000 of
-// 200 and 16, 1.3 M: 28.7 -> 22.0 / 17.6 -> 14.7, 54.4 -> 37.5 / 29.1 -> 19.5, 0.65 M: 16.3 -> 17.6 / 10.7 -> 13.2, 27.1 -> 26.2 / 16.7 -> 15.7.
+// Do the tiles of a group plan go to the tile kernels?  (They address a head's k and v with 32-bit offsets; N = 0: not said, one head.)
+// Where the other kernel is the one for groups (groups_min, the pass's own figure), always: 4500 rows of 200 columns in fp32, width 32 / 64
+// / 128: 17 -> 14, 24 -> 18, 70 -> 28 us.  Where it is a wave per row, from 1.5 M nonzeros over all heads on: a tile takes 10 to 45 us
+// however few there are, and rows in no tile are a launch more.  Us row by row -> on tiles, fp32 / halves: 4096 rows of 256 and 64 random
+// columns, a few rows left over, 1.3 M nonzeros, width 64: 25.4 -> 26.5 / 15.7 -> 19.1, 128: 48.9 -> 47.7 / 25.7 -> 24.9; 3000 of 200 and
+// 16, 1.3 M: 28.7 -> 22.0 / 17.6 -> 14.7, 54.4 -> 37.5 / 29.1 -> 19.5, 0.65 M: 16.3 -> 17.6 / 10.7 -> 13.2, 27.1 -> 26.2 / 16.7 -> 15.7.
 // Where the tiles have all rows (but for fp32 of width 32: 2048 rows of 600 and 96, 1.4 M, 16.3 -> 17.1):
-//   * more than 64 tiles over all heads (with up to 1024 rows every wave of the other kernel has a SIMD of its own), from 0.4 M on:
-//     1280 rows of 400 and 64, width 64 19.5 -> 18.2 / 12.7 -> 10.9, 128 34.2 -> 29.5 / 19.8 -> 15.3; 2000 of 250 12.0 -> 10.7 / 8.5 -> 6.9, 20.4 -> 15.7 / 12.6 -> 8.6;
-//     2800 of 400 23.4 -> 13.9 / 14.7 -> 7.7, 41.7 -> 20.8 / 24.3 -> 10.0; halves of width 32 from 0.6 M: 2000 of 250 and 20 7.0 -> 7.6, 2800 of 250 7.0 -> 6.2;
-//   * fewer, with 700 nonzeros a row, from 0.4 M on but not in fp32 of width 64: 1024 rows of 800 and 64, width 64 22.5 -> 25.9 / 17.1 -> 13.4, 128 48.4 -> 41.6 /
-//     23.9 -> 19.5, halves of width 32 13.1 -> 11.1; of 400 and 64 14.5 -> 18.2 / 11.6 -> 10.8, 26.1 -> 28.7 / 14.5 -> 15.2, 8.5 -> 9.3, training step 68 -> 74 / 64 -> 67.
+//   * more than 64 tiles over all heads (with up to 1024 rows every wave of the other kernel has a SIMD of its own), from 0.4 M on: 1280
+//     rows of 400 and 64, width 64 19.5 -> 18.2 / 12.7 -> 10.9, 128 34.2 -> 29.5 / 19.8 -> 15.3; 2000 of 250 12.0 -> 10.7 / 8.5 -> 6.9,
+//     20.4 -> 15.7 / 12.6 -> 8.6; 2800 of 400 23.4 -> 13.9 / 14.7 -> 7.7, 41.7 -> 20.8 / 24.3 -> 10.0; halves of width 32 from 0.6 M: 2000
+//     of 250 and 20 7.0 -> 7.6, 2800 of 250 7.0 -> 6.2;
+//   * fewer, with 700 nonzeros a row, from 0.4 M on but not in fp32 of width 64: 1024 rows of 800 and 64, width 64 22.5 -> 25.9 / 17.1 ->
+//     13.4, 128 48.4 -> 41.6 / 23.9 -> 19.5, halves of width 32 13.1 -> 11.1; of 400 and 64 14.5 -> 18.2 / 11.6 -> 10.8, 26.1 -> 28.7 /
+//     14.5 -> 15.2, 8.5 -> 9.3, training step 68 -> 74 / 64 -> 67.
 inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads, int N, long long nnz, size_t row_bytes, bool halves)
 {
     if (plan.groups == nullptr || plan.group_counts == nullptr || plan.group_counts[1] <= 0 || plan.group_counts[3] <= 0) return false;

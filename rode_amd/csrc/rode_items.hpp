@@ -492,23 +492,25 @@ __host__ __device__ inline size_t hub_plan_ints(int M, int dense_rows, int nnz, 
 
 __host__ __device__ inline int hub_groups(int slabs, int merge) { return (slabs + merge - 1) / merge; }
 
-// What a call takes of a hub plan: `rows` of its rows (all, or the long ones), and how many slabs together.  A piece should hold
-// enough nonzeros that reading its columns, its last step of 64 and, in SpMM, its partial row are little beside its dense rows,
-// and enough rows should share a slab.  Counted in nonzeros of a row per piece (in brackets) at 4 MB of the operand, an XCD's L2:
+// What a call takes of a hub plan: `rows` of its rows (all, or the long ones), and how many slabs together.  A piece should hold enough
+// nonzeros that reading its columns, its last step of 64 and, in SpMM, its partial row are little beside its dense rows, and enough rows
+// should share a slab.  Counted in nonzeros of a row per piece (in brackets) at 4 MB of the operand, an XCD's L2:
 //   * all rows from 18 on, in SDDMM with a width that is no multiple of its slabs from 28 on, else the long ones.  us, long ones -> all,
-//     power law (p) or 8 nonzeros a row and thousands of rows of 512 to 2000 (s), dense rows x width of SDDMM: p 200 K x 256 659 -> 627 (49),
-//     p 330 K x 512 2173 -> 2264 (18), s 262 K x 256 3393 -> 2477 (23), x 512 6864 -> 8511 (12), s 500 K x 128 1957 -> 1526 (32), x 256 3953 -> 4149 (16);
-//     no multiple: s 262 K x 160 2459 -> 2313 (35), x 192 2775 -> 2994 (23), s 100 K x 320 3914 -> 2935 (29), s 500 K x 160 3007 -> 3870 (25);
-//   * in SpMM also only with 600 rows: 314 of p 70 K x 64 67 -> 79, 412 of p 100 K x 128 halves 105 -> 108, x 320 halves 227 -> 254,
-//     928 of p 200 K x 128 361 -> 325, 2100 of s 100 K x 64 136 -> 109;
+//     power law (p) or 8 nonzeros a row and thousands of rows of 512 to 2000 (s), dense rows x width of SDDMM: p 200 K x 256 659 -> 627
+//     (49), p 330 K x 512 2173 -> 2264 (18), s 262 K x 256 3393 -> 2477 (23), x 512 6864 -> 8511 (12), s 500 K x 128 1957 -> 1526 (32), x
+//     256 3953 -> 4149 (16); no multiple: s 262 K x 160 2459 -> 2313 (35), x 192 2775 -> 2994 (23), s 100 K x 320 3914 -> 2935 (29), s 500
+//     K x 160 3007 -> 3870 (25);
+//   * in SpMM also only with 600 rows: 314 of p 70 K x 64 67 -> 79, 412 of p 100 K x 128 halves 105 -> 108, x 320 halves 227 -> 254, 928 of
+//     p 200 K x 128 361 -> 325, 2100 of s 100 K x 64 136 -> 109;
 //   * 2 MB instead of 4 in operands of up to 320 MB with (40) at that.  SDDMM / SpMM, 2 -> 4 MB: p 200 K x 32 95 / 112 -> 105 / 117 (185),
-//     x 128 310 / 325 -> 323 / 345 (49), p 330 K x 128 496 / 512 -> 490 / 507 (36), s 262 K x 64 517 / 601 -> 482 / 499 (47), x 128 1310 / 1201 -> 919 / 981 (23);
+//     x 128 310 / 325 -> 323 / 345 (49), p 330 K x 128 496 / 512 -> 490 / 507 (36), s 262 K x 64 517 / 601 -> 482 / 499 (47), x 128 1310 /
+//     1201 -> 919 / 981 (23);
 //   * SpMM counts the bytes of the column tile that a grid row works on, as long as that leaves 2048 pieces: s 180 K x 512 2827 -> 2024,
 //     halves 2436 -> 1182;
 //   * the partial rows of SpMM with all rows take no more than eight times the memory of a dense operand of 32 bits (100 000 rows of 1200
 //     nonzeros in 262 K columns: 6.4 M pieces, 3.3 GB at width 128 beside an operand of 134 MB; the long rows have few).
-// With every row, and 2 MB up to 320 MB, wide calls were slower than with the long rows alone: SDDMM s 262 K x 160 2435 -> 4797, x 512 6864 -> 8443, SpMM
-// s 262 K x 512 halves 3494 -> 6179, s 500 K x 1024 halves 8684 -> 17715.
+// With every row, and 2 MB up to 320 MB, wide calls were slower than with the long rows alone: SDDMM s 262 K x 160 2435 -> 4797, x 512 6864
+// -> 8443, SpMM s 262 K x 512 halves 3494 -> 6179, s 500 K x 1024 halves 8684 -> 17715.
 struct HubRows {
     int rows = 0, min_len = 0; // 0: the call goes without the plan
     int merge = 1, mean = 0;   // ..., nonzeros of a row

@@ -47,12 +47,13 @@ namespace {
 // segments on the difference is below 1 %.
 constexpr int kOwnedRowSlots = 1024;
 constexpr int kOwnedMinSegments = 1024;
-// Where the caller knows that no row is longer than this, a matrix of fewer segments has its rows summed whole as well: a wave has no
-// more than six steps to do, every row is stored, and C is not cleared beforehand (us, cleared and added to -> stored, widths 32 / 128 / 128 of
-// halves: 512 x 512 of 16 to 64 nonzeros 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3 -> 15.0, 250 K 150 -> 143; longest
-// row 168 7.7 / 10.6 / 12.0 -> 5.7 / 6.0 / 5.7, 227 7.8 / 9.8 / 10.7 -> 5.7 / 6.4 / 5.7, 338 7.5 / 8.7 / 9.0 -> 5.8 / 7.3 / 6.7, 471 7.9 / 9.9 / 10.4 -> 5.8 / 9.1 / 7.8,
-// 502 8.4 / 8.4 / 8.2 -> 5.9 / 9.4 / 8.2, 1001 7.4 / 8.5 / 7.9 -> 8.0 / 15.0 / 12.6).
-// Each 64 slots of such a row have a sum of their own, as the row's segments had: one chain over all of a row had up to 1.7 times their error.
+// Where the caller knows that no row is longer than this, a matrix of fewer segments has its rows summed whole as well: a wave has no more
+// than six steps to do, every row is stored, and C is not cleared beforehand (us, cleared and added to -> stored, widths 32 / 128 / 128 of
+// halves: 512 x 512 of 16 to 64 nonzeros 8.2 - 9.8 -> 6.0 - 7.0, 8000 of 24 x 128 14.7 -> 10.3, of halves 13.2 -> 6.5, 40 K of 16 x 64 17.3
+// -> 15.0, 250 K 150 -> 143; longest row 168 7.7 / 10.6 / 12.0 -> 5.7 / 6.0 / 5.7, 227 7.8 / 9.8 / 10.7 -> 5.7 / 6.4 / 5.7, 338 7.5 / 8.7 /
+// 9.0 -> 5.8 / 7.3 / 6.7, 471 7.9 / 9.9 / 10.4 -> 5.8 / 9.1 / 7.8, 502 8.4 / 8.4 / 8.2 -> 5.9 / 9.4 / 8.2, 1001 7.4 / 8.5 / 7.9 -> 8.0 /
+// 15.0 / 12.6). Each 64 slots of such a row have a sum of their own, as the row's segments had: one chain over all of a row had up to 1.7
+// times their error.
 constexpr int kShortRowSlots = 384;
 // Without the promise the block kernel may still merge the short segments of a row that
 // the list it was given holds, when there are this many of them.
@@ -425,12 +426,12 @@ spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners
                                    C, plan);
 }
 
-// The rows of C without slots, which are in neither list, where nobody cleared C: 64 at a time to the waves, whose lanes zero the
-// tile of several rows at once, 16 bytes each.  (A matrix may be mostly such rows: in waves of 256 that took one after the other,
-// 100 K x 128 with 50 rows that are not empty took 29.4 us instead of 12.8 with a clearing launch, 1 M x 32 34 instead of 22.)
-// (Rows of more than 1024 slots, which several waves add to, still need the launch before: with a workgroup for each of them in here
-// spmm of 65 K x 128, ten such rows, took 57.8 us instead of 60.0, but the registers of that cost the kernel a wave per SIMD: 40 K rows of 32 x 64
-// 38.6 -> 43.2, lognormal 100 K of 16 x 32 30.4 -> 35.3.)
+// The rows of C without slots, which are in neither list, where nobody cleared C: 64 at a time to the waves, whose lanes zero the tile of
+// several rows at once, 16 bytes each.  (A matrix may be mostly such rows: in waves of 256 that took one after the other, 100 K x 128 with
+// 50 rows that are not empty took 29.4 us instead of 12.8 with a clearing launch, 1 M x 32 34 instead of 22.) (Rows of more than 1024
+// slots, which several waves add to, still need the launch before: with a workgroup for each of them in here spmm of 65 K x 128, ten such
+// rows, took 57.8 us instead of 60.0, but the registers of that cost the kernel a wave per SIMD: 40 K rows of 32 x 64 38.6 -> 43.2,
+// lognormal 100 K of 16 x 32 30.4 -> 35.3.)
 template <typename A, int TN, bool EDGE>
 __device__ __forceinline__ void spmm_empty_rows(int bid, int nblocks, int tile, int rows, int n, const int* __restrict__ row_ptr, A* __restrict__ C)
 {
