@@ -201,10 +201,13 @@ def test_pieces_shared_by_waves(hubs, k, half):
     assert float(err[cond <= 100].max(initial=0.0)) <= tol
 
 
+@pytest.mark.parametrize("way", ["streams", "threads", "graph"])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.float64])
-def test_calls_on_one_matrix_from_two_streams(dtype):
-    """Overlapping products of one matrix have partial rows of their own: every result is the one that the call gives alone.
+def test_calls_on_one_matrix_from_two_streams(dtype, way):
+    """Overlapping products of one matrix have partial rows of their own - on two streams, from two threads on one, and in the replays of
+    a captured graph: every result is the one that the call gives alone.
     (Rows of the plan are summed in one order whatever else runs, so the bits are equal.)"""
+    import threading
     from gpu_common import DEV, make_csr
     from rode_amd import RoDeCSR, rode_sddmm_hip, rode_spmm
     rng = np.random.default_rng(17)
@@ -229,13 +232,33 @@ def test_calls_on_one_matrix_from_two_streams(dtype):
         return rode_spmm(csr, B)
 
     alone = [product(B)[where] for B in operands]
-    streams = [torch.cuda.Stream() for _ in operands]
     torch.cuda.synchronize()
     got = [[], []]
-    for _ in range(8):
-        for i, (s, B) in enumerate(zip(streams, operands)):
-            with torch.cuda.stream(s):
-                got[i].append(product(B)[where])
+    if way == "streams":
+        streams = [torch.cuda.Stream() for _ in operands]
+        for _ in range(8):
+            for i, (s, B) in enumerate(zip(streams, operands)):
+                with torch.cuda.stream(s):
+                    got[i].append(product(B)[where])
+    elif way == "threads":
+        def calls(i):
+            got[i].extend(product(operands[i])[where] for _ in range(8))
+        threads = [threading.Thread(target=calls, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert len(got[0]) == len(got[1]) == 8
+    else:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            captured = [product(B)[where] for B in operands]
+        for _ in range(4):
+            graph.replay()
+            got[0].append(product(operands[0])[where])  # (the program's own work between the replays)
+            for g, c in zip(got, captured):
+                g.append(c.clone())
+            torch.cuda.synchronize()
     torch.cuda.synchronize()
     assert not torch.equal(*alone)
     assert all(torch.equal(a, alone[i]) for i in range(2) for a in got[i])
