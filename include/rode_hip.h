@@ -264,6 +264,10 @@ size_t rode_hip_group_plan_bytes(int M);
 int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_indices, void* d_plan, size_t plan_bytes,
                         int* h_counts, void* stream);
 
+/* The same, and (h_tile_fours not NULL) what rode_hip_plans.tile_fours says of the plan. */
+int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_column_indices, void* d_plan, size_t plan_bytes,
+                              int* h_counts, int* h_tile_fours, void* stream);
+
 /*
  * The plans of one matrix, as the *_planned entry points take them: a struct in HOST
  * memory, read during the call only.  Every member may be NULL / 0; a struct of zeros (or
@@ -300,6 +304,10 @@ int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_ind
  *                         unused where the window kernels do not pay (short rows, a last round of few
  *                         chunks), and dealing tiles out depends on how often a dense row is used.
  *                         Costs time at worst.
+ *   tile_fours            0, or what rode_hip_group_plan_fours said of the group plan: the columns that every four
+ *                         neighbouring tiles cover between them, over the most that four do (a sliding window: about
+ *                         a quarter of the tiles).  With it the attention kernels for halves take four
+ *                         tiles at a time where that pays.  Costs time at worst.
  * Same results as without a plan, up to the order of the fp32 additions inside a row.
  */
 typedef struct rode_hip_plans {
@@ -315,6 +323,7 @@ typedef struct rode_hip_plans {
     int seg_length;
     int columns_local;
     int nonzeros;
+    int tile_fours;
 } rode_hip_plans;
 
 /* rode_hip_spmm_ex with plans. */

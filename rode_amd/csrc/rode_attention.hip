@@ -339,7 +339,7 @@ hipError_t launch_rows(int nheads, int M, int N, int nnz, const int* row_ptr, co
         groups_left -= plan.group_counts[3] * (kTileRows / kGroupRows);
         rows_left -= plan.group_counts[3] * kTileRows;
         const hipError_t e = attention_tiles_launch<T>(nheads, M, N, nnz, D, row_ptr, col, val, q, k, v, scale, out, probs,
-                                                       reinterpret_cast<float*>(stats), plan.groups, stream);
+                                                       reinterpret_cast<float*>(stats), plan.groups, plan.tile_fours, stream);
         if (e != hipSuccess) return e;
     }
     const bool grouped = groups_left >= attention_groups_min<T>();

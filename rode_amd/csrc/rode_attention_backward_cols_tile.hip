@@ -49,8 +49,8 @@ attention_backward_cols_tile_kernel(int n_tiles, const RowTile* __restrict__ til
                                     float* __restrict__ dv, HeadStrides heads)
 {
     constexpr int NB = D / 16;
-    using GStage = TileStage<float, D, false, kColsStep>;
-    using QStage = TileStage<T, D, false, kColsStep>;
+    using GStage = TileStage<float, D, kAcross, kColsStep>;
+    using QStage = TileStage<T, D, kAcross, kColsStep>;
     using Square = TileSquare<float>;
     // Per wave: staged rows of g and q and the step's p and dz; then the wave's sums of dv and dk in the same place, and behind
     // them rows and weights of nonzeros outside the run.  (Width 64: 40 KB, four workgroups per CU.)

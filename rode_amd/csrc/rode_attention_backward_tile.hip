@@ -80,8 +80,8 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
 {
     constexpr int NB = D / 16, PAD = D + 4, NT = tile_blocks<T>(), kStep = 16 * NT;
     constexpr bool kHalf = std::is_same<T, __half>::value;
-    using VStage = TileStage<T, D, true>;  // (v meets g along its elements, k is summed across)
-    using KStage = TileStage<T, D, false>;
+    using VStage = TileStage<T, D, kAlong>;  // (v meets g along its elements, k is summed across)
+    using KStage = TileStage<T, D, tile_columns<T>()>;
     // Per wave: staged rows of v and k, the values and what the forward pass kept of a step.  Then staging for the nonzeros outside
     // the runs, then the wave's partial sums and behind them the sums of its four rows outside their runs.
     constexpr int kPart = kTileRows * PAD, kStageFloats = 2 * VStage::kBytes / 4 + 2 * TileSquare<T>::kFloats;
@@ -332,8 +332,7 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
             TileWeights<T> weights;
             weights.set(dz, range.factor());
             TileCols<T, D> k_cols;
-#pragma unroll
-            for (int j = 0; j < 4 * NT; ++j) k_cols.load(j, KStage::across(lds_k, 16 * (j / 4) + 4 * gq + j % 4, n));
+            k_cols.load(lds_k, lane);
             k_cols.accumulate(weights, acc);
             wave_lds_sync();
         }
@@ -347,7 +346,10 @@ attention_backward_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, c
     float* part = shared[wave];
     const float back = range.back();
 #pragma unroll
-    for (int e = 0; e < D / 4; ++e) part[n * PAD + (D / 4) * gq + e] = again ? 0.f : acc[e % NB][e / NB] * back;
+    for (int c = 0; c < NB; ++c) {
+        const f32x4 sums = TileCols<T, D>::sums(acc, c);
+        *reinterpret_cast<f32x4*>(part + n * PAD + TileCols<T, D>::at(c, gq)) = again ? kNothing : sums * back;
+    }
     __syncthreads();
     const int r = threadIdx.x / 16, e0 = threadIdx.x % 16 * NB;
     float o[NB];

@@ -189,16 +189,27 @@ size_t rode_hip_hub_workspace_bytes(const int* h_hub_counts, int n, int elem_byt
 
 size_t rode_hip_group_plan_bytes(int M) { return M < 0 ? 0 : rode::group_plan_ints(M) * sizeof(int); }
 
-int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_indices, void* d_plan, size_t plan_bytes,
-                        int* h_counts, void* stream)
+int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_column_indices, void* d_plan, size_t plan_bytes,
+                              int* h_counts, int* h_tile_fours, void* stream)
 {
     if (M < 0 || !d_plan || !aligned16(d_plan) || !h_counts || plan_bytes < rode_hip_group_plan_bytes(M))
         return hipErrorInvalidValue;
     if (M > 0 && (!d_row_offsets || !d_column_indices)) return hipErrorInvalidValue;
+    int fours[3] = {0, 0, 0};
     hipError_t e = rode::group_plan_launch(M, d_row_offsets, d_column_indices, static_cast<int*>(d_plan), as_stream(stream));
     if (e == hipSuccess) e = hipMemcpyAsync(h_counts, d_plan, 4 * sizeof(int), hipMemcpyDeviceToHost, as_stream(stream));
-    if (e == hipSuccess) e = hipStreamSynchronize(as_stream(stream));
+    if (e == hipSuccess && h_tile_fours)
+        e = hipMemcpyAsync(fours, static_cast<int*>(d_plan) + rode::group_fours_at(M), sizeof(fours), hipMemcpyDeviceToHost, as_stream(stream));
+    const hipError_t waited = hipStreamSynchronize(as_stream(stream)); // (also after an error: the copies are into memory of this call)
+    if (e == hipSuccess) e = waited;
+    if (e == hipSuccess && h_tile_fours) *h_tile_fours = fours[0] == 0 && fours[2] > 0 ? fours[1] / fours[2] : 0;
     return e;
+}
+
+int rode_hip_group_plan(int M, const int* d_row_offsets, const int* d_column_indices, void* d_plan, size_t plan_bytes,
+                        int* h_counts, void* stream)
+{
+    return rode_hip_group_plan_fours(M, d_row_offsets, d_column_indices, d_plan, plan_bytes, h_counts, nullptr, stream);
 }
 
 namespace {
@@ -219,6 +230,7 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
         if (p->group_counts[3] < 0 || p->group_counts[3] * (rode::kTileRows / rode::kGroupRows) > p->group_counts[1]) return false;
         plan.groups = static_cast<const int*>(p->groups);
         plan.group_counts = p->group_counts;
+        plan.tile_fours = p->tile_fours;
     }
     if (p->hub) {
         // a hub plan needs its header on the host, and excludes a locality plan (the window
@@ -429,6 +441,7 @@ static bool group_plan_only(const rode_hip_plans* plans, int rows, rode::PlanRef
     rode_hip_plans only_groups = {};
     only_groups.groups = plans->groups;
     only_groups.group_counts = plans->group_counts;
+    only_groups.tile_fours = plans->tile_fours;
     return plan_ref(&only_groups, 0, plan) && plan.group_counts[0] == rode::row_groups(rows);
 }
 

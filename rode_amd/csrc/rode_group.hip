@@ -17,7 +17,8 @@
 //                       the group's nonzeros, and the runs start and end within 255 columns
 //                       of each other;
 //   group_tiles_kernel  per four groups: whether their 16 rows make a tile for the attention
-//                       kernels on the matrix cores (rode_tile.hpp).
+//                       kernels on the matrix cores (rode_tile.hpp);
+//   group_fours_kernel  per four tiles: whether they lie together.
 #include "rode_items.hpp"
 #include "rode_internal.hpp"
 
@@ -144,6 +145,27 @@ group_tiles_kernel(int tiles, const RowGroup* __restrict__ groups, const int* __
     if (keep) atomicAdd(plan + 3, 1);
 }
 
+// Four neighbouring tiles a thread: do they lie together - between them no more than half as many columns again as the widest of
+// them - and how many columns is that (attention_wide_kernel walks them for all four)?
+__global__ void __launch_bounds__(kWgThreads)
+group_fours_kernel(int tiles, const RowTile* __restrict__ tile, int* __restrict__ fours)
+{
+    const int first = (blockIdx.x * kWgThreads + threadIdx.x) * 4;
+    if (first >= tiles) return;
+    int lo = 0x7fffffff, hi = 0, widest = 0;
+    for (int t = first; t < min(first + 4, tiles); ++t) {
+        const RowTile d = tile[t];
+        if (d.hi > d.lo) lo = min(lo, d.lo), hi = max(hi, d.hi), widest = max(widest, d.hi - d.lo);
+    }
+    if (widest == 0) return;
+    if (2ll * (hi - lo) > 3ll * widest) {
+        atomicAdd(fours, 1);
+    } else {
+        atomicAdd(fours + 1, hi - lo);
+        atomicMax(fours + 2, hi - lo);
+    }
+}
+
 __global__ void group_header_kernel(int M, int groups, int* __restrict__ plan)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
@@ -151,6 +173,8 @@ __global__ void group_header_kernel(int M, int groups, int* __restrict__ plan)
         plan[1] = 0;
         plan[2] = M; // rows outside the groups with a run: counted down as groups are kept
         plan[3] = 0; // tiles: counted up
+        int* fours = plan + group_fours_at(M);
+        fours[0] = fours[1] = fours[2] = fours[3] = 0;
     }
 }
 
@@ -165,10 +189,12 @@ hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* pla
         group_runs_kernel<<<(M + kWavesPerWg - 1) / kWavesPerWg, kWgThreads, 0, stream>>>(M, row_ptr, col, runs);
         group_desc_kernel<<<(groups + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(groups, row_ptr, runs, plan);
         const int tiles = row_tiles(M);
-        if (tiles > 0)
+        if (tiles > 0) {
+            RowTile* out = reinterpret_cast<RowTile*>(plan + group_tiles_at(M));
             group_tiles_kernel<<<(tiles + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(
-                tiles, reinterpret_cast<const RowGroup*>(plan + kGroupHeaderInts), runs,
-                reinterpret_cast<RowTile*>(plan + group_tiles_at(M)), plan);
+                tiles, reinterpret_cast<const RowGroup*>(plan + kGroupHeaderInts), runs, out, plan);
+            group_fours_kernel<<<(tiles + 4 * kWgThreads - 1) / (4 * kWgThreads), kWgThreads, 0, stream>>>(tiles, out, plan + group_fours_at(M));
+        }
     }
     return hipGetLastError();
 }

@@ -42,6 +42,7 @@ struct PlanRef {
     // A group plan (rode_group.hip) and the host copy of its four header ints (required with it).
     const int* groups = nullptr;
     const int* group_counts = nullptr;
+    int tile_fours = 0;         // of its tiles (rode_hip_plans)
     // SDDMM: the RODE_SPMM_ONLY_* bits of the call (SpMM carries them in its flags)
     int only = 0;
     // SpMM: rows of the dense operand as the caller says (0: not said), and (set by spmm_launch) into how
@@ -129,7 +130,7 @@ inline bool attention_uses_tiles(const PlanRef& plan, int groups_min, int nheads
 template <typename T>
 hipError_t attention_tiles_launch(int nheads, int M, int N, int nnz, int d, const int* row_ptr, const int* col, const float* val,
                                   const T* q, const T* k, const T* v, float scale, float* out, float* probs, float* row_stats,
-                                  const int* plan, hipStream_t stream);
+                                  const int* plan, int plan_fours, hipStream_t stream);
 
 // Gradient of the attention kernel (rode_attention_backward.hip): the row pass over the
 // pattern, then the column pass over the transposed pattern (plan: only a group plan is used,

@@ -14,10 +14,12 @@
 //     columns 4 gq + i of a 16-column block.  A row's statistics are then one number per lane, its
 //     values and scores are 16 consecutive bytes in memory, and the probabilities are operand B of
 //     the next product as they are (k slot (gq, t, i) stands for column 16 t + 4 gq + i);
-//   * the weighted sum too: O^T = V^T P^T.  Operand A has a lane per 16th of the elements: lane m
-//     loads the D / 16 consecutive elements from (D / 16) m of each of its eight columns' rows
-//     (16 lanes, a whole row), product nb takes element nb of each.  Lane (n, gq) ends up with the
-//     D / 4 consecutive elements from (D / 4) gq of row n: element e is acc[e % (D / 16)][e / (D / 16)].
+//   * the weighted sum too: O^T = V^T P^T.  32-bit operands: operand A has a lane per 16th of the elements, lane m
+//     loads the D / 16 consecutive elements from (D / 16) m of each of its four columns' rows
+//     (16 lanes, a whole row), product nb takes element nb of each, and lane (n, gq) ends up with the
+//     D / 4 consecutive elements from (D / 4) gq of row n.  Halves: LDS transposes on the way out (TileCols), product nb
+//     takes elements 16 nb .. 16 nb + 15, and lane (n, gq) ends up with elements 16 nb + 4 gq + i.  TileCols::sums and at
+//     say which, four consecutive elements at a time.
 #pragma once
 #include "rode_items.hpp"
 #include "rode_device.hpp"
@@ -43,7 +45,8 @@ constexpr int tile_blocks()
 // instead of 256; forward of width 128 with scores 258): a kernel that is told keeps the accumulators out of the second half of the
 // registers, and with halves that cost more than it gave (forward, two heads of width 32 / 64 / 128: 39.6, 59.8, 125 us left
 // alone, 40.8, 63.1, 129 told; measured with the nonzeros outside the runs one row after the other).  The row pass with halves of width
-// 128 has one workgroup per CU whatever it is told: its 82 432 bytes of LDS are 512 more than half of what there is.
+// 128 has one workgroup per CU whatever it is told: its 82 432 bytes of LDS are 512 more than half of what there is; the forward of
+// that width, 260 registers by itself, is told two (attention_tile_kernel).
 template <typename T, int D>
 constexpr int tile_waves()
 {
@@ -106,9 +109,16 @@ __device__ __forceinline__ f32x4 mma_rows(const TileRow<T, D>& a, const TileRow<
 // The dense rows of a step on their way through LDS to operand A: loaded in order (every load 1024 consecutive
 // bytes), stored, and read back along or across their elements.  Where 16 bytes are put spreads the
 // 16 lanes that LDS serves together (lanes 0-3, 12-15, 20-27 and their like) over all of its banks:
-//   ALONG: chunk c of row r at position c ^ f(r) of the row (16 rows are read at one c);
-//   else (across, TileCols): the rows of lanes 16 apart, four apart in r, in different parts of 256 bytes.
-template <typename T, int D, bool ALONG, int ROWS = 16 * tile_blocks<T>()>
+//   kAlong: chunk c of row r at position c ^ f(r) of the row (16 rows are read at one c);
+//   kAcross (TileCols, 32-bit sums): the rows of lanes 16 apart, four apart in r, in different parts of 256 bytes;
+//   kTransposed (TileCols, halves): 32 bytes each of eight rows are read together, from eight parts of 256 bytes.
+enum TileRead { kAlong, kAcross, kTransposed };
+template <typename T>
+constexpr TileRead tile_columns() // how operand A of the weighted sums is read
+{
+    return sizeof(T) == 2 ? kTransposed : kAcross;
+}
+template <typename T, int D, TileRead READ, int ROWS = 16 * tile_blocks<T>()>
 struct TileStage {
     static constexpr int kPerRow = D * (int)sizeof(T) / 16; // 16-byte chunks of a row
     static constexpr int kLoads = ROWS * kPerRow / kWave;
@@ -117,9 +127,12 @@ struct TileStage {
     u32x4 x[kLoads];
     static __device__ __forceinline__ int place(int row, int c)
     {
-        if constexpr (ALONG) {
+        if constexpr (READ == kAlong) {
             const int f = kPerRow == 4 ? (-(row >> 2)) & 3 : row & (kPerRow < 16 ? kPerRow - 1 : 15);
             return row * kPerRow + (c ^ f);
+        } else if constexpr (READ == kTransposed) {
+            constexpr int kRows = kPerRow < 16 ? 16 / kPerRow : 1, kPairs = kPerRow < 16 ? kPerRow / 2 : 8; // (rows in 256 bytes; what f goes up to)
+            return row * kPerRow + (c ^ 2 * (row / kRows & (kPairs - 1)));
         } else {
             constexpr int kParts = kPerRow < 16 ? 16 / kPerRow : 1; // rows in 256 bytes
             return (row ^ ((row >> 2) & (kParts - 1))) * kPerRow + c;
@@ -156,6 +169,16 @@ struct TileStage {
         constexpr int kElems = 16 / (int)sizeof(T), NB = D / 16;
         return reinterpret_cast<const T*>(lds + place(r, NB * n / kElems)) + NB * n % kElems;
     }
+    // halves, transposed: element 16 nb + lane % 16 of the rows 16 t + 4 (lane / 16) .. + 3.  (ds_read_b64_tr_b16: of every 16
+    // lanes lane 4 r + p names four halves; lane m gets the m-th of the 16 that lanes 4 r .. 4 r + 3 name, for r = 0 .. 3.)
+    static __device__ __forceinline__ uint2 transposed(const u32x4* lds, int t, int nb, int lane)
+    {
+        static_assert(READ == kTransposed && sizeof(T) == 2, "16-bit elements placed for it");
+        typedef short s16x4 __attribute__((ext_vector_type(4)));
+        const int row = 16 * t + lane / 16 * 4 + lane % 16 / 4, part = lane % 4;
+        const T* at = reinterpret_cast<const T*>(lds + place(row, 2 * nb + part / 2)) + part % 2 * 4;
+        return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(at)));
+    }
 };
 
 // One number per (row of the tile, column) of a step, between the layout that memory wants
@@ -178,14 +201,16 @@ template <>
 struct TileWeights<__half> {
     static constexpr float kScale = 0x1p15f; // probabilities are taken times that
     f16x8 hi, lo;
-    // the weights p times a power of two (both parts by v_fma_mix: a product, a difference and a rounding in one)
+    // the weights p times a power of two (the small part by v_fma_mix: a product, a difference and a rounding in one)
     __device__ __forceinline__ void set(const float (&p)[8], float scale)
     {
+        u32x4 pairs;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            hi[j] = (_Float16)(p[j] * scale);
-            lo[j] = (_Float16)fmaf(p[j], scale, -(float)hi[j]);
-        }
+        for (int j = 0; j < 8; j += 2) pairs[j / 2] = __builtin_bit_cast(unsigned, f16x2{(_Float16)(p[j] * scale), (_Float16)(p[j + 1] * scale)});
+        asm volatile("" : "+v"(pairs)); // (rounded once, in pairs: the compiler would round each again for the difference)
+        hi = __builtin_bit_cast(f16x8, pairs);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) lo[j] = (_Float16)fmaf(p[j], scale, -(float)hi[j]);
     }
 };
 template <>
@@ -207,38 +232,39 @@ template <typename T, int D>
 struct TileCols;
 template <int D>
 struct TileCols<__half, D> {
-    static constexpr int kBlocks = D / 16, kWords = D / 32;
-    uint32_t w[8][kWords];
-    __device__ __forceinline__ void load(int j, const __half* at)
+    static constexpr int kBlocks = D / 16;
+    using Stage = TileStage<__half, D, kTransposed>;
+    uint2 w[kBlocks][2];
+    __device__ __forceinline__ void load(const u32x4* lds, int lane)
     {
-        if constexpr (kWords == 1) {
-            w[j][0] = *reinterpret_cast<const uint32_t*>(at);
-        } else if constexpr (kWords == 2) {
-            const uint2 x = *reinterpret_cast<const uint2*>(at);
-            w[j][0] = x.x, w[j][1] = x.y;
-        } else {
-            const uint4 x = *reinterpret_cast<const uint4*>(at);
-            w[j][0] = x.x, w[j][1] = x.y, w[j][2] = x.z, w[j][3] = x.w;
-        }
+#pragma unroll
+        for (int nb = 0; nb < kBlocks; ++nb)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) w[nb][t] = Stage::transposed(lds, t, nb, lane);
     }
     __device__ __forceinline__ void accumulate(const TileWeights<__half>& p, f32x4 (&acc)[kBlocks]) const
     {
 #pragma unroll
         for (int nb = 0; nb < kBlocks; ++nb) {
-            const uint32_t select = nb % 2 ? 0x07060302u : 0x05040100u; // the upper / lower halves of two rows
-            const uint4 a = make_uint4(__builtin_amdgcn_perm(w[1][nb / 2], w[0][nb / 2], select),
-                                       __builtin_amdgcn_perm(w[3][nb / 2], w[2][nb / 2], select),
-                                       __builtin_amdgcn_perm(w[5][nb / 2], w[4][nb / 2], select),
-                                       __builtin_amdgcn_perm(w[7][nb / 2], w[6][nb / 2], select));
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.lo, acc[nb], 0, 0, 0);
-            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), p.hi, acc[nb], 0, 0, 0);
+            const f16x8 a = __builtin_bit_cast(f16x8, make_uint4(w[nb][0].x, w[nb][0].y, w[nb][1].x, w[nb][1].y));
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p.lo, acc[nb], 0, 0, 0);
+            acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, p.hi, acc[nb], 0, 0, 0);
         }
     }
+    // the c'th four consecutive elements of this lane's sums, and where they are in the row
+    static __device__ __forceinline__ f32x4 sums(const f32x4 (&acc)[kBlocks], int c) { return acc[c]; }
+    static __device__ __forceinline__ int at(int c, int gq) { return 16 * c + 4 * gq; }
 };
 template <int D>
 struct TileCols<float, D> {
     static constexpr int kBlocks = D / 16;
+    using Stage = TileStage<float, D, kAcross>;
     float x[4][kBlocks];
+    __device__ __forceinline__ void load(const u32x4* lds, int lane)
+    {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) load(j, Stage::across(lds, lane / 16 * 4 + j, lane % 16));
+    }
     __device__ __forceinline__ void load(int j, const float* at)
     {
         if constexpr (kBlocks == 2) {
@@ -274,6 +300,14 @@ struct TileCols<float, D> {
             for (int i = 0; i < kAtOnce; ++i) acc[b + i] += sum[i];
         }
     }
+    static __device__ __forceinline__ f32x4 sums(const f32x4 (&acc)[kBlocks], int c)
+    {
+        f32x4 e;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) e[x] = acc[(4 * c + x) % kBlocks][(4 * c + x) / kBlocks];
+        return e;
+    }
+    static __device__ __forceinline__ int at(int c, int gq) { return D / 4 * gq + 4 * c; }
 };
 
 template <int NB>

@@ -271,9 +271,12 @@ class GroupPlan:
     """Group plan of one pattern (``rode_hip_group_plan``): the device array and a host copy
     of its header ``[groups, groups with a shared run, rows outside those groups, tiles]``."""
 
-    def __init__(self, data, counts):
+    tile_fours = 0  # (of a plan from before there was this figure)
+
+    def __init__(self, data, counts, tile_fours=0):
         self.data = data
         self.counts = counts
+        self.tile_fours = tile_fours
         self._header = (ctypes.c_int * 4)(*counts)
         self.rows = None  # (a matrix has one kind of plan)
 
@@ -299,10 +302,11 @@ def group_plan(row_offsets, column_indices, m):
     nbytes = lib.rode_hip_group_plan_bytes(m)
     with torch.cuda.device(dev):
         data = torch.empty(nbytes // 4, dtype=torch.int32, device=dev)
-        counts = (ctypes.c_int * 4)()
-        _lib.check(lib.rode_hip_group_plan(m, row_offsets.data_ptr(), column_indices.data_ptr(), data.data_ptr(), nbytes,
-                                           ctypes.addressof(counts), _stream_handle(dev)), "rode_hip_group_plan")
-    return GroupPlan(data, list(counts))
+        counts, fours = (ctypes.c_int * 4)(), ctypes.c_int()
+        _lib.check(lib.rode_hip_group_plan_fours(m, row_offsets.data_ptr(), column_indices.data_ptr(), data.data_ptr(), nbytes,
+                                                 ctypes.addressof(counts), ctypes.addressof(fours), _stream_handle(dev)),
+                   "rode_hip_group_plan_fours")
+    return GroupPlan(data, list(counts), fours.value)
 
 
 def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0, columns_local=False,
@@ -321,6 +325,7 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
     if isinstance(plan, GroupPlan):
         if plan.usable and whole_lists:
             p.groups, p.group_counts = plan.data.data_ptr(), ctypes.addressof(plan._header)
+            p.tile_fours = plan.tile_fours
     elif isinstance(plan, HubPlan):
         if plan.usable and whole_lists:
             p.hub, p.hub_counts = plan.data.data_ptr(), ctypes.addressof(plan._header)

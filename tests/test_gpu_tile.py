@@ -388,3 +388,73 @@ def test_few_tiles_that_have_all_rows(m, window, extra, d, half):
     out = sparse_attention(csr, *ins, scale=d ** -0.5)
     for a, b in zip((out,) + torch.autograd.grad(out, ins, g), want):
         assert (a.double() - b).norm() <= (2e-3 if half and b is not want[0] else 2e-6) * b.norm()
+
+
+FOURS = [  # m, window, columns the window moves per row, random columns, width, scale; rows of three columns
+    (16, 64, 0, 0, 64, 0.3, ()),              # one tile of four
+    (75, 69, 1, 5, 64, 0.3, ()),              # four tiles and rows after the last
+    (160, 260, 3, 70, 64, -0.3, (40,)),       # two and a half times four, one tile missing; more than 64 nonzeros outside a run
+    (144, 97, 2, 20, 128, 0.2, (3, 70)),      # the first of four missing, the second
+    (128, 130, 1, 16, 32, 0.4, tuple(range(0, 64, 16))),  # none of the first four
+    (80, 400, 2, 130, 32, 0.2, ()),           # three times 64 outside a run
+]
+
+
+@pytest.mark.parametrize("m,window,shift,extra,d,scale,short", FOURS)
+def test_four_tiles_a_workgroup_against_fp64(m, window, shift, extra, d, scale, short):
+    """Halves; four tiles whatever their number (the figure that the call goes by is knowledge and changes no result)."""
+    csr, dense = _mask(m, window, shift, extra, seed=m + window, short_rows=short)
+    assert csr.plan.counts[3] == m // 16 - len(short)
+    csr.call_plans().tile_fours = 1 << 20
+    heads = _heads(csr)
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    q, k, v = (torch.randn(heads, r, d, device="cuda", generator=gen).half() for r in (m, csr.n, csr.n))
+    outs, scores, stats = _attention_call(csr, csr.values, q, k, v, scale, "scores")
+    assert torch.equal(outs, sparse_attention(csr, q, k, v, scale=scale))
+    outs_p, probs, _ = _attention_call(csr, csr.values, q, k, v, scale, "probs")
+    assert torch.equal(outs, outs_p)
+    rows = torch.repeat_interleave(torch.arange(m, device="cuda"), (csr.row_offsets[1:] - csr.row_offsets[:-1]).long())
+    assert (probs - torch.exp(scores - stats[:, rows, 0]) * stats[:, rows, 1]).abs().max() <= 2e-6
+    for h in (0, heads // 3, heads - 1):
+        want = _reference(dense, q[h], k[h], v[h], scale)
+        assert (outs[h].double() - want).abs().max() <= 2e-5 * want.abs().max()
+        s = ((q[h].double() @ k[h].double().t()) * dense * scale)[rows, csr.column_indices.long()]
+        assert (scores[h].double() - s).abs().max() <= 2e-5 * s.abs().max()
+
+
+def test_four_tiles_a_workgroup_without_range():
+    """Infinite scores and rows of v that are not finite, in a run, at its ends and outside it: as with a tile a workgroup."""
+    m, d, inf = 192, 64, float("inf")
+    csr, dense = _mask(m, 100, 2, 30, seed=5)
+    values = csr.values.clone()
+    rows = torch.repeat_interleave(torch.arange(m, device="cuda"), (csr.row_offsets[1:] - csr.row_offsets[:-1]).long())
+    for row, at, value in ((3, slice(None), -inf), (5, slice(0, 40), -inf), (50, slice(129, 130), -inf), (70, slice(50, 51), inf)):
+        values[(rows == row).nonzero().flatten()[at]] = value
+    one, four = (RoDeCSR(csr.row_offsets_cpu, csr.column_indices, values, "cuda", m, csr.n, 64, locality=True) for _ in range(2))
+    one.call_plans().tile_fours, four.call_plans().tile_fours = 0, 1 << 20
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.rand(_heads(csr), r, d, device="cuda", generator=gen).half() for r in (m, csr.n, csr.n))
+    v[:, [1, 130, 2 * 80 + 99, csr.n - 1]] = inf
+    for x, y in zip(*(_attention_call(c, c.values, q, k, v, 0.125, "scores") for c in (four, one))):
+        assert torch.equal(x.isnan(), y.isnan()) and torch.equal(x.isinf(), y.isinf())
+        ok = y.isfinite()
+        assert ok.any() and not ok.all()
+        torch.testing.assert_close(x[ok], y[ok], rtol=2e-5, atol=2e-5)
+
+
+def test_how_many_fours_a_plan_is_worth_and_runs_that_lie_apart():
+    """A sliding window: the columns of all fours over those of one; runs that lie apart: none."""
+    csr, _ = _mask(1040, 200, 1, 4, seed=1)  # 65 tiles: 16 fours of 263 columns (and what random columns add to a run), a last one of 215
+    assert csr.plan.counts[3] == 65 and csr.plan.tile_fours == csr.call_plans().tile_fours == 16
+    csr, _ = _mask(256, 100, 0, 0, seed=1)
+    assert csr.plan.counts[3] == 16 and csr.plan.tile_fours == 4
+    n = 16 * 200
+    first = np.repeat(200 * np.random.default_rng(0).permutation(16), 16)
+    col = (first[:, None] + np.arange(100)).astype(np.int32).ravel()
+    apart = RoDeCSR(torch.arange(0, 25601, 100, dtype=torch.int32), torch.from_numpy(col), torch.ones(25600), "cuda", 256, n, 64, locality=True)
+    assert apart.plan.counts[3] == 16 and apart.plan.tile_fours == 0
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    q, k, v = (torch.randn(_heads(apart), r, 64, device="cuda", generator=gen).half() for r in (256, n, n))
+    one = sparse_attention(apart, q, k, v)
+    apart.call_plans().tile_fours = 1 << 20  # (said all the same: steps that one tile alone wants)
+    torch.testing.assert_close(sparse_attention(apart, q, k, v), one, rtol=2e-5, atol=2e-6)
