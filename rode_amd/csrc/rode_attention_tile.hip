@@ -51,7 +51,7 @@ struct TileSoftmax {
     float ref = -0x1p126f;    // (no score yet)
     float l = 0.f;            // sum of this lane's weights
     f32x4 acc[D / 16];        // weighted sums, times TileWeights<T>::kScale
-    float total_l = 0.f;
+    float total_ref = -0x1p126f, total_l = 0.f;
     f32x4 total[PARTS ? D / 16 : 1];
     __device__ __forceinline__ TileSoftmax()
     {
@@ -62,9 +62,16 @@ struct TileSoftmax {
     }
     __device__ __forceinline__ void put_away()
     {
+        const float corr = __builtin_amdgcn_exp2f(total_ref - ref);
+        total_ref = ref;
 #pragma unroll
-        for (int b = 0; b < D / 16; ++b) total[b] += acc[b], acc[b] = kNothing;
-        total_l += l, l = 0.f;
+        for (int b = 0; b < D / 16; ++b) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) total[b][i] = fmaf(total[b][i], corr, acc[b][i]); // (corr: a power of two)
+            acc[b] = kNothing;
+        }
+        total_l = fmaf(total_l, corr, l);
+        l = 0.f;
     }
     __device__ __forceinline__ void step(const float (&sc)[N], TileWeights<T>& weights)
     {
@@ -78,11 +85,6 @@ struct TileSoftmax {
             l *= corr;
 #pragma unroll
             for (int b = 0; b < D / 16; ++b) acc[b] *= corr;
-            if constexpr (PARTS) {
-                total_l *= corr;
-#pragma unroll
-                for (int b = 0; b < D / 16; ++b) total[b] *= corr;
-            }
             ref = now;
         }
         float p[N], sum[N];
@@ -378,8 +380,8 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
 // with a multiple of their number): a row of k or v then comes out of memory once an XCD and not once in every few of the 9
 // workgroups that want it.
 //
-// Measured (halves, 16 384 rows, eight heads of width 64): window 512 106 -> 78 us (2.9 M lines past the L2s, 370 MB, four fifths of it
-// values, which every head reads for itself), and 64 random columns 207 -> 167 (7.2 M lines, 920 MB: 5.3 TB/s of the 6.5 to 7 that pass
+// Measured (halves, 16 384 rows, eight heads of width 64): window 512 106 -> 76 us (2.9 M lines past the L2s, 370 MB, four fifths of it
+// values, which every head reads for itself), and 64 random columns 207 -> 175 (7.2 M lines, 920 MB: 5.3 TB/s of the 6.5 to 7 that pass
 // the L2s; rows of k and v outside the runs hit in L2 three times out of four).  A build without the products and the softmax took as
 // long along the runs; the steps in the order of the columns 83 and 179; as many heads on an XCD as there are 230.
 // Tried for the nonzeros outside the runs (us, of 176): the scores of all rows before the rows of v (fewer lines past the L2s, 690 MB, but a wave
