@@ -39,6 +39,14 @@ namespace rode {
 
 namespace {
 
+// With 32-bit operands, when a head's k and v are of that size and more (an L2 has 4 MB), the nonzeros outside the runs come before
+// the columns of the runs: the workgroups then begin with them together, all of them at rows of k, then all at rows of v, and find
+// more of those in L2.  us, after the runs -> before them: 16 384 rows, window 512 and 64 random columns, width 64 66.6 -> 60.1, four heads 225 -> 202, 128 129
+// -> 123; 20 000 of 128 and 16, four heads 112 -> 98; 14 000 of 400 and 32 (7.2 MB) 47.4 -> 45.2; 12 000 (6.1 MB) 33.2 -> 36.3, four
+// heads 112 -> 111; 9000 (4.6 MB) 35.5 -> 38.0; width 32, 16 384 rows (4.2 MB) 31.1 -> 34.0.  (Halves: no faster at any size; the gradient's
+// two passes: row pass 97 either way, column pass 73, with halves 1 to 3 % slower.)
+constexpr size_t kOutsideFirstBytes = 7000000;
+
 // Running softmax of the rows of a tile: 4 or 8 scores of this lane's row at a time (-inf: none).  A weight is exp(score)
 // over a power of two, 2^ref, the first one that no score so far passes: the exponent of a weight is then a single rounding away
 // from score * log2(e), and the steps and the waves rescale each other's sums exactly.  PARTS: the sums of a few steps are put away
@@ -259,7 +267,7 @@ __global__ void __launch_bounds__(kWgThreads, (D == 128 ? 2 : tile_waves<T, D>()
 attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int* __restrict__ runs,
                       const int* __restrict__ row_ptr, const int* __restrict__ col, const float* __restrict__ val,
                       const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, float scale,
-                      float* __restrict__ out, float* probs, float2* __restrict__ stats, HeadStrides heads)
+                      float* __restrict__ out, float* probs, float2* __restrict__ stats, bool outside_first, HeadStrides heads)
 {
     constexpr int NB = D / 16, PAD = D + 4, NT = tile_blocks<T>(), kStep = 16 * NT;
     using KStage = TileStage<T, D, kAlong>;
@@ -271,6 +279,8 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     __shared__ __attribute__((aligned(16))) float shared[kWavesPerWg][kStageFloats];
     __shared__ float part_m[kWavesPerWg + 1][kTileRows], part_l[kWavesPerWg + 1][kTileRows]; // (the last: outside the runs)
     __shared__ float part_ref[kWavesPerWg][kTileRows];
+    constexpr bool kMayBeFirst = sizeof(T) == 4; // (outside_first)
+    __shared__ __attribute__((aligned(16))) float ahead[kMayBeFirst ? kWavesPerWg * kOutsideRows * PAD : 4];
     __shared__ int4 extents[kTileRows]; // (for the nonzeros outside the runs: not in registers until then)
     const int tile = xcd_logical_block(blockIdx.x, gridDim.x);
     if (tile >= n_tiles) return;
@@ -283,6 +293,18 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     const TileLane me = tile_lane(tile * kTileRows + n, row_ptr, runs);
     const int base = me.base();
     if (threadIdx.x < kTileRows) extents[threadIdx.x] = me.packed();
+    // the sums of the nonzeros outside the runs: behind the wave's own in the steps' staging, or, where they may come first, apart
+    float* outside = kMayBeFirst ? ahead + wave * kOutsideRows * PAD : shared[wave] + kPart;
+    auto rows_outside_runs = [&](bool whole) __attribute__((always_inline)) {
+        int here = lane; // (nothing worked out from it before is worth a register until then)
+        asm volatile("" : "+v"(here));
+        rows_outside<T, D, KEEP>(extents, wave, tile * kTileRows, whole, here, col, val, q, k, v, scale, probs, shared[wave], outside,
+                                 part_m[kWavesPerWg], part_l[kWavesPerWg]);
+    };
+    if (kMayBeFirst && outside_first) {
+        __syncthreads(); // (extents)
+        rows_outside_runs(false);
+    }
     const int steps = (rt.hi - rt.lo + kStep - 1) / kStep;
     u32x4* lds_k = reinterpret_cast<u32x4*>(shared[wave]);
     u32x4* lds_v = lds_k + KStage::kBytes / 16;
@@ -332,8 +354,7 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
     run_columns();
     const bool again = __syncthreads_or(!sm.finite());
     if (again) sm = TileSoftmax<T, D>();
-    rows_outside<T, D, KEEP>(extents, wave, tile * kTileRows, again, lane, col, val, q, k, v, scale, probs, shared[wave], shared[wave] + kPart,
-                             part_m[kWavesPerWg], part_l[kWavesPerWg]); // (the steps' staging is free)
+    if (!(kMayBeFirst && outside_first) || again) rows_outside_runs(again); // (the steps' staging is free)
 
     // the partial results, a wave's relative to its power of two, those outside the runs to the exponential of their maximum
     float* part = shared[wave];
@@ -347,10 +368,11 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
 #pragma unroll
     for (int w = 1; w <= kWavesPerWg; ++w) top = fmaxf(top, part_m[w][r]);
     const float top_safe = top == -INFINITY ? 0.f : top;
+    const float* outside_of_row = (kMayBeFirst ? ahead + r / kOutsideRows * kOutsideRows * PAD : shared[r / kOutsideRows] + kPart) + r % kOutsideRows * PAD;
     float f = __builtin_amdgcn_exp2f((part_m[kWavesPerWg][r] - top_safe) * kLog2e);
     float total = part_l[kWavesPerWg][r] * f, o[NB];
 #pragma unroll
-    for (int x = 0; x < NB; ++x) o[x] = shared[r / kOutsideRows][kPart + r % kOutsideRows * PAD + e0 + x] * f;
+    for (int x = 0; x < NB; ++x) o[x] = outside_of_row[e0 + x] * f;
 #pragma unroll
     for (int w = 0; w < kWavesPerWg; ++w) {
         f = __builtin_amdgcn_exp2f(-fmaf(top_safe, kLog2e, -part_ref[w][r]));
@@ -574,7 +596,7 @@ hipError_t launch_tiles(int nheads, int M, int N, int nnz, const int* row_ptr, c
     auto kernel = probs == nullptr ? attention_tile_kernel<T, D, kKeepNothing>
                   : stats != nullptr ? attention_tile_kernel<T, D, kKeepScores> : attention_tile_kernel<T, D, kKeepProbs>;
     kernel<<<grid, kWgThreads, 0, stream>>>(n_tiles, group_plan_tiles(plan, M), group_plan_runs(plan, M), row_ptr, col, val, q, k, v,
-                                            scale, out, probs, stats, heads);
+                                            scale, out, probs, stats, 2 * (size_t)N * D * sizeof(T) >= kOutsideFirstBytes, heads);
     return hipGetLastError();
 }
 

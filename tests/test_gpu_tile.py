@@ -458,3 +458,30 @@ def test_how_many_fours_a_plan_is_worth_and_runs_that_lie_apart():
     one = sparse_attention(apart, q, k, v)
     apart.call_plans().tile_fours = 1 << 20  # (said all the same: steps that one tile alone wants)
     torch.testing.assert_close(sparse_attention(apart, q, k, v), one, rtol=2e-5, atol=2e-6)
+
+
+@pytest.mark.parametrize("keep", [None, "scores", "probs"])
+@pytest.mark.parametrize("bad", [False, True])
+def test_nonzeros_outside_the_runs_first(bad, keep):
+    """fp32 with k and v of a head above 7 MB; a row of v that is not finite sends its tiles row by row after that."""
+    m, d, scale = 1712, 64, 0.2
+    csr, dense = _mask(m, 400, 8, 70, seed=3)
+    assert csr.plan.counts[3] == m // 16 and 2 * csr.n * d * 4 >= 7_000_000
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(3, r, d, device="cuda", generator=gen) for r in (m, csr.n, csr.n))
+    clean = _reference(dense, q[1], k[1], v[1], scale)
+    touched = torch.zeros(m, dtype=torch.bool, device="cuda")
+    if bad:
+        v[:, 2400] = float("inf")
+        touched = dense[:, 2400] != 0
+        assert touched.any() and not touched.all()
+    out, scores, stats = _attention_call(csr, csr.values, q, k, v, scale, keep)
+    assert not torch.isfinite(out[1][touched]).all(dim=1).any()
+    assert (out[1].double() - clean)[~touched].abs().max() <= 2e-5 * clean.abs().max()
+    if keep is not None:
+        rows = torch.repeat_interleave(torch.arange(m, device="cuda"), (csr.row_offsets[1:] - csr.row_offsets[:-1]).long())
+        s = (q[1].double() @ k[1].double().t()) * dense * scale
+        if keep == "probs":
+            s = torch.softmax(s.masked_fill(dense == 0, float("-inf")), dim=1)
+        s = s[rows, csr.column_indices.long()]
+        assert (scores[1].double() - s).abs().max() <= 2e-5 * s.abs().max()
