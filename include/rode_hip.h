@@ -275,8 +275,8 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
  *   window, window_rows   both parts of a locality plan made from the lists of the call
  *   window_counts         NULL, or the HOST int[4] header rode_hip_window_plan returned;
  *                         with it, kernels that would find no chunk to work on are not
- *                         launched at all.  fp64 operands, and dense rows of at most 128
- *                         bytes, ignore the locality plan.
+ *                         launched at all.  Dense rows of less than 128 bytes ignore the
+ *                         locality plan, and those of 128 without `nonzeros`.
  *   hub, hub_counts       a hub plan of this matrix and its HOST int[8] header (required
  *                         with it).  Needs the complete decomposition: for SpMM the
  *                         RODE_SPMM_WHOLE_LISTS promise, for SDDMM simply whole lists.

@@ -77,15 +77,39 @@ struct WindowGain {
     float largest;      // ... and above largest_mb
     size_t largest_mb;
 };
+inline float window_gain(const PlanRef& plan, int m2, size_t row_bytes, const WindowGain& of)
+{
+    const float slots = plan.nonzeros < 31ll * m2 ? (float)plan.nonzeros / (float)m2 : 31.f;
+    const size_t mb = 2 * (size_t)m2 * row_bytes >> 20;
+    return (of.base + of.per_slot * slots) * (mb >= of.largest_mb ? of.largest : mb >= of.larger_mb ? of.larger : 1.f);
+}
 inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes, const WindowGain& full_round)
 {
     if (plan.dev == nullptr || plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) return true;
     const int chunks = plan.host_counts[0], rounds = (chunks + round - 1) / round;
-    const float slots = plan.nonzeros < 31ll * m2 ? (float)plan.nonzeros / (float)m2 : 31.f;
-    float gain = full_round.base + full_round.per_slot * slots;
-    const size_t mb = 2 * (size_t)m2 * row_bytes >> 20;
-    gain *= mb >= full_round.largest_mb ? full_round.largest : mb >= full_round.larger_mb ? full_round.larger : 1.f;
-    return gain * (float)chunks >= (float)rounds * (float)round;
+    return window_gain(plan, m2, row_bytes, full_round) * (float)chunks >= (float)rounds * (float)round;
+}
+
+// Do the ring kernels pay for a call?  A strip costs as much as its chunks and a start (the first window, not copied beside any work)
+// worth a chunk and half a chunk per slice; few strips with a chunk more than the others do not count.  gain: time of the standard kernels
+// over that of a chunk of s slots a row, measured as for the window kernels on bands of 128 to 256 columns and 66 K to 1 M rows, SpMM: us, standard
+// -> ring, 9 / 14 / 19 / 27 slots a row (the operands within the last-level cache; beyond it the ring gains up to twice that)
+//   f32 x 64    131 K 20.2 -> 18.8, 24.3 -> 20.8, 29.6 -> 23.0, 38.2 -> 27.2; 350 K 48 -> 42, 60 -> 48, 75 -> 55, 95 -> 66; 90 K 14.8 -> 18.5, 17.5 -> 20.6, 21.5 -> 22.6, 27.3 -> 26.1
+//   f32 x 128   131 K 37 -> 32, 45 -> 37, 57 -> 41, 73 -> 50; 66 K 20.4 -> 20.5, 24.7 -> 23.1, 29.4 -> 25.4, 38.4 -> 30.4; 90 K 26.7 -> 31.4, 32.4 -> 34.8, 39.0 -> 37.7, 51 -> 44
+//   f32 x 32    600 K 44 -> 53, 51 -> 58, 66 -> 64, 87 -> 75; 200 K 17.3 -> 22.6, 20.0 -> 24.5, 24.2 -> 26.2, 31.7 -> 30.5
+//   f16 x 128   200 K 36 -> 43, 43 -> 47, 54 -> 52, 69 -> 61; 600 K 104 -> 101, 124 -> 112, 150 -> 126;  f16 x 64  600 K 54 -> 66, 68 -> 75, 82 -> 85, 102 -> 101
+//   f64 x 32    131 K 21.3 -> 19.7, 25.5 -> 21.6, 31.7 -> 24.5, 40.2 -> 29.1;  f64 x 16  131 K 20.0 -> 14.8, 23.7 -> 16.6, 37.8 -> 21.5 (27)
+// and SDDMM (which takes whole rows only):
+//   f32 x 64    131 K 24.8 -> 21.7, 29.9 -> 23.8, 35.9 -> 27.2, 46.3 -> 31.6; 350 K 60 -> 48, 74 -> 53, 93 -> 65, 119 -> 79; 600 K 100 -> 100, 124 -> 107, 179 -> 120
+//   f32 x 32    350 K 33 -> 40, 41 -> 43, 54 -> 47, 72 -> 55; 600 K 54 -> 65, 68 -> 80, 87 -> 92, 133 -> 107; 1 M 86 -> 126, 125 -> 137, 175 -> 145, 236 -> 171
+//   f16 x 128   131 K 25.0 -> 24.4, 30.4 -> 27.6, 37.3 -> 31.4, 46.9 -> 37.8; 600 K 102 -> 111, 125 -> 122, 179 -> 136;  f16 x 64  350 K 34 -> 43, 42 -> 46, 54 -> 52, 72 -> 62
+inline bool ring_pays(const PlanRef& plan, int m2, int workgroups, int slices, size_t row_bytes, const WindowGain& chunk)
+{
+    if (plan.dev == nullptr) return true;
+    // the number of nonzeros not said: the caller wants the plan used, which rows of 128 bytes never were
+    if (plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) return row_bytes > 128;
+    const int parts = plan.host_counts[0] * slices, rounds = (parts - 16 * slices + workgroups - 1) / workgroups;
+    return window_gain(plan, m2, row_bytes, chunk) * (float)parts >= ((float)rounds + 1.f + 0.5f * (float)slices) * (float)workgroups;
 }
 
 hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* plan, hipStream_t stream);

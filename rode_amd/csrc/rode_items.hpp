@@ -367,9 +367,11 @@ constexpr int kPlanDescInts = 4;
 constexpr int kPlanResidueChunk = 128;     // residue-list entries per chunk
 constexpr int kResidueWindowRowsMax = 512; // dense rows of one window (9 bits of a slot's 16-bit entry)
 
-// Do the window kernels take dense rows of so many bytes?  More than one tile of 128 bytes (with a single tile a
+// Do the window kernels take dense rows of so many bytes (that no ring does)?  More than one tile of 128 bytes (with a single tile a
 // window is not used often enough to repay its copy), and no more than their 32-bit offsets into a window reach.
 constexpr bool window_takes(size_t row_bytes) { return row_bytes > 128 && row_bytes <= (1ull << 32) / kResidueWindowRowsMax; }
+// Dense rows that SpMM takes through a ring (rode_window.hpp): whole, or in so many slices of 256 bytes; 0: not.
+constexpr int ring_slices(size_t row_bytes) { return row_bytes == 128 || row_bytes == 256 ? 1 : row_bytes == 512 ? 2 : row_bytes == 1024 ? 4 : 0; }
 constexpr int kWindowWgs = 256; // workgroups of the window kernels, one per CU: they take the chunks in rounds of that many
 
 // Window of one chunk: dense rows [w0, w0 + wn); wn == 0: no window.  slots / misses: how

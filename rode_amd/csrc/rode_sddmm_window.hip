@@ -174,6 +174,149 @@ sddmm_residue_window_kernel(int m2, int k, const int* __restrict__ col, const fl
         if (result_at[i] >= 0) out[result_at[i]] = result[i];
 }
 
+template <typename T, int TILES>
+__global__ void __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+sddmm_ring_kernel(int m2, int k, const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ lhs,
+                  const T* __restrict__ rhs, float* __restrict__ out, const PlannedChunk* __restrict__ rows)
+{
+    using R = Ring<TILES>;
+    constexpr int VEC = DenseVec<T>::kElems, TW = kResLanes * VEC, QUADS = kBlockItems / 4, OWN = kBlockItems / kResLanes;
+    __shared__ uint4 ring[R::kBytes / 16];
+    __shared__ uint4 records[3 * kRingRecordVecs];
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int group = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
+    const RingWalk walk(m2, 1);
+    int chunk = walk.from(rows, walk.at);
+    if (chunk >= walk.end) return;
+    const char* ring_bytes = reinterpret_cast<const char*>(ring);
+    const unsigned ring_lds = lds_address(ring), rec_lds = lds_address(records);
+
+    auto fetch_rows = [&](int from, int to) __attribute__((always_inline)) {
+        R::fetch(ring_lds, reinterpret_cast<const char*>(rhs), R::kRowBytes, from, to, wave, lane);
+    };
+    auto fetch_record = [&](int rec, int c) __attribute__((always_inline)) { fetch_ring_record(rec_lds + rec * kRingRecordVecs * 16, rows + c, wave); };
+    auto record = [&](int rec) __attribute__((always_inline)) -> const RingRecord& { return *reinterpret_cast<const RingRecord*>(records + rec * kRingRecordVecs); };
+    auto lhs_row = [&](const RingRecord& rc, uint4 (&a)[TILES]) __attribute__((always_inline)) {
+        const int row = rc.meta[group].row;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) a[t] = row >= 0 ? *reinterpret_cast<const uint4*>(lhs + (size_t)row * k + t * TW + ls * VEC) : make_uint4(0, 0, 0, 0);
+    };
+
+    int w0 = rows[chunk].w0, low = w0, high = w0 + rows[chunk].wn; // (the ring has rows [low, high))
+    int after = walk.from(rows, chunk + 1), rec = 0;
+    fetch_rows(low, high);
+    fetch_record(0, chunk);
+    if (after < walk.end) fetch_record(1, after);
+    copies_done();
+    __syncthreads();
+    uint4 a_next[TILES];
+    lhs_row(record(0), a_next);
+    // the dot products of the last chunk, stored during the next one: nobody waits for the stores then
+    float result[OWN];
+    int result_at[OWN];
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) result[i] = 0.f, result_at[i] = -1;
+
+    while (true) {
+        copies_done();
+        __syncthreads(); // the chunk's rows and the next one's record are in LDS, and every wave is done with the chunk before
+        const RingRecord& mine = record(rec);
+        const int4 meta = *reinterpret_cast<const int4*>(&mine.meta[group]);
+        const int cnt = meta.x >= 0 ? meta.z & 0xff : 0;
+        const unsigned missmask = meta.x >= 0 ? (unsigned)meta.w : 0u;
+        unsigned at[kBlockItems / 2];
+#pragma unroll
+        for (int i = 0; i < kBlockItems / 8; ++i) {
+            const uint4 e = reinterpret_cast<const uint4*>(mine.entry[group])[i];
+            at[4 * i] = R::units(e.x, w0, ls), at[4 * i + 1] = R::units(e.y, w0, ls), at[4 * i + 2] = R::units(e.z, w0, ls), at[4 * i + 3] = R::units(e.w, w0, ls);
+        }
+        const int wave_quads = wave_max_quads((cnt + 3) / 4);
+        const bool wave_all_hit = __ballot(missmask != 0) == 0ull;
+        typename DotVec<T>::Reg a[TILES][DotVec<T>::kRegs];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            asm volatile("" : "+v"(a_next[t].x), "+v"(a_next[t].y), "+v"(a_next[t].z), "+v"(a_next[t].w)); // waited for here, before the copies below
+            const uint32_t w[4] = {a_next[t].x, a_next[t].y, a_next[t].z, a_next[t].w};
+            DotVec<T>::load(reinterpret_cast<const T*>(w), a[t]);
+        }
+        const bool last = after >= walk.end;
+        int next_w0 = 0, next_end = 0;
+        bool ahead = true;
+        const int rec1 = rec == 2 ? 0 : rec + 1, rec2 = rec1 == 2 ? 0 : rec1 + 1;
+        int after2 = after;
+        if (!last) {
+            next_w0 = rows[after].w0, next_end = next_w0 + rows[after].wn;
+            const int top = max(high, next_end);
+            ahead = next_w0 >= max(low, top - kRingRows) && top - kRingRows <= w0; // do its rows fit beside this chunk's?
+            if (ahead) {
+                fetch_rows(high, top);
+                high = top, low = max(low, top - kRingRows);
+            }
+            after2 = walk.from(rows, after + 1);
+            if (after2 < walk.end) fetch_record(rec2, after2);
+            lhs_row(record(rec1), a_next);
+        }
+        float v[OWN];
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) {
+            if (result_at[i] >= 0) out[result_at[i]] = result[i];
+            const int pos = i * kResLanes + ls;
+            result_at[i] = pos < cnt ? meta.y + ((mine.entry[group][pos] >> 9) & (kBlockItems - 1)) : -1;
+            v[i] = result_at[i] >= 0 ? val[result_at[i]] : 0.f;
+        }
+        __builtin_amdgcn_sched_barrier(0); // the loads above are issued before the work below, not after it
+        float acc[kBlockItems]; // this lane's share of every position
+#pragma unroll
+        for (int i = 0; i < kBlockItems; ++i) acc[i] = 0.f;
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            if (q < wave_quads) { // the same for every lane of the wave
+                uint4 raw[TILES][4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned pair = at[2 * q + j / 2], off = (j % 2 ? pair >> 16 : pair & 0xffffu) << 4;
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t) raw[t][j] = *reinterpret_cast<const uint4*>(ring_bytes + (off ^ (t * 128u)));
+                }
+                if (!wave_all_hit) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if ((missmask >> (4 * q + j)) & 1u) { // outside the window
+                            const int c = col[meta.y + ((mine.entry[group][4 * q + j] >> 9) & (kBlockItems - 1))];
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t) raw[t][j] = *reinterpret_cast<const uint4*>(rhs + (size_t)c * k + t * TW + ls * VEC);
+                        }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { // (a sum of its own per tile)
+                    acc[4 * q + j] = DotVec<T>::dot_raw(a[0], raw[0][j], 0.f);
+#pragma unroll
+                    for (int t = 1; t < TILES; ++t) acc[4 * q + j] += DotVec<T>::dot_raw(a[t], raw[t][j], 0.f);
+                }
+            }
+        }
+        // lane l of the group has the positions l, 8 + l, 16 + l, 24 + l
+#pragma unroll
+        for (int i = 0; i < OWN; ++i) {
+            float part8[kResLanes];
+#pragma unroll
+            for (int j = 0; j < kResLanes; ++j) part8[j] = acc[i * kResLanes + j];
+            result[i] = v[i] * transpose_reduce8(part8, ls);
+        }
+        if (last) break;
+        if (!ahead) {
+            __syncthreads(); // (the rows of a window that lies apart, in the place of this one's)
+            fetch_rows(next_w0, next_end);
+            low = next_w0, high = next_end;
+        }
+        w0 = next_w0, rec = rec1, after = after2;
+    }
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+        if (result_at[i] >= 0) out[result_at[i]] = result[i];
+}
+
 } // namespace
 
 // The window kernel over the planned chunks of the residue list, for dense rows that window_takes.
@@ -183,7 +326,13 @@ hipError_t sddmm_window_launch(int m2, int k, const int* col, const float* val, 
                                const int* plan, const void* plan_rows, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
-    if (!window_takes((size_t)k * sizeof(T))) return hipErrorInvalidValue;
+    const size_t row_bytes = (size_t)k * sizeof(T);
+    if (ring_slices(row_bytes) == 1) {
+        auto kernel = row_bytes == 128 ? sddmm_ring_kernel<T, 1> : sddmm_ring_kernel<T, 2>;
+        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, static_cast<const PlannedChunk*>(plan_rows));
+        return hipGetLastError();
+    }
+    if (!window_takes(row_bytes)) return hipErrorInvalidValue;
     auto kernel = ((size_t)k * sizeof(T)) % (kResLanes * 16) != 0 ? sddmm_residue_window_kernel<T, true> : sddmm_residue_window_kernel<T, false>;
     kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, static_cast<const PlannedChunk*>(plan_rows));
     return hipGetLastError();

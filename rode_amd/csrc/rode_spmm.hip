@@ -996,8 +996,8 @@ size_t spmm_hub_partial_rows(const int* counts, int n, int acc_bytes)
 
 // n: any positive multiple of the 128-bit vector width (4 fp32, 8 fp16, 2 fp64).  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
-// which `plan` holds a window go to the window kernel where it takes the
-// width (window_takes) and pays (window_pays).
+// which `plan` holds a window go to the ring or window kernel that takes the
+// width (ring_slices, else window_takes) where that pays (ring_pays, window_pays).
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
@@ -1008,8 +1008,15 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
     constexpr WindowGain kWide = {0.87f, 0.0237f, 1.17f, 300, 1.17f, 300}, kNarrow = {0.715f, 0.0235f, 1.f, 380, 1.17f, 380},
                          kHalves = {0.79f, 0.0113f, 1.07f, 270, 1.17f, 380}, kDoubles = {0.75f, 0.0228f, 1.f, 360, 1.17f, 360};
     const size_t row_bytes = (size_t)n * sizeof(T);
-    if (!window_takes(row_bytes) ||
-        !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
+    const int slices = ring_slices(row_bytes);
+    // (a band of 128 columns is worth 5 % less than those of 192 and 256 that the figures beside ring_pays are of)
+    const bool line = row_bytes == 128, whole = slices == 1;
+    const WindowGain ring = sizeof(T) == 8 ? WindowGain{line ? 1.2f : whole ? 1.05f : 1.1f, line ? 0.03f : 0.02f, 1.f, 0, 1.f, 0}
+                            : sizeof(T) == 2 ? WindowGain{line ? 0.73f : whole ? 0.93f : 0.97f, line ? 0.0145f : 0.02f, 1.f, 0, 1.f, 0}
+                                             : WindowGain{line ? 0.69f : whole ? 1.05f : 1.1f, line ? 0.0235f : 0.02f, 1.f, 0, 1.f, 0};
+    if (slices > 0 ? !ring_pays(plan, m2, kWindowWgs, slices, row_bytes, ring)
+                   : !window_takes(row_bytes) ||
+                         !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
         plan.no_window();
     if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
         constexpr int kLine = 128 / (int)sizeof(T);

@@ -186,6 +186,163 @@ spmm_residue_window_kernel(int m2, int n, int owned_slots, const int* __restrict
     write_result();
 }
 
+template <typename T, int TILES>
+__global__ void __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
+spmm_ring_kernel(int m2, int n, int slices, int owned_slots, const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
+                 const T* __restrict__ B, typename DenseVec<T>::Acc* __restrict__ C, const PlannedChunk* __restrict__ rows)
+{
+    using A = typename DenseVec<T>::Acc;
+    using R = Ring<TILES>;
+    constexpr int VEC = DenseVec<T>::kElems, TW = kResLanes * VEC, QUADS = kBlockItems / 4;
+    __shared__ uint4 ring[R::kBytes / 16];
+    __shared__ uint4 records[3 * kRingRecordVecs];
+
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int group = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
+    const RingWalk walk(m2, slices);
+    int chunk = walk.from(rows, walk.at);
+    if (chunk >= walk.end) return;
+    const char* ring_bytes = reinterpret_cast<const char*>(ring);
+    const unsigned ring_lds = lds_address(ring), rec_lds = lds_address(records), row_bytes = (unsigned)n * (unsigned)sizeof(T);
+    const char* dense = reinterpret_cast<const char*>(B) + walk.slice * R::kRowBytes;
+    const int col0 = walk.slice * TILES * TW + ls * VEC; // this lane's first column of B
+
+    auto fetch_rows = [&](int from, int to) __attribute__((always_inline)) { R::fetch(ring_lds, dense, row_bytes, from, to, wave, lane); };
+    auto fetch_record = [&](int rec, int c) __attribute__((always_inline)) { fetch_ring_record(rec_lds + rec * kRingRecordVecs * 16, rows + c, wave); };
+    auto record = [&](int rec) __attribute__((always_inline)) -> const RingRecord& { return *reinterpret_cast<const RingRecord*>(records + rec * kRingRecordVecs); };
+    // a row's values lie in the quads of its group: position 4 q + j in lane j
+    const int lane_of_quad = ls % 4;
+    auto own_values = [&](const RingRecord& rc, A (&v)[QUADS]) __attribute__((always_inline)) {
+        const int4 meta = *reinterpret_cast<const int4*>(&rc.meta[group]);
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            const int pos = 4 * q + lane_of_quad;
+            v[q] = meta.x >= 0 && pos < (meta.z & 0xff) ? val[meta.y + ((rc.entry[group][pos] >> 9) & (kBlockItems - 1))] : A(0);
+        }
+    };
+
+    int w0 = rows[chunk].w0, low = w0, high = w0 + rows[chunk].wn; // (the ring has rows [low, high))
+    int after = walk.from(rows, chunk + 1), rec = 0;
+    fetch_rows(low, high);
+    fetch_record(0, chunk);
+    if (after < walk.end) fetch_record(1, after);
+    copies_done();
+    __syncthreads();
+    A v_next[QUADS];
+    own_values(record(0), v_next);
+    // a chunk's results, written during the next one: nobody waits for the stores then
+    A result[TILES][VEC];
+    A* result_at = nullptr;
+    bool result_adds = false;
+    auto write_result = [&]() __attribute__((always_inline)) {
+        if (result_at == nullptr) return;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+            if (result_adds) {
+#pragma unroll
+                for (int x = 0; x < VEC; ++x) atomicAdd(result_at + t * TW + x, result[t][x]);
+            } else {
+                store_row<VEC>(result_at + t * TW, result[t]);
+            }
+        }
+    };
+
+    while (true) {
+        copies_done();
+        __syncthreads(); // the chunk's rows and the next one's record are in LDS, and every wave is done with the chunk before
+        const RingRecord& mine = record(rec);
+        const int4 meta = *reinterpret_cast<const int4*>(&mine.meta[group]);
+        const bool listed = meta.x >= 0 && !(((meta.z >> 8) & 1) && ((meta.z >> 16) & 0xffff) <= owned_slots);
+        const int cnt = listed ? meta.z & 0xff : 0;
+        const unsigned missmask = listed ? (unsigned)meta.w : 0u;
+        const bool accumulate = (meta.z >> 8) & 1;
+        unsigned at[kBlockItems / 2];
+#pragma unroll
+        for (int i = 0; i < kBlockItems / 8; ++i) {
+            const uint4 e = reinterpret_cast<const uint4*>(mine.entry[group])[i];
+            at[4 * i] = R::units(e.x, w0, ls), at[4 * i + 1] = R::units(e.y, w0, ls), at[4 * i + 2] = R::units(e.z, w0, ls), at[4 * i + 3] = R::units(e.w, w0, ls);
+        }
+        const int wave_quads = wave_max_quads((cnt + 3) / 4);
+        const bool wave_all_hit = __ballot(missmask != 0) == 0ull;
+        A v[QUADS];
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            v[q] = v_next[q];
+            asm volatile("" : "+v"(v[q])); // waited for here, before the copies below
+        }
+        const bool last = after >= walk.end;
+        int next_w0 = 0, next_end = 0;
+        bool ahead = true;
+        const int rec1 = rec == 2 ? 0 : rec + 1, rec2 = rec1 == 2 ? 0 : rec1 + 1;
+        int after2 = after;
+        if (!last) {
+            next_w0 = rows[after].w0, next_end = next_w0 + rows[after].wn;
+            const int top = max(high, next_end);
+            ahead = next_w0 >= max(low, top - kRingRows) && top - kRingRows <= w0; // do its rows fit beside this chunk's?
+            if (ahead) {
+                fetch_rows(high, top);
+                high = top, low = max(low, top - kRingRows);
+            }
+            after2 = walk.from(rows, after + 1);
+            if (after2 < walk.end) fetch_record(rec2, after2);
+            own_values(record(rec1), v_next);
+        }
+        write_result();
+        __builtin_amdgcn_sched_barrier(0); // the loads above are issued before the work below, not after it
+        A acc[TILES][VEC];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) acc[t][x] = A(0);
+#pragma unroll
+        for (int q = 0; q < QUADS; ++q) {
+            if (q < wave_quads) { // the same for every lane of the wave
+                uint4 raw[TILES][4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const unsigned pair = at[2 * q + j / 2], off = (j % 2 ? pair >> 16 : pair & 0xffffu) << 4;
+#pragma unroll
+                    for (int t = 0; t < TILES; ++t) raw[t][j] = *reinterpret_cast<const uint4*>(ring_bytes + (off ^ (t * 128u)));
+                }
+                if (!wave_all_hit) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if ((missmask >> (4 * q + j)) & 1u) { // outside the window: the row of B from memory
+                            const int c = col[meta.y + ((mine.entry[group][4 * q + j] >> 9) & (kBlockItems - 1))];
+#pragma unroll
+                            for (int t = 0; t < TILES; ++t) raw[t][j] = *reinterpret_cast<const uint4*>(B + (size_t)c * n + col0 + t * TW);
+                        }
+                }
+                const A v4[4] = {of_quad<0>(v[q]), of_quad<1>(v[q]), of_quad<2>(v[q]), of_quad<3>(v[q])};
+#pragma unroll
+                for (int t = 0; t < TILES; ++t)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        A b[VEC];
+                        unpack_dense<T>(raw[t][j], b);
+#pragma unroll
+                        for (int x = 0; x < VEC; ++x) acc[t][x] = fma(v4[j], b[x], acc[t][x]);
+                    }
+            }
+        }
+        // a listed row without slots of its own (empty, unaligned start) is stored as zeros
+        result_adds = accumulate;
+        result_at = listed && (cnt > 0 || !accumulate) ? C + (size_t)meta.x * n + col0 : nullptr;
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+#pragma unroll
+            for (int x = 0; x < VEC; ++x) result[t][x] = cnt > 0 ? acc[t][x] : A(0);
+        if (last) break;
+        if (!ahead) {
+            __syncthreads(); // (the rows of a window that lies apart, in the place of this one's)
+            fetch_rows(next_w0, next_end);
+            low = next_w0, high = next_end;
+        }
+        w0 = next_w0, rec = rec1, after = after2;
+    }
+    write_result();
+}
+
 } // namespace
 
 // The window kernel over the planned chunks of the residue list, for dense rows that window_takes.
@@ -194,7 +351,13 @@ hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, co
                               typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
-    if (!window_takes((size_t)n * sizeof(T))) return hipErrorInvalidValue;
+    const size_t row_bytes = (size_t)n * sizeof(T);
+    if (ring_slices(row_bytes) > 0) {
+        auto kernel = row_bytes == 128 ? spmm_ring_kernel<T, 1> : spmm_ring_kernel<T, 2>;
+        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, n, ring_slices(row_bytes), owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
+        return hipGetLastError();
+    }
+    if (!window_takes(row_bytes)) return hipErrorInvalidValue;
     auto kernel = ((size_t)n * sizeof(T)) % (kResLanes * 16) != 0 ? spmm_residue_window_kernel<T, true> : spmm_residue_window_kernel<T, false>;
     kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
     return hipGetLastError();

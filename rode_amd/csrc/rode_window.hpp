@@ -25,6 +25,8 @@
 #pragma once
 #include "rode_items.hpp"
 
+#include <cstddef>
+
 namespace rode {
 
 constexpr int kResLanes = 8;                                   // lanes per residue row: 8 x 16 bytes = one 128-byte tile row
@@ -141,6 +143,72 @@ __device__ __forceinline__ unsigned window_offset(unsigned pair, unsigned buffer
 {
     return __builtin_amdgcn_perm(buffer_bit, pair, ODD ? 0x07060302u : 0x07060100u);
 }
+
+// ---- rings: the windows of a band's chunks one after the other -----------------------------------
+// A workgroup that takes a contiguous strip of chunks finds most of a chunk's window in LDS already: the windows of neighbouring
+// chunks overlap but for about as many rows as a chunk has.  Dense row r lies at row r % kRingRows of a ring; a chunk's new rows are
+// copied during the one before, 1024 bytes a wave and copy.  TILES: 128-byte tiles that a row of the ring has (a dense row
+// or a slice of one).  With two, those of odd rows change places: lane groups that read rows of different parity then meet in
+// different banks here too.
+//
+// What bounds them: the window kernels copy every window whole, three times what a chunk of 128 rows is new in with a band of 256,
+// and a copy has only the work on one tile to arrive in (500 K rows of 27, 32 doubles: 4.1 us a tile of which the LDS reads need 1.8).
+// Here a chunk is one piece of work with one barrier, and its copies are a third and have all of it.  us, window kernels (standard
+// kernels for rows of 128 bytes) -> rings, 27 slots a row and a band of 256: SpMM 500 K x 32 doubles 125 -> 108 (405 MB at 3.8 TB/s; a large
+// copy would take 82), 1 M x 32 doubles 239 -> 200, 1 M x 64 233 -> 191, x 128 (two slices, by two workgroups side by side that share values and
+// records in L2) 404 -> 346, x 128 halves 317 -> 274, 500 K x 16 doubles 125 -> 69, 1 M x 32 199 -> 141; SDDMM 1 M x 64 249 -> 222, x 128 halves 278
+// -> 253, x 32 236 -> 171.  SDDMM of 512-byte rows keeps the window kernel: a row does not fit the ring, and its slices' sums meet.
+constexpr int kRingRows = 512;
+constexpr int kRingRecordVecs = (int)(sizeof(PlannedChunk) - offsetof(PlannedChunk, meta)) / 16; // (the window itself is read apart)
+static_assert(offsetof(PlannedChunk, meta) == 16 && kRingRecordVecs % kWave == 0, "whole copies");
+struct RingRecord {
+    PlannedRowMeta meta[kPlanResidueChunk];
+    unsigned short entry[kPlanResidueChunk][kBlockItems];
+};
+static_assert(sizeof(RingRecord) == kRingRecordVecs * 16, "the same");
+
+__device__ __forceinline__ void fetch_ring_record(unsigned lds, const PlannedChunk* chunk, int wave)
+{
+    if (wave * kWave < kRingRecordVecs) copy_to_lds(lds + wave * kWave * 16, chunk->meta, threadIdx.x * 16u);
+}
+
+template <int TILES>
+struct Ring {
+    static constexpr int kRowBytes = 128 * TILES, kBytes = kRingRows * kRowBytes, kRowsPerCopy = 1024 / kRowBytes;
+    // Dense rows [from, to) into the ring at `lds`; dense: this slice of row 0, row_bytes: of a whole row (at most 2^32 / 8).
+    static __device__ __forceinline__ void fetch(unsigned lds, const char* dense, unsigned row_bytes, int from, int to, int wave, int lane)
+    {
+        const int r = lane * 16 / kRowBytes, tile = TILES == 1 ? 0 : (lane / 8 ^ r) & 1;
+        const unsigned at = (unsigned)r * row_bytes + tile * 128u + lane % 8 * 16u;
+        for (int first = (from / kRowsPerCopy + wave) * kRowsPerCopy; first < to; first += kResThreads / kWave * kRowsPerCopy)
+            if (first + r >= from && first + r < to) // (a lane left out writes nothing)
+                copy_to_lds(lds + (unsigned)(first % kRingRows) * kRowBytes, dense + (size_t)first * row_bytes, at);
+    }
+    // Where the first tile of this lane's 16 bytes of two window rows is, in units of 16 bytes (both halves of a pair of entries).
+    static __device__ __forceinline__ unsigned units(unsigned entries, int w0, int ls)
+    {
+        const unsigned rows = ((entries & 0x01ff01ffu) + (unsigned)(w0 % kRingRows) * 0x10001u) & 0x01ff01ffu;
+        return TILES == 1 ? rows * 8u + ls * 0x10001u : rows * 16u + ((rows & 0x10001u) << 3) + ls * 0x10001u;
+    }
+};
+
+// A strip: chunks [at, end) one after the other, those without a window left out.  Of every XCD's share a strip per workgroup and slice.
+struct RingWalk {
+    int at, end, slice;
+    __device__ __forceinline__ RingWalk(int m2, int slices)
+    {
+        const int chunks = plan_residue_chunks(m2), share = (chunks + kXcds - 1) / kXcds, xcd = blockIdx.x % kXcds;
+        const int first = min(chunks, xcd * share), count = min(chunks, first + share) - first;
+        const int strips = gridDim.x / kXcds / slices, strip = blockIdx.x / kXcds / slices;
+        slice = blockIdx.x / kXcds % slices;
+        at = first + (int)((long long)count * strip / strips), end = first + (int)((long long)count * (strip + 1) / strips);
+    }
+    __device__ __forceinline__ int from(const PlannedChunk* __restrict__ rows, int c) const
+    {
+        while (c < end && rows[c].wn <= 0) ++c; // (the standard kernel has those)
+        return c;
+    }
+};
 
 // Longest row (in slot quads) among the 8 lane groups of the wave, as a scalar: quads at
 // or past it are skipped by the whole wave.

@@ -236,3 +236,52 @@ def test_sddmm_in_windows_is_as_exact_as_without(k, half):
         assert (csr.plan is not None) == how
         errors.append(((rode_sddmm(csr, L, B).double() - want).norm() / want.norm()).item())
     assert 0 < errors[0] <= 1.03 * errors[1]
+
+
+def _strips(m, degree, seed):
+    """Columns of m rows, `degree` ascending ones each: by chunks of 128 rows along the diagonal, some of them apart from their neighbours, before
+    them, two columns further per row (windows of up to 511), without a window, and a column outside the window here and there."""
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    row = torch.arange(m, device=DEV)
+    chunk, local = row // 128, row % 128
+    kind = chunk % 11
+    base = row - 100
+    base = torch.where(kind == 4, base - 250, base)
+    base = torch.where(kind == 6, (row + m // 2) % m, base)
+    base = torch.where(kind == 8, chunk * 128 - 60 + 2 * local, base)
+    base = base.clamp(0, m - 256)
+    pick = torch.rand(m, 256, device=DEV, generator=gen).argsort(1)[:, :degree]
+    col = base[:, None] + pick
+    col[kind == 7] = torch.randint(0, m, (int((kind == 7).sum()), degree), device=DEV, generator=gen)
+    far = (row % 50 == 3) & (kind != 7)
+    col[far, 0] = torch.randint(0, m, (int(far.sum()),), device=DEV, generator=gen)
+    return col.sort(1)[0]
+
+
+@pytest.mark.parametrize("m", [128 * 2560 + 40, 128 * 700 - 3, 128 * 3])  # ten chunks a workgroup (the ring begins again several times), two or three, one at most
+@pytest.mark.parametrize("dtype,k", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.float32, 256), (torch.float16, 64),
+                                     (torch.float16, 128), (torch.float16, 256), (torch.float64, 16), (torch.float64, 32), (torch.float64, 64)])
+def test_rings_against_fp64(m, dtype, k):
+    degree = 11
+    col = _strips(m, degree, seed=k)
+    gen = torch.Generator(device=DEV).manual_seed(k + 1)
+    val = torch.rand(m * degree, device=DEV, generator=gen) + 0.5
+    ro = torch.arange(0, m * degree + 1, degree, dtype=torch.int32)
+    csr, plain = (RoDeCSR(ro, col.flatten().int(), val, DEV, m, m, k, locality=how) for how in (True, False))
+    assert csr.plan is not None and csr.plan.windowed >= csr.plan.counts[0] * 3 // 4
+    csr.plan.nonzeros = 31 * csr.m2  # (rows of 128 bytes want to know, and long rows to be worth it)
+    B, L = (torch.randn(m, k, device=DEV, generator=gen, dtype=torch.float64).to(dtype) for _ in range(2))
+    want = torch.zeros(m, k, device=DEV, dtype=torch.float64)
+    for j in range(degree):
+        want += val.view(m, degree)[:, j:j + 1].double() * B[col[:, j]].double()
+    if dtype == torch.float64:
+        got, other = (rode_sddmm_hip.spmm_forward(c.block_indices, c.residue_indices, c.st_offsets, c.m1, c.m2, c.row_offsets, c.column_indices,
+                                                  c.values.double(), m, m, B, plan=c.plan) for c in (csr, plain))
+        assert (got - want).abs().max() <= 1e-14 * want.abs().max()
+        assert m < 128 * 2560 or not torch.equal(got, other)  # (a row's slots are added in the plan's order)
+        return
+    got, other = rode_spmm(csr, B), rode_spmm(plain, B)
+    assert (got - want).abs().max() <= 2e-6 * want.abs().max()
+    assert m < 128 * 2560 or not torch.equal(got, other)
+    want = torch.stack([val.view(m, degree)[:, j].double() * (L.double() * B[col[:, j]].double()).sum(1) for j in range(degree)], 1).flatten()
+    assert (rode_sddmm(csr, L, B) - want).abs().max() <= 2e-6 * want.abs().max()
