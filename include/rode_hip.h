@@ -201,6 +201,16 @@ int rode_hip_window_plan(int m2, int dense_rows, const int* d_row_indices_residu
 int rode_hip_preprocess_with_plan(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind,
                                   int* h_counts, int capacity_blocks, void* d_workspace, size_t workspace_bytes, int m2, int dense_rows,
                                   const int* d_column_indices, void* d_plan, size_t plan_bytes, void* stream);
+/*
+ * The same in two launches, for a caller that has the row offsets on the host too and has counted both lists there: m1 block segments,
+ * m2 residue rows, and before[t] = the segments (upper 32 bits) and residue rows (lower 32) of all rows before row
+ * t * rode_hip_preprocess_tile_rows(M), for every t up to the last row, in memory that the GPU can read (pinned memory).  d_plan NULL: no plan
+ * (one launch).  The lists are written up to m1 and m2 entries, whatever the offsets on the GPU say; h_counts as above.
+ */
+int rode_hip_preprocess_tile_rows(int M);
+int rode_hip_preprocess_placed(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind, int* h_counts,
+                               int m1, int m2, const unsigned long long* before, int dense_rows, const int* d_column_indices, void* d_plan,
+                               size_t plan_bytes, void* stream);
 size_t rode_hip_window_rows_bytes(int m2);
 int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_row_offsets,
                          const int* d_column_indices, const void* d_plan, void* d_rows, size_t rows_bytes, void* stream);

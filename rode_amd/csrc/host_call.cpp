@@ -368,6 +368,29 @@ __attribute__((target_clones("avx512f", "avx2", "default"))) void row_stats_bloc
     r.hub_nonzeros += hub;
 }
 
+RowStats stats_of(const at::Tensor& ro, long long hub_min_len)
+{
+    const long long rows = ro.size(0) - 1;
+    const void* offsets = data(ro);
+    const bool is_int = ro.scalar_type() == at::kInt;
+    RowStats r;
+    constexpr long long kBlock = 1 << 16; // (a block's sums are added up in 64 bits)
+    for (long long at = 0; at < rows; at += kBlock) {
+        const long long n = std::min(kBlock, rows - at);
+        if (is_int)
+            row_stats_block<int32_t>(static_cast<const int32_t*>(offsets) + at, n, (int32_t)std::min<long long>(hub_min_len, INT32_MAX), r);
+        else
+            row_stats_block<int64_t>(static_cast<const int64_t*>(offsets) + at, n, hub_min_len, r);
+    }
+    if (rows <= 0) r.shortest = r.longest = 0;
+    return r;
+}
+
+PyObject* built(const RowStats& r)
+{
+    return Py_BuildValue("(LLLLLLLL)", r.max_len, r.shortest, r.longest, r.blocked, r.segments_512, r.up_to_512, r.up_to_1024, r.hub_nonzeros);
+}
+
 // row_stats(row offsets on the CPU, int32 or int64; hub_min_len) -> the fields of RowStats
 PyObject* row_stats(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
@@ -377,24 +400,12 @@ PyObject* row_stats(PyObject*, PyObject* const* args, Py_ssize_t count)
     if (!ro || !int_of(args[1], hub_min_len) || !ro->is_cpu() || ro->dim() != 1 || !ro->is_contiguous() ||
         (ro->scalar_type() != at::kInt && ro->scalar_type() != at::kLong))
         return PyErr_Format(PyExc_ValueError, "row_stats takes a contiguous int32 or int64 vector on the CPU and an int");
-    const long long rows = ro->size(0) - 1;
-    const void* offsets = data(*ro);
-    const bool is_int = ro->scalar_type() == at::kInt;
     RowStats r;
     {
         NoGil no_gil;
-        constexpr long long kBlock = 1 << 16; // (a block's sums are added up in 64 bits)
-        for (long long at = 0; at < rows; at += kBlock) {
-            const long long n = std::min(kBlock, rows - at);
-            if (is_int)
-                row_stats_block<int32_t>(static_cast<const int32_t*>(offsets) + at, n, (int32_t)std::min<long long>(hub_min_len, INT32_MAX), r);
-            else
-                row_stats_block<int64_t>(static_cast<const int64_t*>(offsets) + at, n, hub_min_len, r);
-        }
+        r = stats_of(*ro, hub_min_len);
     }
-    if (rows <= 0) r.shortest = r.longest = 0;
-    return Py_BuildValue("(LLLLLLLL)", r.max_len, r.shortest, r.longest, r.blocked, r.segments_512, r.up_to_512, r.up_to_1024,
-                         r.hub_nonzeros);
+    return built(r);
     } catch (...) {
         return raised();
     }
@@ -443,20 +454,46 @@ struct Waited {
     }
 };
 
+// send_offsets(row offsets on the CPU, memory for them on the GPU, hub_min_len, stream) -> what row_stats says of them: the copy is queued
+// first and runs while they are counted here and by decompose (65 K rows: 17 us on its own).  The caller keeps both until the stream has
+// been waited for, as decompose does.
+PyObject* send_offsets(PyObject*, PyObject* const* args, Py_ssize_t count)
+{
+    try {
+    const at::Tensor *host = count == 4 ? strided_of(args[0]) : nullptr, *dev = host ? strided_of(args[1]) : nullptr;
+    long long hub_min_len, stream;
+    if (!dev || !int_of(args[2], hub_min_len) || !int_of(args[3], stream) || !host->is_cpu() || !dev->is_cuda() || host->scalar_type() != at::kInt ||
+        dev->scalar_type() != at::kInt || host->dim() != 1 || dev->dim() != 1 || host->size(0) < 1 || host->size(0) != dev->size(0) ||
+        !host->is_contiguous() || !dev->is_contiguous())
+        return PyErr_Format(PyExc_ValueError, "send_offsets takes int32 row offsets on the CPU and memory for them on the GPU");
+    RowStats r;
+    int code;
+    {
+        NoGil no_gil;
+        code = hipMemcpyAsync(data(*dev), data(*host), (size_t)host->size(0) * sizeof(int), hipMemcpyHostToDevice, reinterpret_cast<hipStream_t>(stream));
+        r = stats_of(*host, hub_min_len);
+    }
+    return code != 0 ? failed("hipMemcpyAsync", code) : built(r);
+    } catch (...) {
+        return raised();
+    }
+}
+
 // decompose(row offsets on the CPU, the same on the GPU, columns or None, dense rows, segment
 // length, stream[, upload]) -> (block_indices, st_offsets, residue_indices, m1, m2, plan, counts): the row
 // decomposition and, with the columns given, the descriptors of a locality plan (tensor and its
 // four counts; else None, None).  The list lengths are counted here, so that the lists are
 // allocated at their size and everything is queued at once: one wait for the whole of it
 // instead of one for the counts, one for the plan and a copy of every list.  With `upload`, the offsets on the GPU are still to be
-// filled: their copy runs while the lists are counted here (65 K rows: 17 us on its own, hidden but for the 5 us of starting it).
+// filled: their copy runs while the lists are counted here (65 K rows: 17 us on its own, hidden but for the 5 us of starting it); `upload`
+// None: send_offsets has queued it.  Either way the GPU's offsets are the host's, and the lists are placed by what is counted here, tile by tile.
 PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
     try {
     long long dense_rows, seg, stream;
     if ((count != 6 && count != 7) || !int_of(args[3], dense_rows) || !int_of(args[4], seg) || !int_of(args[5], stream))
         return PyErr_Format(PyExc_ValueError, "decompose takes 6 or 7 arguments");
-    const bool upload = count == 7 && args[6] == Py_True;
+    const bool upload = count == 7 && args[6] == Py_True, same = upload || (count == 7 && args[6] == Py_None);
     const at::Tensor *host = strided_of(args[0]), *dev = strided_of(args[1]), *col = args[2] == Py_None ? nullptr : strided_of(args[2]);
     if (!host || !dev || !host->is_cpu() || !dev->is_cuda() || host->scalar_type() != at::kInt || dev->scalar_type() != at::kInt ||
         host->dim() != 1 || dev->dim() != 1 || host->size(0) < 1 || host->size(0) != dev->size(0) || !host->is_contiguous() ||
@@ -472,32 +509,49 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         NoGil no_gil;
         hipStream_t s = reinterpret_cast<hipStream_t>(stream);
         Waited queued{s}; // (also when an allocation below fails)
+        queued.used = same;
         if (upload) {
-            queued.used = true;
             what = "hipMemcpyAsync";
             code = hipMemcpyAsync(data(*dev), data(*host), (size_t)(m + 1) * sizeof(int), hipMemcpyHostToDevice, s);
         }
-        list_sizes(static_cast<const int32_t*>(data(*host)), m, (int)seg, m1, m2);
+        const int32_t* offsets = static_cast<const int32_t*>(data(*host));
+        const long long tile = same && m > 0 ? rode_hip_preprocess_tile_rows((int)m) : 0, tiles = tile > 0 ? (m + tile - 1) / tile : 0;
+        // (pinned: the kernels read what lies before every tile and write the counts where the host reads them)
+        counts = at::empty({8 + 2 * tiles}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        int* h = static_cast<int*>(data(counts));
+        unsigned long long* before = reinterpret_cast<unsigned long long*>(h + 8);
+        if (tiles > 0) {
+            for (long long t = 0; t < tiles; ++t) {
+                long long b, r;
+                before[t] = (unsigned long long)m1 << 32 | (unsigned long long)m2;
+                list_sizes(offsets + t * tile, std::min(tile, m - t * tile), (int)seg, b, r);
+                m1 += b, m2 += r;
+            }
+        } else {
+            list_sizes(offsets, m, (int)seg, m1, m2);
+        }
         blk = m1 > 0 ? at::empty({m1}, dev->options()) : at::zeros({1}, dev->options()); // (an empty list has one place that is never read)
         start = at::empty({m1 + 1}, dev->options());
         res = m2 > 0 ? at::empty({m2}, dev->options()) : at::zeros({1}, dev->options());
-        const size_t ws_bytes = rode_hip_preprocess_workspace_bytes((int)m);
-        scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
+        const size_t ws_bytes = tiles > 0 ? 0 : rode_hip_preprocess_workspace_bytes((int)m);
+        if (tiles == 0) scratch = at::empty({(int64_t)((ws_bytes + 7) / 8)}, dev->options().dtype(at::kLong));
         size_t plan_bytes = 0;
         if (col && m2 > 0) {
             plan_bytes = rode_hip_window_plan_bytes((int)m2);
             plan = at::empty({(int64_t)(plan_bytes / 4)}, dev->options());
         }
-        // (pinned: the kernels write the counts where the host reads them)
-        counts = at::empty({8}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
-        int *h = static_cast<int*>(data(counts)), *segments = static_cast<int*>(data(blk)), *starts = static_cast<int*>(data(start));
+        int *segments = static_cast<int*>(data(blk)), *starts = static_cast<int*>(data(start));
         int* rows = static_cast<int*>(data(res));
         h[0] = h[1] = -1;
         const int *rp = static_cast<const int*>(data(*dev)), *columns = plan_bytes ? static_cast<const int*>(data(*col)) : nullptr;
-        void *work = data(scratch), *windows = plan_bytes ? data(plan) : nullptr;
+        void *work = tiles > 0 ? nullptr : data(scratch), *windows = plan_bytes ? data(plan) : nullptr;
         // From here to the end of the wait nothing throws: what is queued uses the memory above.
         queued.used = true;
-        if (code == 0 && plan_bytes) {
+        if (code == 0 && tiles > 0) {
+            what = "rode_hip_preprocess_placed";
+            code = rode_hip_preprocess_placed((int)seg, (int)m, rp, segments, starts, rows, h, (int)m1, (int)m2, before, (int)dense_rows, columns, windows,
+                                              plan_bytes, s);
+        } else if (code == 0 && plan_bytes) {
             what = "rode_hip_preprocess_with_plan";
             code = rode_hip_preprocess_with_plan((int)seg, (int)m, rp, segments, starts, rows, h, (int)m1, work, ws_bytes, (int)m2, (int)dense_rows, columns,
                                                  windows, plan_bytes, s);
@@ -524,6 +578,8 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
 PyMethodDef methods[] = {
     {"row_stats", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(row_stats)), METH_FASTCALL,
      "row_stats(row_offsets, hub_min_len) -> (max_len, shortest, longest, blocked, segments_512, up_to_512, up_to_1024, hub_nonzeros)"},
+    {"send_offsets", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(send_offsets)), METH_FASTCALL,
+     "send_offsets(row_offsets_cpu, row_offsets, hub_min_len, stream) -> row_stats(row_offsets_cpu, hub_min_len), the copy to the GPU queued"},
     {"decompose", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(decompose)), METH_FASTCALL,
      "decompose(row_offsets_cpu, row_offsets, columns or None, dense_rows, seg_length, stream[, upload]) -> (block, start, residue, m1, m2, plan, counts)"},
     {"sddmm", reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(sddmm)), METH_FASTCALL,

@@ -16,6 +16,10 @@ hipError_t preprocess_static_workspace(void** ptr);
 hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind,
                              int* st_off, int* residue_r_ind, int* n_blk, int* n_res, void* workspace,
                              int capacity_blocks, hipStream_t stream, int plan_chunks = 0, int* plan_header = nullptr);
+int preprocess_tile_rows(int M);
+hipError_t preprocess_placed_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind, int* st_off,
+                                    int* residue_r_ind, int* n_blk, int* n_res, const unsigned long long* before, int capacity_blocks,
+                                    int capacity_residue, hipStream_t stream, int plan_chunks, int* plan_header);
 
 // T = dense operand type; values, accumulators and C are float for T = float / __half
 // and double for T = double.

@@ -58,25 +58,39 @@ class RoDeCSR:
             # what the operand checks of the ops compare with
             self.device = torch.device("cuda", torch.cuda.current_device())
         self.row_offsets_cpu = row_offsets.to(dtype=torch.int32, device="cpu").contiguous()
-        # one pass over the row offsets: the longest row, the choice of the segment length and of a plan
-        self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len(8))
+        if isinstance(config, str) and config != "auto":
+            raise ValueError(f'config must be a dict, None or "auto", got {config!r}')
+        if locality not in (True, False, "auto"):
+            raise ValueError(f'locality must be True, False or "auto", got {locality!r}')
+        # one pass over the row offsets: the longest row, the choice of the segment length and of a plan; on a GPU their copy there is
+        # queued first, and nobody waits for it before the decomposition
+        if self.device.type == "cuda":
+            with rode_sddmm_hip._on_device(self.device):
+                self.row_offsets = torch.empty(self.row_offsets_cpu.shape, dtype=torch.int32, device=self.device)
+                try:
+                    self._stats = _lib.host_call().send_offsets(self.row_offsets_cpu, self.row_offsets, self._hub_min_len(8),
+                                                                rode_sddmm_hip._stream_handle(self.device))
+                    self._set_up(column_indices, values, config, locality)
+                except BaseException:
+                    torch.cuda.current_stream(self.device).synchronize()  # (the copy reads the caller's memory)
+                    raise
+        else:
+            self._stats = _lib.host_call().row_stats(self.row_offsets_cpu, self._hub_min_len(8))
+            self.row_offsets = torch.empty(self.row_offsets_cpu.shape, dtype=torch.int32, device=self.device)
+            self._set_up(column_indices, values, config, locality)
+
+    def _set_up(self, column_indices, values, config, locality):
         self.max_row_length = self._stats[0]
-        if isinstance(config, str):
-            if config != "auto":
-                raise ValueError(f'config must be a dict, None or "auto", got {config!r}')
+        if config == "auto":
             config = self._config_from(self._stats)
-        self.config = dict(config) if config is not None else dict(self.CONFIGS.get(k, self.DEFAULT_CONFIG))
+        self.config = dict(config) if config is not None else dict(self.CONFIGS.get(self.k, self.DEFAULT_CONFIG))
         cfg = self.config
         if cfg.get("k_block") != 32 or cfg.get("vec_len") != 4 or cfg.get("seg_length", 0) <= 0 \
                 or cfg["seg_length"] % 32 != 0:
             # the kernels process 32-slot chunks from 4-aligned offsets, as the reference's do
             raise ValueError(f"config must have k_block=32, vec_len=4 and seg_length a positive multiple of 32, got {cfg}")
-
         self.column_indices = column_indices.to(dtype=torch.int32, device=self.device).contiguous()
         self.values = values.to(dtype=torch.float32, device=self.device).contiguous()
-        self.row_offsets = torch.empty(self.row_offsets_cpu.shape, dtype=torch.int32, device=self.device) # (filled along with the decomposition)
-        if locality not in (True, False, "auto"):
-            raise ValueError(f'locality must be True, False or "auto", got {locality!r}')
         self.locality = locality
         self._shared = {}  # per-pattern cache (the transposed pattern); with_values() copies share it
         self._preprocess()
@@ -133,7 +147,7 @@ class RoDeCSR:
         with rode_sddmm_hip._on_device(self.device):
             blk, st, res, m1, m2, data, counts = _lib.host_call().decompose(
                 self.row_offsets_cpu, self.row_offsets, self.column_indices if self.locality and not others else None,
-                self.n, self.config["seg_length"], rode_sddmm_hip._stream_handle(self.device), True)
+                self.n, self.config["seg_length"], rode_sddmm_hip._stream_handle(self.device), None)
         self.block_indices = blk
         self.st_offsets = st
         self.residue_indices = res

@@ -189,3 +189,31 @@ def test_host_pointer_twins():
     assert (nb.value, nr.value) == (0, 0) and one[0] == 0
     assert host(0, 32, 4, 0, z.ctypes.data, one.ctypes.data, one.ctypes.data, one.ctypes.data,
                 ctypes.addressof(nb), ctypes.addressof(nr)) != 0
+
+
+@pytest.mark.parametrize("m", [1, 255, 256, 257, 128 * 1024, 128 * 1024 + 1, 512 * 1024 + 1, 1024 * 1024 + 1])
+def test_lists_placed_by_the_host_equal_the_scanned_ones(m):
+    """The lists whose places the host has counted, tile by tile, against those that the kernel places itself, around the sizes of the
+    tiles (256 rows, 1024 above 128 K, 4096 above 512 K, 8192 above 1 M), with rows above a tile's own list and a hub; byte for byte."""
+    from rode_amd import _lib, rode_sddmm_hip
+    rng = np.random.default_rng(m)
+    lens = rng.integers(0, 90, m)
+    lens[m // 2] = 70000
+    ro = torch.from_numpy(np.concatenate(([0], np.cumsum(lens))).astype(np.int32))
+    stream = rode_sddmm_hip._stream_handle(torch.device("cuda"))
+    want = rode_sddmm_hip.preprocess_device(ro.cuda(), int(ro[-1]), 512, 32, 4)
+    dev = torch.full((m + 1,), -1, dtype=torch.int32, device="cuda")
+    stats = _lib.host_call().send_offsets(ro, dev, 1000, stream)
+    assert stats == _lib.host_call().row_stats(ro, 1000)
+    blk, st, res, m1, m2, plan, counts = _lib.host_call().decompose(ro, dev, None, 1, 512, stream, None)
+    assert torch.equal(dev.cpu(), ro) and (m1, m2) == tuple(want[3:]) and plan is None and counts is None
+    assert torch.equal(blk[:m1], want[0][:m1]) and torch.equal(st, want[1]) and torch.equal(res[:m2], want[2][:m2])
+
+
+def test_what_is_sent_is_checked():
+    from rode_amd import _lib
+    send = _lib.host_call().send_offsets
+    ro, dev = torch.zeros(5, dtype=torch.int32), torch.zeros(5, dtype=torch.int32, device="cuda")
+    for bad in ((ro.long(), dev), (ro, dev[:4]), (ro, ro), (dev, dev), (ro, dev.long()), (ro[:0], dev[:0]), (ro.repeat(2)[::2], dev), (None, dev)):
+        with pytest.raises((ValueError, TypeError)):
+            send(*bad, 8, 0)
