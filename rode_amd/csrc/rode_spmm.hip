@@ -29,6 +29,7 @@
 #include "rode_units.hpp"
 #include "rode_internal.hpp"
 
+#include <climits>
 #include <type_traits>
 
 namespace rode {
@@ -58,6 +59,26 @@ constexpr int kShortRowSlots = 384;
 // Without the promise the block kernel may still merge the short segments of a row that
 // the list it was given holds, when there are this many of them.
 constexpr int kMergeMinSegments = 16384;
+// Rows longer than one wave sums (kOwnedRowSlots), where C is not cleared: the four waves of a workgroup sum such a row, a quarter each with the
+// tail in it, the sums meet in LDS and the row is stored.  Adding to it, segment by segment, takes C cleared before, a launch of 3 to
+// 5 us that reads every row offset.  The workgroup is the first whose four segments are all the row's (there is one among any seven
+// consecutive ones); a row that has none is summed by the wave of its first segment, whatever its length.
+// Where it pays (us, cleared and added to -> stored; lognormal degrees, rows of mean degree x width, longest row L): what a row of L slots
+// takes, about 3.5 ns a slot, is nowhere to be seen while the others take longer.
+//   * L up to 4096: 16 K of 16 x 64 17.1 -> 13.8 (L 2603), 25 K of 10 x 32 11.8 -> 8.3, 36 K of 10 halves x 32 12.5 -> 8.9, 30 K of 24 halves x 128
+//     24.7 -> 20.9, 42 K of 15 x 128 34.7 -> 31.3, 65 K of 16 x 128 60.3 -> 57.0, 100 K of 16 x 64 52.8 -> 49.6 (3349); above it, with less than
+//     300 MB of dense rows to gather: 36 K of 22 halves x 64 18.8 -> 24.8 (6973), 20 K of 26 x 96 25.0 -> 26.4 (5736), 16 K of 32 halves x 32
+//     13.1 -> 11.9 (5206);
+//   * L up to 6656 from 300 MB on: 27 K of 26 x 128 33.4 -> 29.4 (5640), 59 K of 30 halves x 128 52.8 -> 47.8 (6141), 51 K of 19 x 128 50.1 -> 47.6
+//     (6677); 29 K of 32 x 128 40.4 -> 41.9 (7741);
+//   * segments of more than 128 slots, whose rows of up to six segments may have no workgroup, from 500 MB on: 200 K of 16 x 64 120.4 -> 116.5,
+//     150 K x 128 167 -> 163, 180 K of 20 halves x 128 135 -> 132; 113 K of 23 x 32, 332 MB, 44.7 -> 49.6.
+inline bool wide_rows_pay(int longest, int seg_length, size_t gathered)
+{
+    constexpr size_t MB = 1000000;
+    if (seg_length > (gathered >= 500 * MB ? 512 : 128)) return false;
+    return (size_t)longest <= (gathered < 300 * MB ? 4096 : max((size_t)6656, gathered / 100000));
+}
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
 // are processed by one launch (spmm_pair_kernel).  Above it the residue kernel runs on its
@@ -108,13 +129,15 @@ inline bool sharding_pays(int lines, bool halves, size_t dense_rows, long long i
 // last quad are neutralised.  Every lane of the wave returns the wave's total.
 // (split, jump: the slots are [base, base + split) followed by [base + split + jump, ...):
 // a row with a hole that somebody else works on; split >= cnt for one plain range.)
-// PARTS: every 64 slots have a sum of their own, and the total is the sum of those.
-template <typename T, int TN, bool PARTS = false>
+// PART: so many slots (0: all) have a sum of their own, and the total is the sum of those (more than one step's: kept in LDS, in this
+// lane's place `parked`; in registers they cost the kernel of 32-column tiles a wave per SIMD).
+template <typename T, int TN, int PART = 0>
 __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int split, int jump, int lane, int* my_c,
                                                typename DenseVec<T>::Acc* my_v, const T* b_lane, int n,
                                                const int* __restrict__ col,
                                                const typename DenseVec<T>::Acc* __restrict__ val,
-                                               typename DenseVec<T>::Acc (&total)[SpmmShape<T, TN>::kVec])
+                                               typename DenseVec<T>::Acc (&total)[SpmmShape<T, TN>::kVec],
+                                               typename DenseVec<T>::Acc* parked = nullptr)
 {
     using S = SpmmShape<T, TN>;
     using A = typename S::Acc;
@@ -138,7 +161,9 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
     int c = 0;
     A v = A(0);
     fetch(0, c, v);
-    for (int off = 0; off < cnt; off += kWave) {
+    static_assert(PART % kWave == 0, "whole steps");
+    for (int off = 0, end = PART > kWave ? min(PART, cnt) : cnt;;) {
+    for (; off < end; off += kWave) {
         const int slot = off + lane;
         const int live = min(cnt - off, kWave); // 64, or less on the last step
         my_c[lane] = c;
@@ -151,14 +176,22 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
             spmm_gather<T, TN, 16 / G, true>(b_lane, (size_t)n, acc, my_c, my_v, group, G, 16);
         else
             spmm_gather<T, TN, 16 / G, false>(b_lane, (size_t)n, acc, my_c, my_v, group, G, (live + 3) / 4);
-        if constexpr (PARTS) {
+        if constexpr (PART == kWave) {
 #pragma unroll
             for (int x = 0; x < VEC; ++x) parts[x] += acc[x], acc[x] = A(0);
         }
         wave_lds_sync();
     }
+    if (PART <= kWave || off >= cnt) break;
 #pragma unroll
-    for (int x = 0; x < VEC; ++x) total[x] = butterfly_sum<LPR, kWave>(PARTS ? parts[x] : acc[x]);
+    for (int x = 0; x < VEC; ++x) parked[x] = off > PART ? parked[x] + acc[x] : acc[x], acc[x] = A(0);
+    end = min(off + PART, cnt);
+    }
+#pragma unroll
+    for (int x = 0; x < VEC; ++x) {
+        if (PART > kWave && cnt > PART) acc[x] += parked[x];
+        total[x] = butterfly_sum<LPR, kWave>(PART == kWave ? parts[x] : acc[x]);
+    }
 }
 
 // Which column tile of C, and which of the `blocks` workgroups of its grid row, a workgroup is.
@@ -175,11 +208,32 @@ __device__ __forceinline__ TilePlace tile_place(int b, int blocks, int shards)
     return TilePlace{at % (blocks / kXcds) * kXcds + at / (blocks / kXcds), x % shards};
 }
 
+// The work item of the wave of segment `seg` (of a workgroup that has kWavesPerWg consecutive ones) where workgroups take long rows
+// (wide_rows_pay); not whole: a quarter of the row.
+__device__ __forceinline__ bool spmm_wide_item(int seg, int m1, int owned_slots, const int* __restrict__ block_rows, const int* __restrict__ row_ptr,
+                                               BlockItem& it)
+{
+    const int row = block_rows[seg];
+    const int row_start = row_ptr[row], row_end = row_ptr[row + 1], mask = row_start & (kVecLen - 1), base = row_start - mask;
+    const bool first = seg == 0 || block_rows[seg - 1] != row;
+    it.row = row, it.mask = mask, it.base = base, it.cnt = row_end - base, it.whole = true;
+    if (it.cnt <= owned_slots) return first;
+    auto all_of = [&](int s) { return s >= 0 && s + kWavesPerWg <= m1 && block_rows[s] == row && block_rows[s + kWavesPerWg - 1] == row; };
+    const int mine = seg / kWavesPerWg * kWavesPerWg;
+    if (all_of(mine)) {
+        if (mine > 0 && all_of(mine - kWavesPerWg)) return false; // (the workgroup before has the row)
+        const int each = (it.cnt + kWavesPerWg * kWave - 1) / (kWavesPerWg * kWave) * kWave, from = (seg - mine) * each;
+        it.base = base + from, it.mask = from == 0 ? mask : 0, it.cnt = min(each, it.cnt - from), it.whole = false;
+        return true;
+    }
+    return first && !all_of(seg == mine ? mine : mine + kWavesPerWg);
+}
+
 // One wave per block segment (see sddmm_block_kernel for the slot arithmetic,
 // identical at RoDeSpmm.cu:210-234).
 // (bid of nblocks: the workgroup's position in the part of the grid that works on block segments)
 // WALK: 0 one wave per segment only, 1 chunks only (chunk_hint > 1), 2 either, found out here; 3 one wave per segment, which
-// sums its row in parts (kShortRowSlots).
+// sums its row in parts (kShortRowSlots); 4 (with STORE) one per segment too, and a workgroup for a row of more than owned_slots (wide_rows_pay).
 // (Kernels of their own, so that the code of one way does not cost the other registers.)
 // STORE: a row's only work item stores its sum instead of adding it (owners.overwrite; a
 // kernel of its own as well: as a run-time branch it slowed the fp16 kernel of width 128
@@ -207,7 +261,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     if constexpr (WALK == 2)
         chunk = block_chunk_for_grid(owned_slots != 0 && m1 >= kWalkMinSegments ? block_chunk(m1, block_rows, st_off) : 1, m1,
                                      nblocks);
-    if (WALK != 0 && WALK != 3 && chunk > 1) {
+    if (WALK != 0 && WALK < 3 && chunk > 1) {
         const long long first = chunk_first_segment(bid, wave, m1, chunk);
         if (first < 0) return;
         const int last = (int)min(first + chunk, (long long)m1);
@@ -256,7 +310,8 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     const int seg0 = xcd_logical_block(bid, nblocks) * kWavesPerWg;
     const int seg = seg0 + wave;
     BlockItem it{-1, 0, 0, 0};
-    const bool active = seg < m1 && spmm_block_item(seg, m1, owned_slots, owners, lane, block_rows, st_off, row_ptr, it);
+    const bool active = seg < m1 && (WALK == 4 ? spmm_wide_item(seg, m1, owned_slots, block_rows, row_ptr, it)
+                                               : spmm_block_item(seg, m1, owned_slots, owners, lane, block_rows, st_off, row_ptr, it));
     // A wave without a work item leaves at once (with the reference's 32-slot segments that
     // is most waves); the barrier below then counts only the waves that are still running
     // (S_BARRIER waits on the surviving waves of a workgroup).
@@ -267,8 +322,13 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     // such work items instead of one each.
     int item_row[kWavesPerWg]; // the row of each wave's work item, -1: that wave has none (and has left)
     bool shared_row = false;
+    if constexpr (WALK == 4) {
+        shared_row = !it.whole;
 #pragma unroll
-    for (int i = 0; i < kWavesPerWg; ++i) {
+        for (int i = 0; i < kWavesPerWg; ++i) item_row[i] = it.row; // (of a row that is shared)
+    }
+#pragma unroll
+    for (int i = 0; WALK != 4 && i < kWavesPerWg; ++i) {
         item_row[i] = spmm_block_leader_row(seg0 + i, m1, owned_slots, owners, block_rows, st_off, row_ptr);
         if (i > 0) shared_row = shared_row || (item_row[i] >= 0 && item_row[i] == item_row[i - 1]);
     }
@@ -284,8 +344,10 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
 
     // combine the lane groups, then spread the atomics over them
     constexpr int EPG = VEC / G > 0 ? VEC / G : 1; // elements each group adds
+    constexpr int kPart = WALK == 3 ? kWave : WALK == 4 ? kSpmmMergeSlots : 0;
     A total[VEC];
-    spmm_sum_slots<T, TN, WALK == 3>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total);
+    __shared__ __attribute__((aligned(16))) A parked[kPart > kWave ? kWgThreads * VEC : 1];
+    spmm_sum_slots<T, TN, kPart>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total, parked + (kPart > kWave ? threadIdx.x * VEC : 0));
     if (shared_row) {
         __shared__ __attribute__((aligned(16))) A wg_sum[kWavesPerWg][TN];
         if (group == 0) {
@@ -309,7 +371,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
         if (!first_of_run) return;
     }
     A* c_lane = C + (size_t)row * n + tile + ls * VEC;
-    if (STORE && it.whole) { // the row's only work item (the same in every lane): nothing to add to
+    if (STORE && (WALK == 4 || it.whole)) { // the row's only work item (the same in every lane): nothing to add to
 #pragma unroll
         for (int x = 0; x < VEC; ++x)
             if (group == x / EPG && col_ok) c_lane[x] = total[x];
@@ -428,10 +490,7 @@ spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners
 
 // The rows of C without slots, which are in neither list, where nobody cleared C: 64 at a time to the waves, whose lanes zero the tile of
 // several rows at once, 16 bytes each.  (A matrix may be mostly such rows: in waves of 256 that took one after the other, 100 K x 128 with
-// 50 rows that are not empty took 29.4 us instead of 12.8 with a clearing launch, 1 M x 32 34 instead of 22.) (Rows of more than 1024
-// slots, which several waves add to, still need the launch before: with a workgroup for each of them in here spmm of 65 K x 128, ten such
-// rows, took 57.8 us instead of 60.0, but the registers of that cost the kernel a wave per SIMD: 40 K rows of 32 x 64 38.6 -> 43.2,
-// lognormal 100 K of 16 x 32 30.4 -> 35.3.)
+// 50 rows that are not empty took 29.4 us instead of 12.8 with a clearing launch, 1 M x 32 34 instead of 22.)
 template <typename A, int TN, bool EDGE>
 __device__ __forceinline__ void spmm_empty_rows(int bid, int nblocks, int tile, int rows, int n, const int* __restrict__ row_ptr, A* __restrict__ C)
 {
@@ -476,7 +535,7 @@ spmm_pair_kernel(int shards, int g0, int rows, int g1, int m1, int m2, int n, in
         spmm_block_body<T, TN, EDGE, WALK, STORE>(at.bid, g, at.tile * TN, m1, n, owned_slots, chunk_hint, owners, block_rows, st_off, row_ptr, col, val,
                                         B, C);
     else
-        spmm_residue_body<T, TN, EDGE>(at.bid, g, at.tile * TN, m2, n, max(owned_slots, 0), owners, residue_rows,
+        spmm_residue_body<T, TN, EDGE>(at.bid, g, at.tile * TN, m2, n, WALK == 4 ? INT_MAX : max(owned_slots, 0), owners, residue_rows,
                                        row_ptr, col, val,
                                        B, C, plan);
 }
@@ -878,8 +937,11 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     const bool pair = (block || alone) && residue && standard_residue && s1 == s2 &&
                       (long long)(g1 + g2) * tiles <= (shards > 1 ? kPairMaxSharded : kPairMaxWorkgroups);
     int g0 = 0;
+    bool wide = false;
     if (plan.c_rows > 0) { // C is not cleared
-        if (pair && owners.overwrite && !group_plan && plan.dev == nullptr && plan.longest > 0 && plan.longest <= kOwnedRowSlots) {
+        const bool all_stored = pair && owners.overwrite && !group_plan && plan.dev == nullptr && plan.longest > 0;
+        wide = all_stored && chunk_hint == 1 && plan.longest > kOwnedRowSlots && wide_rows_pay(plan.longest, plan.seg_length, (size_t)plan.nonzeros * n * sizeof(T));
+        if (wide || (all_stored && plan.longest <= kOwnedRowSlots)) {
             g0 = empty_row_workgroups(plan.c_rows);
         } else {
             e = spmm_clear_rows_launch(plan.c_rows, (size_t)n * sizeof(typename DenseVec<T>::Acc), owners.overwrite ? kOwnedRowSlots : 0, row_ptr, C, s1);
@@ -891,6 +953,8 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         auto kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 2, true> : spmm_pair_kernel<T, TN, EDGE, 2, false>;
         if (in_parts)
             kernel = spmm_pair_kernel<T, TN, EDGE, 3, true>;
+        else if (wide)
+            kernel = spmm_pair_kernel<T, TN, EDGE, 4, true>;
         else if (chunk_hint == 1)
             kernel = owners.overwrite ? spmm_pair_kernel<T, TN, EDGE, 0, true> : spmm_pair_kernel<T, TN, EDGE, 0, false>;
         else if (chunk_hint > 1)

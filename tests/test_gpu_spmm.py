@@ -809,3 +809,45 @@ def test_new_product_with_plans(kind, k, dtype):
     for longest in (csr.longest_row, 0):
         got = _into_nan(csr, B, longest, plans)
         assert (np.abs(got - want) <= scale * (lens[:, None] + 2) * (2.0 ** -52 if dtype == "f64" else 2.0 ** -24)).all()
+
+
+@pytest.mark.parametrize("k,dtype", [(32, "f32"), (64, "f32"), (96, "f32"), (128, "f32"), (200, "f32"), (32, "f16"), (64, "f16"), (128, "f16"), (64, "f64")])
+@pytest.mark.parametrize("seg,said", [(128, 128), (32, 32), (512, 128)])
+def test_long_rows_by_a_workgroup_each(seg, said, k, dtype):
+    """Rows of 1000 to 4096 aligned slots, which the waves of a workgroup share, into NaN: at the bounds of what one wave sums (1024), of a
+    part (512 of a quarter) and of the row (4096), at every place in a workgroup, first and last in the lists, next to each other and beside
+    empty rows; and, where the segments are longer than said, rows that have no workgroup.  NaN and Inf in dense rows that no long row uses."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, rode_sddmm_hip
+    rng = np.random.default_rng(seg + k)
+    long_ones = [4090, 1024, 1025, 1026, 1023, 1027, 1030, 2047, 2048, 2049, 2052, 3000, 4093, 1100, 1300, 1537, 1800, 2560, 4089]
+    dealt = (k, dtype, seg) == (128, "f32", 128)  # (column tiles dealt out to the XCDs: 4 MB of dense rows, few segments beside the tails)
+    m, n = (8000, 9000) if dealt else (3000, 6000)
+    lens = rng.integers(0, 36 if dealt else 70, m)
+    lens[rng.choice(m, m // 8, replace=False)] = 0
+    lens[0], lens[-1] = 4080, 2200
+    at = np.arange(40, 40 + 97 * len(long_ones), 97)
+    lens[at] = long_ones
+    lens[at[5] + 1: at[5] + 3] = 1200, 1500
+    lens[at[7] - 1] = lens[at[7] + 1] = 0
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n - 1, L, replace=False)) for L in lens]).astype(np.int32)
+    short = np.flatnonzero((lens > 0) & (lens < 1000))[17]
+    col[rp[short + 1] - 1] = n - 1  # the one nonzero of the last column
+    val, dense = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    dense = round_half(dense) if dtype == "f16" else dense
+    dense[n - 1] = np.inf
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, config={"seg_length": seg, "k_block": 32, "vec_len": 4},
+                  locality=False)
+    csr = csr.with_values(csr.values.double()) if dtype == "f64" else csr
+    assert csr.m1 >= 1024 and (not dealt or 3 * csr.m1 <= csr.m2)  # (as many segments as the rule for whole rows wants)
+    assert 4090 <= csr.longest_row <= 4096
+    B = torch.from_numpy(dense).to(DEV, {"f32": torch.float32, "f16": torch.float16, "f64": torch.float64}[dtype])
+    got = _into_nan(csr, B, csr.longest_row, rode_sddmm_hip.plans_struct(None, whole_lists=True, seg_length=said))
+    assert not np.isfinite(got[short]).any()
+    dense[n - 1] = 0
+    want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
+    got[short] = want[short]
+    # roundings of a sum: 512 slots over two lane groups, seven more parts, the groups (5), the waves (3) and the product
+    assert (np.abs(got - want) <= scale * (256 + 7 + 5 + 3 + 1) * (2.0 ** -53 if dtype == "f64" else 2.0 ** -24)).all()
