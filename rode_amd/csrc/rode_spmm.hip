@@ -64,20 +64,23 @@ constexpr int kMergeMinSegments = 16384;
 // 5 us that reads every row offset.  The workgroup is the first whose four segments are all the row's (there is one among any seven
 // consecutive ones); a row that has none is summed by the wave of its first segment, whatever its length.
 // Where it pays (us, cleared and added to -> stored; lognormal degrees, rows of mean degree x width, longest row L): what a row of L slots
-// takes, about 3.5 ns a slot, is nowhere to be seen while the others take longer.
+// takes - 1.1 to 1.6 ns a slot on an idle GPU with tiles of 128 bytes, 2 with 256, 4.5 with 512, 3.5 in a large matrix - is nowhere to be seen
+// while the others take longer.
 //   * L up to 4096: 16 K of 16 x 64 17.1 -> 13.8 (L 2603), 25 K of 10 x 32 11.8 -> 8.3, 36 K of 10 halves x 32 12.5 -> 8.9, 30 K of 24 halves x 128
 //     24.7 -> 20.9, 42 K of 15 x 128 34.7 -> 31.3, 65 K of 16 x 128 60.3 -> 57.0, 100 K of 16 x 64 52.8 -> 49.6 (3349); above it, with less than
 //     300 MB of dense rows to gather: 36 K of 22 halves x 64 18.8 -> 24.8 (6973), 20 K of 26 x 96 25.0 -> 26.4 (5736), 16 K of 32 halves x 32
-//     13.1 -> 11.9 (5206);
+//     13.1 -> 11.9 (5206).  Up to 3072 for tiles of 256 bytes (8000 rows of 40 halves x 128, L 2000 14.7 -> 12.1, 3000 14.8 -> 14.6, 4000 15.2 -> 16.8;
+//     3000 x 64 2000 11.0 -> 7.3, 3000 11.5 -> 9.4, 4000 11.5 -> 11.1), 2048 of 512 (8000 x 128 2000 20.3 -> 19.4, 3000 20.9 -> 24.9);
 //   * L up to 6656 from 300 MB on: 27 K of 26 x 128 33.4 -> 29.4 (5640), 59 K of 30 halves x 128 52.8 -> 47.8 (6141), 51 K of 19 x 128 50.1 -> 47.6
 //     (6677); 29 K of 32 x 128 40.4 -> 41.9 (7741);
 //   * segments of more than 128 slots, whose rows of up to six segments may have no workgroup, from 500 MB on: 200 K of 16 x 64 120.4 -> 116.5,
 //     150 K x 128 167 -> 163, 180 K of 20 halves x 128 135 -> 132; 113 K of 23 x 32, 332 MB, 44.7 -> 49.6.
-inline bool wide_rows_pay(int longest, int seg_length, size_t gathered)
+inline bool wide_rows_pay(int longest, int seg_length, size_t tile_bytes, size_t gathered)
 {
     constexpr size_t MB = 1000000;
     if (seg_length > (gathered >= 500 * MB ? 512 : 128)) return false;
-    return (size_t)longest <= (gathered < 300 * MB ? 4096 : max((size_t)6656, gathered / 100000));
+    if (gathered < (tile_bytes > 256 ? 500 : 300) * MB) return longest <= (tile_bytes > 256 ? 2048 : tile_bytes > 128 ? 3072 : 4096);
+    return (size_t)longest <= max((size_t)6656, gathered / 100000);
 }
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
@@ -940,7 +943,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     bool wide = false;
     if (plan.c_rows > 0) { // C is not cleared
         const bool all_stored = pair && owners.overwrite && !group_plan && plan.dev == nullptr && plan.longest > 0;
-        wide = all_stored && chunk_hint == 1 && plan.longest > kOwnedRowSlots && wide_rows_pay(plan.longest, plan.seg_length, (size_t)plan.nonzeros * n * sizeof(T));
+        wide = all_stored && chunk_hint == 1 && plan.longest > kOwnedRowSlots && wide_rows_pay(plan.longest, plan.seg_length, TN * sizeof(T), (size_t)plan.nonzeros * n * sizeof(T));
         if (wide || (all_stored && plan.longest <= kOwnedRowSlots)) {
             g0 = empty_row_workgroups(plan.c_rows);
         } else {
