@@ -206,11 +206,19 @@ int rode_hip_preprocess_with_plan(int seg_length, int M, const int* d_row_ptr, i
  * m2 residue rows, and before[t] = the segments (upper 32 bits) and residue rows (lower 32) of all rows before row
  * t * rode_hip_preprocess_tile_rows(M), for every t up to the last row, in memory that the GPU can read (pinned memory).  d_plan NULL: no plan
  * (one launch).  The lists are written up to m1 and m2 entries, whatever the offsets on the GPU say; h_counts as above.
+ *
+ * places, for a matrix of which rode_hip_preprocess_plan_too says 1 (else NULL): lists and plan in one launch.  places[c] = the tile (upper 32 bits)
+ * that holds residue row 128 c and the residue rows of that tile before it (lower 32), for every chunk of 128 residue rows, and
+ * h_windows has an int for every chunk, both in memory that the GPU reaches.  Once the stream has been waited for, h_windows[c] says whether chunk c
+ * has a window; the caller counts them and enters the number with rode_hip_window_plan_count (0 stands there already), h_counts + 4
+ * is left alone.  A chunk's workgroup goes through the rows from places[c] on, which is short work only where most rows are residue rows.
  */
 int rode_hip_preprocess_tile_rows(int M);
 int rode_hip_preprocess_placed(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind, int* h_counts,
                                int m1, int m2, const unsigned long long* before, int dense_rows, const int* d_column_indices, void* d_plan,
-                               size_t plan_bytes, void* stream);
+                               size_t plan_bytes, const unsigned long long* places, int* h_windows, void* stream);
+int rode_hip_preprocess_plan_too(int M);
+int rode_hip_window_plan_count(int m2, int windowed, void* d_plan, size_t plan_bytes, void* stream);
 size_t rode_hip_window_rows_bytes(int m2);
 int rode_hip_window_rows(int m2, const int* d_row_indices_residue, const int* d_row_offsets,
                          const int* d_column_indices, const void* d_plan, void* d_rows, size_t rows_bytes, void* stream);

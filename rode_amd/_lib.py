@@ -28,7 +28,9 @@ SIGNATURES = {
     "rode_hip_window_plan_bytes": (c_size_t, [c_int]),
     "rode_hip_window_plan": (c_int, [c_int] * 2 + [c_void_p] * 4 + [c_size_t, c_void_p, c_void_p]),
     "rode_hip_preprocess_tile_rows": (c_int, [c_int]),
-    "rode_hip_preprocess_placed": (c_int, [c_int, c_int] + [c_void_p] * 5 + [c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
+    "rode_hip_preprocess_placed": (c_int, [c_int, c_int] + [c_void_p] * 5 + [c_int, c_int, c_void_p, c_int, c_void_p, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p]),
+    "rode_hip_preprocess_plan_too": (c_int, [c_int]),
+    "rode_hip_window_plan_count": (c_int, [c_int, c_int, c_void_p, c_size_t, c_void_p]),
     "rode_hip_window_rows_bytes": (c_size_t, [c_int]),
     "rode_hip_window_rows": (c_int, [c_int] + [c_void_p] * 5 + [c_size_t, c_void_p]),
     "rode_hip_group_plan_bytes": (c_size_t, [c_int]),

@@ -517,14 +517,20 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         const int32_t* offsets = static_cast<const int32_t*>(data(*host));
         const long long tile = same && m > 0 ? rode_hip_preprocess_tile_rows((int)m) : 0, tiles = tile > 0 ? (m + tile - 1) / tile : 0;
         // (pinned: the kernels read what lies before every tile and write the counts where the host reads them)
-        counts = at::empty({8 + 2 * tiles}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        const long long chunks_most = tiles > 0 && col && rode_hip_preprocess_plan_too((int)m) ? (m + 127) / 128 : 0;
+        counts = at::empty({8 + 2 * tiles + 3 * chunks_most}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
         int* h = static_cast<int*>(data(counts));
         unsigned long long* before = reinterpret_cast<unsigned long long*>(h + 8);
+        unsigned long long* places = before + tiles;
+        int* has_window = reinterpret_cast<int*>(places + chunks_most);
         if (tiles > 0) {
+            long long chunk = 0;
             for (long long t = 0; t < tiles; ++t) {
                 long long b, r;
                 before[t] = (unsigned long long)m1 << 32 | (unsigned long long)m2;
                 list_sizes(offsets + t * tile, std::min(tile, m - t * tile), (int)seg, b, r);
+                for (; chunk < chunks_most && 128 * chunk < m2 + r; ++chunk)
+                    places[chunk] = (unsigned long long)t << 32 | (unsigned long long)(128 * chunk - m2);
                 m1 += b, m2 += r;
             }
         } else {
@@ -547,10 +553,12 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         void *work = tiles > 0 ? nullptr : data(scratch), *windows = plan_bytes ? data(plan) : nullptr;
         // From here to the end of the wait nothing throws: what is queued uses the memory above.
         queued.used = true;
+        // (list and plan at once: a chunk's workgroup goes through two rows for a residue row at most)
+        const bool at_once = chunks_most > 0 && plan_bytes > 0 && 2 * m2 >= m;
         if (code == 0 && tiles > 0) {
             what = "rode_hip_preprocess_placed";
             code = rode_hip_preprocess_placed((int)seg, (int)m, rp, segments, starts, rows, h, (int)m1, (int)m2, before, (int)dense_rows, columns, windows,
-                                              plan_bytes, s);
+                                              plan_bytes, at_once ? places : nullptr, has_window, s);
         } else if (code == 0 && plan_bytes) {
             what = "rode_hip_preprocess_with_plan";
             code = rode_hip_preprocess_with_plan((int)seg, (int)m, rp, segments, starts, rows, h, (int)m1, work, ws_bytes, (int)m2, (int)dense_rows, columns,
@@ -561,6 +569,14 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         }
         const int waited = queued.wait(); // (also after an error: the scratch is in use until then)
         if (code == 0) code = waited;
+        if (code == 0 && at_once) {
+            h[4] = (int)((m2 + 127) / 128), h[5] = h[6] = h[7] = 0;
+            for (int c = 0; c < h[4]; ++c) h[5] += has_window[c] != 0;
+            if (h[5] > 0) {
+                what = "rode_hip_window_plan_count";
+                code = rode_hip_window_plan_count((int)m2, h[5], windows, plan_bytes, s);
+            }
+        }
         if (code == 0 && (h[0] != m1 || h[1] != m2)) error = "the row decomposition on the GPU does not have the expected size";
     }
     if (!error.empty()) return PyErr_Format(PyExc_RuntimeError, "%s", error.c_str());

@@ -124,17 +124,27 @@ int rode_hip_preprocess_tile_rows(int M) { return rode::preprocess_tile_rows(M);
 
 int rode_hip_preprocess_placed(int seg_length, int M, const int* d_row_ptr, int* d_block_r_ind, int* d_st_off, int* d_residue_r_ind, int* h_counts,
                                int m1, int m2, const unsigned long long* before, int dense_rows, const int* d_column_indices, void* d_plan,
-                               size_t plan_bytes, void* stream)
+                               size_t plan_bytes, const unsigned long long* places, int* h_windows, void* stream)
 {
     if (seg_length <= 0 || M <= 0 || m1 < 0 || m2 < 0 || dense_rows < 0) return hipErrorInvalidValue;
     if (!d_row_ptr || !d_block_r_ind || !d_st_off || !d_residue_r_ind || !h_counts || !before || (reinterpret_cast<uintptr_t>(before) & 7u))
         return hipErrorInvalidValue;
     if (d_plan && (m2 == 0 || !d_column_indices || plan_bytes < rode_hip_window_plan_bytes(m2) || !aligned16(d_plan))) return hipErrorInvalidValue;
+    if (places && (!d_plan || !h_windows || !rode::preprocess_plan_too(M) || (reinterpret_cast<uintptr_t>(places) & 7u))) return hipErrorInvalidValue;
     int* plan = static_cast<int*>(d_plan);
     const hipError_t e = rode::preprocess_placed_launch(seg_length, 32, 4, M, d_row_ptr, d_block_r_ind, d_st_off, d_residue_r_ind, h_counts,
-                                                        h_counts + 1, before, m1, m2, as_stream(stream), plan ? rode::window_plan_chunks(m2) : 0, plan);
-    if (e != hipSuccess || !plan) return e;
+                                                        h_counts + 1, before, m1, m2, as_stream(stream), plan ? rode::window_plan_chunks(m2) : 0, plan,
+                                                        places, dense_rows, d_column_indices, h_windows);
+    if (e != hipSuccess || !plan || places) return e;
     return rode::window_plan_launch(m2, dense_rows, d_residue_r_ind, d_row_ptr, d_column_indices, plan, as_stream(stream), h_counts + 4);
+}
+
+int rode_hip_preprocess_plan_too(int M) { return rode::preprocess_plan_too(M) ? 1 : 0; }
+
+int rode_hip_window_plan_count(int m2, int windowed, void* d_plan, size_t plan_bytes, void* stream)
+{
+    if (m2 < 0 || windowed < 0 || !d_plan || !aligned16(d_plan) || plan_bytes < rode_hip_window_plan_bytes(m2)) return hipErrorInvalidValue;
+    return rode::window_plan_header_launch(m2, windowed, static_cast<int*>(d_plan), as_stream(stream));
 }
 
 size_t rode_hip_window_plan_bytes(int m2) { return m2 < 0 ? 0 : rode::window_plan_ints(m2) * sizeof(int); }

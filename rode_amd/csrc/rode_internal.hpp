@@ -19,7 +19,9 @@ hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* 
 int preprocess_tile_rows(int M);
 hipError_t preprocess_placed_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind, int* st_off,
                                     int* residue_r_ind, int* n_blk, int* n_res, const unsigned long long* before, int capacity_blocks,
-                                    int capacity_residue, hipStream_t stream, int plan_chunks, int* plan_header);
+                                    int capacity_residue, hipStream_t stream, int plan_chunks, int* plan_header,
+                                    const unsigned long long* places, int dense_rows, const int* col, int* windows);
+bool preprocess_plan_too(int M); // does it take `places`?
 
 // T = dense operand type; values, accumulators and C are float for T = float / __half
 // and double for T = double.
@@ -197,6 +199,7 @@ size_t window_plan_rows_bytes(int m2);
 // (header_counts: null, or where the last workgroup writes the header's four ints; the header itself is then cleared already,
 // by preprocess_launch, which has `chunks` from window_plan_chunks)
 int window_plan_chunks(int m2);
+hipError_t window_plan_header_launch(int m2, int windowed, int* plan, hipStream_t stream);
 hipError_t window_plan_launch(int m2, int dense_rows, const int* residue_rows, const int* row_ptr, const int* col,
                               int* plan, hipStream_t stream, int* header_counts = nullptr);
 hipError_t window_plan_rows_launch(int m2, const int* residue_rows, const int* row_ptr, const int* col, const int* plan,

@@ -336,9 +336,8 @@ struct ResidueItem {
     bool accumulate;
 };
 
-__device__ __forceinline__ ResidueItem residue_item(int row, const int* __restrict__ row_ptr)
+__device__ __forceinline__ ResidueItem residue_item_of(int s, int e) // (a row's slots [s, e))
 {
-    const int s = row_ptr[row], e = row_ptr[row + 1];
     const int pad = s & (kVecLen - 1);
     ResidueItem it;
     it.aligned = e - s + pad;
@@ -347,6 +346,7 @@ __device__ __forceinline__ ResidueItem residue_item(int row, const int* __restri
     it.cnt = it.accumulate ? it.aligned % kBlockItems : e - s;
     return it;
 }
+__device__ __forceinline__ ResidueItem residue_item(int row, const int* __restrict__ row_ptr) { return residue_item_of(row_ptr[row], row_ptr[row + 1]); }
 
 // ---- locality plan --------------------------------------------------------------
 // A plan cuts the residue list into chunks of consecutive entries and says, for every

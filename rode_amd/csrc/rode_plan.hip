@@ -19,42 +19,21 @@
 // What bounds it: the chain of loads that wait for one another (list entry, row offset, column), with a few workgroups
 // per CU; 65 K rows with 2 M nonzeros: 14.1 us with the counts written to the host from here, 15.5 with one slot of a thread
 // at a time.  Before, 13.2, a launch of 2.0 that set up the header and a copy of 3.7 that brought the counts to the host.
-#include "rode_items.hpp"
+#include "rode_plan.hpp"
 #include "rode_internal.hpp"
-
-#include <climits>
 
 namespace rode {
 
 namespace {
 
-__global__ void plan_header_kernel(int m2, int* __restrict__ plan)
+__global__ void plan_header_kernel(int m2, int windowed, int* __restrict__ plan)
 {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         plan[0] = plan_residue_chunks(m2);
-        plan[1] = 0;
+        plan[1] = windowed;
         plan[2] = 0;
         plan[3] = 0;
     }
-}
-
-__device__ __forceinline__ int wave_reduce_add(int v)
-{
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, kWave);
-    return v;
-}
-__device__ __forceinline__ int wave_reduce_min(int v)
-{
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d, kWave));
-    return v;
-}
-__device__ __forceinline__ int wave_reduce_max(int v)
-{
-#pragma unroll
-    for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
-    return v;
 }
 
 __global__ void __launch_bounds__(kWgThreads)
@@ -62,23 +41,17 @@ plan_chunks_kernel(int m2, int dense_rows, const int* __restrict__ residue_rows,
                    const int* __restrict__ col, int* plan, int* host_counts)
 {
     constexpr int CH = kPlanResidueChunk;
-    constexpr int ROWS_MAX = kResidueWindowRowsMax;
-    static_assert(CH <= kWgThreads, "one thread per entry");
-    __shared__ int first[CH];
-    __shared__ int prefix[CH + 1];
-    __shared__ __attribute__((aligned(16))) int samples[kWgThreads];
-    __shared__ int quart[2];
-    __shared__ int red[3][kWavesPerWg];
-
-    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    __shared__ PlanChunkLds lds;
+    const int tid = threadIdx.x;
     const int chunk = blockIdx.x;
     const int e0 = chunk * CH;
     const int ne = min(CH, m2 - e0);
     int* desc = plan + kPlanHeaderInts + kPlanDescInts * chunk;
     // (one thread) the chunk's descriptor; where the counts go to the host, the last chunk to come here writes them there (one
     // 64-bit counter in the header's last two ints, which end as zero: the chunks done, and above them those with a window)
-    auto finish = [&](int w0, int wn, int slots, int misses) {
-        *reinterpret_cast<int4*>(desc) = make_int4(w0, wn, slots, misses);
+    auto finish = [&](int4 d) {
+        *reinterpret_cast<int4*>(desc) = d;
+        const int wn = d.y;
         if (host_counts == nullptr) {
             if (wn > 0) atomicAdd(plan + 1, 1);
             return;
@@ -92,108 +65,14 @@ plan_chunks_kernel(int m2, int dense_rows, const int* __restrict__ residue_rows,
         host_counts[0] = gridDim.x, host_counts[1] = windowed, host_counts[2] = 0, host_counts[3] = 0;
     };
 
-    // 1. slot range of every entry
     int my_len = 0;
     if (tid < ne) {
         const ResidueItem it = residue_item(residue_rows[e0 + tid], row_ptr);
-        first[tid] = it.first;
+        lds.first[tid] = it.first;
         my_len = it.cnt;
     }
-    static_assert(CH == 2 * kWave, "two waves have the entries");
-    int through = my_len;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int up = __shfl_up(through, d, kWave);
-        if (lane >= d) through += up;
-    }
-    if (tid == kWave - 1) red[0][0] = through;
-    __syncthreads();
-    if (tid < CH) prefix[tid + 1] = through + (wave > 0 ? red[0][0] : 0);
-    if (tid == 0) prefix[0] = 0;
-    if (tid < 2) quart[tid] = INT_MIN;
-    __syncthreads();
-    const int total = prefix[CH];
-    if (total <= 0) {
-        if (tid == 0) finish(0, 0, 0, 0);
-        return;
-    }
-    // entry that holds slot p of the chunk: the last e with prefix[e] <= p
-    auto entry_of = [&](int p) {
-        int lo = 0;
-#pragma unroll
-        for (int half = CH / 2; half > 0; half /= 2) lo += prefix[lo + half] <= p ? half : 0;
-        return lo;
-    };
-
-    // 2. samples and their quartiles
-    {
-        const int p = (int)(((long long)tid * total + total / 2) / kWgThreads);
-        const int e = entry_of(p);
-        samples[tid] = col[first[e] + (p - prefix[e])];
-    }
-    __syncthreads();
-    // the value of rank r is the largest one that at most r of the samples are below
-    {
-        const int mine = samples[tid];
-        int below = 0;
-#pragma unroll 4
-        for (int j = 0; j < kWgThreads; j += 4) {
-            const int4 other = *reinterpret_cast<const int4*>(samples + j);
-            below += (other.x < mine ? 1 : 0) + (other.y < mine ? 1 : 0) + (other.z < mine ? 1 : 0) + (other.w < mine ? 1 : 0);
-        }
-        if (below <= kWgThreads / 4) atomicMax(quart, mine);
-        if (below <= kWgThreads * 3 / 4 - 1) atomicMax(quart + 1, mine);
-    }
-    __syncthreads();
-    const int q25 = quart[0], q75 = quart[1];
-    if ((long long)q75 - q25 + 1 > ROWS_MAX || dense_rows <= 0) {
-        if (tid == 0) finish(0, 0, total, total);
-        return;
-    }
-    int w0 = q25 + (q75 - q25) / 2 - ROWS_MAX / 2;
-    w0 = max(0, min(w0, dense_rows - ROWS_MAX));
-    const int wend = min(dense_rows, w0 + ROWS_MAX);
-
-    // 3. hits and their extent
-    int hits = 0, lo_hit = 0x7fffffff, hi_hit = -1;
-    // (kAhead slots of a thread at a time: each is a search and a load that waits for it)
-    constexpr int kAhead = 8;
-    for (int p0 = tid; p0 < total; p0 += kAhead * kWgThreads) {
-        int c[kAhead];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-            const int p = min(p0 + i * kWgThreads, total - 1), e = entry_of(p);
-            c[i] = col[first[e] + (p - prefix[e])];
-        }
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-            if (p0 + i * kWgThreads < total && c[i] >= w0 && c[i] < wend) {
-                ++hits;
-                lo_hit = min(lo_hit, c[i]);
-                hi_hit = max(hi_hit, c[i]);
-            }
-        }
-    }
-    hits = wave_reduce_add(hits);
-    lo_hit = wave_reduce_min(lo_hit);
-    hi_hit = wave_reduce_max(hi_hit);
-    if (lane == 0) {
-        red[0][wave] = hits;
-        red[1][wave] = lo_hit;
-        red[2][wave] = hi_hit;
-    }
-    __syncthreads();
-    if (tid == 0) {
-        for (int w = 1; w < kWavesPerWg; ++w) {
-            hits += red[0][w];
-            lo_hit = min(lo_hit, red[1][w]);
-            hi_hit = max(hi_hit, red[2][w]);
-        }
-        // 4. decision
-        const int wn = hi_hit - lo_hit + 1;
-        const bool take = hits > 0 && 2ll * hits >= total && hits >= 2ll * wn;
-        finish(take ? lo_hit : 0, take ? wn : 0, total, total - hits);
-    }
+    const int4 d = plan_chunk(lds, my_len, dense_rows, col);
+    if (tid == 0) finish(d);
 }
 
 // Fills the PlannedChunk of every chunk that has a window: 8 threads per residue row.
@@ -283,10 +162,16 @@ size_t window_plan_ints(int m2) { return plan_ints(m2); }
 int window_plan_chunks(int m2) { return plan_residue_chunks(m2); }
 size_t window_plan_rows_bytes(int m2) { return (size_t)plan_residue_chunks(m2) * sizeof(PlannedChunk); }
 
+hipError_t window_plan_header_launch(int m2, int windowed, int* plan, hipStream_t stream)
+{
+    plan_header_kernel<<<1, kWave, 0, stream>>>(m2, windowed, plan);
+    return hipGetLastError();
+}
+
 hipError_t window_plan_launch(int m2, int dense_rows, const int* residue_rows, const int* row_ptr, const int* col,
                               int* plan, hipStream_t stream, int* header_counts)
 {
-    if (header_counts == nullptr) plan_header_kernel<<<1, kWave, 0, stream>>>(m2, plan);
+    if (header_counts == nullptr) plan_header_kernel<<<1, kWave, 0, stream>>>(m2, 0, plan);
     const int chunks = plan_residue_chunks(m2);
     if (chunks > 0) {
         plan_chunks_kernel<<<chunks, kWgThreads, 0, stream>>>(m2, dense_rows, residue_rows, row_ptr, col, plan, header_counts);

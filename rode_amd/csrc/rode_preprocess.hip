@@ -11,6 +11,7 @@
 // array and writes the lists from the scanned offsets, a row with many
 // segments by a whole wave.
 #include "rode_device.hpp"
+#include "rode_plan.hpp"
 #include "rode_internal.hpp"
 
 #include <mutex>
@@ -156,8 +157,8 @@ constexpr int kMaxPolls = 1 << 22;
 // and a whole `RoDeCSR` of 2 M nonzeros, with the offsets on their way before they are counted, 68.7 -> 64.6 (130 K rows 96.6 -> 88.2).
 // (capacity_residue: no list is written past what the caller counted, whatever the offsets say; plan_header: as clear_status_kernel's.)
 template <int THREADS, int RPT, bool PLACED>
-__global__ void __launch_bounds__(THREADS)
-decompose_kernel(Params p, int M, int ntiles, int capacity, int capacity_residue, const int* __restrict__ row_ptr,
+__device__ __forceinline__ void
+decompose_tile(int tile, Params p, int M, int ntiles, int capacity, int capacity_residue, const int* __restrict__ row_ptr,
                  unsigned long long* __restrict__ ws, int* __restrict__ block_r_ind, int* __restrict__ st_off,
                  int* __restrict__ residue_r_ind, int* __restrict__ n_blk, int* __restrict__ n_res, int plan_chunks, int* __restrict__ plan_header)
 {
@@ -172,7 +173,6 @@ decompose_kernel(Params p, int M, int ntiles, int capacity, int capacity_residue
     unsigned long long* counter = ws;       // [0] tickets
     unsigned long long* status = ws + 2;    // one word per tile
     const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
-    int tile = blockIdx.x;
     unsigned long long known = 0;
     if constexpr (PLACED) {
         if (tid == 0) known = ws[tile]; // (it may lie in the host's memory: on its way while the rows are counted)
@@ -281,6 +281,69 @@ decompose_kernel(Params p, int M, int ntiles, int capacity, int capacity_residue
     }
 }
 
+template <int THREADS, int RPT, bool PLACED>
+__global__ void __launch_bounds__(THREADS)
+decompose_kernel(Params p, int M, int ntiles, int capacity, int capacity_residue, const int* __restrict__ row_ptr,
+                 unsigned long long* __restrict__ ws, int* __restrict__ block_r_ind, int* __restrict__ st_off,
+                 int* __restrict__ residue_r_ind, int* __restrict__ n_blk, int* __restrict__ n_res, int plan_chunks, int* __restrict__ plan_header)
+{
+    decompose_tile<THREADS, RPT, PLACED>(blockIdx.x, p, M, ntiles, capacity, capacity_residue, row_ptr, ws, block_r_ind, st_off, residue_r_ind, n_blk,
+                                         n_res, plan_chunks, plan_header);
+}
+
+// The lists and the descriptors of a locality plan at once, the first `chunks` workgroups a chunk each.  Such a workgroup does not wait for the
+// residue list: where its 128 entries begin - a tile, and how many entries of that tile come before - is known as `before` is, and it
+// goes through the rows from there.  Which chunks have a window goes to `windows`, in the host's memory too.  65 K rows, 2 M nonzeros: lists, then
+// plan 7.5 + 14.3 us -> 13.5, a whole `RoDeCSR` 63.5 -> 55.6 (16 K rows of 8 47.8 -> 43.6, 130 K of 16 88.0 -> 76.5, 400 K of 10 186 -> 164).  For tiles
+// of up to 512 K rows: the larger ones have workgroups of 1024 threads.
+template <int THREADS, int RPT>
+__global__ void __launch_bounds__(THREADS)
+decompose_plan_kernel(Params p, int M, int ntiles, int capacity, int capacity_residue, const int* __restrict__ row_ptr,
+                      unsigned long long* __restrict__ before, int* __restrict__ block_r_ind, int* __restrict__ st_off, int* __restrict__ residue_r_ind,
+                      int* __restrict__ n_blk, int* __restrict__ n_res, int chunks, const unsigned long long* __restrict__ places, int dense_rows,
+                      const int* __restrict__ col, int* __restrict__ plan, int* __restrict__ windows)
+{
+    static_assert(THREADS == kWgThreads, "a workgroup for a tile or a chunk");
+    if ((int)blockIdx.x >= chunks) {
+        decompose_tile<THREADS, RPT, true>(blockIdx.x - chunks, p, M, ntiles, capacity, capacity_residue, row_ptr, before, block_r_ind, st_off,
+                                           residue_r_ind, n_blk, n_res, chunks, plan);
+        return;
+    }
+    constexpr int CH = kPlanResidueChunk;
+    __shared__ PlanChunkLds lds;
+    __shared__ int lens[CH], found[kWavesPerWg];
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave, chunk = blockIdx.x;
+    const int entries = min(CH, capacity_residue - chunk * CH);
+    const unsigned long long place = places[chunk];
+    if (tid < CH) lds.first[tid] = lens[tid] = 0;
+    int at = -(int)(place & 0xffffffffull); // of the next residue row, counted from the chunk's first
+    for (long long row = (long long)(place >> 32) * (THREADS * RPT); row < M && at < entries; row += THREADS) {
+        const long long r = row + tid;
+        const int s = r < M ? row_ptr[r] : 0, e = r < M ? row_ptr[r + 1] : 0;
+        const bool mine = (row_counts(p, s, e) & 1ull) != 0;
+        const unsigned long long all = __ballot(mine);
+        if (lane == 0) found[wave] = __builtin_popcountll(all);
+        __syncthreads();
+        int here = at + __builtin_popcountll(all & ((1ull << lane) - 1ull));
+#pragma unroll
+        for (int w = 0; w < kWavesPerWg; ++w) {
+            here += w < wave ? found[w] : 0;
+            at += found[w];
+        }
+        if (mine && here >= 0 && here < entries) {
+            const ResidueItem it = residue_item_of(s, e);
+            lds.first[here] = it.first, lens[here] = it.cnt;
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    const int4 d = plan_chunk(lds, tid < CH ? lens[tid] : 0, dense_rows, col);
+    if (tid == 0) {
+        *reinterpret_cast<int4*>(plan + kPlanHeaderInts + kPlanDescInts * chunk) = d;
+        windows[chunk] = d.y > 0 ? 1 : 0;
+    }
+}
+
 // M == 0: no tile runs; counts and sentinel all the same.
 __global__ void empty_matrix_kernel(const int* __restrict__ row_ptr, int* __restrict__ st_off, int* __restrict__ n_blk,
                                     int* __restrict__ n_res)
@@ -341,15 +404,25 @@ hipError_t preprocess_launch(int seg, int kblock, int veclen, int M, const int* 
 }
 
 int preprocess_tile_rows(int M) { return tile_shape_for((size_t)(M > 0 ? M : 0)).rows(); }
+bool preprocess_plan_too(int M) { return M > 0 && tile_shape_for((size_t)M).threads == kWgThreads; }
 
-// The lists of a caller that has counted them, tile by tile (before: ... up to a tile).
+// The lists of a caller that has counted them, tile by tile (before: ... up to a tile; places: of the plan's chunks, or null, for tiles of
+// workgroups of kWgThreads).
 hipError_t preprocess_placed_launch(int seg, int kblock, int veclen, int M, const int* row_ptr, int* block_r_ind, int* st_off,
                                     int* residue_r_ind, int* n_blk, int* n_res, const unsigned long long* before, int capacity_blocks,
-                                    int capacity_residue, hipStream_t stream, int plan_chunks, int* plan_header)
+                                    int capacity_residue, hipStream_t stream, int plan_chunks, int* plan_header,
+                                    const unsigned long long* places, int dense_rows, const int* col, int* windows)
 {
     const TileShape shape = tile_shape_for((size_t)M);
     const int ntiles = (int)(((size_t)M + shape.rows() - 1) / shape.rows());
     unsigned long long* ws = const_cast<unsigned long long*>(before); // (only read)
+    if (places) { // list and plan at once (preprocess_plan_tile_rows)
+        auto kernel = shape.rows_per_thread == 1 ? decompose_plan_kernel<kWgThreads, 1> : decompose_plan_kernel<kWgThreads, 4>;
+        kernel<<<plan_chunks + ntiles, kWgThreads, 0, stream>>>(make_params(seg, kblock, veclen), M, ntiles, capacity_blocks, capacity_residue, row_ptr, ws,
+                                                                block_r_ind, st_off, residue_r_ind, n_blk, n_res, plan_chunks, places, dense_rows, col,
+                                                                plan_header, windows);
+        return hipGetLastError();
+    }
 #define RODE_DECOMPOSE(THREADS, RPT)                                                                                       \
     decompose_kernel<THREADS, RPT, true><<<ntiles, THREADS, 0, stream>>>(make_params(seg, kblock, veclen), M, ntiles, capacity_blocks, capacity_residue, \
                                                                          row_ptr, ws, block_r_ind, st_off, residue_r_ind, n_blk, n_res, plan_chunks, plan_header)

@@ -217,3 +217,31 @@ def test_what_is_sent_is_checked():
     for bad in ((ro.long(), dev), (ro, dev[:4]), (ro, ro), (dev, dev), (ro, dev.long()), (ro[:0], dev[:0]), (ro.repeat(2)[::2], dev), (None, dev)):
         with pytest.raises((ValueError, TypeError)):
             send(*bad, 8, 0)
+
+
+@pytest.mark.parametrize("share", [1.0, 0.55, 0.45])  # of residue rows: list and plan at once from one half on
+@pytest.mark.parametrize("m", [1, 300, 128 * 1024, 128 * 1024 + 1, 512 * 1024])
+def test_plan_made_along_with_the_lists(m, share):
+    """Lists and plan of one launch (tiles of 256 rows and, above 128 K, of 1024) against the separate kernels, byte for byte: chunks that begin
+    anywhere in a tile and go on over several, rows without residue and without slots, the last chunk part of one."""
+    from rode_amd import _lib, rode_sddmm_hip
+    rng = np.random.default_rng(int(m + 100 * share))
+    listed = rng.random(m) < share
+    lens = np.where(listed, 4 * rng.integers(1, 8, m), 32 * rng.integers(0, 2, m))  # (starts are multiples of four)
+    ro = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    row = np.repeat(np.arange(m), lens)
+    col = np.where(row // 1000 % 3 == 1, rng.integers(0, m, len(row)), np.clip(row + rng.integers(-90, 91, len(row)), 0, m - 1)).astype(np.int32)
+    host, cols = torch.from_numpy(ro), torch.from_numpy(np.append(col, np.int32(0))).cuda()[:len(col)]
+    stream = rode_sddmm_hip._stream_handle(torch.device("cuda"))
+    dev = torch.empty(m + 1, dtype=torch.int32, device="cuda")
+    _lib.host_call().send_offsets(host, dev, 1000, stream)
+    blk, st, res, m1, m2, data, counts = _lib.host_call().decompose(host, dev, cols, m, 512, stream, None)
+    parts = rode_sddmm_hip.preprocess_device(dev, int(ro[-1]), 512, 32, 4)
+    assert (m1, m2) == tuple(parts[3:]) and m2 == listed.sum()
+    assert torch.equal(blk[:m1], parts[0][:m1]) and torch.equal(st, parts[1]) and torch.equal(res[:m2], parts[2][:m2])
+    if m2 == 0:
+        assert data is None and counts is None
+        return
+    plan = rode_sddmm_hip.window_plan(res, m2, dev, cols, m)
+    assert counts == plan.counts and data[:4].tolist() == counts and torch.equal(data[4:4 + 4 * counts[0]], plan.data[4:4 + 4 * counts[0]])
+    assert m < 1000 or counts[1] > 0
