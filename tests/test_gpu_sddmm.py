@@ -544,3 +544,32 @@ def test_device_given_without_an_index():
     dense = csr.to_torch_sparse_csr().to_dense()
     assert torch.allclose(C, dense @ rhs, atol=1e-4, rtol=1e-4)
     assert out.shape == (csr.nnz,) and torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("k", [8, 24, 48, 96, 160, 200, 320])
+def test_lanes_past_the_width_add_nothing(k, half):
+    """Widths that leave lanes of a dense row's group without elements: those read the row's first ones and must drop them.  Infinite first
+    elements give infinite products and no NaN, and finite rows what they should, in rows of every kernel (block, residue)."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, rode_sddmm
+    rng = np.random.default_rng(k)
+    m, n = 300, 400
+    lens = rng.integers(0, 60, m)
+    lens[7], lens[100] = 390, 200
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens]).astype(np.int32)
+    val = rng.uniform(0.5, 1, len(col)).astype(np.float32)
+    lhs, rhs = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(0.5, 1, (n, k)).astype(np.float32)
+    lhs, rhs = (round_half(lhs), round_half(rhs)) if half else (lhs, rhs)
+    rhs[::5, 0] = np.inf
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, locality=False)
+    kind = torch.float16 if half else torch.float32
+    got = rode_sddmm(csr, torch.from_numpy(lhs).to(DEV, kind), torch.from_numpy(rhs).to(DEV, kind)).cpu().numpy().astype(np.float64)
+    infinite = col % 5 == 0
+    assert np.isposinf(got[infinite]).all()
+    row = np.repeat(np.arange(m), lens)
+    want = val.astype(np.float64) * np.einsum("ij,ij->i", lhs[row].astype(np.float64), np.where(np.isinf(rhs), 0, rhs)[col].astype(np.float64))
+    # a rounding per product and sum (k of each at most) and the value's; halves' products are exact
+    assert (np.abs(got - want) <= want * (2 * k + 1) * 2.0 ** -24)[~infinite].all()
