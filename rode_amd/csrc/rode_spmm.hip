@@ -1049,14 +1049,40 @@ static int spmm_tile_width(int n, size_t elem)
     return best;
 }
 
+// ... but for some calls whose least padding is with tiles of 32 columns (widths like 96, 160, 224).
+// Halves: such a tile is half a line of 128 bytes, which is fetched for each of the two.  Tiles of 128, and of 64 where the dense operand is
+// near the size of an L2 and its rows are used less than 20 times (us, 32 -> 64 / 128 columns, width 96; uniform (u) and lognormal degrees): u 4000 rows of
+// 40 10.7 -> 8.9 / 7.1, u 8029 of 56 16.1 -> 13.0 / 10.7, u 16 K of 110 34.6 -> 29.4 / 24.1, 60 K of 24 59.0 -> 52.9 / 45.7, 100 K of 20 94 -> 83 / 74,
+// 300 K of 10 189 -> 158 / 132; u 16 K of 20 9.1 -> 8.4 / 9.0, 20 K of 12 12.6 -> 12.0 / 14.0, 26 K of 16 21.4 -> 18.6 / 20.4, 33 K of 10 21.8 -> 21.4 /
+// 23.7, 60 K of 10 29.6 -> 26.7 / 27.1 (16.5 K of 10 9.9 -> 10.5 / 10.9 is the one that loses); width 224 80 K of 20 183 -> 153 / 138.
+// 32-bit operands: one line at a time keeps more of the operand in the L2s, as long as its tiles fit at all (sharding_pays); below 2.5 MB and above
+// 26 MB a tile whole rows are better, if a quarter of the lanes at most has nothing (width 96: u 4000 of 40 9.9 -> 8.2, 230 K of 12 167 -> 161,
+// 300 K of 10 187 -> 178, between them u 8029 of 56 15.3 -> 14.3, u 10 K of 20 8.2 -> 9.0, u 16 K of 110 37 -> 43, 40 K of 20 34.7 -> 43.9; 224: u 2000
+// of 40 11.0 -> 7.9, 300 K 430 -> 393).
+// Where neighbouring rows' columns lie close together the halves of a line meet in the caches anyway (halves, a band of 128, width 96: 70 K of 12
+// 11.9 -> 12.5, but 200 K of 20 55.9 -> 46.7).
+static int spmm_tile_of_call(int n, size_t elem, size_t dense_rows, size_t nonzeros, bool columns_local)
+{
+    const int least = spmm_tile_width(n, elem);
+    if (least != 32 || n <= 32 || elem > 4 || n % 32 != 0) return least;
+    const size_t bytes = dense_rows * n * elem;
+    if (columns_local && bytes < 26000000) return 32;
+    if (elem == 2) return nonzeros > 0 && nonzeros < 20 * dense_rows && bytes >= 3000000 && bytes <= 12000000 ? 64 : 128;
+    const bool whole = dense_rows > 0 && 3 * ((n + 127) / 128 * 128) <= 4 * n && (bytes <= 2500000 || dense_rows * 128 > ((size_t)26 << 20));
+    return whole ? 128 : 32;
+}
+
 // The partial rows that the hub kernels of an SpMM of this width want, for operands of 4 (or, if more, 2) or of 8 bytes an element.
 size_t spmm_hub_partial_rows(const int* counts, int n, int acc_bytes)
 {
     size_t most = 0;
     for (size_t elem = acc_bytes; elem >= (acc_bytes == 8 ? 8 : 2); elem /= 2) {
-        const HubRows use = spmm_hub_rows(counts, n, spmm_tile_width(n, elem), elem);
-        const size_t rows = (size_t)use.rows * hub_groups(counts[1], use.merge);
-        most = rows > most ? rows : most;
+        for (int tile = 32; tile <= (elem > 4 ? 64 : 128); tile *= 2) { // (any that a call of this width may take)
+            if (tile != spmm_tile_width(n, elem) && (n % 32 != 0 || spmm_tile_width(n, elem) != 32 || n == 32)) continue;
+            const HubRows use = spmm_hub_rows(counts, n, tile, elem);
+            const size_t rows = (size_t)use.rows * hub_groups(counts[1], use.merge);
+            most = rows > most ? rows : most;
+        }
     }
     return most;
 }
@@ -1096,7 +1122,7 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
             return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
         }
     }
-    const int best = spmm_tile_width(n, sizeof(T));
+    const int best = spmm_tile_of_call(n, sizeof(T), plan.dense_rows, plan.nonzeros, plan.columns_local);
     if constexpr (sizeof(T) <= 4) {
         if (best == 128)
             return launch_edge<T, 128>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags,

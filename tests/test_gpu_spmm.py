@@ -853,3 +853,24 @@ def test_long_rows_by_a_workgroup_each(seg, said, k, dtype):
     got[short] = want[short]
     # roundings of a sum: 512 slots over two lane groups, seven more parts, the groups (5), the waves (3) and the product
     assert (np.abs(got - want) <= scale * (256 + 7 + 5 + 3 + 1) * (2.0 ** -53 if dtype == "f64" else 2.0 ** -24)).all()
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,n,mean,k", [(300, 500, 20, 96), (300, 500, 20, 224), (2000, 16500, 30, 96), (20000, 20000, 8, 96), (17000, 17000, 6, 160), (500, 215000, 20, 96)])
+def test_tiles_that_are_not_the_least_padded(m, n, mean, k, half):
+    """Widths of 32 (2 i + 1) columns, where the tile follows from the sizes of the call: 32, 64 or 128 columns, the last tile part of one; into NaN."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR
+    rng = np.random.default_rng(m + k)
+    lens = rng.integers(0, 2 * mean, m)
+    lens[m // 2], lens[m // 3] = 400, 1500 if n > 1500 else 450
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    row = np.repeat(np.arange(m), lens)
+    col = ((np.arange(len(row)) - rp[row]) * n // np.maximum(lens[row], 1)).astype(np.int32)  # (ascending, distinct, far apart)
+    val, dense = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    dense = round_half(dense) if half else dense
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, config="auto", locality=False)
+    want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
+    got = _into_nan(csr, torch.from_numpy(dense).to(DEV, torch.float16 if half else torch.float32), csr.longest_row, csr.call_plans())
+    assert (np.abs(got - want) <= scale * (lens[:, None] + 2) * 2.0 ** -24).all()  # (n + 2 roundings)
