@@ -444,7 +444,7 @@ def main():
         table = json.load(open(tpath))
         prefix = f"{args.workload}/k{k}/{args.dtype}/seg{csr.config['seg_length']}/"
         # with a locality plan the residue rows are the window kernel's
-        windowed = csr.plan is not None and hub is None and grp is None and dominant.endswith("residue") and k * elem > 128
+        windowed = csr.plan is not None and hub is None and grp is None and dominant.endswith("residue") and k * elem >= 128
         entry = table.get(prefix + dominant + "_window") if windowed else None
         entry = entry or table.get(prefix + dominant)
         if entry is not None and entry.get("sources") == kernel_sources_fingerprint():
