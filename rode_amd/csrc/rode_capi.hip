@@ -222,14 +222,16 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
     if (M < 0 || !d_plan || !aligned16(d_plan) || !h_counts || plan_bytes < rode_hip_group_plan_bytes(M))
         return hipErrorInvalidValue;
     if (M > 0 && (!d_row_offsets || !d_column_indices)) return hipErrorInvalidValue;
-    int fours[3] = {0, 0, 0};
+    int got[7] = {0, 0, 0, 0, 0, 0, 0};
+    const bool both = h_tile_fours && rode::row_tiles(M) > 0; // (one copy: with a second one and a launch of its own a first training step on a mask took 30 to 45 us longer)
     hipError_t e = rode::group_plan_launch(M, d_row_offsets, d_column_indices, static_cast<int*>(d_plan), as_stream(stream));
-    if (e == hipSuccess) e = hipMemcpyAsync(h_counts, d_plan, 4 * sizeof(int), hipMemcpyDeviceToHost, as_stream(stream));
-    if (e == hipSuccess && h_tile_fours)
-        e = hipMemcpyAsync(fours, static_cast<int*>(d_plan) + rode::group_fours_at(M), sizeof(fours), hipMemcpyDeviceToHost, as_stream(stream));
-    const hipError_t waited = hipStreamSynchronize(as_stream(stream)); // (also after an error: the copies are into memory of this call)
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(both ? got : h_counts, static_cast<int*>(d_plan) + (both ? rode::group_fours_at(M) : 0), both ? sizeof(got) : 4 * sizeof(int),
+                           hipMemcpyDeviceToHost, as_stream(stream));
+    const hipError_t waited = hipStreamSynchronize(as_stream(stream)); // (also after an error: the copy is into memory of this call)
     if (e == hipSuccess) e = waited;
-    if (e == hipSuccess && h_tile_fours) *h_tile_fours = fours[0] == 0 && fours[2] > 0 ? fours[1] / fours[2] : 0;
+    if (e == hipSuccess && both) h_counts[0] = got[4], h_counts[1] = got[5], h_counts[2] = got[6], h_counts[3] = got[3];
+    if (e == hipSuccess && h_tile_fours) *h_tile_fours = got[0] == 0 && got[2] > 0 ? got[1] / got[2] : 0;
     return e;
 }
 

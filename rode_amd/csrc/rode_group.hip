@@ -18,7 +18,7 @@
 //                       of each other;
 //   group_tiles_kernel  per four groups: whether their 16 rows make a tile for the attention
 //                       kernels on the matrix cores (rode_tile.hpp);
-//   group_fours_kernel  per four tiles: whether they lie together.
+//                       and of four neighbouring ones whether they lie together.
 #include "rode_items.hpp"
 #include "rode_internal.hpp"
 
@@ -121,11 +121,10 @@ group_desc_kernel(int groups, const int* __restrict__ row_ptr, const int* __rest
 // the 16 x (hi - lo) rectangle).
 __global__ void __launch_bounds__(kWgThreads)
 group_tiles_kernel(int tiles, const RowGroup* __restrict__ groups, const int* __restrict__ runs, RowTile* __restrict__ out,
-                   int* __restrict__ plan)
+                   int* __restrict__ plan, int* __restrict__ fours)
 {
     const int t = blockIdx.x * kWgThreads + threadIdx.x;
-    if (t >= tiles) return;
-    bool keep = true;
+    bool keep = t < tiles;
 #pragma unroll
     for (int g = 0; g < kTileRows / kGroupRows; ++g) keep = keep && groups[t * (kTileRows / kGroupRows) + g].len > 0;
     RowTile d{0, 0, 0, 0};
@@ -141,23 +140,25 @@ group_tiles_kernel(int tiles, const RowGroup* __restrict__ groups, const int* __
         keep = d.core_hi > d.core_lo && 2ll * kTileRows * (d.hi - d.lo) <= 3 * held;
     }
     if (!keep) d = RowTile{0, 0, 0, 0};
-    out[t] = d;
-    if (keep) atomicAdd(plan + 3, 1);
-}
-
-// Four neighbouring tiles a thread: do they lie together - between them no more than half as many columns again as the widest of
-// them - and how many columns is that (attention_wide_kernel walks them for all four)?
-__global__ void __launch_bounds__(kWgThreads)
-group_fours_kernel(int tiles, const RowTile* __restrict__ tile, int* __restrict__ fours)
-{
-    const int first = (blockIdx.x * kWgThreads + threadIdx.x) * 4;
-    if (first >= tiles) return;
-    int lo = 0x7fffffff, hi = 0, widest = 0;
-    for (int t = first; t < min(first + 4, tiles); ++t) {
-        const RowTile d = tile[t];
-        if (d.hi > d.lo) lo = min(lo, d.lo), hi = max(hi, d.hi), widest = max(widest, d.hi - d.lo);
+    if (t < tiles) out[t] = d;
+    if (keep) {
+        atomicAdd(plan + 3, 1);
+        atomicAdd(fours + 3, 1);
     }
-    if (widest == 0) return;
+    if (t == 0) { // (the header again, beside these: one copy to the host)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) fours[4 + i] = plan[i];
+    }
+    // Four neighbouring tiles, in four lanes: do they lie together - between them no more than half as many columns again as the widest of
+    // them - and how many columns is that (attention_wide_kernel walks them for all four)?
+    int lo = keep ? d.lo : 0x7fffffff, hi = d.hi, widest = d.hi - d.lo;
+#pragma unroll
+    for (int x = 1; x < 4; x *= 2) {
+        lo = min(lo, __shfl_xor(lo, x, kWave));
+        hi = max(hi, __shfl_xor(hi, x, kWave));
+        widest = max(widest, __shfl_xor(widest, x, kWave));
+    }
+    if (threadIdx.x % 4 != 0 || widest == 0) return;
     if (2ll * (hi - lo) > 3ll * widest) {
         atomicAdd(fours, 1);
     } else {
@@ -165,6 +166,7 @@ group_fours_kernel(int tiles, const RowTile* __restrict__ tile, int* __restrict_
         atomicMax(fours + 2, hi - lo);
     }
 }
+
 
 __global__ void group_header_kernel(int M, int groups, int* __restrict__ plan)
 {
@@ -192,8 +194,7 @@ hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* pla
         if (tiles > 0) {
             RowTile* out = reinterpret_cast<RowTile*>(plan + group_tiles_at(M));
             group_tiles_kernel<<<(tiles + kWgThreads - 1) / kWgThreads, kWgThreads, 0, stream>>>(
-                tiles, reinterpret_cast<const RowGroup*>(plan + kGroupHeaderInts), runs, out, plan);
-            group_fours_kernel<<<(tiles + 4 * kWgThreads - 1) / (4 * kWgThreads), kWgThreads, 0, stream>>>(tiles, out, plan + group_fours_at(M));
+                tiles, reinterpret_cast<const RowGroup*>(plan + kGroupHeaderInts), runs, out, plan, plan + group_fours_at(M));
         }
     }
     return hipGetLastError();
