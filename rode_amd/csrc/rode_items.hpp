@@ -384,7 +384,8 @@ struct WindowDesc {
 // for the LDS banks (see below), entry i = (window row of the slot's column) | (slot << 9),
 // slot counted from the row's first residue slot `first`; a slot whose column is outside
 // the window (bit i of missmask) carries the window row of one that is inside; entries
-// cnt..31 repeat such a window row and have no slot (their value is 0).
+// cnt..31 repeat such a window row and have no slot (their value is 0).  In a row without a column in
+// the window those carry a bit of missmask too, and read its first slot's row instead.
 // Order: a ds_read_b128 of a wave serves lane groups (0, 3), (1, 2), (4, 7), (5, 6) in
 // the same cycles, and two 128-byte window rows of equal parity collide in the banks.
 // Rows that lane groups 0, 1, 4, 5 will take list their even window rows first, the rows

@@ -126,7 +126,9 @@ plan_rows_kernel(int m2, const int* __restrict__ residue_rows, const int* __rest
     }
 #pragma unroll
     for (int m = 1; m < L; m <<= 1) best = min(best, (unsigned)__shfl_xor((int)best, m, kWave));
-    if (best == 0xffffu) best = 0; // no slot inside the window: every read is replaced anyway
+    const bool none_inside = best == 0xffffu && cnt > 0;
+    if (best == 0xffffu) best = 0; // no slot inside the window: every read is replaced, those of places that the row does not fill too (by
+                                   // its first slot's: the window's first row is none of this row's, and may hold what times zero is not zero)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront"); // the 8 threads of a row are lanes of one wave
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -142,7 +144,7 @@ plan_rows_kernel(int m2, const int* __restrict__ residue_rows, const int* __rest
         }
         const unsigned where = key == 0 || key == 1 ? u[i] : best;
         out.entry[local][rank] = (unsigned short)(where | (key <= 2 ? (unsigned)s << 9 : 0u));
-        if (key == 2) missbits |= 1u << rank;
+        if (key == 2 || none_inside) missbits |= 1u << rank;
     }
 #pragma unroll
     for (int m = 1; m < L; m <<= 1) missbits |= (unsigned)__shfl_xor((int)missbits, m, kWave);

@@ -285,3 +285,37 @@ def test_rings_against_fp64(m, dtype, k):
     assert m < 128 * 2560 or not torch.equal(got, other)
     want = torch.stack([val.view(m, degree)[:, j].double() * (L.double() * B[col[:, j]].double()).sum(1) for j in range(degree)], 1).flatten()
     assert (rode_sddmm(csr, L, B) - want).abs().max() <= 2e-6 * want.abs().max()
+
+
+@pytest.mark.parametrize("dtype,k", [(torch.float32, 32), (torch.float32, 64), (torch.float32, 128), (torch.float32, 48), (torch.float16, 64),
+                                     (torch.float16, 128), (torch.float64, 16), (torch.float64, 32), (torch.float64, 20)])
+def test_rows_with_no_column_in_their_window_are_not_reached_by_it(dtype, k):
+    """Rows of 1 to 9 columns, none of them in their chunk's window, among rows of 21 that are: the positions that such a row does not fill
+    are not to read a row of the window (the first one is infinite).  Rings and, for the other widths, windows."""
+    one_line = k * torch.finfo(dtype).bits == 128 * 8  # (rows of 128 bytes take a plan only where it pays)
+    m = 128 * (2560 if one_line else 12)
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    row = torch.arange(m, device=DEV)
+    lens = torch.where(row % 5 == 2, 1 + row // 5 % 9, 21)
+    low = (row - 60).clamp(0, m - 120)
+    low = torch.where(lens < 21, (low + m // 2) % (m - 120), low)
+    col = low[:, None] + torch.rand(m, 120, device=DEV, generator=gen).argsort(1)[:, :21]
+    col = torch.where(torch.arange(21, device=DEV) < lens[:, None], col, m).sort(1)[0]
+    col = col[col < m].int()
+    ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0))).int().cpu()
+    csr = RoDeCSR(ro, col, torch.rand(col.numel(), device=DEV, generator=gen) + 0.5, DEV, m, m, k, locality=True)
+    assert csr.plan is not None and csr.plan.windowed == csr.plan.counts[0] == m // 128
+    csr.plan.nonzeros = 31 * csr.m2 if one_line else 0
+    bad = torch.from_numpy(np.unique(csr.plan.descriptors()[:, 0])).to(DEV)
+    B = torch.randn(m, k, device=DEV, dtype=torch.float64, generator=gen).to(dtype)
+    B[bad.long()] = float("inf")
+    if dtype == torch.float64:
+        C = rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets, csr.column_indices,
+                                        csr.values.double(), m, m, B, plan=csr.plan)
+    else:
+        C = rode_spmm(csr, B)
+    finite = torch.isfinite(C).all(1)
+    touched = torch.zeros(m, dtype=torch.bool, device=DEV)
+    touched[row.repeat_interleave(lens)[torch.isin(col, bad)]] = True
+    assert (~touched & (lens < 21)).sum() > 100
+    assert finite[~touched].all() and not finite[touched].any()
