@@ -523,16 +523,22 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         unsigned long long* before = reinterpret_cast<unsigned long long*>(h + 8);
         unsigned long long* places = before + tiles;
         int* has_window = reinterpret_cast<int*>(places + chunks_most);
+        long long most_tiles = 0; // that the residue rows of a chunk lie in, with those between
         if (tiles > 0) {
-            long long chunk = 0;
+            long long chunk = 0, begins = 0, last = 0; // (tiles: of the chunk before, the last one with a residue row)
             for (long long t = 0; t < tiles; ++t) {
                 long long b, r;
                 before[t] = (unsigned long long)m1 << 32 | (unsigned long long)m2;
                 list_sizes(offsets + t * tile, std::min(tile, m - t * tile), (int)seg, b, r);
-                for (; chunk < chunks_most && 128 * chunk < m2 + r; ++chunk)
+                for (; chunk < chunks_most && 128 * chunk < m2 + r; ++chunk) {
                     places[chunk] = (unsigned long long)t << 32 | (unsigned long long)(128 * chunk - m2);
+                    if (chunk > 0) most_tiles = std::max(most_tiles, (128 * chunk > m2 ? t : last) - begins + 1);
+                    begins = t;
+                }
+                if (r > 0) last = t;
                 m1 += b, m2 += r;
             }
+            most_tiles = std::max(most_tiles, last - begins + 1);
         } else {
             list_sizes(offsets, m, (int)seg, m1, m2);
         }
@@ -553,8 +559,12 @@ PyObject* decompose(PyObject*, PyObject* const* args, Py_ssize_t count)
         void *work = tiles > 0 ? nullptr : data(scratch), *windows = plan_bytes ? data(plan) : nullptr;
         // From here to the end of the wait nothing throws: what is queued uses the memory above.
         queued.used = true;
-        // (list and plan at once: a chunk's workgroup goes through two rows for a residue row at most)
-        const bool at_once = chunks_most > 0 && plan_bytes > 0 && 2 * m2 >= m;
+        // List and plan at once: where at least every second row is a residue row, and no chunk's workgroup - it goes through the rows from its
+        // first residue row to its last, 2 us for 1024 - has so many to go through that the two launches are sooner done: a sixteenth of all.
+        // (us of a build, so many empty rows in the middle: at once / two launches, 65 K rows of 21: 2048 61, 4096 64 / 68, 8192 73 / 67, 32 768 120 / 65;
+        // 131 K: 8192 91 / 93, 16 384 107 / 92; 262 K: 16 384 141 / 147, 32 768 173 / 145; 400 K: 16 384 185 / 193, 32 768 214 / 192, 200 000 515 / 173.)
+        const long long walk_rows = std::min(std::max(m / 16, 1024ll), 16384ll);
+        const bool at_once = chunks_most > 0 && plan_bytes > 0 && 2 * m2 >= m && most_tiles * tile <= walk_rows;
         if (code == 0 && tiles > 0) {
             what = "rode_hip_preprocess_placed";
             code = rode_hip_preprocess_placed((int)seg, (int)m, rp, segments, starts, rows, h, (int)m1, (int)m2, before, (int)dense_rows, columns, windows,
