@@ -133,8 +133,8 @@ inline bool sharding_pays(int lines, bool halves, size_t dense_rows, long long i
 // (split, jump: the slots are [base, base + split) followed by [base + split + jump, ...):
 // a row with a hole that somebody else works on; split >= cnt for one plain range.)
 // PART: so many slots (0: all) have a sum of their own, and the total is the sum of those (more than one step's: kept in LDS, in this
-// lane's place `parked`; in registers they cost the kernel of 32-column tiles a wave per SIMD).
-template <typename T, int TN, int PART = 0>
+// lane's place `parked`; in registers they cost the kernel of 32-column tiles a wave per SIMD).  EIGHTS: see spmm_gather.
+template <typename T, int TN, int PART = 0, bool EIGHTS = false>
 __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int split, int jump, int lane, int* my_c,
                                                typename DenseVec<T>::Acc* my_v, const T* b_lane, int n,
                                                const int* __restrict__ col,
@@ -176,9 +176,9 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
         // halves 368 -> 351; lognormal 20 K x 64 19.8 -> 16.9, 65 K x 128 either way; 16 K rows of 100, width 64 25.8 -> 24.6)
         if (off + kWave < cnt) fetch(off + kWave, c, v);
         if (live == kWave)
-            spmm_gather<T, TN, 16 / G, true>(b_lane, (size_t)n, acc, my_c, my_v, group, G, 16);
+            spmm_gather<T, TN, 16 / G, true, EIGHTS>(b_lane, (size_t)n, acc, my_c, my_v, group, G, 16);
         else
-            spmm_gather<T, TN, 16 / G, false>(b_lane, (size_t)n, acc, my_c, my_v, group, G, (live + 3) / 4);
+            spmm_gather<T, TN, 16 / G, false, EIGHTS>(b_lane, (size_t)n, acc, my_c, my_v, group, G, (live + 3) / 4);
         if constexpr (PART == kWave) {
 #pragma unroll
             for (int x = 0; x < VEC; ++x) parts[x] += acc[x], acc[x] = A(0);
@@ -196,6 +196,14 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
         total[x] = butterfly_sum<LPR, kWave>(PART == kWave ? parts[x] : acc[x]);
     }
 }
+
+// Calls of widths that are a multiple of 32 and not of 128 may take tiles of 128 or 64 columns for tiles of 32 (spmm_tile_of_call), with 2 or 4 times
+// fewer lane groups for a row's slots: their sums are made of sums of eight slots.  2-norms of the errors against fp64 relative to tiles of 32
+// (uniform, width 96): one chain a lane group, 40 nonzeros a row 1.31, halves 1.09, 110 halves 1.38; like this, 34 to 110 nonzeros 0.97 to 1.004,
+// halves 0.985 to 1.001.  Time (us, chain -> this): 4000 rows of 56 7.1 -> 7.2, of 110 x 100 11.1 -> 11.1, 60 K of 56 119 -> 119, halves
+// 8000 of 110 11.9 -> 12.2, 16.5 K of 56 17.0 -> 17.2.
+template <typename T, int TN, bool EDGE>
+constexpr bool kInEights = EDGE && TN >= 64 && sizeof(T) <= 4;
 
 // Which column tile of C, and which of the `blocks` workgroups of its grid row, a workgroup is.
 // shards == 1: tiles in blockIdx.y.  shards > 1 (a divisor of kXcds): XCD x only ever works on tile
@@ -293,7 +301,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
             for (unsigned long long todo = scan.items & ((1ull << count) - 1ull); todo; todo &= todo - 1ull) {
                 const BlockItem it = chunk_item(scan, __builtin_ctzll(todo));
                 A total[VEC];
-                spmm_sum_slots<T, TN>(it.base, it.mask, it.cnt, it.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave,
+                spmm_sum_slots<T, TN, 0, kInEights<T, TN, EDGE>>(it.base, it.mask, it.cnt, it.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave,
                                       b_lane, n, col, val, total);
                 if (it.row != pending) {
                     if (pending >= 0) flush();
@@ -350,7 +358,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     constexpr int kPart = WALK == 3 ? kWave : WALK == 4 ? kSpmmMergeSlots : 0;
     A total[VEC];
     __shared__ __attribute__((aligned(16))) A parked[kPart > kWave ? kWgThreads * VEC : 1];
-    spmm_sum_slots<T, TN, kPart>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total, parked + (kPart > kWave ? threadIdx.x * VEC : 0));
+    spmm_sum_slots<T, TN, kPart, kInEights<T, TN, EDGE>>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total, parked + (kPart > kWave ? threadIdx.x * VEC : 0));
     if (shared_row) {
         __shared__ __attribute__((aligned(16))) A wg_sum[kWavesPerWg][TN];
         if (group == 0) {
@@ -759,7 +767,7 @@ spmm_hub_kernel(int n, HubGrid grid, const int* __restrict__ hub, const int* __r
     for (unsigned long long todo = share.pieces; todo; todo &= todo - 1ull) {
         const int i = __builtin_ctzll(todo);
         const HubPart p = hub_part(share, i);
-        spmm_sum_slots<T, TN>(p.base, 0, p.cnt, p.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
+        spmm_sum_slots<T, TN, 0, kInEights<T, TN, EDGE>>(p.base, 0, p.cnt, p.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
         if (!partial) {
             A* c_lane = C + (size_t)p.row * n + tile + ls * VEC;
 #pragma unroll
@@ -1122,7 +1130,8 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
             return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
         }
     }
-    const int best = spmm_tile_of_call(n, sizeof(T), plan.dense_rows, plan.nonzeros, plan.columns_local);
+    // (a group's four rows have no registers for sums of eight)
+    const int best = plan.groups ? spmm_tile_width(n, sizeof(T)) : spmm_tile_of_call(n, sizeof(T), plan.dense_rows, plan.nonzeros, plan.columns_local);
     if constexpr (sizeof(T) <= 4) {
         if (best == 128)
             return launch_edge<T, 128>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags,
