@@ -51,7 +51,7 @@ constexpr size_t kOutsideFirstBytes = 7000000;
 // over a power of two, 2^ref, the first one that no score so far passes: the exponent of a weight is then a single rounding away
 // from score * log2(e), and the steps and the waves rescale each other's sums exactly.  PARTS: the sums of a few steps are put away
 // into `total` (a wave with all columns of a run: one chain of 6 / 18 steps had 1.13 / 1.36 times the error of four chains put
-// together, in parts of a quarter of the steps or four of them 1.03 / 1.01; 16 heads of 2048 rows, halves of width 64).
+// together, parts of four steps up to 1.05, those of attention_wide_kernel 0.95 to 1.00; 16 heads of 2048 and 4096 rows, halves).
 template <typename T, int D, bool PARTS = false>
 struct TileSoftmax {
     static constexpr int N = 4 * tile_blocks<T>();
@@ -491,7 +491,7 @@ attention_wide_kernel(int nheads, int n_tiles, const RowTile* __restrict__ tiles
         const int steps = (hi - lo + kStep - 1) / kStep;
         int c_next = lo + (steps - lo / kStep % steps) % steps * kStep;
         fetch(c_next);
-        const int part_steps = min((steps + 3) / 4, 4);
+        const int part_steps = 1 + steps / 9; // (a step adds to its part twice, a part to the total once: shorter parts than their number)
         int buffer = 0, left = part_steps;
 #pragma unroll 1
         for (int it = 0; it < steps; ++it, buffer ^= 1) {
@@ -514,7 +514,7 @@ attention_wide_kernel(int nheads, int n_tiles, const RowTile* __restrict__ tiles
             if (now) columns_step<T, D, KEEP, true>(lds_k, lds_v, lds_w, c0, inside(c0), lane, me, f_a, f_end, f_base, q_row, scale, probs, sm);
             if (--left == 0) sm.put_away(), left = part_steps;
         }
-        sm.put_away();
+        sm.put_away(); // (not left for the end: with the nonzeros outside the runs in between its registers make the kernel a fifth slower)
     }
     __syncthreads();
     if (!mine) return;
@@ -526,11 +526,16 @@ attention_wide_kernel(int nheads, int n_tiles, const RowTile* __restrict__ tiles
     for (int quarter = 0; quarter < kTileRows / kOutsideRows; ++quarter)
         rows_outside<T, D, KEEP>(extents[wave], quarter, row0, again, lane, col, val, q, k, v, scale, probs, part + kOut, part + quarter * kOutsideRows * PAD,
                                  out_m[wave], out_l[wave]);
-    // the two partial results, the run's relative to its power of two, the other to the exponential of its maximum
+    // the two partial results, the run's relative to its power of two, the other to the exponential of its maximum: put together relative
+    // to the former where the row's largest score is the run's (its sums, of four waves' before, are not rounded once more for it)
     wave_lds_sync();
     const float m_out = out_m[wave][n], top = fmaxf(sm.m, m_out), top_safe = top == -INFINITY ? 0.f : top;
-    float f_out = __builtin_amdgcn_exp2f((m_out - top_safe) * kLog2e), f_run = __builtin_amdgcn_exp2f(-fmaf(top_safe, kLog2e, -sm.ref));
+    const bool by_run = m_out <= sm.m;
+    float f_out = __builtin_amdgcn_exp2f(by_run ? fmaf(m_out, kLog2e, -sm.ref) : (m_out - top_safe) * kLog2e);
+    const float to_top = __builtin_amdgcn_exp2f(fmaf(top_safe, kLog2e, -sm.ref)); // (2^ref over the exponential of the largest score: 1 over that)
+    float f_run = by_run ? 1.f : __builtin_amdgcn_exp2f(-fmaf(top_safe, kLog2e, -sm.ref));
     const float inv = 1.0f / fmaf(quad_sum(sm.total_l), f_run, out_l[wave][n] * f_out);
+    const float inv_top = by_run ? inv * to_top : inv; // relative to the exponential of the largest score
     f_run *= 1.f / TileWeights<T>::kScale;
 #pragma unroll
     for (int c = 0; c < NB; ++c) {
@@ -548,12 +553,12 @@ attention_wide_kernel(int nheads, int n_tiles, const RowTile* __restrict__ tiles
         const int at = i * kWave + lane;
         to[at] = *reinterpret_cast<const f32x4*>(part + at / (D / 4) * PAD + at % (D / 4) * 4);
     }
-    if (KEEP == kKeepScores && gq == 0) stats[row0 + n] = make_float2(top_safe, inv);
+    if (KEEP == kKeepScores && gq == 0) stats[row0 + n] = make_float2(top_safe, inv_top);
     if (KEEP == kKeepProbs) {
         __threadfence_block(); // (the wave's own scores, normalised in place)
         for (int r = 0; r < kTileRows; ++r) {
             const int4 row = extents[wave][r];
-            const float top_r = __shfl(top_safe, r, kWave), inv_r = __shfl(inv, r, kWave);
+            const float top_r = __shfl(top_safe, r, kWave), inv_r = __shfl(inv_top, r, kWave);
             for (int slot = row.x + lane; slot < row.x + row.y; slot += kWave) probs[slot] = __expf(probs[slot] - top_r) * inv_r;
         }
     }

@@ -422,6 +422,25 @@ def test_four_tiles_a_workgroup_against_fp64(m, window, shift, extra, d, scale, 
         assert (scores[h].double() - s).abs().max() <= 2e-5 * s.abs().max()
 
 
+@pytest.mark.parametrize("d", [32, 64, 128])
+@pytest.mark.parametrize("window,extra", [(96, 0), (160, 20), (330, 0), (520, 30)])
+def test_four_tiles_a_workgroup_are_as_exact_as_one(window, extra, d):
+    """2-norms of the errors against fp64 of at least 520 000 elements, each known to 0.1 %: 0.95 to 1.00 times those of a tile a workgroup. (Parts
+    of four steps, put together with the nonzeros outside by a rescaling of both, had up to 1.05 times.)"""
+    m, heads = 2048, 512 // d
+    errors = []
+    for fours in (0, 1 << 20):
+        csr, dense = _mask(m, window, 1, extra, seed=window)
+        assert csr.plan.counts[3] == m // 16
+        csr.call_plans().tile_fours = fours
+        gen = torch.Generator(device="cuda").manual_seed(d)
+        q, k, v = (torch.randn(max(heads, _heads(csr)), r, d, device="cuda", generator=gen).half() for r in (m, csr.n, csr.n))
+        out = sparse_attention(csr, q, k, v)
+        want = torch.stack([_reference(dense, q[h], k[h], v[h], d ** -0.5) for h in range(heads)])
+        errors.append((out[:heads].double() - want).norm().item())
+    assert errors[0] != errors[1] and errors[1] <= 1.01 * errors[0]
+
+
 def test_four_tiles_a_workgroup_without_range():
     """Infinite scores and rows of v that are not finite, in a run, at its ends and outside it: as with a tile a workgroup."""
     m, d, inf = 192, 64, float("inf")
