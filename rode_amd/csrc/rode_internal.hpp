@@ -39,6 +39,7 @@ struct PlanRef {
     const int* dev = nullptr;         // descriptors
     const void* rows = nullptr;       // planned rows of the chunks with a window
     const int* host_counts = nullptr;
+    bool rings = false;               // the ring kernels take the chunks with a window (choose_windows)
     // A hub plan (rode_hub.hip) and the host copy of its eight header ints (required with it).
     const int* hub = nullptr;
     const int* hub_counts = nullptr;
@@ -89,17 +90,18 @@ inline float window_gain(const PlanRef& plan, int m2, size_t row_bytes, const Wi
     const size_t mb = 2 * (size_t)m2 * row_bytes >> 20;
     return (of.base + of.per_slot * slots) * (mb >= of.largest_mb ? of.largest : mb >= of.larger_mb ? of.larger : 1.f);
 }
-inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes, const WindowGain& full_round)
+// (the time of the standard kernels over that of the window kernels)
+inline float windows_pay(const PlanRef& plan, int m2, int round, size_t row_bytes, const WindowGain& full_round)
 {
-    if (plan.dev == nullptr || plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) return true;
     const int chunks = plan.host_counts[0], rounds = (chunks + round - 1) / round;
-    return window_gain(plan, m2, row_bytes, full_round) * (float)chunks >= (float)rounds * (float)round;
+    return window_gain(plan, m2, row_bytes, full_round) * (float)chunks / ((float)rounds * (float)round);
 }
 
 // Do the ring kernels pay for a call?  A strip costs as much as its chunks and a start (the first window, not copied beside any work)
 // worth a chunk and half a chunk per slice; few strips with a chunk more than the others do not count.  gain: time of the standard kernels
-// over that of a chunk of s slots a row, measured as for the window kernels on bands of 128 to 256 columns and 66 K to 1 M rows, SpMM: us, standard
-// -> ring, 9 / 14 / 19 / 27 slots a row (the operands within the last-level cache; beyond it the ring gains up to twice that)
+// over that of a chunk of s slots a row, measured as for the window kernels on bands of 128 to 256 columns and 66 K to 1 M rows (and set so that
+// of 2100 such calls, three matrices in turn, two lose more than 2 % against what is taken of standard and window kernels, 3 and 4), SpMM: us,
+// standard -> ring, 9 / 14 / 19 / 27 slots a row (the operands within the last-level cache; beyond it the ring gains up to twice that)
 //   f32 x 64    131 K 20.2 -> 18.8, 24.3 -> 20.8, 29.6 -> 23.0, 38.2 -> 27.2; 350 K 48 -> 42, 60 -> 48, 75 -> 55, 95 -> 66; 90 K 14.8 -> 18.5, 17.5 -> 20.6, 21.5 -> 22.6, 27.3 -> 26.1
 //   f32 x 128   131 K 37 -> 32, 45 -> 37, 57 -> 41, 73 -> 50; 66 K 20.4 -> 20.5, 24.7 -> 23.1, 29.4 -> 25.4, 38.4 -> 30.4; 90 K 26.7 -> 31.4, 32.4 -> 34.8, 39.0 -> 37.7, 51 -> 44
 //   f32 x 32    600 K 44 -> 53, 51 -> 58, 66 -> 64, 87 -> 75; 200 K 17.3 -> 22.6, 20.0 -> 24.5, 24.2 -> 26.2, 31.7 -> 30.5
@@ -109,13 +111,35 @@ inline bool window_pays(const PlanRef& plan, int m2, int round, size_t row_bytes
 //   f32 x 64    131 K 24.8 -> 21.7, 29.9 -> 23.8, 35.9 -> 27.2, 46.3 -> 31.6; 350 K 60 -> 48, 74 -> 53, 93 -> 65, 119 -> 79; 600 K 100 -> 100, 124 -> 107, 179 -> 120
 //   f32 x 32    350 K 33 -> 40, 41 -> 43, 54 -> 47, 72 -> 55; 600 K 54 -> 65, 68 -> 80, 87 -> 92, 133 -> 107; 1 M 86 -> 126, 125 -> 137, 175 -> 145, 236 -> 171
 //   f16 x 128   131 K 25.0 -> 24.4, 30.4 -> 27.6, 37.3 -> 31.4, 46.9 -> 37.8; 600 K 102 -> 111, 125 -> 122, 179 -> 136;  f16 x 64  350 K 34 -> 43, 42 -> 46, 54 -> 52, 72 -> 62
-inline bool ring_pays(const PlanRef& plan, int m2, int workgroups, int slices, size_t row_bytes, const WindowGain& chunk)
+inline float rings_pay(const PlanRef& plan, int m2, int workgroups, int slices, size_t row_bytes, const WindowGain& chunk)
 {
-    if (plan.dev == nullptr) return true;
-    // the number of nonzeros not said: the caller wants the plan used, which rows of 128 bytes never were
-    if (plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) return row_bytes > 128;
     const int parts = plan.host_counts[0] * slices, rounds = (parts - 16 * slices + workgroups - 1) / workgroups;
-    return window_gain(plan, m2, row_bytes, chunk) * (float)parts >= ((float)rounds + 1.f + 0.5f * (float)slices) * (float)workgroups;
+    return window_gain(plan, m2, row_bytes, chunk) * (float)parts / (((float)rounds + 1.f + 0.5f * (float)slices) * (float)workgroups);
+}
+
+// Which kernels take the chunks with a window, for dense rows that a ring takes in `slices` (0: not) and the window kernels take or not.
+inline void choose_windows(PlanRef& plan, int m2, int workgroups, int slices, bool window_takes, size_t row_bytes, const WindowGain& of_rings, const WindowGain& of_windows)
+{
+    if (plan.dev == nullptr) return;
+    if (plan.host_counts == nullptr || plan.nonzeros <= 0 || m2 <= 0) {
+        // the number of nonzeros not said: the caller wants the plan used, which rows of 128 bytes never were
+        plan.rings = slices > 0;
+        if (slices > 0 ? row_bytes == 128 : !window_takes) plan.no_window();
+        return;
+    }
+    const float rings = slices > 0 ? rings_pay(plan, m2, workgroups, slices, row_bytes, of_rings) : 0.f;
+    const float windows = window_takes ? windows_pay(plan, m2, workgroups, row_bytes, of_windows) : 0.f;
+    // Chunks without a window stay with the standard kernels, which work on the others as well while the dense rows of those are on their way: what
+    // is taken from them saves less than its share.  Rings in the place of window kernels are faster all the same (1 M rows x 64, 27 slots, one
+    // chunk in ten / two in five without a window, runs of 110 / 73 chunks: standard 421 / 555, windows 359 / 578, rings 321 / 552), but else they are
+    // for matrices with nearly no such chunk: up to a twentieth, of rows of 128 bytes, which the window kernels do not take, as many hundredths
+    // as they have slots above 21 (x 32, 27 slots, a twentieth, runs of 110 / 14 chunks: 203 -> 177, 195 -> 190; a tenth 218 -> 205, 195 -> 219).
+    const long long chunks = plan.host_counts[0], without = chunks - plan.host_counts[1];
+    const bool together = without == 0 || (window_takes ? 20 * without <= chunks || windows >= 1.f : 100 * without * m2 <= (plan.nonzeros - 21ll * m2) * chunks);
+    // (of both, up to four rounds the better one; beyond it the dense operands come from memory, and the rings copy less: 131 K rows of 16
+    // x 128 39 windows, 41 rings; 350 K of 12 halves x 128 90 and 75)
+    plan.rings = rings >= 1.f && together && (chunks > 4 * workgroups || rings >= windows);
+    if (!plan.rings && windows < 1.f) plan.no_window();
 }
 
 hipError_t group_plan_launch(int M, const int* row_ptr, const int* col, int* plan, hipStream_t stream);
@@ -216,7 +240,7 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
 // the window kernel of SpMM over the planned chunks of the residue list
 template <typename T>
 hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
-                              typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream);
+                              typename SpmmAcc<T>::type* C, const PlanRef& plan, hipStream_t stream);
 
 // (stored: rows of at most that many aligned slots are left alone as well)
 hipError_t spmm_clear_rows_launch(int M, size_t row_bytes, int stored, const int* row_ptr, void* C, hipStream_t stream);
@@ -229,7 +253,7 @@ hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int*
 // the window kernel of SDDMM over the planned chunks of the residue list
 template <typename T>
 hipError_t sddmm_window_launch(int m2, int k, const int* col, const float* val, const T* lhs, const T* rhs, float* out,
-                               const int* plan, const void* plan_rows, hipStream_t stream);
+                               const PlanRef& plan, hipStream_t stream);
 
 hipError_t permute_launch(int n, const float* src, const int* index, float* dst, hipStream_t stream);
 size_t csr_transpose_workspace_bytes(int nnz);

@@ -397,7 +397,9 @@ struct PlannedRowMeta {
     unsigned missmask;
 };
 struct PlannedChunk {
-    int w0, wn, reserved[2]; // the chunk's window again: the kernels need nothing else to start
+    int w0, wn; // the chunk's window again: the kernels need nothing else to start
+    int next;   // of a chunk without a window: no sooner than so many chunks on is one (0: not said)
+    int reserved;
     PlannedRowMeta meta[kPlanResidueChunk];
     unsigned short entry[kPlanResidueChunk][kBlockItems];
 };

@@ -88,9 +88,16 @@ plan_rows_kernel(int m2, const int* __restrict__ residue_rows, const int* __rest
     if (threadIdx.x == 0) {
         out.w0 = d.w0;
         out.wn = d.wn;
-        out.reserved[0] = out.reserved[1] = 0;
+        out.next = out.reserved = 0;
     }
-    if (d.wn <= 0) return;
+    if (d.wn <= 0) {
+        const int ahead = chunk + 1 + (int)threadIdx.x;
+        if (threadIdx.x < kWave) {
+            const unsigned long long windows = __ballot(ahead < (int)gridDim.x && plan_residue_desc(plan, min(ahead, (int)gridDim.x - 1)).wn > 0);
+            if (threadIdx.x == 0) out.next = windows ? __builtin_ctzll(windows) + 1 : kWave + 1;
+        }
+        return;
+    }
     const int local = threadIdx.x / L, ls = threadIdx.x % L;
     const int entry = chunk * kPlanResidueChunk + local;
     int row = -1, first = 0, cnt = 0, aligned = 0;

@@ -527,7 +527,7 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
         }
     }
     if (e == hipSuccess && m2 > 0 && window_residue)
-        e = sddmm_window_launch<T>(m2, k, col, val, lhs, rhs, out, plan.dev, plan.rows, s2);
+        e = sddmm_window_launch<T>(m2, k, col, val, lhs, rhs, out, plan, s2);
     return e;
 }
 
@@ -547,7 +547,7 @@ hipError_t launch_edge(bool edge, int m1, int m2, int k, const int* block_rows, 
 // k: any positive multiple of the 128-bit vector width (4 for fp32, 8 for fp16) up to 512.
 // 32, 64 and 128 (the reference has 32 and 128) run without any bounds test.  Chunks of the
 // residue list for which `plan` holds a window go to the ring kernel (rows of 128 and 256 bytes) or
-// the window kernel (other rows of more than 128: window_takes) where that pays (ring_pays, window_pays).
+// the window kernel (rows of more than 128: window_takes) where that pays (choose_windows).
 template <typename T>
 hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int* residue_rows, const int* st_off,
                         const int* row_ptr, const int* col, const float* val, const T* lhs, const T* rhs,
@@ -557,13 +557,11 @@ hipError_t sddmm_launch(int m1, int m2, int k, const int* block_rows, const int*
     constexpr WindowGain kWide = {1.24f, 0.026f, 1.f, 0, 1.f, 0}, kNarrow = {0.95f, 0.0245f, 0.82f, 210, 0.92f, 370},
                          kHalves = {0.92f, 0.0155f, 0.86f, 210, 0.92f, 345};
     const size_t row_bytes = (size_t)k * sizeof(T);
-    const bool ring = ring_slices(row_bytes) == 1, line = row_bytes == 128;
-    const WindowGain of_ring = sizeof(T) == 2 ? WindowGain{line ? 0.72f : 1.11f, line ? 0.026f : 0.019f, line ? 0.82f : 0.86f, line ? 130u : 210u, 0.92f, line ? 220u : 345u}
+    const bool line = row_bytes == 128;
+    const WindowGain of_ring = sizeof(T) == 2 ? WindowGain{line ? 0.57f : 1.06f, line ? 0.030f : 0.023f, line ? 0.79f : 0.86f, line ? 130u : 210u, 0.92f, line ? 220u : 345u}
                                               : WindowGain{line ? 0.62f : 1.17f, line ? 0.032f : 0.024f, 0.82f, line ? 130u : 210u, 0.92f, line ? 220u : 370u};
-    if (ring ? !ring_pays(plan, m2, kWindowWgs, 1, row_bytes, of_ring)
-             : !window_takes(row_bytes) ||
-                   !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
-        plan.no_window();
+    choose_windows(plan, m2, kWindowWgs, ring_slices(row_bytes) == 1 ? 1 : 0, window_takes(row_bytes), row_bytes, of_ring,
+                   sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow);
 #define RODE_SDDMM_CASE(KT, NS)                                                                                   \
     return launch_edge<T, KT, NS>(k != (KT) * (NS), m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, \
                                   lhs, rhs, out, plan, s1, s2)

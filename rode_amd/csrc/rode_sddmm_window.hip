@@ -176,7 +176,7 @@ sddmm_residue_window_kernel(int m2, int k, const int* __restrict__ col, const fl
 
 template <typename T, int TILES>
 __global__ void __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-sddmm_ring_kernel(int m2, int k, const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ lhs,
+sddmm_ring_kernel(int m2, int k, bool all_windows, const int* __restrict__ plan, const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ lhs,
                   const T* __restrict__ rhs, float* __restrict__ out, const PlannedChunk* __restrict__ rows)
 {
     using R = Ring<TILES>;
@@ -186,7 +186,8 @@ sddmm_ring_kernel(int m2, int k, const int* __restrict__ col, const float* __res
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int group = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
-    const RingWalk walk(m2, 1);
+    __shared__ int walk_room[kResThreads / kWave + 2];
+    const RingWalk walk(m2, 1, all_windows, plan, walk_room);
     int chunk = walk.from(rows, walk.at);
     if (chunk >= walk.end) return;
     const char* ring_bytes = reinterpret_cast<const char*>(ring);
@@ -323,24 +324,27 @@ sddmm_ring_kernel(int m2, int k, const int* __restrict__ col, const float* __res
 // T = float or __half.
 template <typename T>
 hipError_t sddmm_window_launch(int m2, int k, const int* col, const float* val, const T* lhs, const T* rhs, float* out,
-                               const int* plan, const void* plan_rows, hipStream_t stream)
+                               const PlanRef& plan, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
     const size_t row_bytes = (size_t)k * sizeof(T);
-    if (ring_slices(row_bytes) == 1) {
+    const PlannedChunk* rows = static_cast<const PlannedChunk*>(plan.rows);
+    if (plan.rings) {
+        if (ring_slices(row_bytes) != 1) return hipErrorInvalidValue;
+        const bool all = plan.host_counts != nullptr && plan.host_counts[1] == plan.host_counts[0];
         auto kernel = row_bytes == 128 ? sddmm_ring_kernel<T, 1> : sddmm_ring_kernel<T, 2>;
-        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, static_cast<const PlannedChunk*>(plan_rows));
+        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, k, all, plan.dev, col, val, lhs, rhs, out, rows);
         return hipGetLastError();
     }
     if (!window_takes(row_bytes)) return hipErrorInvalidValue;
     auto kernel = ((size_t)k * sizeof(T)) % (kResLanes * 16) != 0 ? sddmm_residue_window_kernel<T, true> : sddmm_residue_window_kernel<T, false>;
-    kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, static_cast<const PlannedChunk*>(plan_rows));
+    kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, k, col, val, lhs, rhs, out, rows);
     return hipGetLastError();
 }
 
 template hipError_t sddmm_window_launch<float>(int, int, const int*, const float*, const float*, const float*, float*,
-                                               const int*, const void*, hipStream_t);
+                                               const PlanRef&, hipStream_t);
 template hipError_t sddmm_window_launch<__half>(int, int, const int*, const float*, const __half*, const __half*, float*,
-                                                const int*, const void*, hipStream_t);
+                                                const PlanRef&, hipStream_t);
 
 } // namespace rode

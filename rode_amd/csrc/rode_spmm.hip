@@ -1023,7 +1023,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         e = hipGetLastError();
     }
     if (e == hipSuccess && residue && window_residue)
-        e = spmm_window_launch<T>(m2, n, owned_slots, col, val, B, C, plan.dev, plan.rows, s2);
+        e = spmm_window_launch<T>(m2, n, owned_slots, col, val, B, C, plan, s2);
     return e;
 }
 
@@ -1097,8 +1097,8 @@ size_t spmm_hub_partial_rows(const int* counts, int n, int acc_bytes)
 
 // n: any positive multiple of the 128-bit vector width (4 fp32, 8 fp16, 2 fp64).  Multiples of 32 (all
 // the reference supports) run without any bounds test.  Chunks of the residue list for
-// which `plan` holds a window go to the ring or window kernel that takes the
-// width (ring_slices, else window_takes) where that pays (ring_pays, window_pays).
+// which `plan` holds a window go to the ring or window kernel, of those that take the
+// width (ring_slices, window_takes), where that pays (choose_windows).
 template <typename T>
 hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                        const int* row_ptr, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
@@ -1112,13 +1112,11 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
     const int slices = ring_slices(row_bytes);
     // (a band of 128 columns is worth 5 % less than those of 192 and 256 that the figures beside ring_pays are of)
     const bool line = row_bytes == 128, whole = slices == 1;
-    const WindowGain ring = sizeof(T) == 8 ? WindowGain{line ? 1.2f : whole ? 1.05f : 1.1f, line ? 0.03f : 0.02f, 1.f, 0, 1.f, 0}
-                            : sizeof(T) == 2 ? WindowGain{line ? 0.73f : whole ? 0.93f : 0.97f, line ? 0.0145f : 0.02f, 1.f, 0, 1.f, 0}
-                                             : WindowGain{line ? 0.69f : whole ? 1.05f : 1.1f, line ? 0.0235f : 0.02f, 1.f, 0, 1.f, 0};
-    if (slices > 0 ? !ring_pays(plan, m2, kWindowWgs, slices, row_bytes, ring)
-                   : !window_takes(row_bytes) ||
-                         !window_pays(plan, m2, kWindowWgs, row_bytes, sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow))
-        plan.no_window();
+    const WindowGain ring = sizeof(T) == 8 ? WindowGain{line ? 1.2f : whole ? 0.94f : 1.1f, line ? 0.03f : whole ? 0.025f : 0.02f, 1.f, 0, 1.f, 0}
+                            : sizeof(T) == 2 ? WindowGain{line ? 0.72f : whole ? 0.93f : 0.97f, line ? 0.0145f : 0.02f, 1.f, 0, 1.f, 0}
+                                             : WindowGain{line ? 0.67f : whole ? 0.94f : 1.1f, line ? 0.0235f : whole ? 0.025f : 0.02f, 1.f, 0, 1.f, 0};
+    choose_windows(plan, m2, kWindowWgs, slices, window_takes(row_bytes), row_bytes, ring,
+                   sizeof(T) == 8 ? kDoubles : sizeof(T) == 2 ? kHalves : row_bytes > 256 ? kWide : kNarrow);
     if constexpr (!std::is_same<T, double>::value) { // (a line of doubles is no tile width)
         constexpr int kLine = 128 / (int)sizeof(T);
         const int lines = n / kLine;

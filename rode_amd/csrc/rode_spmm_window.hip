@@ -188,7 +188,7 @@ spmm_residue_window_kernel(int m2, int n, int owned_slots, const int* __restrict
 
 template <typename T, int TILES>
 __global__ void __launch_bounds__(kResThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
-spmm_ring_kernel(int m2, int n, int slices, int owned_slots, const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
+spmm_ring_kernel(int m2, int n, int slices, int owned_slots, bool all_windows, const int* __restrict__ plan, const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
                  const T* __restrict__ B, typename DenseVec<T>::Acc* __restrict__ C, const PlannedChunk* __restrict__ rows)
 {
     using A = typename DenseVec<T>::Acc;
@@ -199,7 +199,8 @@ spmm_ring_kernel(int m2, int n, int slices, int owned_slots, const int* __restri
 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x % kWave;
     const int group = threadIdx.x / kResLanes, ls = threadIdx.x % kResLanes;
-    const RingWalk walk(m2, slices);
+    __shared__ int walk_room[kResThreads / kWave + 2];
+    const RingWalk walk(m2, slices, all_windows, plan, walk_room);
     int chunk = walk.from(rows, walk.at);
     if (chunk >= walk.end) return;
     const char* ring_bytes = reinterpret_cast<const char*>(ring);
@@ -348,23 +349,26 @@ spmm_ring_kernel(int m2, int n, int slices, int owned_slots, const int* __restri
 // The window kernel over the planned chunks of the residue list, for dense rows that window_takes.
 template <typename T>
 hipError_t spmm_window_launch(int m2, int n, int owned_slots, const int* col, const typename SpmmAcc<T>::type* val, const T* B,
-                              typename SpmmAcc<T>::type* C, const int* plan, const void* plan_rows, hipStream_t stream)
+                              typename SpmmAcc<T>::type* C, const PlanRef& plan, hipStream_t stream)
 {
     if (m2 <= 0) return hipSuccess;
     const size_t row_bytes = (size_t)n * sizeof(T);
-    if (ring_slices(row_bytes) > 0) {
+    const PlannedChunk* rows = static_cast<const PlannedChunk*>(plan.rows);
+    if (plan.rings) {
+        if (ring_slices(row_bytes) == 0) return hipErrorInvalidValue;
+        const bool all = plan.host_counts != nullptr && plan.host_counts[1] == plan.host_counts[0];
         auto kernel = row_bytes == 128 ? spmm_ring_kernel<T, 1> : spmm_ring_kernel<T, 2>;
-        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, n, ring_slices(row_bytes), owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
+        kernel<<<kWindowWgs, kResThreads, 0, stream>>>(m2, n, ring_slices(row_bytes), owned_slots, all, plan.dev, col, val, B, C, rows);
         return hipGetLastError();
     }
     if (!window_takes(row_bytes)) return hipErrorInvalidValue;
     auto kernel = ((size_t)n * sizeof(T)) % (kResLanes * 16) != 0 ? spmm_residue_window_kernel<T, true> : spmm_residue_window_kernel<T, false>;
-    kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, static_cast<const PlannedChunk*>(plan_rows));
+    kernel<<<window_grid(m2), kResThreads, 0, stream>>>(m2, n, owned_slots, col, val, B, C, rows);
     return hipGetLastError();
 }
 
-template hipError_t spmm_window_launch<float>(int, int, int, const int*, const float*, const float*, float*, const int*, const void*, hipStream_t);
-template hipError_t spmm_window_launch<double>(int, int, int, const int*, const double*, const double*, double*, const int*, const void*, hipStream_t);
-template hipError_t spmm_window_launch<__half>(int, int, int, const int*, const float*, const __half*, float*, const int*, const void*, hipStream_t);
+template hipError_t spmm_window_launch<float>(int, int, int, const int*, const float*, const float*, float*, const PlanRef&, hipStream_t);
+template hipError_t spmm_window_launch<double>(int, int, int, const int*, const double*, const double*, double*, const PlanRef&, hipStream_t);
+template hipError_t spmm_window_launch<__half>(int, int, int, const int*, const float*, const __half*, float*, const PlanRef&, hipStream_t);
 
 } // namespace rode

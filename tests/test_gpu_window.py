@@ -319,3 +319,58 @@ def test_rows_with_no_column_in_their_window_are_not_reached_by_it(dtype, k):
     touched[row.repeat_interleave(lens)[torch.isin(col, bad)]] = True
     assert (~touched & (lens < 21)).sum() > 100
     assert finite[~touched].all() and not finite[touched].any()
+
+
+def _some_banded(m, degree, banded, seed):
+    """`degree` ascending columns a row: of the 192 around the diagonal where `banded` (of every chunk of 128 rows) says so, else anywhere."""
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    row = torch.arange(m, device=DEV)
+    near = (row - 96).clamp(0, m - 192)[:, None] + torch.rand(m, 192, device=DEV, generator=gen).argsort(1)[:, :degree]
+    far = (torch.rand(m, degree, device=DEV, generator=gen) * (m // degree)).long() + torch.arange(degree, device=DEV) * (m // degree)
+    col = torch.where(banded.to(DEV)[row // 128, None], near, far).sort(1)[0]
+    ro = torch.arange(0, m * degree + 1, degree, dtype=torch.int32)
+    return ro, col, torch.rand(m * degree, device=DEV, generator=gen) + 0.5
+
+
+@pytest.mark.parametrize("dtype,k", [(torch.float32, 64), (torch.float32, 128), (torch.float16, 128), (torch.float64, 64)])
+@pytest.mark.parametrize("kind", ["one run", "short runs", "few", "all but few"])
+def test_rings_where_chunks_with_a_window_lie_together(kind, dtype, k):
+    """1400 chunks, 175 of an XCD's share, dealt out to 32, 16 or 8 strips by their windows: all in three shares, in runs of 5 and 90 with 90 and 5 between,
+    seven in all, all but seven."""
+    chunks, degree = 1400, 9
+    c = torch.arange(chunks)
+    banded = {"one run": (c > 300) & (c < 777), "short runs": (c % 95 < 5) ^ (c > 700), "few": c % 200 == 150, "all but few": c % 200 != 150}[kind]
+    m = 128 * chunks - 3
+    ro, col, val = _some_banded(m, degree, banded, seed=k)
+    csr = RoDeCSR(ro, col.flatten().int(), val, DEV, m, m, k, locality=True)
+    assert csr.plan.windowed == int(banded.sum()) and csr.plan.nonzeros == 0
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    B, L = (torch.randn(m, k, device=DEV, generator=gen, dtype=torch.float64).to(dtype) for _ in range(2))
+    want = torch.zeros(m, k, device=DEV, dtype=torch.float64)
+    for j in range(degree):
+        want += val.view(m, degree)[:, j:j + 1].double() * B[col[:, j]].double()
+    if dtype == torch.float64:
+        got = rode_sddmm_hip.spmm_forward(csr.block_indices, csr.residue_indices, csr.st_offsets, csr.m1, csr.m2, csr.row_offsets, csr.column_indices,
+                                          val.double(), m, m, B, plan=csr.plan)
+        assert (got - want).abs().max() <= 1e-14 * want.abs().max()
+        return
+    assert (rode_spmm(csr, B) - want).abs().max() <= 2e-6 * want.abs().max()
+    want = torch.stack([val.view(m, degree)[:, j].double() * (L.double() * B[col[:, j]].double()).sum(1) for j in range(degree)], 1).flatten()
+    assert (rode_sddmm(csr, L, B) - want).abs().max() <= 2e-6 * want.abs().max()
+
+
+def test_chunks_without_a_window_and_what_pays():
+    """Six chunks in ten with a window, rows of 128 bytes: the standard kernels take all (they took 243 us for a million such rows, and 328 with the
+    others by themselves). 704 chunks with one, SDDMM of 256-byte rows: too few for rings, but not for windows (21.4 us, standard kernels 30)."""
+    m = 128 * 7813
+    ro, col, val = _some_banded(m, 27, torch.arange(7813) % 10 < 6, seed=1)
+    csr, plain = (RoDeCSR(ro, col.flatten().int(), val, DEV, m, m, 32, locality=how) for how in ("auto", False))
+    assert csr.plan is not None and csr.plan.windowed * 10 <= 7 * csr.plan.counts[0]
+    B, L = (torch.randn(m, 32, device=DEV) for _ in range(2))
+    assert torch.equal(rode_spmm(csr, B), rode_spmm(plain, B)) and torch.equal(rode_sddmm(csr, L, B), rode_sddmm(plain, L, B))
+    m = 128 * 704
+    ro, col, val = _some_banded(m, 20, torch.ones(704, dtype=torch.bool), seed=2)
+    csr, plain = (RoDeCSR(ro, col.flatten().int(), val, DEV, m, m, 64, locality=how) for how in ("auto", False))
+    B, L = (torch.randn(m, 64, device=DEV) for _ in range(2))
+    got, other = rode_sddmm(csr, L, B), rode_sddmm(plain, L, B)
+    assert not torch.equal(got, other) and (got - other).abs().max() <= 2e-6 * other.abs().max()
