@@ -1057,27 +1057,37 @@ static int spmm_tile_width(int n, size_t elem)
     return best;
 }
 
-// ... but for some calls whose least padding is with tiles of 32 columns (widths like 96, 160, 224).
-// Halves: such a tile is half a line of 128 bytes, which is fetched for each of the two.  Tiles of 128, and of 64 where the dense operand is
-// near the size of an L2 and its rows are used less than 20 times (us, 32 -> 64 / 128 columns, width 96; uniform (u) and lognormal degrees): u 4000 rows of
-// 40 10.7 -> 8.9 / 7.1, u 8029 of 56 16.1 -> 13.0 / 10.7, u 16 K of 110 34.6 -> 29.4 / 24.1, 60 K of 24 59.0 -> 52.9 / 45.7, 100 K of 20 94 -> 83 / 74,
-// 300 K of 10 189 -> 158 / 132; u 16 K of 20 9.1 -> 8.4 / 9.0, 20 K of 12 12.6 -> 12.0 / 14.0, 26 K of 16 21.4 -> 18.6 / 20.4, 33 K of 10 21.8 -> 21.4 /
-// 23.7, 60 K of 10 29.6 -> 26.7 / 27.1 (16.5 K of 10 9.9 -> 10.5 / 10.9 is the one that loses); width 224 80 K of 20 183 -> 153 / 138.
+// ... but for some calls whose least padding is with tiles of 32 columns (widths like 96, 160, 224).  us of 32 / 64 / 128 columns, uniform (u)
+// and lognormal degrees, two matrices in turn:
+// Halves: a tile of 32 is half a line of 128 bytes, which is fetched for each of the two.  Tiles of 128 (u 16 K of 110 x 96 34.6 / 29.4 / 24.1, 60 K of 20
+// 51 / 44 / 37, 400 K of 14 336 / 279 / 218), but of 64
+//   * where those of 128 have a quarter of their lanes and more idle (x 160: u 33 K of 110 120 / 119 / 144, 8000 of 14 8.3 MB 0.91 / 1.15);
+//   * where the dense operand is near the size of an L2 and its rows are used less than 12 times (u 33 K of 8 x 96 13.3 / 13.4 / 14.7), up to 3.5 MB
+//     less than 24 (16.5 K of 20 x 96 9.9 / 9.4 / 10.6); less than 10 times and 12 to 16 MB, those of 32 (u 33 K of 8 x 224 22.8 / 25.6 / 24.9);
+//   * where one wave has all of a row, and the wider its tiles the longer for it, up to 1024 slots at 1 to 2.5 ns: 128 columns from 200 KB to
+//     gather for each of its slots on, 64 from 90 KB (x 96: 12 K of 14, 899 slots, 36 KB each 11.4 / 14.5 / 16.3; 20 K of 20, 72 KB 18.9 / 17.4 / 20.2;
+//     26 K of 32, 155 KB 32 / 27 / 30; 60 K of 14, 156 KB 38 / 34 / 33; 60 K of 32, 360 KB 74 / 70 / 60).
 // 32-bit operands: one line at a time keeps more of the operand in the L2s, as long as its tiles fit at all (sharding_pays); below 2.5 MB and above
-// 26 MB a tile whole rows are better, if a quarter of the lanes at most has nothing (width 96: u 4000 of 40 9.9 -> 8.2, 230 K of 12 167 -> 161,
-// 300 K of 10 187 -> 178, between them u 8029 of 56 15.3 -> 14.3, u 10 K of 20 8.2 -> 9.0, u 16 K of 110 37 -> 43, 40 K of 20 34.7 -> 43.9; 224: u 2000
-// of 40 11.0 -> 7.9, 300 K 430 -> 393).
+// 26 MB a tile whole rows are better, if a quarter of the lanes at most has nothing and with 500 KB to gather for each slot of the longest row
+// (u 4000 of 40 x 96 9.9 -> 8.2, 230 K of 12 167 -> 161, 300 K of 10 187 -> 178, between them u 10 K of 20 8.2 -> 9.0, u 16 K of 110 37 -> 43; 4000 of 32,
+// 1024 slots, 48 KB 8.4 -> 15.2).
 // Where neighbouring rows' columns lie close together the halves of a line meet in the caches anyway (halves, a band of 128, width 96: 70 K of 12
 // 11.9 -> 12.5, but 200 K of 20 55.9 -> 46.7).
-static int spmm_tile_of_call(int n, size_t elem, size_t dense_rows, size_t nonzeros, bool columns_local)
+static int spmm_tile_of_call(int n, size_t elem, const PlanRef& plan)
 {
     const int least = spmm_tile_width(n, elem);
-    if (least != 32 || n <= 32 || elem > 4 || n % 32 != 0) return least;
-    const size_t bytes = dense_rows * n * elem;
-    if (columns_local && bytes < 26000000) return 32;
-    if (elem == 2) return nonzeros > 0 && nonzeros < 20 * dense_rows && bytes >= 3000000 && bytes <= 12000000 ? 64 : 128;
-    const bool whole = dense_rows > 0 && 3 * ((n + 127) / 128 * 128) <= 4 * n && (bytes <= 2500000 || dense_rows * 128 > ((size_t)26 << 20));
-    return whole ? 128 : 32;
+    // (a group's four rows have no registers for sums of eight)
+    if (least != 32 || n <= 32 || elem > 4 || n % 32 != 0 || plan.groups) return least;
+    constexpr size_t KB = 1000, MB = 1000000;
+    const size_t rows = plan.dense_rows, nonzeros = plan.nonzeros, bytes = rows * n * elem, gathered = nonzeros * n * elem;
+    const size_t slots = plan.longest > 0 && plan.longest < kOwnedRowSlots ? plan.longest : kOwnedRowSlots;
+    auto enough = [&](size_t each) { return nonzeros == 0 || gathered >= slots * each; }; // (not said: taken to be)
+    if (plan.columns_local && bytes < 26 * MB) return 32;
+    const bool filled = 3 * ((n + 127) / 128 * 128) <= 4 * n;
+    if (elem == 4) return filled && rows > 0 && (bytes <= 5 * MB / 2 || rows * 128 > 27 * MB) && enough(500 * KB) ? 128 : 32;
+    if (nonzeros > 0 && nonzeros < 10 * rows && bytes > 12 * MB && bytes < 16 * MB) return 32;
+    const bool near_l2 = nonzeros > 0 && nonzeros < (bytes < 7 * MB / 2 ? 24 : 12) * rows && bytes >= 3 * MB && bytes <= 12 * MB;
+    return filled && !near_l2 && enough(200 * KB) ? 128 : enough(90 * KB) ? 64 : 32;
 }
 
 // The partial rows that the hub kernels of an SpMM of this width want, for operands of 4 (or, if more, 2) or of 8 bytes an element.
@@ -1128,8 +1138,7 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
             return launch<T, kLine, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
         }
     }
-    // (a group's four rows have no registers for sums of eight)
-    const int best = plan.groups ? spmm_tile_width(n, sizeof(T)) : spmm_tile_of_call(n, sizeof(T), plan.dense_rows, plan.nonzeros, plan.columns_local);
+    const int best = spmm_tile_of_call(n, sizeof(T), plan);
     if constexpr (sizeof(T) <= 4) {
         if (best == 128)
             return launch_edge<T, 128>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags,

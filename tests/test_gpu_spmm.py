@@ -896,3 +896,20 @@ def test_wider_tiles_are_as_exact_as_those_of_32_columns(half, width, rows, degr
         want.index_add_(0, row[part], csr.values[part, None].double() * B[col[part]].double())
     narrow = torch.cat([rode_spmm(csr, B[:, at:at + 32].contiguous()) for at in range(0, width, 32)], 1)
     assert (rode_spmm(csr, B).double() - want).norm() <= 1.01 * (narrow.double() - want).norm()
+
+
+@pytest.mark.parametrize("half,width,rows,degree,longest", [(True, 96, 12000, 14, 900), (True, 160, 4000, 32, 1020), (False, 96, 4000, 32, 1020), (False, 224, 2000, 56, 1000)])
+def test_a_long_row_in_a_small_matrix_keeps_the_narrow_tiles(half, width, rows, degree, longest):
+    """One wave has all of a row of up to 1024 slots, and twice to four times as long for it with wider tiles: the same bits as 32 columns at a time.
+    (12 K rows of 14 halves x 96, longest 899: 11.4 us, and 16.3 with tiles of 128 columns.)"""
+    from gpu_common import DEV
+    from rode_amd import RoDeCSR, rode_spmm
+    gen = torch.Generator(device=DEV).manual_seed(rows)
+    lens = torch.randint(degree // 2, degree + degree // 2, (rows,), device=DEV, generator=gen)
+    lens[::40], lens[rows // 2] = 100, longest
+    ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0)))
+    col = torch.randint(0, rows, (int(ro[-1]),), device=DEV, generator=gen).int()
+    csr = RoDeCSR(ro.int().cpu(), col, torch.rand(col.numel(), device=DEV, generator=gen), DEV, rows, rows, width, config="auto")
+    B = torch.randn(rows, width, device=DEV, generator=gen).to(torch.float16 if half else torch.float32)
+    narrow = torch.cat([rode_spmm(csr, B[:, at:at + 32].contiguous()) for at in range(0, width, 32)], 1)
+    assert torch.equal(rode_spmm(csr, B), narrow)
