@@ -10,7 +10,7 @@ namespace rode {
 // KT = width of the lane tile (32, 64 or 128 elements): LPR = KT / VEC lanes read KT
 // consecutive elements of a dense row per load instruction.  A row of K elements is
 // covered by NS such slabs (KT * NS >= K); EDGE says that the last slab is partial, in
-// which case the lanes past K read nothing and contribute zero.
+// which case the lanes past K contribute zero.
 template <typename T, int KT>
 struct SddmmShape {
     static constexpr int kVec = DenseVec<T>::kElems;
@@ -22,9 +22,12 @@ struct SddmmShape {
                   "unsupported tile width for this dense type");
 };
 
-// <lhs row, rhs row> restricted to this lane's elements.  A lane past K reads the row's first elements and drops what it makes of them: loads
+// <lhs row, rhs row> restricted to this lane's elements.  A lane past K reads the row's last elements and drops what it makes of them: loads
 // under a condition are sent one by one, each waited for (us, SDDMM of width 96, condition -> none: 29 K rows of 12 28.0 -> 19.4, 100 K of 20 154
-// -> 104, power law 200 K 428 -> 250; halves 88 -> 67; width 48 88 -> 66; 4000 rows of 40 8.7 -> 9.0 is the one that does not gain).
+// -> 104, power law 200 K 428 -> 250; halves 88 -> 67; width 48 88 -> 66; 4000 rows of 40 8.3 either way, x 100 8.2 -> 8.4, with the row's first
+// elements 8.7).  Widths whose rows are no whole lines lose where the operand is a few times the L2s and its rows are used often (60 K rows of
+// 110 x 100 314 -> 365, halves x 104 175 -> 190; of 8 and 40 they gain): not for more loads at a time, four at once take 362, nor for those
+// of the lanes past K, without them 356.
 template <typename T, int KT, int NS, bool EDGE>
 __device__ __forceinline__ float lane_dot(const typename DotVec<T>::Reg (&a)[NS][DotVec<T>::kRegs],
                                           const T* __restrict__ row_lane, int k, int lane_elem)
@@ -33,7 +36,7 @@ __device__ __forceinline__ float lane_dot(const typename DotVec<T>::Reg (&a)[NS]
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const bool ok = !EDGE || lane_elem + s * KT < k;
-        const float more = DotVec<T>::dot(a[s], row_lane + (ok ? s * KT : -lane_elem), d);
+        const float more = DotVec<T>::dot(a[s], row_lane + (ok ? s * KT : k - SddmmShape<T, KT>::kVec - lane_elem), d);
         d = ok ? more : d;
     }
     return d;

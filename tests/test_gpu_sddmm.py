@@ -546,10 +546,11 @@ def test_device_given_without_an_index():
     assert out.shape == (csr.nnz,) and torch.isfinite(out).all()
 
 
+@pytest.mark.parametrize("infinite_at", [0, -1])
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("k", [8, 24, 48, 96, 160, 200, 320])
-def test_lanes_past_the_width_add_nothing(k, half):
-    """Widths that leave lanes of a dense row's group without elements: those read the row's first ones and must drop them.  Infinite first
+def test_lanes_past_the_width_add_nothing(k, half, infinite_at):
+    """Widths that leave lanes of a dense row's group without elements: those read others of the row and must drop them.  Infinite first or last
     elements give infinite products and no NaN, and finite rows what they should, in rows of every kernel (block, residue)."""
     import oracle
     from gpu_common import DEV, round_half
@@ -563,7 +564,7 @@ def test_lanes_past_the_width_add_nothing(k, half):
     val = rng.uniform(0.5, 1, len(col)).astype(np.float32)
     lhs, rhs = rng.uniform(0.5, 1, (m, k)).astype(np.float32), rng.uniform(0.5, 1, (n, k)).astype(np.float32)
     lhs, rhs = (round_half(lhs), round_half(rhs)) if half else (lhs, rhs)
-    rhs[::5, 0] = np.inf
+    rhs[::5, infinite_at] = np.inf
     csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, locality=False)
     kind = torch.float16 if half else torch.float32
     got = rode_sddmm(csr, torch.from_numpy(lhs).to(DEV, kind), torch.from_numpy(rhs).to(DEV, kind)).cpu().numpy().astype(np.float64)
