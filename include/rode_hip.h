@@ -324,7 +324,7 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
  *                         Costs time at worst.
  *   tile_fours            0, or what rode_hip_group_plan_fours said of the group plan: the columns that every four
  *                         neighbouring tiles cover between them, over the most that four do (a sliding window: about
- *                         a quarter of the tiles).  With it the attention kernels for halves take four
+ *                         a quarter of the tiles); 0 where more than one in sixteen fours lie apart.  With it the attention kernels for halves take four
  *                         tiles at a time where that pays.  Costs time at worst.
  * Same results as without a plan, up to the order of the fp32 additions inside a row.
  */

@@ -231,7 +231,8 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
     const hipError_t waited = hipStreamSynchronize(as_stream(stream)); // (also after an error: the copy is into memory of this call)
     if (e == hipSuccess) e = waited;
     if (e == hipSuccess && both) h_counts[0] = got[4], h_counts[1] = got[5], h_counts[2] = got[6], h_counts[3] = got[3];
-    if (e == hipSuccess && h_tile_fours) *h_tile_fours = got[0] == 0 && got[2] > 0 ? got[1] / got[2] : 0;
+    // (a few fours that lie apart - the ends of documents in a packed batch - count as long as they are)
+    if (e == hipSuccess && h_tile_fours) *h_tile_fours = got[2] > 0 && 64ll * got[0] <= rode::row_tiles(M) ? got[1] / got[2] : 0;
     return e;
 }
 

@@ -159,14 +159,10 @@ group_tiles_kernel(int tiles, const RowGroup* __restrict__ groups, const int* __
         widest = max(widest, __shfl_xor(widest, x, kWave));
     }
     if (threadIdx.x % 4 != 0 || widest == 0) return;
-    if (2ll * (hi - lo) > 3ll * widest) {
-        atomicAdd(fours, 1);
-    } else {
-        atomicAdd(fours + 1, hi - lo);
-        atomicMax(fours + 2, hi - lo);
-    }
+    if (2ll * (hi - lo) > 3ll * widest) atomicAdd(fours, 1);
+    atomicAdd(fours + 1, hi - lo);
+    atomicMax(fours + 2, hi - lo);
 }
-
 
 __global__ void group_header_kernel(int M, int groups, int* __restrict__ plan)
 {

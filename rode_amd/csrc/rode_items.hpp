@@ -455,7 +455,7 @@ __host__ __device__ inline int row_tiles(int M) { return M / kTileRows; }
 // 16-byte aligned, a RowTile per 16 rows.
 __host__ __device__ inline size_t group_runs_at(int M) { return kGroupHeaderInts + (size_t)row_groups(M) * (sizeof(RowGroup) / sizeof(int)); }
 __host__ __device__ inline size_t group_tiles_at(int M) { return (group_runs_at(M) + 3 * (size_t)M + 3) & ~(size_t)3; }
-// (behind the tiles, of every four of them with a run: how many lie apart, the columns that the others cover in all, the most that four do;
+// (behind the tiles, of every four of them with a run: how many lie apart, the columns that all of them cover, the most that four do;
 // then the header's tiles, groups, groups with a run and rows outside those again; only where there are 16 rows)
 __host__ __device__ inline size_t group_fours_at(int M) { return group_tiles_at(M) + (size_t)row_tiles(M) * (sizeof(RowTile) / sizeof(int)); }
 __host__ __device__ inline size_t group_plan_ints(int M) { return group_fours_at(M) + 8; }

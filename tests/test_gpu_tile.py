@@ -479,6 +479,26 @@ def test_how_many_fours_a_plan_is_worth_and_runs_that_lie_apart():
     torch.testing.assert_close(sparse_attention(apart, q, k, v), one, rtol=2e-5, atol=2e-6)
 
 
+def test_a_few_fours_that_lie_apart():
+    """Documents of 528 rows in a batch, a window of 160: at their ends, between tiles and inside of 64 rows, four tiles lie apart, three fours in
+    thirty-two; with one end one."""
+    m, d = 2048, 64
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    row, column = np.arange(m)[:, None], np.arange(m)[None]
+    for ends, worth in ((np.arange(528, m, 528), False), (np.array([528]), True)):
+        which = np.searchsorted(ends, np.arange(m), side="right")
+        allowed = (np.abs(row - column) <= 80) & (which[:, None] == which[None])
+        col = np.nonzero(allowed)[1].astype(np.int32)
+        rp = np.concatenate(([0], np.cumsum(allowed.sum(1)))).astype(np.int32)
+        csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.ones(len(col)), "cuda", m, m, d, locality=True)
+        assert csr.plan.tile_fours > 20 if worth else csr.plan.tile_fours == 0
+        csr.call_plans().tile_fours = 1 << 20
+        q, k, v = (torch.randn(_heads(csr), m, d, device="cuda", generator=gen).half() for _ in range(3))
+        out = sparse_attention(csr, q, k, v, scale=0.2)
+        want = _reference(torch.from_numpy(allowed.astype(np.float64)).cuda(), q[0], k[0], v[0], 0.2)
+        assert (out[0].double() - want).abs().max() <= 2e-5 * want.abs().max()
+
+
 @pytest.mark.parametrize("keep", [None, "scores", "probs"])
 @pytest.mark.parametrize("bad", [False, True])
 def test_nonzeros_outside_the_runs_first(bad, keep):
