@@ -72,15 +72,19 @@ constexpr int kMergeMinSegments = 16384;
 //     13.1 -> 11.9 (5206).  Up to 3072 for tiles of 256 bytes (8000 rows of 40 halves x 128, L 2000 14.7 -> 12.1, 3000 14.8 -> 14.6, 4000 15.2 -> 16.8;
 //     3000 x 64 2000 11.0 -> 7.3, 3000 11.5 -> 9.4, 4000 11.5 -> 11.1), 2048 of 512 (8000 x 128 2000 20.3 -> 19.4, 3000 20.9 -> 24.9);
 //   * L up to 6656 from 300 MB on: 27 K of 26 x 128 33.4 -> 29.4 (5640), 59 K of 30 halves x 128 52.8 -> 47.8 (6141), 51 K of 19 x 128 50.1 -> 47.6
-//     (6677); 29 K of 32 x 128 40.4 -> 41.9 (7741);
+//     (6677); 29 K of 32 x 128 40.4 -> 41.9 (7741).  Above 666 MB a slot for every 100 KB, up to the 20 000 that have been measured: 100 K of 24 x 128
+//     (1.2 GB) 152.2 -> 146.8 (12 000), 300 K of 16 (2.4 GB) 363.6 -> 363.4 (12 000), 383.3 -> 382.5 (20 000), 400 K (3.3 GB) 493 -> 491 (20 000), of 24
+//     (4.8 GB) 682 -> 688 (12 000), 686 -> 691 (20 000), of halves 368.5 either way;
 //   * segments of more than 128 slots, whose rows of up to six segments may have no workgroup, from 500 MB on: 200 K of 16 x 64 120.4 -> 116.5,
 //     150 K x 128 167 -> 163, 180 K of 20 halves x 128 135 -> 132; 113 K of 23 x 32, 332 MB, 44.7 -> 49.6.
+// 2-norms of the long rows' errors against fp64, relative to adding their segments up (which were merged to 512 slots as well): 0.97 to 1.006,
+// rows of 1100 to 6500, widths 32 to 128, both types.
 inline bool wide_rows_pay(int longest, int seg_length, size_t tile_bytes, size_t gathered)
 {
     constexpr size_t MB = 1000000;
     if (seg_length > (gathered >= 500 * MB ? 512 : 128)) return false;
     if (gathered < (tile_bytes > 256 ? 500 : 300) * MB) return longest <= (tile_bytes > 256 ? 2048 : tile_bytes > 128 ? 3072 : 4096);
-    return (size_t)longest <= max((size_t)6656, gathered / 100000);
+    return (size_t)longest <= min(max((size_t)6656, gathered / 100000), (size_t)20000);
 }
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists

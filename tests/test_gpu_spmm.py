@@ -906,10 +906,40 @@ def test_a_long_row_in_a_small_matrix_keeps_the_narrow_tiles(half, width, rows, 
     from rode_amd import RoDeCSR, rode_spmm
     gen = torch.Generator(device=DEV).manual_seed(rows)
     lens = torch.randint(degree // 2, degree + degree // 2, (rows,), device=DEV, generator=gen)
-    lens[::40], lens[rows // 2] = 100, longest
+    lens[::8], lens[rows // 2] = 100, longest
     ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0)))
     col = torch.randint(0, rows, (int(ro[-1]),), device=DEV, generator=gen).int()
     csr = RoDeCSR(ro.int().cpu(), col, torch.rand(col.numel(), device=DEV, generator=gen), DEV, rows, rows, width, config="auto")
+    assert csr.m1 >= 1024  # (rows with one work item each: no sum depends on the order of several)
     B = torch.randn(rows, width, device=DEV, generator=gen).to(torch.float16 if half else torch.float32)
     narrow = torch.cat([rode_spmm(csr, B[:, at:at + 32].contiguous()) for at in range(0, width, 32)], 1)
     assert torch.equal(rode_spmm(csr, B), narrow)
+
+
+@pytest.mark.parametrize("k,dtype", [(32, "f32"), (64, "f32"), (128, "f32"), (64, "f16"), (128, "f16"), (64, "f64")])
+def test_rows_of_thousands_of_slots_by_a_workgroup_each(k, dtype):
+    """Rows of 5 000 to 20 000 aligned slots in segments of 512, which the rule leaves to workgroups in matrices with 2 GB to gather (said of a smaller one): quarters
+    of two to ten parts.  Not the bits of adding their segments up, and none left of what C held."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, rode_sddmm_hip
+    rng = np.random.default_rng(k)
+    m, n = 3000, 24000
+    lens = rng.integers(0, 70, m)
+    long_ones = np.arange(100, 900, 100)
+    lens[long_ones] = 5000, 6656, 19990, 8191, 8193, 12001, 4097, 16001
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens]).astype(np.int32)
+    val, dense = rng.uniform(-1, 1, len(col)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    dense = round_half(dense) if dtype == "f16" else dense
+    csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, config={"seg_length": 512, "k_block": 32, "vec_len": 4},
+                  locality=False)
+    csr = csr.with_values(csr.values.double()) if dtype == "f64" else csr
+    assert csr.m1 >= 1024 and 19990 <= csr.longest_row <= 20000
+    B = torch.from_numpy(dense).to(DEV, {"f32": torch.float32, "f16": torch.float16, "f64": torch.float64}[dtype])
+    plans = rode_sddmm_hip.plans_struct(None, whole_lists=True, seg_length=512, nonzeros=2_000_000_000 // (k * B.element_size()))
+    got, added = (_into_nan(csr, B, longest, plans) for longest in (csr.longest_row, 0))
+    assert not np.array_equal(got[long_ones], added[long_ones])
+    want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
+    # roundings of a sum: 512 slots over two lane groups, nine more parts, the groups (5), the waves (3) and the product
+    assert (np.abs(got - want) <= scale * (256 + 9 + 5 + 3 + 1) * (2.0 ** -53 if dtype == "f64" else 2.0 ** -24)).all()
