@@ -155,6 +155,30 @@ def test_decomposition_without_memory_leaves_nothing_running():
         assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
 
 
+def test_decomposition_of_sent_offsets_without_memory_leaves_nothing_running():
+    """As `RoDeCSR` calls it: a copy of the offsets is on its way whatever fails."""
+    m = 1_000_000  # (rows of 40: both lists have entries)
+    ro = torch.arange(m + 1, dtype=torch.int32) * 40
+    col = torch.arange(40 * m, dtype=torch.int32, device="cuda") // 40
+    stream = rode_sddmm_hip._stream_handle(col.device)
+    refused, results = 0, []
+    while len(results) < 2:
+        on_gpu = torch.full((m + 1,), -1, dtype=torch.int32, device="cuda")
+        torch.cuda.synchronize()
+        _lib.host_call().send_offsets(ro, on_gpu, 8, stream)
+        mode = _Refuse(refused + 1 if not results else -1)
+        with mode:
+            try:
+                results.append(_lib.host_call().decompose(ro, on_gpu, col, m, 512, stream, None))
+            except MemoryError:
+                refused += 1
+                assert torch.cuda.current_stream().query()
+        assert torch.equal(on_gpu.cpu(), ro)
+    assert refused >= 5 and results[1][5] is not None  # the lists, the plan and the counts
+    for a, b in zip(*results):
+        assert torch.equal(a, b) if isinstance(a, torch.Tensor) else a == b
+
+
 @pytest.mark.parametrize("upload", [False, True])
 @pytest.mark.parametrize("m,n", [(1, 600), (127, 600), (128, 600), (129, 600), (33000, 33000)])
 def test_decomposition_with_a_plan_equals_its_parts(m, n, upload):
