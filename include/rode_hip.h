@@ -314,10 +314,12 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
  *                         wavefront, and with the length known the grid is sized for that.
  *                         Without it the kernels read the length off the lists and the
  *                         grid is capped instead.  A wrong value costs time, never a result.
- *   columns_local         0, or nonzero when the columns of neighbouring rows lie close together
+ *   columns_local         0, or 1 when the columns of neighbouring rows lie close together
  *                         (most chunks of the residue list have a window: a band).  Knowledge as
  *                         well: SpMM then does not deal column tiles out to the XCDs, which pays
- *                         when dense rows are referenced at random.  Costs time at worst.
+ *                         when dense rows are referenced at random.  Plus, where no row has more than twice as many
+ *                         as there are on average, twice the nonzeros a row: SDDMM of widths other than 32, 64, 128 and
+ *                         their multiples then decides by them how many dense rows a wave has on their way.  Costs time at worst.
  *   nonzeros              0, or the nonzeros of the matrix.  With it a call may leave a locality plan
  *                         unused where the window kernels do not pay (short rows, a last round of few
  *                         chunks), and dealing tiles out depends on how often a dense row is used.
@@ -339,7 +341,7 @@ typedef struct rode_hip_plans {
     const void* groups;
     const int* group_counts;
     int seg_length;
-    int columns_local;
+    int columns_local; /* and nonzeros a row (above) */
     int nonzeros;
     int tile_fours;
 } rode_hip_plans;

@@ -249,7 +249,8 @@ bool plan_ref(const rode_hip_plans* p, int m2, rode::PlanRef& plan)
     if (!p) return true;
     if (p->seg_length < 0) return false;
     plan.seg_length = p->seg_length;
-    plan.columns_local = p->columns_local != 0;
+    plan.columns_local = (p->columns_local & 1) != 0;
+    plan.equal_rows = p->columns_local > 1 ? p->columns_local >> 1 : 0;
     plan.nonzeros = p->nonzeros;
     const bool window = p->window && p->window_rows; // (one without rows: the standard kernels do everything)
     if (p->groups) {
@@ -407,13 +408,13 @@ int rode_hip_sddmm_planned(int dtype, int flags, int m1, int m2, int n, int k, c
                            const void* d_rhs_matrix, float* d_out, const rode_hip_plans* plans, void* stream1,
                            void* stream2)
 {
-    (void)n;
     if (m1 < 0 || m2 < 0 || (flags & ~rode::kOnlyMask) || (flags & (flags - 1))) return hipErrorInvalidValue;
     if (m1 == 0 && m2 == 0) return hipSuccess;
     if (!aligned16(d_lhs_matrix) || !aligned16(d_rhs_matrix)) return hipErrorInvalidValue;
     rode::PlanRef plan;
     if (!plan_ref(plans, m2, plan)) return hipErrorInvalidValue;
     plan.only = flags;
+    plan.dense_rows = n > 0 ? n : 0;
     switch (dtype) {
     case RODE_DENSE_F32:
         return rode::sddmm_launch<float>(m1, m2, k, d_row_indices_block, d_row_indices_residue, d_st_offsets,

@@ -59,6 +59,7 @@ struct PlanRef {
     // SpMM: rows of C where it is not cleared (0: it is, or every row is stored), the longest row in aligned slots (0: not said)
     int c_rows = 0, longest = 0;
     bool columns_local = false; // the caller knows that the columns of neighbouring rows lie close together
+    int equal_rows = 0;         // nonzeros a row where no row has more than twice as many (0: not so, or not said)
     // Segment length of the decomposition the lists were made with, 0: not known
     int seg_length = 0;
 };

@@ -35,7 +35,7 @@ namespace {
 // quarter of the waves in registers and gives 0 to 1.5 % where block segments have a launch of their own (this switch
 // alone, us: power law 2 M x 64 halves 949 -> 945, 2 M x 128 3727 -> 3715, 300 K x 128 645 -> 637, of halves 338 -> 333; 400 K rows of 100,
 // width 64 1456 -> 1444; lognormal 65 K either way); not for small matrices (14 K rows of 40: 24.7 -> 26.1).
-template <typename T, int KT, int NS, bool EDGE, bool AHEAD>
+template <typename T, int KT, int NS, int EDGE, bool AHEAD>
 __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int cnt, int split, int jump, int k, int lane,
                                                 int* lds_cols,
                                                 const int* __restrict__ col, const float* __restrict__ val,
@@ -84,7 +84,7 @@ __device__ __forceinline__ void sddmm_row_slots(int row, int base, int mask, int
 // (bid of nblocks: the workgroup's position in the part of the grid that works on block segments)
 // WALK: 0 one wave per segment only, 1 chunks only (chunk_hint > 1), 2 either, found out here.  (Kernels of their
 // own, so that the code of one way does not cost the other registers.)
-template <typename T, int KT, int NS, bool EDGE, int WALK, bool AHEAD>
+template <typename T, int KT, int NS, int EDGE, int WALK, bool AHEAD>
 __device__ __forceinline__ void
 sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                  const int* __restrict__ st_off,
@@ -134,7 +134,7 @@ sddmm_block_body(int bid, int nblocks, int m1, int k, int chunk_hint, RowOwners 
 // with N = len + (s & 3), rows with N >= 32 keep only their last N % 32 slots
 // starting at (s & ~3) + floor(N / 32) * 32; shorter rows are taken whole.
 // Lane ls of the group owns the slots ls, ls + LPR, ... (value, result, store).
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 __device__ __forceinline__ void
 sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const int* __restrict__ residue_rows,
                    const int* __restrict__ row_ptr, const int* __restrict__ col, const float* __restrict__ val,
@@ -211,7 +211,7 @@ sddmm_residue_body(int bid, int nblocks, int m2, int k, RowOwners owners, const 
     }
 }
 
-template <typename T, int KT, int NS, bool EDGE, int WALK>
+template <typename T, int KT, int NS, int EDGE, int WALK>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_block_kernel(int m1, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                    const int* __restrict__ st_off,
@@ -222,7 +222,7 @@ sddmm_block_kernel(int m1, int k, int chunk_hint, RowOwners owners, const int* _
                                       lhs, rhs, out);
 }
 
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_residue_kernel(int m2, int k, RowOwners owners, const int* __restrict__ residue_rows, const int* __restrict__ row_ptr,
                      const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ lhs,
@@ -234,7 +234,7 @@ sddmm_residue_kernel(int m2, int k, RowOwners owners, const int* __restrict__ re
 
 // Both lists in one launch: the first g1 workgroups work on block segments, the others on
 // residue rows.  For matrices so small that a launch costs as much as its kernel.
-template <typename T, int KT, int NS, bool EDGE, int WALK>
+template <typename T, int KT, int NS, int EDGE, int WALK>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_pair_kernel(int g1, int m1, int m2, int k, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                   const int* __restrict__ residue_rows,
@@ -254,7 +254,7 @@ sddmm_pair_kernel(int g1, int m1, int m2, int k, int chunk_hint, RowOwners owner
 // and step, their columns and values loaded together, their dot products one row after the
 // other without a wait in between (row after row, a wave sits through the memory round trips
 // of every row).  lds_cols: kGroupRows * 64 ints of this wave.
-template <typename T, int KT, bool EDGE>
+template <typename T, int KT, int EDGE>
 __device__ __forceinline__ void sddmm_group_leftovers(const RowGroup& d, int row0, int k, int lane,
                                                       int* lds_cols, const int* __restrict__ row_ptr,
                                                       const int* __restrict__ col, const float* __restrict__ val,
@@ -319,7 +319,7 @@ __device__ __forceinline__ void sddmm_group_leftovers(const RowGroup& d, int row
 // (A variant in which the four waves of a workgroup took four consecutive groups and read
 // the union of their runs through LDS tiles, loaded once per workgroup, ran in the same
 // time on config 5 - 0.049 ms fp32, 0.035 against 0.033 ms fp16 - and was taken out.)
-template <typename T, int KT, bool EDGE, int WPG>
+template <typename T, int KT, int EDGE, int WPG>
 __global__ void __launch_bounds__(kWgThreads)
 sddmm_group_kernel(int k, int n_groups, const RowGroup* __restrict__ groups, const int* __restrict__ row_ptr,
                    const int* __restrict__ col, const float* __restrict__ val, const T* __restrict__ lhs,
@@ -424,7 +424,7 @@ sddmm_group_kernel(int k, int n_groups, const RowGroup* __restrict__ groups, con
 
 // The rows of a hub plan, cut into pieces by column slab (rode_items.hpp), slab after slab, so that the hub rows' nonzeros of
 // one slab of rhs are worked on at the same time on one XCD and find rhs's rows in its L2.
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 __global__ void __launch_bounds__(kHubWavesMax * kWave)
 sddmm_hub_kernel(int k, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col, const float* __restrict__ val,
                  const T* __restrict__ lhs, const T* __restrict__ rhs, float* __restrict__ out)
@@ -452,7 +452,7 @@ inline int grid_for_waves(long long nwaves)
     return wgs * kWgThreads < (1ll << 32) ? (int)wgs : -1;
 }
 
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* residue_rows, const int* st_off,
                   const int* row_ptr, const int* col, const float* val, const T* lhs, const T* rhs, float* out,
                   PlanRef plan, hipStream_t s1, hipStream_t s2)
@@ -508,7 +508,7 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     if (e == hipSuccess && hubs) {
         const HubGrid hub_wgs = hub_grid(hub_rows, plan.hub_counts[1]);
         if (hub_wgs.wgs < 0) return hipErrorInvalidConfiguration;
-        sddmm_hub_kernel<T, KT, NS, EDGE><<<hub_wgs.wgs, hub_wgs.waves * kWave, 0, s1>>>(k, hub_wgs, plan.hub, col, val, lhs, rhs, out);
+        sddmm_hub_kernel<T, KT, NS, (EDGE != 0 ? kPartial : 0)><<<hub_wgs.wgs, hub_wgs.waves * kWave, 0, s1>>>(k, hub_wgs, plan.hub, col, val, lhs, rhs, out);
         e = hipGetLastError();
     }
     if constexpr (NS == 1) {
@@ -517,10 +517,10 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
             // (two waves per group, 8192 waves on config 5: 0.052 ms instead of 0.038)
             if (plan.group_counts[1] >= kGroupWaveEach) {
                 const int wgs = (owners.n_groups + kWavesPerWg - 1) / kWavesPerWg;
-                sddmm_group_kernel<T, KT, EDGE, 1><<<(wgs + kXcds - 1) / kXcds * kXcds, kWgThreads, 0, s1>>>(
+                sddmm_group_kernel<T, KT, (EDGE != 0 ? kPartial : 0), 1><<<(wgs + kXcds - 1) / kXcds * kXcds, kWgThreads, 0, s1>>>(
                     k, owners.n_groups, owners.groups, row_ptr, col, val, lhs, rhs, out);
             } else {
-                sddmm_group_kernel<T, KT, EDGE, kWavesPerWg><<<(owners.n_groups + kXcds - 1) / kXcds * kXcds, kWgThreads, 0, s1>>>(
+                sddmm_group_kernel<T, KT, (EDGE != 0 ? kPartial : 0), kWavesPerWg><<<(owners.n_groups + kXcds - 1) / kXcds * kXcds, kWgThreads, 0, s1>>>(
                     k, owners.n_groups, owners.groups, row_ptr, col, val, lhs, rhs, out);
             }
             e = hipGetLastError();
@@ -531,14 +531,33 @@ hipError_t launch(int m1, int m2, int k, const int* block_rows, const int* resid
     return e;
 }
 
+// Rows of about equal length go through their ascending columns side by side, and what one wave brings into L2 the others are about to use:
+// with many loads of a wave on their way the waves are further apart, and more of those rows are gone (28 K rows of 200, widths 116 and 128 in turn: L2
+// hits of both together 51 -> 37 % without the condition of lane_dot for 116).  So operands of 5 MB and more are read one by one where that costs more than the waiting: the larger
+// the operand, the longer the rows and their tails, and the fewer lanes have nothing.  us, condition -> none, uniform degrees: 24 K
+// rows of 110 x 200 190 -> 235, 28 K of 200 x 116 1.46 times, 40 K of 110 x 100 175 -> 212, 60 K 316 -> 363, halves x 104 176 -> 191; 40 K of 80 x 80 0.86 times,
+// 16 K of 110 x 100 0.83, 90 K of 40 x 100 0.90.  Lognormal degrees: 0.6 to 1.0 at all sizes.  Fitted to 4218 calls (36 to 496 columns, 8 K to 300 K rows
+// of 8 to 200): 75 of them are more than 3 % slower than with the condition (without this rule 642), the most 1.20 (1.47), and all together take
+// 0.861 of that time (0.870).
+inline bool loads_apart(const PlanRef& plan, size_t row_bytes, float filled)
+{
+    const size_t bytes = plan.dense_rows * row_bytes;
+    if (plan.equal_rows == 0 || plan.columns_local || plan.dev || plan.groups || plan.hub || bytes < 5000000) return false;
+    const float size = logf((float)bytes / 8e6f), slots = (float)plan.equal_rows, tail = (float)(plan.equal_rows % kBlockItems) / (float)kBlockItems;
+    return 0.16f * size - 0.035f * size * size + 0.0014f * slots + 0.31f * filled + 0.067f * tail > 0.48f;
+}
+
 template <typename T, int KT, int NS>
 hipError_t launch_edge(bool edge, int m1, int m2, int k, const int* block_rows, const int* residue_rows,
                        const int* st_off, const int* row_ptr, const int* col, const float* val, const T* lhs,
                        const T* rhs, float* out, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
-    return edge ? launch<T, KT, NS, true>(m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs, out,
+    if constexpr (KT >= 64)
+        if (edge && loads_apart(plan, (size_t)k * sizeof(T), (float)k / (float)(KT * NS)))
+            return launch<T, KT, NS, kPartialApart>(m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs, out, plan, s1, s2);
+    return edge ? launch<T, KT, NS, kPartial>(m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs, out,
                                           plan, s1, s2)
-                : launch<T, KT, NS, false>(m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs,
+                : launch<T, KT, NS, 0>(m1, m2, k, block_rows, residue_rows, st_off, row_ptr, col, val, lhs, rhs,
                                            out, plan, s1, s2);
 }
 

@@ -9,8 +9,10 @@ namespace rode {
 // ---- SDDMM ------------------------------------------------------------------
 // KT = width of the lane tile (32, 64 or 128 elements): LPR = KT / VEC lanes read KT
 // consecutive elements of a dense row per load instruction.  A row of K elements is
-// covered by NS such slabs (KT * NS >= K); EDGE says that the last slab is partial, in
+// covered by NS such slabs (KT * NS >= K); EDGE (kPartial, kPartialApart) says that the last slab is partial, in
 // which case the lanes past K contribute zero.
+constexpr int kPartial = 1;
+constexpr int kPartialApart = 2; // ... and the loads of the slots come one by one (lane_dot)
 template <typename T, int KT>
 struct SddmmShape {
     static constexpr int kVec = DenseVec<T>::kElems;
@@ -25,10 +27,8 @@ struct SddmmShape {
 // <lhs row, rhs row> restricted to this lane's elements.  A lane past K reads the row's last elements and drops what it makes of them: loads
 // under a condition are sent one by one, each waited for (us, SDDMM of width 96, condition -> none: 29 K rows of 12 28.0 -> 19.4, 100 K of 20 154
 // -> 104, power law 200 K 428 -> 250; halves 88 -> 67; width 48 88 -> 66; 4000 rows of 40 8.3 either way, x 100 8.2 -> 8.4, with the row's first
-// elements 8.7).  Widths whose rows are no whole lines lose where the operand is a few times the L2s and its rows are used often (60 K rows of
-// 110 x 100 314 -> 365, halves x 104 175 -> 190; of 8 and 40 they gain): not for more loads at a time, four at once take 362, nor for those
-// of the lanes past K, without them 356.
-template <typename T, int KT, int NS, bool EDGE>
+// elements 8.7).  kPartialApart keeps the condition, for the calls that are faster with it (loads_apart, rode_sddmm.hip).
+template <typename T, int KT, int NS, int EDGE>
 __device__ __forceinline__ float lane_dot(const typename DotVec<T>::Reg (&a)[NS][DotVec<T>::kRegs],
                                           const T* __restrict__ row_lane, int k, int lane_elem)
 {
@@ -36,6 +36,10 @@ __device__ __forceinline__ float lane_dot(const typename DotVec<T>::Reg (&a)[NS]
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         const bool ok = !EDGE || lane_elem + s * KT < k;
+        if constexpr (EDGE == kPartialApart) {
+            if (ok) d = DotVec<T>::dot(a[s], row_lane + s * KT, d);
+            continue;
+        }
         const float more = DotVec<T>::dot(a[s], row_lane + (ok ? s * KT : k - SddmmShape<T, KT>::kVec - lane_elem), d);
         d = ok ? more : d;
     }
@@ -58,7 +62,7 @@ __device__ __forceinline__ float sddmm_quad_reduce(const float (&p)[4], int ls)
 
 // Dot products of the 32-slot units of one step, the slots' columns already in lds_cols
 // (lds_cols[e] = column of lane e's slot).  Returns the dot product for this lane's slot.
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 __device__ __forceinline__ float sddmm_unit_staged(const T* __restrict__ rhs_lane,
                                                    const typename DotVec<T>::Reg (&a)[NS][DotVec<T>::kRegs], int k,
                                                    const int* lds_cols, int lane)
@@ -86,7 +90,7 @@ __device__ __forceinline__ float sddmm_unit_staged(const T* __restrict__ rhs_lan
 
 // Dot products of one 32-slot unit of a block segment.  `my_col` is the column of this
 // lane's slot.  Returns the dot product for this lane's slot.
-template <typename T, int KT, int NS, bool EDGE>
+template <typename T, int KT, int NS, int EDGE>
 __device__ __forceinline__ float sddmm_unit(const T* __restrict__ rhs_lane,
                                             const typename DotVec<T>::Reg (&a)[NS][DotVec<T>::kRegs], int my_col, int k,
                                             int* lds_cols, int lane)
@@ -100,7 +104,7 @@ __device__ __forceinline__ float sddmm_unit(const T* __restrict__ rhs_lane,
 // hint, so that the stream of lhs rows does not displace gathered rhs rows (config 4: residue
 // kernel 1.375 -> 1.334 ms at K=128, 0.656 -> 0.626 at K=64; for the group kernels, which
 // read their lhs rows twice, the hint costs 8 %).
-template <typename T, int KT, int NS, bool EDGE, bool ONCE = false>
+template <typename T, int KT, int NS, int EDGE, bool ONCE = false>
 __device__ __forceinline__ void load_lhs_slice(const T* __restrict__ lhs, int row, int k, int lane,
                                                typename DotVec<T>::Reg (&a)[NS][DotVec<T>::kRegs])
 {

@@ -38,6 +38,7 @@ class RoDeCSR:
 
     DEFAULT_CONFIG = {"seg_length": 512, "k_block": 32, "vec_len": 4}  # for a k that is not in CONFIGS
     MAX_K = 512
+    equal_rows = 0  # nonzeros a row where no row has more than twice as many, else 0
     # Windowed chunks of 128 residue rows below which "auto" drops the plan: two full rounds of the window
     # kernels.  With fewer, what is won by some calls (us without -> with a plan, 400 chunks of rows of 27: SDDMM
     # of width 128 34.8 -> 22.9, of 64 18.8 -> 14.8, of 128 halves 18.8 -> 16.3, SpMM of 128 28.3 -> 23.7) others lose
@@ -81,6 +82,8 @@ class RoDeCSR:
 
     def _set_up(self, column_indices, values, config, locality):
         self.max_row_length = self._stats[0]
+        if self.max_row_length * self.m <= 2 * self.nnz:
+            self.equal_rows = min(self.nnz // max(self.m, 1), 1 << 20)
         if config == "auto":
             config = self._config_from(self._stats)
         self.config = dict(config) if config is not None else dict(self.CONFIGS.get(self.k, self.DEFAULT_CONFIG))
@@ -217,7 +220,7 @@ class RoDeCSR:
             # (set once: of two threads' first calls one struct stays, for both)
             plans = self._shared.setdefault(key, rode_sddmm_hip.plans_struct(
                 self.plan, spmm_width, spmm_elem_bytes, True, seg_length=self.config["seg_length"], columns_local=self.columns_local,
-                nonzeros=self.nnz))
+                nonzeros=self.nnz, equal_rows=self.equal_rows))
         return plans
 
     def plans_address(self, spmm_width=None):

@@ -310,16 +310,17 @@ def group_plan(row_offsets, column_indices, m):
 
 
 def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg_length=0, columns_local=False,
-                 nonzeros=0):
+                 nonzeros=0, equal_rows=0):
     """The ``rode_hip_plans`` struct of one call (keep it alive until the call returns; pass
     it with ``ctypes.byref``).  ``plan``: a ``WindowPlan``, a ``HubPlan``, a ``GroupPlan`` or None.
     ``spmm_width``: the dense width of SpMM calls that share the hub plan's kept workspace (None: none is
     attached).  ``whole_lists``: without that promise a hub or group plan is left out.
     ``seg_length``: the segment length the lists were made with, 0 when not known.
     ``columns_local``: the columns of neighbouring rows are known to lie close together.
-    ``nonzeros``: of the matrix, 0 when not known."""
+    ``nonzeros``: of the matrix, 0 when not known.
+    ``equal_rows``: nonzeros a row where no row has more than twice as many, else 0."""
     p = _lib.Plans()
-    p.columns_local = int(columns_local)
+    p.columns_local = int(columns_local) | equal_rows << 1
     p.nonzeros = int(nonzeros)
     p.seg_length = int(seg_length or 0)  # (the segment length of the decomposition, when the caller knows it)
     if isinstance(plan, GroupPlan):
@@ -336,7 +337,7 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
         p.window, p.window_rows = plan.data.data_ptr(), plan.rows.data_ptr()
         p.window_counts = ctypes.addressof(plan._header)
         p.nonzeros = plan.nonzeros
-        p.columns_local = int(columns_local or 2 * plan.windowed > plan.counts[0])
+        p.columns_local |= int(2 * plan.windowed > plan.counts[0])
     return p
 
 

@@ -574,3 +574,64 @@ def test_lanes_past_the_width_add_nothing(k, half, infinite_at):
     want = val.astype(np.float64) * np.einsum("ij,ij->i", lhs[row].astype(np.float64), np.where(np.isinf(rhs), 0, rhs)[col].astype(np.float64))
     # a rounding per product and sum (k of each at most) and the value's; halves' products are exact
     assert (np.abs(got - want) <= want * (2 * k + 1) * 2.0 ** -24)[~infinite].all()
+
+
+@pytest.mark.parametrize("k,half", [(36, False), (60, False), (68, False), (100, False), (124, False), (132, False), (200, False), (300, False), (500, False),
+                                    (72, True), (120, True), (136, True), (248, True), (400, True)])
+def test_dense_rows_read_one_by_one(k, half):
+    """Rows of equal length and a large operand, as the rule asks for (said of a matrix that is neither): the bits of reading as many as there are registers
+    for, in block segments, tails and rows without either, and those of the oracle."""
+    import oracle
+    from gpu_common import DEV, round_half
+    from rode_amd import RoDeCSR, rode_sddmm
+    rng = np.random.default_rng(k)
+    m, n = 300, 60_000
+    lens = rng.integers(0, 70, m)
+    lens[7], lens[100] = 1390, 200
+    rp = np.concatenate(([0], np.cumsum(lens))).astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, L, replace=False)) for L in lens]).astype(np.int32)
+    val = rng.uniform(-1, 1, len(col)).astype(np.float32)
+    lhs, rhs = rng.standard_normal((m, k)).astype(np.float32), rng.standard_normal((n, k)).astype(np.float32)
+    lhs, rhs = (round_half(lhs), round_half(rhs)) if half else (lhs, rhs)
+    kind = torch.float16 if half else torch.float32
+    out = []
+    for equal_rows in (0, 700):
+        csr = RoDeCSR(torch.from_numpy(rp), torch.from_numpy(col), torch.from_numpy(val), DEV, m, n, k, locality=False)
+        csr.equal_rows = equal_rows
+        out.append(rode_sddmm(csr, torch.from_numpy(lhs).to(DEV, kind), torch.from_numpy(rhs).to(DEV, kind)))
+        assert csr.call_plans().columns_local == 2 * equal_rows
+    assert torch.equal(*out)
+    want, scale = oracle.sddmm_f64(rp, col, val, lhs, rhs, with_abs=True)
+    # a rounding per product and sum of a lane and of the lanes' sums (k of each at most) and the value's
+    assert (np.abs(out[1].cpu().numpy() - want) <= scale * (2 * k + 1) * 2.0 ** -24).all()
+
+
+def test_rows_of_equal_length_stay_together():
+    """28 000 rows of 200 x 116 go through their columns side by side and find each other's dense rows in L2: with many of them on a wave's way
+    the call takes 1.4 times as long."""
+    from gpu_common import DEV
+    from rode_amd import RoDeCSR, rode_sddmm
+    m, degree, k = 28_000, 200, 116
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    lens = torch.poisson(torch.full((m,), float(degree), device=DEV), generator=gen).long()
+    ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0)))
+    row = torch.arange(m, device=DEV).repeat_interleave(lens)
+    col = (torch.sort(torch.randint(0, m, (len(row),), device=DEV, generator=gen) + row * m)[0] % m).int()
+    lhs, rhs = (torch.randn(m, k, device=DEV, generator=gen) for _ in range(2))
+    took = []
+    for known in (False, True):
+        csr = RoDeCSR(ro.int().cpu(), col, torch.ones(len(col), device=DEV), DEV, m, m, k, config="auto")
+        assert csr.equal_rows == len(col) // m
+        if not known:
+            csr.equal_rows = 0
+        best = float("inf")
+        for _ in range(8):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(4):
+                rode_sddmm(csr, lhs, rhs)
+            end.record()
+            torch.cuda.synchronize()
+            best = min(best, begin.elapsed_time(end))
+        took.append(best)
+    assert took[1] <= 0.85 * took[0], took
