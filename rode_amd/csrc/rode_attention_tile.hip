@@ -13,9 +13,10 @@
 // row by row.
 //
 // Measured (16 384 rows, window 512 and 64 random columns, width 64): eight heads of halves 0.552 ms with four rows at a time on
-// the vector ALUs, 0.206 here; eight heads in fp32 0.693 -> 0.39.  No rate is at its limit: the vector ALUs issue 66 % of the time
-// (a fifth of it the tiles' prologues, once per head), the address units are busy for 63 %, 3.2 GB leave the L2s and 0.62 GB pass
-// them (3.1 TB/s); 2.7 waves per SIMD, which the registers allow, wait for memory 48 % of their time.  What was slow on
+// the vector ALUs, 0.206 here, 0.176 with four tiles a workgroup, which take that call now (attention_wide_kernel); eight heads in fp32 0.693 -> 0.39.
+// No rate was at its limit with those halves: the vector ALUs issued 66 % of the time (a fifth of it the tiles' prologues, once per
+// head), the address units were busy for 63 %, 3.2 GB left the L2s and 0.62 GB passed them (3.1 TB/s); 2.7 waves per SIMD waited for memory
+// 48 % of their time (all before LDS transposed on the way out).  What was slow on
 // the way: dense rows and values loaded straight into operand layout (adjacent lanes on different rows: 64 clocks of the
 // memory pipe per load, 0.38 ms); the nonzeros outside the run of one row after the other (us, fp32 / halves of width 64, one head:
 // 75 / 36 -> 69 / 34, width 128 164 / 68 -> 131 / 58; 20 000 rows of 300 and 96 random columns 121 / 62 -> 97 / 55, width 128 274 / 129 ->
@@ -403,8 +404,9 @@ attention_tile_kernel(int n_tiles, const RowTile* __restrict__ tiles, const int*
 // workgroups that want it.
 //
 // Measured (halves, 16 384 rows, eight heads of width 64): window 512 106 -> 76 us (2.9 M lines past the L2s, 370 MB, four fifths of it
-// values, which every head reads for itself), and 64 random columns 207 -> 175 (7.2 M lines, 920 MB: 5.3 TB/s of the 6.5 to 7 that pass
-// the L2s; rows of k and v outside the runs hit in L2 three times out of four).  A build without the products and the softmax took as
+// values, which every head reads for itself), and 64 random columns 207 -> 176 (6.95 M lines read and 34 MB written past the L2s, 922 MB: 5.2 TB/s of
+// the 6.5 to 7 that pass them; 72 % of the requests hit).  The lines are not all of it: where k and v are one array 3.9 M are read, 533 MB,
+// and the call takes an eighth less (in one program 165 -> 145).  A build without the products and the softmax took as
 // long along the runs; the steps in the order of the columns 83 and 179; as many heads on an XCD as there are 230.
 // Tried for the nonzeros outside the runs (us, of 176): the scores of all rows before the rows of v (fewer lines past the L2s, 690 MB, but a wave
 // per SIMD less) 176; half of the rows at a time 176; those of every other workgroup before its run 178; all loads of four rows at once 194.
@@ -565,18 +567,27 @@ attention_wide_kernel(int nheads, int n_tiles, const RowTile* __restrict__ tiles
 }
 
 // Four tiles a workgroup (attention_wide_kernel, halves) or one?  fours: how many workgroups of four a head's longest one is worth
-// (rode_hip_plans.tile_fours), 0 where the four lie apart or nothing is known.  A wave per tile has to fill the GPU: 512 workgroups, for
-// width 64 640 where rows are long, for width 32 - the values, not shared, are half of what is read - 1024.  us, one tile -> four:
-//   width 64   512: window 400 and 32 random columns 41.7 -> 41.6, 160 + 16 27.6 -> 24.8, 600 + 64 57.3 -> 60.1, 16 heads 37.6 -> 35.0,
-//              25.2 -> 20.8, 49.7 -> 49.8; 256: 25.1 -> 35.2; 640: 45.6 -> 41.4, 768: 77.8 -> 68.3 (600 + 64), 1024: 75.7 -> 61.9
-//   width 128  256: 42.7 -> 47.3; 512: 81.3 -> 69.4, 67.2 -> 50.6, 44.0 -> 29.7 (160 + 16); 640: 82.8 -> 77.3; 1024: 156.6 -> 130.0
-//   width 32   512: 27.6 -> 33.3; 768: 37.0 -> 38.9, 53.2 -> 57.8 (600 + 64); 1024: 50.9 -> 47.4, 32.3 -> 27.7 (160 + 16)
+// (rode_hip_plans.tile_fours), 0 where the four lie apart or nothing is known.  The GPU has room for 1280, 1024 and 512 workgroups at a time
+// (widths 32, 64 and 128; a wave per tile, the other kernel four): a few more than that take a second round nearly alone, and a wave per tile has to
+// fill the GPU.  Width 32, where the values, not shared, are half of what is read, gains by it with short rows or after two rounds.  Time of four
+// over that of one (64 and more random columns; none or few): 2700 masks of 1500 to 20 000 rows, windows of 128 to 640 and 0 to 96 random columns, 1 to 16 heads
+//   width 128  375 workgroups 0.97 to 1.13; 0.83 to 1.04, 450 to 512 0.78 to 0.93; 0.67 to 0.92, 524 to 600 up to 1.16; 1.10, 700 0.90 to 1.08; 0.85 to
+//              0.98, 750 0.84 to 1.02; 0.73 to 0.96, 1025 to 1300 0.81 to 0.98; 0.74 to 0.96
+//   width 64   512 0.98 to 1.10; 0.76 to 1.14 (up to 300 nonzeros a row 1.04), 650 0.94 to 1.01; 0.92 to 0.97, 1000 0.80 to 0.93; 0.65 to 0.86, 1050 up to
+//              1.12, 1150 1.06, 1250 0.94 to 1.02; 0.74 to 1.03, 2000 0.82 to 0.92; 0.65 to 0.87
+//   width 32   1000 0.97 to 1.10; 0.75 to 1.04, 1300 up to 1.22, 1500 1.19, 2000 0.93 to 1.10; 0.72 to 1.06, 2500 0.93 to 0.97; 0.72 to 0.98
+// One of those calls is more than 3 % slower than with a tile a workgroup (1.04).  From 512 workgroups on (1024 for width 32, 640 for rows of 600 of
+// width 64), without a look at the rounds, 298 were, the most 1.22 (8352 rows of 578 and 96 random columns, four heads of 128: 152 -> 181 us).
 //   fp32 (not taken), width 64 768: 104 -> 96, 640: 86 -> 92; 1024: 157 -> 152; width 128 1024: 349 -> 351; width 32 1024: 78 -> 78
 inline bool tiles_in_fours(int d, int nheads, int M, int nnz, int fours)
 {
-    const long long wgs = (long long)fours * nheads;
-    if (d == 32) return wgs >= 1024;
-    return wgs >= (d == 64 && (long long)nnz >= 600ll * M ? 640 : 512);
+    if (fours <= 0) return false;
+    const long long worth = (long long)fours * nheads, quads = (row_tiles(M) + kWavesPerWg - 1) / kWavesPerWg;
+    const long long wgs = quads * nheads > worth ? quads * nheads : worth;
+    const auto rows_of = [&](int most) { return (long long)nnz < (long long)most * M; };
+    if (d == 32) return wgs <= 1280 ? worth >= 900 && rows_of(220) : worth >= (rows_of(300) ? 1900 : 2450);
+    if (d == 64) return wgs <= 1024 ? worth >= (rows_of(300) ? 512 : 640) : worth >= 1024 && wgs >= 1230;
+    return wgs <= 512 ? worth >= 440 : worth >= 600 && wgs >= 740;
 }
 
 template <typename T, int D>

@@ -524,3 +524,21 @@ def test_nonzeros_outside_the_runs_first(bad, keep):
             s = torch.softmax(s.masked_fill(dense == 0, float("-inf")), dim=1)
         s = s[rows, csr.column_indices.long()]
         assert (scores[1].double() - s).abs().max() <= 2e-5 * s.abs().max()
+
+
+@pytest.mark.parametrize("m,window,extra,d,heads,taken", [(8352, 578, 96, 128, 4, False), (8192, 320, 0, 128, 4, True), (6016, 320, 0, 128, 8, True), (17024, 440, 64, 64, 4, False),
+                                                          (16384, 440, 0, 64, 4, True), (5248, 440, 64, 32, 16, False), (16384, 128, 0, 32, 4, True)])
+def test_four_tiles_where_the_last_round_is_not_a_few(m, window, extra, d, heads, taken):
+    """512, 1024 and 1280 workgroups of four tiles run at a time; with a few more than that the others wait for a second round of those (8352 rows x
+    128, 524 workgroups: 152 us with a tile a workgroup, 181).  The bits of a tile a workgroup, or others."""
+    gen, n = torch.Generator(device="cuda").manual_seed(d), m + window
+    row = torch.arange(m, device="cuda")[:, None]
+    col = torch.cat((row + torch.arange(window, device="cuda"), torch.randint(0, n, (m, extra), device="cuda", generator=gen)), 1)
+    keys = torch.unique(row * n + col)
+    ro = torch.searchsorted(keys, torch.arange(m + 1, device="cuda") * n).int().cpu()
+    csr = RoDeCSR(ro, (keys % n).int(), torch.ones(len(keys), device="cuda"), "cuda", m, n, d, config="auto")
+    assert csr.plan.counts[3] == m // 16
+    q, k, v = (torch.randn(heads, r, d, device="cuda", generator=gen).half() for r in (m, csr.n, csr.n))
+    out = sparse_attention(csr, q, k, v)
+    csr.call_plans().tile_fours = 0
+    assert torch.equal(out, sparse_attention(csr, q, k, v)) != taken
