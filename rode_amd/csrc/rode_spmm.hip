@@ -204,10 +204,12 @@ __device__ __forceinline__ void spmm_sum_slots(int base, int mask, int cnt, int 
 // Calls of widths that are a multiple of 32 and not of 128 may take tiles of 128 or 64 columns for tiles of 32 (spmm_tile_of_call), with 2 or 4 times
 // fewer lane groups for a row's slots: their sums are made of sums of eight slots.  2-norms of the errors against fp64 relative to tiles of 32
 // (uniform, width 96): one chain a lane group, 40 nonzeros a row 1.31, halves 1.09, 110 halves 1.38; like this, 34 to 110 nonzeros 0.97 to 1.004,
-// halves 0.985 to 1.001.  Time (us, chain -> this): 4000 rows of 56 7.1 -> 7.2, of 110 x 100 11.1 -> 11.1, 60 K of 56 119 -> 119, halves
+// halves 0.985 to 1.001.  Time (us, chain -> this): 4000 rows of 56 7.1 -> 7.2, 60 K of 56 119 -> 119, halves
 // 8000 of 110 11.9 -> 12.2, 16.5 K of 56 17.0 -> 17.2.
-template <typename T, int TN, bool EDGE>
-constexpr bool kInEights = EDGE && TN >= 64 && sizeof(T) <= 4;
+// (Not for other widths, which had tiles of that many columns before: lognormal 100 K of 30 x 48 93 -> 100 us, 12 K of 14 14.3 -> 15.7.)
+constexpr int kPartialEights = 2; // (EDGE: the last tile is partial (kPartial), and so the sums are)
+template <int EDGE>
+constexpr bool kInEights = EDGE == kPartialEights;
 
 // Which column tile of C, and which of the `blocks` workgroups of its grid row, a workgroup is.
 // shards == 1: tiles in blockIdx.y.  shards > 1 (a divisor of kXcds): XCD x only ever works on tile
@@ -253,7 +255,7 @@ __device__ __forceinline__ bool spmm_wide_item(int seg, int m1, int owned_slots,
 // STORE: a row's only work item stores its sum instead of adding it (owners.overwrite; a
 // kernel of its own as well: as a run-time branch it slowed the fp16 kernel of width 128
 // that never takes it from 0.97 to 1.13 ms on the power-law benchmark).
-template <typename T, int TN, bool EDGE, int WALK, bool STORE>
+template <typename T, int TN, int EDGE, int WALK, bool STORE>
 __device__ __forceinline__ void
 spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, int chunk_hint, RowOwners owners,
                 const int* __restrict__ block_rows,
@@ -305,7 +307,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
             for (unsigned long long todo = scan.items & ((1ull << count) - 1ull); todo; todo &= todo - 1ull) {
                 const BlockItem it = chunk_item(scan, __builtin_ctzll(todo));
                 A total[VEC];
-                spmm_sum_slots<T, TN, 0, kInEights<T, TN, EDGE>>(it.base, it.mask, it.cnt, it.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave,
+                spmm_sum_slots<T, TN, 0, kInEights<EDGE>>(it.base, it.mask, it.cnt, it.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave,
                                       b_lane, n, col, val, total);
                 if (it.row != pending) {
                     if (pending >= 0) flush();
@@ -362,7 +364,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
     constexpr int kPart = WALK == 3 ? kWave : WALK == 4 ? kSpmmMergeSlots : 0;
     A total[VEC];
     __shared__ __attribute__((aligned(16))) A parked[kPart > kWave ? kWgThreads * VEC : 1];
-    spmm_sum_slots<T, TN, kPart, kInEights<T, TN, EDGE>>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total, parked + (kPart > kWave ? threadIdx.x * VEC : 0));
+    spmm_sum_slots<T, TN, kPart, kInEights<EDGE>>(base, mask, cnt, cnt, 0, lane, my_c, my_v, b_lane, n, col, val, total, parked + (kPart > kWave ? threadIdx.x * VEC : 0));
     if (shared_row) {
         __shared__ __attribute__((aligned(16))) A wg_sum[kWavesPerWg][TN];
         if (group == 0) {
@@ -399,7 +401,7 @@ spmm_block_body(int bid, int nblocks, int tile, int m1, int n, int owned_slots, 
 
 // One group of LPR lanes per residue row (tail selection: RoDeSpmm.cu:71-82); the
 // group walks its row's slot quads one after the other, no cross-lane reduction.
-template <typename T, int TN, bool EDGE>
+template <typename T, int TN, int EDGE>
 __device__ __forceinline__ void
 spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots, RowOwners owners,
                   const int* __restrict__ residue_rows,
@@ -478,7 +480,7 @@ spmm_residue_body(int bid, int nblocks, int tile, int m2, int n, int owned_slots
     }
 }
 
-template <typename T, int TN, bool EDGE, int WALK, bool STORE>
+template <typename T, int TN, int EDGE, int WALK, bool STORE>
 __global__ void __launch_bounds__(kWgThreads)
 spmm_block_kernel(int shards, int m1, int n, int owned_slots, int chunk_hint, RowOwners owners, const int* __restrict__ block_rows,
                   const int* __restrict__ st_off,
@@ -491,7 +493,7 @@ spmm_block_kernel(int shards, int m1, int n, int owned_slots, int chunk_hint, Ro
                                        row_ptr, col, val, B, C);
 }
 
-template <typename T, int TN, bool EDGE>
+template <typename T, int TN, int EDGE>
 __global__ void __launch_bounds__(kWgThreads)
 spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners, const int* __restrict__ residue_rows,
                     const int* __restrict__ row_ptr, const int* __restrict__ col,
@@ -506,7 +508,7 @@ spmm_residue_kernel(int shards, int m2, int n, int owned_slots, RowOwners owners
 // The rows of C without slots, which are in neither list, where nobody cleared C: 64 at a time to the waves, whose lanes zero the tile of
 // several rows at once, 16 bytes each.  (A matrix may be mostly such rows: in waves of 256 that took one after the other, 100 K x 128 with
 // 50 rows that are not empty took 29.4 us instead of 12.8 with a clearing launch, 1 M x 32 34 instead of 22.)
-template <typename A, int TN, bool EDGE>
+template <typename A, int TN, int EDGE>
 __device__ __forceinline__ void spmm_empty_rows(int bid, int nblocks, int tile, int rows, int n, const int* __restrict__ row_ptr, A* __restrict__ C)
 {
     constexpr int VEC = 16 / (int)sizeof(A), LPR = TN / VEC, AT_ONCE = kWave / LPR;
@@ -529,7 +531,7 @@ inline int empty_row_workgroups(int rows) { return (min((rows + kWgThreads - 1) 
 // grid) work on block segments, the others on residue rows.  For matrices so small that a launch costs as much as its
 // kernel (a kernel of a few microseconds); the two parts then also fill the GPU together.
 // g0 > 0 (with STORE: every other row is stored): as many workgroups after them zero the rows without slots.
-template <typename T, int TN, bool EDGE, int WALK, bool STORE>
+template <typename T, int TN, int EDGE, int WALK, bool STORE>
 __global__ void __launch_bounds__(kWgThreads)
 spmm_pair_kernel(int shards, int g0, int rows, int g1, int m1, int m2, int n, int owned_slots, int chunk_hint, RowOwners owners,
                  const int* __restrict__ block_rows,
@@ -562,7 +564,7 @@ spmm_pair_kernel(int shards, int g0, int rows, int g1, int m1, int m2, int n, in
 // column index is read).  Then the rows' other nonzeros: with one wave per group, of the four rows together;
 // with a workgroup, wave w adds row w's, the waves' sums meet in LDS, and wave w adds the
 // total of row w to C.  A row is in no other work item: no atomics.
-template <typename T, int TN, bool EDGE, int WPG>
+template <typename T, int TN, int EDGE, int WPG>
 __global__ void __launch_bounds__(kWgThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 spmm_group_kernel(int n, int n_groups, const RowGroup* __restrict__ groups, const int* __restrict__ row_ptr,
                   const int* __restrict__ col, const typename DenseVec<T>::Acc* __restrict__ val,
@@ -744,7 +746,7 @@ spmm_group_kernel(int n, int n_groups, const RowGroup* __restrict__ groups, cons
 // pieces up), or, without that workspace, is added to its row of C atomically (a hub row
 // then gets one atomic row update per slab: slower than the plain kernels at 512-byte rows).
 // A piece that waves share is finished by the wave that has its first step.
-template <typename T, int TN, bool EDGE>
+template <typename T, int TN, int EDGE>
 __global__ void __launch_bounds__(kHubWavesMax * kWave)
 spmm_hub_kernel(int n, HubGrid grid, const int* __restrict__ hub, const int* __restrict__ col,
                 const typename DenseVec<T>::Acc* __restrict__ val, const T* __restrict__ B,
@@ -771,7 +773,7 @@ spmm_hub_kernel(int n, HubGrid grid, const int* __restrict__ hub, const int* __r
     for (unsigned long long todo = share.pieces; todo; todo &= todo - 1ull) {
         const int i = __builtin_ctzll(todo);
         const HubPart p = hub_part(share, i);
-        spmm_sum_slots<T, TN, 0, kInEights<T, TN, EDGE>>(p.base, 0, p.cnt, p.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
+        spmm_sum_slots<T, TN, 0, kInEights<EDGE>>(p.base, 0, p.cnt, p.cnt, 0, lane, lds_c + wave * kWave, lds_v + wave * kWave, b_lane, n, col, val, total);
         if (!partial) {
             A* c_lane = C + (size_t)p.row * n + tile + ls * VEC;
 #pragma unroll
@@ -894,7 +896,7 @@ inline HubRows spmm_hub_rows(const int* counts, int n, int tile, size_t elem)
     return hub_rows_of_call(counts, n * elem, tile * elem, (n + tile - 1) / tile, 18, 600, (size_t)8 * kHubSlabRows * counts[1]);
 }
 
-template <typename T, int TN, bool EDGE>
+template <typename T, int TN, int EDGE>
 hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* residue_rows, const int* st_off,
                   const int* row_ptr, const int* col, const typename DenseVec<T>::Acc* val, const T* B,
                   typename DenseVec<T>::Acc* C, int flags, PlanRef plan, hipStream_t s1, hipStream_t s2)
@@ -994,7 +996,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         }
         if (residue && standard_residue) {
             dim3 grid(g2 * shards, tile_rows);
-            spmm_residue_kernel<T, TN, EDGE><<<grid, kWgThreads, 0, s2>>>(shards, m2, n, owned_slots, owners, residue_rows, row_ptr, col,
+            spmm_residue_kernel<T, TN, (EDGE != 0 ? kPartial : 0)><<<grid, kWgThreads, 0, s2>>>(shards, m2, n, owned_slots, owners, residue_rows, row_ptr, col,
                                                                           val, B, C, plan.dev);
             if (e == hipSuccess) e = hipGetLastError();
         }
@@ -1017,11 +1019,11 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
         if (plan.group_counts[1] >= kGroupWaveEach) {
             const int wgs = (owners.n_groups + kWavesPerWg - 1) / kWavesPerWg;
             dim3 grid((wgs + kXcds - 1) / kXcds * kXcds, tiles);
-            spmm_group_kernel<T, TN, EDGE, 1><<<grid, kWgThreads, 0, s1>>>(n, owners.n_groups, owners.groups, row_ptr, col,
+            spmm_group_kernel<T, TN, (EDGE != 0 ? kPartial : 0), 1><<<grid, kWgThreads, 0, s1>>>(n, owners.n_groups, owners.groups, row_ptr, col,
                                                                            val, B, C, overwrite);
         } else {
             dim3 grid((owners.n_groups + kXcds - 1) / kXcds * kXcds, tiles);
-            spmm_group_kernel<T, TN, EDGE, kWavesPerWg><<<grid, kWgThreads, 0, s1>>>(n, owners.n_groups, owners.groups, row_ptr,
+            spmm_group_kernel<T, TN, (EDGE != 0 ? kPartial : 0), kWavesPerWg><<<grid, kWgThreads, 0, s1>>>(n, owners.n_groups, owners.groups, row_ptr,
                                                                                      col, val, B, C, overwrite);
         }
         e = hipGetLastError();
@@ -1036,10 +1038,13 @@ hipError_t launch_edge(int m1, int m2, int n, const int* block_rows, const int* 
                        const int* row_ptr, const int* col, const typename DenseVec<T>::Acc* val, const T* B,
                        typename DenseVec<T>::Acc* C, int flags, PlanRef plan, hipStream_t s1, hipStream_t s2)
 {
-    return n % TN ? launch<T, TN, true>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C,
-                                        flags, plan, s1, s2)
-                  : launch<T, TN, false>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C,
-                                         flags, plan, s1, s2);
+    if constexpr (TN >= 64 && sizeof(T) <= 4)
+        if (n % TN && n % 32 == 0) // (spmm_tile_of_call)
+            return launch<T, TN, kPartialEights>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C, flags, plan, s1, s2);
+    return n % TN ? launch<T, TN, kPartial>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C,
+                                            flags, plan, s1, s2)
+                  : launch<T, TN, 0>(m1, m2, n, block_rows, residue_rows, st_off, row_ptr, col, val, B, C,
+                                     flags, plan, s1, s2);
 }
 
 } // namespace
@@ -1124,7 +1129,7 @@ hipError_t spmm_launch(int m1, int m2, int n, const int* block_rows, const int* 
                          kHalves = {0.79f, 0.0113f, 1.07f, 270, 1.17f, 380}, kDoubles = {0.75f, 0.0228f, 1.f, 360, 1.17f, 360};
     const size_t row_bytes = (size_t)n * sizeof(T);
     const int slices = ring_slices(row_bytes);
-    // (a band of 128 columns is worth 5 % less than those of 192 and 256 that the figures beside ring_pays are of)
+    // (a band of 128 columns is worth 5 % less than those of 192 and 256 that the figures beside rings_pay are of)
     const bool line = row_bytes == 128, whole = slices == 1;
     const WindowGain ring = sizeof(T) == 8 ? WindowGain{line ? 1.2f : whole ? 0.94f : 1.1f, line ? 0.03f : whole ? 0.025f : 0.02f, 1.f, 0, 1.f, 0}
                             : sizeof(T) == 2 ? WindowGain{line ? 0.72f : whole ? 0.93f : 0.97f, line ? 0.0145f : 0.02f, 1.f, 0, 1.f, 0}

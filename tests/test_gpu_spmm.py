@@ -943,3 +943,20 @@ def test_rows_of_thousands_of_slots_by_a_workgroup_each(k, dtype):
     want, scale = oracle.spmm_f64(rp, col, val, dense, with_abs=True)
     # roundings of a sum: 512 slots over two lane groups, nine more parts, the groups (5), the waves (3) and the product
     assert (np.abs(got - want) <= scale * (256 + 9 + 5 + 3 + 1) * (2.0 ** -53 if dtype == "f64" else 2.0 ** -24)).all()
+
+
+@pytest.mark.parametrize("half,width,tiles", [(False, 48, 64), (False, 100, 128), (False, 40, 64), (True, 48, 64), (True, 104, 128)])
+def test_widths_that_are_no_multiple_of_32_are_summed_as_those_that_are(half, width, tiles):
+    """Tiles of that many columns are theirs anyway: the bits of the same columns of a whole tile, not sums of eight slots (rows of 30 on average, lognormal,
+    100 K x 48: 93.3 us, and 100.2 with those)."""
+    from gpu_common import DEV
+    from rode_amd import RoDeCSR, rode_spmm
+    gen = torch.Generator(device=DEV).manual_seed(width)
+    rows = 3000
+    lens = torch.randint(33, 120, (rows,), device=DEV, generator=gen)
+    ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0)))
+    col = torch.randint(0, rows, (int(ro[-1]),), device=DEV, generator=gen).int()
+    csr = RoDeCSR(ro.int().cpu(), col, torch.rand(col.numel(), device=DEV, generator=gen), DEV, rows, rows, width, config="auto")
+    assert csr.m1 >= 1024  # (rows with one work item each)
+    B = torch.randn(rows, tiles, device=DEV, generator=gen).to(torch.float16 if half else torch.float32)
+    assert torch.equal(rode_spmm(csr, B[:, :width].contiguous()), rode_spmm(csr, B)[:, :width])
