@@ -319,7 +319,8 @@ int rode_hip_group_plan_fours(int M, const int* d_row_offsets, const int* d_colu
  *                         well: SpMM then does not deal column tiles out to the XCDs, which pays
  *                         when dense rows are referenced at random.  Plus, where no row has more than twice as many
  *                         as there are on average, twice the nonzeros a row: SDDMM of widths other than 32, 64, 128 and
- *                         their multiples then decides by them how many dense rows a wave has on their way.  Costs time at worst.
+ *                         their multiples then decides by them how many dense rows a wave has on their way, SpMM of halves
+ *                         of widths like 96 how wide its tiles are.  Costs time at worst.
  *   nonzeros              0, or the nonzeros of the matrix.  With it a call may leave a locality plan
  *                         unused where the window kernels do not pay (short rows, a last round of few
  *                         chunks), and dealing tiles out depends on how often a dense row is used.

@@ -1070,12 +1070,18 @@ static int spmm_tile_width(int n, size_t elem)
 // and lognormal degrees, two matrices in turn:
 // Halves: a tile of 32 is half a line of 128 bytes, which is fetched for each of the two.  Tiles of 128 (u 16 K of 110 x 96 34.6 / 29.4 / 24.1, 60 K of 20
 // 51 / 44 / 37, 400 K of 14 336 / 279 / 218), but of 64
-//   * where those of 128 have a quarter of their lanes and more idle (x 160: u 33 K of 110 120 / 119 / 144, 8000 of 14 8.3 MB 0.91 / 1.15);
+//   * where those of 128 have a quarter of their lanes and more idle, up to 30 MB (x 160: u 33 K of 110 120 / 119 / 144; 48 MB and more 1 / 0.80 to
+//     0.89 / 0.73 to 0.86);
 //   * where the dense operand is near the size of an L2 and its rows are used less than 12 times (u 33 K of 8 x 96 13.3 / 13.4 / 14.7), up to 3.5 MB
 //     less than 24 (16.5 K of 20 x 96 9.9 / 9.4 / 10.6); less than 10 times and 12 to 16 MB, those of 32 (u 33 K of 8 x 224 22.8 / 25.6 / 24.9);
 //   * where one wave has all of a row, and the wider its tiles the longer for it, up to 1024 slots at 1 to 2.5 ns: 128 columns from 200 KB to
 //     gather for each of its slots on, 64 from 90 KB (x 96: 12 K of 14, 899 slots, 36 KB each 11.4 / 14.5 / 16.3; 20 K of 20, 72 KB 18.9 / 17.4 / 20.2;
 //     26 K of 32, 155 KB 32 / 27 / 30; 60 K of 14, 156 KB 38 / 34 / 33; 60 K of 32, 360 KB 74 / 70 / 60).
+//     Rows of equal length have no such row, if they are more than tails (u x 96, 1 / 128 columns: 4000 of 30 0.81, of 60 0.72, 12 K of 60 0.68, 30 K of 22
+//     0.77, but 4000 of 8 to 22 1.13 to 1.20).
+//   * Both are otherwise with rows of unequal length and an operand past the L2s, which is waited for longer than that row: from 60 KB on, and near the
+//     size of an L2 as well (lognormal x 96: 30 K of 8, 42 KB 15.6 / - / 19.1, 30 K of 22, 124 KB 28.2 / 26.1 / 24.1, 60 K of 8, 90 KB 27.1 / 27.1 / 24.1, 100 K of
+//     8 44.0 / 41.8 / 36.5).
 // 32-bit operands: one line at a time keeps more of the operand in the L2s, as long as its tiles fit at all (sharding_pays); below 2.5 MB and above
 // 26 MB a tile whole rows are better, if a quarter of the lanes at most has nothing and with 500 KB to gather for each slot of the longest row
 // (u 4000 of 40 x 96 9.9 -> 8.2, 230 K of 12 167 -> 161, 300 K of 10 187 -> 178, between them u 10 K of 20 8.2 -> 9.0, u 16 K of 110 37 -> 43; 4000 of 32,
@@ -1089,14 +1095,16 @@ static int spmm_tile_of_call(int n, size_t elem, const PlanRef& plan)
     if (least != 32 || n <= 32 || elem > 4 || n % 32 != 0 || plan.groups) return least;
     constexpr size_t KB = 1000, MB = 1000000;
     const size_t rows = plan.dense_rows, nonzeros = plan.nonzeros, bytes = rows * n * elem, gathered = nonzeros * n * elem;
-    const size_t slots = plan.longest > 0 && plan.longest < kOwnedRowSlots ? plan.longest : kOwnedRowSlots;
+    size_t slots = plan.longest > 0 && plan.longest < kOwnedRowSlots ? plan.longest : kOwnedRowSlots;
+    if (plan.equal_rows >= (bytes < 5 * MB ? 28 : 16)) slots = min(slots, (size_t)2 * plan.equal_rows); // (not said in calls whose rows are all stored)
     auto enough = [&](size_t each) { return nonzeros == 0 || gathered >= slots * each; }; // (not said: taken to be)
     if (plan.columns_local && bytes < 26 * MB) return 32;
     const bool filled = 3 * ((n + 127) / 128 * 128) <= 4 * n;
     if (elem == 4) return filled && rows > 0 && (bytes <= 5 * MB / 2 || rows * 128 > 27 * MB) && enough(500 * KB) ? 128 : 32;
-    if (nonzeros > 0 && nonzeros < 10 * rows && bytes > 12 * MB && bytes < 16 * MB) return 32;
-    const bool near_l2 = nonzeros > 0 && nonzeros < (bytes < 7 * MB / 2 ? 24 : 12) * rows && bytes >= 3 * MB && bytes <= 12 * MB;
-    return filled && !near_l2 && enough(200 * KB) ? 128 : enough(90 * KB) ? 64 : 32;
+    const bool ragged = plan.equal_rows == 0 && bytes >= 11 * MB / 2;
+    if (!ragged && nonzeros > 0 && nonzeros < 10 * rows && bytes > 12 * MB && bytes < 16 * MB) return 32;
+    const bool near_l2 = !ragged && nonzeros > 0 && nonzeros < (bytes < 7 * MB / 2 ? 24 : 12) * rows && bytes >= 3 * MB && bytes <= 12 * MB;
+    return (filled || bytes >= 30 * MB) && !near_l2 && enough((ragged ? 60 : 200) * KB) ? 128 : enough((ragged ? 60 : 90) * KB) ? 64 : 32;
 }
 
 // The partial rows that the hub kernels of an SpMM of this width want, for operands of 4 (or, if more, 2) or of 8 bytes an element.
