@@ -79,12 +79,14 @@ constexpr int kMergeMinSegments = 16384;
 //     150 K x 128 167 -> 163, 180 K of 20 halves x 128 135 -> 132; 113 K of 23 x 32, 332 MB, 44.7 -> 49.6.
 // 2-norms of the long rows' errors against fp64, relative to adding their segments up (which were merged to 512 slots as well): 0.97 to 1.006,
 // rows of 1100 to 6500, widths 32 to 128, both types.
-inline bool wide_rows_pay(int longest, int seg_length, size_t tile_bytes, size_t gathered)
+// Not above 6656 slots with partial tiles, whose matrices have B past the L2s and no tiles of one line (30 K of 110 x 100 154 -> 166, x 112 165 -> 177, 60 K
+// of 60 x 100 212 -> 224, of 110 x 56 202 -> 213).
+inline bool wide_rows_pay(int longest, int seg_length, size_t tile_bytes, size_t gathered, bool partial)
 {
     constexpr size_t MB = 1000000;
     if (seg_length > (gathered >= 500 * MB ? 512 : 128)) return false;
     if (gathered < (tile_bytes > 256 ? 500 : 300) * MB) return longest <= (tile_bytes > 256 ? 2048 : tile_bytes > 128 ? 3072 : 4096);
-    return (size_t)longest <= min(max((size_t)6656, gathered / 100000), (size_t)20000);
+    return (size_t)longest <= (partial ? (size_t)6656 : min(max((size_t)6656, gathered / 100000), (size_t)20000));
 }
 
 // Up to this many workgroups, and when both kernels go to the same stream, the two lists
@@ -957,7 +959,7 @@ hipError_t launch(int m1, int m2, int n, const int* block_rows, const int* resid
     bool wide = false;
     if (plan.c_rows > 0) { // C is not cleared
         const bool all_stored = pair && owners.overwrite && !group_plan && plan.dev == nullptr && plan.longest > 0;
-        wide = all_stored && chunk_hint == 1 && plan.longest > kOwnedRowSlots && wide_rows_pay(plan.longest, plan.seg_length, TN * sizeof(T), (size_t)plan.nonzeros * n * sizeof(T));
+        wide = all_stored && chunk_hint == 1 && plan.longest > kOwnedRowSlots && wide_rows_pay(plan.longest, plan.seg_length, TN * sizeof(T), (size_t)plan.nonzeros * n * sizeof(T), EDGE != 0);
         if (wide || (all_stored && plan.longest <= kOwnedRowSlots)) {
             g0 = empty_row_workgroups(plan.c_rows);
         } else {

@@ -979,3 +979,27 @@ def test_rows_of_equal_length_take_the_wider_tiles(rows, degree, width, wide):
     got = rode_spmm(csr, B)
     assert torch.equal(got, narrow) != wide
     assert (got - narrow).abs().max() <= 1e-5 * narrow.abs().max()
+
+
+def test_longest_rows_with_partial_tiles_are_added_to():
+    """Rows of 12 000 slots in a matrix with 1.3 GB to gather, width 100: not by a workgroup each (30 K rows of 110: 154 us added to, 166 stored), of 6000 they are.
+    Said of a smaller matrix; what is by a workgroup is summed in quarters."""
+    from gpu_common import DEV
+    from rode_amd import RoDeCSR, rode_sddmm_hip
+    gen = torch.Generator(device=DEV).manual_seed(0)
+    rows, width = 3000, 100
+    lens = torch.randint(33, 60, (rows,), device=DEV, generator=gen)
+    lens[5] = 5996
+    ro = torch.cat((torch.zeros(1, dtype=torch.int64, device=DEV), lens.cumsum(0))).int().cpu()
+    col = torch.randint(0, 20000, (int(ro[-1]),), device=DEV, generator=gen).int()
+    csr = RoDeCSR(ro, col, torch.rand(col.numel(), device=DEV, generator=gen), DEV, rows, 20000, width, locality=False, config="auto")
+    B = torch.randn(20000, width, device=DEV, generator=gen)
+    plans = rode_sddmm_hip.plans_struct(None, whole_lists=True, seg_length=csr.config["seg_length"], nonzeros=1_300_000_000 // (width * 4))
+    short, long_one, added = (torch.from_numpy(_into_nan(csr, B, longest, plans)) for longest in (6000, 12000, 0))
+    others = torch.arange(rows) != 5
+    assert torch.equal(short[others], added[others]) and torch.equal(long_one[others], added[others])
+    assert not torch.equal(short[5], long_one[5]) and not torch.equal(short[5], added[5])  # (adding its segments up has another order)
+    part = csr.values[ro[5]:ro[6]].double(), B[col[ro[5]:ro[6]].long()].double()
+    # roundings of a sum: 512 slots over two lane groups, up to 47 segments, the groups (5), the waves (3) and the product
+    bound = (part[0] @ part[1].abs()).cpu() * (256 + 47 + 5 + 3 + 1) * 2.0 ** -24
+    assert all(((C[5] - (part[0] @ part[1]).cpu()).abs() <= bound).all() for C in (short, long_one, added))
