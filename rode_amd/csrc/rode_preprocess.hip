@@ -416,7 +416,7 @@ hipError_t preprocess_placed_launch(int seg, int kblock, int veclen, int M, cons
     const TileShape shape = tile_shape_for((size_t)M);
     const int ntiles = (int)(((size_t)M + shape.rows() - 1) / shape.rows());
     unsigned long long* ws = const_cast<unsigned long long*>(before); // (only read)
-    if (places) { // list and plan at once (preprocess_plan_tile_rows)
+    if (places) { // list and plan at once (preprocess_plan_too)
         auto kernel = shape.rows_per_thread == 1 ? decompose_plan_kernel<kWgThreads, 1> : decompose_plan_kernel<kWgThreads, 4>;
         kernel<<<plan_chunks + ntiles, kWgThreads, 0, stream>>>(make_params(seg, kblock, veclen), M, ntiles, capacity_blocks, capacity_residue, row_ptr, ws,
                                                                 block_r_ind, st_off, residue_r_ind, n_blk, n_res, plan_chunks, places, dense_rows, col,
