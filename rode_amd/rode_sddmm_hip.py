@@ -320,7 +320,7 @@ def plans_struct(plan, spmm_width=None, spmm_elem_bytes=4, whole_lists=True, seg
     ``nonzeros``: of the matrix, 0 when not known.
     ``equal_rows``: nonzeros a row where no row has more than twice as many, else 0."""
     p = _lib.Plans()
-    p.columns_local = int(columns_local) | equal_rows << 1
+    p.columns_local = int(bool(columns_local)) | equal_rows << 1
     p.nonzeros = int(nonzeros)
     p.seg_length = int(seg_length or 0)  # (the segment length of the decomposition, when the caller knows it)
     if isinstance(plan, GroupPlan):

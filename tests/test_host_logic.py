@@ -130,3 +130,9 @@ def test_auto_config_with_more_rows_than_a_library_quantile_takes():
     lens[: m // 20] = 1500  # 5 % long rows: the 90th percentile is 40 (+ 0..3 of alignment) -> 512
     rp[1:] = torch.cumsum(lens, 0)
     assert RoDeCSR.auto_config(rp)["seg_length"] == 512
+
+
+@pytest.mark.parametrize("local,equal_rows,field", [(False, 0, 0), (True, 0, 1), (2, 0, 1), (np.int64(6), 0, 1), (False, 40, 80), (2, 40, 81), (True, 1 << 20, (2 << 20) + 1)])
+def test_what_is_said_of_columns_and_of_rows_is_kept_apart(local, equal_rows, field):
+    """Any true value says that columns lie close together, and nothing of the rows' lengths."""
+    assert rode_sddmm_hip.plans_struct(None, columns_local=local, equal_rows=equal_rows).columns_local == field
